@@ -356,7 +356,85 @@ __global__ __launch_bounds__(THREADS) void layer_norm_kernel(const char* x, long
   }
 }
 
-// Rotary only: x, y [B, S, H, D]; one thread per (row, pair).
+// Rotary only, x and y contiguous [B, S, H, D] (may be the same memory): HBM bound, every element read and written
+// once.  A lane owns the 16-byte vector at pair offset p and the one at p + R2, so a rotated pair never leaves it (and in
+// place works), or two vectors of the pass-through tail; a row is 2^lpr_log2 lanes and a workgroup owns one contiguous
+// piece of ROT_ROWS rows per row slot, all of whose loads are in flight together.  cos / sin rows come from the
+// caches: the heads of a token read the same one.  fp32 [37440, 24, 128]: 160 us, 5.8 TB/s (what a plain copy
+// reaches), against 300-313 us, 3.0 TB/s, with one pair of elements per lane (the form below); bf16 86 against 263 us.
+constexpr int ROT_ROWS = 2;  // rows per lane
+template <bool BF16>
+__global__ __launch_bounds__(THREADS) void rotary_vec_kernel(const char* xin, const float* cosp, const float* sinp, char* yout,
+                                                             unsigned rows, int S, int H, int R2, int lpr_log2) {
+  constexpr int VE = BF16 ? 8 : 4;  // elements per vector
+  const int row_bytes = 32 << lpr_log2;
+  const int slots = THREADS >> lpr_log2;  // rows in flight per pass of the workgroup
+  const int j = threadIdx.x & ((1 << lpr_log2) - 1), slot = threadIdx.x >> lpr_log2;
+  const unsigned first = blockIdx.x * (unsigned)(slots * ROT_ROWS);
+  const bool rot = j < R2 / VE;
+  const int ea = rot ? VE * j : 2 * R2 + 2 * VE * (j - R2 / VE);
+  const int eb = rot ? ea + R2 : ea + VE;
+  constexpr int ES = BF16 ? 2 : 4;
+  u32x4 va[ROT_ROWS], vb[ROT_ROWS];
+  f32x4 cs[ROT_ROWS][VE / 4], sn[ROT_ROWS][VE / 4];
+#pragma unroll
+  for (int k = 0; k < ROT_ROWS; ++k) {
+    const unsigned row = first + (unsigned)(slot + k * slots);
+    if (row < rows) {
+      const char* src = xin + (long)row * row_bytes;
+      va[k] = *(const u32x4*)(src + ea * ES);
+      vb[k] = *(const u32x4*)(src + eb * ES);
+      if (rot) {
+        const long at = (long)(row / (unsigned)H % (unsigned)S) * R2 + VE * j;
+#pragma unroll
+        for (int i = 0; i < VE / 4; ++i) {
+          cs[k][i] = *(const f32x4*)(cosp + at + 4 * i);
+          sn[k][i] = *(const f32x4*)(sinp + at + 4 * i);
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < ROT_ROWS; ++k) {
+    const unsigned row = first + (unsigned)(slot + k * slots);
+    if (row >= rows) break;
+    if (rot) {
+      float a[VE], b[VE];
+      if constexpr (BF16) {
+        unpack8(va[k], a);
+        unpack8(vb[k], b);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {  // (whole vectors: a bit cast of one element of a vector reads element 0)
+          a[i] = __builtin_bit_cast(f32x4, va[k])[i];
+          b[i] = __builtin_bit_cast(f32x4, vb[k])[i];
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < VE; ++i) {
+        const float x1 = a[i], x2 = b[i], c = cs[k][i >> 2][i & 3], sv = sn[k][i >> 2][i & 3];
+        a[i] = x1 * c - x2 * sv;
+        b[i] = x1 * sv + x2 * c;
+      }
+      if constexpr (BF16) {
+        va[k] = pack8(a);
+        vb[k] = pack8(b);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          va[k][i] = __builtin_bit_cast(unsigned, a[i]);
+          vb[k][i] = __builtin_bit_cast(unsigned, b[i]);
+        }
+      }
+    }
+    char* dst = yout + (long)row * row_bytes;
+    *(u32x4*)(dst + ea * ES) = va[k];
+    *(u32x4*)(dst + eb * ES) = vb[k];
+  }
+}
+
+// The same for row lengths, rotary widths or addresses that do not split into 16-byte vectors; one thread per
+// (row, pair).
 template <bool BF16>
 __global__ __launch_bounds__(THREADS) void rotary_kernel(const void* xin, const float* cosp, const float* sinp,
                                                          void* yout, long rows, int S, int H, int Dd, int R2) {
@@ -511,6 +589,23 @@ hipError_t launch_rotary(const void* x, const float* cos, const float* sin, void
   const long rows = (long)B * S * H;
   const long threads = rows * (Dd / 2);
   if (threads <= 0) return hipSuccess;
+  const int ve = is_bf16 ? 8 : 4;
+  const int lpr = Dd / (2 * ve);  // lanes per row of the vector form
+  const uintptr_t addr = (uintptr_t)x | (uintptr_t)y | (R2 > 0 ? (uintptr_t)cos | (uintptr_t)sin : 0);
+  if (Dd % (2 * ve) == 0 && (lpr & (lpr - 1)) == 0 && lpr <= THREADS && R2 % ve == 0 && (addr & 15u) == 0 &&
+      rows < 0x7fffff00L) {
+    const long per_wg = (long)(THREADS / lpr) * ROT_ROWS;
+    const dim3 grid((unsigned)((rows + per_wg - 1) / per_wg));
+    const char* xp = static_cast<const char*>(x);
+    char* yp = static_cast<char*>(y);
+    if (is_bf16)
+      hipLaunchKernelGGL(rotary_vec_kernel<true>, grid, dim3(THREADS), 0, stream, xp, cos, sin, yp, (unsigned)rows, S, H, R2,
+                         __builtin_ctz(lpr));
+    else
+      hipLaunchKernelGGL(rotary_vec_kernel<false>, grid, dim3(THREADS), 0, stream, xp, cos, sin, yp, (unsigned)rows, S, H, R2,
+                         __builtin_ctz(lpr));
+    return hipGetLastError();
+  }
   const unsigned grid = (unsigned)((threads + THREADS - 1) / THREADS);
   if (is_bf16)
     hipLaunchKernelGGL(rotary_kernel<true>, dim3(grid), dim3(THREADS), 0, stream, x, cos, sin, y, rows, S, H, Dd, R2);

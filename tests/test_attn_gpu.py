@@ -181,6 +181,28 @@ def test_apply_rotary_emb_matches_oracle(dev):
         M.apply_rotary_emb(x.to(dev).transpose(1, 2).contiguous().transpose(1, 2), cos.to(dev), sin.to(dev), inplace=True)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("B,S,H,D,R2", [(1, 1, 1, 128, 48), (1, 33, 1, 128, 48), (2, 17, 5, 128, 64), (1, 40, 24, 128, 0),
+                                        (3, 7, 2, 32, 8), (1, 9, 3, 256, 96),            # 16-byte vectors
+                                        (1, 11, 3, 96, 24), (2, 5, 2, 128, 18), (1, 6, 1, 10, 3)])  # one element at a time
+def test_rotary_row_lengths_widths_and_remainders(dev, B, S, H, D, R2, dtype):
+    """Both forms of the rotary kernel at whole and partial workgroups (and an address that is not 16-byte aligned)
+    against float64.  Bound: two products and one sum in fp32 (3 ulp of |x1| + |x2|), plus half a bf16 ulp."""
+    g = torch.Generator().manual_seed(D + R2)
+    x = torch.randn(B, S, H, D, generator=g).to(dtype)
+    ang = torch.randn(S, R2, generator=g)
+    cos, sin = ang.cos(), ang.sin()
+    x1, x2 = x[..., :R2].double(), x[..., R2:2 * R2].double()
+    c, s = cos.double()[None, :, None], sin.double()[None, :, None]
+    ref = torch.cat([x1 * c - x2 * s, x1 * s + x2 * c, x[..., 2 * R2:].double()], dim=-1)
+    mag = torch.cat([x1.abs() + x2.abs()] * 2 + [torch.zeros_like(x[..., 2 * R2:]).double()], dim=-1)
+    bound = 3 * 2.0 ** -24 * mag + (2.0 ** -8 * ref.abs() * (mag > 0) if dtype == torch.bfloat16 else 0)
+    odd = torch.empty(x.numel() + 1, dtype=dtype, device=dev)[1:].view(x.shape).copy_(x)  # starts off a 16-byte boundary
+    for xd in (x.to(dev), odd):
+        y = M.apply_rotary_emb(xd, cos.to(dev), sin.to(dev))
+        assert ((y.cpu().double() - ref).abs() <= bound).all()
+
+
 def test_rejects_bad_arguments(dev):
     q = torch.zeros(8, 2, 64, dtype=torch.bfloat16, device=dev)
     r = torch.zeros(1, 2, dtype=torch.int32, device=dev)
