@@ -34,7 +34,7 @@ struct AttnKernArgs {
   int scale_chunk_tokens;
   int scale_split_chunk;  // first chunk served by the side segment's scale tables (INT_MAX without them)
   int flags;  // MAGI_ATTN_* bits of the public header, plus ATTN_BOUNDED / ATTN_SCALE_Q
-  unsigned total_wgs, per_xcd;
+  unsigned per_xcd;  // workgroups per XCD (the grid is 8 of these)
   float scale_log2;  // softmax_scale * log2(e)
   float q_norm_eps;
   int q_norm_kind;  // MAGI_NORM_LAYERNORM_1P / MAGI_NORM_RMSNORM_1P

@@ -181,6 +181,20 @@ def test_apply_rotary_emb_matches_oracle(dev):
         M.apply_rotary_emb(x.to(dev).transpose(1, 2).contiguous().transpose(1, 2), cos.to(dev), sin.to(dev), inplace=True)
 
 
+@pytest.mark.parametrize("Hq,Hkv", [(1, 1), (6, 2), (3, 3), (8, 4), (5, 5), (7, 7), (9, 9), (20, 10), (12, 12), (16, 16)])
+def test_every_head_count_is_dealt_completely(dev, Hq, Hkv):
+    """Key heads that do not divide over the eight XCDs: with V = head index every row of every head has to come out
+    as its own kv head's index (bit exact: the weights are a convex combination of one value), whatever kernel runs."""
+    tq, tk = _ranges(dev, [[0, 130], [130, 200], [200, 657]], [[0, 70], [10, 300], [0, 64]])
+    q = torch.randn(657, Hq, 128, device=dev, generator=torch.Generator(device=dev).manual_seed(Hq)).bfloat16()
+    k = torch.randn(300, Hkv, 128, device=dev, generator=torch.Generator(device=dev).manual_seed(Hkv)).bfloat16()
+    v = torch.arange(Hkv, device=dev).bfloat16().view(1, Hkv, 1).expand(300, Hkv, 128).contiguous()
+    want = (torch.arange(Hq, device=dev) // (Hq // Hkv)).bfloat16().view(1, Hq, 1)
+    for kw in ({}, {"score_bound": 60.0}):
+        out, _ = M.range_attention(q, k, v, tq, tk, 457, **kw)
+        assert torch.equal(out, want.expand_as(out))
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("B,S,H,D,R2", [(1, 1, 1, 128, 48), (1, 33, 1, 128, 48), (2, 17, 5, 128, 64), (1, 40, 24, 128, 0),
                                         (3, 7, 2, 32, 8), (1, 9, 3, 256, 96),            # 16-byte vectors
