@@ -65,6 +65,9 @@ extern "C" {
  * 0 and total_k that no range names are measured too (a looser bound, still a bound); a NaN anywhere selects the
  * online-softmax kernel.  Not with score_bound, q_norm, q_tile_rows or MAGI_ATTN_BOUNDED_MFMA32. */
 #define MAGI_ATTN_AUTO_BOUND 16
+/* Rows of `out` that no q range covers become zeros (and their lse -inf) in the same launch, so that the caller need not
+ * clear the output first; without the flag they are left untouched.  1 to 64 ranges. */
+#define MAGI_ATTN_ZERO_UNCOVERED 32
 
 #define MAGI_RANGES_PAIRS 0 /* int32 [n, 2]: range i = [r[2i], r[2i+1])          */
 #define MAGI_RANGES_CU 1    /* int32 [n + 1] cumulative: range i = [r[i], r[i+1]) */
@@ -90,7 +93,7 @@ uint64_t magi_launch_count(void);
  *     out[q_range_i, h, :] = softmax(q[q_range_i, h] . k[k_range_i, h / (Hq/Hkv)]^T * scale) v[k_range_i, h / (Hq/Hkv)]
  *
  * with no mask inside a rectangle.  q ranges must be disjoint; rows of `out` that no range
- * covers are left untouched; a range with no keys writes zeros (and lse = -inf).
+ * covers are left untouched (zeros with MAGI_ATTN_ZERO_UNCOVERED); a range with no keys writes zeros (and lse = -inf).
  *
  * Stands in for
  *   flex_flash_attn_func(q, k, v, q_ranges, k_ranges, max_seqlen_q, max_seqlen_k, softmax_scale, ...)

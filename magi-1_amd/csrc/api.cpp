@@ -120,6 +120,9 @@ int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace) {
     return fail(MAGI_EINVAL, "magi_attn_fwd: negative size");
   if (p->ranges_mode != MAGI_RANGES_PAIRS && p->ranges_mode != MAGI_RANGES_CU)
     return fail(MAGI_EINVAL, "magi_attn_fwd: unknown ranges_mode %d", p->ranges_mode);
+  static_assert(MAGI_ATTN_ZERO_UNCOVERED == magi::ATTN_ZERO_GAPS, "flag bits of the header and the kernels");
+  if ((p->flags & MAGI_ATTN_ZERO_UNCOVERED) && (p->n_ranges < 1 || p->n_ranges > 64 || (p->total_q > 0 && p->max_seqlen_q == 0)))
+    return fail(MAGI_ENOSYS, "magi_attn_fwd: MAGI_ATTN_ZERO_UNCOVERED needs 1 to 64 ranges and max_seqlen_q > 0");
   if (p->n_ranges == 0 || p->total_q == 0 || p->max_seqlen_q == 0) return MAGI_OK;
   if (!p->q || !p->out || !p->q_ranges || !p->k_ranges) return fail(MAGI_EINVAL, "magi_attn_fwd: NULL q/out/ranges");
   const bool all_in_second = p->k2 && p->v2 && p->k_split == 0;  // an empty first segment may be NULL

@@ -84,6 +84,18 @@ struct WorkItem {
   bool valid;   // false: nothing to do (grid padding, or the q tile lies beyond the range)
 };
 
+// This workgroup's share (one of tiles_per_range) of the rows [r0, r1) of its head that no q range covers: zeros, lse =
+// -inf.  Done here, by the launch that writes the other rows, the caller needs no clearing pass over the whole output
+// (93600 x 24 heads of text cross attention: 596 -> 528 us; two passes per layer forward otherwise).
+__device__ __forceinline__ void zero_rows(const AttnKernArgs& a, const WorkItem& wi, int r0, int r1, int tile, int tid) {
+  const int per = (r1 - r0 + a.tiles_per_range - 1) / a.tiles_per_range;
+  const int b = min(r1, r0 + tile * per), e = min(r1, b + per);
+  for (int r = b + (tid >> 4); r < e; r += (int)(blockDim.x >> 4)) {
+    *(u32x4*)(a.out + (long)r * a.os_t + wi.o_head + 16 * (tid & 15)) = u32x4{0, 0, 0, 0};
+    if (a.lse && (tid & 15) == 0) a.lse[(long)wi.h * a.total_q + r] = -__builtin_inff();
+  }
+}
+
 // blockIdx -> (kv head, range slot, q tile, q head within the GQA group), laid out so that the workgroups an
 // XCD receives (blockIdx % 8) share a KV head and walk the same keys at about the same time (each XCD has its
 // own L2).  XCD x owns the heads x * (Hkv / 8) .. of the first 8 * (Hkv / 8); the Hkv % 8 heads that are left are
@@ -91,7 +103,7 @@ struct WorkItem {
 // range's tiles and the last XCDs ran dry (6 q heads / 1 kv head, four 720p chunks behind eight: 46.4 -> 45.5 ms).  Ranges are visited longest key span first (ties
 // by index), ranked here from the device-side list.
 // Every thread of the workgroup must call this (it contains a barrier); s_sel is LOCATE_WORDS ints of LDS.
-constexpr int LOCATE_WORDS = 4;
+constexpr int LOCATE_WORDS = 8;
 __device__ __forceinline__ WorkItem locate_work(const AttnKernArgs& a, int BM, int tid, int* s_sel) {
   WorkItem wi;
   wi.valid = false;
@@ -129,9 +141,53 @@ __device__ __forceinline__ WorkItem locate_work(const AttnKernArgs& a, int BM, i
   wi.o_head = a.out_group > 0 ? (long)(wi.h / a.out_group) * a.os_g + (long)(wi.h % a.out_group) * a.os_h
                               : (long)wi.h * a.os_h;
   int qs;
-  if (a.n_ranges <= MAX_SORT) {
-    // thread t ranks range t; the one whose rank is this workgroup's slot publishes the range itself (its q rows were
-    // requested together with the key ranges: one memory latency for everything)
+  if (a.n_ranges <= 64) {
+    // Lane t of the first wave holds range t: one memory latency for all of them, the ranking and the gaps between the
+    // q ranges come from registers.
+    if (tid < 64) {
+      const int t = tid;
+      const bool mine = t < a.n_ranges;
+      int s = 0, e = 0, q_s = a.total_q, q_e = a.total_q;
+      if (mine) {
+        load_range(a.k_ranges, a.ranges_mode, t, a.total_k, s, e);
+        load_range(a.q_ranges, a.ranges_mode, t, a.total_q, q_s, q_e);
+      }
+      // rows the launch computes of this range (max_seqlen_q may be smaller than the range)
+      const int q_end = min(q_e, q_s + a.tiles_per_range * BM);
+      const int my = e - s;
+      int rank = 0, gap_e = a.total_q, lead = a.total_q;
+      for (int j = 0; j < a.n_ranges; ++j) {
+        const int lj = __builtin_amdgcn_readlane(my, j), sj = __builtin_amdgcn_readlane(q_s, j), ej = __builtin_amdgcn_readlane(q_end, j);
+        rank += (lj > my) || (lj == my && j < t);
+        if (sj < ej) {
+          // the gap behind range t ends where the next range starts, and is none if another range covers its start
+          gap_e = min(gap_e, sj >= q_end ? sj : ej > q_end ? q_end : a.total_q);
+          lead = min(lead, sj);
+        }
+      }
+      if (mine && rank == (int)rslot) {
+        s_sel[0] = q_s;
+        s_sel[1] = q_e;
+        s_sel[2] = s;
+        s_sel[3] = e;
+        s_sel[4] = q_end;
+        s_sel[5] = gap_e;
+        s_sel[6] = rank == 0 ? lead : 0;  // rows ahead of the first range
+      }
+    }
+    __syncthreads();
+    qs = __builtin_amdgcn_readfirstlane(s_sel[0]);
+    wi.qe = __builtin_amdgcn_readfirstlane(s_sel[1]);
+    wi.ks = __builtin_amdgcn_readfirstlane(s_sel[2]);
+    wi.ke = __builtin_amdgcn_readfirstlane(s_sel[3]);
+    if (a.flags & ATTN_ZERO_GAPS) {
+      const int g0 = __builtin_amdgcn_readfirstlane(s_sel[4]), g1 = __builtin_amdgcn_readfirstlane(s_sel[5]);
+      const int lead = __builtin_amdgcn_readfirstlane(s_sel[6]);
+      if (g1 > g0) zero_rows(a, wi, g0, g1, (int)tile, tid);
+      if (lead > 0) zero_rows(a, wi, 0, lead, (int)tile, tid);
+    }
+  } else if (a.n_ranges <= MAX_SORT) {
+    // thread t ranks range t; the one whose rank is this workgroup's slot publishes the range itself
     if (tid < a.n_ranges) {
       int s, e, q_s, q_e;
       load_range(a.k_ranges, a.ranges_mode, tid, a.total_k, s, e);

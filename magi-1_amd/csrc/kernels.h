@@ -51,6 +51,8 @@ struct AttnKernArgs {
 constexpr int ATTN_BOUNDED = 1 << 8;
 // internal flag (with ATTN_BOUNDED): q is unscaled, the kernel multiplies it by scale_log2 while loading it
 constexpr int ATTN_SCALE_Q = 1 << 9;
+// MAGI_ATTN_ZERO_UNCOVERED of the public header
+constexpr int ATTN_ZERO_GAPS = 32;
 
 hipError_t launch_attn_fwd_bf16(const AttnKernArgs& a, hipStream_t stream);
 hipError_t launch_attn_fwd_bf16_w64(const AttnKernArgs& a, hipStream_t stream);

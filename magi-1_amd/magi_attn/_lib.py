@@ -23,6 +23,7 @@ MAGI_ATTN_Q_PRESCALED = 2
 MAGI_ATTN_FP8_FAST_EXP2 = 4
 MAGI_ATTN_BOUNDED_MFMA32 = 8
 MAGI_ATTN_AUTO_BOUND = 16
+MAGI_ATTN_ZERO_UNCOVERED = 32
 MAGI_SCORE_BOUND_MAX = 64.0
 
 

@@ -133,11 +133,16 @@ def range_attention(
         n = q_ranges.numel() - 1
         if q_ranges.numel() != k_ranges.numel():
             raise ValueError("cu_seqlens_q / cu_seqlens_k must have the same length")
+    # Rows that no range covers are zeros (lse -inf).  Where the ranges can cover the rows, the attention launch takes care
+    # of the few that are left; a clearing pass over the whole output only where it would have to write most of it.
+    by_kernel = out is None and 1 <= n <= 64 and max_seqlen_q > 0 and n * max_seqlen_q >= Tq
+    zero_gaps = by_kernel and (zero_init or return_lse)
     if out is None:
-        out = (torch.zeros if zero_init else torch.empty)((Tq, Hq, D), dtype=torch.bfloat16, device=q.device)
+        out = (torch.zeros if zero_init and not by_kernel else torch.empty)((Tq, Hq, D), dtype=torch.bfloat16, device=q.device)
     lse = None
     if return_lse:
-        lse = torch.full((Hq, Tq), float("-inf"), dtype=torch.float32, device=q.device)
+        lse = torch.empty((Hq, Tq), dtype=torch.float32, device=q.device) if zero_gaps else \
+            torch.full((Hq, Tq), float("-inf"), dtype=torch.float32, device=q.device)
     a = L.AttnArgs()
     a.q, a.k, a.v, a.k2, a.v2 = _ptr(q), _ptr(k), _ptr(v), _ptr(k2), _ptr(v2)
     a.out, a.lse = _ptr(out), _ptr(lse)
@@ -180,7 +185,7 @@ def range_attention(
     a.softmax_scale = 0.0 if softmax_scale is None else float(softmax_scale)
     a.flags = ((L.MAGI_ATTN_FP8_POW2_PRESCALED if fp8_pow2_prescaled else 0) | (L.MAGI_ATTN_Q_PRESCALED if q_prescaled else 0)
                | (L.MAGI_ATTN_FP8_FAST_EXP2 if fp8_fast_exp2 else 0) | (L.MAGI_ATTN_BOUNDED_MFMA32 if bounded_mfma32 else 0)
-               | (L.MAGI_ATTN_AUTO_BOUND if auto_bound else 0))
+               | (L.MAGI_ATTN_AUTO_BOUND if auto_bound else 0) | (L.MAGI_ATTN_ZERO_UNCOVERED if zero_gaps else 0))
     workspace = None
     if auto_bound and not static_scratch:
         workspace = torch.empty(4, dtype=torch.float32, device=q.device)  # (alive until the launches are enqueued)
