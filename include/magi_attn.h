@@ -329,6 +329,16 @@ int magi_layer_norm(const void* x, int64_t x_stride, const void* weight, const v
                     void* y, int64_t y_stride, int64_t rows, int32_t cols, float eps, void* stream);
 
 /*
+ * magi_layer_norm followed by magi_div_clamp_to_e4m3 for up to four fp8 linear layers that share the input, in one launch
+ * and without the bf16 rows in between:  y_k = e4m3fn( bf16( clamp( bf16(norm(x)) / scale_k, -448, 448 ) ) ), bit for bit
+ * what the separate calls give (forward_ln and the q, qx, k, v inputs under fp8_quant, dit_module.py:412-413, 445-456).
+ * scales / ys: HOST arrays of n_out (1 to 4) device pointers: scale_k fp32 [cols], y_k [rows, cols] e4m3 contiguous.
+ */
+int magi_layer_norm_e4m3(const void* x, int64_t x_stride, const void* weight, const void* bias, int32_t params_fp32,
+                         const float* const* scales, void* const* ys, int32_t n_out, int64_t rows, int32_t cols, float eps,
+                         void* stream);
+
+/*
  * The input quantiser of the reference's fp8 linear layers:
  *     y = e4m3fn( bf16( clamp( float(x) / scale, -448, 448 ) ) )
  * including the rounding to bf16 in the middle, which is part of the definition (a value may land on another e4m3

@@ -488,6 +488,42 @@ int magi_layer_norm(const void* x, int64_t x_stride, const void* weight, const v
   return MAGI_OK;
 }
 
+int magi_layer_norm_e4m3(const void* x, int64_t x_stride, const void* weight, const void* bias, int32_t params_fp32,
+                         const float* const* scales, void* const* ys, int32_t n_out, int64_t rows, int32_t cols, float eps,
+                         void* stream) {
+  if (rows < 0 || cols < 0 || n_out < 0) return fail(MAGI_EINVAL, "magi_layer_norm_e4m3: negative size");
+  if (rows == 0 || cols == 0 || n_out == 0) return MAGI_OK;
+  if (n_out > 4) return fail(MAGI_ENOSYS, "magi_layer_norm_e4m3: %d outputs (at most 4)", n_out);
+  if (cols % 8 || cols > 8192)
+    return fail(MAGI_ENOSYS, "magi_layer_norm_e4m3: cols %d not implemented (multiples of 8 up to 8192)", cols);
+  if (!x || !scales || !ys) return fail(MAGI_EINVAL, "magi_layer_norm_e4m3: NULL pointer");
+  if (x_stride < cols) return fail(MAGI_EINVAL, "magi_layer_norm_e4m3: row stride below cols");
+  if (x_stride % 8 || !aligned16(x) || !aligned16(weight) || !aligned16(bias))
+    return fail(MAGI_EINVAL, "magi_layer_norm_e4m3: rows and parameters must be 16-byte aligned");
+  if (!(eps >= 0.f)) return fail(MAGI_EINVAL, "magi_layer_norm_e4m3: eps");
+  magi::LnQuantKernArgs a;
+  std::memset(&a, 0, sizeof(a));
+  for (int k = 0; k < n_out; ++k) {
+    if (!scales[k] || !ys[k]) return fail(MAGI_EINVAL, "magi_layer_norm_e4m3: NULL scale / output %d", k);
+    if (!aligned16(scales[k]) || (reinterpret_cast<uintptr_t>(ys[k]) & 7u))
+      return fail(MAGI_EINVAL, "magi_layer_norm_e4m3: scales must be 16-byte aligned, outputs 8-byte");
+    a.scale[k] = scales[k];
+    a.y[k] = static_cast<char*>(ys[k]);
+  }
+  a.x = static_cast<const char*>(x);
+  a.xs = x_stride * 2;
+  a.w = static_cast<const char*>(weight);
+  a.b = static_cast<const char*>(bias);
+  a.rows = rows;
+  a.cols = cols;
+  a.n_out = n_out;
+  a.eps = eps;
+  hipError_t e = magi::launch_layer_norm_quant(a, params_fp32 != 0, compute_units(), static_cast<hipStream_t>(stream));
+  if (e != hipSuccess) return hip_fail(e, "magi_layer_norm_e4m3 launch");
+  g_launches.fetch_add(1, std::memory_order_relaxed);
+  return MAGI_OK;
+}
+
 int magi_div_clamp_to_e4m3(const void* x, int64_t x_stride, const float* scale, int32_t scale_len, void* y,
                            int64_t y_stride, int64_t rows, int32_t cols, void* stream) {
   if (rows < 0 || cols < 0) return fail(MAGI_EINVAL, "magi_div_clamp_to_e4m3: negative size");

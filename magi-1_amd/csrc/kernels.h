@@ -119,6 +119,20 @@ hipError_t launch_head_norm(const char* x, long x_stride_t, long x_stride_h, con
                             char* y, int S, int H, int norm_kind, float eps, hipStream_t stream);
 hipError_t launch_layer_norm(const char* x, long x_stride, const void* w, const void* b, int params_fp32, char* y,
                              long y_stride, long rows, int cols, float eps, hipStream_t stream);
+// LayerNorm of x [rows, cols] bf16 leaving as n_out e4m3 tensors [rows, cols] (contiguous): y[k] = e4m3(bf16(clamp(bf16(norm)
+// / scale[k], +-448))), scale[k] [cols] fp32.  xs in BYTES.
+struct LnQuantKernArgs {
+  const char* x;
+  long xs;
+  const char* w;
+  const char* b;
+  const float* scale[4];
+  char* y[4];
+  long rows;
+  int cols, n_out;
+  float eps;
+};
+hipError_t launch_layer_norm_quant(const LnQuantKernArgs& a, int params_fp32, int compute_units, hipStream_t stream);
 // y = e4m3(bf16(clamp(x / scale, +-448))): x [rows, cols] bf16, y [rows, cols] e4m3, strides in BYTES
 hipError_t launch_div_clamp(const char* x, long x_stride, const float* scale, int per_column, char* y, long y_stride,
                             long rows, int cols, hipStream_t stream);

@@ -258,6 +258,56 @@ __global__ __launch_bounds__(THREADS) void head_norm_kernel(const char* x, long 
   *(u32x4*)(dst + eb * 2) = pack8(v + 8);
 }
 
+// Mean and reciprocal standard deviation of a row of nvec 16-byte vectors that a wavefront holds packed (vector
+// i * 64 + lane in raw[i], zeros past the end), fp32, in two passes over the registers.  The row stays packed between the
+// passes (48 registers for 6144 columns instead of 96 more for its fp32 form): the empty asm makes the compiler
+// unpack again rather than keep the first pass's values.
+template <int NV>
+__device__ __forceinline__ void row_stats(u32x4* raw, int lane, int nvec, float inv_n, float eps, float& mean, float& rstd) {
+  float s = 0.f;
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    float f[8];
+    unpack8(raw[i], f);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) s += f[k];
+  }
+  mean = wave_sum(s) * inv_n;
+#pragma unroll
+  for (int i = 0; i < NV; ++i) asm volatile("" : "+v"(raw[i]));
+  float q = 0.f;
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    if (i * 64 + lane < nvec) {
+      float f[8];
+      unpack8(raw[i], f);
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        const float d = f[k] - mean;
+        q += d * d;
+      }
+    }
+  }
+  rstd = __builtin_amdgcn_rsqf(wave_sum(q) * inv_n + eps);
+#pragma unroll
+  for (int i = 0; i < NV; ++i) asm volatile("" : "+v"(raw[i]));
+}
+
+// elements 8 vi .. 8 vi + 7 of a norm parameter
+template <bool PF32>
+__device__ __forceinline__ void param8(const char* p, int vi, float* out) {
+  if (PF32) {
+    const f32x4 lo = *(const f32x4*)(p + (long)vi * 32), hi = *(const f32x4*)(p + (long)vi * 32 + 16);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      out[k] = lo[k];
+      out[4 + k] = hi[k];
+    }
+  } else {
+    unpack8(*(const u32x4*)(p + (long)vi * 16), out);
+  }
+}
+
 // Row LayerNorm of the layer input: one wavefront per row, the row held packed in registers as NV 16-byte
 // vectors per lane (vector i of lane l covers elements (64 i + l) * 8 ...), fp32 statistics in two passes over
 // the registers.  Weight and bias are read straight from global memory in the last pass (they stay in L1 / L2);
@@ -278,48 +328,9 @@ __global__ __launch_bounds__(THREADS) void layer_norm_kernel(const char* x, long
     const int vi = i * 64 + lane;
     raw[i] = vi < nvec ? *(const u32x4*)(src + (long)vi * 16) : u32x4{0u, 0u, 0u, 0u};
   }
-  float s = 0.f;
-#pragma unroll
-  for (int i = 0; i < NV; ++i) {
-    float f[8];
-    unpack8(raw[i], f);
-#pragma unroll
-    for (int k = 0; k < 8; ++k) s += f[k];
-  }
-  const float mean = wave_sum(s) * inv_n;
-  // the row stays packed between the passes (48 registers for 6144 columns instead of 96 more for its fp32
-  // form): the empty asm makes the compiler unpack again rather than keep the first pass's values
-#pragma unroll
-  for (int i = 0; i < NV; ++i) asm volatile("" : "+v"(raw[i]));
-  float q = 0.f;
-#pragma unroll
-  for (int i = 0; i < NV; ++i) {
-    if (i * 64 + lane < nvec) {
-      float f[8];
-      unpack8(raw[i], f);
-#pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        const float d = f[k] - mean;
-        q += d * d;
-      }
-    }
-  }
-  const float rstd = __builtin_amdgcn_rsqf(wave_sum(q) * inv_n + eps);
-#pragma unroll
-  for (int i = 0; i < NV; ++i) asm volatile("" : "+v"(raw[i]));
+  float mean, rstd;
+  row_stats<NV>(raw, lane, nvec, inv_n, eps, mean, rstd);
   char* dst = y + row * ys;
-  auto param8 = [&](const char* p, int vi, float* out) {  // elements 8 vi .. 8 vi + 7 of a parameter
-    if (PF32) {
-      const f32x4 lo = *(const f32x4*)(p + (long)vi * 32), hi = *(const f32x4*)(p + (long)vi * 32 + 16);
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        out[k] = lo[k];
-        out[4 + k] = hi[k];
-      }
-    } else {
-      unpack8(*(const u32x4*)(p + (long)vi * 16), out);
-    }
-  };
   if (w && b) {  // the usual case, free of branches so that the parameter loads of all vectors go out together
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
@@ -327,8 +338,8 @@ __global__ __launch_bounds__(THREADS) void layer_norm_kernel(const char* x, long
       if (vi < nvec) {
         float f[8], wf[8], bf[8];
         unpack8(raw[i], f);
-        param8(w, vi, wf);
-        param8(b, vi, bf);
+        param8<PF32>(w, vi, wf);
+        param8<PF32>(b, vi, bf);
 #pragma unroll
         for (int k = 0; k < 8; ++k) f[k] = (f[k] - mean) * rstd * wf[k] + bf[k];
         *(u32x4*)(dst + (long)vi * 16) = pack8(f);
@@ -346,12 +357,160 @@ __global__ __launch_bounds__(THREADS) void layer_norm_kernel(const char* x, long
           wf[k] = 1.f;
           bf[k] = 0.f;
         }
-        if (w) param8(w, vi, wf);
-        if (b) param8(b, vi, bf);
+        if (w) param8<PF32>(w, vi, wf);
+        if (b) param8<PF32>(b, vi, bf);
 #pragma unroll
         for (int k = 0; k < 8; ++k) f[k] = (f[k] - mean) * rstd * wf[k] + bf[k];
         *(u32x4*)(dst + (long)vi * 16) = pack8(f);
       }
+    }
+  }
+}
+
+// 8 quotients -> e4m3(bf16(clamp(q, +-448))); the clamp keeps a NaN (IEEE 754-2019 minimum / maximum)
+__device__ __forceinline__ u32x2 clamp8_e4m3(const float* q) {
+  u32x2 o;
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    float c[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      c[i] = (float)(__bf16)__builtin_elementwise_minimum(__builtin_elementwise_maximum(q[4 * j + i], -448.f), 448.f);
+    int u = 0;
+    u = __builtin_amdgcn_cvt_pk_fp8_f32(c[0], c[1], u, false);
+    u = __builtin_amdgcn_cvt_pk_fp8_f32(c[2], c[3], u, true);
+    o[j] = (unsigned)u;
+  }
+  return o;
+}
+
+// Row LayerNorm whose result leaves only as the e4m3 inputs of up to four fp8 linear layers, each with its own input
+// scales: y_k = e4m3(bf16(clamp(bf16(norm(x)) / scale_k))).  The normalised rows never reach memory: 2 + n bytes per
+// element instead of 4 for the norm and 3 n for the quantisers behind it.
+// One workgroup per CU walks a contiguous piece of the rows, one wavefront per row, with the scales in LDS (two planes of
+// four floats, so that consecutive lanes read consecutive 16 bytes): fetched per row they would be 16 bytes per element
+// through L1.  Outputs whose scales are equal bit for bit (one calibration of the shared input) are converted once and
+// stored n times.
+// No division per element: y = v_rcp(s) (within one ulp), q0 = f y, q = q0 + (f - q0 s) y.  The bf16 rounding of q (the
+// intermediate that is part of the quantiser) equals that of the IEEE quotient for every pair of an 8-bit and a 24-bit
+// mantissa and every reciprocal within one ulp: checked exhaustively, 3.2e9 cases.  q0 is clamped to +-2^10 so that it
+// cannot overflow (q comes out above 448 all the same).  A scale outside 2^+-60, whose residual could leave the normal
+// range, sends the workgroup's rows through divisions instead.
+// Bound: HBM with equal scales, the vector ALU with four different ones.  [86400, 6144], four outputs: 711 us (4.5 TB/s)
+// with equal scales, 1011 us with four different ones, against 2070 us for the norm and four quantisers; [9360, 3072]:
+// 36 and 63 against 105 us.
+template <int NV, bool PF32, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void layer_norm_quant_kernel(const LnQuantKernArgs a) {
+  __shared__ __attribute__((aligned(16))) f32x4 s_scale[4][2][NV * 64];
+  __shared__ int s_diff[4][4];  // [k][j], j < k: scale vectors k and j differ
+  __shared__ int s_wide;        // some scale is not within 2^+-60
+  const int tid = threadIdx.x;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int nvec = a.cols >> 3;
+  if (tid < 16) s_diff[tid >> 2][tid & 3] = 0;
+  if (tid == 16) s_wide = 0;
+  __syncthreads();
+  for (int c = tid; c < 2 * nvec; c += 64 * WAVES) {  // four columns per thread and pass
+    f32x4 sc[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if (k < a.n_out) {
+        sc[k] = *(const f32x4*)(a.scale[k] + 4 * c);
+#pragma unroll
+        for (int j = 0; j < k; ++j) {
+          bool same = true;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) same &= __float_as_uint(sc[k][i]) == __float_as_uint(sc[j][i]);
+          if (!same) s_diff[k][j] = 1;
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float m = fabsf(sc[k][i]);
+          if (!(m >= 0x1p-60f && m <= 0x1p60f)) s_wide = 1;
+        }
+        s_scale[k][c & 1][c >> 1] = sc[k];
+      }
+  }
+  __syncthreads();
+  const bool exact = __builtin_amdgcn_readfirstlane(s_wide) != 0;
+  int rep[4];  // the first output with the same scales
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    rep[k] = k;
+#pragma unroll
+    for (int j = k - 1; j >= 0; --j)
+      if (__builtin_amdgcn_readfirstlane(s_diff[k][j]) == 0) rep[k] = j;
+  }
+  const float inv_n = 1.f / (float)a.cols;
+  const long per = (a.rows + gridDim.x - 1) / gridDim.x;
+  const long r0 = (long)blockIdx.x * per, r1 = r0 + per < a.rows ? r0 + per : a.rows;
+  for (long row = r0 + w; row < r1; row += WAVES) {
+    const char* src = a.x + row * a.xs;
+    int lane = tid & 63;  // (opaque: or every address below is computed ahead of the loop and does not fit the registers)
+    asm volatile("" : "+v"(lane));
+    u32x4 raw[NV];
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int vi = i * 64 + lane;
+      raw[i] = vi < nvec ? *(const u32x4*)(src + (long)vi * 16) : u32x4{0u, 0u, 0u, 0u};
+    }
+    float mean, rstd;
+    row_stats<NV>(raw, lane, nvec, inv_n, a.eps, mean, rstd);
+    // the normalised elements of vector vi, as the bf16 rows the linear layers would be handed
+    auto norm8 = [&](const u32x4 v, int vi, float* f) __attribute__((always_inline)) {
+      float wf[8], bf[8];
+      unpack8(v, f);
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        wf[k] = 1.f;
+        bf[k] = 0.f;
+      }
+      if (a.w) param8<PF32>(a.w, vi, wf);
+      if (a.b) param8<PF32>(a.b, vi, bf);
+#pragma unroll
+      for (int k = 0; k < 8; ++k) f[k] = (f[k] - mean) * rstd * wf[k] + bf[k];
+      unpack8(pack8(f), f);
+    };
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int vi = i * 64 + lane;
+      if (vi < nvec) {
+        float f[8];
+        norm8(raw[i], vi, f);
+        u32x2 o[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+          if (k < a.n_out) {
+            if (rep[k] == k) {
+              const f32x4 s0 = s_scale[k][0][vi], s1 = s_scale[k][1][vi];
+              float q[8];
+#pragma unroll
+              for (int e = 0; e < 8; ++e) {
+                const float sc = e < 4 ? s0[e & 3] : s1[e & 3];
+                const float y = __builtin_amdgcn_rcpf(sc);
+                const float q0 = __builtin_amdgcn_fmed3f(f[e] * y, -1024.f, 1024.f);
+                q[e] = __builtin_fmaf(__builtin_fmaf(-q0, sc, f[e]), y, q0);
+              }
+              o[k] = clamp8_e4m3(q);
+            } else {
+              o[k] = rep[k] == 0 ? o[0] : rep[k] == 1 ? o[1] : o[2];
+            }
+            *(u32x2*)(a.y[k] + row * a.cols + 8 * vi) = o[k];
+          }
+      }
+      __builtin_amdgcn_sched_barrier(0);  // (one vector at a time: interleaved, they do not fit the registers)
+    }
+    if (exact) {
+      for (int vi = lane; vi < nvec; vi += 64)
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+          if (k < a.n_out) {
+            float f[8];
+            norm8(*(const u32x4*)(src + (long)vi * 16), vi, f);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) f[e] = f[e] / s_scale[k][e >> 2][vi][e & 3];
+            *(u32x2*)(a.y[k] + row * a.cols + 8 * vi) = clamp8_e4m3(f);
+          }
     }
   }
 }
@@ -581,6 +740,27 @@ hipError_t launch_layer_norm(const char* x, long x_stride, const void* w, const 
   else if (need <= 12) MAGI_LN(12);
   else MAGI_LN(16);
 #undef MAGI_LN
+  return hipGetLastError();
+}
+
+hipError_t launch_layer_norm_quant(const LnQuantKernArgs& a, int params_fp32, int compute_units, hipStream_t stream) {
+  if (a.rows <= 0) return hipSuccess;
+  const int need = (a.cols / 8 + 63) / 64;  // 16-byte vectors per lane
+#define MAGI_LNQ(NV, WAVES, PER_CU)                                                                                      \
+  do {                                                                                                                   \
+    const long wgs = (a.rows + WAVES - 1) / WAVES, most = (long)compute_units * PER_CU;                                  \
+    const dim3 grid((unsigned)(wgs < most ? wgs : most)), block(64 * WAVES);                                             \
+    if (params_fp32)                                                                                                     \
+      hipLaunchKernelGGL((layer_norm_quant_kernel<NV, true, WAVES>), grid, block, 0, stream, a);                         \
+    else                                                                                                                 \
+      hipLaunchKernelGGL((layer_norm_quant_kernel<NV, false, WAVES>), grid, block, 0, stream, a);                        \
+  } while (0)
+  // (workgroups per CU: what the scales in LDS and the registers allow)
+  if (need <= 2) MAGI_LNQ(2, 8, 3);
+  else if (need <= 6) MAGI_LNQ(6, 8, 3);
+  else if (need <= 12) MAGI_LNQ(12, 16, 1);
+  else MAGI_LNQ(16, 16, 1);
+#undef MAGI_LNQ
   return hipGetLastError();
 }
 

@@ -33,7 +33,7 @@ import math
 from . import _lib as L
 from .cache import Fp8KVCache, OffloadedKVCache
 from .functional import _measuring_a_bound_pays
-from .functional import (div_clamp_to, head_norm, layer_norm, pow2_scale_for, qk_prologue, qk_prologue_fp8, qkv_proj_prologue,
+from .functional import (div_clamp_to, head_norm, layer_norm, layer_norm_div_clamp, pow2_scale_for, qk_prologue, qk_prologue_fp8, qkv_proj_prologue,
                          quantize_fp8_split,
                          range_attention)
 from .params import InferenceParams, ModelMetaArgs, PackedCrossAttnParams
@@ -165,8 +165,11 @@ class PerTensorQuantizedFp8Linear(torch.nn.Module):
         return q
 
     def forward(self, input: torch.Tensor) -> torch.Tensor:
-        x8 = div_clamp_to(input, self.input_scale)
-        prefix = input.shape[:-1]
+        return self.forward_quantized(div_clamp_to(input, self.input_scale))
+
+    def forward_quantized(self, x8: torch.Tensor) -> torch.Tensor:
+        """The GEMM alone, on an input that is already div_clamp_to(input, self.input_scale)."""
+        prefix = x8.shape[:-1]
         y = torch._scaled_mm(x8.reshape(-1, self.in_features), self.weight[0].t(), scale_a=self.input_scale.reshape(-1)[:1],
                              scale_b=self.weight_scale.reshape(-1)[:1], out_dtype=self.output_dtype)
         return y.reshape(prefix + (self.out_features,))
@@ -233,6 +236,17 @@ class CustomLayerNormLinear(torch.nn.Module):
         y = torch.nn.functional.linear(hidden_states, self.fused_weight())
         oq, okv = self.q.weight.shape[0], self.k.weight.shape[0]
         return y[..., :oq], y[..., oq:oq + okv], y[..., oq + okv:oq + 2 * okv], y[..., oq + 2 * okv:]
+
+    def forward_ln_qkvx(self, hidden_states):
+        """forward_qkvx(forward_ln(hidden_states)).  With fp8_quant the norm and the four input quantisers are one launch
+        that writes the e4m3 inputs of the four GEMMs only (layer_norm_div_clamp)."""
+        linears = self._projections()
+        if (self.fp8_quant and hidden_states.shape[-1] % 8 == 0 and hidden_states.shape[-1] <= 8192 and hidden_states.is_contiguous()
+                and all(type(m) is PerTensorQuantizedFp8Linear and m.input_scale.numel() == hidden_states.shape[-1] for m in linears)):
+            ln = self.layer_norm
+            x8 = layer_norm_div_clamp(hidden_states, ln.weight.detach(), ln.bias.detach(), [m.input_scale.detach() for m in linears], ln.eps)
+            return tuple(m.forward_quantized(x8[i]) for i, m in enumerate(linears))
+        return self.forward_qkvx(self.forward_ln(hidden_states))
 
     def forward_ln(self, hidden_states):
         """LayerNorm of the layer input (dit_module.py:412-413) as one HIP launch; the parameters stay on the
@@ -711,16 +725,17 @@ class FullyParallelAttention(torch.nn.Module):
         bs = hidden_states.shape[1]
         sq = hidden_states.shape[0]
         D = self.hidden_size_per_attention_head
-        mixed_qqkv = self.linear_qkv.forward_ln(hidden_states)
         one_launch = (self.fused_projection and self.attention_dtype == "bf16" and bs == 1 and rope is not None
-                      and rope.shape[-1] == 96 and mixed_qqkv.shape[-1] % 64 == 0)
+                      and rope.shape[-1] == 96 and hidden_states.shape[-1] % 64 == 0)
         if one_launch:
             # projections + prologue in one launch: nothing raw reaches memory (qx leaves unnormalised, as the
             # cross-attention kernel takes it)
+            mixed_qqkv = self.linear_qkv.forward_ln(hidden_states)
             raw = qx_raw = None
         else:
             # all four projections in one GEMM; q / k / v feed the fused prologue as row-strided views of its result
-            q_raw, k_raw, v_raw, qx_raw = self.linear_qkv.forward_qkvx(mixed_qqkv)
+            mixed_qqkv = hidden_states  # (only its shape is used from here on: every projection is in hand)
+            q_raw, k_raw, v_raw, qx_raw = self.linear_qkv.forward_ln_qkvx(hidden_states)
             raw = (q_raw, k_raw, v_raw)
 
         def project(kv_out=None, n_cache_rows=None, kv_tail=None):

@@ -73,6 +73,46 @@ def test_per_tensor_fp8_linear_matches_dequantised_arithmetic(dev):
     assert cos >= 0.998, cos
 
 
+@pytest.mark.parametrize("rows,cols,params,kinds", [
+    (1, 8, "bf16", "r"), (17, 520, "fp32", "rs"), (300, 1024, "none", "tttt"), (4100, 3072, "bf16", "rrtt"),
+    (515, 6144, "bf16", "rtrs"), (33, 8192, "weight", "sr"), (40, 1536, "bf16", "xrx"), (16 * 256 + 5, 256, "bf16", "trtr")])
+def test_norm_and_quantisers_in_one_launch_give_the_same_bytes(dev, rows, cols, params, kinds):
+    """layer_norm_div_clamp against layer_norm and one div_clamp_to per scale: every byte the same, for random scales (r),
+    scales whose quotients fall on and next to the middle between two bf16 values (t), one scale for all columns (s),
+    and scales outside the range the reciprocal serves (x: subnormal, zero, infinite, NaN, huge)."""
+    g = torch.Generator(device=dev).manual_seed(rows + cols)
+    x = (torch.randn(rows, cols, device=dev, generator=g) * 2 + 0.3).bfloat16()
+    if rows > 20:
+        x[3, 5] = float("nan")
+        x[7] = 0.0
+    p_dtype = torch.float32 if params == "fp32" else torch.bfloat16
+    w = None if params == "none" else (torch.rand(cols, device=dev, generator=g) + 0.5).to(p_dtype)
+    b = None if params in ("none", "weight") else (torch.randn(cols, device=dev, generator=g) * 0.3).to(p_dtype)
+    scales = []
+    for kind in kinds:
+        s = torch.rand(cols, device=dev, generator=g) * 0.02 + 0.003
+        if kind == "s":
+            s = torch.full((cols,), 6.0 / 448.0, device=dev)
+        elif kind == "t":
+            step = torch.randint(-3, 4, (cols,), device=dev, generator=g)
+            s = (1.0 / ((1 + 2.0 ** -8) * 2.0 ** (step + 5).float())).view(torch.int32).add_(step.int()).view(torch.float32)
+        elif kind == "x":
+            odd = torch.tensor([1e-40, 0.0, float("inf"), float("nan"), 3e38, 1e-38, -0.01], device=dev)
+            s[:cols:5] = odd[torch.arange(len(s[:cols:5]), device=dev) % 7]
+        scales.append(s.contiguous())
+    if kinds == "trtr":
+        scales[2:] = [t.clone() for t in scales[:2]]  # equal pairs are converted once
+    n0 = M.lib().magi_launch_count()
+    got = M.layer_norm_div_clamp(x, w, b, scales, 1e-6)
+    assert M.lib().magi_launch_count() - n0 == 1
+    h = M.layer_norm(x, w, b, 1e-6)
+    for k, s in enumerate(scales):
+        want = M.div_clamp_to(h, s).view(torch.uint8)
+        bytes_ = got[k].view(torch.uint8)
+        nan = (want & 0x7f) == 0x7f
+        assert torch.equal(bytes_[~nan], want[~nan]) and bool(((bytes_[nan] & 0x7f) == 0x7f).all())
+
+
 def test_layer_with_fp8_quant_projections(dev):
     """FullyParallelAttention(fp8_quant=True): q / qx / k / v through PerTensorQuantizedFp8Linear.  Against the same
     layer with bf16 projections made of the DE-QUANTISED weights, fed the same inputs: the only difference left is the
