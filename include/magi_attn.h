@@ -204,6 +204,14 @@ typedef struct magi_attn_args {
   /* MAGI_ATTN_AUTO_BOUND: 16 bytes of DEVICE memory, 16-byte aligned, that the call may overwrite (the measured
    * bound; calls that overlap on the device need a workspace each).  NULL otherwise. */
   float* workspace;
+  /* Version 104 (a struct that ends here, struct_size = offsetof(magi_attn_args, q_batch_rows), is accepted too: the fields
+   * below are then 0).
+   * q_batch_rows: 0 = off.  > 0: the q rows are a batch of blocks of this many rows that are not laid out one behind the
+   * other: row r is row r % q_batch_rows of block r / q_batch_rows, at that row times *_stride_t plus the block times
+   * *_stride_b, in q and in out (the lse stays [Hq, total_q]).  The cross attention of a batch whose activations are
+   * [position, batch, ...] reads and writes them in place that way.  bf16 with a score_bound in force, 256-row tiles. */
+  int32_t q_batch_rows;
+  int64_t q_stride_b, o_stride_b;
 } magi_attn_args;
 
 int magi_attn_fwd(const magi_attn_args* args, void* stream);

@@ -3,6 +3,7 @@
 #include <atomic>
 #include <cmath>
 #include <cstdarg>
+#include <cstddef>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -80,11 +81,21 @@ int static_scratch(void** out) {
 
 int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace);
 
+// the caller's struct as this version lays it out: itself, or `full` filled from the shorter one of version 103
+const magi_attn_args* current_layout(const magi_attn_args* p, magi_attn_args* full) {
+  constexpr size_t v103 = offsetof(magi_attn_args, q_batch_rows);
+  if (p->struct_size != v103) return p;
+  std::memset(full, 0, sizeof(*full));
+  std::memcpy(full, p, v103);
+  full->struct_size = sizeof(*full);
+  return full;
+}
+
 }  // namespace
 
 extern "C" {
 
-int magi_version(void) { return 103; }
+int magi_version(void) { return 104; }
 
 uint64_t magi_launch_count(void) { return g_launches.load(std::memory_order_relaxed); }
 
@@ -92,12 +103,16 @@ const char* magi_last_error(void) { return g_err; }
 
 int magi_attn_fwd(const magi_attn_args* p, void* stream) {
   if (!p) return fail(MAGI_EINVAL, "magi_attn_fwd: args is NULL");
+  magi_attn_args full;
+  p = current_layout(p, &full);
   MAGI_CHECK_LAYOUT("magi_attn_fwd", p);
   return attn_fwd_impl(p, stream, p->workspace);
 }
 
 int magi_attn_fwd_static_scratch(const magi_attn_args* p, void* stream) {
   if (!p) return fail(MAGI_EINVAL, "magi_attn_fwd_static_scratch: args is NULL");
+  magi_attn_args full;
+  p = current_layout(p, &full);
   MAGI_CHECK_LAYOUT("magi_attn_fwd_static_scratch", p);
   static_assert(4 * sizeof(float) <= SCRATCH_BYTES, "the measured score bound needs four words");
   void* ws = nullptr;
@@ -240,6 +255,17 @@ int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace) {
     return fail(MAGI_EINVAL, "magi_attn_fwd: q_tile_rows %d (fp8: 128)", p->q_tile_rows);
   const bool promised = p->dtype == MAGI_DTYPE_BF16 && p->score_bound > 0.f && p->score_bound <= MAGI_SCORE_BOUND_MAX;
   const bool mfma32 = (p->flags & MAGI_ATTN_BOUNDED_MFMA32) != 0;
+  if (p->q_batch_rows != 0) {
+    if (p->q_batch_rows < 0 || p->total_q % p->q_batch_rows)
+      return fail(MAGI_EINVAL, "magi_attn_fwd: q_batch_rows %d must divide total_q=%d", p->q_batch_rows, p->total_q);
+    if (!promised || mfma32 || (p->q_tile_rows != 0 && p->q_tile_rows != 256))
+      return fail(MAGI_ENOSYS, "magi_attn_fwd: q_batch_rows is implemented for bf16 with a score_bound in force and 256-row tiles");
+    if (p->q_stride_b % 8 || p->o_stride_b % 8)
+      return fail(MAGI_EINVAL, "magi_attn_fwd: batch strides must keep rows 16-byte aligned");
+    a.batch_rows = p->q_batch_rows;
+    a.qs_b = p->q_stride_b * 2;
+    a.os_b = p->o_stride_b * 2;
+  }
   if (mfma32 && !(promised && (p->flags & MAGI_ATTN_Q_PRESCALED)))
     return fail(MAGI_EINVAL, "magi_attn_fwd: MAGI_ATTN_BOUNDED_MFMA32 goes with bf16, MAGI_ATTN_Q_PRESCALED and a score_bound in force");
   a.Hq = p->Hq;

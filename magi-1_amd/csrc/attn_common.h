@@ -84,6 +84,13 @@ struct WorkItem {
   bool valid;   // false: nothing to do (grid padding, or the q tile lies beyond the range)
 };
 
+// byte offset of q row r (stride s_t between rows, s_b between blocks of batch_rows of them)
+__device__ __forceinline__ long row_offset(const AttnKernArgs& a, int r, long s_t, long s_b) {
+  if (a.batch_rows == 0) return (long)r * s_t;
+  const int b = (int)((unsigned)r / (unsigned)a.batch_rows);
+  return (long)(r - b * a.batch_rows) * s_t + (long)b * s_b;
+}
+
 // This workgroup's share (one of tiles_per_range) of the rows [r0, r1) of its head that no q range covers: zeros, lse =
 // -inf.  Done here, by the launch that writes the other rows, the caller needs no clearing pass over the whole output
 // (93600 x 24 heads of text cross attention: 596 -> 528 us; two passes per layer forward otherwise).
@@ -91,7 +98,7 @@ __device__ __forceinline__ void zero_rows(const AttnKernArgs& a, const WorkItem&
   const int per = (r1 - r0 + a.tiles_per_range - 1) / a.tiles_per_range;
   const int b = min(r1, r0 + tile * per), e = min(r1, b + per);
   for (int r = b + (tid >> 4); r < e; r += (int)(blockDim.x >> 4)) {
-    *(u32x4*)(a.out + (long)r * a.os_t + wi.o_head + 16 * (tid & 15)) = u32x4{0, 0, 0, 0};
+    *(u32x4*)(a.out + row_offset(a, r, a.os_t, a.os_b) + wi.o_head + 16 * (tid & 15)) = u32x4{0, 0, 0, 0};
     if (a.lse && (tid & 15) == 0) a.lse[(long)wi.h * a.total_q + r] = -__builtin_inff();
   }
 }
@@ -224,7 +231,7 @@ __device__ __forceinline__ WorkItem locate_work(const AttnKernArgs& a, int BM, i
 
 // A q row whose range has no keys: zeros, lse = -inf.  Lane (row, g) writes half g of the 256-byte row.
 __device__ __forceinline__ void store_empty_row(const AttnKernArgs& a, const WorkItem& wi, int q_row, int g) {
-  char* op = a.out + (long)q_row * a.os_t + wi.o_head + g * 128;
+  char* op = a.out + row_offset(a, q_row, a.os_t, a.os_b) + wi.o_head + g * 128;
 #pragma unroll
   for (int c = 0; c < 8; ++c) *(u32x4*)(op + c * 16) = u32x4{0, 0, 0, 0};
   if (a.lse && g == 0) a.lse[(long)wi.h * a.total_q + q_row] = -__builtin_inff();

@@ -162,7 +162,7 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_bf16_x16_kernel(const AttnKer
 #pragma unroll
   for (int qb = 0; qb < 4; ++qb) {
     const int qr = min(row0 + 16 * qb + n, qe - 1);
-    const char* qp = a.q + (long)qr * a.qs_t + (long)wi.h * a.qs_h + g * 16;
+    const char* qp = a.q + row_offset(a, qr, a.qs_t, a.qs_b) + (long)wi.h * a.qs_h + g * 16;
 #pragma unroll
     for (int kk = 0; kk < 4; ++kk) qf[qb][kk] = *(const bf16x8*)(qp + kk * 64);
   }
@@ -416,7 +416,7 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_bf16_x16_kernel(const AttnKer
     const int r = 4 * it + ge;
     const u32x4 v = *LDS_PTR(const u32x4, stage + r * ROW_BYTES + ((ne ^ (r & 15)) << 4));
     const int q_row = row0 + r;
-    if (q_row < qe) *(u32x4*)(a.out + (long)q_row * a.os_t + wi.o_head + 16 * ne) = v;
+    if (q_row < qe) *(u32x4*)(a.out + row_offset(a, q_row, a.os_t, a.os_b) + wi.o_head + 16 * ne) = v;
   }
 }
 

@@ -27,6 +27,8 @@ struct AttnKernArgs {
   long k2_scale_delta, v2_scale_delta;
   long os_g;     // byte stride between output head groups (out_group > 0)
   int out_group; // heads per output group, 0 = heads addressed by os_h alone
+  long qs_b, os_b;  // strides between blocks of batch_rows q rows (batch_rows > 0)
+  int batch_rows;   // 0: row r at r * qs_t / r * os_t
   int total_q, total_k, k_split;
   int n_ranges, ranges_mode, tiles_per_range;
   int block_m;  // q rows per workgroup (the launchers map it to an instantiation)

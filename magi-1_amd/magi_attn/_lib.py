@@ -62,6 +62,7 @@ class AttnArgs(_SizedStructure):
         ("q_norm_gamma", C.c_void_p), ("q_norm_beta", C.c_void_p), ("q_norm_eps", C.c_float), ("q_norm_kind", C.c_int32),
         ("k2_scale", C.c_void_p), ("v2_scale", C.c_void_p),
         ("workspace", C.c_void_p),
+        ("q_batch_rows", C.c_int32), ("q_stride_b", C.c_int64), ("o_stride_b", C.c_int64),
     ]
 
 
@@ -106,7 +107,7 @@ class QuantizeArgs(_SizedStructure):
     ]
 
 
-ABI_VERSION = 103  # magi_version() of the library these mirrors were written for
+ABI_VERSION = 104  # magi_version() of the library these mirrors were written for
 
 EXPORTS = ("magi_version", "magi_last_error", "magi_launch_count", "magi_attn_fwd", "magi_attn_fwd_static_scratch",
            "magi_qk_prologue", "magi_head_norm",

@@ -103,13 +103,17 @@ def range_attention(
     picks the bounded-score kernel on the device when their product allows it, MAGI_ATTN_AUTO_BOUND.  Its 16-byte
     workspace is a fresh tensor, or with static_scratch the library's own device array (magi_attn_fwd_static_scratch:
     no allocation at all when `out` is given and return_lse is False; such calls must not overlap on one GPU).
+    q may be [batch, rows, Hq, D] with any batch stride (batch of activations laid out [position, batch, ...]): its rows
+    count as batch * rows tokens for the ranges, out is (or comes back as) a tensor of q's shape, by default
+    [rows, batch, Hq, D] transposed.  Needs a score_bound in force.
     q_norm: (gamma, beta or None, eps[, norm_kind]): q is the raw projection, normalised per (token, head) row inside
     the kernel (fp32, zero-centred gamma) and scaled by softmax_scale * log2(e); needs score_bound.
     """
-    _check_thd(q, "q")
+    batched = q.dim() == 4
+    _check_thd(q[0] if batched else q, "q")
     _check_thd(k, "k")
     _check_thd(v, "v")
-    Tq, Hq, D = q.shape
+    Tq, Hq, D = (q.shape[0] * q.shape[1],) + tuple(q.shape[2:]) if batched else q.shape
     Hkv = k.shape[1]
     total_k = k.shape[0] if k2 is None else int(k_split) + k2.shape[0]
     if k2 is not None:
@@ -138,7 +142,9 @@ def range_attention(
     by_kernel = out is None and 1 <= n <= 64 and max_seqlen_q > 0 and n * max_seqlen_q >= Tq
     zero_gaps = by_kernel and (zero_init or return_lse)
     if out is None:
-        out = (torch.zeros if zero_init and not by_kernel else torch.empty)((Tq, Hq, D), dtype=torch.bfloat16, device=q.device)
+        new = torch.zeros if zero_init and not by_kernel else torch.empty
+        out = new((q.shape[1], q.shape[0], Hq, D), dtype=torch.bfloat16, device=q.device).transpose(0, 1) if batched else \
+            new((Tq, Hq, D), dtype=torch.bfloat16, device=q.device)
     lse = None
     if return_lse:
         lse = torch.empty((Hq, Tq), dtype=torch.float32, device=q.device) if zero_gaps else \
@@ -166,10 +172,15 @@ def range_attention(
         for name, t, rows, heads in need:
             if t is not None and (t.dim() != 2 or t.shape[0] < rows or t.shape[1] != heads):
                 raise ValueError(f"{name} must be [>= {rows} chunks, {heads} heads], got {tuple(t.shape)}")
-    a.q_stride_t, a.q_stride_h = q.stride(0), q.stride(1)
+    a.q_stride_t, a.q_stride_h = q.stride(-3), q.stride(-2)
     a.k_stride_t, a.k_stride_h = k.stride(0), k.stride(1)
     a.v_stride_t, a.v_stride_h = v.stride(0), v.stride(1)
-    if out.dim() == 4:  # [Tq, groups, heads per group, D]: two-level head addressing
+    if batched:
+        if out.shape != q.shape or out.stride(3) != 1:
+            raise ValueError("out must have the shape of a batched q, with contiguous rows")
+        a.o_stride_t, a.o_stride_h = out.stride(1), out.stride(2)
+        a.q_batch_rows, a.q_stride_b, a.o_stride_b = q.shape[1], q.stride(0), out.stride(0)
+    elif out.dim() == 4:  # [Tq, groups, heads per group, D]: two-level head addressing
         if out.shape[0] != Tq or out.shape[1] * out.shape[2] != Hq or out.shape[3] != D or out.stride(3) != 1:
             raise ValueError("a 4-D out must be [Tq, groups, Hq / groups, D] with contiguous rows")
         a.o_stride_t, a.o_stride_g, a.o_stride_h, a.out_group_heads = out.stride(0), out.stride(1), out.stride(2), out.shape[2]

@@ -664,16 +664,20 @@ class FullyParallelAttention(torch.nn.Module):
 
     def _cross_attention_fused(self, qx_raw: torch.Tensor, key_value_states: torch.Tensor,
                                cross_attn_params: PackedCrossAttnParams, out: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
-        """Batch-1 cross attention on the RAW qx projection [sq, 1, Hq*D]: the attention kernel applies
-        q_layernorm_xattn while it loads q (no normalised copy of q in memory) and, the scores of normed q and k
-        being bounded, runs without a running maximum.  Returns None when that path does not apply (then the
-        caller takes get_xqkv + cross_attention); else the [sq, Hq, D]-shaped result (`out` if given)."""
+        """Cross attention on the RAW qx projection [sq, b, Hq*D]: the attention kernel applies q_layernorm_xattn while it
+        loads q (no normalised copy of q in memory) and, the scores of normed q and k being bounded, runs without a
+        running maximum; at batch > 1 it reads and writes the [position, batch] rows where they are.  Returns None
+        when that path does not apply (then the caller takes get_xqkv + cross_attention); else the result, [sq, b, Hq, D]
+        contiguous (or `out`, batch 1 only)."""
         bound = self.score_bounds()[1]
-        if qx_raw.shape[1] != 1 or not (0.0 < bound <= L.MAGI_SCORE_BOUND_MAX):
+        if not (0.0 < bound <= L.MAGI_SCORE_BOUND_MAX):
             return None
         D = self.hidden_size_per_attention_head
-        sq = qx_raw.shape[0]
-        q = qx_raw.reshape(sq, -1, D)  # row-strided view of the projection
+        sq, b = qx_raw.shape[0], qx_raw.shape[1]
+        if b == 1:
+            q = qx_raw.reshape(sq, -1, D)  # row-strided view of the projection
+        else:
+            q = qx_raw.view(sq, b, -1, D).transpose(0, 1)
         kv = torch.nn.functional.linear(key_value_states, self.linear_kv_xattn.weight)
         kv = kv.view(key_value_states.shape[0], -1, 2 * D)
         gk, bk = self.k_layernorm_xattn.gamma_beta_fp32()
@@ -683,7 +687,7 @@ class FullyParallelAttention(torch.nn.Module):
                                cross_attn_params.max_seqlen_q, cross_attn_params.max_seqlen_kv,
                                ranges_mode=L.MAGI_RANGES_CU, out=out, return_lse=False, zero_init=True,
                                score_bound=bound, q_norm=(gq, bq, self.eps))
-        return o
+        return o if b == 1 else o.transpose(0, 1)
 
     # ------------------------------------------------------------------ forward
     def forward(self, hidden_states: torch.Tensor, key_value_states: torch.Tensor,
@@ -720,7 +724,7 @@ class FullyParallelAttention(torch.nn.Module):
             "core": "fp8" if self.attention_dtype == "fp8" else
             ("measured bound: bounded-score or online softmax, chosen on the device" if measured else bounded(bound_core)),
             "core_score_bound": bound_core,
-            "cross": bounded(self.score_bounds()[1] if hidden_states.shape[1] == 1 else float("inf")),
+            "cross": bounded(self.score_bounds()[1]),
             "cross_score_bound": self.score_bounds()[1]}
         bs = hidden_states.shape[1]
         sq = hidden_states.shape[0]
@@ -823,7 +827,7 @@ class FullyParallelAttention(torch.nn.Module):
         core_attn_out = core.view(sq, bs, -1)
         xo = self._cross_attention_fused(qx_raw, key_value_states, meta_args.cross_attn_params, None)
         if xo is not None:
-            xattn_out = xo.view(sq, 1, -1)
+            xattn_out = xo.reshape(sq, bs, -1)
         else:
             xattn_out = self.cross_attention(mixed_qqkv, key_value_states, meta_args.cross_attn_params, get_xqkv)
         if proj_layout:

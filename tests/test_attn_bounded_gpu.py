@@ -291,3 +291,28 @@ def test_query_norm_inside_the_kernel(dev, kind):
     with pytest.raises(M.MagiError):  # needs the bound
         M.range_attention(q_raw.to(dev), k.to(dev), v.to(dev), tq, tk, Lq, 800, ranges_mode=M.MAGI_RANGES_CU,
                           q_norm=(gamma.to(dev), beta.to(dev), eps, code))
+
+
+@pytest.mark.parametrize("B,rows,cu", [(1, 100, [0, 100]), (3, 70, [0, 70, 140, 210]), (2, 300, [0, 300, 600]),
+                                       (5, 33, [0, 40, 40, 165]), (7, 1, [0, 7]), (4, 64, [20, 130, 256])])
+def test_batch_of_position_major_rows_read_and_written_in_place(dev, B, rows, cu):
+    """q [batch, rows, H, D] as a view of [rows, batch, ...] activations (q_batch_rows): the same bits as the call on a
+    batch-major copy, with ranges that end inside a tile, cross block boundaries or leave rows uncovered; raw q with the
+    norm applied by the kernel, and unscaled q with the lse."""
+    Hq, Hkv, D, Tk = 4, 2, 128, 150
+    g = torch.Generator(device=dev).manual_seed(B + rows)
+    act = torch.randn(rows, B, Hq * D + 64, device=dev, generator=g).bfloat16()[..., :Hq * D]  # a slice of a projection
+    q4 = act.view(rows, B, Hq, D).transpose(0, 1)
+    q3 = q4.reshape(B * rows, Hq, D)
+    k, v = (torch.randn(Tk, Hkv, D, device=dev, generator=g).bfloat16() for _ in range(2))
+    cu_q = torch.tensor(cu, dtype=torch.int32, device=dev)
+    cu_k = torch.tensor(np.linspace(0, Tk, len(cu)).astype(int), dtype=torch.int32, device=dev)
+    gam = torch.randn(D, device=dev, generator=g) * 0.1
+    for kw in (dict(score_bound=30.0), dict(score_bound=60.0, q_norm=(gam, gam, 1e-6))):
+        args = (cu_q, cu_k, max(np.diff(cu)))
+        want, lse_w = M.range_attention(q3, k, v, *args, ranges_mode=M.MAGI_RANGES_CU, **kw)
+        got, lse = M.range_attention(q4, k, v, *args, ranges_mode=M.MAGI_RANGES_CU, **kw)
+        assert got.shape == q4.shape and got.transpose(0, 1).is_contiguous()
+        assert torch.equal(got.reshape(want.shape), want) and torch.equal(lse, lse_w)
+    with pytest.raises(M.MagiError):  # no bound in force
+        M.range_attention(q4, k, v, *args, ranges_mode=M.MAGI_RANGES_CU)
