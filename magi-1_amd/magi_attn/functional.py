@@ -23,12 +23,26 @@ import torch
 from . import _lib as L
 
 
-def _stream() -> C.c_void_p:
-    return C.c_void_p(torch.cuda.current_stream().cuda_stream)
+def _launch(dev: torch.device, fn, *args) -> None:
+    """fn(*args, stream) with `dev` current, on its current stream; raises on a negative code."""
+    index = dev.index
+    if torch._C._cuda_getDevice() == index:
+        code = fn(*args, torch._C._cuda_getCurrentRawStream(index))
+    else:
+        with torch.cuda.device(dev):
+            code = fn(*args, torch._C._cuda_getCurrentRawStream(index))
+    if code != 0:
+        L.check(code)
 
 
-def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
-    return None if t is None else t.data_ptr()
+def _launch_packed(dev: torch.device, name: str, args: type, *fields) -> None:
+    """The same for an entry point that takes an argument struct: its fields behind struct_size, in order."""
+    call = L.packed(name, args)
+    _launch(dev, call.fn, call.pack(call.size, *fields))
+
+
+def _ptr(t: Optional[torch.Tensor]) -> int:
+    return 0 if t is None else t.data_ptr()
 
 
 def _check_thd(t: torch.Tensor, name: str) -> None:
@@ -149,16 +163,11 @@ def range_attention(
     if return_lse:
         lse = torch.empty((Hq, Tq), dtype=torch.float32, device=q.device) if zero_gaps else \
             torch.full((Hq, Tq), float("-inf"), dtype=torch.float32, device=q.device)
-    a = L.AttnArgs()
-    a.q, a.k, a.v, a.k2, a.v2 = _ptr(q), _ptr(k), _ptr(v), _ptr(k2), _ptr(v2)
-    a.out, a.lse = _ptr(out), _ptr(lse)
-    a.q_ranges, a.k_ranges = _ptr(q_ranges), _ptr(k_ranges)
-    a.q_scale, a.k_scale, a.v_scale = _ptr(q_scale), _ptr(k_scale), _ptr(v_scale)
-    for name, t in (("q_scale", q_scale), ("k_scale", k_scale), ("v_scale", v_scale), ("k2_scale", k2_scale),
-                    ("v2_scale", v2_scale)):
-        if t is not None and (t.dtype != torch.float32 or not t.is_contiguous() or t.device != q.device):
-            raise ValueError(f"{name} must be a contiguous fp32 tensor on q's device")
-    a.k2_scale, a.v2_scale = _ptr(k2_scale), _ptr(v2_scale)
+    if q_scale is not None or k_scale is not None or v_scale is not None or k2_scale is not None or v2_scale is not None:
+        for name, t in (("q_scale", q_scale), ("k_scale", k_scale), ("v_scale", v_scale), ("k2_scale", k2_scale),
+                        ("v2_scale", v2_scale)):
+            if t is not None and (t.dtype != torch.float32 or not t.is_contiguous() or t.device != q.device):
+                raise ValueError(f"{name} must be a contiguous fp32 tensor on q's device")
     if q.dtype == torch.float8_e4m3fn and scale_chunk_tokens > 0:
         # the kernel indexes the tables by token / scale_chunk_tokens without a bound of its own
         C_ = int(scale_chunk_tokens)
@@ -172,48 +181,40 @@ def range_attention(
         for name, t, rows, heads in need:
             if t is not None and (t.dim() != 2 or t.shape[0] < rows or t.shape[1] != heads):
                 raise ValueError(f"{name} must be [>= {rows} chunks, {heads} heads], got {tuple(t.shape)}")
-    a.q_stride_t, a.q_stride_h = q.stride(-3), q.stride(-2)
-    a.k_stride_t, a.k_stride_h = k.stride(0), k.stride(1)
-    a.v_stride_t, a.v_stride_h = v.stride(0), v.stride(1)
+    q_stride, o_stride = q.stride(), out.stride()
+    group_heads = o_stride_g = batch_rows = q_stride_b = o_stride_b = 0
     if batched:
-        if out.shape != q.shape or out.stride(3) != 1:
+        if out.shape != q.shape or o_stride[3] != 1:
             raise ValueError("out must have the shape of a batched q, with contiguous rows")
-        a.o_stride_t, a.o_stride_h = out.stride(1), out.stride(2)
-        a.q_batch_rows, a.q_stride_b, a.o_stride_b = q.shape[1], q.stride(0), out.stride(0)
-    elif out.dim() == 4:  # [Tq, groups, heads per group, D]: two-level head addressing
-        if out.shape[0] != Tq or out.shape[1] * out.shape[2] != Hq or out.shape[3] != D or out.stride(3) != 1:
+        batch_rows, q_stride_b, o_stride_b = q.shape[1], q_stride[0], o_stride[0]
+    elif len(o_stride) == 4:  # [Tq, groups, heads per group, D]: two-level head addressing
+        if out.shape[0] != Tq or out.shape[1] * out.shape[2] != Hq or out.shape[3] != D or o_stride[3] != 1:
             raise ValueError("a 4-D out must be [Tq, groups, Hq / groups, D] with contiguous rows")
-        a.o_stride_t, a.o_stride_g, a.o_stride_h, a.out_group_heads = out.stride(0), out.stride(1), out.stride(2), out.shape[2]
-    else:
-        a.o_stride_t, a.o_stride_h = out.stride(0), out.stride(1)
-    a.total_q, a.total_k = Tq, total_k
-    a.k_split = total_k if k2 is None else int(k_split)
-    a.n_ranges, a.ranges_mode = max(n, 0), ranges_mode
-    a.max_seqlen_q, a.max_seqlen_k = int(max_seqlen_q), int(max_seqlen_k)
-    a.Hq, a.Hkv, a.D = Hq, Hkv, D
-    a.dtype = _dtype_code(q)
-    a.scale_chunk_tokens = int(scale_chunk_tokens)
-    a.softmax_scale = 0.0 if softmax_scale is None else float(softmax_scale)
-    a.flags = ((L.MAGI_ATTN_FP8_POW2_PRESCALED if fp8_pow2_prescaled else 0) | (L.MAGI_ATTN_Q_PRESCALED if q_prescaled else 0)
-               | (L.MAGI_ATTN_FP8_FAST_EXP2 if fp8_fast_exp2 else 0) | (L.MAGI_ATTN_BOUNDED_MFMA32 if bounded_mfma32 else 0)
-               | (L.MAGI_ATTN_AUTO_BOUND if auto_bound else 0) | (L.MAGI_ATTN_ZERO_UNCOVERED if zero_gaps else 0))
+        o_stride_g, group_heads = o_stride[1], out.shape[2]
+    o_stride_t = o_stride[0] if group_heads else o_stride[-3]
+    flags = ((L.MAGI_ATTN_FP8_POW2_PRESCALED if fp8_pow2_prescaled else 0) | (L.MAGI_ATTN_Q_PRESCALED if q_prescaled else 0)
+             | (L.MAGI_ATTN_FP8_FAST_EXP2 if fp8_fast_exp2 else 0) | (L.MAGI_ATTN_BOUNDED_MFMA32 if bounded_mfma32 else 0)
+             | (L.MAGI_ATTN_AUTO_BOUND if auto_bound else 0) | (L.MAGI_ATTN_ZERO_UNCOVERED if zero_gaps else 0))
     workspace = None
     if auto_bound and not static_scratch:
         workspace = torch.empty(4, dtype=torch.float32, device=q.device)  # (alive until the launches are enqueued)
-        a.workspace = _ptr(workspace)
-    a.score_bound = float(score_bound)
-    a.q_tile_rows = int(q_tile_rows)
-    keep = None
+    gamma = beta = None  # (alive until the launch is enqueued)
+    norm_eps, norm_kind = 0.0, 0
     if q_norm is not None:
-        g_ = q_norm[0].to(torch.float32).contiguous()
-        b_ = None if q_norm[1] is None else q_norm[1].to(torch.float32).contiguous()
-        keep = (g_, b_)  # (alive until the launch is enqueued)
-        a.q_norm_gamma, a.q_norm_beta = _ptr(g_), _ptr(b_)
-        a.q_norm_eps = float(q_norm[2])
-        a.q_norm_kind = int(q_norm[3]) if len(q_norm) > 3 else L.MAGI_NORM_LAYERNORM_1P
-    with torch.cuda.device(q.device):
-        entry = L.lib().magi_attn_fwd_static_scratch if static_scratch else L.lib().magi_attn_fwd
-        L.check(entry(C.byref(a), _stream()))
+        gamma = q_norm[0].to(torch.float32).contiguous()
+        beta = None if q_norm[1] is None else q_norm[1].to(torch.float32).contiguous()
+        norm_eps = float(q_norm[2])
+        norm_kind = int(q_norm[3]) if len(q_norm) > 3 else L.MAGI_NORM_LAYERNORM_1P
+    k_stride, v_stride = k.stride(), v.stride()
+    _launch_packed(
+        q.device, "magi_attn_fwd_static_scratch" if static_scratch else "magi_attn_fwd", L.AttnArgs,
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), _ptr(k2), _ptr(v2), out.data_ptr(), _ptr(lse), q_ranges.data_ptr(),
+        k_ranges.data_ptr(), _ptr(q_scale), _ptr(k_scale), _ptr(v_scale), q_stride[-3], q_stride[-2], k_stride[0], k_stride[1],
+        v_stride[0], v_stride[1], o_stride_t, o_stride[-2], Tq, total_k, total_k if k2 is None else int(k_split), max(n, 0),
+        ranges_mode, int(max_seqlen_q), int(max_seqlen_k), Hq, Hkv, D, _dtype_code(q), int(scale_chunk_tokens),
+        0.0 if softmax_scale is None else float(softmax_scale), flags, group_heads, o_stride_g,
+        min(float(score_bound), 3e38), int(q_tile_rows), _ptr(gamma), _ptr(beta), norm_eps, norm_kind, _ptr(k2_scale),
+        _ptr(v2_scale), _ptr(workspace), batch_rows, q_stride_b, o_stride_b)
     return out, lse
 
 
@@ -314,9 +315,8 @@ def apply_rotary_emb(x, cos, sin, interleaved=False, inplace=False, **_unused):
     y = xc if inplace else torch.empty_like(xc)
     cosf = cos.to(torch.float32).contiguous()
     sinf = sin.to(torch.float32).contiguous()
-    with torch.cuda.device(x.device):
-        L.check(L.lib().magi_apply_rotary(xc.data_ptr(), cosf.data_ptr(), sinf.data_ptr(), y.data_ptr(), B, S, H, D, R2,
-                                          int(x.dtype == torch.bfloat16), _stream()))
+    _launch(x.device, L.lib().magi_apply_rotary, xc.data_ptr(), cosf.data_ptr(), sinf.data_ptr(), y.data_ptr(), B, S, H, D, R2,
+            int(x.dtype == torch.bfloat16))
     return y
 
 
@@ -356,24 +356,16 @@ def qk_prologue(q_raw, k_raw, v_raw, rope, gq, bq, gk, bk, *, Hq: int, Hkv: int,
         raise ValueError("kv_tail is shorter than S - n_cache_rows")
     f32 = lambda t: None if t is None else t.to(torch.float32).contiguous()
     gq, bq, gk, bk = f32(gq), f32(bq), f32(gk), f32(bk)
-    a = L.PrologueArgs()
     R2 = 0
     if rope is not None:
         if rope.dtype != torch.float32 or rope.dim() != 2 or rope.shape[0] * max(batch, 1) != S or not rope.is_contiguous():
             raise ValueError("rope must be a contiguous fp32 [S / batch, 2*R2] tensor")
         R2 = rope.shape[1] // 2
-    a.q_raw, a.k_raw, a.v_raw, a.rope = _ptr(q_raw), _ptr(k_raw), _ptr(v_raw), _ptr(rope)
-    a.gq, a.bq, a.gk, a.bk = _ptr(gq), _ptr(bq), _ptr(gk), _ptr(bk)
-    a.q_out, a.kv_out, a.kv_tail = _ptr(q_out), _ptr(kv_out), _ptr(kv_tail)
-    a.q_raw_stride_t, a.k_raw_stride_t, a.v_raw_stride_t = q_raw.stride(0), k_raw.stride(0), v_raw.stride(0)
-    a.kv_stride_t = 0 if kv_out is None else kv_out.stride(0)
-    a.kv_tail_stride_t = 0 if kv_tail is None else kv_tail.stride(0)
-    a.S, a.n_cache_rows = S, int(n_cache_rows)
-    a.Hq, a.Hkv, a.D, a.R2 = Hq, Hkv, D, R2
-    a.norm_kind, a.eps, a.batch = int(norm_kind), float(eps), int(batch)
-    a.q_premul = float(q_premul)
-    with torch.cuda.device(dev):
-        L.check(L.lib().magi_qk_prologue(C.byref(a), _stream()))
+    _launch_packed(dev, "magi_qk_prologue", L.PrologueArgs, q_raw.data_ptr(), k_raw.data_ptr(), v_raw.data_ptr(), _ptr(rope),
+                   _ptr(gq), _ptr(bq), _ptr(gk), _ptr(bk), q_out.data_ptr(), _ptr(kv_out), _ptr(kv_tail), q_raw.stride(0),
+                   k_raw.stride(0), v_raw.stride(0), 0 if kv_out is None else kv_out.stride(0),
+                   0 if kv_tail is None else kv_tail.stride(0), S, int(n_cache_rows), Hq, Hkv, D, R2, int(norm_kind), float(eps),
+                   int(batch), float(q_premul), L.MAGI_DTYPE_BF16, 0.0, 0.0)
     return q_out, kv_out, kv_tail
 
 
@@ -413,26 +405,16 @@ def qk_prologue_fp8(q_raw, k_raw, rope, gq, bq, gk, bk, *, Hq: int, Hkv: int, q_
         raise ValueError("k_tail is shorter than S - n_cache_rows")
     f32 = lambda t: None if t is None else t.to(torch.float32).contiguous()
     gq, bq, gk, bk = f32(gq), f32(bq), f32(gk), f32(bk)
-    a = L.PrologueArgs()
     R2 = 0
     if rope is not None:
         if rope.dtype != torch.float32 or rope.dim() != 2 or rope.shape[0] * max(batch, 1) != S or not rope.is_contiguous():
             raise ValueError("rope must be a contiguous fp32 [S / batch, 2*R2] tensor")
         R2 = rope.shape[1] // 2
-    a.q_raw, a.k_raw, a.v_raw, a.rope = _ptr(q_raw), _ptr(k_raw), None, _ptr(rope)
-    a.gq, a.bq, a.gk, a.bk = _ptr(gq), _ptr(bq), _ptr(gk), _ptr(bk)
-    a.q_out, a.kv_out, a.kv_tail = _ptr(q_out), _ptr(k_out), _ptr(k_tail)
-    a.q_raw_stride_t, a.k_raw_stride_t = q_raw.stride(0), k_raw.stride(0)
-    a.kv_stride_t = 0 if k_out is None else k_out.stride(0)
-    a.kv_tail_stride_t = 0 if k_tail is None else k_tail.stride(0)
-    a.S, a.n_cache_rows = S, int(n_cache_rows)
-    a.Hq, a.Hkv, a.D, a.R2 = Hq, Hkv, D, R2
-    a.norm_kind, a.eps, a.batch = int(norm_kind), float(eps), int(batch)
-    a.q_premul = float(q_premul)
-    a.out_dtype = L.MAGI_DTYPE_FP8_E4M3
-    a.q_quant_scale, a.k_quant_scale = float(q_scale), float(k_scale)
-    with torch.cuda.device(dev):
-        L.check(L.lib().magi_qk_prologue(C.byref(a), _stream()))
+    _launch_packed(dev, "magi_qk_prologue", L.PrologueArgs, q_raw.data_ptr(), k_raw.data_ptr(), 0, _ptr(rope), _ptr(gq), _ptr(bq),
+                   _ptr(gk), _ptr(bk), q_out.data_ptr(), _ptr(k_out), _ptr(k_tail), q_raw.stride(0), k_raw.stride(0), 0,
+                   0 if k_out is None else k_out.stride(0), 0 if k_tail is None else k_tail.stride(0), S, int(n_cache_rows), Hq,
+                   Hkv, D, R2, int(norm_kind), float(eps), int(batch), float(q_premul), L.MAGI_DTYPE_FP8_E4M3, float(q_scale),
+                   float(k_scale))
     return q_out, k_out, k_tail
 
 
@@ -476,24 +458,15 @@ def qkv_proj_prologue(x: torch.Tensor, w: torch.Tensor, rope, gq, bq, gk, bk, *,
         raise ValueError("kv_tail is shorter than S - n_cache_rows")
     f32 = lambda t: None if t is None else t.to(torch.float32).contiguous()
     gq, bq, gk, bk = f32(gq), f32(bq), f32(gk), f32(bk)
-    a = L.QkvProjArgs()
     R2 = 0
     if rope is not None:
         if rope.dtype != torch.float32 or rope.dim() != 2 or rope.shape[0] * max(batch, 1) != S or not rope.is_contiguous():
             raise ValueError("rope must be a contiguous fp32 [S / batch, 2*R2] tensor")
         R2 = rope.shape[1] // 2
-    a.x, a.w, a.x_stride, a.w_stride = _ptr(x), _ptr(w), x.stride(0), w.stride(0)
-    a.S, a.K = S, K
-    a.Hq, a.Hkv, a.Hqx, a.D = Hq, Hkv, Hqx, D
-    a.rope, a.R2 = _ptr(rope), R2
-    a.gq, a.bq, a.gk, a.bk = _ptr(gq), _ptr(bq), _ptr(gk), _ptr(bk)
-    a.norm_kind, a.eps, a.batch, a.q_premul = int(norm_kind), float(eps), int(batch), float(q_premul)
-    a.q_out, a.kv_out, a.kv_tail, a.qx_out = _ptr(q_out), _ptr(kv_out), _ptr(kv_tail), _ptr(qx_out)
-    a.kv_stride_t = 0 if kv_out is None else kv_out.stride(0)
-    a.kv_tail_stride_t = 0 if kv_tail is None else kv_tail.stride(0)
-    a.n_cache_rows = int(n_cache_rows)
-    with torch.cuda.device(dev):
-        L.check(L.lib().magi_qkv_proj_prologue(C.byref(a), _stream()))
+    _launch_packed(dev, "magi_qkv_proj_prologue", L.QkvProjArgs, x.data_ptr(), w.data_ptr(), x.stride(0), w.stride(0), S, K, Hq, Hkv,
+                   Hqx, D, _ptr(rope), R2, _ptr(gq), _ptr(bq), _ptr(gk), _ptr(bk), int(norm_kind), float(eps), int(batch),
+                   float(q_premul), q_out.data_ptr(), _ptr(kv_out), _ptr(kv_tail), 0 if kv_out is None else kv_out.stride(0),
+                   0 if kv_tail is None else kv_tail.stride(0), int(n_cache_rows), _ptr(qx_out))
     return q_out, kv_out, kv_tail, qx_out
 
 
@@ -535,9 +508,8 @@ def layer_norm(x: torch.Tensor, weight: Optional[torch.Tensor], bias: Optional[t
             raise TypeError("weight and bias must share a dtype")
         fp32 = p.dtype == torch.float32
     rows = x2.shape[0]
-    with torch.cuda.device(x.device):
-        L.check(L.lib().magi_layer_norm(x2.data_ptr(), x2.stride(0) if rows > 1 else cols, _ptr(weight), _ptr(bias),
-                                        int(bool(fp32)), y.data_ptr(), cols, rows, cols, float(eps), _stream()))
+    _launch(x.device, L.lib().magi_layer_norm, x2.data_ptr(), x2.stride(0) if rows > 1 else cols, _ptr(weight), _ptr(bias),
+            int(bool(fp32)), y.data_ptr(), cols, rows, cols, float(eps))
     return y
 
 
@@ -560,9 +532,8 @@ def div_clamp_to(x: torch.Tensor, scale: torch.Tensor, out: Optional[torch.Tenso
     if y.shape != x.shape or y.dtype != torch.float8_e4m3fn or y.device != x.device or not y.is_contiguous():
         raise ValueError("out must be a contiguous float8_e4m3fn tensor of x's shape on x's device")
     rows = x2.shape[0]
-    with torch.cuda.device(x.device):
-        L.check(L.lib().magi_div_clamp_to_e4m3(x2.data_ptr(), x2.stride(0) if rows > 1 else cols, sc.data_ptr(), sc.numel(),
-                                               y.data_ptr(), cols, rows, cols, _stream()))
+    _launch(x.device, L.lib().magi_div_clamp_to_e4m3, x2.data_ptr(), x2.stride(0) if rows > 1 else cols, sc.data_ptr(), sc.numel(),
+            y.data_ptr(), cols, rows, cols)
     return y
 
 
@@ -593,9 +564,8 @@ def layer_norm_div_clamp(x: torch.Tensor, weight: Optional[torch.Tensor], bias: 
     rows = x.numel() // max(cols, 1)
     sp = (C.c_void_p * n)(*[s.data_ptr() for s in scales])
     yp = (C.c_void_p * n)(*[y.data_ptr() + k * x.numel() for k in range(n)])
-    with torch.cuda.device(x.device):
-        L.check(L.lib().magi_layer_norm_e4m3(x.data_ptr(), cols, _ptr(weight), _ptr(bias), int(bool(fp32)), sp, yp, n, rows, cols,
-                                             float(eps), _stream()))
+    _launch(x.device, L.lib().magi_layer_norm_e4m3, x.data_ptr(), cols, _ptr(weight), _ptr(bias), int(bool(fp32)), sp, yp, n, rows,
+            cols, float(eps))
     return y
 
 
@@ -608,9 +578,8 @@ def head_norm(x: torch.Tensor, gamma, beta, eps: float = 1e-6, norm_kind: int = 
     y = torch.empty((S, H, D), dtype=torch.bfloat16, device=x.device)
     g = None if gamma is None else gamma.to(torch.float32).contiguous()
     b = None if beta is None else beta.to(torch.float32).contiguous()
-    with torch.cuda.device(x.device):
-        L.check(L.lib().magi_head_norm(x.data_ptr(), x.stride(0), x.stride(1), _ptr(g), _ptr(b), y.data_ptr(), S, H, D,
-                                       int(norm_kind), float(eps), _stream()))
+    _launch(x.device, L.lib().magi_head_norm, x.data_ptr(), x.stride(0), x.stride(1), _ptr(g), _ptr(b), y.data_ptr(), S, H, D,
+            int(norm_kind), float(eps))
     return y
 
 
@@ -637,9 +606,8 @@ def quantize_fp8(x: torch.Tensor, chunk_tokens: int, premul: float = 1.0, pow2_s
     if (scales.dtype != torch.float32 or tuple(scales.shape) != (n_chunks, H) or not scales.is_contiguous()
             or scales.device != x.device):
         raise ValueError("scales_out must be a contiguous fp32 [ceil(T / chunk_tokens), H] tensor on x's device")
-    with torch.cuda.device(x.device):
-        L.check(L.lib().magi_quantize_fp8(x.data_ptr(), x.stride(0), x.stride(1), y.data_ptr(), scales.data_ptr(), T, H, D,
-                                          int(chunk_tokens), float(premul), int(pow2_scales), _stream()))
+    _launch(x.device, L.lib().magi_quantize_fp8, x.data_ptr(), x.stride(0), x.stride(1), y.data_ptr(), scales.data_ptr(), T, H, D,
+            int(chunk_tokens), float(premul), int(pow2_scales))
     return y, scales
 
 
@@ -668,11 +636,5 @@ def quantize_fp8_split(x: torch.Tensor, chunk_tokens: int, n_rows_first: int, ou
         if (sc is None or sc.dtype != torch.float32 or sc.dim() != 2 or sc.shape[0] < chunks or sc.shape[1] != H
                 or not sc.is_contiguous() or sc.device != x.device):
             raise ValueError(f"the scales of {name} must be a contiguous fp32 [>= {chunks}, H] tensor on x's device")
-    a = L.QuantizeArgs()
-    a.x, a.x_stride_t, a.x_stride_h = _ptr(x), x.stride(0), x.stride(1)
-    a.T, a.H, a.D, a.chunk_tokens = T, H, D, int(chunk_tokens)
-    a.premul, a.pow2_scales = float(premul), int(pow2_scales)
-    a.y, a.scales, a.n_rows_first = _ptr(out), _ptr(scales_out), n1
-    a.y2, a.scales2 = _ptr(out2), _ptr(scales2_out)
-    with torch.cuda.device(x.device):
-        L.check(L.lib().magi_quantize_fp8_split(C.byref(a), _stream()))
+    _launch_packed(x.device, "magi_quantize_fp8_split", L.QuantizeArgs, x.data_ptr(), x.stride(0), x.stride(1), T, H, D,
+                   int(chunk_tokens), float(premul), int(pow2_scales), _ptr(out), _ptr(scales_out), n1, _ptr(out2), _ptr(scales2_out))

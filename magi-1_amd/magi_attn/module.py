@@ -69,14 +69,16 @@ class FusedLayerNorm(torch.nn.Module):
         parameter values (no launches on later calls) and kept until a parameter is modified or replaced."""
         # (a write through `.data` does not advance _version: callers that patch parameters that way call
         # invalidate_cached_parameters())
-        key = tuple(x for t in (self.weight, self.bias) for x in (id(t), t._version, t.data_ptr(), t.dtype, t.device))
-        if self.__dict__.get("_gb_key") != key:
-            w = self.weight.detach()
-            g = ((w + 1).float() - 1.0) if self.zero_centered_gamma else (w.float() - 1.0)
-            self.__dict__["_gb"] = (g.contiguous(), self.bias.detach().float().contiguous())
-            self.__dict__["_gb_key"] = key
-            self.__dict__["_gb_epoch"] = self.__dict__.get("_gb_epoch", 0) + 1
-        return self.__dict__["_gb"]
+        w, b = self._parameters["weight"], self._parameters["bias"]
+        key = (id(w), w._version, w.data_ptr(), w.dtype, w.device, id(b), b._version, b.data_ptr(), b.dtype, b.device)
+        state = self.__dict__
+        if state.get("_gb_key") != key:
+            g = w.detach()
+            g = ((g + 1).float() - 1.0) if self.zero_centered_gamma else (g.float() - 1.0)
+            state["_gb"] = (g.contiguous(), b.detach().float().contiguous())
+            state["_gb_key"] = key
+            state["_gb_epoch"] = state.get("_gb_epoch", 0) + 1
+        return state["_gb"]
 
     def parameter_epoch(self) -> int:
         """A counter that advances whenever gamma_beta_fp32() had to convert the parameters anew: what values derived
@@ -328,15 +330,16 @@ class FullyParallelAttention(torch.nn.Module):
         larger values make them fall back to it.  Computed once per set of parameter values (it reads them on the
         host) and cached until a parameter is modified or replaced (see invalidate_cached_parameters)."""
         lns = (self.q_layernorm, self.k_layernorm, self.q_layernorm_xattn, self.k_layernorm_xattn)
-        key = tuple(ln.parameter_epoch() for ln in lns)
-        if getattr(self, "_bounds_key", None) != key:
+        key = (lns[0].parameter_epoch(), lns[1].parameter_epoch(), lns[2].parameter_epoch(), lns[3].parameter_epoch())
+        state = self.__dict__
+        if state.get("_bounds_key") != key:
             self._bounds, self._bounds_key = {}, key
+        bounds = state["_bounds"]
         r = int(rotary_half)
-        if r not in self._bounds:  # (the cross-attention half does not depend on r)
-            cross = next(iter(self._bounds.values()))[1] if self._bounds else \
-                1.01 * self._q_premul * qk_score_bound(lns[2], lns[3], 0)
-            self._bounds[r] = (1.01 * self._q_premul * qk_score_bound(lns[0], lns[1], r), cross)
-        return self._bounds[r]
+        if r not in bounds:  # (the cross-attention half does not depend on r)
+            cross = next(iter(bounds.values()))[1] if bounds else 1.01 * self._q_premul * qk_score_bound(lns[2], lns[3], 0)
+            bounds[r] = (1.01 * self._q_premul * qk_score_bound(lns[0], lns[1], r), cross)
+        return bounds[r]
 
     def invalidate_cached_parameters(self) -> None:
         """Forget everything derived from the norm parameters (their fp32 forms, the score bounds, the e4m3 operand
@@ -663,13 +666,13 @@ class FullyParallelAttention(torch.nn.Module):
         return out.transpose(0, 1).contiguous() if b > 1 else out.view(sq, 1, -1)
 
     def _cross_attention_fused(self, qx_raw: torch.Tensor, key_value_states: torch.Tensor,
-                               cross_attn_params: PackedCrossAttnParams, out: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
+                               cross_attn_params: PackedCrossAttnParams, out: Optional[torch.Tensor],
+                               bound: float) -> Optional[torch.Tensor]:
         """Cross attention on the RAW qx projection [sq, b, Hq*D]: the attention kernel applies q_layernorm_xattn while it
         loads q (no normalised copy of q in memory) and, the scores of normed q and k being bounded, runs without a
         running maximum; at batch > 1 it reads and writes the [position, batch] rows where they are.  Returns None
         when that path does not apply (then the caller takes get_xqkv + cross_attention); else the result, [sq, b, Hq, D]
         contiguous (or `out`, batch 1 only)."""
-        bound = self.score_bounds()[1]
         if not (0.0 < bound <= L.MAGI_SCORE_BOUND_MAX):
             return None
         D = self.hidden_size_per_attention_head
@@ -703,7 +706,7 @@ class FullyParallelAttention(torch.nn.Module):
         sin_emb, cos_emb = rotary_pos_emb.tensor_split(2, -1)
         # the incoming table already is the [sin | cos] layout the prologue takes
         rope = rotary_pos_emb if (rotary_pos_emb.dtype == torch.float32 and rotary_pos_emb.is_contiguous()) else None
-        bound_core = self.score_bounds(rotary_pos_emb.shape[-1] // 2)[0]
+        bound_core, bound_cross = self.score_bounds(rotary_pos_emb.shape[-1] // 2)
         core_bound_kw = {"score_bound": bound_core}  # (above the limit: the online-softmax kernel, unless measured)
         measured = False
         if not (0.0 < bound_core <= L.MAGI_SCORE_BOUND_MAX) and self.attention_dtype == "bf16" and hidden_states.shape[1] == 1:
@@ -724,8 +727,8 @@ class FullyParallelAttention(torch.nn.Module):
             "core": "fp8" if self.attention_dtype == "fp8" else
             ("measured bound: bounded-score or online softmax, chosen on the device" if measured else bounded(bound_core)),
             "core_score_bound": bound_core,
-            "cross": bounded(self.score_bounds()[1]),
-            "cross_score_bound": self.score_bounds()[1]}
+            "cross": bounded(bound_cross),
+            "cross_score_bound": bound_cross}
         bs = hidden_states.shape[1]
         sq = hidden_states.shape[0]
         D = self.hidden_size_per_attention_head
@@ -821,11 +824,11 @@ class FullyParallelAttention(torch.nn.Module):
                 if offloaded is not None:  # the persisted rows go back to the host behind the attention launch
                     offloaded.release(start, persisted)
         if fused is not None:
-            if self._cross_attention_fused(qx_raw, key_value_states, meta_args.cross_attn_params, cross_dst) is None:
+            if self._cross_attention_fused(qx_raw, key_value_states, meta_args.cross_attn_params, cross_dst, bound_cross) is None:
                 self.cross_attention(mixed_qqkv, key_value_states, meta_args.cross_attn_params, get_xqkv, out=cross_dst)
             return fused
         core_attn_out = core.view(sq, bs, -1)
-        xo = self._cross_attention_fused(qx_raw, key_value_states, meta_args.cross_attn_params, None)
+        xo = self._cross_attention_fused(qx_raw, key_value_states, meta_args.cross_attn_params, None, bound_cross)
         if xo is not None:
             xattn_out = xo.reshape(sq, bs, -1)
         else:
