@@ -311,9 +311,9 @@ int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace) {
     const double total = (double)p->Hq * p->n_ranges * a.tiles_per_range;
     if (total > 2.0e9) return fail(MAGI_EINVAL, "magi_attn_fwd: grid too large (%.3g workgroups)", total);
     // workgroups of one XCD's list (attn_common.h, locate_work): its Hkv / 8 whole heads, and its share of the rest
-    const int left = p->Hkv % 8, groups = p->n_ranges * a.tiles_per_range;
-    const int dealt = left == 0 ? 0 : 8 % left == 0 ? (groups + 8 / left - 1) / (8 / left) : (left * groups + 7) / 8;
-    a.per_xcd = (unsigned)((p->Hkv / 8) * groups + dealt) * (unsigned)a.G;
+    const long left = p->Hkv % 8, per_head = (long)p->n_ranges * a.tiles_per_range * a.G;
+    const long dealt = (left * per_head + 7) / 8;
+    a.per_xcd = (unsigned)((p->Hkv / 8) * per_head + dealt);
     hipError_t e;
     if (p->dtype != MAGI_DTYPE_BF16)
       e = magi::launch_attn_fwd_fp8(a, static_cast<hipStream_t>(stream));

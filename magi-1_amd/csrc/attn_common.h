@@ -106,8 +106,8 @@ __device__ __forceinline__ void zero_rows(const AttnKernArgs& a, const WorkItem&
 // blockIdx -> (kv head, range slot, q tile, q head within the GQA group), laid out so that the workgroups an
 // XCD receives (blockIdx % 8) share a KV head and walk the same keys at about the same time (each XCD has its
 // own L2).  XCD x owns the heads x * (Hkv / 8) .. of the first 8 * (Hkv / 8); the Hkv % 8 heads that are left are
-// shared, their (range, tile) groups dealt to the XCDs in turn: cut into contiguous pieces instead, an XCD got one
-// range's tiles and the last XCDs ran dry (6 q heads / 1 kv head, four 720p chunks behind eight: 46.4 -> 45.5 ms).  Ranges are visited longest key span first (ties
+// shared, their (range, tile, q head) items dealt to the XCDs one by one: cut into contiguous pieces instead, an XCD got
+// one range's tiles and the last XCDs ran dry.  Ranges are visited longest key span first (ties
 // by index), ranked here from the device-side list.
 // Every thread of the workgroup must call this (it contains a barrier); s_sel is LOCATE_WORDS ints of LDS.
 constexpr int LOCATE_WORDS = 8;
@@ -128,19 +128,20 @@ __device__ __forceinline__ WorkItem locate_work(const AttnKernArgs& a, int BM, i
     hg = i - grp * G;
   } else {
     i -= whole * per_head;
-    grp = i / G;
-    hg = i - grp * G;
+    unsigned u;  // position in the list of one shared head, or of all the heads that are left
     if ((8u % left) == 0u) {  // 8 / left XCDs share a head
       const unsigned share = 8u / left;
       kvh = 8u * whole + xcd / share;
-      grp = xcd % share + share * grp;
+      u = xcd % share + share * i;
     } else {
-      const unsigned u = xcd + 8u * grp;
-      kvh = u / groups;
-      grp = u - kvh * groups;
+      u = xcd + 8u * i;
+      kvh = u / per_head;
+      u -= kvh * per_head;
       kvh += 8u * whole;
     }
-    if (grp >= groups || kvh >= (unsigned)a.Hkv) return wi;
+    if (u >= per_head || kvh >= (unsigned)a.Hkv) return wi;
+    grp = u / G;
+    hg = u - grp * G;
   }
   const unsigned rslot = grp / tiles, tile = grp - rslot * tiles;
   wi.kvh = (int)kvh;
