@@ -1073,3 +1073,19 @@ def test_rope_table_built_on_the_device_matches_the_oracle(dev):
     got = LearnableRotaryEmbeddingCat(128, device=dev).get_embed_for_forward(4, 5, 7, 1, 2)
     want = O.rope_for_forward(4, 5, 7, 1, 2)
     assert (got.cpu() - want).abs().max().item() <= 1e-6
+
+
+@pytest.mark.parametrize("rows", [7, 2047, 2048, 2049, 3276, 3277, 4096, 4097, 6143])
+def test_projection_rows_cut_at_whole_rounds_of_tiles(dev, rows):
+    """8192 output columns: 2048 rows are a round of the library's tiles; every row of both parts against float64.
+    Bound: K fp32 additions of products in any order, and one rounding to bf16."""
+    K, N = 1024, 8192
+    g = torch.Generator(device=dev).manual_seed(rows)
+    x = torch.randn(rows, 1, K, device=dev, generator=g).bfloat16()
+    w = (torch.randn(N, K, device=dev, generator=g) * K ** -0.5).bfloat16()
+    y = MOD._linear_in_whole_rounds(x, w)
+    assert y.shape == (rows, 1, N) and y.is_contiguous()
+    cols = torch.arange(0, N, 61, device=dev)
+    ref = x[:, 0].double() @ w[cols].double().t()
+    mag = x[:, 0].double().abs() @ w[cols].double().abs().t()
+    assert ((y[:, 0][:, cols].double() - ref).abs() <= 2.0 ** -8 * ref.abs() + K * 2.0 ** -24 * mag).all()
