@@ -68,6 +68,14 @@ extern "C" {
 /* Rows of `out` that no q range covers become zeros (and their lse -inf) in the same launch, so that the caller need not
  * clear the output first; without the flag they are left untouched.  1 to 64 ranges. */
 #define MAGI_ATTN_ZERO_UNCOVERED 32
+/* For bf16 callers that promise nothing about the scores: run the bounded-score kernel as if they were bounded, have it
+ * judge by its row sums whether they were (sums within 2^+-64: no score above 64, nothing of weight underflowed), and
+ * repeat in a second launch, with a running maximum, the 64-row blocks where they were not.  No passes over q and k
+ * (MAGI_ATTN_AUTO_BOUND) and the right result for any input; inputs with larger scores throughout cost about 2.5 times
+ * as much.  args->workspace: 16 bytes of DEVICE memory per q head, range and 256 rows of max_seqlen_q (any content), 16-byte
+ * aligned, one for each of the calls that may overlap.  Not with score_bound, q_norm, q_tile_rows,
+ * MAGI_ATTN_BOUNDED_MFMA32 or MAGI_ATTN_AUTO_BOUND. */
+#define MAGI_ATTN_CHECKED 64
 
 #define MAGI_RANGES_PAIRS 0 /* int32 [n, 2]: range i = [r[2i], r[2i+1])          */
 #define MAGI_RANGES_CU 1    /* int32 [n + 1] cumulative: range i = [r[i], r[i+1]) */
@@ -201,7 +209,7 @@ typedef struct magi_attn_args {
    * cache's tables.  NULL (both): k_scale / v_scale are indexed across k_split as one table. */
   const float* k2_scale;
   const float* v2_scale;
-  /* MAGI_ATTN_AUTO_BOUND: 16 bytes of DEVICE memory, 16-byte aligned, that the call may overwrite (the measured
+  /* MAGI_ATTN_CHECKED: see there.  MAGI_ATTN_AUTO_BOUND: 16 bytes of DEVICE memory, 16-byte aligned, that the call may overwrite (the measured
    * bound; calls that overlap on the device need a workspace each).  NULL otherwise. */
   float* workspace;
   /* Version 104 (a struct that ends here, struct_size = offsetof(magi_attn_args, q_batch_rows), is accepted too: the fields

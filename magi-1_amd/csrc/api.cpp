@@ -114,6 +114,8 @@ int magi_attn_fwd_static_scratch(const magi_attn_args* p, void* stream) {
   magi_attn_args full;
   p = current_layout(p, &full);
   MAGI_CHECK_LAYOUT("magi_attn_fwd_static_scratch", p);
+  if (p->flags & MAGI_ATTN_CHECKED)
+    return fail(MAGI_ENOSYS, "magi_attn_fwd_static_scratch: the workspace of MAGI_ATTN_CHECKED grows with the problem");
   static_assert(4 * sizeof(float) <= SCRATCH_BYTES, "the measured score bound needs four words");
   void* ws = nullptr;
   const int rc = static_scratch(&ws);
@@ -189,6 +191,16 @@ int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace) {
                                "q_tile_rows and MAGI_ATTN_BOUNDED_MFMA32 (it measures the bound and picks the kernel itself)");
     if (!workspace || !aligned16(workspace))
       return fail(MAGI_EINVAL, "magi_attn_fwd: MAGI_ATTN_AUTO_BOUND needs a 16-byte workspace on the device, 16-byte aligned");
+  }
+  const bool checked = (p->flags & MAGI_ATTN_CHECKED) != 0;
+  if (checked) {
+    if (p->dtype != MAGI_DTYPE_BF16 || p->score_bound > 0.f || q_norm || p->q_tile_rows != 0 ||
+        (p->flags & (MAGI_ATTN_BOUNDED_MFMA32 | MAGI_ATTN_AUTO_BOUND)))
+      return fail(MAGI_EINVAL, "magi_attn_fwd: MAGI_ATTN_CHECKED goes with bf16 and without score_bound, q_norm, q_tile_rows, "
+                               "MAGI_ATTN_BOUNDED_MFMA32 and MAGI_ATTN_AUTO_BOUND");
+    if (!workspace || !aligned16(workspace))
+      return fail(MAGI_EINVAL, "magi_attn_fwd: MAGI_ATTN_CHECKED needs a workspace on the device, 16-byte aligned, of 16 bytes "
+                               "per q head, range and 256 rows of max_seqlen_q");
   }
   if (p->out_group_heads < 0 || (p->out_group_heads > 0 && (p->Hq % p->out_group_heads || p->o_stride_g % 8)))
     return fail(MAGI_EINVAL, "magi_attn_fwd: out_group_heads must divide Hq and o_stride_g keep rows 16-byte aligned");
@@ -284,11 +296,12 @@ int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace) {
   // (with q_norm, or a score bound on unscaled q, the kernel multiplies q by scale_log2 itself while loading it, after
   // which the same holds)
 
-  // One launch of `a` as the bounded-score kernel (bounded) or as the kernel without a promise about the scores.
+  // One launch of `a` as the bounded-score kernel (bounded) or as the kernel without a promise about the scores; with
+  // MAGI_ATTN_CHECKED the bounded-score kernel and the launch that repeats what it could not be trusted with.
   auto launch = [&](bool bounded) -> int {
     // a bound stated for unscaled q (what the reference's callers pass): the kernel applies the softmax scale while
     // it loads q, after which the scores are exp2 exponents as with MAGI_ATTN_Q_PRESCALED
-    const bool scale_q = bounded && !q_norm && !(p->flags & MAGI_ATTN_Q_PRESCALED);
+    const bool scale_q = bounded && !q_norm && !checked && !(p->flags & MAGI_ATTN_Q_PRESCALED);
     a.block_m = 128;
     if (p->dtype == MAGI_DTYPE_BF16) {
       const double wg384 = (double)p->Hq * p->n_ranges * ((p->max_seqlen_q + 383) / 384);
@@ -317,6 +330,8 @@ int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace) {
     hipError_t e;
     if (p->dtype != MAGI_DTYPE_BF16)
       e = magi::launch_attn_fwd_fp8(a, static_cast<hipStream_t>(stream));
+    else if (checked)
+      e = magi::launch_attn_fwd_bf16_checked(a, compute_units(), static_cast<hipStream_t>(stream));
     else if (bounded && a.block_m == 256 && !mfma32)
       e = magi::launch_attn_fwd_bf16_x16(a, static_cast<hipStream_t>(stream));
     else if (bounded)
@@ -324,10 +339,14 @@ int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace) {
     else
       e = magi::launch_attn_fwd_bf16(a, static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return hip_fail(e, "magi_attn_fwd launch");
-    g_launches.fetch_add(1, std::memory_order_relaxed);
+    g_launches.fetch_add(checked ? 2 : 1, std::memory_order_relaxed);
     return MAGI_OK;
   };
 
+  if (checked) {
+    a.verdict = reinterpret_cast<int*>(workspace);
+    return launch(true);
+  }
   if (!auto_bound) return launch(promised);
 
   // No promise about the scores: measure one.  Two streaming passes leave the largest squared length of a q row and

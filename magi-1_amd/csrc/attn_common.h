@@ -81,6 +81,7 @@ struct WorkItem {
   int h, kvh;
   int q0, qe, ks, ke;
   long o_head;  // byte offset of head h inside a row of `out`
+  int item;     // (h, range slot, q tile) in that order: the same work in every launch over the same ranges and tiles
   bool valid;   // false: nothing to do (grid padding, or the q tile lies beyond the range)
 };
 
@@ -111,24 +112,23 @@ __device__ __forceinline__ void zero_rows(const AttnKernArgs& a, const WorkItem&
 // by index), ranked here from the device-side list.
 // Every thread of the workgroup must call this (it contains a barrier); s_sel is LOCATE_WORDS ints of LDS.
 constexpr int LOCATE_WORDS = 8;
-__device__ __forceinline__ WorkItem locate_work(const AttnKernArgs& a, int BM, int tid, int* s_sel) {
-  WorkItem wi;
-  wi.valid = false;
-  const unsigned xcd = blockIdx.x & 7u;
-  unsigned i = blockIdx.x >> 3;  // position in this XCD's list
+
+// the arithmetic part: workgroup `block` -> heads, range slot, tile; false for the padding of the grid
+__device__ __forceinline__ bool decode_block(const AttnKernArgs& a, unsigned block, unsigned& kvh, unsigned& hg, unsigned& rslot,
+                                             unsigned& tile) {
+  const unsigned xcd = block & 7u;
+  unsigned i = block >> 3;  // position in this XCD's list
   const unsigned G = (unsigned)a.G, tiles = (unsigned)a.tiles_per_range, groups = (unsigned)a.n_ranges * tiles;
   const unsigned whole = (unsigned)a.Hkv >> 3, left = (unsigned)a.Hkv & 7u;
-  unsigned kvh, grp, hg;  // kv head, (range slot, tile), q head within the GQA group
+  unsigned u;  // position in the list of one head: (range slot, tile, q head)
   const unsigned per_head = groups * G;
   if (i < whole * per_head) {
     const unsigned n = i / per_head;
     kvh = xcd * whole + n;
-    i -= n * per_head;
-    grp = i / G;
-    hg = i - grp * G;
+    u = i - n * per_head;
   } else {
     i -= whole * per_head;
-    unsigned u;  // position in the list of one shared head, or of all the heads that are left
+    if (left == 0u) return false;
     if ((8u % left) == 0u) {  // 8 / left XCDs share a head
       const unsigned share = 8u / left;
       kvh = 8u * whole + xcd / share;
@@ -139,13 +139,26 @@ __device__ __forceinline__ WorkItem locate_work(const AttnKernArgs& a, int BM, i
       u -= kvh * per_head;
       kvh += 8u * whole;
     }
-    if (u >= per_head || kvh >= (unsigned)a.Hkv) return wi;
-    grp = u / G;
-    hg = u - grp * G;
+    if (u >= per_head || kvh >= (unsigned)a.Hkv) return false;
   }
-  const unsigned rslot = grp / tiles, tile = grp - rslot * tiles;
+  const unsigned grp = u / G;
+  hg = u - grp * G;
+  rslot = grp / tiles;
+  tile = grp - rslot * tiles;
+  return true;
+}
+__device__ __forceinline__ int item_of(const AttnKernArgs& a, unsigned kvh, unsigned hg, unsigned rslot, unsigned tile) {
+  return (int)(((kvh * a.G + hg) * (unsigned)a.n_ranges + rslot) * (unsigned)a.tiles_per_range + tile);
+}
+
+__device__ __forceinline__ WorkItem locate_work(const AttnKernArgs& a, int BM, int tid, int* s_sel, unsigned block) {
+  WorkItem wi;
+  wi.valid = false;
+  unsigned kvh, hg, rslot, tile;
+  if (!decode_block(a, block, kvh, hg, rslot, tile)) return wi;
   wi.kvh = (int)kvh;
   wi.h = (int)(kvh * a.G + hg);
+  wi.item = item_of(a, kvh, hg, rslot, tile);
   wi.o_head = a.out_group > 0 ? (long)(wi.h / a.out_group) * a.os_g + (long)(wi.h % a.out_group) * a.os_h
                               : (long)wi.h * a.os_h;
   int qs;

@@ -72,7 +72,7 @@ __global__ __launch_bounds__(64 * NW, OCC) void attn_fwd_bf16_kernel(const AttnK
   if (gate_closed(a)) return;
   const int tid = threadIdx.x;
   // ---- which piece of work is this workgroup? ----
-  const WorkItem wi = locate_work(a, BM, tid, s_sel);
+  const WorkItem wi = locate_work(a, BM, tid, s_sel, blockIdx.x);
   if (!wi.valid) return;
   const int h = wi.h, q0 = wi.q0, qe = wi.qe, ks = wi.ks, ke = wi.ke;
   const unsigned kvh = (unsigned)wi.kvh;

@@ -71,7 +71,7 @@ __global__ __launch_bounds__(64 * NW, OCC) void attn_fwd_bf16_w64_kernel(const A
   __shared__ int s_sel[LOCATE_WORDS];
 
   const int tid = threadIdx.x;
-  const WorkItem wi = locate_work(a, BM, tid, s_sel);
+  const WorkItem wi = locate_work(a, BM, tid, s_sel, blockIdx.x);
   if (!wi.valid) return;
   const int qe = wi.qe, ks = wi.ks, ke = wi.ke;
 

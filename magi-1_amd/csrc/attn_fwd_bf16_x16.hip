@@ -55,6 +55,21 @@ __device__ __forceinline__ int swz(int base, int tie) {
   return r;
 }
 
+// K as the A operand of the score MFMAs: rows 16 KB + n of a tile, features 32 KK + 8 g .. +8 (base: see the kernel)
+template <int KB, int KK>
+__device__ __forceinline__ bf16x8 read_k(const unsigned char* Kt, int base) {
+  return *LDS_PTR(const bf16x8, Kt + (base + KK * 64 + 4 * KB * K_GROUP));
+}
+// V^T as the A operand of the PV MFMAs: feature block DB, the two 16-key blocks of half T of a tile
+template <int T, int DB>
+__device__ __forceinline__ bf16x8 read_v(const unsigned char* Vt, int base, int tie) {
+  const int bv = swz<((DB & 3) << 5), 16 * T + (DB & 3)>(base, tie) + (DB >> 2) * 128;
+  const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(LDS_PTR(s16x4, Vt + (bv + (8 * T) * V_GROUP)));
+  const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(LDS_PTR(s16x4, Vt + (bv + (8 * T + 4) * V_GROUP)));
+  const s16x8 va = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+  return __builtin_bit_cast(bf16x8, va);
+}
+
 // QMODE: what q holds.  0: q as the score MFMAs take it (pre-scaled by the caller).  1: the raw query projection:
 // per-(token, head) norm in fp32 while it is loaded, times the softmax scale, one rounding to bf16.  2: unscaled
 // bf16 q as the reference's callers pass it: multiplied by the softmax scale while it is loaded (a second rounding
@@ -62,10 +77,21 @@ __device__ __forceinline__ int swz(int base, int tie) {
 // order in which the feature blocks of V^T are visited: 0, 4, 1, 5, 2, 6, 3, 7
 constexpr int v_block(int i) { return (i >> 1) + 4 * (i & 1); }
 
-constexpr int Q_AS_IS = 0, Q_NORM = 1, Q_SCALE = 2;
+// Q_CHECK: unscaled bf16 q as it is, the scores multiplied by the softmax scale in fp32 (as the online-softmax kernel does),
+// and nobody's promise that they are bounded: see CHECK.
+constexpr int Q_AS_IS = 0, Q_NORM = 1, Q_SCALE = 2, Q_CHECK = 3;
 
+// Row sums that the kernel without a running maximum can be trusted with (CHECK, below).
+constexpr float SUM_MIN = 0x1p-64f, SUM_MAX = 0x1p64f;
+
+// CHECK (QMODE Q_CHECK): nobody has promised that the scores are bounded.  The kernel computes as if they were, and each wavefront
+// leaves a verdict on its 64 rows in a.verdict[4 * item + wavefront]: 2^score and the accumulators are good where
+// SUM_MIN <= row sum <= SUM_MAX (then no score is above 64, and the terms that underflow are below 2^-42 of the sum; an
+// overflow leaves inf or NaN in the sum, so nothing outside can pass).  attn_fwd_bf16_redo_kernel, launched behind it,
+// computes the others again with a running maximum.
 template <int QMODE>
 __global__ __launch_bounds__(256, 2) void attn_fwd_bf16_x16_kernel(const AttnKernArgs a) {
+  constexpr bool CHECK = QMODE == Q_CHECK;
   constexpr int NW = 4, BM = 64 * NW;
   constexpr int LOADS = BN / (4 * NW);  // direct loads per wave per matrix per tile (4 rows each)
   constexpr int RING = 4;               // operand fragments in flight between LDS and the MFMAs
@@ -76,10 +102,12 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_bf16_x16_kernel(const AttnKer
   __shared__ __attribute__((aligned(1024))) unsigned char sK1[K_TILE_BYTES];
   __shared__ __attribute__((aligned(1024))) unsigned char sV1[V_TILE_BYTES];
   __shared__ int s_sel[LOCATE_WORDS];
+  __shared__ int s_over;  // CHECK: the first tile overflowed
 
   if (gate_closed(a)) return;
   const int tid = threadIdx.x;
-  const WorkItem wi = locate_work(a, BM, tid, s_sel);
+  if (CHECK && tid == 0) s_over = 0;
+  const WorkItem wi = locate_work(a, BM, tid, s_sel, blockIdx.x);
   if (!wi.valid) return;
   const int qe = wi.qe, ks = wi.ks, ke = wi.ke;
 
@@ -90,6 +118,7 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_bf16_x16_kernel(const AttnKer
 #pragma unroll
     for (int b = 0; b < 2; ++b)
       if (row0 + 32 * b + (l & 31) < qe) store_empty_row(a, wi, row0 + 32 * b + (l & 31), l >> 5);
+    if (CHECK && l == 0) a.verdict[4 * (long)wi.item + w] = 0;
     return;
   }
 
@@ -253,17 +282,10 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_bf16_x16_kernel(const AttnKer
     auto read_op = [&](auto oc) __attribute__((always_inline)) -> bf16x8 {
       constexpr int o = decltype(oc)::value;
       constexpr int t = o >> 4, j = o & 15;
-      if constexpr (j < 8) {  // K rows 32 t + 16 kb + n, features 32 kk + 8 g .. +8
-        constexpr int kb = j >> 2, kk = j & 3;
-        return *LDS_PTR(const bf16x8, Kt + (base_k + kk * 64 + (8 * t + 4 * kb) * K_GROUP));
-      } else {  // V^T: feature block db, the two 16-key blocks of half t
-        constexpr int db = v_block(j - 8);
-        const int bv = swz<((db & 3) << 5), 16 * t + (db & 3)>(base_v, k0) + (db >> 2) * 128;
-        const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(LDS_PTR(s16x4, Vt + (bv + (8 * t) * V_GROUP)));
-        const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(LDS_PTR(s16x4, Vt + (bv + (8 * t + 4) * V_GROUP)));
-        const s16x8 va = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-        return __builtin_bit_cast(bf16x8, va);
-      }
+      if constexpr (j < 8)
+        return read_k<2 * t + (j >> 2), (j & 3)>(Kt, base_k);
+      else
+        return read_v<t, v_block(j - 8)>(Vt, base_v, k0);
     };
     constexpr int RD = RING;
     bf16x8 ring[RD];
@@ -282,8 +304,9 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_bf16_x16_kernel(const AttnKer
         constexpr int kb = decltype(kc)::value, qb = decltype(qc)::value;
         // Row sums in fp32 by plain additions on the unrounded values (rounding to bf16 is unbiased, so this is as
         // good a denominator; dot instructions would hold the matrix pipe up)
-        const float p0 = __builtin_amdgcn_exp2f(sc[kb][qb][0]), p1 = __builtin_amdgcn_exp2f(sc[kb][qb][1]);
-        const float p2 = __builtin_amdgcn_exp2f(sc[kb][qb][2]), p3 = __builtin_amdgcn_exp2f(sc[kb][qb][3]);
+        const float c = CHECK ? a.scale_log2 : 1.f;
+        const float p0 = __builtin_amdgcn_exp2f(sc[kb][qb][0] * c), p1 = __builtin_amdgcn_exp2f(sc[kb][qb][1] * c);
+        const float p2 = __builtin_amdgcn_exp2f(sc[kb][qb][2] * c), p3 = __builtin_amdgcn_exp2f(sc[kb][qb][3] * c);
         l_run[qb] += (p0 + p1) + (p2 + p3);
         pf[qb][2 * kb] = pack_bf16x2(p0, p1);
         pf[qb][2 * kb + 1] = pack_bf16x2(p2, p3);
@@ -371,27 +394,44 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_bf16_x16_kernel(const AttnKer
     compute_tile(B ? sK1 : sK0, B ? sV1 : sV0, ks + cur * BN, ragged);
   };
   step(last, 0, slot0, std::true_type{});
+  int end = last;
+  if constexpr (CHECK) {
+    // Inputs with large scores throughout show it in the first tile: no need to go on (a sum that is too small so far
+    // may still grow; an overflow is final).
+    bool over = false;
+#pragma unroll
+    for (int qb = 0; qb < 4; ++qb) over |= !(l_run[qb] <= SUM_MAX);
+    if (wave_on && over) s_over = 1;
+    __syncthreads();
+    if (__builtin_amdgcn_readfirstlane(s_over) != 0) {
+      end = 0;
+      wait_vmcnt<0>();  // (the next tile is on its way into LDS)
+    }
+  }
   int j = 0;
-  for (; j + 1 < last; j += 2) {
+  for (; j + 1 < end; j += 2) {
     step(j, j + 1, slot1, std::false_type{});
     step(j + 1, j + 2, slot0, std::false_type{});
   }
-  if (j < last) step(j, j + 1, slot1, std::false_type{});
+  if (j < end) step(j, j + 1, slot1, std::false_type{});
 
   // ---- epilogue: normalise, transpose through LDS, store whole rows ----
   __syncthreads();  // every wave is done with the tile slots: wave w takes slot w as its 64 x 256-byte staging area
-  if (!wave_on) return;
+  if (!wave_on) {
+    if (CHECK && l == 0) a.verdict[4 * (long)wi.item + w] = 0;
+    return;
+  }
   unsigned char* const stage = w == 0 ? sK0 : w == 1 ? sV0 : w == 2 ? sK1 : sV1;
   int lane_e = l;
   asm volatile("" : "+v"(lane_e));
   const int ne = lane_e & 15, ge = lane_e >> 4;
-  float l_tot[4];
+  bool bad = false;
 #pragma unroll
   for (int qb = 0; qb < 4; ++qb) {
     float s = l_run[qb];
     s += __shfl_xor(s, 16);
     s += __shfl_xor(s, 32);
-    l_tot[qb] = s;
+    if constexpr (CHECK) bad |= end != last || !(s >= SUM_MIN && s <= SUM_MAX);
     const float inv = 1.f / s;
     // lane (ne, ge) holds O[row 16 qb + ne][d = 16 db + 4 ge + r]: 8 bytes of bf16 at byte 32 db + 8 ge of the row,
     // i.e. half (ge & 1) of 16-byte chunk 2 db + ge / 2, kept at chunk ^ (row & 15) = chunk ^ ne
@@ -405,6 +445,10 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_bf16_x16_kernel(const AttnKer
     const int q_row = row0 + 16 * qb + ne;
     if (a.lse && ge == 0 && q_row < qe)
       a.lse[(long)wi.h * a.total_q + q_row] = __builtin_amdgcn_logf(s) * 0.6931471805599453f;
+  }
+  if constexpr (CHECK) {
+    const bool any = __builtin_amdgcn_ballot_w64(bad) != 0;
+    if (lane_e == 0) a.verdict[4 * (long)wi.item + w] = any ? 1 : 0;
   }
   // (the staging area is this wave's own: its LDS operations complete in order, no workgroup barrier is needed)
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -420,6 +464,184 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_bf16_x16_kernel(const AttnKer
   }
 }
 
+// The rows that a CHECK launch of the kernel above could not be trusted with, again, with a running maximum: same ranges,
+// tiles and items.  A workgroup goes through every gridDim.x-th block of that launch, 64 verdicts at a time, and does the
+// flagged ones (usually none: the launch then costs one look at 16 bytes per 256 rows and head).  32 rows per wavefront
+// at a time, the two halves of its 64 one after the other.  The maximum of a row is raised only when a score comes out
+// more than RAISE above it: within that sums and products keep their full precision, and rescaling the accumulators is
+// rare.
+__global__ __launch_bounds__(256, 2) void attn_fwd_bf16_redo_kernel(const AttnKernArgs a) {
+  constexpr int NW = 4, BM = 64 * NW, LOADS = BN / (4 * NW);
+  constexpr float RAISE = 32.f;
+  __shared__ __attribute__((aligned(1024))) unsigned char sK0[K_TILE_BYTES];
+  __shared__ __attribute__((aligned(1024))) unsigned char sV0[V_TILE_BYTES];
+  __shared__ __attribute__((aligned(1024))) unsigned char sK1[K_TILE_BYTES];
+  __shared__ __attribute__((aligned(1024))) unsigned char sV1[V_TILE_BYTES];
+  __shared__ int s_sel[LOCATE_WORDS];
+  const int tid = threadIdx.x, l = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const unsigned blocks = 8u * a.per_xcd;
+  for (unsigned base = blockIdx.x; base < blocks; base += 64u * gridDim.x) {
+    const unsigned mine = base + (unsigned)l * gridDim.x;
+    unsigned kvh, hg, rslot, tile_;
+    bool flagged = false;
+    if (mine < blocks && decode_block(a, mine, kvh, hg, rslot, tile_)) {
+      const u32x4 v = *(const u32x4*)(a.verdict + 4 * (long)item_of(a, kvh, hg, rslot, tile_));
+      flagged = (v[0] | v[1] | v[2] | v[3]) != 0;
+    }
+    for (unsigned long todo = __builtin_amdgcn_ballot_w64(flagged); todo; todo &= todo - 1) {
+      __syncthreads();  // (s_sel and the tile slots are free again)
+      const WorkItem wi = locate_work(a, BM, tid, s_sel, base + (unsigned)__builtin_ctzl(todo) * gridDim.x);
+      if (!wi.valid || wi.ke <= wi.ks) continue;  // (a tile beyond its range has no verdict; one without keys is done)
+      const int qe = wi.qe, ks = wi.ks, ke = wi.ke, n_tiles = (ke - ks + BN - 1) / BN;
+      const int row0 = wi.q0 + 64 * w;
+      const bool wave_on = row0 < qe && __builtin_amdgcn_readfirstlane(a.verdict[4 * (long)wi.item + w]) != 0;
+      // one row per 16 lanes, four rows per load, each row through the segment it lives in, clamped to the last key
+      auto issue_mat = [&](int k0, unsigned char* tile_base, bool is_v) __attribute__((always_inline)) {
+        const long st = is_v ? a.vs_t : a.ks_t;
+        const char* const col = is_v ? a.v + (long)wi.kvh * a.vs_h : a.k + (long)wi.kvh * a.ks_h;
+        const char* const col2 = is_v ? a.v2 + (long)wi.kvh * a.vs_h : a.k2 + (long)wi.kvh * a.ks_h;
+        const int group = is_v ? V_GROUP : K_GROUP, lr = l >> 4, sl = l & 15;
+        const int chunk = is_v ? (sl ^ (lr << 1)) : (sl ^ lr);
+#pragma unroll
+        for (int j = 0; j < LOADS; ++j) {
+          const int row = min(k0 + 4 * w + lr + 4 * NW * j, ke - 1);
+          const char* p = row < a.k_split ? col + (long)row * st : col2 + (long)(row - a.k_split) * st;
+          __builtin_amdgcn_global_load_lds(GLOBAL_PTR(p + chunk * 16), LDS_PTR(void, tile_base + (w + NW * j) * group), 16, 0, 0);
+        }
+      };
+#pragma nounroll
+      for (int half = 0; half < 2; ++half) {
+        const int rh = row0 + 32 * half;
+        const bool on = wave_on && rh < qe;
+        const int n = l & 15, g = l >> 4;
+        const int base_k = (n >> 2) * K_GROUP + (n & 3) * ROW_BYTES + ((g ^ (n & 3)) << 4);
+        const int base_v = g * V_GROUP + (n >> 2) * ROW_BYTES + ((n >> 2) << 5) + ((n & 3) << 3);
+        bf16x8 q2[2][4];
+#pragma unroll
+        for (int qb = 0; qb < 2; ++qb) {
+          const int qr = min(rh + 16 * qb + n, qe - 1);
+          const char* qp = a.q + row_offset(a, qr, a.qs_t, a.qs_b) + (long)wi.h * a.qs_h + g * 16;
+#pragma unroll
+          for (int kk = 0; kk < 4; ++kk) q2[qb][kk] = *(const bf16x8*)(qp + kk * 64);
+        }
+        f32x4v o2[8][2];
+#pragma unroll
+        for (int db = 0; db < 8; ++db)
+#pragma unroll
+          for (int qb = 0; qb < 2; ++qb) o2[db][qb] = f32x4v{0.f, 0.f, 0.f, 0.f};
+        float sum2[2] = {0.f, 0.f}, m2[2] = {0.f, 0.f};
+        bool first = true;
+        auto tile = [&](const unsigned char* Kt, const unsigned char* Vt, int k0) __attribute__((always_inline)) {
+          static_for<0, 2>([&](auto tc) __attribute__((always_inline)) {
+            constexpr int t = decltype(tc)::value;
+            if (k0 + 32 * t >= ke) return;
+            f32x4v s2[2][2];
+            static_for<0, 2>([&](auto kc) __attribute__((always_inline)) {
+              constexpr int kb = decltype(kc)::value;
+#pragma unroll
+              for (int qb = 0; qb < 2; ++qb) s2[kb][qb] = f32x4v{0.f, 0.f, 0.f, 0.f};
+              static_for<0, 4>([&](auto kkc) __attribute__((always_inline)) {
+                const bf16x8 kf = read_k<2 * t + kb, decltype(kkc)::value>(Kt, base_k);
+#pragma unroll
+                for (int qb = 0; qb < 2; ++qb)
+                  s2[kb][qb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, q2[qb][decltype(kkc)::value], s2[kb][qb], 0, 0, 0);
+              });
+            });
+            float mx[2];
+            bool up = first;
+#pragma unroll
+            for (int qb = 0; qb < 2; ++qb) {
+              mx[qb] = -__builtin_inff();
+#pragma unroll
+              for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                  s2[kb][qb][r] = s2[kb][qb][r] * a.scale_log2 - m2[qb];
+                  if (k0 + 32 * t + 16 * kb + 4 * g + r >= ke) s2[kb][qb][r] = -__builtin_inff();  // (the ragged end)
+                  mx[qb] = fmaxf(mx[qb], s2[kb][qb][r]);
+                }
+              up |= __builtin_amdgcn_ballot_w64(mx[qb] > RAISE) != 0;
+            }
+            if (up) {
+#pragma unroll
+              for (int qb = 0; qb < 2; ++qb) {
+                float m = fmaxf(mx[qb], __shfl_xor(mx[qb], 16));  // (the four lanes of a query)
+                m = fmaxf(m, __shfl_xor(m, 32));
+                const float delta = (first || m > RAISE) ? m : 0.f;
+                const float alpha = first ? 1.f : __builtin_amdgcn_exp2f(-delta);
+                m2[qb] += delta;
+                sum2[qb] *= alpha;
+#pragma unroll
+                for (int kb = 0; kb < 2; ++kb) s2[kb][qb] -= delta;
+#pragma unroll
+                for (int db = 0; db < 8; ++db) o2[db][qb] *= alpha;
+              }
+              first = false;
+            }
+            u32x4 p2[2];
+#pragma unroll
+            for (int qb = 0; qb < 2; ++qb)
+#pragma unroll
+              for (int kb = 0; kb < 2; ++kb) {
+                float p[4];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) p[r] = __builtin_amdgcn_exp2f(s2[kb][qb][r]);
+                sum2[qb] += (p[0] + p[1]) + (p[2] + p[3]);
+                p2[qb][2 * kb] = pack_bf16x2(p[0], p[1]);
+                p2[qb][2 * kb + 1] = pack_bf16x2(p[2], p[3]);
+              }
+            __builtin_amdgcn_sched_barrier(0);
+            static_for<0, 8>([&](auto dbc) __attribute__((always_inline)) {
+              const bf16x8 vf = read_v<t, decltype(dbc)::value>(Vt, base_v, k0);
+#pragma unroll
+              for (int qb = 0; qb < 2; ++qb)
+                o2[decltype(dbc)::value][qb] =
+                    __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, __builtin_bit_cast(bf16x8, p2[qb]), o2[decltype(dbc)::value][qb], 0, 0, 0);
+            });
+          });
+        };
+        __syncthreads();  // (every wave is done with the tile slots of the half before)
+        issue_mat(ks, sK0, false);
+        issue_mat(ks, sV0, true);
+        for (int j = 0; j < n_tiles; j += 2) {
+          wait_vmcnt<0>();
+          __syncthreads();
+          if (j + 1 < n_tiles) {
+            issue_mat(ks + (j + 1) * BN, sK1, false);
+            issue_mat(ks + (j + 1) * BN, sV1, true);
+          }
+          if (on) tile(sK0, sV0, ks + j * BN);
+          if (j + 1 >= n_tiles) break;
+          wait_vmcnt<0>();
+          __syncthreads();
+          if (j + 2 < n_tiles) {
+            issue_mat(ks + (j + 2) * BN, sK0, false);
+            issue_mat(ks + (j + 2) * BN, sV0, true);
+          }
+          if (on) tile(sK1, sV1, ks + (j + 1) * BN);
+        }
+        if (!on) continue;
+#pragma unroll
+        for (int qb = 0; qb < 2; ++qb) {
+          float sum = sum2[qb];
+          sum += __shfl_xor(sum, 16);
+          sum += __shfl_xor(sum, 32);
+          const float inv = 1.f / sum;
+          const int q_row = rh + 16 * qb + n;
+          if (q_row >= qe) continue;
+          char* const op = a.out + row_offset(a, q_row, a.os_t, a.os_b) + wi.o_head + 8 * g;
+#pragma unroll
+          for (int db = 0; db < 8; ++db)
+            *(u32x2*)(op + 32 * db) = u32x2{pack_bf16x2(o2[db][qb][0] * inv, o2[db][qb][1] * inv),
+                                            pack_bf16x2(o2[db][qb][2] * inv, o2[db][qb][3] * inv)};
+          if (a.lse && g == 0) a.lse[(long)wi.h * a.total_q + q_row] = (m2[qb] + __builtin_amdgcn_logf(sum)) * 0.6931471805599453f;
+        }
+      }
+    }
+  }
+}
+
 }  // namespace
 
 hipError_t launch_attn_fwd_bf16_x16(const AttnKernArgs& a, hipStream_t stream) {
@@ -430,6 +652,16 @@ hipError_t launch_attn_fwd_bf16_x16(const AttnKernArgs& a, hipStream_t stream) {
     hipLaunchKernelGGL(attn_fwd_bf16_x16_kernel<Q_SCALE>, grid, dim3(256), 0, stream, a);
   else
     hipLaunchKernelGGL(attn_fwd_bf16_x16_kernel<Q_AS_IS>, grid, dim3(256), 0, stream, a);
+  return hipGetLastError();
+}
+
+hipError_t launch_attn_fwd_bf16_checked(const AttnKernArgs& a, int compute_units, hipStream_t stream) {
+  const dim3 grid(a.per_xcd * 8u);
+  // (two workgroups per CU, a multiple of eight so that a block keeps its XCD)
+  const unsigned most = (unsigned)(compute_units / 4) * 8u;
+  const dim3 again(grid.x < most || most == 0 ? grid.x : most);
+  hipLaunchKernelGGL(attn_fwd_bf16_x16_kernel<Q_CHECK>, grid, dim3(256), 0, stream, a);
+  hipLaunchKernelGGL(attn_fwd_bf16_redo_kernel, again, dim3(256), 0, stream, a);
   return hipGetLastError();
 }
 

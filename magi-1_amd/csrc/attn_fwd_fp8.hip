@@ -48,7 +48,7 @@ __global__ __launch_bounds__(64 * NW, 3) void attn_fwd_fp8_kernel(const AttnKern
   __shared__ int s_sel[LOCATE_WORDS];
 
   const int tid = threadIdx.x;
-  const WorkItem wi = locate_work(a, BM, tid, s_sel);
+  const WorkItem wi = locate_work(a, BM, tid, s_sel, blockIdx.x);
   if (!wi.valid) return;
   const int h = wi.h, kvh = wi.kvh, q0 = wi.q0, qe = wi.qe, ks = wi.ks, ke = wi.ke;
   const long o_head = wi.o_head;

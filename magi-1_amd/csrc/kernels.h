@@ -46,6 +46,8 @@ struct AttnKernArgs {
   // gate_want (the bounded-score kernel: 1, the online-softmax kernel launched behind it: 0).  NULL: no test.
   const float* gate;
   int gate_want;
+  // Checked launches (MAGI_ATTN_CHECKED): four words per item, one per wavefront of the 256-row kernel
+  int* verdict;
 };
 
 
@@ -59,6 +61,8 @@ constexpr int ATTN_ZERO_GAPS = 32;
 hipError_t launch_attn_fwd_bf16(const AttnKernArgs& a, hipStream_t stream);
 hipError_t launch_attn_fwd_bf16_w64(const AttnKernArgs& a, hipStream_t stream);
 hipError_t launch_attn_fwd_bf16_x16(const AttnKernArgs& a, hipStream_t stream);
+// the bounded-score kernel without a promise, and behind it the launch that repeats what it could not be trusted with
+hipError_t launch_attn_fwd_bf16_checked(const AttnKernArgs& a, int compute_units, hipStream_t stream);
 hipError_t launch_attn_fwd_fp8(const AttnKernArgs& a, hipStream_t stream);
 // ws[0..3] = 0 (a kernel, not a memset: the call may be under graph capture)
 hipError_t launch_gate_init(unsigned* ws, hipStream_t stream);

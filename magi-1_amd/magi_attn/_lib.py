@@ -25,6 +25,7 @@ MAGI_ATTN_FP8_FAST_EXP2 = 4
 MAGI_ATTN_BOUNDED_MFMA32 = 8
 MAGI_ATTN_AUTO_BOUND = 16
 MAGI_ATTN_ZERO_UNCOVERED = 32
+MAGI_ATTN_CHECKED = 64
 MAGI_SCORE_BOUND_MAX = 64.0
 
 

@@ -89,6 +89,7 @@ def range_attention(
     q_tile_rows: int = 0,
     bounded_mfma32: bool = False,
     auto_bound: bool = False,
+    checked: bool = False,
     static_scratch: bool = False,
     q_norm: Optional[tuple] = None,
     out: Optional[torch.Tensor] = None,
@@ -117,6 +118,8 @@ def range_attention(
     picks the bounded-score kernel on the device when their product allows it, MAGI_ATTN_AUTO_BOUND.  Its 16-byte
     workspace is a fresh tensor, or with static_scratch the library's own device array (magi_attn_fwd_static_scratch:
     no allocation at all when `out` is given and return_lse is False; such calls must not overlap on one GPU).
+    checked (bf16, instead of score_bound): the bounded-score kernel judges by its row sums whether the scores were
+    bounded, and a second launch repeats the blocks of rows where they were not, MAGI_ATTN_CHECKED.
     q may be [batch, rows, Hq, D] with any batch stride (batch of activations laid out [position, batch, ...]): its rows
     count as batch * rows tokens for the ranges, out is (or comes back as) a tensor of q's shape, by default
     [rows, batch, Hq, D] transposed.  Needs a score_bound in force.
@@ -194,8 +197,11 @@ def range_attention(
     o_stride_t = o_stride[0] if group_heads else o_stride[-3]
     flags = ((L.MAGI_ATTN_FP8_POW2_PRESCALED if fp8_pow2_prescaled else 0) | (L.MAGI_ATTN_Q_PRESCALED if q_prescaled else 0)
              | (L.MAGI_ATTN_FP8_FAST_EXP2 if fp8_fast_exp2 else 0) | (L.MAGI_ATTN_BOUNDED_MFMA32 if bounded_mfma32 else 0)
-             | (L.MAGI_ATTN_AUTO_BOUND if auto_bound else 0) | (L.MAGI_ATTN_ZERO_UNCOVERED if zero_gaps else 0))
+             | (L.MAGI_ATTN_AUTO_BOUND if auto_bound else 0) | (L.MAGI_ATTN_ZERO_UNCOVERED if zero_gaps else 0)
+             | (L.MAGI_ATTN_CHECKED if checked else 0))
     workspace = None
+    if checked:
+        workspace = torch.empty(max(4 * Hq * max(n, 0) * ((int(max_seqlen_q) + 255) // 256), 4), dtype=torch.int32, device=q.device)
     if auto_bound and not static_scratch:
         workspace = torch.empty(4, dtype=torch.float32, device=q.device)  # (alive until the launches are enqueued)
     gamma = beta = None  # (alive until the launch is enqueued)
@@ -241,6 +247,35 @@ def _measuring_a_bound_pays(q, k, n_ranges: int, max_seqlen_q: int, max_seqlen_k
     return 0.12 * attention_s > 2 * passes_s
 
 
+def _checking_pays(Hq: int, n_ranges: int, max_seqlen_q: int, keys: float, device) -> bool:
+    """A bf16 call without a score_bound: does the checked bounded-score kernel (256-row workgroups, a second launch
+    behind it; range_attention's checked) beat the online-softmax one (128- or 384-row workgroups)?  It does once its
+    workgroups come near filling the chip's slots, two per CU, and have more than a few tiles of keys each, or are many;
+    `keys` is the (average) length of a key range.  Measured, online against checked: 8880 workgroups over 400 keys 718 /
+    529 us; 1296 over 684 keys 137 / 125; 432 over 4600 keys 290 / 228; but 576 over 400 keys 47 / 51, 144 over 1536 keys
+    52 / 55, 864 over 60 keys 29 / 33."""
+    workgroups = Hq * n_ranges * ((max_seqlen_q + 255) // 256)
+    return keys >= 96 and workgroups >= (1.6 if keys >= 512 else 4) * torch.cuda.get_device_properties(device).multi_processor_count
+
+
+def _unbounded_mode(q, k, n_ranges: int, max_seqlen_q: int, max_seqlen_k: int, keys: float, score_bound: float,
+                    auto_bound: Optional[bool]) -> dict:
+    """How a reference-shaped callable runs: with the bound it was given, as it was told to (auto_bound), with a measured
+    bound where the two passes are small beside the attention, or checked where that pays."""
+    if score_bound != 0.0:
+        return {"score_bound": score_bound}
+    if auto_bound is not None:
+        return {"auto_bound": bool(auto_bound)}
+    if q.dtype != torch.bfloat16 or not q.is_cuda:
+        return {}
+    fills = _checking_pays(q.shape[-2], n_ranges, max_seqlen_q, keys, q.device)
+    # (below that, ranges of unequal length leave the 256-row workgroups' last round to the longest one: 240 of them over
+    # four ranges of up to 35000 keys 961 us measured against 854 us online; 216 over one range 1222 against 1320)
+    if (fills or n_ranges == 1) and _measuring_a_bound_pays(q, k, n_ranges, max_seqlen_q, max_seqlen_k):
+        return {"auto_bound": True}
+    return {"checked": True} if fills else {}
+
+
 def flex_flash_attn_func(q, k, v, q_ranges, k_ranges, max_seqlen_q, max_seqlen_k, softmax_scale=None,
                          deterministic=False, disable_fwd_atomic_reduction=True, score_bound: float = 0.0,
                          auto_bound: Optional[bool] = None, **_unused):
@@ -253,12 +288,13 @@ def flex_flash_attn_func(q, k, v, q_ranges, k_ranges, max_seqlen_q, max_seqlen_k
     without a running maximum, which applies the scale while it loads q.
 
     auto_bound: without a score_bound the library can measure one (range_attention's auto_bound).  None (default):
-    it does where the two passes over q and k are small beside the attention itself, which is how the reference's
-    own call, unchanged, reaches the bounded-score kernel on its QK-normed q and k."""
-    if auto_bound is None:
-        auto_bound = score_bound == 0.0 and _measuring_a_bound_pays(q, k, q_ranges.shape[0], max_seqlen_q, max_seqlen_k)
-    return range_attention(q, k, v, q_ranges, k_ranges, max_seqlen_q, max_seqlen_k, softmax_scale,
-                           score_bound=score_bound, auto_bound=bool(auto_bound) and score_bound == 0.0)
+    it does where the two passes over q and k are small beside the attention itself, and launches below that which still
+    fill the chip take the bounded-score kernel that checks itself (range_attention's checked): that is how the
+    reference's own call, unchanged, runs on its QK-normed q and k.  True / False: measure always / take the
+    online-softmax kernel."""
+    mode = _unbounded_mode(q, k, q_ranges.shape[0], max_seqlen_q, max_seqlen_k,
+                           max_seqlen_k if max_seqlen_k > 0 else k.shape[0], score_bound, auto_bound)
+    return range_attention(q, k, v, q_ranges, k_ranges, max_seqlen_q, max_seqlen_k, softmax_scale, **mode)
 
 
 def flash_attn_func(q, k, v, dropout_p=0.0, softmax_scale=None, causal=False, deterministic=False,
@@ -274,11 +310,9 @@ def flash_attn_func(q, k, v, dropout_p=0.0, softmax_scale=None, causal=False, de
     v3 = v.reshape(B * Sk, v.shape[2], D)
     cu_q = torch.arange(0, (B + 1) * Sq, Sq, dtype=torch.int32, device=q.device)
     cu_k = torch.arange(0, (B + 1) * Sk, Sk, dtype=torch.int32, device=q.device)
-    if auto_bound is None:
-        auto_bound = score_bound == 0.0 and _measuring_a_bound_pays(q3, k3, B, Sq, Sk)
+    mode = _unbounded_mode(q3, k3, B, Sq, Sk, Sk, score_bound, auto_bound)
     out, _ = range_attention(q3, k3, v3, cu_q, cu_k, Sq, Sk, softmax_scale, ranges_mode=L.MAGI_RANGES_CU,
-                             return_lse=False, zero_init=False, score_bound=score_bound,
-                             auto_bound=bool(auto_bound) and score_bound == 0.0)
+                             return_lse=False, zero_init=False, **mode)
     return out.view(B, Sq, Hq, D)
 
 
@@ -289,11 +323,10 @@ def flash_attn_varlen_func(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, ma
     A segment without keys yields zero rows.  score_bound, auto_bound: as in flex_flash_attn_func."""
     if dropout_p != 0.0 or causal:
         raise NotImplementedError("dropout / causal are not part of the MAGI-1 attention path")
-    if auto_bound is None:
-        auto_bound = score_bound == 0.0 and _measuring_a_bound_pays(q, k, cu_seqlens_q.numel() - 1, max_seqlen_q, max_seqlen_k)
+    n = cu_seqlens_q.numel() - 1
+    mode = _unbounded_mode(q, k, n, max_seqlen_q, max_seqlen_k, k.shape[0] / max(n, 1), score_bound, auto_bound)
     out, _ = range_attention(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, softmax_scale,
-                             ranges_mode=L.MAGI_RANGES_CU, return_lse=False, zero_init=True, score_bound=score_bound,
-                             auto_bound=bool(auto_bound) and score_bound == 0.0)
+                             ranges_mode=L.MAGI_RANGES_CU, return_lse=False, zero_init=True, **mode)
     return out
 
 

@@ -1,0 +1,139 @@
+"""GPU tests of the bounded-score kernel that checks itself (MAGI_ATTN_CHECKED): on inputs whose scores are bounded it gives
+the bits of the call with a stated bound; every 64-row block whose row sums leave the window is computed again with a
+running maximum, whatever the reason (scores too large or too small, in the first tile or later, non-finite inputs)."""
+import numpy as np
+import pytest
+import torch
+
+import magi_attn as M
+from magi_attn import functional as F
+from oracle import magi_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def _ranges(dev, *arrs):
+    return [torch.tensor(np.asarray(a), dtype=torch.int32, device=dev) for a in arrs]
+
+
+def _close(out, ref):
+    d = (out.float().cpu() - ref).abs()
+    assert torch.isfinite(out).all() and d.max().item() <= 2e-2, d.max().item()
+
+
+@pytest.mark.parametrize("L,dn,sp,Hq,Hkv", [(1, 3, 2, 6, 1), (64, 2, 1, 4, 2), (200, 3, 1, 6, 2), (333, 4, 3, 12, 4), (257, 2, 0, 3, 3)])
+def test_bounded_inputs_give_the_bits_of_a_stated_bound(dev, L, dn, sp, Hq, Hkv):
+    q, k, v = O.synthetic_qkv(dn * L, (sp + dn) * L, Hq, Hkv, 128, seed=L)
+    qr, kr = O.q_ranges_for(dn, L), O.default_kvrange(sp, dn, L)
+    tq, tk = _ranges(dev, qr, kr)
+    qp = (q.float() * (128 ** -0.5 * 1.4426950408889634)).bfloat16().to(dev)
+    kd, vd = k.to(dev), v.to(dev)
+    n0 = M.lib().magi_launch_count()
+    out, lse = M.range_attention(qp, kd, vd, tq, tk, L, checked=True, q_prescaled=True)
+    assert M.lib().magi_launch_count() - n0 == 2
+    want, lse_w = M.range_attention(qp, kd, vd, tq, tk, L, score_bound=17.0, q_prescaled=True)
+    assert torch.equal(out, want) and torch.equal(lse, lse_w)
+    # unscaled q: the scale is applied to the fp32 scores, q is not rounded a second time
+    out, lse = M.range_attention(q.to(dev), kd, vd, tq, tk, L, checked=True)
+    online, lse_o = M.range_attention(q.to(dev), kd, vd, tq, tk, L)
+    _close(out, O.range_attention(q, k, v, qr, kr))
+    assert (lse - lse_o).abs().max().item() <= 1e-3
+
+
+@pytest.mark.parametrize("where", ["everywhere", "first tile", "late tile", "one row", "tiny sums", "side segment"])
+@pytest.mark.parametrize("L,Tk", [(300, 700), (65, 64), (130, 1000)])
+def test_blocks_outside_the_window_are_computed_again(dev, where, L, Tk):
+    """Scores far above 64 (and, for tiny sums, all far below -64) in the places named, against the fp32 oracle; blocks
+    around them stay right.  lse against the online-softmax kernel's: both sum fp32 probabilities."""
+    Hq, Hkv = 4, 2
+    g = torch.Generator().manual_seed(L + Tk)
+    q = torch.randn(2 * L, Hq, 128, generator=g).bfloat16()
+    k = torch.randn(Tk, Hkv, 128, generator=g).bfloat16()
+    v = torch.randn(Tk, Hkv, 128, generator=g).bfloat16()
+    split = None
+    if where == "everywhere":
+        q = (q.float() * 12).bfloat16()
+    elif where == "first tile":  # the kernel starts with the last tile of the range
+        k[-3, 1] *= 40
+    elif where == "late tile":
+        k[5, 0] *= 40
+    elif where == "one row":
+        q[L + 1, 2] *= 40
+    elif where == "tiny sums":  # one direction shared by all keys, one query against it
+        k[:, 0] = (k[:, 0].float() * 0.05 + 8.0).bfloat16()
+        q[3, 0] = -8.0
+    else:
+        split = Tk // 2 + 3
+        k[split + 2, 1] *= 40
+    qr, kr = [[0, L], [L, 2 * L]], [[0, Tk], [0, Tk - 1]]
+    tq, tk = _ranges(dev, qr, kr)
+    qd, kd, vd = q.to(dev), k.to(dev), v.to(dev)
+    kw = {} if split is None else dict(k2=kd[split:], v2=vd[split:], k_split=split)
+    k1, v1 = (kd, vd) if split is None else (kd[:split], vd[:split])
+    out, lse = M.range_attention(qd, k1, v1, tq, tk, L, checked=True, **kw)
+    _close(out, O.range_attention(q, k, v, np.array(qr), np.array(kr)))
+    online, lse_o = M.range_attention(qd, k1, v1, tq, tk, L, **kw)
+    assert (lse - lse_o).abs().max().item() <= 1e-3 + 1e-6 * lse_o.abs().max().item()
+    # pre-scaled q, output in groups of heads
+    qp = (q.float() * (128 ** -0.5 * 1.4426950408889634)).bfloat16().to(dev)
+    buf = torch.zeros(2 * L, 2, 2, 2, 128, dtype=torch.bfloat16, device=dev)
+    M.range_attention(qp, k1, v1, tq, tk, L, checked=True, q_prescaled=True, out=buf[:, :, 0], return_lse=False, **kw)
+    plain, _ = M.range_attention(qp, k1, v1, tq, tk, L, q_prescaled=True, **kw)
+    assert (buf[:, :, 0].reshape(plain.shape).float() - plain.float()).abs().max().item() <= 2e-2  # (the same rounded q)
+    assert torch.count_nonzero(buf[:, :, 1]) == 0
+
+
+def test_non_finite_inputs_stay_where_they_belong(dev):
+    L, Hq, Hkv = 200, 4, 2
+    q, k, v = O.synthetic_qkv(2 * L, 2 * L, Hq, Hkv, 128, seed=3)
+    k[7, 1, 5] = float("nan")
+    q[L + 3, 0, 0] = float("inf")
+    tq, tk = _ranges(dev, [[0, L], [L, 2 * L]], [[0, L], [L, 2 * L]])
+    out, _ = M.range_attention(q.to(dev), k.to(dev), v.to(dev), tq, tk, L, checked=True)
+    nan = torch.isnan(out).any(-1).cpu()
+    want = torch.zeros_like(nan)
+    want[:L, 2:] = True   # every row that sees the key with a NaN
+    want[L + 3, 0] = True
+    assert torch.equal(nan, want)
+
+
+def test_many_ranges_empty_ranges_and_gaps(dev):
+    """More ranges than one wavefront (and than the workgroup) ranks, some without keys, some rows in no range."""
+    for n in (3, 65, 300):
+        g = torch.Generator().manual_seed(n)
+        lens = torch.randint(0, 70, (n,), generator=g).numpy()
+        starts = np.concatenate([[0], np.cumsum(lens + 3)])
+        qr = np.stack([starts[:-1], starts[:-1] + lens], 1)
+        ks = torch.randint(0, 300, (n,), generator=g).numpy()
+        kr = np.stack([ks, ks + np.where(np.arange(n) % 4 == 1, 0, 90)], 1)
+        Tq = int(starts[-1]) + 2
+        q, k, v = O.synthetic_qkv(Tq, 400, 3, 1, 128, seed=n)
+        q[::7] = (q[::7].float() * 12).bfloat16()
+        ref = O.range_attention(q, k, v, qr, kr)
+        out, _ = M.range_attention(q.to(dev), k.to(dev), v.to(dev), *_ranges(dev, qr, kr), 70, checked=True)
+        _close(out, ref)
+
+
+def test_reference_shaped_callables_check_where_it_pays(dev):
+    """varlen, flex and flash calls without a bound: two launches (checked) once the workgroups fill the chip, one below."""
+    assert F._checking_pays(24, 10, 9360, 400, dev) and not F._checking_pays(24, 10, 9360, 60, dev)
+    assert not F._checking_pays(24, 2, 1400, 400, dev)
+    L, n, Hq, Hkv = 2600, 4, 24, 8
+    q, k, v = (t.to(dev) for t in O.synthetic_qkv(n * L, n * 130, Hq, Hkv, 128, seed=9))
+    cq = torch.arange(0, (n + 1) * L, L, dtype=torch.int32, device=dev)
+    ck = torch.tensor([0, 130, 130, 390, 520], dtype=torch.int32, device=dev)
+    for launches, kw in ((2, {}), (1, {"auto_bound": False}), (1, {"score_bound": 17.0})):
+        n0 = M.lib().magi_launch_count()
+        out = M.flash_attn_varlen_func(q, k, v, cq, ck, L, 800, **kw)
+        assert M.lib().magi_launch_count() - n0 == launches
+        if launches == 2:
+            first = out
+    assert (first.float() - out.float()).abs().max().item() <= 2e-2 and torch.count_nonzero(first[L:2 * L]) == 0
+
+
+def test_checked_argument_checks(dev):
+    q = torch.zeros(8, 2, 128, dtype=torch.bfloat16, device=dev)
+    r = torch.tensor([[0, 8]], dtype=torch.int32, device=dev)
+    for kw in ({"score_bound": 10.0}, {"auto_bound": True}, {"q_tile_rows": 128}, {"static_scratch": True}):
+        with pytest.raises(M.MagiError):
+            M.range_attention(q, q, q, r, r, 8, checked=True, **kw)
