@@ -45,6 +45,11 @@ def _ptr(t: Optional[torch.Tensor]) -> int:
     return 0 if t is None else t.data_ptr()
 
 
+def _fp32(t: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
+    """t as a contiguous fp32 tensor (itself when it is one)."""
+    return t if t is None or (t.dtype is torch.float32 and t.is_contiguous()) else t.to(torch.float32).contiguous()
+
+
 def _check_thd(t: torch.Tensor, name: str) -> None:
     if t.dim() != 3:
         raise ValueError(f"{name} must be [tokens, heads, head_dim], got {tuple(t.shape)}")
@@ -207,8 +212,7 @@ def range_attention(
     gamma = beta = None  # (alive until the launch is enqueued)
     norm_eps, norm_kind = 0.0, 0
     if q_norm is not None:
-        gamma = q_norm[0].to(torch.float32).contiguous()
-        beta = None if q_norm[1] is None else q_norm[1].to(torch.float32).contiguous()
+        gamma, beta = _fp32(q_norm[0]), _fp32(q_norm[1])
         norm_eps = float(q_norm[2])
         norm_kind = int(q_norm[3]) if len(q_norm) > 3 else L.MAGI_NORM_LAYERNORM_1P
     k_stride, v_stride = k.stride(), v.stride()
@@ -346,8 +350,7 @@ def apply_rotary_emb(x, cos, sin, interleaved=False, inplace=False, **_unused):
         raise ValueError("inplace=True needs a contiguous x (a copy would be rotated instead of x)")
     xc = x.contiguous()
     y = xc if inplace else torch.empty_like(xc)
-    cosf = cos.to(torch.float32).contiguous()
-    sinf = sin.to(torch.float32).contiguous()
+    cosf, sinf = _fp32(cos), _fp32(sin)
     _launch(x.device, L.lib().magi_apply_rotary, xc.data_ptr(), cosf.data_ptr(), sinf.data_ptr(), y.data_ptr(), B, S, H, D, R2,
             int(x.dtype == torch.bfloat16))
     return y
@@ -387,8 +390,7 @@ def qk_prologue(q_raw, k_raw, v_raw, rope, gq, bq, gk, bk, *, Hq: int, Hkv: int,
         raise ValueError("kv_out is shorter than n_cache_rows")
     if kv_tail is not None and kv_tail.shape[0] < S - n_cache_rows:
         raise ValueError("kv_tail is shorter than S - n_cache_rows")
-    f32 = lambda t: None if t is None else t.to(torch.float32).contiguous()
-    gq, bq, gk, bk = f32(gq), f32(bq), f32(gk), f32(bk)
+    gq, bq, gk, bk = _fp32(gq), _fp32(bq), _fp32(gk), _fp32(bk)
     R2 = 0
     if rope is not None:
         if rope.dtype != torch.float32 or rope.dim() != 2 or rope.shape[0] * max(batch, 1) != S or not rope.is_contiguous():
@@ -436,8 +438,7 @@ def qk_prologue_fp8(q_raw, k_raw, rope, gq, bq, gk, bk, *, Hq: int, Hkv: int, q_
         raise ValueError("k_out is shorter than n_cache_rows")
     if k_tail is not None and k_tail.shape[0] < S - n_cache_rows:
         raise ValueError("k_tail is shorter than S - n_cache_rows")
-    f32 = lambda t: None if t is None else t.to(torch.float32).contiguous()
-    gq, bq, gk, bk = f32(gq), f32(bq), f32(gk), f32(bk)
+    gq, bq, gk, bk = _fp32(gq), _fp32(bq), _fp32(gk), _fp32(bk)
     R2 = 0
     if rope is not None:
         if rope.dtype != torch.float32 or rope.dim() != 2 or rope.shape[0] * max(batch, 1) != S or not rope.is_contiguous():
@@ -489,8 +490,7 @@ def qkv_proj_prologue(x: torch.Tensor, w: torch.Tensor, rope, gq, bq, gk, bk, *,
         raise ValueError("kv_out is shorter than n_cache_rows")
     if kv_tail is not None and kv_tail.shape[0] < S - n_cache_rows:
         raise ValueError("kv_tail is shorter than S - n_cache_rows")
-    f32 = lambda t: None if t is None else t.to(torch.float32).contiguous()
-    gq, bq, gk, bk = f32(gq), f32(bq), f32(gk), f32(bk)
+    gq, bq, gk, bk = _fp32(gq), _fp32(bq), _fp32(gk), _fp32(bk)
     R2 = 0
     if rope is not None:
         if rope.dtype != torch.float32 or rope.dim() != 2 or rope.shape[0] * max(batch, 1) != S or not rope.is_contiguous():
@@ -609,8 +609,7 @@ def head_norm(x: torch.Tensor, gamma, beta, eps: float = 1e-6, norm_kind: int = 
         raise TypeError("x must be bf16")
     S, H, D = x.shape
     y = torch.empty((S, H, D), dtype=torch.bfloat16, device=x.device)
-    g = None if gamma is None else gamma.to(torch.float32).contiguous()
-    b = None if beta is None else beta.to(torch.float32).contiguous()
+    g, b = _fp32(gamma), _fp32(beta)
     _launch(x.device, L.lib().magi_head_norm, x.data_ptr(), x.stride(0), x.stride(1), _ptr(g), _ptr(b), y.data_ptr(), S, H, D,
             int(norm_kind), float(eps))
     return y

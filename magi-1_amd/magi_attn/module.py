@@ -42,6 +42,14 @@ from .params import InferenceParams, ModelMetaArgs, PackedCrossAttnParams
 PROJ_GROUPS = 8  # head groups of the linear_proj input (hard-coded "hn=8", dit_module.py:1338)
 
 
+def _halves(kv: torch.Tensor, rows: int) -> Tuple[torch.Tensor, torch.Tensor]:
+    """(K, V) views [rows, H, D] of the first rows of an interleaved [tokens, H, 2*D] tensor."""
+    st, sh, _ = kv.stride()
+    D, off = kv.shape[2] // 2, kv.storage_offset()
+    size = (rows, kv.shape[1], D)
+    return kv.as_strided(size, (st, sh, 1), off), kv.as_strided(size, (st, sh, 1), off + D)
+
+
 def attn_linear_proj_input(core_attn_out: torch.Tensor, cross_attn_out: torch.Tensor) -> torch.Tensor:
     """[sq, b, Hq*D] x 2 -> [sq, b, 2*Hq*D] in "(hn n hd)" order: the concat + rearrange that precedes linear_proj
     in attn_linear_proj (dit_module.py:1336-1339), done with torch copies."""
@@ -198,10 +206,11 @@ class PerTensorQuantizedFp8Linear(torch.nn.Module):
 
     def forward_quantized(self, x8: torch.Tensor) -> torch.Tensor:
         """The GEMM alone, on an input that is already div_clamp_to(input, self.input_scale)."""
-        prefix = x8.shape[:-1]
-        y = torch._scaled_mm(x8.reshape(-1, self.in_features), self.weight[0].t(), scale_a=self.input_scale.reshape(-1)[:1],
-                             scale_b=self.weight_scale.reshape(-1)[:1], out_dtype=self.output_dtype)
-        return y.reshape(prefix + (self.out_features,))
+        p = self._parameters
+        x2 = x8 if x8.dim() == 2 else x8.reshape(-1, self.in_features)
+        y = torch._scaled_mm(x2, p["weight"][0].t(), scale_a=p["input_scale"].reshape(-1)[:1],
+                             scale_b=p["weight_scale"].reshape(-1)[:1], out_dtype=self.output_dtype)
+        return y if x2 is x8 else y.reshape(x8.shape[:-1] + (self.out_features,))
 
 
 class CustomLayerNormLinear(torch.nn.Module):
@@ -230,7 +239,8 @@ class CustomLayerNormLinear(torch.nn.Module):
             self._fuse_weights()
 
     def _projections(self):
-        return (self.q, self.k, self.v, self.qx)  # row order of the shared buffer
+        m = self._modules
+        return m["q"], m["k"], m["v"], m["qx"]  # row order of the shared buffer
 
     def _fuse_weights(self) -> torch.Tensor:
         """Move the four weights into one [2*out_q + 2*out_kv, in] buffer and make each parameter a view of it."""
@@ -240,48 +250,58 @@ class CustomLayerNormLinear(torch.nn.Module):
         for m, w in zip(self._projections(), ws):
             m.weight.data = fused[row:row + w.shape[0]]
             row += w.shape[0]
+        self.__dict__["_fused"] = fused
         return fused
 
     def fused_weight(self) -> torch.Tensor:
         """The [q | k | v | qx] weight as one tensor (rebuilt first if the parameters no longer share a buffer)."""
-        ws = [m.weight.data for m in self._projections()]
-        base = ws[0]
-        ptr = base.data_ptr()
-        shared = True
-        for w in ws:
-            shared &= (w.data_ptr() == ptr and w.is_contiguous() and w.dtype == base.dtype and w.device == base.device
-                       and w.untyped_storage().data_ptr() == base.untyped_storage().data_ptr())
-            ptr += w.numel() * w.element_size()
-        if not shared:
+        fused = self.__dict__.get("_fused")
+        if fused is None:
             return self._fuse_weights()
-        rows = sum(w.shape[0] for w in ws)
-        return base.as_strided((rows, base.shape[1]), (base.shape[1], 1))
+        # (the buffer is held, so memory inside it is nobody else's: parameters of its dtype that lie in it back to back
+        # are its rows)
+        ptr, rows, row_bytes = fused.data_ptr(), 0, fused.stride(0) * fused.element_size()
+        for m in self._projections():
+            w = m._parameters["weight"]
+            if w.data_ptr() != ptr or w.dtype is not fused.dtype or not w.is_contiguous():
+                return self._fuse_weights()
+            ptr += w.shape[0] * row_bytes
+            rows += w.shape[0]
+        return fused if rows == fused.shape[0] else self._fuse_weights()
+
+    def _qkvx_rows(self, x: torch.Tensor):
+        """The four projections of (already normalised) rows x [tokens, in] -> views (q, k, v, qx) [tokens, out]."""
+        if self.fp8_quant:
+            return tuple(m(x) for m in self._projections())
+        y = _linear_in_whole_rounds(x, self.fused_weight())
+        oq, okv = self.q.weight.shape[0], self.k.weight.shape[0]
+        return y.split((oq, okv, okv, oq), dim=-1)
 
     def forward_qkvx(self, hidden_states):
         """One GEMM for all four projections of the (already normalised) input -> views (q, k, v, qx) of one
         [..., 2*out_q + 2*out_kv] result.  (fp8_quant: four quantise + fp8 GEMM pairs, each with its own scales.)"""
-        if self.fp8_quant:
-            return self.q(hidden_states), self.k(hidden_states), self.v(hidden_states), self.qx(hidden_states)
-        y = _linear_in_whole_rounds(hidden_states, self.fused_weight())
-        oq, okv = self.q.weight.shape[0], self.k.weight.shape[0]
-        return y[..., :oq], y[..., oq:oq + okv], y[..., oq + okv:oq + 2 * okv], y[..., oq + 2 * okv:]
+        lead = hidden_states.shape[:-1]
+        return tuple(t.view(lead + (t.shape[-1],)) for t in self._qkvx_rows(hidden_states.reshape(-1, hidden_states.shape[-1])))
 
-    def forward_ln_qkvx(self, hidden_states):
-        """forward_qkvx(forward_ln(hidden_states)).  With fp8_quant the norm and the four input quantisers are one launch
-        that writes the e4m3 inputs of the four GEMMs only (layer_norm_div_clamp)."""
-        linears = self._projections()
-        if (self.fp8_quant and hidden_states.shape[-1] % 8 == 0 and hidden_states.shape[-1] <= 8192 and hidden_states.is_contiguous()
-                and all(type(m) is PerTensorQuantizedFp8Linear and m.input_scale.numel() == hidden_states.shape[-1] for m in linears)):
-            ln = self.layer_norm
-            x8 = layer_norm_div_clamp(hidden_states, ln.weight.detach(), ln.bias.detach(), [m.input_scale.detach() for m in linears], ln.eps)
-            return tuple(m.forward_quantized(x8[i]) for i, m in enumerate(linears))
-        return self.forward_qkvx(self.forward_ln(hidden_states))
+    def forward_ln_qkvx_rows(self, hidden_states):
+        """forward_qkvx(forward_ln(hidden_states)) as [tokens, out] rows.  With fp8_quant the norm and the four input
+        quantisers are one launch that writes the e4m3 inputs of the four GEMMs only (layer_norm_div_clamp)."""
+        cols = hidden_states.shape[-1]
+        if self.fp8_quant:
+            linears = self._projections()
+            if (cols % 8 == 0 and cols <= 8192 and hidden_states.is_contiguous()
+                    and all(type(m) is PerTensorQuantizedFp8Linear and m.input_scale.numel() == cols for m in linears)):
+                ln = self.layer_norm
+                x8 = layer_norm_div_clamp(hidden_states.view(-1, cols), ln.weight.detach(), ln.bias.detach(),
+                                          [m.input_scale.detach() for m in linears], ln.eps)
+                return tuple(m.forward_quantized(x) for m, x in zip(linears, x8.unbind(0)))
+        return self._qkvx_rows(self.forward_ln(hidden_states).view(-1, cols))
 
     def forward_ln(self, hidden_states):
         """LayerNorm of the layer input (dit_module.py:412-413) as one HIP launch; the parameters stay on the
         torch.nn.LayerNorm sub-module under the reference's names."""
-        ln = self.layer_norm
-        return layer_norm(hidden_states, ln.weight.detach(), ln.bias.detach(), ln.eps)
+        ln = self._modules["layer_norm"]
+        return layer_norm(hidden_states, ln._parameters["weight"], ln._parameters["bias"], ln.eps)
 
     def forward_q(self, hidden_states):
         return self.q(hidden_states)
@@ -356,7 +376,8 @@ class FullyParallelAttention(torch.nn.Module):
         MAGI_SCORE_BOUND_MAX the attention kernels then need no running maximum (magi_attn_args.score_bound);
         larger values make them fall back to it.  Computed once per set of parameter values (it reads them on the
         host) and cached until a parameter is modified or replaced (see invalidate_cached_parameters)."""
-        lns = (self.q_layernorm, self.k_layernorm, self.q_layernorm_xattn, self.k_layernorm_xattn)
+        m = self._modules
+        lns = (m["q_layernorm"], m["k_layernorm"], m["q_layernorm_xattn"], m["k_layernorm_xattn"])
         key = (lns[0].parameter_epoch(), lns[1].parameter_epoch(), lns[2].parameter_epoch(), lns[3].parameter_epoch())
         state = self.__dict__
         if state.get("_bounds_key") != key:
@@ -449,7 +470,7 @@ class FullyParallelAttention(torch.nn.Module):
         Hq, Hkv = self.num_attention_heads, self.num_query_groups_per_partition
         Lc = meta_args.clip_token_nums
         p = meta_args.core_attn_params
-        q_raw, k_raw, v_raw = (t.reshape(t.shape[0] * t.shape[1], -1) for t in raw)
+        q_raw, k_raw, v_raw = raw  # [S, n]
         S = q_raw.shape[0]
         dev = q_raw.device
         n_chunks = (S + Lc - 1) // Lc
@@ -547,14 +568,14 @@ class FullyParallelAttention(torch.nn.Module):
 
     def _fused_qkv(self, mixed_qqkv, cos_emb, sin_emb, want_q=True, kv_out=None, n_cache_rows=None, kv_tail=None,
                    raw=None, q_premul=1.0, rope=None):
-        """raw: (q_raw, k_raw, v_raw) already projected (views of forward_qkvx's result), else projected here.
+        """raw: (q_raw, k_raw, v_raw) already projected ([sq, b, n] or [sq * b, n] views), else projected here.
         q_premul: factor folded into q ahead of its rounding to bf16 (see qk_prologue).
         rope: the [S, 2*R2] sin | cos table when the caller has it in one piece (else built from the two halves)."""
         sq, b = mixed_qqkv.shape[0], mixed_qqkv.shape[1]
         S = sq * b
         Hq, Hkv = self.num_attention_heads, self.num_query_groups_per_partition
         if raw is not None:
-            q_raw, k_raw, v_raw = (t.reshape(S, -1) for t in raw)  # [sq, b, n] row-strided: still a view
+            q_raw, k_raw, v_raw = (t if t.dim() == 2 else t.reshape(S, -1) for t in raw)  # [sq, b, n] row-strided: still a view
         else:
             k_raw = self.linear_qkv.forward_k(mixed_qqkv).reshape(S, -1)
             v_raw = self.linear_qkv.forward_v(mixed_qqkv).reshape(S, -1)
@@ -564,8 +585,8 @@ class FullyParallelAttention(torch.nn.Module):
                 q_raw = k_raw[:, :0]
         if rope is None:
             rope = torch.cat([sin_emb, cos_emb], dim=-1).float().contiguous()
-        gq, bq = self.q_layernorm.gamma_beta_fp32()
-        gk, bk = self.k_layernorm.gamma_beta_fp32()
+        gq, bq = self._modules["q_layernorm"].gamma_beta_fp32()
+        gk, bk = self._modules["k_layernorm"].gamma_beta_fp32()
         q, kv, tail = qk_prologue(q_raw, k_raw, v_raw, rope, gq, bq, gk, bk, Hq=Hq if want_q else 0, Hkv=Hkv,
                                   eps=self.eps, kv_out=kv_out, n_cache_rows=n_cache_rows, kv_tail=kv_tail, batch=b,
                                   q_premul=q_premul)
@@ -692,10 +713,10 @@ class FullyParallelAttention(torch.nn.Module):
         out = out.view(b, sq, -1)
         return out.transpose(0, 1).contiguous() if b > 1 else out.view(sq, 1, -1)
 
-    def _cross_attention_fused(self, qx_raw: torch.Tensor, key_value_states: torch.Tensor,
+    def _cross_attention_fused(self, qx_raw: torch.Tensor, sq: int, b: int, key_value_states: torch.Tensor,
                                cross_attn_params: PackedCrossAttnParams, out: Optional[torch.Tensor],
                                bound: float) -> Optional[torch.Tensor]:
-        """Cross attention on the RAW qx projection [sq, b, Hq*D]: the attention kernel applies q_layernorm_xattn while it
+        """Cross attention on the RAW qx projection [sq * b, Hq*D]: the attention kernel applies q_layernorm_xattn while it
         loads q (no normalised copy of q in memory) and, the scores of normed q and k being bounded, runs without a
         running maximum; at batch > 1 it reads and writes the [position, batch] rows where they are.  Returns None
         when that path does not apply (then the caller takes get_xqkv + cross_attention); else the result, [sq, b, Hq, D]
@@ -703,17 +724,14 @@ class FullyParallelAttention(torch.nn.Module):
         if not (0.0 < bound <= L.MAGI_SCORE_BOUND_MAX):
             return None
         D = self.hidden_size_per_attention_head
-        sq, b = qx_raw.shape[0], qx_raw.shape[1]
-        if b == 1:
-            q = qx_raw.reshape(sq, -1, D)  # row-strided view of the projection
-        else:
-            q = qx_raw.view(sq, b, -1, D).transpose(0, 1)
-        kv = torch.nn.functional.linear(key_value_states, self.linear_kv_xattn.weight)
-        kv = kv.view(key_value_states.shape[0], -1, 2 * D)
-        gk, bk = self.k_layernorm_xattn.gamma_beta_fp32()
-        kx = head_norm(kv[..., :D], gk, bk, self.eps)
-        gq, bq = self.q_layernorm_xattn.gamma_beta_fp32()
-        o, _ = range_attention(q, kx, kv[..., D:], cross_attn_params.cu_seqlens_q, cross_attn_params.cu_seqlens_kv,
+        q = qx_raw.view(sq, -1, D) if b == 1 else qx_raw.view(sq, b, -1, D).transpose(0, 1)  # row-strided views of the projection
+        m = self._modules
+        kv = torch.nn.functional.linear(key_value_states, m["linear_kv_xattn"]._parameters["weight"])
+        k_, v_ = _halves(kv.view(key_value_states.shape[0], -1, 2 * D), kv.shape[0])
+        gk, bk = m["k_layernorm_xattn"].gamma_beta_fp32()
+        kx = head_norm(k_, gk, bk, self.eps)
+        gq, bq = m["q_layernorm_xattn"].gamma_beta_fp32()
+        o, _ = range_attention(q, kx, v_, cross_attn_params.cu_seqlens_q, cross_attn_params.cu_seqlens_kv,
                                cross_attn_params.max_seqlen_q, cross_attn_params.max_seqlen_kv,
                                ranges_mode=L.MAGI_RANGES_CU, out=out, return_lse=False, zero_init=True,
                                score_bound=bound, q_norm=(gq, bq, self.eps))
@@ -730,9 +748,9 @@ class FullyParallelAttention(torch.nn.Module):
         at batch 1 both attention launches write straight into it."""
         if rotary_pos_emb is None:
             raise ValueError("FullyParallelAttention needs rotary_pos_emb")
-        sin_emb, cos_emb = rotary_pos_emb.tensor_split(2, -1)
         # the incoming table already is the [sin | cos] layout the prologue takes
-        rope = rotary_pos_emb if (rotary_pos_emb.dtype == torch.float32 and rotary_pos_emb.is_contiguous()) else None
+        rope = rotary_pos_emb if (rotary_pos_emb.dtype == torch.float32 and rotary_pos_emb.is_contiguous()) else \
+            rotary_pos_emb.float().contiguous()
         bound_core, bound_cross = self.score_bounds(rotary_pos_emb.shape[-1] // 2)
         core_bound_kw = {"score_bound": bound_core}  # (above the limit: the online-softmax kernel, unless measured)
         measured = False
@@ -750,7 +768,7 @@ class FullyParallelAttention(torch.nn.Module):
         # which attention kernels this forward selects (diagnostics; the choice follows from the norm parameters)
         bounded = lambda b: "bounded-score, 64 rows per wavefront" if 0.0 < b <= L.MAGI_SCORE_BOUND_MAX \
             else "online softmax, 32 rows per wavefront"
-        self.last_forward_kernels = {
+        self.__dict__["last_forward_kernels"] = {
             "core": "fp8" if self.attention_dtype == "fp8" else
             ("measured bound: bounded-score or online softmax, chosen on the device" if measured else bounded(bound_core)),
             "core_score_bound": bound_core,
@@ -759,7 +777,7 @@ class FullyParallelAttention(torch.nn.Module):
         bs = hidden_states.shape[1]
         sq = hidden_states.shape[0]
         D = self.hidden_size_per_attention_head
-        one_launch = (self.fused_projection and self.attention_dtype == "bf16" and bs == 1 and rope is not None
+        one_launch = (self.fused_projection and self.attention_dtype == "bf16" and bs == 1
                       and rope.shape[-1] == 96 and hidden_states.shape[-1] % 64 == 0)
         if one_launch:
             # projections + prologue in one launch: nothing raw reaches memory (qx leaves unnormalised, as the
@@ -769,13 +787,13 @@ class FullyParallelAttention(torch.nn.Module):
         else:
             # all four projections in one GEMM; q / k / v feed the fused prologue as row-strided views of its result
             mixed_qqkv = hidden_states  # (only its shape is used from here on: every projection is in hand)
-            q_raw, k_raw, v_raw, qx_raw = self.linear_qkv.forward_ln_qkvx(hidden_states)
+            q_raw, k_raw, v_raw, qx_raw = self._modules["linear_qkv"].forward_ln_qkvx_rows(hidden_states)
             raw = (q_raw, k_raw, v_raw)
 
         def project(kv_out=None, n_cache_rows=None, kv_tail=None):
-            """-> (q [S, Hq, D] carrying the softmax scale, kv destination(s), qx_raw [sq, 1, Hq*D])"""
+            """-> (q [S, Hq, D] carrying the softmax scale, kv destination(s), qx_raw [sq * b, Hq*D])"""
             if not one_launch:
-                q_, kv_ = self._fused_qkv(mixed_qqkv, cos_emb, sin_emb, kv_out=kv_out, n_cache_rows=n_cache_rows,
+                q_, kv_ = self._fused_qkv(mixed_qqkv, None, None, kv_out=kv_out, n_cache_rows=n_cache_rows,
                                           kv_tail=kv_tail, raw=raw, q_premul=self._q_premul, rope=rope)
                 return q_, kv_, qx_raw
             gq_, bq_ = self.q_layernorm.gamma_beta_fp32()
@@ -784,9 +802,9 @@ class FullyParallelAttention(torch.nn.Module):
                 mixed_qqkv.view(sq, -1), self.linear_qkv.fused_weight(), rope, gq_, bq_, gk_, bk_,
                 Hq=self.num_attention_heads, Hkv=self.num_query_groups_per_partition, Hqx=self.num_attention_heads,
                 eps=self.eps, kv_out=kv_out, n_cache_rows=n_cache_rows, kv_tail=kv_tail, q_premul=self._q_premul)
-            return q_, (kv_ if tail_ is None else (kv_, tail_)), qx_.view(sq, 1, -1)
+            return q_, (kv_ if tail_ is None else (kv_, tail_)), qx_.view(sq, -1)
 
-        get_xqkv = lambda m, y: self.get_xqkv(m, y, qx_raw=qx_raw)
+        get_xqkv = lambda m, y: self.get_xqkv(m, y, qx_raw=qx_raw.view(sq, bs, -1))
         p = meta_args.core_attn_params
         Hq = self.num_attention_heads
         fused = None
@@ -803,11 +821,10 @@ class FullyParallelAttention(torch.nn.Module):
         if self.attention_dtype == "fp8":
             if bs != 1 or (use_cache and inference_params.max_batch_size != 1):
                 raise ValueError("the fp8 self-attention runs at batch 1")
-            rope8 = rope if rope is not None else torch.cat([sin_emb, cos_emb], dim=-1).float().contiguous()
-            core = self._core_attention_fp8(raw, rope8, inference_params, meta_args, use_cache, core_dst)
+            core = self._core_attention_fp8(raw, rope, inference_params, meta_args, use_cache, core_dst)
         elif not use_cache:
             q, kv, qx_raw = project()
-            core = self.core_attention(q, kv[..., :D], kv[..., D:], bs, meta_args, out=core_dst, q_prescaled=True,
+            core = self.core_attention(q, *_halves(kv, kv.shape[0]), bs, meta_args, out=core_dst, q_prescaled=True,
                                        **core_bound_kw)
         else:
             if bs != 1 or inference_params.max_batch_size != 1:
@@ -838,24 +855,25 @@ class FullyParallelAttention(torch.nn.Module):
             try:
                 q, _, qx_raw = project(kv_out=cache[start:], n_cache_rows=n_keep, kv_tail=tail)
                 split = start + n_keep
-                kc, vc = cache[:split, :, :D], cache[:split, :, D:]
+                kc, vc = _halves(cache, split)
                 if tail is None:
                     core, _ = range_attention(q, kc, vc, p.q_range, p.k_range, p.max_seqlen_q, p.max_seqlen_k,
                                               out=core_dst, return_lse=False, q_prescaled=True, **core_bound_kw)
                 else:
+                    k2, v2 = _halves(tail, tail.shape[0])
                     core, _ = range_attention(q, kc, vc, p.q_range, p.k_range, p.max_seqlen_q, p.max_seqlen_k,
-                                              k2=tail[:, :, :D], v2=tail[:, :, D:], k_split=split, out=core_dst,
+                                              k2=k2, v2=v2, k_split=split, out=core_dst,
                                               return_lse=False, q_prescaled=True, **core_bound_kw)
                 persisted = n_keep
             finally:
                 if offloaded is not None:  # the persisted rows go back to the host behind the attention launch
                     offloaded.release(start, persisted)
         if fused is not None:
-            if self._cross_attention_fused(qx_raw, key_value_states, meta_args.cross_attn_params, cross_dst, bound_cross) is None:
+            if self._cross_attention_fused(qx_raw, sq, bs, key_value_states, meta_args.cross_attn_params, cross_dst, bound_cross) is None:
                 self.cross_attention(mixed_qqkv, key_value_states, meta_args.cross_attn_params, get_xqkv, out=cross_dst)
             return fused
         core_attn_out = core.view(sq, bs, -1)
-        xo = self._cross_attention_fused(qx_raw, key_value_states, meta_args.cross_attn_params, None, bound_cross)
+        xo = self._cross_attention_fused(qx_raw, sq, bs, key_value_states, meta_args.cross_attn_params, None, bound_cross)
         if xo is not None:
             xattn_out = xo.reshape(sq, bs, -1)
         else:
