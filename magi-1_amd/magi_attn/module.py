@@ -59,6 +59,13 @@ def attn_linear_proj_input(core_attn_out: torch.Tensor, cross_attn_out: torch.Te
     return both.reshape(sq, b, 2 * hd)
 
 
+def _param(m: torch.nn.Module, name: str) -> torch.Tensor:
+    """m.<name>: straight from the parameters where it is one (attribute lookup on a module costs several times as much), else
+    whatever the attribute gives (parametrised, sharded and wrapped modules)."""
+    p = m._parameters.get(name)
+    return p if p is not None else getattr(m, name)
+
+
 class FusedLayerNorm(torch.nn.Module):
     """Parameter holder of a per-head LayerNorm with zero-centred gamma (dit_module.py:323-357).
     The arithmetic runs inside the fused kernels; forward() is the stand-alone form."""
@@ -77,7 +84,7 @@ class FusedLayerNorm(torch.nn.Module):
         parameter values (no launches on later calls) and kept until a parameter is modified or replaced."""
         # (a write through `.data` does not advance _version: callers that patch parameters that way call
         # invalidate_cached_parameters())
-        w, b = self._parameters["weight"], self._parameters["bias"]
+        w, b = _param(self, "weight"), _param(self, "bias")
         key = (id(w), w._version, w.data_ptr(), w.dtype, w.device, id(b), b._version, b.data_ptr(), b.dtype, b.device)
         state = self.__dict__
         if state.get("_gb_key") != key:
@@ -154,9 +161,11 @@ def _linear_in_whole_rounds(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     and 1367; where one call is fine (8000, 10000, 18720 rows) the two cost 0 to 2 % more.  With a single whole round
     ahead of it a long rest is slower apart (3500 and 4000 rows: 4 %), so the rest is then at most 0.6 of a round.  Column
     counts whose tiles do not divide the CUs (14336: 56 tiles) gain nothing on average and are left alone."""
-    rows, cols = x.numel() // x.shape[-1], w.shape[0]
+    cols = w.shape[0]
     tiles = cols // 256
-    if cols % 256 == 0 and w.shape[1] >= 1024 and x.is_contiguous() and not (torch.is_grad_enabled() and x.requires_grad):
+    if (cols % 256 == 0 and tiles and w.shape[1] >= 1024 and x.is_cuda and x.is_contiguous() and x.dtype is w.dtype
+            and not torch.is_autocast_enabled() and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad))):
+        rows = x.numel() // x.shape[-1]
         cus = torch.cuda.get_device_properties(x.device).multi_processor_count
         if tiles <= cus and cus % tiles == 0:
             round_rows = 256 * (cus // tiles)
@@ -206,10 +215,9 @@ class PerTensorQuantizedFp8Linear(torch.nn.Module):
 
     def forward_quantized(self, x8: torch.Tensor) -> torch.Tensor:
         """The GEMM alone, on an input that is already div_clamp_to(input, self.input_scale)."""
-        p = self._parameters
         x2 = x8 if x8.dim() == 2 else x8.reshape(-1, self.in_features)
-        y = torch._scaled_mm(x2, p["weight"][0].t(), scale_a=p["input_scale"].reshape(-1)[:1],
-                             scale_b=p["weight_scale"].reshape(-1)[:1], out_dtype=self.output_dtype)
+        y = torch._scaled_mm(x2, _param(self, "weight")[0].t(), scale_a=_param(self, "input_scale").reshape(-1)[:1],
+                             scale_b=_param(self, "weight_scale").reshape(-1)[:1], out_dtype=self.output_dtype)
         return y if x2 is x8 else y.reshape(x8.shape[:-1] + (self.out_features,))
 
 
@@ -250,38 +258,41 @@ class CustomLayerNormLinear(torch.nn.Module):
         for m, w in zip(self._projections(), ws):
             m.weight.data = fused[row:row + w.shape[0]]
             row += w.shape[0]
-        self.__dict__["_fused"] = fused
         return fused
 
     def fused_weight(self) -> torch.Tensor:
         """The [q | k | v | qx] weight as one tensor (rebuilt first if the parameters no longer share a buffer)."""
-        fused = self.__dict__.get("_fused")
-        if fused is None:
-            return self._fuse_weights()
-        # (the buffer is held, so memory inside it is nobody else's: parameters of its dtype that lie in it back to back
-        # are its rows)
-        ptr, rows, row_bytes = fused.data_ptr(), 0, fused.stride(0) * fused.element_size()
-        for m in self._projections():
-            w = m._parameters["weight"]
-            if w.data_ptr() != ptr or w.dtype is not fused.dtype or not w.is_contiguous():
+        ws = [_param(m, "weight") for m in self._projections()]
+        base = ws[0]
+        ptr, rows = base.data_ptr(), 0
+        row_bytes = base.shape[1] * base.element_size()
+        for w in ws:
+            if w.data_ptr() != ptr or w.dtype is not base.dtype or not w.is_contiguous():
                 return self._fuse_weights()
             ptr += w.shape[0] * row_bytes
             rows += w.shape[0]
-        return fused if rows == fused.shape[0] else self._fuse_weights()
-
-    def _qkvx_rows(self, x: torch.Tensor):
-        """The four projections of (already normalised) rows x [tokens, in] -> views (q, k, v, qx) [tokens, out]."""
-        if self.fp8_quant:
-            return tuple(m(x) for m in self._projections())
-        y = _linear_in_whole_rounds(x, self.fused_weight())
-        oq, okv = self.q.weight.shape[0], self.k.weight.shape[0]
-        return y.split((oq, okv, okv, oq), dim=-1)
+        # back to back, and all of it inside the first one's allocation
+        if base.untyped_storage().nbytes() - base.storage_offset() * base.element_size() < rows * row_bytes:
+            return self._fuse_weights()
+        return base.data.as_strided((rows, base.shape[1]), (base.shape[1], 1))
 
     def forward_qkvx(self, hidden_states):
         """One GEMM for all four projections of the (already normalised) input -> views (q, k, v, qx) of one
         [..., 2*out_q + 2*out_kv] result.  (fp8_quant: four quantise + fp8 GEMM pairs, each with its own scales.)"""
-        lead = hidden_states.shape[:-1]
-        return tuple(t.view(lead + (t.shape[-1],)) for t in self._qkvx_rows(hidden_states.reshape(-1, hidden_states.shape[-1])))
+        if self.fp8_quant:
+            return tuple(m(hidden_states) for m in self._projections())
+        return self._split(torch.nn.functional.linear(hidden_states, self.fused_weight()))
+
+    def _split(self, y: torch.Tensor):
+        oq, okv = _param(self.q, "weight").shape[0], _param(self.k, "weight").shape[0]
+        return y.split((oq, okv, okv, oq), dim=-1)
+
+    def _takes_e4m3(self, m, cols: int) -> bool:
+        """Whether the fused norm may hand m its quantised input: nothing that watches or replaces m's own call, and an
+        input_scale as layer_norm_div_clamp takes it."""
+        s = m.input_scale
+        return (type(m) is PerTensorQuantizedFp8Linear and not m._forward_hooks and not m._forward_pre_hooks
+                and s.shape == (cols,) and s.dtype == torch.float32 and s.is_contiguous())
 
     def forward_ln_qkvx_rows(self, hidden_states):
         """forward_qkvx(forward_ln(hidden_states)) as [tokens, out] rows.  With fp8_quant the norm and the four input
@@ -289,19 +300,20 @@ class CustomLayerNormLinear(torch.nn.Module):
         cols = hidden_states.shape[-1]
         if self.fp8_quant:
             linears = self._projections()
-            if (cols % 8 == 0 and cols <= 8192 and hidden_states.is_contiguous()
-                    and all(type(m) is PerTensorQuantizedFp8Linear and m.input_scale.numel() == cols for m in linears)):
+            if cols % 8 == 0 and cols <= 8192 and hidden_states.is_contiguous() and all(self._takes_e4m3(m, cols) for m in linears):
                 ln = self.layer_norm
                 x8 = layer_norm_div_clamp(hidden_states.view(-1, cols), ln.weight.detach(), ln.bias.detach(),
                                           [m.input_scale.detach() for m in linears], ln.eps)
                 return tuple(m.forward_quantized(x) for m, x in zip(linears, x8.unbind(0)))
-        return self._qkvx_rows(self.forward_ln(hidden_states).view(-1, cols))
+            x = self.forward_ln(hidden_states).view(-1, cols)
+            return tuple(m(x) for m in linears)
+        return self._split(_linear_in_whole_rounds(self.forward_ln(hidden_states).view(-1, cols), self.fused_weight()))
 
     def forward_ln(self, hidden_states):
         """LayerNorm of the layer input (dit_module.py:412-413) as one HIP launch; the parameters stay on the
         torch.nn.LayerNorm sub-module under the reference's names."""
         ln = self._modules["layer_norm"]
-        return layer_norm(hidden_states, ln._parameters["weight"], ln._parameters["bias"], ln.eps)
+        return layer_norm(hidden_states, _param(ln, "weight"), _param(ln, "bias"), ln.eps)
 
     def forward_q(self, hidden_states):
         return self.q(hidden_states)
@@ -726,7 +738,7 @@ class FullyParallelAttention(torch.nn.Module):
         D = self.hidden_size_per_attention_head
         q = qx_raw.view(sq, -1, D) if b == 1 else qx_raw.view(sq, b, -1, D).transpose(0, 1)  # row-strided views of the projection
         m = self._modules
-        kv = torch.nn.functional.linear(key_value_states, m["linear_kv_xattn"]._parameters["weight"])
+        kv = torch.nn.functional.linear(key_value_states, _param(m["linear_kv_xattn"], "weight"))
         k_, v_ = _halves(kv.view(key_value_states.shape[0], -1, 2 * D), kv.shape[0])
         gk, bk = m["k_layernorm_xattn"].gamma_beta_fp32()
         kx = head_norm(k_, gk, bk, self.eps)

@@ -296,6 +296,39 @@ def test_projection_weights_share_one_buffer():
     assert torch.equal(w3[80:], sd["qx.weight"].bfloat16())
 
 
+def test_projection_buffer_is_released_and_wrapped_weights_are_read_through_their_attribute():
+    """The shared buffer lives as long as the parameters in it and no longer; a parametrised weight, which is no parameter
+    under its name, is read through its attribute; forward_qkvx runs on the CPU and carries gradients and tangents at sizes
+    whose rows the device path cuts in two."""
+    from torch.multiprocessing.reductions import StorageWeakRef
+
+    from magi_attn.module import CustomLayerNormLinear, FusedLayerNorm
+
+    class Double(torch.nn.Module):
+        def forward(self, w):
+            return 2 * w
+
+    m = CustomLayerNormLinear(64, 48, 16, dtype=torch.float32)
+    buffer = StorageWeakRef(m.fused_weight().untyped_storage())
+    m = m.to(torch.bfloat16)
+    assert buffer.expired()
+    for lin in (m.q, m.v):
+        lin.weight.data.normal_()
+    torch.nn.utils.parametrize.register_parametrization(m.v, "weight", Double())
+    assert torch.equal(m.fused_weight()[64:80], m.v.weight) and torch.equal(m.fused_weight()[:48], m.q.weight)
+    n = FusedLayerNorm(16, dtype=torch.float32)
+    n.weight.data.fill_(0.5)
+    torch.nn.utils.parametrize.register_parametrization(n, "weight", Double())
+    assert torch.equal(n.gamma_beta_fp32()[0], torch.ones(16))
+
+    m = CustomLayerNormLinear(1024, 96, 32, dtype=torch.float32)
+    x, t = torch.randn(2, 1, 1024, requires_grad=True), torch.randn(2, 1, 1024)
+    grad = torch.autograd.grad(m.forward_qkvx(x)[0].sum(), x)[0]
+    assert torch.allclose(grad, m.q.weight.sum(0).expand(2, 1, -1), atol=1e-4)
+    tangent = torch.func.jvp(lambda x_: m.forward_qkvx(x_)[3], (x.detach(),), (t,))[1]
+    assert torch.allclose(tangent, m.forward_qx(t), atol=1e-4)
+
+
 def test_fp8_kv_cache_shapes_and_layer_option():
     from magi_attn.cache import Fp8KVCache
     from magi_attn.module import FullyParallelAttention
