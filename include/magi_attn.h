@@ -69,7 +69,7 @@ extern "C" {
  * clear the output first; without the flag they are left untouched.  1 to 64 ranges. */
 #define MAGI_ATTN_ZERO_UNCOVERED 32
 /* For bf16 callers that promise nothing about the scores: run the bounded-score kernel as if they were bounded, have it
- * judge by its row sums whether they were (sums within 2^+-64: no score above 64, nothing of weight underflowed), and
+ * judge by its row sums whether they were (sums from 2^-16 to 2^64, finite results: no score above 64, nothing of weight underflowed), and
  * repeat in a second launch, with a running maximum, the 64-row blocks where they were not.  No passes over q and k
  * (MAGI_ATTN_AUTO_BOUND) and the right result for any input; inputs with larger scores throughout cost about 2.5 times
  * as much.  args->workspace: 16 bytes of DEVICE memory per q head, range and 256 rows of max_seqlen_q (any content), 16-byte

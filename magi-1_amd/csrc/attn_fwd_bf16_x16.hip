@@ -82,12 +82,13 @@ constexpr int v_block(int i) { return (i >> 1) + 4 * (i & 1); }
 constexpr int Q_AS_IS = 0, Q_NORM = 1, Q_SCALE = 2, Q_CHECK = 3;
 
 // Row sums that the kernel without a running maximum can be trusted with (CHECK, below).
-constexpr float SUM_MIN = 0x1p-64f, SUM_MAX = 0x1p64f;
+constexpr float SUM_MIN = 0x1p-16f, SUM_MAX = 0x1p64f;
 
 // CHECK (QMODE Q_CHECK): nobody has promised that the scores are bounded.  The kernel computes as if they were, and each wavefront
-// leaves a verdict on its 64 rows in a.verdict[4 * item + wavefront]: 2^score and the accumulators are good where
-// SUM_MIN <= row sum <= SUM_MAX (then no score is above 64, and the terms that underflow are below 2^-42 of the sum; an
-// overflow leaves inf or NaN in the sum, so nothing outside can pass).  attn_fwd_bf16_redo_kernel, launched behind it,
+// leaves a verdict on its 64 rows in a.verdict[4 * item + wavefront]: they are good where SUM_MIN <= row sum <= SUM_MAX
+// (then no score is above 64, and the terms that underflow are below 2^-90 of the sum; an overflow leaves inf or NaN in
+// it) and every accumulator is finite (2^64 times a value above 2^63 is not).  The lower end keeps products with values
+// down to 2^-110 normal numbers.  attn_fwd_bf16_redo_kernel, launched behind it,
 // computes the others again with a running maximum.
 template <int QMODE>
 __global__ __launch_bounds__(256, 2) void attn_fwd_bf16_x16_kernel(const AttnKernArgs a) {
@@ -329,12 +330,12 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_bf16_x16_kernel(const AttnKer
         // The accumulators of a key block start from 0.  In the ragged copy of the body, keys past the end of the
         // range (whose LDS rows hold copies of the last valid key: the loader clamps) start from -1e4 instead: their
         // scores stay far below any real one (|score| <= 64), 2^score is exactly 0, and neither the row sums nor
-        // the P operand see them.  Register r of the lanes of group g is key 16 kb + 4 g + r of the half.
+        // the P operand see them.  (CHECK multiplies the scores by the caller's scale afterwards: -inf there.)  Register r of the lanes of group g is key 16 kb + 4 g + r of the half.
         f32x4v c0 = zero4;
         if constexpr (decltype(ragged)::value && kk == 0) {
           const int left = ke - (k0 + 32 * t) - 16 * kb - 4 * (l >> 4);  // valid keys from this lane's first one on
 #pragma unroll
-          for (int r = 0; r < 4; ++r) c0[r] = r < left ? 0.f : -1.0e4f;
+          for (int r = 0; r < 4; ++r) c0[r] = r < left ? 0.f : (CHECK ? -__builtin_inff() : -1.0e4f);
         }
 #pragma unroll
         for (int qb = 0; qb < 4; ++qb)
@@ -431,7 +432,14 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_bf16_x16_kernel(const AttnKer
     float s = l_run[qb];
     s += __shfl_xor(s, 16);
     s += __shfl_xor(s, 32);
-    if constexpr (CHECK) bad |= end != last || !(s >= SUM_MIN && s <= SUM_MAX);
+    if constexpr (CHECK) {
+      float fine = 0.f;  // (NaN once an accumulator is not finite)
+#pragma unroll
+      for (int db = 0; db < 8; ++db)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) fine = __builtin_fmaf(o_acc[db][qb][r], 0.f, fine);
+      bad |= end != last || !(s >= SUM_MIN && s <= SUM_MAX) || fine != fine;
+    }
     const float inv = 1.f / s;
     // lane (ne, ge) holds O[row 16 qb + ne][d = 16 db + 4 ge + r]: 8 bytes of bf16 at byte 32 db + 8 ge of the row,
     // i.e. half (ge & 1) of 16-byte chunk 2 db + ge / 2, kept at chunk ^ (row & 15) = chunk ^ ne
@@ -468,11 +476,11 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_bf16_x16_kernel(const AttnKer
 // tiles and items.  A workgroup goes through every gridDim.x-th block of that launch, 64 verdicts at a time, and does the
 // flagged ones (usually none: the launch then costs one look at 16 bytes per 256 rows and head).  32 rows per wavefront
 // at a time, the two halves of its 64 one after the other.  The maximum of a row is raised only when a score comes out
-// more than RAISE above it: within that sums and products keep their full precision, and rescaling the accumulators is
-// rare.
+// more than RAISE above it: within that sums and products keep their full precision (values up to 2^110 do not
+// overflow them), and rescaling the accumulators is rare.
 __global__ __launch_bounds__(256, 2) void attn_fwd_bf16_redo_kernel(const AttnKernArgs a) {
   constexpr int NW = 4, BM = 64 * NW, LOADS = BN / (4 * NW);
-  constexpr float RAISE = 32.f;
+  constexpr float RAISE = 8.f;
   __shared__ __attribute__((aligned(1024))) unsigned char sK0[K_TILE_BYTES];
   __shared__ __attribute__((aligned(1024))) unsigned char sV0[V_TILE_BYTES];
   __shared__ __attribute__((aligned(1024))) unsigned char sK1[K_TILE_BYTES];

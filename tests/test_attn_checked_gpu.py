@@ -97,6 +97,31 @@ def test_non_finite_inputs_stay_where_they_belong(dev):
     assert torch.equal(nan, want)
 
 
+@pytest.mark.parametrize("size", [2.0 ** 83, 2.0 ** -83])
+def test_values_of_any_size(dev, size):
+    """Exponents around 52 or around -52 are within the kernel's, but not times values as large or as small as these: the
+    accumulators would overflow or go subnormal.  Relative to the values, against the oracle."""
+    L, Hq, Hkv = 150, 4, 2
+    q, k, v = O.synthetic_qkv(2 * L, 300, Hq, Hkv, 128, seed=8)
+    k[:, 0] = (k[:, 0].float() * 0.05 + 2.0).bfloat16()
+    q[:, :2] = (q[:, :2].float() * 0.05 + (1.6 if size > 1 else -1.6)).bfloat16()
+    qr, kr = np.array([[0, L], [L, 2 * L]]), np.array([[0, 300], [7, 299]])
+    out, _ = M.range_attention(q.to(dev), k.to(dev), (v.float() * size).bfloat16().to(dev), *_ranges(dev, qr, kr), L, checked=True)
+    _close(out.float() / size, O.range_attention(q, k, v, qr, kr))
+
+
+@pytest.mark.parametrize("Tk", [5, 70, 97])
+def test_keys_past_the_end_stay_out_at_a_small_softmax_scale(dev, Tk):
+    """The masked keys of a ragged tile take no part whatever the scale that the scores are multiplied by."""
+    L, Hq, Hkv = 70, 2, 1
+    q, k, v = O.synthetic_qkv(L, Tk, Hq, Hkv, 128, seed=Tk)
+    tq, tk = _ranges(dev, [[0, L]], [[0, Tk]])
+    for scale in (1e-3, 1e-6):
+        out, lse = M.range_attention(q.to(dev), k.to(dev), v.to(dev), tq, tk, L, softmax_scale=scale, checked=True)
+        online, lse_o = M.range_attention(q.to(dev), k.to(dev), v.to(dev), tq, tk, L, softmax_scale=scale)
+        assert (out.float() - online.float()).abs().max().item() <= 2e-2 and (lse - lse_o).abs().max().item() <= 1e-3
+
+
 def test_many_ranges_empty_ranges_and_gaps(dev):
     """More ranges than one wavefront (and than the workgroup) ranks, some without keys, some rows in no range."""
     for n in (3, 65, 300):
