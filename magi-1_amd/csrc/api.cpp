@@ -79,6 +79,53 @@ int static_scratch(void** out) {
   return MAGI_OK;
 }
 
+// Workgroups of one XCD's list (attn_common.h, locate_work): its Hkv / 8 whole heads, and its share of the rest.
+unsigned items_per_xcd(int Hq, int Hkv, int n_ranges, int tiles_per_range) {
+  const long left = Hkv % 8, per_head = (long)n_ranges * tiles_per_range * (Hq / Hkv);
+  return (unsigned)((Hkv / 8) * per_head + (left * per_head + 7) / 8);
+}
+
+// Which items of a 256-row launch without a running maximum have their keys shared by several workgroups (AttnKernArgs::split_*).
+struct SplitPlan {
+  unsigned from, pieces, num, den;
+  int64_t bytes(unsigned per_xcd) const { return from < per_xcd ? 4ll * magi::SPLIT_FLOATS * 8 * (per_xcd - from) * pieces : 0; }
+};
+// The last round of a launch has `left` items for `slots` places (two workgroups per CU) on each XCD.  At most half of them: equal pieces, as
+// many as the places allow.  More: two pieces, the first so much longer that the others' second pieces fill the places
+// left over in the time it takes (at 47 of 64, 3/4: three quarters on one slot take as long as a slot's three quarters).  A tile
+// of 64 keys takes a workgroup about 3 us, 1.9 us alone on its CU (0.62; behind two rounds and more, out of step by then, 1.5); what the shorter round saves is put at half of that
+// beside other workgroups (they slow down: the chip is power limited) and has to exceed the price, two launches' latency and
+// the partial sums written and read at about 3.3 TB/s.  Measured, whole / split, at 24 / 8 heads: 18 of 64 items over 7680
+// keys 208 / 137 us, 9 over 6300 keys 173 / 77, 47 over 46800 keys behind one whole round 4438 / 4020, over 9360 keys
+// 845 / 818; and where the rule says no: 60 over 25000 keys 1131 / 1144, 54 over 4608 keys 159 / 174, 18 over 1536 keys
+// 48 / 52.  4 over 99000 keys behind five whole rounds 9009 / 8583.  Behind eight and more
+// the round is a small part of the launch.
+SplitPlan split_plan(unsigned items, int max_seqlen_k) {
+  SplitPlan s = {UINT32_MAX, 1, 1, 1};
+  const unsigned slots = (unsigned)compute_units() / 4;  // of one XCD: two workgroups per CU
+  if (slots == 0 || max_seqlen_k <= 0) return s;
+  const unsigned rounds = items / slots, left = items % slots, tiles = (unsigned)(max_seqlen_k + 63) / 64;
+  if (left == 0 || rounds >= 8) return s;
+  unsigned num, den;
+  if (left * 2 > slots) {
+    num = (left + slots - left - 1) / (slots - left);
+    den = num + 1;
+  } else {
+    num = 1;
+    den = slots / left < 8 ? slots / left : 8;
+    if (den > tiles / 8) den = tiles / 8;
+  }
+  if (den < 2 || num > 4 || tiles < 4 * den) return s;
+  const double round_us = 3.0 * tiles, piece = (double)num / den, mb = 8e-6 * left * (den - num + 1) * 4 * magi::SPLIT_FLOATS;
+  const double saved_us = left * 2 > slots ? 0.5 * (1.0 - piece) * round_us : ((rounds >= 2 ? 0.5 : 0.62) - piece) * round_us;
+  if (saved_us < 8.0 + 0.3 * mb) return s;
+  s.from = rounds * slots;
+  s.pieces = den - num + 1;
+  s.num = num;
+  s.den = den;
+  return s;
+}
+
 int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace);
 
 // the caller's struct as this version lays it out: itself, or `full` filled from the shorter one of version 103
@@ -100,6 +147,14 @@ int magi_version(void) { return 104; }
 uint64_t magi_launch_count(void) { return g_launches.load(std::memory_order_relaxed); }
 
 const char* magi_last_error(void) { return g_err; }
+
+int64_t magi_attn_split_bytes(int32_t Hq, int32_t Hkv, int32_t n_ranges, int32_t max_seqlen_q, int32_t max_seqlen_k) {
+  if (Hq <= 0 || Hkv <= 0 || Hq % Hkv || n_ranges <= 0 || max_seqlen_q <= 0) return 0;
+  const int tiles = max_seqlen_q / 256 + (max_seqlen_q % 256 != 0);
+  if ((double)Hq * n_ranges * tiles > 2.0e9) return 0;
+  const unsigned items = items_per_xcd(Hq, Hkv, n_ranges, tiles);
+  return split_plan(items, max_seqlen_k).bytes(items);
+}
 
 int magi_attn_fwd(const magi_attn_args* p, void* stream) {
   if (!p) return fail(MAGI_EINVAL, "magi_attn_fwd: args is NULL");
@@ -202,6 +257,8 @@ int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace) {
       return fail(MAGI_EINVAL, "magi_attn_fwd: MAGI_ATTN_CHECKED needs a workspace on the device, 16-byte aligned, of 16 bytes "
                                "per q head, range and 256 rows of max_seqlen_q");
   }
+  if (p->split_workspace && (!aligned16(p->split_workspace) || p->split_workspace_bytes < 0))
+    return fail(MAGI_EINVAL, "magi_attn_fwd: split_workspace must be 16-byte aligned");
   if (p->out_group_heads < 0 || (p->out_group_heads > 0 && (p->Hq % p->out_group_heads || p->o_stride_g % 8)))
     return fail(MAGI_EINVAL, "magi_attn_fwd: out_group_heads must divide Hq and o_stride_g keep rows 16-byte aligned");
   int k_split = p->total_k;
@@ -323,10 +380,18 @@ int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace) {
     a.flags = p->flags | (bounded ? magi::ATTN_BOUNDED : 0) | (scale_q ? magi::ATTN_SCALE_Q : 0);
     const double total = (double)p->Hq * p->n_ranges * a.tiles_per_range;
     if (total > 2.0e9) return fail(MAGI_EINVAL, "magi_attn_fwd: grid too large (%.3g workgroups)", total);
-    // workgroups of one XCD's list (attn_common.h, locate_work): its Hkv / 8 whole heads, and its share of the rest
-    const long left = p->Hkv % 8, per_head = (long)p->n_ranges * a.tiles_per_range * a.G;
-    const long dealt = (left * per_head + 7) / 8;
-    a.per_xcd = (unsigned)((p->Hkv / 8) * per_head + dealt);
+    a.per_xcd = items_per_xcd(p->Hq, p->Hkv, p->n_ranges, a.tiles_per_range);
+    a.split_from = UINT32_MAX;
+    if (bounded && a.block_m == 256 && !mfma32 && p->split_workspace) {
+      const SplitPlan s = split_plan(a.per_xcd, p->max_seqlen_k);
+      if (s.from < a.per_xcd && s.bytes(a.per_xcd) <= p->split_workspace_bytes) {
+        a.partial = static_cast<float*>(p->split_workspace);
+        a.split_from = s.from;
+        a.split_pieces = s.pieces;
+        a.split_num = s.num;
+        a.split_den = s.den;
+      }
+    }
     hipError_t e;
     if (p->dtype != MAGI_DTYPE_BF16)
       e = magi::launch_attn_fwd_fp8(a, static_cast<hipStream_t>(stream));
@@ -339,7 +404,7 @@ int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace) {
     else
       e = magi::launch_attn_fwd_bf16(a, static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return hip_fail(e, "magi_attn_fwd launch");
-    g_launches.fetch_add(checked ? 2 : 1, std::memory_order_relaxed);
+    g_launches.fetch_add((checked ? 2 : 1) + (a.split_from < a.per_xcd), std::memory_order_relaxed);
     return MAGI_OK;
   };
 

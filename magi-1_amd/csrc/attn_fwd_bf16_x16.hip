@@ -90,6 +90,33 @@ constexpr float SUM_MIN = 0x1p-16f, SUM_MAX = 0x1p64f;
 // it) and every accumulator is finite (2^64 times a value above 2^63 is not).  The lower end keeps products with values
 // down to 2^-110 normal numbers.  attn_fwd_bf16_redo_kernel, launched behind it,
 // computes the others again with a running maximum.
+//
+// A launch whose last round of workgroups leaves slots (two per CU) empty has the keys of that round's items shared by
+// several workgroups each (a.split_*, split_plan in api.cpp).  Without a running maximum the pieces simply add up: each leaves its
+// unnormalised accumulators and row sums in fp32, attn_fwd_bf16_merge_kernel adds them in the order of the keys.
+struct SplitPiece {
+  float* out;  // nullptr: a whole item
+  unsigned piece;
+};
+// workgroup `block` of the grid with split items -> `block` of the grid without, and the piece of it
+__device__ __forceinline__ SplitPiece split_piece(const AttnKernArgs& a, unsigned& block) {
+  const unsigned pos = block >> 3, xcd = block & 7u;
+  if (pos < a.split_from) return {nullptr, 0u};
+  const unsigned items = a.per_xcd - a.split_from;  // (the longer first pieces of all items ahead of the others)
+  const unsigned piece = (pos - a.split_from) / items, i = (pos - a.split_from) - piece * items;
+  block = ((a.split_from + i) << 3) | xcd;
+  return {a.partial + (long)((i * 8u + xcd) * a.split_pieces + piece) * SPLIT_FLOATS, piece};
+}
+__device__ __forceinline__ unsigned split_cut(const AttnKernArgs& a, unsigned tiles, unsigned piece) {
+  return piece == 0u ? 0u : (unsigned)((unsigned long long)tiles * (a.split_num + piece - 1u) / a.split_den);
+}
+__device__ __forceinline__ void store_partial_zero(float* out, int w, int l) {
+  f32x4v* const dst = (f32x4v*)out + w * 2048 + l;
+#pragma unroll
+  for (int i = 0; i < 32; ++i) dst[i * 64] = f32x4v{0.f, 0.f, 0.f, 0.f};
+  out[256 * 128 + 64 * w + l] = 0.f;
+}
+
 template <int QMODE>
 __global__ __launch_bounds__(256, 2) void attn_fwd_bf16_x16_kernel(const AttnKernArgs a) {
   constexpr bool CHECK = QMODE == Q_CHECK;
@@ -108,9 +135,12 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_bf16_x16_kernel(const AttnKer
   if (gate_closed(a)) return;
   const int tid = threadIdx.x;
   if (CHECK && tid == 0) s_over = 0;
-  const WorkItem wi = locate_work(a, BM, tid, s_sel, blockIdx.x);
+  unsigned block = blockIdx.x;
+  const SplitPiece sp = split_piece(a, block);
+  const WorkItem wi = locate_work(a, BM, tid, s_sel, block);
   if (!wi.valid) return;
-  const int qe = wi.qe, ks = wi.ks, ke = wi.ke;
+  const int qe = wi.qe;
+  int ks = wi.ks, ke = wi.ke;
 
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l = tid & 63, n = l & 15, g = l >> 4;
@@ -121,6 +151,16 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_bf16_x16_kernel(const AttnKer
       if (row0 + 32 * b + (l & 31) < qe) store_empty_row(a, wi, row0 + 32 * b + (l & 31), l >> 5);
     if (CHECK && l == 0) a.verdict[4 * (long)wi.item + w] = 0;
     return;
+  }
+  if (sp.out) {
+    const unsigned tiles = (unsigned)(ke - ks + BN - 1) / BN;
+    const int b = (int)split_cut(a, tiles, sp.piece), e = (int)split_cut(a, tiles, sp.piece + 1);
+    if (b == e) {  // (a range with fewer tiles than pieces)
+      store_partial_zero(sp.out, w, l);
+      return;
+    }
+    ke = min(ke, ks + e * BN);
+    ks += b * BN;
   }
 
   // ---- K/V tile loader: wave w fills rows 4 * (w + 4 j) .. +3; lane l sits at row +(l >> 4), slot l & 15 ----
@@ -416,6 +456,23 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_bf16_x16_kernel(const AttnKer
   }
   if (j < end) step(j, j + 1, slot1, std::false_type{});
 
+  // ---- a piece of an item: accumulators and row sums as they are, one contiguous 1 KB per instruction ----
+  if (sp.out) {
+    if (!wave_on) return;
+    f32x4v* const dst = (f32x4v*)sp.out + w * 2048 + l;
+#pragma unroll
+    for (int qb = 0; qb < 4; ++qb) {
+      float s = l_run[qb];
+      s += __shfl_xor(s, 16);
+      s += __shfl_xor(s, 32);
+      if (CHECK && end != last) s = __builtin_nanf("");
+      if (g == 0) sp.out[256 * 128 + 64 * w + 16 * qb + n] = s;
+#pragma unroll
+      for (int db = 0; db < 8; ++db) dst[(4 * db + qb) * 64] = o_acc[db][qb];
+    }
+    return;
+  }
+
   // ---- epilogue: normalise, transpose through LDS, store whole rows ----
   __syncthreads();  // every wave is done with the tile slots: wave w takes slot w as its 64 x 256-byte staging area
   if (!wave_on) {
@@ -472,7 +529,63 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_bf16_x16_kernel(const AttnKer
   }
 }
 
-// The rows that a CHECK launch of the kernel above could not be trusted with, again, with a running maximum: same ranges,
+// The split items of a launch of the kernel above: sums their pieces, normalises, writes the rows (CHECK: and the verdicts).
+// One workgroup per item, a wavefront for each 64 rows, lane layout of the accumulators as above.  Memory bound: SPLIT_FLOATS
+// * 4 bytes read per piece.
+template <bool CHECK>
+__global__ __launch_bounds__(256) void attn_fwd_bf16_merge_kernel(const AttnKernArgs a) {
+  __shared__ int s_sel[LOCATE_WORDS];
+  if (gate_closed(a)) return;
+  const int tid = threadIdx.x, l = tid & 63, n = l & 15, g = l >> 4;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const WorkItem wi = locate_work(a, 256, tid, s_sel, blockIdx.x + 8u * a.split_from);
+  const int row0 = wi.q0 + 64 * w;
+  if (!wi.valid || wi.ke <= wi.ks) return;  // (nothing there, or without keys: done)
+  if (row0 >= wi.qe) {
+    if (CHECK && l == 0) a.verdict[4 * (long)wi.item + w] = 0;
+    return;
+  }
+  const float* const base = a.partial + (long)blockIdx.x * a.split_pieces * SPLIT_FLOATS;
+  const int pieces = (int)a.split_pieces;
+  bool bad = false;
+#pragma unroll
+  for (int qb = 0; qb < 4; ++qb) {
+    const float* p = base;
+    float s = 0.f;
+    f32x4v o[8];
+#pragma unroll
+    for (int db = 0; db < 8; ++db) o[db] = f32x4v{0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < pieces; ++i, p += SPLIT_FLOATS) {
+      const f32x4v* const src = (const f32x4v*)p + w * 2048 + l;
+#pragma unroll
+      for (int db = 0; db < 8; ++db) o[db] += src[(4 * db + qb) * 64];
+      s += p[256 * 128 + 64 * w + 16 * qb + n];
+    }
+    if constexpr (CHECK) {
+      float fine = 0.f;
+#pragma unroll
+      for (int db = 0; db < 8; ++db)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) fine = __builtin_fmaf(o[db][r], 0.f, fine);
+      bad |= !(s >= SUM_MIN && s <= SUM_MAX) || fine != fine;
+    }
+    const int q_row = row0 + 16 * qb + n;
+    if (q_row >= wi.qe) continue;
+    const float inv = 1.f / s;
+    char* const op = a.out + row_offset(a, q_row, a.os_t, a.os_b) + wi.o_head + 8 * g;
+#pragma unroll
+    for (int db = 0; db < 8; ++db)
+      *(u32x2*)(op + 32 * db) = u32x2{pack_bf16x2(o[db][0] * inv, o[db][1] * inv), pack_bf16x2(o[db][2] * inv, o[db][3] * inv)};
+    if (a.lse && g == 0) a.lse[(long)wi.h * a.total_q + q_row] = __builtin_amdgcn_logf(s) * 0.6931471805599453f;
+  }
+  if constexpr (CHECK) {
+    // (rows beyond the range repeat its last row, as in the kernel that left the pieces: they raise no flag of their own)
+    const bool any = __builtin_amdgcn_ballot_w64(bad) != 0;
+    if (l == 0) a.verdict[4 * (long)wi.item + w] = any ? 1 : 0;
+  }
+}
+
+// The rows that a CHECK launch of the kernels above could not be trusted with, again, with a running maximum: same ranges,
 // tiles and items.  A workgroup goes through every gridDim.x-th block of that launch, 64 verdicts at a time, and does the
 // flagged ones (usually none: the launch then costs one look at 16 bytes per 256 rows and head).  32 rows per wavefront
 // at a time, the two halves of its 64 one after the other.  The maximum of a row is raised only when a score comes out
@@ -652,23 +765,42 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_bf16_redo_kernel(const AttnKe
 
 }  // namespace
 
+namespace {
+unsigned split_items(const AttnKernArgs& a) { return a.split_from < a.per_xcd ? a.per_xcd - a.split_from : 0u; }
+dim3 grid_of(const AttnKernArgs& a) {
+  const unsigned items = split_items(a);
+  return dim3(8u * (a.per_xcd - items + items * a.split_pieces));
+}
+template <bool CHECK>
+void launch_merge(const AttnKernArgs& a, hipStream_t stream) {
+  if (const unsigned items = split_items(a)) {
+    AttnKernArgs m = a;
+    m.flags &= ~ATTN_ZERO_GAPS;  // (the rows no range covers are clear by now)
+    hipLaunchKernelGGL(attn_fwd_bf16_merge_kernel<CHECK>, dim3(8u * items), dim3(256), 0, stream, m);
+  }
+}
+}  // namespace
+
 hipError_t launch_attn_fwd_bf16_x16(const AttnKernArgs& a, hipStream_t stream) {
-  const dim3 grid(a.per_xcd * 8u);
+  const dim3 grid = grid_of(a);
   if (a.q_norm_gamma)  // raw q, normalised while it is loaded (cross attention)
     hipLaunchKernelGGL(attn_fwd_bf16_x16_kernel<Q_NORM>, grid, dim3(256), 0, stream, a);
   else if (a.flags & ATTN_SCALE_Q)  // unscaled q, scaled while it is loaded (the reference-shaped callables)
     hipLaunchKernelGGL(attn_fwd_bf16_x16_kernel<Q_SCALE>, grid, dim3(256), 0, stream, a);
   else
     hipLaunchKernelGGL(attn_fwd_bf16_x16_kernel<Q_AS_IS>, grid, dim3(256), 0, stream, a);
+  launch_merge<false>(a, stream);
   return hipGetLastError();
 }
 
 hipError_t launch_attn_fwd_bf16_checked(const AttnKernArgs& a, int compute_units, hipStream_t stream) {
-  const dim3 grid(a.per_xcd * 8u);
+  const dim3 grid = grid_of(a);
   // (two workgroups per CU, a multiple of eight so that a block keeps its XCD)
   const unsigned most = (unsigned)(compute_units / 4) * 8u;
-  const dim3 again(grid.x < most || most == 0 ? grid.x : most);
+  const unsigned blocks = 8u * a.per_xcd;
+  const dim3 again(blocks < most || most == 0 ? blocks : most);
   hipLaunchKernelGGL(attn_fwd_bf16_x16_kernel<Q_CHECK>, grid, dim3(256), 0, stream, a);
+  launch_merge<true>(a, stream);
   hipLaunchKernelGGL(attn_fwd_bf16_redo_kernel, again, dim3(256), 0, stream, a);
   return hipGetLastError();
 }

@@ -48,7 +48,14 @@ struct AttnKernArgs {
   int gate_want;
   // Checked launches (MAGI_ATTN_CHECKED): four words per item, one per wavefront of the 256-row kernel
   int* verdict;
+  // Items whose keys are shared by several workgroups (split_plan in api.cpp; the 256-row kernel only): the items from
+  // position split_from of each XCD's list on, in split_pieces pieces each.  Piece p starts at tile n_tiles * (split_num +
+  // p - 1) / split_den of the item's key range, piece 0 at tile 0.  `partial`: SPLIT_FLOATS floats per piece.
+  float* partial;
+  unsigned split_from, split_pieces, split_num, split_den;  // split_from: UINT_MAX = nothing is split
 };
+// 256 rows x 128 accumulators, and the 256 row sums behind them
+constexpr int SPLIT_FLOATS = 256 * 128 + 256;
 
 
 // internal flag: the caller promised bounded scores (magi_attn_args.score_bound within MAGI_SCORE_BOUND_MAX)
@@ -60,6 +67,7 @@ constexpr int ATTN_ZERO_GAPS = 32;
 
 hipError_t launch_attn_fwd_bf16(const AttnKernArgs& a, hipStream_t stream);
 hipError_t launch_attn_fwd_bf16_w64(const AttnKernArgs& a, hipStream_t stream);
+// (with items to split: and behind it the launch that adds their pieces up)
 hipError_t launch_attn_fwd_bf16_x16(const AttnKernArgs& a, hipStream_t stream);
 // the bounded-score kernel without a promise, and behind it the launch that repeats what it could not be trusted with
 hipError_t launch_attn_fwd_bf16_checked(const AttnKernArgs& a, int compute_units, hipStream_t stream);

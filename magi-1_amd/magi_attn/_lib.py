@@ -65,6 +65,7 @@ class AttnArgs(_SizedStructure):
         ("k2_scale", C.c_void_p), ("v2_scale", C.c_void_p),
         ("workspace", C.c_void_p),
         ("q_batch_rows", C.c_int32), ("q_stride_b", C.c_int64), ("o_stride_b", C.c_int64),
+        ("split_workspace", C.c_void_p), ("split_workspace_bytes", C.c_int64),
     ]
 
 
@@ -112,6 +113,7 @@ class QuantizeArgs(_SizedStructure):
 ABI_VERSION = 104  # magi_version() of the library these mirrors were written for
 
 EXPORTS = ("magi_version", "magi_last_error", "magi_launch_count", "magi_attn_fwd", "magi_attn_fwd_static_scratch",
+           "magi_attn_split_bytes",
            "magi_qk_prologue", "magi_head_norm",
            "magi_apply_rotary", "magi_quantize_fp8", "magi_quantize_fp8_split", "magi_layer_norm", "magi_qkv_proj_prologue", "magi_div_clamp_to_e4m3",
            "magi_layer_norm_e4m3")
@@ -134,6 +136,8 @@ def lib() -> C.CDLL:
                                "rebuild the library (`make -C magi-1_amd/csrc`)")
         l.magi_launch_count.restype = C.c_uint64
         l.magi_last_error.restype = C.c_char_p
+        l.magi_attn_split_bytes.argtypes = [C.c_int32] * 5
+        l.magi_attn_split_bytes.restype = C.c_int64
         l.magi_attn_fwd.argtypes = [C.POINTER(AttnArgs), C.c_void_p]
         l.magi_attn_fwd.restype = C.c_int
         l.magi_attn_fwd_static_scratch.argtypes = [C.POINTER(AttnArgs), C.c_void_p]

@@ -100,6 +100,7 @@ def range_attention(
     out: Optional[torch.Tensor] = None,
     return_lse: bool = True,
     zero_init: bool = True,
+    split_keys: bool = True,
 ) -> Tuple[torch.Tensor, Optional[torch.Tensor]]:
     """out[q_range_i] = softmax(q k^T * scale) v over k[k_range_i]; see magi_attn_fwd.
 
@@ -125,6 +126,8 @@ def range_attention(
     no allocation at all when `out` is given and return_lse is False; such calls must not overlap on one GPU).
     checked (bf16, instead of score_bound): the bounded-score kernel judges by its row sums whether the scores were
     bounded, and a second launch repeats the blocks of rows where they were not, MAGI_ATTN_CHECKED.
+    split_keys: False keeps the library from sharing the keys of a row among workgroups where that fills the chip better
+    (magi_attn_args.split_workspace; the sums are then added in another order).  Needs max_seqlen_k.
     q may be [batch, rows, Hq, D] with any batch stride (batch of activations laid out [position, batch, ...]): its rows
     count as batch * rows tokens for the ranges, out is (or comes back as) a tensor of q's shape, by default
     [rows, batch, Hq, D] transposed.  Needs a score_bound in force.
@@ -209,6 +212,14 @@ def range_attention(
         workspace = torch.empty(max(4 * Hq * max(n, 0) * ((int(max_seqlen_q) + 255) // 256), 4), dtype=torch.int32, device=q.device)
     if auto_bound and not static_scratch:
         workspace = torch.empty(4, dtype=torch.float32, device=q.device)  # (alive until the launches are enqueued)
+    split, split_bytes = None, 0
+    if split_keys and not static_scratch and max_seqlen_k >= 512 and (checked or auto_bound or 0.0 < score_bound <= L.MAGI_SCORE_BOUND_MAX):
+        split_bytes = L.lib().magi_attn_split_bytes(Hq, Hkv, max(n, 0), int(max_seqlen_q), int(max_seqlen_k))
+        if split_bytes:
+            try:
+                split = torch.empty(split_bytes, dtype=torch.uint8, device=q.device)
+            except torch.OutOfMemoryError:  # (a call that fits without it still runs)
+                split_bytes = 0
     gamma = beta = None  # (alive until the launch is enqueued)
     norm_eps, norm_kind = 0.0, 0
     if q_norm is not None:
@@ -224,7 +235,7 @@ def range_attention(
         ranges_mode, int(max_seqlen_q), int(max_seqlen_k), Hq, Hkv, D, _dtype_code(q), int(scale_chunk_tokens),
         0.0 if softmax_scale is None else float(softmax_scale), flags, group_heads, o_stride_g,
         min(float(score_bound), 3e38), int(q_tile_rows), _ptr(gamma), _ptr(beta), norm_eps, norm_kind, _ptr(k2_scale),
-        _ptr(v2_scale), _ptr(workspace), batch_rows, q_stride_b, o_stride_b)
+        _ptr(v2_scale), _ptr(workspace), batch_rows, q_stride_b, o_stride_b, _ptr(split), split_bytes)
     return out, lse
 
 
@@ -257,9 +268,22 @@ def _checking_pays(Hq: int, n_ranges: int, max_seqlen_q: int, keys: float, devic
     workgroups come near filling the chip's slots, two per CU, and have more than a few tiles of keys each, or are many;
     `keys` is the (average) length of a key range.  Measured, online against checked: 8880 workgroups over 400 keys 718 /
     529 us; 1296 over 684 keys 137 / 125; 432 over 4600 keys 290 / 228; but 576 over 400 keys 47 / 51, 144 over 1536 keys
-    52 / 55, 864 over 60 keys 29 / 33."""
+    52 / 55, 864 over 60 keys 29 / 33.  (Fewer workgroups: _sharing_keys_pays.)"""
     workgroups = Hq * n_ranges * ((max_seqlen_q + 255) // 256)
     return keys >= 96 and workgroups >= (1.6 if keys >= 512 else 4) * torch.cuda.get_device_properties(device).multi_processor_count
+
+
+def _sharing_keys_pays(Hq: int, Hkv: int, n_ranges: int, max_seqlen_q: int, max_seqlen_k: int, device) -> bool:
+    """The same for fewer workgroups, whose keys the checked kernel can share among more of them.  Measured, online against
+    checked: 144 workgroups over 7680 keys 216 / 153 us, 240 over 12000 keys 379 / 307, 72 over 6300 keys 133 / 103, 24 over
+    14000 keys 283 / 114, 48 over four ranges of up to 5760 keys 121 / 97.  Ranges of unequal length in more than a third of the
+    chip's slots gain little (288 over four ranges of up to 4200 keys 137 / 134, 288 of up to 12000 keys 320 / 309)."""
+    if max_seqlen_k < 512 or max_seqlen_q <= 0:
+        return False
+    workgroups = Hq * n_ranges * ((max_seqlen_q + 255) // 256)
+    slots = 2 * torch.cuda.get_device_properties(device).multi_processor_count
+    return ((3 * workgroups <= slots or (n_ranges == 1 and workgroups <= slots))
+            and L.lib().magi_attn_split_bytes(Hq, Hkv, n_ranges, int(max_seqlen_q), int(max_seqlen_k)) > 0)
 
 
 def _unbounded_mode(q, k, n_ranges: int, max_seqlen_q: int, max_seqlen_k: int, keys: float, score_bound: float,
@@ -272,7 +296,8 @@ def _unbounded_mode(q, k, n_ranges: int, max_seqlen_q: int, max_seqlen_k: int, k
         return {"auto_bound": bool(auto_bound)}
     if q.dtype != torch.bfloat16 or not q.is_cuda:
         return {}
-    fills = _checking_pays(q.shape[-2], n_ranges, max_seqlen_q, keys, q.device)
+    fills = (_checking_pays(q.shape[-2], n_ranges, max_seqlen_q, keys, q.device)
+             or _sharing_keys_pays(q.shape[-2], k.shape[-2], n_ranges, max_seqlen_q, max_seqlen_k, q.device))
     # (below that, ranges of unequal length leave the 256-row workgroups' last round to the longest one: 240 of them over
     # four ranges of up to 35000 keys 961 us measured against 854 us online; 216 over one range 1222 against 1320)
     if (fills or n_ranges == 1) and _measuring_a_bound_pays(q, k, n_ranges, max_seqlen_q, max_seqlen_k):

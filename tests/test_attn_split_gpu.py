@@ -1,0 +1,112 @@
+"""GPU tests of launches whose last round of items is shared by several workgroups each (magi_attn_args.split_workspace): the
+pieces' fp32 sums, added up, give what one workgroup gives, up to the order of the additions."""
+import pytest
+import torch
+
+import magi_attn as M
+from magi_attn import _lib as L
+from oracle import magi_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+PRE = 128 ** -0.5 * 1.4426950408889634
+
+
+def _inputs(dev, Tq, Tk, Hq, Hkv, seed):
+    q, k, v = O.synthetic_qkv(Tq, Tk, Hq, Hkv, 128, seed=seed)
+    return q.to(dev), k.to(dev), v.to(dev)
+
+
+def _same_but_for_the_order(a, b, lse_a, lse_b):
+    """fp32 sums of at most 2^13 terms in another order differ by a few 2^-24 of the sum of the terms' sizes (values of about 1,
+    outputs of about 0.05): far less than half a bf16 step, so elements differ by one such step at most, or where they
+    are near 0 by 1e-5."""
+    d = (a.float() - b.float()).abs()
+    assert torch.isfinite(a).all() and (d <= b.float().abs() * 2.0 ** -7 + 1e-5).all(), d.max().item()
+    fin = torch.isfinite(lse_b)
+    assert torch.equal(fin, torch.isfinite(lse_a)) and (lse_a - lse_b)[fin].abs().max().item() <= 1e-5
+
+
+# (rows per range, ranges, cached ranges, heads, max_seqlen_k): equal pieces, two unequal ones behind whole rounds, odd head counts
+# (padding in the grid), ranges with fewer keys than the launch was sized for (down to fewer tiles than pieces), none at all
+CASES = [(500, 2, 2, 6, 2, 0), (257, 1, 8, 3, 1, 0), (64, 3, 40, 12, 4, 0), (9000, 1, 0, 24, 8, 0), (700, 2, 8, 24, 8, 0),
+         (300, 4, 0, 5, 5, 4000), (1, 1, 4096, 1, 1, 0), (2000, 2, 3, 24, 8, 0)]
+
+
+@pytest.mark.parametrize("mode", ["bounded", "scaled", "norm", "checked", "auto"])
+@pytest.mark.parametrize("rows,n,sp,Hq,Hkv,max_k", CASES)
+def test_split_items_give_what_whole_ones_give(dev, rows, n, sp, Hq, Hkv, max_k, mode):
+    Tk = (sp + n) * rows
+    mk = max_k or Tk
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    assert cus != 256 or L.lib().magi_attn_split_bytes(Hq, Hkv, n, rows, mk) > 0
+    q, k, v = _inputs(dev, n * rows + 7, Tk, Hq, Hkv, seed=rows + n)
+    qr = torch.tensor([[i * rows, (i + 1) * rows] for i in range(n)], dtype=torch.int32, device=dev)
+    kr = torch.tensor([[0, (sp + 1 + i) * rows] for i in range(n)], dtype=torch.int32, device=dev)
+    if max_k:
+        kr[0] = kr[0, 0]  # no keys
+        kr[1, 1] = 3
+    kw = {"bounded": {"q_prescaled": True, "score_bound": 40.0}, "scaled": {"score_bound": 40.0}, "checked": {"checked": True},
+          "norm": {"score_bound": 40.0, "q_norm": (torch.zeros(128, device=dev), None, 1e-6)}, "auto": {"auto_bound": True}}[mode]
+    if mode == "bounded":
+        q = (q.float() * PRE).bfloat16()
+    n0 = M.lib().magi_launch_count()
+    a, la = M.range_attention(q, k, v, qr, kr, rows, mk, **kw)
+    n1 = M.lib().magi_launch_count()
+    b, lb = M.range_attention(q, k, v, qr, kr, rows, mk, split_keys=False, **kw)
+    assert n1 - n0 == M.lib().magi_launch_count() - n1 + (1 if cus == 256 else 0)
+    _same_but_for_the_order(a, b, la, lb)
+    assert torch.equal(a, M.range_attention(q, k, v, qr, kr, rows, mk, **kw)[0])  # whatever order the pieces end in
+    if rows == 500 and mode != "norm":  # (the oracle takes normed q)
+        ref = O.range_attention((q.float() / PRE if mode == "bounded" else q).bfloat16().cpu(), k.cpu(), v.cpu(), qr.cpu().numpy(), kr.cpu().numpy())
+        assert (a[:n * rows].float().cpu() - ref[:n * rows]).abs().max().item() <= 2e-2
+
+
+@pytest.mark.parametrize("where", ["everywhere", "first piece", "last piece", "tiny sums", "large values", "side segment"])
+def test_split_blocks_outside_the_window_are_computed_again(dev, where):
+    rows, Hq, Hkv, Tk = 300, 4, 2, 3000
+    q, k, v = _inputs(dev, 2 * rows, Tk, Hq, Hkv, seed=11)
+    k2 = v2 = None
+    split = Tk
+    if where == "everywhere":
+        q = (q.float() * 30).bfloat16()
+    elif where == "first piece":
+        k[2, 1] *= 60
+    elif where == "last piece":
+        k[-3, 0] *= 60
+    elif where == "tiny sums":
+        k[:, 0] = (k[:, 0].float() * 0.05 + 8.0).bfloat16()
+        q[3, 0] = -8.0
+    elif where == "large values":
+        v[:, 1] *= 2.0 ** 100
+    else:
+        split = 1501
+        k[split + 5, 1] *= 60
+    qr = torch.tensor([[0, rows], [rows, 2 * rows]], dtype=torch.int32, device=dev)
+    kr = torch.tensor([[0, Tk], [0, Tk - 1]], dtype=torch.int32, device=dev)
+    kw = {}
+    kc, vc = k, v
+    if split < Tk:
+        kc, vc = k[:split].contiguous(), v[:split].contiguous()
+        kw = {"k2": k[split:].contiguous(), "v2": v[split:].contiguous(), "k_split": split}
+    n0 = M.lib().magi_launch_count()
+    a, la = M.range_attention(q, kc, vc, qr, kr, rows, Tk, checked=True, **kw)
+    n1 = M.lib().magi_launch_count() - n0
+    b, lb = M.range_attention(q, kc, vc, qr, kr, rows, Tk, **kw)
+    assert n1 == 3 or torch.cuda.get_device_properties(dev).multi_processor_count != 256
+    # probabilities are rounded to bf16 relative to different maxima: 2^-8 each, of sums of values of the column's size
+    scale = v.float().abs().amax(dim=(0, 2)).repeat_interleave(Hq // Hkv)[None, :, None]
+    assert torch.isfinite(a).all() and ((a.float() - b.float()).abs() <= 2.0 ** -7 * scale).all()
+    assert (la - lb).abs().max().item() <= 1e-3
+
+
+def test_a_workspace_that_is_too_small_leaves_the_items_whole(dev, monkeypatch):
+    q, k, v = _inputs(dev, 256, 4096, 2, 1, seed=5)
+    qr = torch.tensor([[0, 256]], dtype=torch.int32, device=dev)
+    kr = torch.tensor([[0, 4096]], dtype=torch.int32, device=dev)
+    call = lambda **kw: M.range_attention(q, k, v, qr, kr, 256, 4096, score_bound=40.0, **kw)[0]
+    whole = call(split_keys=False)
+    real = L.lib().magi_attn_split_bytes
+    monkeypatch.setattr(L.lib(), "magi_attn_split_bytes", lambda *a: max(real(*a) - 1, 16))
+    n0 = M.lib().magi_launch_count()
+    assert torch.equal(call(), whole) and M.lib().magi_launch_count() - n0 == 1
