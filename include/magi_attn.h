@@ -221,15 +221,15 @@ typedef struct magi_attn_args {
   int32_t q_batch_rows;
   int64_t q_stride_b, o_stride_b;
   /* Optional scratch memory on the DEVICE (any content, 16-byte aligned, one for each of the calls that may overlap), of
-   * magi_attn_split_bytes() or more.  With it, a launch of the kernel without a running maximum whose last round of workgroups would leave
-   * part of the chip idle has the keys of that round's rows shared by several workgroups, whose unnormalised fp32 sums a
+   * magi_attn_split_bytes() or more.  With it, a launch of the fp8 kernel, or of the bf16 kernel without a running maximum, whose last round of
+   * workgroups would leave part of the chip idle has the keys of that round's rows shared by several workgroups, whose unnormalised fp32 sums a
    * launch behind it adds in the order of the keys (same precision, deterministic).  NULL, or too small: not split. */
   void* split_workspace;
   int64_t split_workspace_bytes;
 } magi_attn_args;
 
-/* Bytes of split_workspace that a bf16 call of these sizes makes use of; 0: such a call is not split. */
-int64_t magi_attn_split_bytes(int32_t Hq, int32_t Hkv, int32_t n_ranges, int32_t max_seqlen_q, int32_t max_seqlen_k);
+/* Bytes of split_workspace that a call of these sizes makes use of (dtype: MAGI_DTYPE_*); 0: such a call is not split. */
+int64_t magi_attn_split_bytes(int32_t Hq, int32_t Hkv, int32_t n_ranges, int32_t max_seqlen_q, int32_t max_seqlen_k, int32_t dtype);
 
 int magi_attn_fwd(const magi_attn_args* args, void* stream);
 

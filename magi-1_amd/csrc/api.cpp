@@ -88,7 +88,9 @@ unsigned items_per_xcd(int Hq, int Hkv, int n_ranges, int tiles_per_range) {
 // Which items of a 256-row launch without a running maximum have their keys shared by several workgroups (AttnKernArgs::split_*).
 struct SplitPlan {
   unsigned from, pieces, num, den;
-  int64_t bytes(unsigned per_xcd) const { return from < per_xcd ? 4ll * magi::SPLIT_FLOATS * 8 * (per_xcd - from) * pieces : 0; }
+  bool fp8;
+  int64_t piece_bytes() const { return 4ll * (fp8 ? magi::SPLIT_FLOATS_FP8 : magi::SPLIT_FLOATS); }
+  int64_t bytes(unsigned per_xcd) const { return from < per_xcd ? piece_bytes() * 8 * (per_xcd - from) * pieces : 0; }
 };
 // The last round of a launch has `left` items for `slots` places (two workgroups per CU) on each XCD.  At most half of them: equal pieces, as
 // many as the places allow.  More: two pieces, the first so much longer that the others' second pieces fill the places
@@ -100,12 +102,18 @@ struct SplitPlan {
 // 845 / 818; and where the rule says no: 60 over 25000 keys 1131 / 1144, 54 over 4608 keys 159 / 174, 18 over 1536 keys
 // 48 / 52.  4 over 99000 keys behind five whole rounds 9009 / 8583.  Behind eight and more
 // the round is a small part of the launch.
-SplitPlan split_plan(unsigned items, int max_seqlen_k) {
-  SplitPlan s = {UINT32_MAX, 1, 1, 1};
-  const unsigned slots = (unsigned)compute_units() / 4;  // of one XCD: two workgroups per CU
+// fp8: three workgroups of 128 rows per CU; a tile takes 1.4 us, 0.46 of that alone on a CU, 0.73 two by two.  Measured, whole /
+// split, with items in the last round: 30 of 96 over 46800 keys 2662 / 2551 us, 24 over 25000 keys 866 / 779, 18 over 14400 keys 474
+// / 414; and not split, 30 over 9360 keys 570 / 564, 48 over 6000 keys 192 / 203.  The probabilities are rounded to
+// e4m3 relative to the maximum so far, which a piece sees only its part of: rows that are split differ from whole ones
+// by as much as those two roundings do (3e-2 of the result; neither is nearer to the exact one).  So only launches
+// whose rows are mostly whole are split, behind one whole round at least.
+SplitPlan split_plan(unsigned items, int max_seqlen_k, bool fp8) {
+  SplitPlan s = {UINT32_MAX, 1, 1, 1, fp8};
+  const unsigned cus = (unsigned)compute_units() / 8, slots = cus * (fp8 ? 3 : 2);  // of one XCD
   if (slots == 0 || max_seqlen_k <= 0) return s;
   const unsigned rounds = items / slots, left = items % slots, tiles = (unsigned)(max_seqlen_k + 63) / 64;
-  if (left == 0 || rounds >= 8) return s;
+  if (left == 0 || rounds >= 8 || (fp8 && rounds == 0)) return s;
   unsigned num, den;
   if (left * 2 > slots) {
     num = (left + slots - left - 1) / (slots - left);
@@ -116,9 +124,15 @@ SplitPlan split_plan(unsigned items, int max_seqlen_k) {
     if (den > tiles / 8) den = tiles / 8;
   }
   if (den < 2 || num > 4 || tiles < 4 * den) return s;
-  const double round_us = 3.0 * tiles, piece = (double)num / den, mb = 8e-6 * left * (den - num + 1) * 4 * magi::SPLIT_FLOATS;
-  const double saved_us = left * 2 > slots ? 0.5 * (1.0 - piece) * round_us : ((rounds >= 2 ? 0.5 : 0.62) - piece) * round_us;
-  if (saved_us < 8.0 + 0.3 * mb) return s;
+  const double piece = (double)num / den, cost_us = 8.0 + 0.3 * 8e-6 * left * (den - num + 1) * s.piece_bytes();
+  double saved_us;
+  if (fp8) {
+    const double round = left <= cus ? 0.46 : left <= 2 * cus ? 0.73 : 1.0;
+    saved_us = (round - piece) * 1.4 * tiles / 1.5;
+  } else {
+    saved_us = (left * 2 > slots ? 0.5 * (1.0 - piece) : (rounds >= 2 ? 0.5 : 0.62) - piece) * 3.0 * tiles;
+  }
+  if (saved_us < cost_us) return s;
   s.from = rounds * slots;
   s.pieces = den - num + 1;
   s.num = num;
@@ -148,12 +162,14 @@ uint64_t magi_launch_count(void) { return g_launches.load(std::memory_order_rela
 
 const char* magi_last_error(void) { return g_err; }
 
-int64_t magi_attn_split_bytes(int32_t Hq, int32_t Hkv, int32_t n_ranges, int32_t max_seqlen_q, int32_t max_seqlen_k) {
+int64_t magi_attn_split_bytes(int32_t Hq, int32_t Hkv, int32_t n_ranges, int32_t max_seqlen_q, int32_t max_seqlen_k,
+                              int32_t dtype) {
   if (Hq <= 0 || Hkv <= 0 || Hq % Hkv || n_ranges <= 0 || max_seqlen_q <= 0) return 0;
-  const int tiles = max_seqlen_q / 256 + (max_seqlen_q % 256 != 0);
+  const bool fp8 = dtype == MAGI_DTYPE_FP8_E4M3;
+  const int rows = fp8 ? 128 : 256, tiles = max_seqlen_q / rows + (max_seqlen_q % rows != 0);
   if ((double)Hq * n_ranges * tiles > 2.0e9) return 0;
   const unsigned items = items_per_xcd(Hq, Hkv, n_ranges, tiles);
-  return split_plan(items, max_seqlen_k).bytes(items);
+  return split_plan(items, max_seqlen_k, fp8).bytes(items);
 }
 
 int magi_attn_fwd(const magi_attn_args* p, void* stream) {
@@ -382,8 +398,9 @@ int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace) {
     if (total > 2.0e9) return fail(MAGI_EINVAL, "magi_attn_fwd: grid too large (%.3g workgroups)", total);
     a.per_xcd = items_per_xcd(p->Hq, p->Hkv, p->n_ranges, a.tiles_per_range);
     a.split_from = UINT32_MAX;
-    if (bounded && a.block_m == 256 && !mfma32 && p->split_workspace) {
-      const SplitPlan s = split_plan(a.per_xcd, p->max_seqlen_k);
+    const bool fp8 = p->dtype == MAGI_DTYPE_FP8_E4M3;
+    if ((fp8 || (bounded && a.block_m == 256 && !mfma32)) && p->split_workspace) {
+      const SplitPlan s = split_plan(a.per_xcd, p->max_seqlen_k, fp8);
       if (s.from < a.per_xcd && s.bytes(a.per_xcd) <= p->split_workspace_bytes) {
         a.partial = static_cast<float*>(p->split_workspace);
         a.split_from = s.from;

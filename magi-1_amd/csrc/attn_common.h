@@ -243,6 +243,24 @@ __device__ __forceinline__ WorkItem locate_work(const AttnKernArgs& a, int BM, i
   return wi;
 }
 
+// Items whose keys are shared by several workgroups (a.split_*): what this workgroup has of its item.
+struct SplitPiece {
+  float* out;  // nullptr: a whole item
+  unsigned piece;
+};
+// workgroup `block` of the grid with split items -> `block` of the grid without, and the piece of it
+template <int FLOATS>
+__device__ __forceinline__ SplitPiece split_piece(const AttnKernArgs& a, unsigned& block) {
+  const unsigned pos = block >> 3, xcd = block & 7u;
+  if (pos < a.split_from) return {nullptr, 0u};
+  const unsigned items = a.per_xcd - a.split_from;  // (the longer first pieces of all items ahead of the others)
+  const unsigned piece = (pos - a.split_from) / items, i = (pos - a.split_from) - piece * items;
+  block = ((a.split_from + i) << 3) | xcd;
+  return {a.partial + (long)((i * 8u + xcd) * a.split_pieces + piece) * FLOATS, piece};
+}
+__device__ __forceinline__ unsigned split_cut(const AttnKernArgs& a, unsigned tiles, unsigned piece) {
+  return piece == 0u ? 0u : (unsigned)((unsigned long long)tiles * (a.split_num + piece - 1u) / a.split_den);
+}
 // A q row whose range has no keys: zeros, lse = -inf.  Lane (row, g) writes half g of the 256-byte row.
 __device__ __forceinline__ void store_empty_row(const AttnKernArgs& a, const WorkItem& wi, int q_row, int g) {
   char* op = a.out + row_offset(a, q_row, a.os_t, a.os_b) + wi.o_head + g * 128;

@@ -94,22 +94,6 @@ constexpr float SUM_MIN = 0x1p-16f, SUM_MAX = 0x1p64f;
 // A launch whose last round of workgroups leaves slots (two per CU) empty has the keys of that round's items shared by
 // several workgroups each (a.split_*, split_plan in api.cpp).  Without a running maximum the pieces simply add up: each leaves its
 // unnormalised accumulators and row sums in fp32, attn_fwd_bf16_merge_kernel adds them in the order of the keys.
-struct SplitPiece {
-  float* out;  // nullptr: a whole item
-  unsigned piece;
-};
-// workgroup `block` of the grid with split items -> `block` of the grid without, and the piece of it
-__device__ __forceinline__ SplitPiece split_piece(const AttnKernArgs& a, unsigned& block) {
-  const unsigned pos = block >> 3, xcd = block & 7u;
-  if (pos < a.split_from) return {nullptr, 0u};
-  const unsigned items = a.per_xcd - a.split_from;  // (the longer first pieces of all items ahead of the others)
-  const unsigned piece = (pos - a.split_from) / items, i = (pos - a.split_from) - piece * items;
-  block = ((a.split_from + i) << 3) | xcd;
-  return {a.partial + (long)((i * 8u + xcd) * a.split_pieces + piece) * SPLIT_FLOATS, piece};
-}
-__device__ __forceinline__ unsigned split_cut(const AttnKernArgs& a, unsigned tiles, unsigned piece) {
-  return piece == 0u ? 0u : (unsigned)((unsigned long long)tiles * (a.split_num + piece - 1u) / a.split_den);
-}
 __device__ __forceinline__ void store_partial_zero(float* out, int w, int l) {
   f32x4v* const dst = (f32x4v*)out + w * 2048 + l;
 #pragma unroll
@@ -136,7 +120,7 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_bf16_x16_kernel(const AttnKer
   const int tid = threadIdx.x;
   if (CHECK && tid == 0) s_over = 0;
   unsigned block = blockIdx.x;
-  const SplitPiece sp = split_piece(a, block);
+  const SplitPiece sp = split_piece<SPLIT_FLOATS>(a, block);
   const WorkItem wi = locate_work(a, BM, tid, s_sel, block);
   if (!wi.valid) return;
   const int qe = wi.qe;
@@ -766,11 +750,6 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_bf16_redo_kernel(const AttnKe
 }  // namespace
 
 namespace {
-unsigned split_items(const AttnKernArgs& a) { return a.split_from < a.per_xcd ? a.per_xcd - a.split_from : 0u; }
-dim3 grid_of(const AttnKernArgs& a) {
-  const unsigned items = split_items(a);
-  return dim3(8u * (a.per_xcd - items + items * a.split_pieces));
-}
 template <bool CHECK>
 void launch_merge(const AttnKernArgs& a, hipStream_t stream) {
   if (const unsigned items = split_items(a)) {
@@ -782,7 +761,7 @@ void launch_merge(const AttnKernArgs& a, hipStream_t stream) {
 }  // namespace
 
 hipError_t launch_attn_fwd_bf16_x16(const AttnKernArgs& a, hipStream_t stream) {
-  const dim3 grid = grid_of(a);
+  const dim3 grid(split_grid(a));
   if (a.q_norm_gamma)  // raw q, normalised while it is loaded (cross attention)
     hipLaunchKernelGGL(attn_fwd_bf16_x16_kernel<Q_NORM>, grid, dim3(256), 0, stream, a);
   else if (a.flags & ATTN_SCALE_Q)  // unscaled q, scaled while it is loaded (the reference-shaped callables)
@@ -794,7 +773,7 @@ hipError_t launch_attn_fwd_bf16_x16(const AttnKernArgs& a, hipStream_t stream) {
 }
 
 hipError_t launch_attn_fwd_bf16_checked(const AttnKernArgs& a, int compute_units, hipStream_t stream) {
-  const dim3 grid = grid_of(a);
+  const dim3 grid(split_grid(a));
   // (two workgroups per CU, a multiple of eight so that a block keeps its XCD)
   const unsigned most = (unsigned)(compute_units / 4) * 8u;
   const unsigned blocks = 8u * a.per_xcd;

@@ -33,6 +33,31 @@ constexpr int BM = 32 * NW;
 constexpr int LOADS = 8 / NW;  // direct loads per wave per matrix per tile (8 rows each)
 constexpr float P_SHIFT = 8.f;
 
+// acc * inv as bf16 rows wi.q0 + row0 .. + 31 of out; acc in the lane layout of the PV MFMAs.
+// A lane holds four consecutive features per (mb, b), its partner in the other half wave the next four: the
+// halves trade the odd-b registers of the lower half for the even-b registers of the upper one, after which
+// every lane owns eight consecutive features and stores 16 bytes at a time.  (The row address is derived from
+// an opaque copy of the lane index so that it is computed here and not carried through the main loop.)
+__device__ __forceinline__ void store_rows(const AttnKernArgs& a, const WorkItem& wi, int row0, int l, const f32x16 (&acc)[4], float inv) {
+  int lane_e = l;
+  asm volatile("" : "+v"(lane_e));
+  const bool row_ok = wi.q0 + row0 + (l & 31) < wi.qe;
+  char* const op = a.out + (long)(wi.q0 + row0 + (lane_e & 31)) * a.os_t + wi.o_head + 16 * (lane_e >> 5);
+#pragma unroll
+  for (int mb = 0; mb < 4; ++mb)
+#pragma unroll
+    for (int bp = 0; bp < 2; ++bp) {
+      unsigned ev[2], od[2];
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        ev[e] = pack_bf16x2(acc[mb][8 * bp + 2 * e] * inv, acc[mb][8 * bp + 2 * e + 1] * inv);
+        od[e] = pack_bf16x2(acc[mb][8 * bp + 4 + 2 * e] * inv, acc[mb][8 * bp + 4 + 2 * e + 1] * inv);
+        half_swap(ev[e], od[e]);  // lower half: (own even, partner's even); upper half: (partner's odd, own odd)
+      }
+      if (row_ok) *(u32x4*)(op + (32 * mb + 16 * bp) * 2) = u32x4{ev[0], ev[1], od[0], od[1]};
+    }
+}
+
 // FASTP (with POW2): the probabilities come from a piecewise-linear exp2 built on the matrix pipe's scaling
 // instead of the quarter-rate v_exp_f32: the score registers hold e4m3 codes (see the softmax below).
 template <bool POW2, bool FASTP = false>
@@ -48,10 +73,12 @@ __global__ __launch_bounds__(64 * NW, 3) void attn_fwd_fp8_kernel(const AttnKern
   __shared__ int s_sel[LOCATE_WORDS];
 
   const int tid = threadIdx.x;
-  const WorkItem wi = locate_work(a, BM, tid, s_sel, blockIdx.x);
+  unsigned block = blockIdx.x;
+  const SplitPiece sp = split_piece<SPLIT_FLOATS_FP8>(a, block);
+  const WorkItem wi = locate_work(a, BM, tid, s_sel, block);
   if (!wi.valid) return;
-  const int h = wi.h, kvh = wi.kvh, q0 = wi.q0, qe = wi.qe, ks = wi.ks, ke = wi.ke;
-  const long o_head = wi.o_head;
+  const int h = wi.h, kvh = wi.kvh, q0 = wi.q0, qe = wi.qe;
+  int ks = wi.ks, ke = wi.ke;
 
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l = tid & 63, i = l & 31, g = l >> 5;
@@ -85,6 +112,22 @@ __global__ __launch_bounds__(64 * NW, 3) void attn_fwd_fp8_kernel(const AttnKern
   for (int cidx = ks / C; cidx <= (ke - 1) / C; ++cidx)
     v_max = fmaxf(v_max, a.v_scale[(long)cidx * a.Hkv + kvh + (cidx < a.scale_split_chunk ? 0 : a.v2_scale_delta)]);
   const float log2_vmax = __builtin_amdgcn_logf(v_max);
+  if (sp.out) {  // (a piece: behind v_max, which all pieces of an item share)
+    const unsigned tiles = (unsigned)(ke - ks + BN - 1) / BN;
+    const int b = (int)split_cut(a, tiles, sp.piece), e = (int)split_cut(a, tiles, sp.piece + 1);
+    if (b == e) {  // (a range with fewer tiles than pieces)
+      f32x4* const dst = (f32x4*)sp.out + w * 1024 + l;
+#pragma unroll
+      for (int j = 0; j < 16; ++j) dst[j * 64] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (g == 0) {
+        sp.out[128 * 128 + 32 * w + i] = 0.f;
+        sp.out[128 * 128 + 128 + 32 * w + i] = -__builtin_inff();
+      }
+      return;
+    }
+    ke = min(ke, ks + e * BN);
+    ks += b * BN;
+  }
 
   // ---- tile loader: wave w fills rows 8*(w + NW*j) .. +7; lane l sits at row +(l >> 3), slot l & 7 ----
   const int lrow = l >> 3, slot = l & 7;
@@ -414,32 +457,59 @@ __global__ __launch_bounds__(64 * NW, 3) void attn_fwd_fp8_kernel(const AttnKern
   }
 
   if (!wave_on) return;
+  if (sp.out) {  // accumulators in units of v, row sum and maximum, in the lane layout of the MFMA results
+    const float unit = v_max * __builtin_amdgcn_exp2f(-P_SHIFT);
+    f32x4* const dst = (f32x4*)sp.out + w * 1024 + l;
+#pragma unroll
+    for (int mb = 0; mb < 4; ++mb)
+#pragma unroll
+      for (int b = 0; b < 4; ++b)
+        dst[(4 * mb + b) * 64] = f32x4{o_acc[mb][4 * b] * unit, o_acc[mb][4 * b + 1] * unit, o_acc[mb][4 * b + 2] * unit, o_acc[mb][4 * b + 3] * unit};
+    if (g == 0) {
+      sp.out[128 * 128 + 32 * w + i] = l_run;
+      sp.out[128 * 128 + 128 + 32 * w + i] = m_run;
+    }
+    return;
+  }
   const float l_tot = l_run;  // (the row-sum MFMA hands every lane the sum over all keys of its query)
-  const float inv = v_max * __builtin_amdgcn_exp2f(-P_SHIFT) / l_tot;
-  // A lane holds four consecutive features per (mb, b), its partner in the other half wave the next four: the
-  // halves trade the odd-b registers of the lower half for the even-b registers of the upper one, after which
-  // every lane owns eight consecutive features and stores 16 bytes at a time.  (The row address is derived from
-  // an opaque copy of the lane index so that it is computed here and not carried through the main loop.)
-  int lane_e = l;
-  asm volatile("" : "+v"(lane_e));
-  char* const op = a.out + (long)(q0 + 32 * w + (lane_e & 31)) * a.os_t + o_head + 16 * (lane_e >> 5);
+  store_rows(a, wi, 32 * w, l, o_acc, v_max * __builtin_amdgcn_exp2f(-P_SHIFT) / l_tot);
+  if (a.lse && g == 0 && row_ok) a.lse[(long)h * a.total_q + q_row] = (m_run + __builtin_amdgcn_logf(l_tot)) * 0.6931471805599453f;
+}
+
+// The split items of a launch of the kernel above (a.split_*): brings the pieces' sums to a common maximum, adds them in the order
+// of the keys, normalises, writes the rows.  One workgroup per item, lanes and wavefronts as there.  Memory bound.
+__global__ __launch_bounds__(64 * NW) void attn_fwd_fp8_merge_kernel(const AttnKernArgs a) {
+  __shared__ int s_sel[LOCATE_WORDS];
+  const int tid = threadIdx.x, l = tid & 63, i = l & 31, g = l >> 5;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const WorkItem wi = locate_work(a, BM, tid, s_sel, blockIdx.x + 8u * a.split_from);
+  if (!wi.valid || wi.ke <= wi.ks || wi.q0 + 32 * w >= wi.qe) return;
+  const int pieces = (int)a.split_pieces, row = 32 * w + i;
+  const float* const base = a.partial + (long)blockIdx.x * pieces * SPLIT_FLOATS_FP8;
+  float m = -__builtin_inff();
+  for (int p = 0; p < pieces; ++p) m = fmaxf(m, base[(long)p * SPLIT_FLOATS_FP8 + 128 * 128 + 128 + row]);
+  float sum = 0.f;
+  f32x16 o[4];
 #pragma unroll
   for (int mb = 0; mb < 4; ++mb)
 #pragma unroll
-    for (int bp = 0; bp < 2; ++bp) {
-      unsigned ev[2], od[2];
+    for (int v = 0; v < 16; ++v) o[mb][v] = 0.f;
+  for (int p = 0; p < pieces; ++p) {
+    const float* const src = base + (long)p * SPLIT_FLOATS_FP8;
+    const float f = __builtin_amdgcn_exp2f(src[128 * 128 + 128 + row] - m);
+    sum += src[128 * 128 + row] * f;
+    const f32x4* const acc = (const f32x4*)src + w * 1024 + l;
 #pragma unroll
-      for (int e = 0; e < 2; ++e) {
-        ev[e] = pack_bf16x2(o_acc[mb][8 * bp + 2 * e] * inv, o_acc[mb][8 * bp + 2 * e + 1] * inv);
-        od[e] = pack_bf16x2(o_acc[mb][8 * bp + 4 + 2 * e] * inv, o_acc[mb][8 * bp + 4 + 2 * e + 1] * inv);
-        half_swap(ev[e], od[e]);  // lower half: (own even, partner's even); upper half: (partner's odd, own odd)
+    for (int mb = 0; mb < 4; ++mb)
+#pragma unroll
+      for (int b = 0; b < 4; ++b) {
+        const f32x4 x = acc[(4 * mb + b) * 64];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[mb][4 * b + e] += x[e] * f;
       }
-      if (row_ok) *(u32x4*)(op + (32 * mb + 16 * bp) * 2) = u32x4{ev[0], ev[1], od[0], od[1]};
-    }
-  if (row_ok) {
-    if (a.lse && g == 0)
-      a.lse[(long)h * a.total_q + q_row] = (m_run + __builtin_amdgcn_logf(l_tot)) * 0.6931471805599453f;
   }
+  store_rows(a, wi, 32 * w, l, o, 1.f / sum);
+  if (a.lse && g == 0 && wi.q0 + row < wi.qe) a.lse[(long)wi.h * a.total_q + wi.q0 + row] = (m + __builtin_amdgcn_logf(sum)) * 0.6931471805599453f;
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -594,13 +664,18 @@ __global__ __launch_bounds__(QT1) void quantize_groups_kernel(const char* x, lon
 }  // namespace
 
 hipError_t launch_attn_fwd_fp8(const AttnKernArgs& a, hipStream_t stream) {
-  const unsigned grid = a.per_xcd * 8u;
+  const unsigned grid = split_grid(a);
   if ((a.flags & 1) && (a.flags & 4))
     hipLaunchKernelGGL((attn_fwd_fp8_kernel<true, true>), dim3(grid), dim3(64 * NW), 0, stream, a);
   else if (a.flags & 1)
     hipLaunchKernelGGL(attn_fwd_fp8_kernel<true>, dim3(grid), dim3(64 * NW), 0, stream, a);
   else
     hipLaunchKernelGGL(attn_fwd_fp8_kernel<false>, dim3(grid), dim3(64 * NW), 0, stream, a);
+  if (const unsigned items = split_items(a)) {
+    AttnKernArgs m = a;
+    m.flags &= ~ATTN_ZERO_GAPS;  // (the rows no range covers are clear by now)
+    hipLaunchKernelGGL(attn_fwd_fp8_merge_kernel, dim3(8u * items), dim3(64 * NW), 0, stream, m);
+  }
   return hipGetLastError();
 }
 

@@ -48,7 +48,7 @@ struct AttnKernArgs {
   int gate_want;
   // Checked launches (MAGI_ATTN_CHECKED): four words per item, one per wavefront of the 256-row kernel
   int* verdict;
-  // Items whose keys are shared by several workgroups (split_plan in api.cpp; the 256-row kernel only): the items from
+  // Items whose keys are shared by several workgroups (split_plan in api.cpp; the 256-row bf16 kernel and the fp8 kernel): the items from
   // position split_from of each XCD's list on, in split_pieces pieces each.  Piece p starts at tile n_tiles * (split_num +
   // p - 1) / split_den of the item's key range, piece 0 at tile 0.  `partial`: SPLIT_FLOATS floats per piece.
   float* partial;
@@ -56,6 +56,14 @@ struct AttnKernArgs {
 };
 // 256 rows x 128 accumulators, and the 256 row sums behind them
 constexpr int SPLIT_FLOATS = 256 * 128 + 256;
+// fp8: 128 rows x 128 accumulators, 128 row sums, 128 row maxima
+constexpr int SPLIT_FLOATS_FP8 = 128 * 128 + 256;
+// the items of one XCD's list that are split, and the workgroups of the launch
+inline unsigned split_items(const AttnKernArgs& a) { return a.split_from < a.per_xcd ? a.per_xcd - a.split_from : 0u; }
+inline unsigned split_grid(const AttnKernArgs& a) {
+  const unsigned items = split_items(a);
+  return 8u * (a.per_xcd - items + items * a.split_pieces);
+}
 
 
 // internal flag: the caller promised bounded scores (magi_attn_args.score_bound within MAGI_SCORE_BOUND_MAX)

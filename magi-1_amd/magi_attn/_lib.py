@@ -136,7 +136,7 @@ def lib() -> C.CDLL:
                                "rebuild the library (`make -C magi-1_amd/csrc`)")
         l.magi_launch_count.restype = C.c_uint64
         l.magi_last_error.restype = C.c_char_p
-        l.magi_attn_split_bytes.argtypes = [C.c_int32] * 5
+        l.magi_attn_split_bytes.argtypes = [C.c_int32] * 6
         l.magi_attn_split_bytes.restype = C.c_int64
         l.magi_attn_fwd.argtypes = [C.POINTER(AttnArgs), C.c_void_p]
         l.magi_attn_fwd.restype = C.c_int

@@ -213,8 +213,9 @@ def range_attention(
     if auto_bound and not static_scratch:
         workspace = torch.empty(4, dtype=torch.float32, device=q.device)  # (alive until the launches are enqueued)
     split, split_bytes = None, 0
-    if split_keys and not static_scratch and max_seqlen_k >= 512 and (checked or auto_bound or 0.0 < score_bound <= L.MAGI_SCORE_BOUND_MAX):
-        split_bytes = L.lib().magi_attn_split_bytes(Hq, Hkv, max(n, 0), int(max_seqlen_q), int(max_seqlen_k))
+    if split_keys and not static_scratch and max_seqlen_k >= 512 and (
+            checked or auto_bound or 0.0 < score_bound <= L.MAGI_SCORE_BOUND_MAX or q.dtype is torch.float8_e4m3fn):
+        split_bytes = L.lib().magi_attn_split_bytes(Hq, Hkv, max(n, 0), int(max_seqlen_q), int(max_seqlen_k), _dtype_code(q))
         if split_bytes:
             try:
                 split = torch.empty(split_bytes, dtype=torch.uint8, device=q.device)
@@ -283,7 +284,7 @@ def _sharing_keys_pays(Hq: int, Hkv: int, n_ranges: int, max_seqlen_q: int, max_
     workgroups = Hq * n_ranges * ((max_seqlen_q + 255) // 256)
     slots = 2 * torch.cuda.get_device_properties(device).multi_processor_count
     return ((3 * workgroups <= slots or (n_ranges == 1 and workgroups <= slots))
-            and L.lib().magi_attn_split_bytes(Hq, Hkv, n_ranges, int(max_seqlen_q), int(max_seqlen_k)) > 0)
+            and L.lib().magi_attn_split_bytes(Hq, Hkv, n_ranges, int(max_seqlen_q), int(max_seqlen_k), L.MAGI_DTYPE_BF16) > 0)
 
 
 def _unbounded_mode(q, k, n_ranges: int, max_seqlen_q: int, max_seqlen_k: int, keys: float, score_bound: float,

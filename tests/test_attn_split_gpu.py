@@ -39,7 +39,7 @@ def test_split_items_give_what_whole_ones_give(dev, rows, n, sp, Hq, Hkv, max_k,
     Tk = (sp + n) * rows
     mk = max_k or Tk
     cus = torch.cuda.get_device_properties(dev).multi_processor_count
-    assert cus != 256 or L.lib().magi_attn_split_bytes(Hq, Hkv, n, rows, mk) > 0
+    assert cus != 256 or L.lib().magi_attn_split_bytes(Hq, Hkv, n, rows, mk, L.MAGI_DTYPE_BF16) > 0
     q, k, v = _inputs(dev, n * rows + 7, Tk, Hq, Hkv, seed=rows + n)
     qr = torch.tensor([[i * rows, (i + 1) * rows] for i in range(n)], dtype=torch.int32, device=dev)
     kr = torch.tensor([[0, (sp + 1 + i) * rows] for i in range(n)], dtype=torch.int32, device=dev)
@@ -110,3 +110,56 @@ def test_a_workspace_that_is_too_small_leaves_the_items_whole(dev, monkeypatch):
     monkeypatch.setattr(L.lib(), "magi_attn_split_bytes", lambda *a: max(real(*a) - 1, 16))
     n0 = M.lib().magi_launch_count()
     assert torch.equal(call(), whole) and M.lib().magi_launch_count() - n0 == 1
+
+
+def _exact(q, k, v, kr, rows):
+    """float64 attention of q (scale and log2(e) folded in) over the operands as given."""
+    G = q.shape[1] // k.shape[1]
+    out = []
+    for i, (b, e) in enumerate(kr):
+        kk, vv = (t[b:e].double().repeat_interleave(G, 1).transpose(0, 1) for t in (k, v))
+        p = torch.softmax(q[i * rows:(i + 1) * rows].double().transpose(0, 1) @ kk.transpose(1, 2) * 0.6931471805599453, -1)
+        out.append((p @ vv).transpose(0, 1))
+    return torch.cat(out)
+
+
+@pytest.mark.parametrize("pow2", [True, False])
+@pytest.mark.parametrize("rows,n,sp,Hq,Hkv,chunk,split", [(1300, 1, 12, 80, 8, 1300, None), (1300, 2, 12, 50, 5, 650, 9000),
+                                                          (129, 13, 150, 64, 8, 129, None)])
+def test_split_items_of_the_fp8_kernel(dev, rows, n, sp, Hq, Hkv, chunk, split, pow2):
+    """e4m3 operands with a scale per (chunk, head), cuts inside and at the ends of scale chunks, two key segments: the split launch
+    is as near to float64 on the same operands as the whole one (both round the probabilities to e4m3: 2^-4 each at most)."""
+    Tk, f8 = (sp + n) * rows, torch.float8_e4m3fn
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    assert cus != 256 or L.lib().magi_attn_split_bytes(Hq, Hkv, n, rows, Tk, L.MAGI_DTYPE_FP8_E4M3) > 0
+    q, k, v = _inputs(dev, n * rows, Tk, Hq, Hkv, seed=rows)
+    tab = lambda T, H, x: x * 2.0 ** torch.arange(((T + chunk - 1) // chunk) * H, device=dev).remainder(3).float().view(-1, H)
+    qs, ks, vs = tab(n * rows, Hq, 2.0 ** -6), tab(Tk, Hkv, 2.0 ** -5), tab(Tk, Hkv, 2.0 ** -5)
+    if not pow2:
+        qs, ks, vs = qs * 1.1, ks * 0.9, vs * 1.2
+    row = lambda s, T: s.repeat_interleave(chunk, 0)[:T, :, None]
+    enc = lambda x, s: (x.float() / row(s, x.shape[0])).clamp(-448, 448).to(f8)
+    q8, k8, v8 = enc(q * PRE if pow2 else q, qs), enc(k, ks), enc(v, vs)
+    qr = torch.tensor([[i * rows, (i + 1) * rows] for i in range(n)], dtype=torch.int32, device=dev)
+    ends = [(0, (sp + 1 + i) * rows - 5 * (i == n - 1)) for i in range(n)]
+    kr = torch.tensor(ends, dtype=torch.int32, device=dev)
+    kc, vc, kw = k8, v8, {}
+    if split:
+        kc, vc = k8[:split].contiguous(), v8[:split].contiguous()
+        kw = {"k2": k8[split:].contiguous(), "v2": v8[split:].contiguous(), "k_split": split}
+    call = lambda s: M.range_attention(q8, kc, vc, qr, kr, rows, Tk, q_scale=qs, k_scale=ks, v_scale=vs, scale_chunk_tokens=chunk,
+                                       fp8_pow2_prescaled=pow2, split_keys=s, **kw)
+    n0 = M.lib().magi_launch_count()
+    a, la = call(True)
+    assert M.lib().magi_launch_count() - n0 == (2 if cus == 256 else 1)
+    b, lb = call(False)
+    assert torch.equal(a, call(True)[0])
+    heads = slice(0, Hq, max(1, Hq // 5))  # (float64 on a few heads)
+    G = Hq // Hkv
+    dq = (q8.float() * row(qs, q8.shape[0]))[:, heads] * (1.0 if pow2 else PRE)
+    kv_heads = [h // G for h in range(Hq)][heads]
+    dk, dv = ((t.float() * row(s, Tk))[:, kv_heads] for t, s in ((k8, ks), (v8, vs)))
+    want = _exact(dq, dk, dv, ends, rows)
+    err = lambda x: ((x[:, heads].double() - want).norm() / want.norm()).item()
+    assert torch.isfinite(a).all() and err(a) <= 1.05 * err(b) + 1e-3 and err(b) <= 2.0 ** -4, (err(a), err(b))
+    assert (la - lb).abs().max().item() <= 2e-2  # the row sums are of rounded probabilities too
