@@ -108,12 +108,24 @@ struct SplitPlan {
 // e4m3 relative to the maximum so far, which a piece sees only its part of: rows that are split differ from whole ones
 // by as much as those two roundings do (3e-2 of the result; neither is nearer to the exact one).  So only launches
 // whose rows are mostly whole are split, behind one whole round at least.
-SplitPlan split_plan(unsigned items, int max_seqlen_k, bool fp8) {
+// Several ranges behind a whole round: the items go longest range first, so the last ones belong to the shortest range, and
+// the others' unequal lengths have filled most of the last round already.  The host does not know the lengths; of ranges
+// that end a chunk of max_seqlen_q keys apart the shortest is max_seqlen_k less all but one of these.  bf16, whole / split where
+// that is below half of the longest: four ranges of 1500 to 3750 keys 160 / 188 us, of 2800 to 7015 277 / 308, 10368 rows x 48
+// heads over 2592 to 10368 keys a layer of 2896 / 2999 (but six heads over 13000 to 32440 keys 1458 / 1339); two ranges
+// of one and two chunks of 7070 keys 1317 / 1334; at half and above: three of 11562 to 23124 keys 2746 / 2629, four of
+// 5600 to 9800 475 / 442, two of 32526 to 37947 3971 / 3516.  Ranges of a chunk or less each (a batch) do not differ that way.
+// fp8 gains in all of them or loses nothing (500 / 502 us at the least).
+SplitPlan split_plan(unsigned items, int n_ranges, int max_seqlen_q, int max_seqlen_k, bool fp8) {
   SplitPlan s = {UINT32_MAX, 1, 1, 1, fp8};
   const unsigned cus = (unsigned)compute_units() / 8, slots = cus * (fp8 ? 3 : 2);  // of one XCD
   if (slots == 0 || max_seqlen_k <= 0) return s;
   const unsigned rounds = items / slots, left = items % slots, tiles = (unsigned)(max_seqlen_k + 63) / 64;
   if (left == 0 || rounds >= 8 || (fp8 && rounds == 0)) return s;
+  if (!fp8 && rounds > 0 && n_ranges > 1 && max_seqlen_k > max_seqlen_q) {
+    const int64_t shortest = max_seqlen_k - (int64_t)(n_ranges - 1) * max_seqlen_q;
+    if (2 * shortest < max_seqlen_k || shortest <= max_seqlen_q) return s;
+  }
   unsigned num, den;
   if (left * 2 > slots) {
     num = (left + slots - left - 1) / (slots - left);
@@ -169,7 +181,7 @@ int64_t magi_attn_split_bytes(int32_t Hq, int32_t Hkv, int32_t n_ranges, int32_t
   const int rows = fp8 ? 128 : 256, tiles = max_seqlen_q / rows + (max_seqlen_q % rows != 0);
   if ((double)Hq * n_ranges * tiles > 2.0e9) return 0;
   const unsigned items = items_per_xcd(Hq, Hkv, n_ranges, tiles);
-  return split_plan(items, max_seqlen_k, fp8).bytes(items);
+  return split_plan(items, n_ranges, max_seqlen_q, max_seqlen_k, fp8).bytes(items);
 }
 
 int magi_attn_fwd(const magi_attn_args* p, void* stream) {
@@ -400,7 +412,7 @@ int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace) {
     a.split_from = UINT32_MAX;
     const bool fp8 = p->dtype == MAGI_DTYPE_FP8_E4M3;
     if ((fp8 || (bounded && a.block_m == 256 && !mfma32)) && p->split_workspace) {
-      const SplitPlan s = split_plan(a.per_xcd, p->max_seqlen_k, fp8);
+      const SplitPlan s = split_plan(a.per_xcd, p->n_ranges, p->max_seqlen_q, p->max_seqlen_k, fp8);
       if (s.from < a.per_xcd && s.bytes(a.per_xcd) <= p->split_workspace_bytes) {
         a.partial = static_cast<float*>(p->split_workspace);
         a.split_from = s.from;

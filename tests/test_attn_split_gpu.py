@@ -163,3 +163,17 @@ def test_split_items_of_the_fp8_kernel(dev, rows, n, sp, Hq, Hkv, chunk, split, 
     err = lambda x: ((x[:, heads].double() - want).norm() / want.norm()).item()
     assert torch.isfinite(a).all() and err(a) <= 1.05 * err(b) + 1e-3 and err(b) <= 2.0 ** -4, (err(a), err(b))
     assert (la - lb).abs().max().item() <= 2e-2  # the row sums are of rounded probabilities too
+
+
+@pytest.mark.parametrize("n,rows,mk,dtype,split", [
+    (4, 1403, 7015, "bf16", False), (4, 1400, 9800, "bf16", True),  # a shortest range of 2 of 5 chunks, of 4 of 7
+    (2, 7070, 14140, "bf16", False), (2, 3612, 10836, "bf16", True),  # of 1 of 2, of 2 of 3
+    (3, 5781, 23124, "bf16", True), (3, 5781, 23122, "bf16", False),  # of half of the longest, of just less
+    (4, 4644, 4644, "bf16", True),  # a batch: every range its own rows
+    (4, 200, 12000, "bf16", True), (4, 200, 700, "bf16", False),  # no whole round: lengths do not matter, the time saved does
+    (4, 3830, 15320, "fp8", True)])
+def test_which_launches_share_the_keys_of_several_ranges(dev, n, rows, mk, dtype, split):
+    if torch.cuda.get_device_properties(dev).multi_processor_count != 256:
+        pytest.skip("the sizes are chosen for 256 CUs")
+    code = L.MAGI_DTYPE_BF16 if dtype == "bf16" else L.MAGI_DTYPE_FP8_E4M3
+    assert (L.lib().magi_attn_split_bytes(24, 8, n, rows, mk, code) > 0) == split
