@@ -71,8 +71,9 @@ extern "C" {
 /* For bf16 callers that promise nothing about the scores: run the bounded-score kernel as if they were bounded, have it
  * judge by its row sums whether they were (sums from 2^-16 to 2^64, finite results: no score above 64, nothing of weight underflowed), and
  * repeat in a second launch, with a running maximum, the 64-row blocks where they were not.  No passes over q and k
- * (MAGI_ATTN_AUTO_BOUND) and the right result for any input; inputs with larger scores throughout cost about 2.5 times
- * as much.  args->workspace: 16 bytes of DEVICE memory per q head, range and 256 rows of max_seqlen_q (any content), 16-byte
+ * (MAGI_ATTN_AUTO_BOUND) and a result within the tolerance for any input, but not the online softmax's accuracy: the
+ * probability of a row's largest score is rounded to bf16 where there it is 1 (relative error against float64 1 to 12 % larger
+ * at unit scores, 10 to 27 % at twice that); inputs with larger scores throughout cost about 2.5 times as much.  args->workspace: 16 bytes of DEVICE memory per q head, range and 256 rows of max_seqlen_q (any content), 16-byte
  * aligned, one for each of the calls that may overlap.  Not with score_bound, q_norm, q_tile_rows,
  * MAGI_ATTN_BOUNDED_MFMA32 or MAGI_ATTN_AUTO_BOUND. */
 #define MAGI_ATTN_CHECKED 64

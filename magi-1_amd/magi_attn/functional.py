@@ -125,7 +125,8 @@ def range_attention(
     workspace is a fresh tensor, or with static_scratch the library's own device array (magi_attn_fwd_static_scratch:
     no allocation at all when `out` is given and return_lse is False; such calls must not overlap on one GPU).
     checked (bf16, instead of score_bound): the bounded-score kernel judges by its row sums whether the scores were
-    bounded, and a second launch repeats the blocks of rows where they were not, MAGI_ATTN_CHECKED.
+    bounded, and a second launch repeats the blocks of rows where they were not, MAGI_ATTN_CHECKED.  Faster than the online
+    softmax where the workgroups fill the chip, and its results are further from the exact ones (see _unbounded_mode).
     split_keys: False keeps the library from sharing the keys of a row among workgroups where that fills the chip better
     (magi_attn_args.split_workspace; the sums are then added in another order).  Needs max_seqlen_k.
     q may be [batch, rows, Hq, D] with any batch stride (batch of activations laid out [position, batch, ...]): its rows
@@ -263,47 +264,20 @@ def _measuring_a_bound_pays(q, k, n_ranges: int, max_seqlen_q: int, max_seqlen_k
     return 0.12 * attention_s > 2 * passes_s
 
 
-def _checking_pays(Hq: int, n_ranges: int, max_seqlen_q: int, keys: float, device) -> bool:
-    """A bf16 call without a score_bound: does the checked bounded-score kernel (256-row workgroups, a second launch
-    behind it; range_attention's checked) beat the online-softmax one (128- or 384-row workgroups)?  It does once its
-    workgroups come near filling the chip's slots, two per CU, and have more than a few tiles of keys each, or are many;
-    `keys` is the (average) length of a key range.  Measured, online against checked: 8880 workgroups over 400 keys 718 /
-    529 us; 1296 over 684 keys 137 / 125; 432 over 4600 keys 290 / 228; but 576 over 400 keys 47 / 51, 144 over 1536 keys
-    52 / 55, 864 over 60 keys 29 / 33.  (Fewer workgroups: _sharing_keys_pays.)"""
-    workgroups = Hq * n_ranges * ((max_seqlen_q + 255) // 256)
-    return keys >= 96 and workgroups >= (1.6 if keys >= 512 else 4) * torch.cuda.get_device_properties(device).multi_processor_count
-
-
-def _sharing_keys_pays(Hq: int, Hkv: int, n_ranges: int, max_seqlen_q: int, max_seqlen_k: int, device) -> bool:
-    """The same for fewer workgroups, whose keys the checked kernel can share among more of them.  Measured, online against
-    checked: 144 workgroups over 7680 keys 216 / 153 us, 240 over 12000 keys 379 / 307, 72 over 6300 keys 133 / 103, 24 over
-    14000 keys 283 / 114, 48 over four ranges of up to 5760 keys 121 / 97.  Ranges of unequal length in more than a third of the
-    chip's slots gain little (288 over four ranges of up to 4200 keys 137 / 134, 288 of up to 12000 keys 320 / 309)."""
-    if max_seqlen_k < 512 or max_seqlen_q <= 0:
-        return False
-    workgroups = Hq * n_ranges * ((max_seqlen_q + 255) // 256)
-    slots = 2 * torch.cuda.get_device_properties(device).multi_processor_count
-    return ((3 * workgroups <= slots or (n_ranges == 1 and workgroups <= slots))
-            and L.lib().magi_attn_split_bytes(Hq, Hkv, n_ranges, int(max_seqlen_q), int(max_seqlen_k), L.MAGI_DTYPE_BF16) > 0)
-
-
-def _unbounded_mode(q, k, n_ranges: int, max_seqlen_q: int, max_seqlen_k: int, keys: float, score_bound: float,
+def _unbounded_mode(q, k, n_ranges: int, max_seqlen_q: int, max_seqlen_k: int, score_bound: float,
                     auto_bound: Optional[bool]) -> dict:
-    """How a reference-shaped callable runs: with the bound it was given, as it was told to (auto_bound), with a measured
-    bound where the two passes are small beside the attention, or checked where that pays."""
+    """How a reference-shaped callable runs: with the bound it was given, as it was told to (auto_bound), else with a
+    measured bound where the two passes are small beside the attention, and with the online softmax below that.
+
+    Not range_attention's checked, which would be faster there (93600 rows x 24 heads over 400 keys 515 us against 694 us,
+    three chunks of 1536 rows 221 against 295): its probabilities are 2^score and not relative to the row's maximum, whose
+    own is then 1 and not rounded, so its results are further from float64 (1 to 12 % at unit scores, 10 to 27 % at twice
+    that), and where scores are above 64 throughout it takes 1.6 to 1.9 times as long."""
     if score_bound != 0.0:
         return {"score_bound": score_bound}
-    if auto_bound is not None:
-        return {"auto_bound": bool(auto_bound)}
-    if q.dtype != torch.bfloat16 or not q.is_cuda:
-        return {}
-    fills = (_checking_pays(q.shape[-2], n_ranges, max_seqlen_q, keys, q.device)
-             or _sharing_keys_pays(q.shape[-2], k.shape[-2], n_ranges, max_seqlen_q, max_seqlen_k, q.device))
-    # (below that, ranges of unequal length leave the 256-row workgroups' last round to the longest one: 240 of them over
-    # four ranges of up to 35000 keys 961 us measured against 854 us online; 216 over one range 1222 against 1320)
-    if (fills or n_ranges == 1) and _measuring_a_bound_pays(q, k, n_ranges, max_seqlen_q, max_seqlen_k):
-        return {"auto_bound": True}
-    return {"checked": True} if fills else {}
+    if auto_bound is None:
+        auto_bound = _measuring_a_bound_pays(q, k, n_ranges, max_seqlen_q, max_seqlen_k)
+    return {"auto_bound": bool(auto_bound)}
 
 
 def flex_flash_attn_func(q, k, v, q_ranges, k_ranges, max_seqlen_q, max_seqlen_k, softmax_scale=None,
@@ -318,12 +292,10 @@ def flex_flash_attn_func(q, k, v, q_ranges, k_ranges, max_seqlen_q, max_seqlen_k
     without a running maximum, which applies the scale while it loads q.
 
     auto_bound: without a score_bound the library can measure one (range_attention's auto_bound).  None (default):
-    it does where the two passes over q and k are small beside the attention itself, and launches below that which still
-    fill the chip take the bounded-score kernel that checks itself (range_attention's checked): that is how the
-    reference's own call, unchanged, runs on its QK-normed q and k.  True / False: measure always / take the
-    online-softmax kernel."""
-    mode = _unbounded_mode(q, k, q_ranges.shape[0], max_seqlen_q, max_seqlen_k,
-                           max_seqlen_k if max_seqlen_k > 0 else k.shape[0], score_bound, auto_bound)
+    it does where the two passes over q and k are small beside the attention itself, which is how the reference's
+    own call, unchanged, reaches the bounded-score kernel on its QK-normed q and k.  True / False: measure always / take
+    the online-softmax kernel."""
+    mode = _unbounded_mode(q, k, q_ranges.shape[0], max_seqlen_q, max_seqlen_k, score_bound, auto_bound)
     return range_attention(q, k, v, q_ranges, k_ranges, max_seqlen_q, max_seqlen_k, softmax_scale, **mode)
 
 
@@ -340,7 +312,7 @@ def flash_attn_func(q, k, v, dropout_p=0.0, softmax_scale=None, causal=False, de
     v3 = v.reshape(B * Sk, v.shape[2], D)
     cu_q = torch.arange(0, (B + 1) * Sq, Sq, dtype=torch.int32, device=q.device)
     cu_k = torch.arange(0, (B + 1) * Sk, Sk, dtype=torch.int32, device=q.device)
-    mode = _unbounded_mode(q3, k3, B, Sq, Sk, Sk, score_bound, auto_bound)
+    mode = _unbounded_mode(q3, k3, B, Sq, Sk, score_bound, auto_bound)
     out, _ = range_attention(q3, k3, v3, cu_q, cu_k, Sq, Sk, softmax_scale, ranges_mode=L.MAGI_RANGES_CU,
                              return_lse=False, zero_init=False, **mode)
     return out.view(B, Sq, Hq, D)
@@ -353,8 +325,7 @@ def flash_attn_varlen_func(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, ma
     A segment without keys yields zero rows.  score_bound, auto_bound: as in flex_flash_attn_func."""
     if dropout_p != 0.0 or causal:
         raise NotImplementedError("dropout / causal are not part of the MAGI-1 attention path")
-    n = cu_seqlens_q.numel() - 1
-    mode = _unbounded_mode(q, k, n, max_seqlen_q, max_seqlen_k, k.shape[0] / max(n, 1), score_bound, auto_bound)
+    mode = _unbounded_mode(q, k, cu_seqlens_q.numel() - 1, max_seqlen_q, max_seqlen_k, score_bound, auto_bound)
     out, _ = range_attention(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, softmax_scale,
                              ranges_mode=L.MAGI_RANGES_CU, return_lse=False, zero_init=True, **mode)
     return out

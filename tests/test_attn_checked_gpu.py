@@ -6,7 +6,6 @@ import pytest
 import torch
 
 import magi_attn as M
-from magi_attn import functional as F
 from oracle import magi_oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -139,21 +138,35 @@ def test_many_ranges_empty_ranges_and_gaps(dev):
         _close(out, ref)
 
 
-def test_reference_shaped_callables_check_where_it_pays(dev):
-    """varlen, flex and flash calls without a bound: two launches (checked) once the workgroups fill the chip, one below."""
-    assert F._checking_pays(24, 10, 9360, 400, dev) and not F._checking_pays(24, 10, 9360, 60, dev)
-    assert not F._checking_pays(24, 2, 1400, 400, dev)
-    L, n, Hq, Hkv = 2600, 4, 24, 8
-    q, k, v = (t.to(dev) for t in O.synthetic_qkv(n * L, n * 130, Hq, Hkv, 128, seed=9))
+@pytest.mark.parametrize("gain", [1.0, 2.0, 40.0])
+@pytest.mark.parametrize("L,n,cu_k", [(2600, 4, [0, 130, 130, 390, 520]),  # short key ranges, one of them empty
+                                      (1536, 3, [0, 1536, 3072, 4608])])
+def test_reference_shaped_callables_round_relative_to_the_maximum(dev, L, n, cu_k, gain):
+    """varlen, flex and flash calls that promise nothing about the scores give the online softmax's bits in its one launch, also
+    where 256-row workgroups would fill the chip.  The probability of a row's largest score is then 1 exactly, which the
+    checked kernel rounds: it is further from float64 than these calls may be."""
+    Hq, Hkv, D = 24, 8, 128
+    q, k, v = (t.to(dev) for t in O.synthetic_qkv(n * L, cu_k[-1], Hq, Hkv, D, seed=9))
+    q = (q.float() * gain).bfloat16()
     cq = torch.arange(0, (n + 1) * L, L, dtype=torch.int32, device=dev)
-    ck = torch.tensor([0, 130, 130, 390, 520], dtype=torch.int32, device=dev)
-    for launches, kw in ((2, {}), (1, {"auto_bound": False}), (1, {"score_bound": 17.0})):
+    ck = torch.tensor(cu_k, dtype=torch.int32, device=dev)
+    qr, kr = torch.stack([cq[:-1], cq[1:]], 1).contiguous(), torch.stack([ck[:-1], ck[1:]], 1).contiguous()
+    online, lse = M.range_attention(q, k, v, qr, kr, L)
+    calls = [lambda: M.flash_attn_varlen_func(q, k, v, cq, ck, L, 800), lambda: M.flex_flash_attn_func(q, k, v, qr, kr, L, 800)[0]]
+    if len(set(np.diff(cu_k))) == 1:
+        calls.append(lambda: M.flash_attn_func(*(t.view(n, -1, t.shape[1], D) for t in (q, k, v))).view(n * L, Hq, D))
+    for call in calls:
         n0 = M.lib().magi_launch_count()
-        out = M.flash_attn_varlen_func(q, k, v, cq, ck, L, 800, **kw)
-        assert M.lib().magi_launch_count() - n0 == launches
-        if launches == 2:
-            first = out
-    assert (first.float() - out.float()).abs().max().item() <= 2e-2 and torch.count_nonzero(first[L:2 * L]) == 0
+        out = call()
+        assert M.lib().magi_launch_count() - n0 == 1 and torch.equal(out, online)
+    if gain > 2:
+        return
+    checked, _ = M.range_attention(q, k, v, qr, kr, L, checked=True)
+    sel = torch.arange(0, L, 13, device=dev)
+    k64, v64 = (t[:cu_k[1]].double().repeat_interleave(Hq // Hkv, 1).transpose(0, 1) for t in (k, v))
+    want = (torch.softmax(q[sel].double().transpose(0, 1) @ k64.transpose(1, 2) * D ** -0.5, -1) @ v64).transpose(0, 1)
+    err = lambda x: ((x[sel].double() - want).norm() / want.norm()).item()
+    assert err(online) < err(checked), (err(online), err(checked))
 
 
 def test_checked_argument_checks(dev):
