@@ -218,7 +218,8 @@ typedef struct magi_attn_args {
    * q_batch_rows: 0 = off.  > 0: the q rows are a batch of blocks of this many rows that are not laid out one behind the
    * other: row r is row r % q_batch_rows of block r / q_batch_rows, at that row times *_stride_t plus the block times
    * *_stride_b, in q and in out (the lse stays [Hq, total_q]).  The cross attention of a batch whose activations are
-   * [position, batch, ...] reads and writes them in place that way.  bf16 with a score_bound in force, 256-row tiles. */
+   * [position, batch, ...] reads and writes them in place that way.  bf16 with a score_bound: in force (256-row tiles), or
+   * above MAGI_SCORE_BOUND_MAX (INFINITY, say), which selects the online softmax here as everywhere. */
   int32_t q_batch_rows;
   int64_t q_stride_b, o_stride_b;
   /* Optional scratch memory on the DEVICE (any content, 16-byte aligned, one for each of the calls that may overlap), of

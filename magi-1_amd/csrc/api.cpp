@@ -355,8 +355,8 @@ int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace) {
   if (p->q_batch_rows != 0) {
     if (p->q_batch_rows < 0 || p->total_q % p->q_batch_rows)
       return fail(MAGI_EINVAL, "magi_attn_fwd: q_batch_rows %d must divide total_q=%d", p->q_batch_rows, p->total_q);
-    if (!promised || mfma32 || (p->q_tile_rows != 0 && p->q_tile_rows != 256))
-      return fail(MAGI_ENOSYS, "magi_attn_fwd: q_batch_rows is implemented for bf16 with a score_bound in force and 256-row tiles");
+    if (p->dtype != MAGI_DTYPE_BF16 || !(p->score_bound > 0.f) || mfma32 || (promised && p->q_tile_rows != 0 && p->q_tile_rows != 256))
+      return fail(MAGI_ENOSYS, "magi_attn_fwd: q_batch_rows is implemented for bf16 with a score_bound, 256-row tiles where it is in force");
     if (p->q_stride_b % 8 || p->o_stride_b % 8)
       return fail(MAGI_EINVAL, "magi_attn_fwd: batch strides must keep rows 16-byte aligned");
     a.batch_rows = p->q_batch_rows;

@@ -92,7 +92,7 @@ __global__ __launch_bounds__(64 * NW, OCC) void attn_fwd_bf16_kernel(const AttnK
   bf16x8 qf[8];
   {
     const int qr = min(q_row, qe - 1);
-    const char* qp = a.q + (long)qr * a.qs_t + (long)h * a.qs_h + g * 16;
+    const char* qp = a.q + row_offset(a, qr, a.qs_t, a.qs_b) + (long)h * a.qs_h + g * 16;
 #pragma unroll
     for (int kk = 0; kk < 8; ++kk) qf[kk] = *(const bf16x8*)(qp + kk * 32);
 
@@ -410,7 +410,7 @@ __global__ __launch_bounds__(64 * NW, OCC) void attn_fwd_bf16_kernel(const AttnK
   // do not have)
   int lane_e = l;
   asm volatile("" : "+v"(lane_e));
-  char* const op = a.out + (long)(q0 + 32 * w + (lane_e & 31)) * a.os_t + o_head + 16 * (lane_e >> 5);
+  char* const op = a.out + row_offset(a, q0 + 32 * w + (lane_e & 31), a.os_t, a.os_b) + o_head + 16 * (lane_e >> 5);
 #pragma unroll
   for (int mb = 0; mb < 4; ++mb)
 #pragma unroll

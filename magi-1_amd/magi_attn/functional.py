@@ -131,7 +131,7 @@ def range_attention(
     (magi_attn_args.split_workspace; the sums are then added in another order).  Needs max_seqlen_k.
     q may be [batch, rows, Hq, D] with any batch stride (batch of activations laid out [position, batch, ...]): its rows
     count as batch * rows tokens for the ranges, out is (or comes back as) a tensor of q's shape, by default
-    [rows, batch, Hq, D] transposed.  Needs a score_bound in force.
+    [rows, batch, Hq, D] transposed.  Needs a score_bound (math.inf: the online softmax).
     q_norm: (gamma, beta or None, eps[, norm_kind]): q is the raw projection, normalised per (token, head) row inside
     the kernel (fp32, zero-centred gamma) and scaled by softmax_scale * log2(e); needs score_bound.
     """

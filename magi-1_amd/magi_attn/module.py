@@ -728,25 +728,30 @@ class FullyParallelAttention(torch.nn.Module):
     def _cross_attention_fused(self, qx_raw: torch.Tensor, sq: int, b: int, key_value_states: torch.Tensor,
                                cross_attn_params: PackedCrossAttnParams, out: Optional[torch.Tensor],
                                bound: float) -> Optional[torch.Tensor]:
-        """Cross attention on the RAW qx projection [sq * b, Hq*D]: the attention kernel applies q_layernorm_xattn while it
-        loads q (no normalised copy of q in memory) and, the scores of normed q and k being bounded, runs without a
-        running maximum; at batch > 1 it reads and writes the [position, batch] rows where they are.  Returns None
-        when that path does not apply (then the caller takes get_xqkv + cross_attention); else the result, [sq, b, Hq, D]
-        contiguous (or `out`, batch 1 only)."""
-        if not (0.0 < bound <= L.MAGI_SCORE_BOUND_MAX):
+        """Cross attention on the RAW qx projection [sq * b, Hq*D].  Batch 1: the attention kernel applies q_layernorm_xattn
+        while it loads q (no normalised copy of q in memory) and, the scores of normed q and k being bounded, runs without a
+        running maximum; returns None when that path does not apply (then the caller takes get_xqkv + cross_attention).
+        Batch > 1: head norm and online softmax, the arithmetic of get_xqkv + cross_attention bit for bit, on the [position,
+        batch] rows where they are (no copy to batch-major order and back: 230 MB each way at the 480p unconditional pass).
+        -> [sq, b, Hq, D] contiguous (or `out`, batch 1 only)."""
+        if b == 1 and not (0.0 < bound <= L.MAGI_SCORE_BOUND_MAX):
             return None
         D = self.hidden_size_per_attention_head
-        q = qx_raw.view(sq, -1, D) if b == 1 else qx_raw.view(sq, b, -1, D).transpose(0, 1)  # row-strided views of the projection
+        q = qx_raw.view(sq * b, -1, D)  # row-strided view of the projection
         m = self._modules
         kv = torch.nn.functional.linear(key_value_states, _param(m["linear_kv_xattn"], "weight"))
         k_, v_ = _halves(kv.view(key_value_states.shape[0], -1, 2 * D), kv.shape[0])
         gk, bk = m["k_layernorm_xattn"].gamma_beta_fp32()
         kx = head_norm(k_, gk, bk, self.eps)
         gq, bq = m["q_layernorm_xattn"].gamma_beta_fp32()
+        if b == 1:
+            q_kw = {"score_bound": bound, "q_norm": (gq, bq, self.eps)}
+        else:
+            q = head_norm(q, gq, bq, self.eps).view(sq, b, -1, D).transpose(0, 1)
+            q_kw = {"score_bound": math.inf}
         o, _ = range_attention(q, kx, v_, cross_attn_params.cu_seqlens_q, cross_attn_params.cu_seqlens_kv,
                                cross_attn_params.max_seqlen_q, cross_attn_params.max_seqlen_kv,
-                               ranges_mode=L.MAGI_RANGES_CU, out=out, return_lse=False, zero_init=True,
-                               score_bound=bound, q_norm=(gq, bq, self.eps))
+                               ranges_mode=L.MAGI_RANGES_CU, out=out, return_lse=False, zero_init=True, **q_kw)
         return o if b == 1 else o.transpose(0, 1)
 
     # ------------------------------------------------------------------ forward
@@ -784,7 +789,7 @@ class FullyParallelAttention(torch.nn.Module):
             "core": "fp8" if self.attention_dtype == "fp8" else
             ("measured bound: bounded-score or online softmax, chosen on the device" if measured else bounded(bound_core)),
             "core_score_bound": bound_core,
-            "cross": bounded(bound_cross),
+            "cross": bounded(bound_cross if hidden_states.shape[1] == 1 else float("inf")),
             "cross_score_bound": bound_cross}
         bs = hidden_states.shape[1]
         sq = hidden_states.shape[0]

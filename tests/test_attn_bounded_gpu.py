@@ -316,3 +316,25 @@ def test_batch_of_position_major_rows_read_and_written_in_place(dev, B, rows, cu
         assert torch.equal(got.reshape(want.shape), want) and torch.equal(lse, lse_w)
     with pytest.raises(M.MagiError):  # no bound in force
         M.range_attention(q4, k, v, *args, ranges_mode=M.MAGI_RANGES_CU)
+
+
+@pytest.mark.parametrize("bound", [float("inf"), 65.0])
+@pytest.mark.parametrize("B,rows,cu", [(3, 70, [0, 70, 140, 210]), (2, 300, [0, 300, 600]), (5, 33, [0, 40, 40, 165]),
+                                       (4, 64, [20, 130, 256]), (2, 4700, [0, 4700, 9400])])
+def test_batch_of_position_major_rows_without_a_bound_in_force(dev, B, rows, cu, bound):
+    """The same with the online softmax (a stated bound above the limit), 128-row tiles and, in the largest case, 384-row
+    ones: the bits of the call on a batch-major copy; scores that the kernel without a running maximum could not take."""
+    Hq, Hkv, D, Tk = (4, 2, 128, 150) if rows < 4000 else (96, 8, 128, 8300)
+    g = torch.Generator(device=dev).manual_seed(B + rows)
+    act = (torch.randn(rows, B, Hq * D + 64, device=dev, generator=g) * 8).bfloat16()[..., :Hq * D]
+    q4 = act.view(rows, B, Hq, D).transpose(0, 1)
+    q3 = q4.reshape(B * rows, Hq, D)
+    k, v = (torch.randn(Tk, Hkv, D, device=dev, generator=g).bfloat16() for _ in range(2))
+    cu_q = torch.tensor(cu, dtype=torch.int32, device=dev)
+    cu_k = torch.tensor(np.linspace(0, Tk, len(cu)).astype(int), dtype=torch.int32, device=dev)
+    args = (cu_q, cu_k, max(np.diff(cu)), max(np.diff(cu_k.tolist())))
+    for kw in ({}, {"q_prescaled": True}):
+        want, lse_w = M.range_attention(q3, k, v, *args, ranges_mode=M.MAGI_RANGES_CU, **kw)
+        got, lse = M.range_attention(q4, k, v, *args, ranges_mode=M.MAGI_RANGES_CU, score_bound=bound, **kw)
+        assert got.transpose(0, 1).is_contiguous() and torch.isfinite(got).all()
+        assert torch.equal(got.reshape(want.shape), want) and torch.equal(lse, lse_w)

@@ -629,6 +629,33 @@ def test_layer_batched_cacheless_pass(dev):
         assert _cosine(core[:, b], c_ref[:, 0]) >= 0.9999 and _cosine(xo[:, b], x_ref[:, 0]) >= 0.9999
 
 
+@pytest.mark.parametrize("L,B,text", [(24, 3, [3, 0, 8]), (700, 2, [400, 260]), (129, 5, [1, 64, 65, 0, 77])])
+def test_batched_cross_attention_is_the_reference_shaped_composition_bit_for_bit(dev, L, B, text):
+    """At batch > 1 the forward's cross attention, which leaves the rows in [position, batch] order, gives the bits of
+    get_xqkv + cross_attention on its copy in batch-major order: head norm rounded to bf16 once, online softmax."""
+    hidden, Hq, Hkv = 256, 6, 2
+    layer = _make_layer(dev, hidden, Hq, Hkv, seed=L)
+    g = torch.Generator().manual_seed(L)
+    angle = torch.rand(L, 48, generator=g) * 6
+    rope = torch.cat([angle.sin(), angle.cos()], dim=-1).to(dev)
+    hs = torch.randn(L, B, hidden, generator=g).bfloat16().to(dev)
+    mask = (torch.arange(max(text))[None] < torch.tensor(text)[:, None]).float().view(B, 1, 1, -1)
+    y = torch.randn(sum(text), hidden, generator=g).bfloat16().to(dev)
+    k_range = R.generate_kv_range_for_uncondition(B, L).to(dev)
+    meta = P.ModelMetaArgs(H=1, W=L, cp_pad_size=None, cp_split_sizes=None, slice_point=0, denoising_range_num=1,
+                           range_num=1, extract_prefix_video_feature=False, fwd_extra_1st_chunk=False,
+                           distill_nearly_clean_chunk=False, clip_token_nums=L, enable_cuda_graph=False,
+                           core_attn_params=P.build_core_attn_params(k_range, k_range, L),
+                           cross_attn_params=P.build_cross_attn_params(mask.to(dev), L, max(text)))
+    with torch.no_grad():
+        _, xo = layer(hs, y, None, rope, meta)
+        x = layer.linear_qkv.forward_ln(hs)
+        qx = layer.linear_qkv.forward_qkvx(x)[3]
+        want = layer.cross_attention(x, y, meta.cross_attn_params, lambda m, t: layer.get_xqkv(m, t, qx_raw=qx))
+    assert xo.shape == want.shape and xo.is_contiguous() and torch.equal(xo, want)
+    assert "online" in layer.last_forward_kernels["cross"]
+
+
 def test_layer_output_in_linear_proj_layout(dev):
     """proj_layout=True: both attention launches write into the "(hn n hd)" buffer that linear_proj consumes
     (dit_module.py:1336-1339).  Same kernels, other store addresses: bit-identical to re-ordering the two
