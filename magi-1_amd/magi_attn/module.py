@@ -657,16 +657,19 @@ class FullyParallelAttention(torch.nn.Module):
 
     def core_attention(self, query: torch.Tensor, key: torch.Tensor, value: torch.Tensor, bs: int,
                        meta_args: ModelMetaArgs, out: Optional[torch.Tensor] = None,
-                       q_prescaled: bool = False, score_bound: float = 0.0, auto_bound: bool = False) -> torch.Tensor:
+                       q_prescaled: bool = False, score_bound: float = 0.0, auto_bound: bool = False,
+                       split_keys: bool = False) -> torch.Tensor:
         """query [(sq b), Hq, D], key / value [(sk b), Hkv, D] -> [(sq b), Hq, D]; dit_module.py:1023-1066.
         bs > 1 only occurs with one range per batch row (asserted there too).  `out` (bs == 1 only) is a
         destination view, possibly in the grouped layout of range_attention.  q_prescaled: query carries
-        softmax_scale * log2(e); score_bound, auto_bound: see range_attention."""
+        softmax_scale * log2(e); score_bound, auto_bound: see range_attention.  split_keys: whether the keys of a row may
+        be shared among workgroups, the sums added in an order that depends on what else the launch holds; without it a
+        row's bits are those of full_attention on its range alone."""
         p = meta_args.core_attn_params
         if bs == 1:
             out, _ = range_attention(query, key, value, p.q_range, p.k_range, p.max_seqlen_q, p.max_seqlen_k,
                                      out=out, return_lse=False, q_prescaled=q_prescaled, score_bound=score_bound,
-                                     auto_bound=auto_bound)
+                                     auto_bound=auto_bound, split_keys=split_keys)
             return out
         if meta_args.denoising_range_num > 1:
             raise ValueError("bs > 1 with several denoising ranges is not a layout the pipeline produces")
@@ -686,7 +689,7 @@ class FullyParallelAttention(torch.nn.Module):
         o, _ = range_attention(query.view(sq, bs * Hq, D), key.as_strided((sk, bs * Hkv, D), (bs * key.stride(0), key.stride(1), 1)),
                                value.as_strided((sk, bs * Hkv, D), (bs * value.stride(0), value.stride(1), 1)),
                                ranges[1], ranges[2], sq, sk, return_lse=False, q_prescaled=q_prescaled,
-                               score_bound=score_bound)
+                               score_bound=score_bound, split_keys=split_keys)
         return o.view(sq * bs, Hq, D)
 
     def full_attention(self, bs: int, meta_args: ModelMetaArgs, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, i: int,
@@ -700,7 +703,7 @@ class FullyParallelAttention(torch.nn.Module):
         p = meta_args.core_attn_params
         q_range = (p.q_range[i:i + 1] - p.q_range[i, 0]).contiguous()
         out, _ = range_attention(q, k, v, q_range, p.k_range[i:i + 1].contiguous(), p.max_seqlen_q, p.max_seqlen_k,
-                                 return_lse=False, score_bound=score_bound)
+                                 return_lse=False, score_bound=score_bound, split_keys=False)
         return out
 
     def cross_attention(self, mixed_qqkv: torch.Tensor, key_value_states: torch.Tensor,
@@ -842,7 +845,7 @@ class FullyParallelAttention(torch.nn.Module):
         elif not use_cache:
             q, kv, qx_raw = project()
             core = self.core_attention(q, *_halves(kv, kv.shape[0]), bs, meta_args, out=core_dst, q_prescaled=True,
-                                       **core_bound_kw)
+                                       split_keys=True, **core_bound_kw)
         else:
             if bs != 1 or inference_params.max_batch_size != 1:
                 raise ValueError("the cached path runs at batch 1 (as the reference pipeline does)")

@@ -384,6 +384,27 @@ def test_reference_forward_written_out_method_by_method(dev):
     assert torch.equal(q3, query) and torch.equal(k3, key_and_value[..., :D]) and torch.equal(v3, key_and_value[..., D:])
 
 
+@pytest.mark.parametrize("L,dn,sp,Hq,Hkv", [(700, 3, 6, 6, 2), (9360, 2, 0, 24, 8)])
+def test_full_attention_gives_the_rows_of_core_attention_where_launches_leave_the_chip_idle(dev, L, dn, sp, Hq, Hkv):
+    """The equality above at sizes where the launch of one range alone would have its keys shared among workgroups, and
+    with it other bits than the launch of all ranges: with and without a bound."""
+    from magi_attn import _lib
+    D, cus = 128, torch.cuda.get_device_properties(dev).multi_processor_count
+    assert cus != 256 or _lib.lib().magi_attn_split_bytes(Hq, Hkv, 1, L, (sp + dn) * L, _lib.MAGI_DTYPE_BF16) > 0
+    layer = _make_layer(dev, 256, Hq, Hkv, seed=1)
+    q, k, v = (t.to(dev) for t in O.synthetic_qkv(dn * L, (sp + dn) * L, Hq, Hkv, D, seed=L))
+    q_range, k_range = R.q_ranges_from_chunks(dn, L).to(dev), R.generate_default_kvrange(sp, dn, L).to(dev)
+    meta = P.ModelMetaArgs(H=1, W=L, cp_pad_size=None, cp_split_sizes=None, slice_point=sp, denoising_range_num=dn,
+                           range_num=sp + dn, extract_prefix_video_feature=False, fwd_extra_1st_chunk=False,
+                           distill_nearly_clean_chunk=False, clip_token_nums=L, enable_cuda_graph=False,
+                           core_attn_params=P.build_core_attn_params(q_range, k_range, L), cross_attn_params=None)
+    for bound in (30.0, 0.0):
+        whole = layer.core_attention(q, k, v, 1, meta, score_bound=bound)
+        for i in range(dn):
+            rows = slice(i * L, (i + 1) * L)
+            assert torch.equal(layer.full_attention(1, meta, q[rows], k, v, i, score_bound=bound), whole[rows]), (bound, i)
+
+
 @pytest.mark.parametrize("proj_layout", [False, True])
 def test_whole_layer_forward_captured_in_a_graph(dev, proj_layout):
     """The reference's enable_cuda_graph case at the level of the layer: one FullyParallelAttention.forward on the
