@@ -225,7 +225,8 @@ typedef struct magi_attn_args {
   /* Optional scratch memory on the DEVICE (any content, 16-byte aligned, one for each of the calls that may overlap), of
    * magi_attn_split_bytes() or more.  With it, a launch of the fp8 kernel, or of the bf16 kernel without a running maximum, whose last round of
    * workgroups would leave part of the chip idle has the keys of that round's rows shared by several workgroups, whose unnormalised fp32 sums a
-   * launch behind it adds in the order of the keys (same precision, deterministic).  NULL, or too small: not split. */
+   * launch behind it adds in the order of the keys (same precision).  NULL, or too small: not split.  A call's bits are the same
+   * each time for the same sizes and the same choice of this memory; split and not split differ in the order of fp32 sums. */
   void* split_workspace;
   int64_t split_workspace_bytes;
 } magi_attn_args;

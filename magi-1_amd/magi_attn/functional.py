@@ -128,7 +128,8 @@ def range_attention(
     bounded, and a second launch repeats the blocks of rows where they were not, MAGI_ATTN_CHECKED.  Faster than the online
     softmax where the workgroups fill the chip, and its results are further from the exact ones (see _unbounded_mode).
     split_keys: False keeps the library from sharing the keys of a row among workgroups where that fills the chip better
-    (magi_attn_args.split_workspace; the sums are then added in another order).  Needs max_seqlen_k.
+    (magi_attn_args.split_workspace, up to 135 MB of scratch memory for the call; the fp32 sums are then added in another
+    order).  Whether it does follows from the sizes of the launch alone.  Needs max_seqlen_k.
     q may be [batch, rows, Hq, D] with any batch stride (batch of activations laid out [position, batch, ...]): its rows
     count as batch * rows tokens for the ranges, out is (or comes back as) a tensor of q's shape, by default
     [rows, batch, Hq, D] transposed.  Needs a score_bound (math.inf: the online softmax).
@@ -217,11 +218,8 @@ def range_attention(
     if split_keys and not static_scratch and max_seqlen_k >= 512 and (
             checked or auto_bound or 0.0 < score_bound <= L.MAGI_SCORE_BOUND_MAX or q.dtype is torch.float8_e4m3fn):
         split_bytes = L.lib().magi_attn_split_bytes(Hq, Hkv, max(n, 0), int(max_seqlen_q), int(max_seqlen_k), _dtype_code(q))
-        if split_bytes:
-            try:
-                split = torch.empty(split_bytes, dtype=torch.uint8, device=q.device)
-            except torch.OutOfMemoryError:  # (a call that fits without it still runs)
-                split_bytes = 0
+        if split_bytes:  # (no going on without it where memory is short: the same call would give other bits then)
+            split = torch.empty(split_bytes, dtype=torch.uint8, device=q.device)
     gamma = beta = None  # (alive until the launch is enqueued)
     norm_eps, norm_kind = 0.0, 0
     if q_norm is not None:

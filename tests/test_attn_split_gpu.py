@@ -112,6 +112,25 @@ def test_a_workspace_that_is_too_small_leaves_the_items_whole(dev, monkeypatch):
     assert torch.equal(call(), whole) and M.lib().magi_launch_count() - n0 == 1
 
 
+def test_short_memory_is_an_error_and_not_another_order_of_the_sums(dev, monkeypatch):
+    q, k, v = _inputs(dev, 256, 4096, 2, 1, seed=5)
+    qr = torch.tensor([[0, 256]], dtype=torch.int32, device=dev)
+    kr = torch.tensor([[0, 4096]], dtype=torch.int32, device=dev)
+    if not L.lib().magi_attn_split_bytes(2, 1, 1, 256, 4096, L.MAGI_DTYPE_BF16):
+        pytest.skip("not split on this card")
+    real = torch.empty
+
+    def empty(*size, dtype=None, **kw):
+        if dtype is torch.uint8:
+            raise torch.OutOfMemoryError("no scratch memory")
+        return real(*size, dtype=dtype, **kw)
+
+    monkeypatch.setattr(torch, "empty", empty)
+    with pytest.raises(torch.OutOfMemoryError):
+        M.range_attention(q, k, v, qr, kr, 256, 4096, score_bound=40.0)
+    M.range_attention(q, k, v, qr, kr, 256, 4096, score_bound=40.0, split_keys=False)
+
+
 def _exact(q, k, v, kr, rows):
     """float64 attention of q (scale and log2(e) folded in) over the operands as given."""
     G = q.shape[1] // k.shape[1]
