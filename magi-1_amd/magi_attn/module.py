@@ -180,6 +180,11 @@ def _linear_in_whole_rounds(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return torch.nn.functional.linear(x, w)
 
 
+def _global_hooks() -> bool:
+    """Whether hooks are registered that see every module's call (torch.nn.modules.module.register_module_forward_hook)."""
+    return torch.nn.modules.module._has_any_global_hook()
+
+
 class PerTensorQuantizedFp8Linear(torch.nn.Module):
     """The reference's fp8 linear layer (dit_module.py:431-456) with its parameter names and shapes, so that its
     checkpoints load: `weight` [1, out, in] float8_e4m3fn, `weight_scale` [1] fp32, `input_scale` [in] fp32.
@@ -288,11 +293,15 @@ class CustomLayerNormLinear(torch.nn.Module):
         return y.split((oq, okv, okv, oq), dim=-1)
 
     def _takes_e4m3(self, m, cols: int) -> bool:
-        """Whether the fused norm may hand m its quantised input: nothing that watches or replaces m's own call, and an
-        input_scale as layer_norm_div_clamp takes it."""
-        s = m.input_scale
-        return (type(m) is PerTensorQuantizedFp8Linear and not m._forward_hooks and not m._forward_pre_hooks
-                and s.shape == (cols,) and s.dtype == torch.float32 and s.is_contiguous())
+        """Whether the fused norm may hand m its quantised input: m is the fp8 linear itself (another class has its own
+        attributes and its own idea of the input), nothing watches or replaces its call, and its input_scale is as
+        layer_norm_div_clamp takes it."""
+        if type(m) is not PerTensorQuantizedFp8Linear or "forward" in m.__dict__ or m._forward_hooks or m._forward_pre_hooks:
+            return False
+        if _global_hooks():
+            return False
+        s, w = m.input_scale, self.layer_norm.weight
+        return s.shape == (cols,) and s.dtype == torch.float32 and s.is_contiguous() and s.device == w.device
 
     def forward_ln_qkvx_rows(self, hidden_states):
         """forward_qkvx(forward_ln(hidden_states)) as [tokens, out] rows.  With fp8_quant the norm and the four input

@@ -344,6 +344,46 @@ def test_fp8_kv_cache_shapes_and_layer_option():
     assert FullyParallelAttention(64, 2, 1, attention_dtype="fp8").attention_dtype == "fp8"
 
 
+def test_replaced_fp8_projections_are_called_and_not_read(monkeypatch):
+    """fp8_quant hands the quantised input only to a PerTensorQuantizedFp8Linear that nothing replaces, patches, watches or
+    keeps elsewhere; any other projection is called with the normalised input."""
+    from magi_attn import module as MOD
+
+    K = 64
+    c = MOD.CustomLayerNormLinear(K, 256, 128, fp8_quant=True)
+    assert all(c._takes_e4m3(m, K) for m in c._projections()) and not c._takes_e4m3(c.q, 2 * K)
+    c.q.register_forward_hook(lambda m, i, o: None)
+    c.k.register_forward_pre_hook(lambda m, i: None)
+    c.v.forward = lambda x: x.new_zeros(x.shape[0], 128)
+    assert not any(c._takes_e4m3(m, K) for m in (c.q, c.k, c.v)) and c._takes_e4m3(c.qx, K)
+    handle = torch.nn.modules.module.register_module_forward_hook(lambda m, i, o: None)
+    try:
+        assert not c._takes_e4m3(c.qx, K)
+    finally:
+        handle.remove()
+    for scale in (torch.ones(1), torch.ones(K).half(), torch.ones(2 * K)[::2], torch.ones(K, device="meta")):
+        c.qx.input_scale = torch.nn.Parameter(scale, requires_grad=False)
+        assert not c._takes_e4m3(c.qx, K)
+    # classes without input_scale among the four, called in their places
+    c = MOD.CustomLayerNormLinear(K, 256, 128, fp8_quant=True)
+    calls = []
+
+    class Fixed(torch.nn.Module):
+        def __init__(self, name, n):
+            super().__init__()
+            self.name, self.n = name, n
+
+        def forward(self, x):
+            calls.append(self.name)
+            return x.new_full((x.shape[0], self.n), ord(self.name[-1]))
+
+    for name, n in (("q", 256), ("k", 128), ("v", 128), ("qx", 256)):
+        setattr(c, name, Fixed(name, n))
+    monkeypatch.setattr(MOD, "layer_norm", lambda x, w, b, eps: torch.nn.functional.layer_norm(x, (K,), w, b, eps))
+    out = c.forward_ln_qkvx_rows(torch.randn(5, 1, K).bfloat16())
+    assert sorted(calls) == ["k", "q", "qx", "v"] and [t[0, 0].item() for t in out] == [ord(x) for x in "qkvx"]
+
+
 def test_attention_kernels_keep_their_registers():
     """A register spill inside a tile loop costs a drain of the tile loads per tile (parity stays green while the
     launch runs 1.7x slower), and the allocator decides per instantiation: compile the attention sources for
