@@ -26,9 +26,11 @@ from __future__ import annotations
 
 from typing import Callable, Optional, Tuple
 
-import torch
-
+import itertools
 import math
+import os
+
+import torch
 
 from . import _lib as L
 from .cache import Fp8KVCache, OffloadedKVCache
@@ -38,6 +40,10 @@ from .functional import (div_clamp_to, head_norm, layer_norm, layer_norm_div_cla
                          range_attention)
 from .params import InferenceParams, ModelMetaArgs, PackedCrossAttnParams
 
+
+# Epochs of all FusedLayerNorm instances (itertools.count draws are atomic): two modules never share one, and neither do the
+# modules of two processes, one of which may have been pickled in the other.
+_EPOCHS = itertools.count(int.from_bytes(os.urandom(6), "little"))
 
 PROJ_GROUPS = 8  # head groups of the linear_proj input (hard-coded "hn=8", dit_module.py:1338)
 
@@ -92,12 +98,12 @@ class FusedLayerNorm(torch.nn.Module):
             g = ((g + 1).float() - 1.0) if self.zero_centered_gamma else (g.float() - 1.0)
             state["_gb"] = (g.contiguous(), b.detach().float().contiguous())
             state["_gb_key"] = key
-            state["_gb_epoch"] = state.get("_gb_epoch", 0) + 1
+            state["_gb_epoch"] = next(_EPOCHS)
         return state["_gb"]
 
     def parameter_epoch(self) -> int:
-        """A counter that advances whenever gamma_beta_fp32() had to convert the parameters anew: what values derived
-        from the parameters (score bounds, quantisation scales) key their own caches on."""
+        """A number that is drawn anew whenever gamma_beta_fp32() had to convert the parameters, and that no other module
+        has: what values derived from the parameters (score bounds, quantisation scales) key their own caches on."""
         self.gamma_beta_fp32()
         return self.__dict__["_gb_epoch"]
 
@@ -182,7 +188,7 @@ def _linear_in_whole_rounds(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 
 def _global_hooks() -> bool:
     """Whether hooks are registered that see every module's call (torch.nn.modules.module.register_module_forward_hook)."""
-    return torch.nn.modules.module._has_any_global_hook()
+    return bool(torch.nn.modules.module._has_any_global_hook())
 
 
 class PerTensorQuantizedFp8Linear(torch.nn.Module):

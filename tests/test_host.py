@@ -384,6 +384,36 @@ def test_replaced_fp8_projections_are_called_and_not_read(monkeypatch):
     assert sorted(calls) == ["k", "q", "qx", "v"] and [t[0, 0].item() for t in out] == [ord(x) for x in "qkvx"]
 
 
+def test_a_replaced_norm_module_is_noticed():
+    """Score bounds and e4m3 operand scales belong to the norm modules they were derived from, not to how often those had
+    converted their parameters."""
+    from magi_attn import module as MOD
+
+    def norm(gain):
+        ln = MOD.FusedLayerNorm(128, dtype=torch.float32)
+        torch.nn.init.constant_(ln.weight, gain - 1.0)
+        return ln
+
+    def fresh(gains):
+        layer = MOD.FullyParallelAttention(64, 2, 1)
+        for name, gain in zip(names, gains):
+            setattr(layer, name, norm(gain))
+        return layer.score_bounds(), layer.fp8_operand_scales()
+
+    names = ("q_layernorm", "k_layernorm", "q_layernorm_xattn", "k_layernorm_xattn")
+    layer = MOD.FullyParallelAttention(64, 2, 1)
+    gains = [1.0] * 4
+    for i, gain in ((None, 1.0), (0, 21.0), (1, 0.5), (2, 3.0), (3, 7.0), (0, 1.0)):
+        if i is not None:
+            gains[i] = gain
+            setattr(layer, names[i], norm(gain))
+        assert (layer.score_bounds(), layer.fp8_operand_scales()) == fresh(gains), (i, gain)
+    # two norms exchanged
+    layer.q_layernorm, layer.q_layernorm_xattn = layer.q_layernorm_xattn, layer.q_layernorm
+    gains[0], gains[2] = gains[2], gains[0]
+    assert (layer.score_bounds(), layer.fp8_operand_scales()) == fresh(gains)
+
+
 def test_attention_kernels_keep_their_registers():
     """A register spill inside a tile loop costs a drain of the tile loads per tile (parity stays green while the
     launch runs 1.7x slower), and the allocator decides per instantiation: compile the attention sources for
