@@ -91,9 +91,14 @@ class FusedLayerNorm(torch.nn.Module):
         # (a write through `.data` does not advance _version: callers that patch parameters that way call
         # invalidate_cached_parameters())
         w, b = _param(self, "weight"), _param(self, "bias")
-        key = (id(w), w._version, w.data_ptr(), w.dtype, w.device, id(b), b._version, b.data_ptr(), b.dtype, b.device)
+        key = (w._version, w.data_ptr(), w.dtype, w.device, b._version, b.data_ptr(), b.dtype, b.device)
         state = self.__dict__
-        if state.get("_gb_key") != key:
+        # (the two parameters are held, so that a new one cannot come to lie where the old one was; a parametrised weight,
+        # computed anew for every look at it, is no parameter and is converted every time)
+        of = state.get("_gb_of")
+        if of is None or of[0] is not w or of[1] is not b or state.get("_gb_key") != key:
+            own = w is self._parameters.get("weight") and b is self._parameters.get("bias")
+            state["_gb_of"] = (w, b) if own else None
             g = w.detach()
             g = ((g + 1).float() - 1.0) if self.zero_centered_gamma else (g.float() - 1.0)
             state["_gb"] = (g.contiguous(), b.detach().float().contiguous())

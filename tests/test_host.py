@@ -1,6 +1,7 @@
 """CPU tests of the host side: range generators and rope table of the product against the
 oracle and the reference's worked examples, the metadata builders, and the C-ABI library
 (loads, exports every declared symbol, rejects bad arguments before touching a GPU)."""
+import copy
 import ctypes as C
 import os
 import re
@@ -412,6 +413,32 @@ def test_a_replaced_norm_module_is_noticed():
     layer.q_layernorm, layer.q_layernorm_xattn = layer.q_layernorm_xattn, layer.q_layernorm
     gains[0], gains[2] = gains[2], gains[0]
     assert (layer.score_bounds(), layer.fp8_operand_scales()) == fresh(gains)
+
+
+def test_a_norm_parameter_at_the_address_of_the_last_one_is_noticed():
+    """A parametrised weight is a new tensor at every look, here always at one address and now and then with the id of the
+    one before."""
+    from magi_attn import module as MOD
+
+    memory = np.zeros(128, np.float32)
+
+    class Twice(torch.nn.Module):
+        def forward(self, x):
+            np.multiply(x.detach().numpy(), 2.0, out=memory)
+            return torch.from_numpy(memory)
+
+    ln = MOD.FusedLayerNorm(128, dtype=torch.float32)
+    torch.nn.utils.parametrize.register_parametrization(ln, "weight", Twice())
+    with torch.no_grad():
+        for i in range(200):
+            ln.parametrizations.weight.original.fill_(float(i))
+            assert ln.gamma_beta_fp32()[0][0].item() == 2.0 * i
+    plain = MOD.FusedLayerNorm(128, dtype=torch.float32)
+    first = plain.gamma_beta_fp32()
+    assert plain.gamma_beta_fp32() is first  # (converted once)
+    twin = copy.deepcopy(plain)
+    torch.nn.init.constant_(twin.weight, 3.0)
+    assert twin.gamma_beta_fp32()[0][0].item() == 3.0 and plain.gamma_beta_fp32() is first
 
 
 def test_attention_kernels_keep_their_registers():
