@@ -196,6 +196,15 @@ def _global_hooks() -> bool:
     return bool(torch.nn.modules.module._has_any_global_hook())
 
 
+def _is_own(m, cls: type, *names: str) -> bool:
+    """Whether calling these methods of m runs cls's own code: neither a subclass nor the instance replaces one."""
+    t, state = type(m), m.__dict__
+    for name in names:
+        if getattr(t, name, None) is not getattr(cls, name) or name in state:
+            return False
+    return True
+
+
 class PerTensorQuantizedFp8Linear(torch.nn.Module):
     """The reference's fp8 linear layer (dit_module.py:431-456) with its parameter names and shapes, so that its
     checkpoints load: `weight` [1, out, in] float8_e4m3fn, `weight_scale` [1] fp32, `input_scale` [in] fp32.
@@ -777,6 +786,15 @@ class FullyParallelAttention(torch.nn.Module):
                                ranges_mode=L.MAGI_RANGES_CU, out=out, return_lse=False, zero_init=True, **q_kw)
         return o if b == 1 else o.transpose(0, 1)
 
+    def _project_rows(self, hidden_states: torch.Tensor):
+        """-> (q, k, v, qx) of the normalised input as [tokens, out] rows, and that input where it exists: with the library's
+        own projections only the rows are formed, others have their forward_ln and forward_qkvx called."""
+        m = self._modules["linear_qkv"]
+        if _is_own(m, CustomLayerNormLinear, "forward_ln", "forward_qkvx"):
+            return m.forward_ln_qkvx_rows(hidden_states), None
+        x = m.forward_ln(hidden_states)
+        return tuple(t.reshape(-1, t.shape[-1]) for t in m.forward_qkvx(x)), x
+
     # ------------------------------------------------------------------ forward
     def forward(self, hidden_states: torch.Tensor, key_value_states: torch.Tensor,
                 inference_params: Optional[InferenceParams], rotary_pos_emb: torch.Tensor, meta_args: ModelMetaArgs,
@@ -826,9 +844,11 @@ class FullyParallelAttention(torch.nn.Module):
             raw = qx_raw = None
         else:
             # all four projections in one GEMM; q / k / v feed the fused prologue as row-strided views of its result
-            mixed_qqkv = hidden_states  # (only its shape is used from here on: every projection is in hand)
-            q_raw, k_raw, v_raw, qx_raw = self._modules["linear_qkv"].forward_ln_qkvx_rows(hidden_states)
+            (q_raw, k_raw, v_raw, qx_raw), mixed_qqkv = self._project_rows(hidden_states)
             raw = (q_raw, k_raw, v_raw)
+        own_cross = _is_own(self, FullyParallelAttention, "get_xqkv", "cross_attention")
+        if mixed_qqkv is None:  # (the library's own methods use its shape only: every projection is in hand)
+            mixed_qqkv = hidden_states if own_cross else self.linear_qkv.forward_ln(hidden_states)
 
         def project(kv_out=None, n_cache_rows=None, kv_tail=None):
             """-> (q [S, Hq, D] carrying the softmax scale, kv destination(s), qx_raw [sq * b, Hq*D])"""
@@ -843,6 +863,11 @@ class FullyParallelAttention(torch.nn.Module):
                 Hq=self.num_attention_heads, Hkv=self.num_query_groups_per_partition, Hqx=self.num_attention_heads,
                 eps=self.eps, kv_out=kv_out, n_cache_rows=n_cache_rows, kv_tail=kv_tail, q_premul=self._q_premul)
             return q_, (kv_ if tail_ is None else (kv_, tail_)), qx_.view(sq, -1)
+
+        def cross_fused(dst):
+            if bs > 1 and not own_cross:  # (a replaced cross attention runs; at batch 1 with a bound in force it never did)
+                return None
+            return self._cross_attention_fused(qx_raw, sq, bs, key_value_states, meta_args.cross_attn_params, dst, bound_cross)
 
         get_xqkv = lambda m, y: self.get_xqkv(m, y, qx_raw=qx_raw.view(sq, bs, -1))
         p = meta_args.core_attn_params
@@ -909,11 +934,11 @@ class FullyParallelAttention(torch.nn.Module):
                 if offloaded is not None:  # the persisted rows go back to the host behind the attention launch
                     offloaded.release(start, persisted)
         if fused is not None:
-            if self._cross_attention_fused(qx_raw, sq, bs, key_value_states, meta_args.cross_attn_params, cross_dst, bound_cross) is None:
+            if cross_fused(cross_dst) is None:
                 self.cross_attention(mixed_qqkv, key_value_states, meta_args.cross_attn_params, get_xqkv, out=cross_dst)
             return fused
         core_attn_out = core.view(sq, bs, -1)
-        xo = self._cross_attention_fused(qx_raw, sq, bs, key_value_states, meta_args.cross_attn_params, None, bound_cross)
+        xo = cross_fused(None)
         if xo is not None:
             xattn_out = xo.reshape(sq, bs, -1)
         else:

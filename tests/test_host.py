@@ -385,6 +385,44 @@ def test_replaced_fp8_projections_are_called_and_not_read(monkeypatch):
     assert sorted(calls) == ["k", "q", "qx", "v"] and [t[0, 0].item() for t in out] == [ord(x) for x in "qkvx"]
 
 
+def test_replaced_projection_methods_are_called(monkeypatch):
+    """forward() projects through linear_qkv.forward_ln and .forward_qkvx where these are not the library's own: another module
+    that offers the two, a subclass, a method patched onto the instance."""
+    from magi_attn import module as MOD
+
+    K, widths = 64, (256, 128, 128, 256)
+    monkeypatch.setattr(MOD, "layer_norm", lambda x, w, b, eps: torch.nn.functional.layer_norm(x, (K,), w, b, eps))
+    layer = MOD.FullyParallelAttention(K, 2, 1)
+    x = torch.randn(6, 3, K).bfloat16()
+    rows, mixed = layer._project_rows(x)
+    assert mixed is None and [t.shape for t in rows] == [(18, n) for n in widths]
+
+    class Sub(MOD.CustomLayerNormLinear):
+        def forward_qkvx(self, h):
+            return tuple(t * 2 for t in super().forward_qkvx(h))
+
+    class Other(torch.nn.Module):  # (no forward_ln_qkvx_rows)
+        def forward_ln(self, h):
+            return h + 1
+
+        def forward_qkvx(self, h):
+            return tuple(h[..., :1].expand(*h.shape[:-1], n) for n in widths)
+
+    own = layer.linear_qkv
+    sub = Sub(K, 256, 128)
+    sub.load_state_dict(own.state_dict())
+    layer.linear_qkv = sub
+    got, mixed = layer._project_rows(x)
+    assert torch.equal(mixed, own.forward_ln(x)) and all(torch.equal(a, 2 * b) for a, b in zip(got, rows))
+    layer.linear_qkv = Other()
+    got, mixed = layer._project_rows(x)
+    assert torch.equal(mixed, x + 1) and all(torch.equal(a, (x + 1)[..., :1].reshape(18, 1).expand(18, n)) for a, n in zip(got, widths))
+    layer.linear_qkv = own
+    own.forward_ln = lambda h: h * 0
+    got, mixed = layer._project_rows(x)
+    assert not mixed.any() and not any(t.any() for t in got)
+
+
 def test_a_replaced_norm_module_is_noticed():
     """Score bounds and e4m3 operand scales belong to the norm modules they were derived from, not to how often those had
     converted their parameters."""

@@ -675,6 +675,12 @@ def test_batched_cross_attention_is_the_reference_shaped_composition_bit_for_bit
         want = layer.cross_attention(x, y, meta.cross_attn_params, lambda m, t: layer.get_xqkv(m, t, qx_raw=qx))
     assert xo.shape == want.shape and xo.is_contiguous() and torch.equal(xo, want)
     assert "online" in layer.last_forward_kernels["cross"]
+    # a cross attention put in its place runs, on the normalised input
+    seen, own = [], layer.cross_attention
+    layer.cross_attention = lambda m, *a, **kw: seen.append(m) or own(m, *a, **kw)
+    with torch.no_grad():
+        _, again = layer(hs, y, None, rope, meta)
+    assert torch.equal(again, want) and len(seen) == 1 and torch.equal(seen[0], x)
 
 
 def test_layer_output_in_linear_proj_layout(dev):
