@@ -565,11 +565,12 @@ def div_clamp_to(x: torch.Tensor, scale: torch.Tensor, out: Optional[torch.Tenso
     return y
 
 
-def layer_norm_div_clamp(x: torch.Tensor, weight: Optional[torch.Tensor], bias: Optional[torch.Tensor], scales, eps: float = 1e-5
-                         ) -> torch.Tensor:
+def layer_norm_div_clamp(x: torch.Tensor, weight: Optional[torch.Tensor], bias: Optional[torch.Tensor], scales, eps: float = 1e-5,
+                         out=None):
     """[div_clamp_to(layer_norm(x, weight, bias, eps), s) for s in scales] in one launch, bit for bit the same, without the
     normalised rows in memory (magi_layer_norm_e4m3).  x: contiguous bf16 [..., cols], cols a multiple of 8 up to 8192;
-    scales: 1 to 4 contiguous fp32 [cols] tensors.  -> float8_e4m3fn [len(scales), ..., cols]."""
+    scales: 1 to 4 contiguous fp32 [cols] tensors.  -> float8_e4m3fn [len(scales), ..., cols]; or `out`, one contiguous
+    float8_e4m3fn tensor of x's shape per scale (tensors of their own can be given back one by one)."""
     if x.dtype != torch.bfloat16:
         raise TypeError("x must be bf16")
     cols = x.shape[-1]
@@ -588,10 +589,13 @@ def layer_norm_div_clamp(x: torch.Tensor, weight: Optional[torch.Tensor], bias: 
     for s in scales:
         if s.dtype != torch.float32 or s.shape != (cols,) or not s.is_contiguous() or s.device != x.device:
             raise ValueError(f"scales must be contiguous fp32 [{cols}] tensors on x's device")
-    y = torch.empty((n,) + x.shape, dtype=torch.float8_e4m3fn, device=x.device)
+    y = torch.empty((n,) + x.shape, dtype=torch.float8_e4m3fn, device=x.device) if out is None else out
+    if out is not None and (len(out) != n or any(t.shape != x.shape or t.dtype != torch.float8_e4m3fn or t.device != x.device
+                                                 or not t.is_contiguous() for t in out)):
+        raise ValueError("out must be one contiguous float8_e4m3fn tensor of x's shape per scale, on x's device")
     rows = x.numel() // max(cols, 1)
     sp = (C.c_void_p * n)(*[s.data_ptr() for s in scales])
-    yp = (C.c_void_p * n)(*[y.data_ptr() + k * x.numel() for k in range(n)])
+    yp = (C.c_void_p * n)(*[t.data_ptr() for t in (y.unbind(0) if out is None else out)])
     _launch(x.device, L.lib().magi_layer_norm_e4m3, x.data_ptr(), cols, _ptr(weight), _ptr(bias), int(bool(fp32)), sp, yp, n, rows,
             cols, float(eps))
     return y

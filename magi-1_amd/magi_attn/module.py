@@ -331,9 +331,12 @@ class CustomLayerNormLinear(torch.nn.Module):
             linears = self._projections()
             if cols % 8 == 0 and cols <= 8192 and hidden_states.is_contiguous() and all(self._takes_e4m3(m, cols) for m in linears):
                 ln = self.layer_norm
-                x8 = layer_norm_div_clamp(hidden_states.view(-1, cols), ln.weight.detach(), ln.bias.detach(),
-                                          [m.input_scale.detach() for m in linears], ln.eps)
-                return tuple(m.forward_quantized(x) for m, x in zip(linears, x8.unbind(0)))
+                x2 = hidden_states.view(-1, cols)
+                # (a tensor each, given back behind its GEMM: together they would take more memory than the norm's bf16
+                # rows and one e4m3 input at a time)
+                x8 = [torch.empty_like(x2, dtype=torch.float8_e4m3fn) for _ in linears]
+                layer_norm_div_clamp(x2, ln.weight.detach(), ln.bias.detach(), [m.input_scale.detach() for m in linears], ln.eps, out=x8)
+                return tuple([m.forward_quantized(x8.pop(0)) for m in linears])
             x = self.forward_ln(hidden_states).view(-1, cols)
             return tuple(m(x) for m in linears)
         return self._split(_linear_in_whole_rounds(self.forward_ln(hidden_states).view(-1, cols), self.fused_weight()))

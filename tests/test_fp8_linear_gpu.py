@@ -113,6 +113,24 @@ def test_norm_and_quantisers_in_one_launch_give_the_same_bytes(dev, rows, cols, 
         assert torch.equal(bytes_[~nan], want[~nan]) and bool(((bytes_[nan] & 0x7f) == 0x7f).all())
 
 
+def test_projections_hold_no_more_memory_than_norm_and_quantisers_apart(dev):
+    """The e4m3 inputs of the four linears are given back one by one: the most that is held is below the outputs, the norm's
+    bf16 rows and one e4m3 input, which is what separate calls hold."""
+    rows, K, q, kv = 4096, 1024, 2048, 512
+    c = MOD.CustomLayerNormLinear(K, q, kv, device=dev, fp8_quant=True)
+    x = torch.randn(rows, 1, K, device=dev).bfloat16()
+    with torch.no_grad():
+        want = tuple(m(c.forward_ln(x)).view(rows, -1) for m in c._projections())
+        c.forward_ln_qkvx_rows(x)  # (the library's workspace is there from here on)
+        torch.cuda.synchronize()
+        base = torch.cuda.memory_allocated()
+        torch.cuda.reset_peak_memory_stats()
+        got = c.forward_ln_qkvx_rows(x)
+        peak = torch.cuda.max_memory_allocated() - base
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+    assert peak <= 2 * rows * (2 * q + 2 * kv) + 3 * rows * K, peak
+
+
 def test_layer_with_fp8_quant_projections(dev):
     """FullyParallelAttention(fp8_quant=True): q / qx / k / v through PerTensorQuantizedFp8Linear.  Against the same
     layer with bf16 projections made of the DE-QUANTISED weights, fed the same inputs: the only difference left is the
