@@ -162,32 +162,42 @@ def qk_score_bound(q_norm: FusedLayerNorm, k_norm: FusedLayerNorm, rotary_half: 
     return float(bound.item())
 
 
-def _linear_in_whole_rounds(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
-    """torch.nn.functional.linear(x, w), the rows cut in two where that suits the library's 256 x 256 tiles better: first
-    as many as give every CU the same number of tiles, then the rest.
+def _rows_ahead(rows: int, cols: int, depth: int, cus: int) -> int:
+    """How many rows of a [rows, depth] x [cols, depth]^T product to run in a call of their own, 0: none.
 
-    With 8192 output columns (32 column tiles) 2048 rows are one round of tiles on 256 CUs.  One call over a number of rows
-    in between leaves the last round partly empty or falls back to slower tiles: at K = 3072, 9360 rows take 444 us in one
-    call and 352 us as 8192 + 1168; 4680 rows 281 and 185, 5658 rows 318 and 221, 16974 rows 714 and 616, 37440 rows 1470
-    and 1367; where one call is fine (8000, 10000, 18720 rows) the two cost 0 to 2 % more.  With a single whole round
-    ahead of it a long rest is slower apart (3500 and 4000 rows: 4 %), so the rest is then at most 0.6 of a round.  Column
-    counts whose tiles do not divide the CUs (14336: 56 tiles) gain nothing on average and are left alone."""
-    cols = w.shape[0]
+    The library works in tiles of 256 x 256.  Where the column tiles divide the CUs, 256 * cus / tiles rows are one round of
+    tiles (2048 rows at 8192 columns); one call over a number of rows in between leaves the last round partly empty or falls
+    back to slower tiles.  Cut where that happens: whole rounds first, then the rest.  Measured, one call / cut, over 1 to
+    41 rounds and 14 rests each at depth 3072 and 8192 columns (9360 rows 444 / 352 us, 2604 183 / 105, 25268 958 / 836, 54902
+    1971 / 1852): the cut takes 1.5 % less time (41 rounds) to 37 % less (one or two) as long as the rest leaves a row of
+    tiles empty, 0 to 2 % more now and then; with a rest that fills its round, or with more than half a round behind a
+    single one, it takes 1 to 4 % more and gains nothing, so these are left alone.  2048 and 4096 deep, and 4096 and 16384
+    columns, draw the same lines.  Column counts whose tiles do not divide the CUs (14336: 56 tiles) gain nothing on
+    average."""
     tiles = cols // 256
-    if (cols % 256 == 0 and tiles and w.shape[1] >= 1024 and x.is_cuda and x.is_contiguous() and x.dtype is w.dtype
+    if cols % 256 or not 0 < tiles <= cus or cus % tiles or depth < 1024:
+        return 0
+    row_tiles = cus // tiles  # of one round
+    rounds, rest = divmod(rows, 256 * row_tiles)
+    used = (rest + 255) // 256
+    if rounds == 0 or used == 0 or used == row_tiles or (rounds == 1 and 2 * rest > 256 * row_tiles):
+        return 0
+    return rows - rest
+
+
+def _linear_in_whole_rounds(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """torch.nn.functional.linear(x, w), the rows cut in two where that suits the library's tiles better (_rows_ahead)."""
+    if (x.is_cuda and x.is_contiguous() and x.dtype is w.dtype
             and not torch.is_autocast_enabled() and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad))):
-        rows = x.numel() // x.shape[-1]
-        cus = torch.cuda.get_device_properties(x.device).multi_processor_count
-        if tiles <= cus and cus % tiles == 0:
-            round_rows = 256 * (cus // tiles)
-            head = rows // round_rows * round_rows
-            rest = rows - head
-            if rest and head and (head >= 2 * round_rows or rest <= 0.6 * round_rows):
-                x2, wt = x.view(rows, -1), w.t()
-                y = torch.empty((rows, cols), dtype=x.dtype, device=x.device)
-                torch.mm(x2[:head], wt, out=y[:head])
-                torch.mm(x2[head:], wt, out=y[head:])
-                return y.view(x.shape[:-1] + (cols,))
+        cols, depth = w.shape
+        rows = x.numel() // max(depth, 1)
+        head = _rows_ahead(rows, cols, depth, torch.cuda.get_device_properties(x.device).multi_processor_count)
+        if head:
+            x2, wt = x.view(rows, depth), w.t()
+            y = torch.empty((rows, cols), dtype=x.dtype, device=x.device)
+            torch.mm(x2[:head], wt, out=y[:head])
+            torch.mm(x2[head:], wt, out=y[head:])
+            return y.view(x.shape[:-1] + (cols,))
     return torch.nn.functional.linear(x, w)
 
 

@@ -385,6 +385,21 @@ def test_replaced_fp8_projections_are_called_and_not_read(monkeypatch):
     assert sorted(calls) == ["k", "q", "qx", "v"] and [t[0, 0].item() for t in out] == [ord(x) for x in "qkvx"]
 
 
+@pytest.mark.parametrize("cols,round_rows", [(8192, 2048), (4096, 4096), (16384, 1024), (256, 65536)])
+def test_projection_rows_are_cut_only_where_a_round_of_tiles_is_left_partly_empty(cols, round_rows):
+    from magi_attn.module import _rows_ahead
+
+    for rounds in (0, 1, 2, 5, 41):
+        for rest in (0, 1, 255, 256, 257, round_rows // 2, round_rows // 2 + 1, round_rows - 256, round_rows - 255, round_rows - 1):
+            if not 0 <= rest < round_rows:
+                continue
+            gap = -(-rest // 256) < round_rows // 256  # (a row of tiles of the last round stays empty)
+            cut = rounds > 0 and rest > 0 and gap and (rounds > 1 or rest <= round_rows // 2)
+            assert _rows_ahead(rounds * round_rows + rest, cols, 3072, 256) == (rounds * round_rows if cut else 0), (rounds, rest)
+    for cols_, depth, cus in ((14336, 6144, 256), (8192, 1016, 256), (8200, 3072, 256), (0, 3072, 256), (8192, 3072, 304), (131072, 3072, 256)):
+        assert _rows_ahead(9360, cols_, depth, cus) == 0
+
+
 def test_replaced_projection_methods_are_called(monkeypatch):
     """forward() projects through linear_qkv.forward_ln and .forward_qkvx where these are not the library's own: another module
     that offers the two, a subclass, a method patched onto the instance."""
