@@ -59,8 +59,8 @@ extern "C" {
  * at the 720p shape) leave the largest squared row length of each in `workspace`; |q . k| <= |q| |k| for every pair,
  * so the bounded-score kernel and the online-softmax kernel are both launched behind them, each tests
  * max|q| max|k| softmax_scale log2(e) * 1.01 <= MAGI_SCORE_BOUND_MAX on the device, and only the one the test selects
- * runs (the other returns at once).  Five launches, no host synchronisation, capturable.  This is what the reference's
- * call sites get without any change to them: they pass QK-normed q and k and no bound (dit_module.py:1032-1043), and
+ * runs (the other returns at once).  Five launches, one more with a second key segment and one with shared keys
+ * (split_workspace), no host synchronisation, capturable.  This is what the reference's call sites get without any change to them: they pass QK-normed q and k and no bound (dit_module.py:1032-1043), and
  * the measured bound selects the kernel without a running maximum (15 % faster on the 720p layer).  Rows of k between
  * 0 and total_k that no range names are measured too (a looser bound, still a bound); a NaN anywhere selects the
  * online-softmax kernel.  Not with score_bound, q_norm, q_tile_rows or MAGI_ATTN_BOUNDED_MFMA32. */

@@ -121,7 +121,7 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_bf16_x16_kernel(const AttnKer
   if (CHECK && tid == 0) s_over = 0;
   unsigned block = blockIdx.x;
   const SplitPiece sp = split_piece<SPLIT_FLOATS>(a, block);
-  const WorkItem wi = locate_work(a, BM, tid, s_sel, block);
+  const WorkItem wi = locate_work(a, BM, tid, s_sel, block, sp.piece == 0u);
   if (!wi.valid) return;
   const int qe = wi.qe;
   int ks = wi.ks, ke = wi.ke;
@@ -780,7 +780,9 @@ hipError_t launch_attn_fwd_bf16_checked(const AttnKernArgs& a, int compute_units
   const dim3 again(blocks < most || most == 0 ? blocks : most);
   hipLaunchKernelGGL(attn_fwd_bf16_x16_kernel<Q_CHECK>, grid, dim3(256), 0, stream, a);
   launch_merge<true>(a, stream);
-  hipLaunchKernelGGL(attn_fwd_bf16_redo_kernel, again, dim3(256), 0, stream, a);
+  AttnKernArgs r = a;
+  r.flags &= ~ATTN_ZERO_GAPS;  // (as in launch_merge)
+  hipLaunchKernelGGL(attn_fwd_bf16_redo_kernel, again, dim3(256), 0, stream, r);
   return hipGetLastError();
 }
 

@@ -184,6 +184,52 @@ def test_split_items_of_the_fp8_kernel(dev, rows, n, sp, Hq, Hkv, chunk, split, 
     assert (la - lb).abs().max().item() <= 2e-2  # the row sums are of rounded probabilities too
 
 
+def _fp8_call(dev, Tq, Tk, Hq, Hkv, qr, kr, max_q, **kw):
+    """range_attention on e4m3 operands with power-of-two scales; -> call(split_keys, out=None), the de-quantised operands"""
+    q, k, v = _inputs(dev, Tq, Tk, Hq, Hkv, seed=Tq)
+    (q8, qs), (k8, ks), (v8, vs) = M.quantize_fp8(q, 1 << 20, PRE, True), M.quantize_fp8(k, 1 << 20, 1.0, True), M.quantize_fp8(v, 1 << 20, 1.0, True)
+    deq = [x.float() * s[:1, :, None] for x, s in ((q8, qs), (k8, ks), (v8, vs))]
+    return lambda split, out=None: M.range_attention(q8, k8, v8, qr, kr, max_q, Tk, q_scale=qs, k_scale=ks, v_scale=vs,
+                                                     scale_chunk_tokens=1 << 20, fp8_pow2_prescaled=True, split_keys=split, out=out, **kw), deq
+
+
+@pytest.mark.parametrize("kind", ["bounded", "checked", "again", "fp8"])
+def test_rows_outside_the_ranges_of_split_items_are_cleared(dev, kind):
+    """Gaps ahead of, between and behind ranges whose items are shared (one piece of each clears), and all of whose blocks are
+    computed again; the memory of out and lse is poisoned."""
+    if kind == "fp8":
+        Tq, Tk, Hq, Hkv, max_q, spans = 1310, 16900, 80, 8, 1310, [(5, 1301)]
+    else:
+        Tq, Tk, Hq, Hkv, max_q, spans = 660, 3000, 4, 2, 330, [(20, 320), (345, 645)]
+    qr = torch.tensor(spans, dtype=torch.int32, device=dev)
+    kr = torch.tensor([[0, Tk]] * len(spans), dtype=torch.int32, device=dev)
+    assert len(spans) * max_q >= Tq  # (what has the launch clear the gaps)
+    if kind == "fp8":
+        call, _ = _fp8_call(dev, Tq, Tk, Hq, Hkv, qr, kr, max_q)
+    else:
+        q, k, v = _inputs(dev, Tq, Tk, Hq, Hkv, seed=3)
+        q = (q.float() * 30).bfloat16() if kind == "again" else q
+        kw = {"score_bound": 40.0} if kind == "bounded" else {"checked": True}
+        call = lambda split: M.range_attention(q, k, v, qr, kr, max_q, Tk, split_keys=split, **kw)
+    res = []
+    for split in (True, False):
+        for t, n in ((torch.bfloat16, Tq * Hq * 128), (torch.float32, Hq * Tq)):
+            poison = torch.full((n,), float("nan"), dtype=t, device=dev)
+            del poison
+        n0 = M.lib().magi_launch_count()
+        res.append(call(split) + (M.lib().magi_launch_count() - n0,))
+    (a, la, na), (b, lb, nb) = res
+    assert na == nb + 1 or torch.cuda.get_device_properties(dev).multi_processor_count != 256
+    done = torch.zeros(Tq, dtype=torch.bool, device=dev)
+    for s, e in spans:
+        done[s:e] = True
+    for o, lse in ((a, la), (b, lb)):
+        assert torch.isfinite(o).all() and (o[done].abs().sum(-1) > 0).all() and torch.count_nonzero(o[~done]) == 0
+        assert (lse[:, ~done] == float("-inf")).all() and torch.isfinite(lse[:, done]).all()
+    if kind in ("bounded", "checked"):
+        _same_but_for_the_order(a, b, la, lb)
+
+
 @pytest.mark.parametrize("n,rows,mk,dtype,split", [
     (4, 1403, 7015, "bf16", False), (4, 1400, 9800, "bf16", True),  # a shortest range of 2 of 5 chunks, of 4 of 7
     (2, 7070, 14140, "bf16", False), (2, 3612, 10836, "bf16", True),  # of 1 of 2, of 2 of 3
