@@ -230,6 +230,59 @@ def test_rows_outside_the_ranges_of_split_items_are_cleared(dev, kind):
         _same_but_for_the_order(a, b, la, lb)
 
 
+@pytest.mark.parametrize("kind", ["grouped", "grouped fp8", "batch"])
+def test_split_items_write_grouped_and_batched_outputs(dev, kind):
+    """The launch that adds the pieces up addresses the rows itself: two-level head strides, [position, batch] rows.  What lies
+    between the rows stays."""
+    fp8 = kind.endswith("fp8")
+    rows, Tk, Hq, Hkv, n = (1300, 16900, 80, 8, 1) if fp8 else (300, 3000, 4, 2, 2)
+    qr = torch.tensor([[i * rows, (i + 1) * rows] for i in range(n)], dtype=torch.int32, device=dev)
+    kr = torch.tensor([[0, Tk - 9 * i] for i in range(n)], dtype=torch.int32, device=dev)
+    if fp8:
+        call, _ = _fp8_call(dev, rows, Tk, Hq, Hkv, qr, kr, rows)
+    else:
+        q, k, v = _inputs(dev, n * rows, Tk, Hq, Hkv, seed=4)
+        if kind == "batch":
+            q4 = q.view(n, rows, Hq, 128).transpose(0, 1).contiguous().transpose(0, 1)
+            assert not q4.is_contiguous()
+        call = lambda split, out=None: M.range_attention(q4 if kind == "batch" and split else q, k, v, qr, kr, rows, Tk, score_bound=40.0,
+                                                         split_keys=split, out=out)
+    n0 = M.lib().magi_launch_count()
+    plain, lse = call(False)
+    assert M.lib().magi_launch_count() - n0 == 1
+    if kind == "batch":
+        got, lse_g = call(True)
+        assert got.transpose(0, 1).is_contiguous()
+        got = got.reshape(plain.shape)
+    else:
+        both = torch.full((n * rows, 2, 2, Hq // 2, 128), 7.0, dtype=torch.bfloat16, device=dev)
+        out, lse_g = call(True, both[:, :, 1])
+        assert (both[:, :, 0] == 7.0).all()
+        got = out.reshape(plain.shape)
+    assert M.lib().magi_launch_count() - n0 == (3 if torch.cuda.get_device_properties(dev).multi_processor_count == 256 else 2)
+    if fp8:  # (each rounds its probabilities to e4m3, 2^-4 at most, of columns of values of about 1)
+        assert (got.float() - plain.float()).norm() <= 2.0 ** -4 * plain.float().norm() and (lse_g - lse).abs().max().item() <= 2e-2
+    else:
+        _same_but_for_the_order(got, plain, lse_g, lse)
+
+
+def test_split_items_of_the_fp8_kernel_with_piecewise_linear_exponentials(dev):
+    """MAGI_ATTN_FP8_FAST_EXP2: probabilities are off by -4 to +6.2 % each, by where their exponents lie, whole or in pieces: both
+    within that of float64, the pieces no further than the whole rows, row sums within the two ends of each other."""
+    rows, Tk, Hq, Hkv = 1300, 16900, 80, 8
+    qr, kr = (torch.tensor([[0, n]], dtype=torch.int32, device=dev) for n in (rows, Tk))
+    call, (dq, dk, dv) = _fp8_call(dev, rows, Tk, Hq, Hkv, qr, kr, rows, fp8_fast_exp2=True)
+    n0 = M.lib().magi_launch_count()
+    a, la = call(True)
+    assert M.lib().magi_launch_count() - n0 == 2 or torch.cuda.get_device_properties(dev).multi_processor_count != 256
+    b, lb = call(False)
+    heads = [3, 41, 79]
+    want = _exact(dq[:, heads], *(t[:, [h // (Hq // Hkv) for h in heads]] for t in (dk, dv)), [(0, Tk)], rows)
+    err = lambda x: ((x[:, heads].double() - want).norm() / want.norm()).item()
+    assert torch.isfinite(a).all() and err(a) <= 1.05 * err(b) + 1e-3 and err(b) <= 0.1, (err(a), err(b))
+    assert (la - lb).abs().max().item() <= 0.102  # ln(1.062 / 0.96) and the roundings
+
+
 @pytest.mark.parametrize("n,rows,mk,dtype,split", [
     (4, 1403, 7015, "bf16", False), (4, 1400, 9800, "bf16", True),  # a shortest range of 2 of 5 chunks, of 4 of 7
     (2, 7070, 14140, "bf16", False), (2, 3612, 10836, "bf16", True),  # of 1 of 2, of 2 of 3
