@@ -97,35 +97,43 @@ struct SplitPlan {
 // left over in the time it takes (at 47 of 64, 3/4: three quarters on one slot take as long as a slot's three quarters).  A tile
 // of 64 keys takes a workgroup about 3 us, 1.9 us alone on its CU (0.62; behind two rounds and more, out of step by then, 1.5); what the shorter round saves is put at half of that
 // beside other workgroups (they slow down: the chip is power limited) and has to exceed the price, two launches' latency and
-// the partial sums written and read at about 3.3 TB/s.  Measured, whole / split, at 24 / 8 heads: 18 of 64 items over 7680
-// keys 208 / 137 us, 9 over 6300 keys 173 / 77, 47 over 46800 keys behind one whole round 4438 / 4020, over 9360 keys
-// 845 / 818; and where the rule says no: 60 over 25000 keys 1131 / 1144, 54 over 4608 keys 159 / 174, 18 over 1536 keys
-// 48 / 52.  4 over 99000 keys behind five whole rounds 9009 / 8583.  Behind eight and more
-// the round is a small part of the launch.
+// the partial sums written and read at about 3.3 TB/s.  Measured, whole / split (profiles/shared_keys_sweep.txt, drawn sizes with the
+// rule set aside): 148 launches that it splits 0.999 to 3.8, 1.38 on average; 92 that it does not 0.76 to 1.11, 0.97 on
+// average; fp8 behind a whole round, 53 that it splits 0.984 to 1.3, 1.04 on average.  At 24 / 8 heads: 18 of 64 items over 7680 keys 208 / 144 us, 9 over 6300 keys 169 / 84, 47 over
+// 46800 keys behind one whole round 4463 / 4099, over 9360 keys 876 / 849; not split, 48 over 4016 keys 173 / 187, 42 over 1766
+// keys 81 / 98.  Behind eight and more the round is a small part of the launch.
 // fp8: three workgroups of 128 rows per CU; a tile takes 1.4 us, 0.46 of that alone on a CU, 0.73 two by two.  Measured, whole /
-// split, with items in the last round: 30 of 96 over 46800 keys 2662 / 2551 us, 24 over 25000 keys 866 / 779, 18 over 14400 keys 474
-// / 414; and not split, 30 over 9360 keys 570 / 564, 48 over 6000 keys 192 / 203.  The probabilities are rounded to
-// e4m3 relative to the maximum so far, which a piece sees only its part of: rows that are split differ from whole ones
-// by as much as those two roundings do (3e-2 of the result; neither is nearer to the exact one).  So only launches
-// whose rows are mostly whole are split, behind one whole round at least.
-// Several ranges behind a whole round: the items go longest range first, so the last ones belong to the shortest range, and
+// split, with items in the last round: 30 of 96 over 46800 keys 2788 / 2733 us, 24 over 25000 keys 905 / 830, 18 over 14400 keys 534
+// / 474.  The probabilities are rounded to e4m3 relative to the maximum so far, which a piece sees only its part of: rows that
+// are split differ from whole ones by as much as those two roundings do (3e-2 of the result).  Their error against float64 is
+// 0.92 to 1.002 of the whole rows' over 30 drawn sizes, 0.974 on average.  Only launches whose rows are mostly whole are
+// split all the same, behind one whole round at least.
+// Several ranges: the items go longest range first, so the last ones belong to the shortest range, and
 // the others' unequal lengths have filled most of the last round already.  The host does not know the lengths; of ranges
-// that end a chunk of max_seqlen_q keys apart the shortest is max_seqlen_k less all but one of these.  bf16, whole / split where
+// that end a chunk of max_seqlen_q keys apart the shortest is max_seqlen_k less all but one of these (others are only split
+// or not split where the other would have been as good or a few per cent better).  bf16 behind a whole round, whole / split where
 // that is below half of the longest: four ranges of 1500 to 3750 keys 160 / 188 us, of 2800 to 7015 277 / 308, 10368 rows x 48
 // heads over 2592 to 10368 keys a layer of 2896 / 2999 (but six heads over 13000 to 32440 keys 1458 / 1339); two ranges
-// of one and two chunks of 7070 keys 1317 / 1334; at half and above: three of 11562 to 23124 keys 2746 / 2629, four of
-// 5600 to 9800 475 / 442, two of 32526 to 37947 3971 / 3516.  Ranges of a chunk or less each (a batch) do not differ that way.
-// fp8 gains in all of them or loses nothing (500 / 502 us at the least).
+// of one and two chunks of 7070 keys 1317 / 1334; at half and above: four of 5600 to 9800 500 / 462, two of 32526 to 37947
+// 4089 / 3539.  Ranges of a chunk or less each (a batch) do not differ that way.  bf16 without a whole round: up to 5/8 of
+// the slots gain (36 of 64 over two ranges of 2766 and 4149 keys 133 / 126), more of them from about 150 tiles on (42 over
+// 14308 keys 408 / 352, 45 over 30708 979 / 935; but 42 over 5268 keys 173 / 185, 45 over 6215 203 / 211, 48 over 7216 245 / 258).
+// fp8: a few items of a range of half the longest or less fit beside the first round (of 96 slots 3 over 4185 to 16740 keys 299 /
+// 315 us, 3 over 5505 to 16515 357 / 377, 6 over 2131 and 4262 116 / 127, 9 over 11852 to 35556 748 / 776; but 9 over 8766 to
+// 21915 525 / 454); 14 and more gain 2.5 % on average and lose 1.3 % at the most.
 SplitPlan split_plan(unsigned items, int n_ranges, int max_seqlen_q, int max_seqlen_k, bool fp8) {
   SplitPlan s = {UINT32_MAX, 1, 1, 1, fp8};
   const unsigned cus = (unsigned)compute_units() / 8, slots = cus * (fp8 ? 3 : 2);  // of one XCD
   if (slots == 0 || max_seqlen_k <= 0) return s;
   const unsigned rounds = items / slots, left = items % slots, tiles = (unsigned)(max_seqlen_k + 63) / 64;
   if (left == 0 || rounds >= 8 || (fp8 && rounds == 0)) return s;
-  if (!fp8 && rounds > 0 && n_ranges > 1 && max_seqlen_k > max_seqlen_q) {
+  if (n_ranges > 1 && max_seqlen_k > max_seqlen_q) {
     const int64_t shortest = max_seqlen_k - (int64_t)(n_ranges - 1) * max_seqlen_q;
-    if (2 * shortest < max_seqlen_k || shortest <= max_seqlen_q) return s;
+    if (fp8 ? left * 8 <= slots && 2 * shortest <= max_seqlen_k
+            : rounds > 0 && (2 * shortest < max_seqlen_k || shortest <= max_seqlen_q))
+      return s;
   }
+  if (!fp8 && rounds == 0 && n_ranges > 1 && left * 8 > slots * 5 && tiles < 150) return s;
   unsigned num, den;
   if (left * 2 > slots) {
     num = (left + slots - left - 1) / (slots - left);

@@ -289,6 +289,10 @@ def test_split_items_of_the_fp8_kernel_with_piecewise_linear_exponentials(dev):
     (3, 5781, 23124, "bf16", True), (3, 5781, 23122, "bf16", False),  # of half of the longest, of just less
     (4, 4644, 4644, "bf16", True),  # a batch: every range its own rows
     (4, 200, 12000, "bf16", True), (4, 200, 700, "bf16", False),  # no whole round: lengths do not matter, the time saved does
+    (2, 1756, 5268, "bf16", False),  # but for several ranges in more than 5/8 of the slots: 42 of 64,
+    (3, 1200, 9536, "bf16", False), (3, 1200, 9537, "bf16", True),  # 45 over 149 and 150 tiles,
+    (2, 1383, 4149, "bf16", True), (1, 3500, 5268, "bf16", True),  # 36 of 64, and 42 of one range
+    (2, 2131, 4262, "fp8", False), (2, 2131, 4264, "fp8", True),  # six items behind a round, of half of the longest and of more
     (4, 3830, 15320, "fp8", True)])
 def test_which_launches_share_the_keys_of_several_ranges(dev, n, rows, mk, dtype, split):
     if torch.cuda.get_device_properties(dev).multi_processor_count != 256:
