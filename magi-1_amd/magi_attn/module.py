@@ -91,14 +91,14 @@ class FusedLayerNorm(torch.nn.Module):
         # (a write through `.data` does not advance _version: callers that patch parameters that way call
         # invalidate_cached_parameters())
         w, b = _param(self, "weight"), _param(self, "bias")
-        key = (w._version, w.data_ptr(), w.dtype, w.device, b._version, b.data_ptr(), b.dtype, b.device)
         state = self.__dict__
         # (the two parameters are held, so that a new one cannot come to lie where the old one was; a parametrised weight,
         # computed anew for every look at it, is no parameter and is converted every time)
-        of = state.get("_gb_of")
-        if of is None or of[0] is not w or of[1] is not b or state.get("_gb_key") != key:
+        held = state.get("_gb_key", (None, None))
+        if (held[0] is not w or held[1] is not b
+                or held[2] != (w._version, w.data_ptr(), w.dtype, b._version, b.data_ptr(), b.dtype)):
             own = w is self._parameters.get("weight") and b is self._parameters.get("bias")
-            state["_gb_of"] = (w, b) if own else None
+            key = (w, b, (w._version, w.data_ptr(), w.dtype, b._version, b.data_ptr(), b.dtype)) if own else (None, None)
             g = w.detach()
             g = ((g + 1).float() - 1.0) if self.zero_centered_gamma else (g.float() - 1.0)
             state["_gb"] = (g.contiguous(), b.detach().float().contiguous())
@@ -169,7 +169,7 @@ def _rows_ahead(rows: int, cols: int, depth: int, cus: int) -> int:
     tiles (2048 rows at 8192 columns); one call over a number of rows in between leaves the last round partly empty or falls
     back to slower tiles.  Cut where that happens: whole rounds first, then the rest.  Measured, one call / cut, over 1 to
     41 rounds and 14 rests each at depth 3072 and 8192 columns (9360 rows 444 / 352 us, 2604 183 / 105, 25268 958 / 836, 54902
-    1971 / 1852): the cut takes 1.5 % less time (41 rounds) to 37 % less (one or two) as long as the rest leaves a row of
+    1971 / 1852): the cut takes 1.5 % (41 rounds) to 43 % less time (one or two) as long as the rest leaves a row of
     tiles empty, 0 to 2 % more now and then; with a rest that fills its round, or with more than half a round behind a
     single one, it takes 1 to 4 % more and gains nothing, so these are left alone.  2048 and 4096 deep, and 4096 and 16384
     columns, draw the same lines.  Column counts whose tiles do not divide the CUs (14336: 56 tiles) gain nothing on
@@ -187,10 +187,10 @@ def _rows_ahead(rows: int, cols: int, depth: int, cus: int) -> int:
 
 def _linear_in_whole_rounds(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """torch.nn.functional.linear(x, w), the rows cut in two where that suits the library's tiles better (_rows_ahead)."""
-    if (x.is_cuda and x.is_contiguous() and x.dtype is w.dtype
+    cols, depth = w.shape
+    if (depth >= 1024 and cols % 256 == 0 and x.is_cuda and x.is_contiguous() and x.dtype is w.dtype
             and not torch.is_autocast_enabled() and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad))):
-        cols, depth = w.shape
-        rows = x.numel() // max(depth, 1)
+        rows = x.numel() // depth
         head = _rows_ahead(rows, cols, depth, torch.cuda.get_device_properties(x.device).multi_processor_count)
         if head:
             x2, wt = x.view(rows, depth), w.t()
@@ -206,11 +206,12 @@ def _global_hooks() -> bool:
     return bool(torch.nn.modules.module._has_any_global_hook())
 
 
-def _is_own(m, cls: type, *names: str) -> bool:
-    """Whether calling these methods of m runs cls's own code: neither a subclass nor the instance replaces one."""
+def _is_own(m: torch.nn.Module, own: dict) -> bool:
+    """Whether calling these methods of m runs the library's code as it stands here ({name: function}): no subclass, no patch of
+    the class and none of the instance replaces one."""
     t, state = type(m), m.__dict__
-    for name in names:
-        if getattr(t, name, None) is not getattr(cls, name) or name in state:
+    for name, f in own.items():
+        if getattr(t, name, None) is not f or name in state:
             return False
     return True
 
@@ -326,9 +327,9 @@ class CustomLayerNormLinear(torch.nn.Module):
         """Whether the fused norm may hand m its quantised input: m is the fp8 linear itself (another class has its own
         attributes and its own idea of the input), nothing watches or replaces its call, and its input_scale is as
         layer_norm_div_clamp takes it."""
-        if type(m) is not PerTensorQuantizedFp8Linear or "forward" in m.__dict__ or m._forward_hooks or m._forward_pre_hooks:
+        if type(m) is not PerTensorQuantizedFp8Linear or not _is_own(m, _OWN_FP8_LINEAR):
             return False
-        if _global_hooks():
+        if m._forward_hooks or m._forward_pre_hooks or _global_hooks():
             return False
         s, w = m.input_scale, self.layer_norm.weight
         return s.shape == (cols,) and s.dtype == torch.float32 and s.is_contiguous() and s.device == w.device
@@ -803,7 +804,7 @@ class FullyParallelAttention(torch.nn.Module):
         """-> (q, k, v, qx) of the normalised input as [tokens, out] rows, and that input where it exists: with the library's
         own projections only the rows are formed, others have their forward_ln and forward_qkvx called."""
         m = self._modules["linear_qkv"]
-        if _is_own(m, CustomLayerNormLinear, "forward_ln", "forward_qkvx"):
+        if _is_own(m, _OWN_PROJECTIONS):
             return m.forward_ln_qkvx_rows(hidden_states), None
         x = m.forward_ln(hidden_states)
         return tuple(t.reshape(-1, t.shape[-1]) for t in m.forward_qkvx(x)), x
@@ -859,7 +860,7 @@ class FullyParallelAttention(torch.nn.Module):
             # all four projections in one GEMM; q / k / v feed the fused prologue as row-strided views of its result
             (q_raw, k_raw, v_raw, qx_raw), mixed_qqkv = self._project_rows(hidden_states)
             raw = (q_raw, k_raw, v_raw)
-        own_cross = _is_own(self, FullyParallelAttention, "get_xqkv", "cross_attention")
+        own_cross = _is_own(self, _OWN_CROSS)
         if mixed_qqkv is None:  # (the library's own methods use its shape only: every projection is in hand)
             mixed_qqkv = hidden_states if own_cross else self.linear_qkv.forward_ln(hidden_states)
 
@@ -959,3 +960,9 @@ class FullyParallelAttention(torch.nn.Module):
         if proj_layout:
             return attn_linear_proj_input(core_attn_out, xattn_out)
         return core_attn_out, xattn_out
+
+
+# the methods whose work forward() does in another shape, as long as they are these
+_OWN_FP8_LINEAR = {"forward": PerTensorQuantizedFp8Linear.forward}
+_OWN_PROJECTIONS = {"forward_ln": CustomLayerNormLinear.forward_ln, "forward_qkvx": CustomLayerNormLinear.forward_qkvx}
+_OWN_CROSS = {"get_xqkv": FullyParallelAttention.get_xqkv, "cross_attention": FullyParallelAttention.cross_attention}

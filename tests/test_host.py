@@ -365,6 +365,11 @@ def test_replaced_fp8_projections_are_called_and_not_read(monkeypatch):
     for scale in (torch.ones(1), torch.ones(K).half(), torch.ones(2 * K)[::2], torch.ones(K, device="meta")):
         c.qx.input_scale = torch.nn.Parameter(scale, requires_grad=False)
         assert not c._takes_e4m3(c.qx, K)
+    c = MOD.CustomLayerNormLinear(K, 256, 128, fp8_quant=True)
+    with monkeypatch.context() as patch:
+        patch.setattr(MOD.PerTensorQuantizedFp8Linear, "forward", lambda self, x: x)
+        assert not c._takes_e4m3(c.q, K)
+    assert c._takes_e4m3(c.q, K)
     # classes without input_scale among the four, called in their places
     c = MOD.CustomLayerNormLinear(K, 256, 128, fp8_quant=True)
     calls = []
@@ -436,6 +441,13 @@ def test_replaced_projection_methods_are_called(monkeypatch):
     own.forward_ln = lambda h: h * 0
     got, mixed = layer._project_rows(x)
     assert not mixed.any() and not any(t.any() for t in got)
+    del own.forward_ln
+    assert layer._project_rows(x)[1] is None
+    # and onto the class
+    was = MOD.CustomLayerNormLinear.forward_qkvx
+    monkeypatch.setattr(MOD.CustomLayerNormLinear, "forward_qkvx", lambda self, h: tuple(-t for t in was(self, h)))
+    got, mixed = layer._project_rows(x)
+    assert torch.equal(mixed, own.forward_ln(x)) and all(torch.equal(a, -b) for a, b in zip(got, rows))
 
 
 def test_a_replaced_norm_module_is_noticed():
