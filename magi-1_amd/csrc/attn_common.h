@@ -110,8 +110,7 @@ __device__ __forceinline__ void zero_rows(const AttnKernArgs& a, const WorkItem&
 // shared, their (range, tile, q head) items dealt to the XCDs one by one: cut into contiguous pieces instead, an XCD got
 // one range's tiles and the last XCDs ran dry.  Ranges are visited longest key span first (ties
 // by index), ranked here from the device-side list.
-// Every thread of the workgroup must call this (it contains a barrier); s_sel is LOCATE_WORDS ints of LDS.  `clears`: whether this
-// workgroup does the item's share of the rows no range covers (one of several that work on an item is enough).
+// Every thread of the workgroup must call this (it contains a barrier); s_sel is LOCATE_WORDS ints of LDS.
 constexpr int LOCATE_WORDS = 8;
 
 // the arithmetic part: workgroup `block` -> heads, range slot, tile; false for the padding of the grid
@@ -152,7 +151,7 @@ __device__ __forceinline__ int item_of(const AttnKernArgs& a, unsigned kvh, unsi
   return (int)(((kvh * a.G + hg) * (unsigned)a.n_ranges + rslot) * (unsigned)a.tiles_per_range + tile);
 }
 
-__device__ __forceinline__ WorkItem locate_work(const AttnKernArgs& a, int BM, int tid, int* s_sel, unsigned block, bool clears = true) {
+__device__ __forceinline__ WorkItem locate_work(const AttnKernArgs& a, int BM, int tid, int* s_sel, unsigned block) {
   WorkItem wi;
   wi.valid = false;
   unsigned kvh, hg, rslot, tile;
@@ -202,7 +201,7 @@ __device__ __forceinline__ WorkItem locate_work(const AttnKernArgs& a, int BM, i
     wi.qe = __builtin_amdgcn_readfirstlane(s_sel[1]);
     wi.ks = __builtin_amdgcn_readfirstlane(s_sel[2]);
     wi.ke = __builtin_amdgcn_readfirstlane(s_sel[3]);
-    if ((a.flags & ATTN_ZERO_GAPS) && clears) {
+    if (a.flags & ATTN_ZERO_GAPS) {
       const int g0 = __builtin_amdgcn_readfirstlane(s_sel[4]), g1 = __builtin_amdgcn_readfirstlane(s_sel[5]);
       const int lead = __builtin_amdgcn_readfirstlane(s_sel[6]);
       if (g1 > g0) zero_rows(a, wi, g0, g1, (int)tile, tid);

@@ -121,7 +121,7 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_bf16_x16_kernel(const AttnKer
   if (CHECK && tid == 0) s_over = 0;
   unsigned block = blockIdx.x;
   const SplitPiece sp = split_piece<SPLIT_FLOATS>(a, block);
-  const WorkItem wi = locate_work(a, BM, tid, s_sel, block, sp.piece == 0u);
+  const WorkItem wi = locate_work(a, BM, tid, s_sel, block);
   if (!wi.valid) return;
   const int qe = wi.qe;
   int ks = wi.ks, ke = wi.ke;

@@ -75,7 +75,7 @@ __global__ __launch_bounds__(64 * NW, 3) void attn_fwd_fp8_kernel(const AttnKern
   const int tid = threadIdx.x;
   unsigned block = blockIdx.x;
   const SplitPiece sp = split_piece<SPLIT_FLOATS_FP8>(a, block);
-  const WorkItem wi = locate_work(a, BM, tid, s_sel, block, sp.piece == 0u);
+  const WorkItem wi = locate_work(a, BM, tid, s_sel, block);
   if (!wi.valid) return;
   const int h = wi.h, kvh = wi.kvh, q0 = wi.q0, qe = wi.qe;
   int ks = wi.ks, ke = wi.ke;

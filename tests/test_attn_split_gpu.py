@@ -195,8 +195,8 @@ def _fp8_call(dev, Tq, Tk, Hq, Hkv, qr, kr, max_q, **kw):
 
 @pytest.mark.parametrize("kind", ["bounded", "checked", "again", "fp8"])
 def test_rows_outside_the_ranges_of_split_items_are_cleared(dev, kind):
-    """Gaps ahead of, between and behind ranges whose items are shared (one piece of each clears), and all of whose blocks are
-    computed again; the memory of out and lse is poisoned."""
+    """Gaps ahead of, between and behind ranges whose items are shared, and all of whose blocks are computed again; the memory of
+    out and lse is poisoned."""
     if kind == "fp8":
         Tq, Tk, Hq, Hkv, max_q, spans = 1310, 16900, 80, 8, 1310, [(5, 1301)]
     else:
