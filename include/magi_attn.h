@@ -346,6 +346,53 @@ typedef struct magi_qkv_proj_args {
 int magi_qkv_proj_prologue(const magi_qkv_proj_args* args, void* stream);
 
 /*
+ * The projections of a small layer and what comes around them, in ONE launch: for rows of a few hundred tokens, where a
+ * library GEMM, the norm ahead of it and the prologue behind it are mostly launch and memory latency.
+ *
+ * Hidden rows (S > 0): x [S, K] bf16 -> LayerNorm over K (ln_w / ln_b, bf16 or fp32, eps ln_eps; both NULL: x is taken as it is),
+ * rounded to bf16 -> columns [q | k | v | qx] heads of w [(Hq + 2 Hkv + Hqx) * 128, K] (contiguous rows), rounded to bf16 -> as
+ * magi_qk_prologue with norm_kind LayerNorm-1p: q (times q_premul) to q_out [S, Hq, 128], K | V to kv_out / kv_tail; qx to
+ * qx_out [S, Hqx, 128] as it is.
+ * Text rows (T > 0): text [T, Kt] bf16 -> columns [kv head][K | V] of w_text [2 Hkv 128, Kt] -> text_out [T, Hkv, 256], the K
+ * halves normed with gkx / bkx (LayerNorm-1p, eps).
+ * K and Kt: multiples of 64, with ln_w at most 1024.  Strides in elements, rows 16-byte aligned.
+ */
+typedef struct magi_small_proj_args {
+  uint32_t struct_size; /* sizeof(magi_small_proj_args) */
+  const void* x;
+  const void* w;
+  const void* ln_w;
+  const void* ln_b;
+  int64_t x_stride;
+  int32_t S, K, ln_params_fp32;
+  float ln_eps;
+  int32_t Hq, Hkv, Hqx, R2;
+  const float* rope; /* [S / batch, 2 R2] sin | cos, or NULL */
+  const float* gq;
+  const float* bq;
+  const float* gk;
+  const float* bk;
+  float eps;
+  int32_t batch;
+  float q_premul;
+  int32_t n_cache_rows;
+  void* q_out;
+  void* kv_out;
+  void* kv_tail;
+  int64_t kv_stride_t, kv_tail_stride_t;
+  void* qx_out;
+  const void* text;
+  const void* w_text;
+  int64_t text_stride;
+  int32_t T, Kt;
+  const float* gkx;
+  const float* bkx;
+  void* text_out;
+} magi_small_proj_args;
+
+int magi_small_projections(const magi_small_proj_args* args, void* stream);
+
+/*
  * LayerNorm of the layer input over its last axis: x [rows, cols] bf16 -> y [rows, cols] bf16 with fp32
  * statistics, y = (x - mean) / sqrt(var + eps) * weight + bias (plain weight, not the "+1" form).
  * Stands in for torch.nn.LayerNorm in CustomLayerNormLinear.forward_ln (dit_module.py:401, 412-413;

@@ -137,6 +137,37 @@ struct QkvGemmKernArgs {
 };
 hipError_t launch_qkv_gemm_prologue(const QkvGemmKernArgs& a, hipStream_t stream);
 
+// The projections of a small layer and what comes around them, in one launch (small_proj.hip).  Strides in BYTES.
+struct SmallProjKernArgs {
+  // S rows of the layer input (0: none): LayerNorm (ln_w null: as they are), then columns [q | k | v | qx] heads of w [.., K]
+  const char* x;
+  const char* w;
+  const char* ln_w;
+  const char* ln_b;
+  const float* rope;
+  const float* gq;
+  const float* bq;
+  const float* gk;
+  const float* bk;
+  char* q_out;
+  char* kv_out;
+  char* kv_tail;
+  char* qx_out;
+  // T text rows (0: none): columns [head][K | V] of w_text [2 Hkv 128, Kt], K normed
+  const char* text;
+  const char* w_text;
+  const float* gkx;
+  const float* bkx;
+  char* text_out;
+  long x_stride, text_stride, kv_stride_t, kv_tail_stride_t;
+  int S, K, T, Kt, n_cache_rows;
+  int Hq, Hkv, Hqx, R2;
+  int ln_fp32, batch;
+  float ln_eps, eps, q_premul;
+  int hidden_blocks;  // filled by the launcher
+};
+hipError_t launch_small_proj(const SmallProjKernArgs& a, int compute_units, hipStream_t stream);
+
 hipError_t launch_head_norm(const char* x, long x_stride_t, long x_stride_h, const float* gamma, const float* beta,
                             char* y, int S, int H, int norm_kind, float eps, hipStream_t stream);
 hipError_t launch_layer_norm(const char* x, long x_stride, const void* w, const void* b, int params_fp32, char* y,

@@ -1,0 +1,333 @@
+// The projections of a small layer with everything around them, in one launch, for gfx950: LayerNorm of the layer input,
+// q | k | v | qx projections, per-head norm, rotary, cast, KV-cache append; and for the text tokens the K | V projection with
+// the K norm.  Every rounding to bf16 that the separate launches make is made here too (the normalised input, the raw
+// projections, the results), sums are in fp32.
+//
+// What bounds it: latency.  Below about a thousand rows the library's GEMM, the norm ahead of it and the prologue behind it
+// each live for little more than a launch and a few trips to memory, and a library call costs the host 18 us to issue.
+// So: many small workgroups.  A workgroup of four wavefronts forms 32 rows x one head (128 columns); the weight rows stream
+// through LDS in steps of 64 elements of K, three stages filled by direct global->LDS loads, 128 bytes of a row per eight lanes
+// (operands loaded straight into registers, 16 bytes per lane from 16 rows at a time, move 16 bytes per clock and CU: 33 us
+// for 400 text tokens at K = 3072), one barrier per step.  The product is formed transposed, W X^T on
+// v_mfma_f32_16x16x32_bf16 with the weight rows as the A operand: register r of lane (n, g) of a result block is column 4 g + r
+// of the block, row n; it goes through LDS to eight lanes per row, which do with it what the prologue does.
+// RES: the workgroup's rows are in LDS whole (K up to 1024), normalised ahead of the product; their statistics are merged from
+// pieces of eight elements, which is as exact as two passes.  Otherwise the rows, not to be normalised, stream beside the weights.
+#include "attn_common.h"
+#include "row_ops.h"
+
+namespace magi {
+namespace {
+
+constexpr int NW = 4;    // wavefronts
+constexpr int BK = 64;   // elements of K per stage: 128 bytes of a row
+constexpr int STAGE_W = D * BK * 2;
+constexpr int LDS_MAX = 160 * 1024;
+// bytes per resident row: 16 more than its elements, so that the 16 rows of an operand read fall on different banks
+__device__ __forceinline__ int resident_row(int K) { return 2 * K + 16; }
+// Resident rows (RES): how long they may be, beside three stages of weights
+template <int ROWS>
+constexpr int res_max_k() { return ROWS == 32 ? 1024 : 768; }
+
+// What a thread needs from memory to finish its row (eight lanes per row, as in the prologue: a rotary pair (i, i + R2) in one
+// lane): requested ahead of the product, not behind it.
+template <int HALVES>
+struct RowParams {
+  f32x4 gam[4], bet[4], sin_cos[HALVES][4];  // elements ea .. +7, eb .. +7; the lane's eight sines and cosines
+  bool normed, rot;
+  int ea, eb;
+};
+template <int HALVES>
+__device__ __forceinline__ void load_row_params(const SmallProjKernArgs& a, RowParams<HALVES>& p, bool text, int head, int row0, int rows, int tid) {
+  const int j = tid & 7, nr = a.R2 >> 3;
+  const bool rot_lane = j < nr;
+  p.ea = rot_lane ? 8 * j : 2 * a.R2 + 16 * (j - nr);
+  p.eb = rot_lane ? a.R2 + 8 * j : p.ea + 8;
+  const float *gam = nullptr, *bet = nullptr;
+  const bool q = !text && head < a.Hq, k = !text && !q && head < a.Hq + a.Hkv;
+  if (q || k) {
+    gam = k ? a.gk : a.gq;
+    bet = k ? a.bk : a.bq;
+  } else if (text && (head & 1) == 0) {
+    gam = a.gkx;
+    bet = a.bkx;
+  }
+  p.normed = gam != nullptr;
+  p.rot = (q || k) && a.rope && rot_lane;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int e = (i < 2 ? p.ea : p.eb) + 4 * (i & 1);
+    p.gam[i] = gam ? *(const f32x4*)(gam + e) : f32x4{0.f, 0.f, 0.f, 0.f};
+    p.bet[i] = gam && bet ? *(const f32x4*)(bet + e) : f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  if (p.rot) {
+#pragma unroll
+    for (int h = 0; h < HALVES; ++h) {
+      const float* rp = a.rope + (long)(min(row0 + 32 * h + (tid >> 3), rows - 1) / a.batch) * (2 * a.R2) + 8 * j;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) p.sin_cos[h][i] = *(const f32x4*)(rp + (i < 2 ? 0 : a.R2) + 4 * (i & 1));
+    }
+  }
+}
+
+// The 32 rows row0 .. of one head as the product left them in LDS
+template <int HALVES>
+__device__ __forceinline__ void store_rows32(const SmallProjKernArgs& a, const RowParams<HALVES>& p, int half, const float* out, bool text, int head,
+                                             int row0, int rows, int tid) {
+  const int r = tid >> 3, s = row0 + r;
+  float v[16];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const f32x4 y = *LDS_PTR(const f32x4, out + r * D + (((((q < 2 ? p.ea : p.eb) >> 2) + (q & 1)) ^ (r & 15)) << 2));
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[4 * q + e] = (float)(__bf16)y[e];  // what the projection by itself returns
+  }
+  if (s >= rows) return;
+  char* dst;
+  float mul = 1.f;
+  if (text) {
+    dst = a.text_out + ((long)s * a.Hkv * 2 + head) * (D * 2);
+  } else if (head < a.Hq) {
+    mul = a.q_premul;
+    dst = a.q_out + ((long)s * a.Hq + head) * (D * 2);
+  } else if (head < a.Hq + 2 * a.Hkv) {
+    const bool is_v = head >= a.Hq + a.Hkv;
+    char* const row = s < a.n_cache_rows ? a.kv_out + (long)s * a.kv_stride_t : a.kv_tail + (long)(s - a.n_cache_rows) * a.kv_tail_stride_t;
+    dst = row + (long)(head - a.Hq - (is_v ? a.Hkv : 0)) * (2 * D * 2) + (is_v ? D * 2 : 0);
+  } else {
+    dst = a.qx_out + ((long)s * a.Hqx + (head - a.Hq - 2 * a.Hkv)) * (D * 2);
+  }
+  if (p.normed) {  // (as norm16)
+    float sum = 0.f, sq = 0.f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) sum += v[i];
+    const float mean = group8_sum(sum) * (1.f / D);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const float d = v[i] - mean;
+      sq += d * d;
+    }
+    const float rstd = __builtin_amdgcn_rsqf(group8_sum(sq) * (1.f / D) + a.eps);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) v[i] = (v[i] - mean) * rstd * (p.gam[i >> 2][i & 3] + 1.f) + p.bet[i >> 2][i & 3];
+  }
+  if (p.rot) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const float sn = p.sin_cos[half][i >> 2][i & 3], cs = p.sin_cos[half][2 + (i >> 2)][i & 3];
+      const float x1 = v[i], x2 = v[8 + i];
+      v[i] = x1 * cs - x2 * sn;
+      v[8 + i] = x1 * sn + x2 * cs;
+    }
+  }
+  if (mul != 1.f) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) v[i] *= mul;
+  }
+  *(u32x4*)(dst + p.ea * 2) = pack8(v);
+  *(u32x4*)(dst + p.eb * 2) = pack8(v + 8);
+}
+
+// RES: the rows whole in LDS ahead of the product, normalised on the way there; else they stream beside the weights, as they are
+template <bool RES, int ROWS>
+__global__ __launch_bounds__(64 * NW, RES ? 1 : 2) void small_proj_kernel(const SmallProjKernArgs a) {
+  constexpr int NST = RES && ROWS == 64 ? 3 : 4;  // stages
+  constexpr int TB = ROWS / 16;                   // blocks of 16 rows
+  constexpr int STAGE_X = RES ? 16 : ROWS * BK * 2;
+  // the stages, named statically (an operand read then does not wait for the loads in flight to another stage)
+  __shared__ __attribute__((aligned(1024))) unsigned char sW0[STAGE_W], sW1[STAGE_W], sW2[STAGE_W], sW3[NST > 3 ? STAGE_W : 16];
+  __shared__ __attribute__((aligned(1024))) unsigned char sX0[STAGE_X], sX1[STAGE_X], sX2[STAGE_X], sX3[STAGE_X];
+  __shared__ __attribute__((aligned(1024))) unsigned char sR[RES ? ROWS * (2 * res_max_k<ROWS>() + 16) : 16];
+  static_assert((RES ? 0 : 4 * STAGE_X) + NST * STAGE_W + (RES ? (int)sizeof(sR) : 0) <= (RES ? LDS_MAX : LDS_MAX / 2), "LDS");
+  const int tid = threadIdx.x;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l = tid & 63, n = l & 15, g = l >> 4;
+
+  // ---- which rows, which head: the hidden rows' workgroups, then the text rows' ----
+  const bool text = blockIdx.x >= (unsigned)a.hidden_blocks;
+  const unsigned b = text ? blockIdx.x - (unsigned)a.hidden_blocks : blockIdx.x;
+  const unsigned heads = text ? 2u * (unsigned)a.Hkv : (unsigned)(a.Hq + 2 * a.Hkv + a.Hqx);
+  const unsigned tile = b / heads;
+  const int head = (int)(b - tile * heads);
+  const int row0 = (int)tile * ROWS, rows = text ? a.T : a.S, K = text ? a.Kt : a.K;
+  const char* const x = text ? a.text : a.x;
+  const long xs = text ? a.text_stride : a.x_stride;
+  const char* const wt = (text ? a.w_text : a.w) + (long)head * D * K * 2;
+  const int steps = K / BK;
+  const bool ln = RES && !text && a.ln_w != nullptr;
+
+  // ---- loader: a wave-wide load of 64 x 16 bytes fills eight rows of 128 bytes; lane l sits at row l / 8, slot l % 8, and fetches
+  // the chunk that belongs there: row r keeps chunk c at c ^ ((r / 2) % 8), so that the 16 rows of an operand read fall on
+  // different banks.  Wavefront w fills rows 8 (w + 4 j) .. +7 of the weights, j = 0 .. 3, and rows 8 w .. +7 of x (where they stream).
+  const int lr = l >> 3, chunk = (l & 7) ^ ((4 * w + (lr >> 1)) & 7);
+  const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void*)wt, 0, 0x7fffffff, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((void*)(x + (long)row0 * xs), 0, 0x7fffffff, 0x00020000);
+  const unsigned vw = (unsigned)(8 * w + lr) * (unsigned)(K * 2) + 16u * (unsigned)chunk;
+  static_assert(RES || ROWS == 32, "one load of x per wavefront and stage");
+  const unsigned vx = (unsigned)min(8 * w + lr, rows - 1 - row0) * (unsigned)xs + 16u * (unsigned)chunk;
+  constexpr int LOADS = RES ? 4 : 5;  // per wavefront and stage
+  auto load = [&](int step, unsigned char* W, unsigned char* X) __attribute__((always_inline)) {
+    if (step >= steps) return;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, LDS_PTR(void, W + (w + 4 * j) * 1024), 16, vw,
+                                               (int)((unsigned)step * (BK * 2) + (unsigned)(32 * j) * (unsigned)(K * 2)), 0, 0);
+    if constexpr (!RES)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, LDS_PTR(void, X + w * 1024), 16, vx, (int)((unsigned)step * (BK * 2)), 0, 0);
+  };
+  RowParams<ROWS / 32> params;
+  load_row_params(a, params, text, head, row0, rows, tid);
+  load(0, sW0, sX0);
+  load(1, sW1, sX1);
+  if constexpr (NST > 3) load(2, sW2, sX2);
+
+  // ---- RES: the workgroup's rows, their statistics and norm, eight lanes a row ----
+  const int x_row = resident_row(K);
+  if constexpr (RES) {
+#pragma unroll
+    for (int half = 0; half < ROWS / 32; ++half) {
+    const int r = 32 * half + (tid >> 3), j = tid & 7;
+    const char* const rp = x + (long)min(row0 + r, rows - 1) * xs;
+    constexpr int NV = res_max_k<ROWS>() / 64;  // pieces of eight elements per lane: j, j + 8, ...
+    const int nv = K >> 6;
+    u32x4 raw[NV];
+#pragma unroll
+    for (int i = 0; i < NV; ++i) raw[i] = i < nv ? *(const u32x4*)(rp + (8 * i + j) * 16) : u32x4{0u, 0u, 0u, 0u};
+    u32x4 lnw[NV], lnb[NV];  // bf16 parameters, requested with the rows
+    if (ln && !a.ln_fp32) {
+#pragma unroll
+      for (int i = 0; i < NV; ++i) {
+        lnw[i] = i < nv ? *(const u32x4*)(a.ln_w + (8 * i + j) * 16) : u32x4{0u, 0u, 0u, 0u};
+        lnb[i] = i < nv ? *(const u32x4*)(a.ln_b + (8 * i + j) * 16) : u32x4{0u, 0u, 0u, 0u};
+      }
+    }
+    float mean = 0.f, m2 = 0.f;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      if (i >= nv) continue;
+      float f[8], s = 0.f, q = 0.f;
+      unpack8(raw[i], f);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) s += f[e];
+      s *= 0.125f;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) q += (f[e] - s) * (f[e] - s);
+      const float d = s - mean, share = 1.f / (float)(i + 1);  // 8 i elements so far, 8 more
+      m2 += q + d * d * (8.f * (float)i * share);
+      mean += d * share;
+    }
+    float cnt = 8.f * (float)nv;  // per lane; all lanes of a row hold as many
+#pragma unroll
+    for (int m = 1; m < 8; m <<= 1) {
+      const float mo = __shfl_xor(mean, m), d = mo - mean;
+      m2 += __shfl_xor(m2, m) + d * d * (0.5f * cnt);
+      mean = 0.5f * (mean + mo);
+      cnt *= 2.f;
+    }
+    const float rstd = __builtin_amdgcn_rsqf(m2 / (float)K + a.ln_eps);
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      if (i >= nv) continue;
+      float f[8], wf[8], bf[8];
+      unpack8(raw[i], f);
+      if (!ln) {
+        *LDS_PTR(u32x4, sR + r * x_row + (8 * i + j) * 16) = raw[i];
+        continue;
+      }
+      if (a.ln_fp32) {
+        param8<true>(a.ln_w, 8 * i + j, wf);
+        param8<true>(a.ln_b, 8 * i + j, bf);
+      } else {
+        unpack8(lnw[i], wf);
+        unpack8(lnb[i], bf);
+      }
+#pragma unroll
+      for (int e = 0; e < 8; ++e) f[e] = (f[e] - mean) * rstd * wf[e] + bf[e];
+      *LDS_PTR(u32x4, sR + r * x_row + (8 * i + j) * 16) = pack8(f);
+    }
+   }
+  }
+
+  // ---- operand reads: lane (n, g) holds elements 32 kk + 8 g .. +8 of weight row 32 w + 16 fb + n and of row 16 tb + n ----
+  const int sw = (g ^ ((n >> 1) & 3)) << 4, sh = ((n >> 3) & 1) << 6;  // chunk (4 kk + g) ^ (n / 2): the low bits, the high bit
+  const int base_w = (32 * w + n) * (BK * 2) + sw, base_x = RES ? n * x_row + 16 * g : n * (BK * 2) + sw;
+  f32x4 acc[2][TB];
+#pragma unroll
+  for (int fb = 0; fb < 2; ++fb)
+#pragma unroll
+    for (int tb = 0; tb < TB; ++tb) acc[fb][tb] = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto step = [&](int s, const unsigned char* W, const unsigned char* X, unsigned char* Wn, unsigned char* Xn) __attribute__((always_inline)) {
+    if (s >= steps) return;
+    // (the loads of the stages behind this one may be outstanding; RES: the barrier also publishes the rows)
+    const int behind = steps - 1 - s;
+    if (behind >= NST - 2)
+      wait_vmcnt<LOADS * (NST - 2)>();
+    else if (NST > 3 && behind == 1)
+      wait_vmcnt<LOADS>();
+    else
+      wait_vmcnt<0>();
+    __syncthreads();
+    load(s + NST - 1, Wn, Xn);
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+      bf16x8 wf[2], xf[TB];
+#pragma unroll
+      for (int fb = 0; fb < 2; ++fb) wf[fb] = *LDS_PTR(const bf16x8, W + ((base_w + ((64 * kk) ^ sh)) + fb * 16 * (BK * 2)));
+#pragma unroll
+      for (int tb = 0; tb < TB; ++tb)
+        xf[tb] = RES ? *LDS_PTR(const bf16x8, sR + (base_x + tb * 16 * x_row + s * (BK * 2) + 64 * kk))
+                     : *LDS_PTR(const bf16x8, X + ((base_x + ((64 * kk) ^ sh)) + tb * 16 * (BK * 2)));
+#pragma unroll
+      for (int fb = 0; fb < 2; ++fb)
+#pragma unroll
+        for (int tb = 0; tb < TB; ++tb) acc[fb][tb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[fb], xf[tb], acc[fb][tb], 0, 0, 0);
+    }
+  };
+  for (int s = 0; s < steps; s += NST) {
+    if constexpr (NST == 4) {
+      step(s, sW0, sX0, sW3, sX3);
+      step(s + 1, sW1, sX1, sW0, sX0);
+      step(s + 2, sW2, sX2, sW1, sX1);
+      step(s + 3, sW3, sX3, sW2, sX2);
+    } else {
+      step(s, sW0, sX0, sW2, sX2);
+      step(s + 1, sW1, sX1, sW0, sX0);
+      step(s + 2, sW2, sX2, sW1, sX1);
+    }
+  }
+  // 32 rows at a time through LDS: 512 bytes a row, its 16-byte chunk c at c ^ (row % 16)
+  float* const out = (float*)sW0;
+#pragma unroll
+ for (int half = 0; half < ROWS / 32; ++half) {
+  __syncthreads();
+#pragma unroll
+  for (int fb = 0; fb < 2; ++fb)
+#pragma unroll
+    for (int tb = 0; tb < 2; ++tb)
+      *LDS_PTR(f32x4, out + (16 * tb + n) * D + (((8 * w + 4 * fb + g) ^ n) << 2)) = acc[fb][2 * half + tb];
+  __syncthreads();
+  store_rows32(a, params, half, out, text, head, row0 + 32 * half, rows, tid);
+ }
+}
+
+}  // namespace
+
+hipError_t launch_small_proj(const SmallProjKernArgs& a_in, int compute_units, hipStream_t stream) {
+  SmallProjKernArgs a = a_in;
+  const int heads = a.Hq + 2 * a.Hkv + a.Hqx;
+  auto blocks = [&](int rows) { return ((a.S + rows - 1) / rows) * heads + ((a.T + rows - 1) / rows) * 2 * a.Hkv; };
+  if (blocks(32) == 0) return hipSuccess;
+  const int K = (a.S > 0 && a.K > a.Kt) || a.T == 0 ? a.K : a.Kt;  // the longer rows
+  const bool res = K <= res_max_k<32>(), tall = K <= res_max_k<64>() && blocks(32) > compute_units;
+  a.hidden_blocks = (tall ? (a.S + 63) / 64 : (a.S + 31) / 32) * heads;
+  const dim3 grid((unsigned)blocks(tall ? 64 : 32)), threads(64 * NW);
+  if (!res)
+    hipLaunchKernelGGL((small_proj_kernel<false, 32>), grid, threads, 0, stream, a);
+  else if (tall)
+    hipLaunchKernelGGL((small_proj_kernel<true, 64>), grid, threads, 0, stream, a);
+  else
+    hipLaunchKernelGGL((small_proj_kernel<true, 32>), grid, threads, 0, stream, a);
+  return hipGetLastError();
+}
+
+}  // namespace magi

@@ -110,13 +110,28 @@ class QuantizeArgs(_SizedStructure):
     ]
 
 
+class SmallProjArgs(_SizedStructure):
+    _fields_ = [
+        ("struct_size", C.c_uint32),
+        ("x", C.c_void_p), ("w", C.c_void_p), ("ln_w", C.c_void_p), ("ln_b", C.c_void_p), ("x_stride", C.c_int64),
+        ("S", C.c_int32), ("K", C.c_int32), ("ln_params_fp32", C.c_int32), ("ln_eps", C.c_float),
+        ("Hq", C.c_int32), ("Hkv", C.c_int32), ("Hqx", C.c_int32), ("R2", C.c_int32),
+        ("rope", C.c_void_p), ("gq", C.c_void_p), ("bq", C.c_void_p), ("gk", C.c_void_p), ("bk", C.c_void_p),
+        ("eps", C.c_float), ("batch", C.c_int32), ("q_premul", C.c_float),
+        ("n_cache_rows", C.c_int32), ("q_out", C.c_void_p), ("kv_out", C.c_void_p), ("kv_tail", C.c_void_p),
+        ("kv_stride_t", C.c_int64), ("kv_tail_stride_t", C.c_int64), ("qx_out", C.c_void_p),
+        ("text", C.c_void_p), ("w_text", C.c_void_p), ("text_stride", C.c_int64), ("T", C.c_int32), ("Kt", C.c_int32),
+        ("gkx", C.c_void_p), ("bkx", C.c_void_p), ("text_out", C.c_void_p),
+    ]
+
+
 ABI_VERSION = 104  # magi_version() of the library these mirrors were written for
 
 EXPORTS = ("magi_version", "magi_last_error", "magi_launch_count", "magi_attn_fwd", "magi_attn_fwd_static_scratch",
            "magi_attn_split_bytes",
            "magi_qk_prologue", "magi_head_norm",
            "magi_apply_rotary", "magi_quantize_fp8", "magi_quantize_fp8_split", "magi_layer_norm", "magi_qkv_proj_prologue", "magi_div_clamp_to_e4m3",
-           "magi_layer_norm_e4m3")
+           "magi_layer_norm_e4m3", "magi_small_projections")
 
 _lib = None
 
@@ -164,6 +179,8 @@ def lib() -> C.CDLL:
         l.magi_quantize_fp8.restype = C.c_int
         l.magi_qkv_proj_prologue.argtypes = [C.POINTER(QkvProjArgs), C.c_void_p]
         l.magi_qkv_proj_prologue.restype = C.c_int
+        l.magi_small_projections.argtypes = [C.POINTER(SmallProjArgs), C.c_void_p]
+        l.magi_small_projections.restype = C.c_int
         l.magi_quantize_fp8_split.argtypes = [C.POINTER(QuantizeArgs), C.c_void_p]
         l.magi_quantize_fp8_split.restype = C.c_int
         _lib = l

@@ -498,6 +498,83 @@ def qkv_proj_prologue(x: torch.Tensor, w: torch.Tensor, rope, gq, bq, gk, bk, *,
     return q_out, kv_out, kv_tail, qx_out
 
 
+def _rows(t: torch.Tensor, name: str) -> None:
+    if t.dim() != 2 or t.dtype != torch.bfloat16 or t.stride(1) != 1 or not t.is_cuda:
+        raise ValueError(f"{name} must be a 2-D bf16 device tensor with contiguous rows")
+
+
+def small_projections(x: Optional[torch.Tensor], w: Optional[torch.Tensor], rope, gq, bq, gk, bk, *, Hq: int, Hkv: int, Hqx: int = 0,
+                      ln: Optional[tuple] = None, eps: float = 1e-6, batch: int = 1, q_premul: float = 1.0,
+                      kv_out: Optional[torch.Tensor] = None, n_cache_rows: Optional[int] = None,
+                      kv_tail: Optional[torch.Tensor] = None, text: Optional[tuple] = None):
+    """The projections of a small layer and what comes around them in one launch (magi_small_projections).
+
+    x [S, K] bf16 (None: no such rows): ln = (weight, bias, eps) normalises it first; w [(Hq + 2 Hkv + Hqx) * 128, K] bf16 with rows
+    ordered q | k | v | qx heads; rope, norm parameters, q_premul, batch and the K | V destinations as in qk_prologue.  qx leaves raw.
+    text = (rows [T, Kt], weight [2 Hkv 128, Kt], gamma, beta): K | V of the text tokens, K normed.
+    -> (q [S, Hq, 128], kv_out, kv_tail, qx [S, Hqx, 128], text K | V [T, Hkv, 256]); None for what was not
+    asked for."""
+    D = 128
+    q = qx = text_kv = None
+    S = K = R2 = ln_fp32 = 0
+    ln_eps = 0.0
+    ln_w = ln_b = 0
+    dev = None
+    if x is not None:
+        _rows(x, "x")
+        _rows(w, "w")
+        S, K = x.shape
+        dev = x.device
+        if w.shape != ((Hq + 2 * Hkv + Hqx) * D, K) or not w.is_contiguous() or w.device != dev:
+            raise ValueError("w must be a contiguous [(Hq + 2 Hkv + Hqx) * 128, K] tensor on x's device")
+        if ln is not None:
+            lw, lb, ln_eps = ln
+            if (lw.shape != (K,) or lb.shape != (K,) or lw.dtype != lb.dtype or lw.dtype not in (torch.bfloat16, torch.float32)
+                    or not (lw.is_contiguous() and lb.is_contiguous()) or lw.device != dev or lb.device != dev):
+                raise ValueError("ln must be (weight, bias, eps) with contiguous bf16 or fp32 [K] tensors on x's device")
+            ln_w, ln_b, ln_fp32 = lw.data_ptr(), lb.data_ptr(), int(lw.dtype is torch.float32)
+        if kv_out is None and kv_tail is None:
+            kv_out, n_cache_rows = torch.empty((S, Hkv, 2 * D), dtype=torch.bfloat16, device=dev), S
+        if n_cache_rows is None:
+            n_cache_rows = S if kv_tail is None else 0
+        for name, t, rows in (("kv_out", kv_out, n_cache_rows), ("kv_tail", kv_tail, S - n_cache_rows)):
+            if t is None:
+                if rows:
+                    raise ValueError(f"{name} is needed for {rows} rows")
+            elif t.dtype != torch.bfloat16 or t.shape[1:] != (Hkv, 2 * D) or t.stride(2) != 1 or t.stride(1) != 2 * D or t.shape[0] < rows:
+                raise ValueError(f"{name} must be bf16 [>= {rows}, Hkv, 2*D] with contiguous heads")
+        if rope is not None:
+            if rope.dtype != torch.float32 or rope.dim() != 2 or rope.shape[0] * max(batch, 1) != S or not rope.is_contiguous():
+                raise ValueError("rope must be a contiguous fp32 [S / batch, 2*R2] tensor")
+            R2 = rope.shape[1] // 2
+        q = torch.empty((S, Hq, D), dtype=torch.bfloat16, device=dev)
+        if Hqx:
+            qx = torch.empty((S, Hqx, D), dtype=torch.bfloat16, device=dev)
+        gq, bq, gk, bk = _fp32(gq), _fp32(bq), _fp32(gk), _fp32(bk)
+    T = Kt = 0
+    tx = wt = gkx = bkx = None
+    if text is not None:
+        tx, wt, gkx, bkx = text
+        _rows(tx, "text")
+        _rows(wt, "the text weight")
+        T, Kt = tx.shape
+        dev = tx.device
+        if wt.shape != (2 * Hkv * D, Kt) or not wt.is_contiguous() or wt.device != dev or (x is not None and x.device != dev):
+            raise ValueError("the text weight must be a contiguous [2 Hkv 128, Kt] tensor on the text's device")
+        gkx, bkx = _fp32(gkx), _fp32(bkx)
+        text_kv = torch.empty((T, Hkv, 2 * D), dtype=torch.bfloat16, device=dev)
+    if dev is None:
+        raise ValueError("neither x nor text given")
+    _launch_packed(
+        dev, "magi_small_projections", L.SmallProjArgs, _ptr(x), _ptr(w) if x is not None else 0, ln_w, ln_b,
+        x.stride(0) if S > 1 else K, S, K, ln_fp32, ln_eps, Hq, Hkv, Hqx, R2, _ptr(rope) if R2 else 0, _ptr(gq), _ptr(bq), _ptr(gk),
+        _ptr(bk), eps, batch, q_premul,
+        n_cache_rows or 0, _ptr(q), _ptr(kv_out), _ptr(kv_tail),
+        0 if kv_out is None else kv_out.stride(0), 0 if kv_tail is None else kv_tail.stride(0), _ptr(qx), _ptr(tx), _ptr(wt),
+        (tx.stride(0) if T > 1 else Kt) if tx is not None else 0, T, Kt, _ptr(gkx), _ptr(bkx), _ptr(text_kv))
+    return q, kv_out, kv_tail, qx, text_kv
+
+
 def pow2_scale_for(bound: float) -> float:
     """Smallest power of two s with bound / s <= 448 (the largest e4m3 value): the scale to quantise values of
     magnitude <= bound with.  e4m3 being a floating-point format, a bound that is a few times too large costs

@@ -37,7 +37,7 @@ from .cache import Fp8KVCache, OffloadedKVCache
 from .functional import _measuring_a_bound_pays
 from .functional import (div_clamp_to, head_norm, layer_norm, layer_norm_div_clamp, pow2_scale_for, qk_prologue, qk_prologue_fp8, qkv_proj_prologue,
                          quantize_fp8_split,
-                         range_attention)
+                         range_attention, small_projections)
 from .params import InferenceParams, ModelMetaArgs, PackedCrossAttnParams
 
 
@@ -191,7 +191,7 @@ def _linear_in_whole_rounds(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     if (depth >= 1024 and cols % 256 == 0 and x.is_cuda and x.is_contiguous() and x.dtype is w.dtype
             and not torch.is_autocast_enabled() and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad))):
         rows = x.numel() // depth
-        head = _rows_ahead(rows, cols, depth, torch.cuda.get_device_properties(x.device).multi_processor_count)
+        head = _rows_ahead(rows, cols, depth, _compute_units(x.device))
         if head:
             x2, wt = x.view(rows, depth), w.t()
             y = torch.empty((rows, cols), dtype=x.dtype, device=x.device)
@@ -199,6 +199,47 @@ def _linear_in_whole_rounds(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
             torch.mm(x2[head:], wt, out=y[head:])
             return y.view(x.shape[:-1] + (cols,))
     return torch.nn.functional.linear(x, w)
+
+
+def _plain_rows(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether x [rows, K] and the weight w [n, K] are as small_projections takes them: bf16 rows of the same device, aligned, of a
+    multiple of 64 elements, and no autocast that would have the library's product convert them."""
+    if x.dim() != 2 or x.dtype is not torch.bfloat16 or w.dtype is not torch.bfloat16 or torch.is_autocast_enabled():
+        return False
+    K = x.shape[1]
+    if K % 64 or w.dim() != 2 or w.shape[1] != K or not w.is_contiguous() or x.shape[0] == 0 or not x.is_cuda or w.device != x.device:
+        return False
+    st = x.stride()
+    return st[1] == 1 and K <= st[0] <= 1 << 24 and st[0] % 8 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+
+
+_CUS = {}  # compute units by device index
+
+
+def _compute_units(device: torch.device) -> int:
+    n = _CUS.get(device.index)
+    if n is None:
+        n = _CUS[device.index] = torch.cuda.get_device_properties(device).multi_processor_count
+    return n
+
+
+def _projects_in_one_launch(rows: int, heads: int, text_rows: int, text_heads: int, K: int, cus: int) -> bool:
+    """Whether a layer's projections run as one launch of small_projections: where its workgroups (32 rows x one head each, 64 rows up
+    to K = 768) are one round, or two of the taller ones.  In one round the launch takes less time than the norm, the library's two
+    products, the prologue and the text's head norm (240 + 24 rows at K = 768, 20 + 4 heads, 12.7 against 22 us; 672 rows 19.4
+    against 26), in two about 10 us more (1344 rows 36 against 29), and the host issues it 60 us sooner, which such a layer is waiting
+    for: 840 rows behind 1120, 167 against 105 us for the layer."""
+    tile = lambda n: ((rows + n - 1) // n) * heads + ((text_rows + n - 1) // n) * text_heads  # noqa: E731
+    return tile(64) <= 2 * cus if K <= 768 else tile(32) <= cus
+
+
+def _text_in_one_launch(flop: float, rows: int, heads: int, K: int, cus: int) -> bool:
+    """Whether the K | V projection of the text rows and the K norm run as one launch of small_projections rather than as the library's
+    product and a head norm.  In one round of its workgroups (32 rows x one of the `heads`) that takes the device about as long
+    (K = 3072, 16 heads: 183 rows 16.2 against 15.2 us, 402 rows 18.9 against 18.8, 800 rows 29 against 24; K = 768, 4 heads: 1500 rows
+    10.7 against 10.4) and the host 8.5 instead of 29 us, which counts where the layer is waiting for the host: below about 150 us of
+    work, `flop` at 1e15 a second.  At K = 6144 the weight rows collide in the caches: 47 us against 18."""
+    return flop < 1.5e11 and K <= 3072 and (rows + 31) // 32 * heads <= cus
 
 
 def _global_hooks() -> bool:
@@ -773,22 +814,32 @@ class FullyParallelAttention(torch.nn.Module):
 
     def _cross_attention_fused(self, qx_raw: torch.Tensor, sq: int, b: int, key_value_states: torch.Tensor,
                                cross_attn_params: PackedCrossAttnParams, out: Optional[torch.Tensor],
-                               bound: float) -> Optional[torch.Tensor]:
+                               bound: float, text_kv: Optional[torch.Tensor] = None, own_text: bool = False) -> Optional[torch.Tensor]:
         """Cross attention on the RAW qx projection [sq * b, Hq*D].  Batch 1: the attention kernel applies q_layernorm_xattn
         while it loads q (no normalised copy of q in memory) and, the scores of normed q and k being bounded, runs without a
         running maximum; returns None when that path does not apply (then the caller takes get_xqkv + cross_attention).
         Batch > 1: head norm and online softmax, the arithmetic of get_xqkv + cross_attention bit for bit, on the [position,
         batch] rows where they are (no copy to batch-major order and back: 230 MB each way at the 480p unconditional pass).
+        text_kv: the K | V rows of the text tokens [Ty, Hkv, 2D], K normed, where the caller has them.  own_text: they come from small_projections where it takes the states (else the library's GEMM and a head norm).
         -> [sq, b, Hq, D] contiguous (or `out`, batch 1 only)."""
         if b == 1 and not (0.0 < bound <= L.MAGI_SCORE_BOUND_MAX):
             return None
         D = self.hidden_size_per_attention_head
         q = qx_raw.view(sq * b, -1, D)  # row-strided view of the projection
         m = self._modules
-        kv = torch.nn.functional.linear(key_value_states, _param(m["linear_kv_xattn"], "weight"))
-        k_, v_ = _halves(kv.view(key_value_states.shape[0], -1, 2 * D), kv.shape[0])
-        gk, bk = m["k_layernorm_xattn"].gamma_beta_fp32()
-        kx = head_norm(k_, gk, bk, self.eps)
+        if text_kv is None and own_text:
+            w = _param(m["linear_kv_xattn"], "weight")
+            if _plain_rows(key_value_states, w):
+                gk, bk = m["k_layernorm_xattn"].gamma_beta_fp32()
+                text_kv = small_projections(None, None, None, None, None, None, None, Hq=0, Hkv=self.num_query_groups_per_partition,
+                                            eps=self.eps, text=(key_value_states, w.detach(), gk, bk))[4]
+        if text_kv is not None:
+            kx, v_ = _halves(text_kv, text_kv.shape[0])
+        else:
+            kv = torch.nn.functional.linear(key_value_states, _param(m["linear_kv_xattn"], "weight"))
+            k_, v_ = _halves(kv.view(key_value_states.shape[0], -1, 2 * D), kv.shape[0])
+            gk, bk = m["k_layernorm_xattn"].gamma_beta_fp32()
+            kx = head_norm(k_, gk, bk, self.eps)
         gq, bq = m["q_layernorm_xattn"].gamma_beta_fp32()
         if b == 1:
             q_kw = {"score_bound": bound, "q_norm": (gq, bq, self.eps)}
@@ -808,6 +859,35 @@ class FullyParallelAttention(torch.nn.Module):
             return m.forward_ln_qkvx_rows(hidden_states), None
         x = m.forward_ln(hidden_states)
         return tuple(t.reshape(-1, t.shape[-1]) for t in m.forward_qkvx(x)), x
+
+    def _small_layer(self, hidden_states: torch.Tensor, key_value_states: torch.Tensor):
+        """Batch 1, bf16: what small_projections needs of a small layer whose projections are the library's own: a callable
+        (destinations as keywords) -> its results.  None where the separate launches run: other projections, larger layers, tensors of
+        other types or layouts."""
+        S, _, K = hidden_states.shape
+        if K > 1024 or key_value_states.dim() != 2 or not hidden_states.is_cuda:
+            return None
+        Hq, Hkv, (T, Kt) = self.num_attention_heads, self.num_query_groups_per_partition, key_value_states.shape
+        if Kt > 1024 or not _projects_in_one_launch(S, 2 * (Hq + Hkv), T, 2 * Hkv, max(K, Kt), _compute_units(hidden_states.device)):
+            return None
+        m = self._modules
+        lin = m["linear_qkv"]
+        if lin.__dict__.get("fp8_quant", True) or self.fused_projection or not hidden_states.is_contiguous():
+            return None
+        if not (_is_own(lin, _OWN_PROJECTIONS) and _is_own(self, _OWN_CROSS)):
+            return None
+        x = hidden_states.view(S, K)
+        w, wt, ln = lin.fused_weight(), _param(m["linear_kv_xattn"], "weight"), lin._modules["layer_norm"]
+        lw, lb = _param(ln, "weight"), _param(ln, "bias")
+        if not (_plain_rows(x, w) and _plain_rows(key_value_states, wt)) or lw is None or lb is None or lw.dtype is not lb.dtype:
+            return None
+        if lw.dtype not in (torch.bfloat16, torch.float32) or not (lw.is_contiguous() and lb.is_contiguous()) or (
+                lw.data_ptr() | lb.data_ptr()) % 16:
+            return None
+        par = m["q_layernorm"].gamma_beta_fp32() + m["k_layernorm"].gamma_beta_fp32()
+        text = (key_value_states, wt.detach()) + m["k_layernorm_xattn"].gamma_beta_fp32()
+        return lambda rope, **dst: small_projections(x, w, rope, *par, Hq=Hq, Hkv=Hkv, Hqx=Hq, ln=(lw.detach(), lb.detach(), ln.eps), eps=self.eps,
+                                                     q_premul=self._q_premul, text=text, **dst)
 
     # ------------------------------------------------------------------ forward
     def forward(self, hidden_states: torch.Tensor, key_value_states: torch.Tensor,
@@ -851,7 +931,13 @@ class FullyParallelAttention(torch.nn.Module):
         D = self.hidden_size_per_attention_head
         one_launch = (self.fused_projection and self.attention_dtype == "bf16" and bs == 1
                       and rope.shape[-1] == 96 and hidden_states.shape[-1] % 64 == 0)
-        if one_launch:
+        small = None
+        text_kv = None
+        if bs == 1 and self.attention_dtype == "bf16" and 0.0 < bound_cross <= L.MAGI_SCORE_BOUND_MAX:
+            small = self._small_layer(hidden_states, key_value_states) if rope.shape[-1] % 16 == 0 and rope.shape[-1] <= D else None
+        if small is not None:
+            mixed_qqkv, raw, qx_raw = hidden_states, None, None
+        elif one_launch:
             # projections + prologue in one launch: nothing raw reaches memory (qx leaves unnormalised, as the
             # cross-attention kernel takes it)
             mixed_qqkv = self.linear_qkv.forward_ln(hidden_states)
@@ -866,6 +952,10 @@ class FullyParallelAttention(torch.nn.Module):
 
         def project(kv_out=None, n_cache_rows=None, kv_tail=None):
             """-> (q [S, Hq, D] carrying the softmax scale, kv destination(s), qx_raw [sq * b, Hq*D])"""
+            nonlocal text_kv
+            if small is not None:
+                q_, kv_, tail_, qx_, text_kv = small(rope, kv_out=kv_out, n_cache_rows=n_cache_rows, kv_tail=kv_tail)
+                return q_, (kv_ if tail_ is None else (kv_, tail_)), qx_.view(sq, -1)
             if not one_launch:
                 q_, kv_ = self._fused_qkv(mixed_qqkv, None, None, kv_out=kv_out, n_cache_rows=n_cache_rows,
                                           kv_tail=kv_tail, raw=raw, q_premul=self._q_premul, rope=rope)
@@ -881,7 +971,12 @@ class FullyParallelAttention(torch.nn.Module):
         def cross_fused(dst):
             if bs > 1 and not own_cross:  # (a replaced cross attention runs; at batch 1 with a bound in force it never did)
                 return None
-            return self._cross_attention_fused(qx_raw, sq, bs, key_value_states, meta_args.cross_attn_params, dst, bound_cross)
+            flop = 512.0 * sq * Hq * (hidden_states.shape[2] + p.max_seqlen_k)
+            own_text = (bs == 1 and text_kv is None and key_value_states.dim() == 2 and hidden_states.is_cuda and _text_in_one_launch(
+                flop, key_value_states.shape[0], 2 * self.num_query_groups_per_partition, key_value_states.shape[1],
+                _compute_units(hidden_states.device)))
+            return self._cross_attention_fused(qx_raw, sq, bs, key_value_states, meta_args.cross_attn_params, dst, bound_cross, text_kv,
+                                               own_text)
 
         get_xqkv = lambda m, y: self.get_xqkv(m, y, qx_raw=qx_raw.view(sq, bs, -1))
         p = meta_args.core_attn_params

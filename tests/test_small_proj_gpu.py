@@ -1,0 +1,229 @@
+"""The projections of a small layer in one launch (magi_small_projections) against float64, and the layer that takes it.
+
+Expected values: the normalised input in float64 rounded to bf16, the product in float64 rounded to bf16 (the raw projection), norm,
+rotary and factor in float64.  The kernel rounds at the same places from fp32 sums, so a value beside a rounding boundary may
+land on the neighbouring bf16, as in any product summed in another order: the 2-norm of a difference stays near that of the one
+rounding to bf16 that the expected values do without (2^-9 / sqrt(3) = 1.1e-3 uniformly, 1.7e-3 at the low end of a binade), bar
+2.5e-3, and no element is further off than 2^-6 of its row's largest."""
+import ctypes as C
+import os
+import subprocess
+
+import pytest
+import torch
+
+import magi_attn as M
+from magi_attn import _lib as L
+from magi_attn import module as MOD
+from magi_attn import params as P
+from magi_attn import ranges as R
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+D = 128
+
+
+def _near(got, want, what):
+    got, want = got.double().cpu().reshape(-1, D), want.double().cpu().reshape(-1, D)
+    assert torch.isfinite(got).all(), what
+    assert (got - want).norm() <= 2.5e-3 * want.norm(), (what, float((got - want).norm() / want.norm()))
+    assert ((got - want).abs().amax(1) <= 2.0 ** -6 * want.abs().amax(1) + 1e-12).all(), what
+
+
+def _head_norm(raw, gamma, beta, eps=1e-6):
+    x = raw.view(raw.shape[0], -1, D)
+    return torch.nn.functional.layer_norm(x, (D,), eps=eps) * (gamma.double() + 1) + (0 if beta is None else beta.double())
+
+
+def _rotate(x, rope, batch, R2):
+    t = rope.double().repeat_interleave(batch, 0)[:, None]
+    s, c = t[..., :R2], t[..., R2:]
+    a, b = x[..., :R2], x[..., R2:2 * R2]
+    return torch.cat([a * c - b * s, a * s + b * c, x[..., 2 * R2:]], -1)
+
+
+# K: one stage, fewer stages than the kernel keeps in flight, all remainders of the ring, resident limits; S and T: edges of 32
+# and 64 rows; the taller workgroups (more than one round of the 32-row ones, K up to 768); rows that stream (K above 1024)
+@pytest.mark.gpu
+@pytest.mark.parametrize("S,K,T,Kt,Hq,Hkv,batch,kept,ln,beta,R2", [
+    (1, 64, 1, 64, 2, 1, 1, 1, "bf16", True, 48), (31, 128, 33, 192, 6, 2, 1, 0, "fp32", True, 48), (33, 192, 65, 64, 3, 3, 3, 20, "bf16", False, 48),
+    (64, 256, 31, 320, 6, 2, 2, 64, None, True, 32), (240, 768, 24, 768, 6, 2, 1, 120, "bf16", True, 48), (97, 1024, 40, 1024, 4, 2, 1, 97, "bf16", True, 0),
+    (1313, 256, 129, 256, 6, 2, 1, 700, "bf16", True, 48), (700, 768, 63, 704, 6, 2, 1, 699, "fp32", False, 48), (1281, 64, 0, 0, 6, 2, 1, 1281, "bf16", True, 64),
+    (65, 1088, 33, 3072, 2, 2, 1, 1, None, True, 48), (0, 0, 402, 3072, 0, 8, 1, 0, None, True, 0), (0, 0, 1, 1088, 0, 1, 1, 0, None, False, 0)])
+def test_small_projections_against_float64(dev, S, K, T, Kt, Hq, Hkv, batch, kept, ln, beta, R2):
+    g = torch.Generator(device=dev).manual_seed(S + T + K)
+    rnd = lambda *s: torch.randn(*s, device=dev, generator=g)  # noqa: E731
+    par = [rnd(D) * 0.2 for _ in range(6)]
+    if not beta:
+        par[1] = par[3] = par[5] = None
+    kw, x, w, rope = {}, None, None, None
+    if S:
+        heads = 2 * Hq + 2 * Hkv
+        x = (rnd(S, K + 8) * 3 + 1).bfloat16()[:, :K]  # (rows further apart than they are long, a mean well away from zero)
+        w = (rnd(heads * D, K) * K ** -0.5).bfloat16()
+        if ln:
+            dt = torch.float32 if ln == "fp32" else torch.bfloat16
+            kw["ln"] = ((1 + 0.1 * rnd(K)).to(dt), (0.1 * rnd(K)).to(dt), 1e-5)
+        if R2:
+            angle = torch.rand(S // batch, R2, device=dev, generator=g) * 60
+            rope = torch.cat([angle.sin(), angle.cos()], -1)
+        cache, tail = (torch.full((n, Hkv, 2 * D), 7.0, device=dev, dtype=torch.bfloat16) for n in (kept + 2, S - kept + 2))
+        kw.update(kv_out=cache if kept else None, kv_tail=tail if kept < S else None, n_cache_rows=kept)
+    if T:
+        y = (rnd(T, Kt + 16) * 0.5).bfloat16()[:, :Kt]
+        wt = (rnd(2 * Hkv * D, Kt) * Kt ** -0.5).bfloat16()
+        kw["text"] = (y, wt, par[4], par[5])
+    q, _, _, qx, kv_text = M.small_projections(x, w, rope, *par[:4], Hq=Hq, Hkv=Hkv, Hqx=Hq if S else 0, batch=batch, q_premul=0.1275, **kw)
+    if S:
+        xn = x.double()
+        if ln:
+            lw, lb, le = kw["ln"]
+            xn = torch.nn.functional.layer_norm(xn, (K,), lw.double(), lb.double(), le).bfloat16().double()
+        raw = (xn @ w.double().T).bfloat16().double()
+        rq, rk, rv, rx = raw.split((Hq * D, Hkv * D, Hkv * D, Hq * D), -1)
+        want = [_head_norm(rq, par[0], par[1]), _head_norm(rk, par[2], par[3])]
+        if R2:
+            want = [_rotate(t, rope, batch, R2) for t in want]
+        _near(q, want[0] * 0.1275, "q")
+        _near(qx, rx, "qx")
+        kv = torch.cat([cache[:kept], tail[:S - kept]])
+        _near(kv[..., :D], want[1], "k")
+        _near(kv[..., D:], rv, "v")
+        assert (cache[kept:] == 7).all() and (tail[S - kept:] == 7).all()  # nothing beyond the rows asked for
+    if T:
+        raw = (y.double() @ wt.double().T).bfloat16().double().view(T, Hkv, 2 * D)
+        _near(kv_text[..., :D], _head_norm(raw[..., :D].reshape(T, -1), par[4], par[5]), "text k")
+        _near(kv_text[..., D:], raw[..., D:], "text v")
+
+
+@pytest.mark.gpu
+def test_small_projections_refuses_what_it_does_not_implement(dev):
+    b = lambda *s: torch.zeros(*s, device=dev, dtype=torch.bfloat16)  # noqa: E731
+    p = torch.zeros(D, device=dev)
+    call = lambda K, **kw: M.small_projections(b(4, K), b(3 * D, K), None, p, p, p, p, Hq=1, Hkv=1, **kw)  # noqa: E731
+    for K, kw in ((96, {}), (1088, {"ln": (b(1088), b(1088), 1e-6)}), (64, {"ln": (b(64), b(64), 1e-6), "text": (b(2, 1088), b(2 * D, 1088), p, p)})):
+        with pytest.raises(M.MagiError):
+            call(K, **kw)
+    with pytest.raises(ValueError):
+        call(64, kv_out=b(3, 1, 2 * D), n_cache_rows=4)
+    with pytest.raises(ValueError):
+        M.small_projections(None, None, None, p, p, p, p, Hq=1, Hkv=1)
+
+
+def _layer_case(dev, hidden, frames, rows, cols, dn, sp, cache, proj, text, seed=3):
+    from magi_attn.rope import LearnableRotaryEmbeddingCat
+
+    Hq, Hkv, Lc = 8, 2, frames * rows * cols
+    torch.manual_seed(seed)
+    layer = MOD.FullyParallelAttention(hidden, Hq, Hkv, layer_number=1, device=dev)
+    with torch.no_grad():
+        for q in layer.parameters():
+            q.copy_(torch.randn_like(q.float()) * (hidden ** -0.5 if q.dim() == 2 else 0.1))
+        layer.linear_qkv.layer_norm.weight.add_(1.0)
+    hs = torch.randn(dn * Lc, 1, hidden, device=dev).bfloat16()
+    y = torch.randn(sum(text), hidden, device=dev).bfloat16()
+    mask = (torch.arange(max(text))[None] < torch.tensor(text)[:, None]).float().view(dn, 1, 1, -1)
+    meta = P.ModelMetaArgs(
+        H=rows, W=cols, cp_pad_size=None, cp_split_sizes=None, slice_point=sp, denoising_range_num=dn, range_num=sp + dn,
+        extract_prefix_video_feature=False, fwd_extra_1st_chunk=False, distill_nearly_clean_chunk=cache == "distill", clip_token_nums=Lc,
+        enable_cuda_graph=False, core_attn_params=P.build_core_attn_params(R.q_ranges_from_chunks(dn, Lc).to(dev),
+                                                                          R.generate_default_kvrange(sp, dn, Lc).to(dev), Lc),
+        cross_attn_params=P.build_cross_attn_params(mask.to(dev), Lc, max(text)))
+    rope = LearnableRotaryEmbeddingCat(D, device=dev).get_embed_for_forward(dn * frames, rows, cols, sp, dn)
+    prefix = torch.randn(sp * Lc, Hkv, 2 * D, device=dev).bfloat16()
+
+    def run():
+        ip = None
+        if cache != "none":
+            ip = P.InferenceParams(1, (sp + dn) * Lc)
+            ip.update_kv_cache = cache != "side"
+            kept = torch.zeros((sp + dn) * Lc, Hkv, 2 * D, dtype=torch.bfloat16, device=dev)
+            kept[:sp * Lc] = prefix
+            ip.key_value_memory_dict[1] = kept
+        n0 = M.lib().magi_launch_count()
+        with torch.no_grad():
+            out = layer(hs, y, ip, rope, meta, proj_layout=proj)
+        n = M.lib().magi_launch_count() - n0
+        return (list(out) if isinstance(out, tuple) else [out]) + ([] if ip is None else [kept]), n
+
+    return layer, run, (hs, y, meta, rope)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("hidden,grid,dn,sp,cache,proj,text", [
+    (768, (2, 6, 10), 2, 2, "append", False, [24, 13]), (768, (2, 6, 10), 2, 2, "side", True, [3, 800]), (256, (1, 5, 9), 3, 1, "distill", False, [8, 0, 1]),
+    (1024, (1, 3, 11), 1, 0, "none", True, [40]), (768, (2, 14, 10), 3, 2, "append", False, [300, 9, 77])])
+def test_small_layer_gives_what_the_separate_launches_give(dev, monkeypatch, hidden, grid, dn, sp, cache, proj, text):
+    """Outputs and cache rows, within what the order of the products' sums does to them (the bar of the fused projection: cosine
+    0.9999, 2e-2 of magnitude-one outputs); three launches instead of five of this library's, and no library product."""
+    layer, run, _ = _layer_case(dev, hidden, *grid, dn, sp, cache, proj, text)
+    got, n_small = run()
+    monkeypatch.setattr(MOD, "_projects_in_one_launch", lambda *a: False)
+    monkeypatch.setattr(MOD, "_text_in_one_launch", lambda *a: False)
+    want, n_apart = run()
+    assert n_small == n_apart - 2
+    for a, b in zip(got, want):
+        x, y = a.double().flatten(), b.double().flatten()
+        assert a.shape == b.shape and float(x @ y / (x.norm() * y.norm())) >= 0.9999 and float((x - y).abs().max()) <= 2e-2 * max(1.0, float(y.abs().max()))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("what", ["patched forward_ln", "hidden rows apart", "text rows backwards", "fp32 text", "autocast", "above the bound", "batch"])
+def test_layers_that_the_one_launch_does_not_take(dev, monkeypatch, what):
+    """Replaced projections are called; other layouts, types and modes go where they went."""
+    layer, run, (hs, y, meta, rope) = _layer_case(dev, 256, 1, 4, 6, 2, 1, "none", False, [8, 5])
+    taken = []
+    monkeypatch.setattr(MOD, "small_projections", lambda *a, **k: taken.append(1) or M.small_projections(*a, **k))
+    call = lambda h, t: layer(h, t, None, rope, meta)  # noqa: E731
+    with torch.no_grad():
+        want = call(hs, y)
+        assert taken
+        taken.clear()
+        if what == "patched forward_ln":
+            calls, own = [], layer.linear_qkv.forward_ln
+            layer.linear_qkv.forward_ln = lambda t: calls.append(1) or own(t)
+            got = call(hs, y)
+            assert calls
+        elif what == "hidden rows apart":
+            got = call(torch.cat([hs, hs], -1)[..., :256], y)
+        elif what == "text rows backwards":  # (columns apart: not rows in one piece)
+            got = call(hs, torch.stack([y, y], -1)[..., 0])
+        elif what == "fp32 text":
+            with pytest.raises(RuntimeError):
+                call(hs, y.float())
+            return
+        elif what == "autocast":
+            with torch.autocast("cuda", dtype=torch.bfloat16):
+                got = call(hs, y)
+        elif what == "above the bound":
+            layer.q_layernorm_xattn.weight.fill_(20.0)
+            got, want = call(hs, y), None
+        else:
+            with pytest.raises(ValueError):  # (as ever: a batch is one range)
+                layer(torch.cat([hs, hs], 1), y, None, rope, meta)
+            return
+    text_only = what in ("patched forward_ln", "hidden rows apart")
+    assert len(taken) <= (1 if text_only else 0)
+    if want is not None:
+        for a, b in zip(got, want):
+            assert float((a.float() - b.float()).abs().max()) <= 2e-2 * max(1.0, float(b.abs().max()))
+
+
+def test_which_layers_take_the_one_launch():
+    cus = 256
+    one = MOD._projects_in_one_launch
+    assert one(240, 20, 48, 4, 768, cus) and one(1600, 20, 0, 4, 768, cus) and not one(1633, 20, 40, 4, 768, cus)
+    assert one(380, 20, 100, 4, 1024, cus) and not one(400, 20, 100, 4, 1024, cus)  # (no taller workgroups there: one round)
+    text = MOD._text_in_one_launch
+    assert text(1e11, 512, 16, 3072, cus) and not text(1e11, 513, 16, 3072, cus) and text(1e11, 2048, 4, 768, cus)
+    assert not text(1e11, 100, 16, 6144, cus) and not text(1.6e11, 100, 16, 3072, cus)
+
+
+def test_struct_layout_matches_header(tmp_path):
+    fields = [f[0] for f in L.SmallProjArgs._fields_]
+    src = ['#include <stdio.h>', '#include <stddef.h>', '#include "magi_attn.h"', 'int main(void){', 'printf("%zu\\n", sizeof(magi_small_proj_args));']
+    src += ['printf("%%zu\\n", offsetof(magi_small_proj_args, %s));' % f for f in fields] + ['return 0;}']
+    c, exe = tmp_path / "layout.c", tmp_path / "layout"
+    c.write_text("\n".join(src))
+    subprocess.run(["gcc", "-I", os.path.join(ROOT, "include"), str(c), "-o", str(exe)], check=True)
+    out = [int(v) for v in subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout.split()]
+    assert out == [C.sizeof(L.SmallProjArgs)] + [getattr(L.SmallProjArgs, f).offset for f in fields]
