@@ -237,9 +237,10 @@ def _text_in_one_launch(flop: float, rows: int, heads: int, K: int, cus: int) ->
     """Whether the K | V projection of the text rows and the K norm run as one launch of small_projections rather than as the library's
     product and a head norm.  In one round of its workgroups (32 rows x one of the `heads`) that takes the device about as long
     (K = 3072, 16 heads: 183 rows 16.2 against 15.2 us, 402 rows 18.9 against 18.8, 800 rows 29 against 24; K = 768, 4 heads: 1500 rows
-    10.7 against 10.4) and the host 8.5 instead of 29 us, which counts where the layer is waiting for the host: below about 150 us of
-    work, `flop` at 1e15 a second.  At K = 6144 the weight rows collide in the caches: 47 us against 18."""
-    return flop < 1.5e11 and K <= 3072 and (rows + 31) // 32 * heads <= cus
+    10.7 against 10.4; with the weights not in the caches up to 8 us more) and the host 8.5 instead of 29 us, which counts where the
+    layer is waiting for the host: whole layers of 24 heads, 468 rows over 2340 keys (3.1e10 flop) 163 / 145 us, 840 over 3360
+    (6.6e10) 167 / 160, but 924 over 4620 in fp8 (8.7e10) 191 / 198.  At K = 6144 the weight rows collide in the caches: 47 us against 18."""
+    return flop < 7e10 and K <= 3072 and (rows + 31) // 32 * heads <= cus
 
 
 def _global_hooks() -> bool:
