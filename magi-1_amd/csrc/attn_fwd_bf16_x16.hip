@@ -513,27 +513,35 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_bf16_x16_kernel(const AttnKer
   }
 }
 
+// workgroups per item of the kernel below
+template <bool CHECK>
+constexpr int MERGE_SHARES = CHECK ? 1 : 4;
+
 // The split items of a launch of the kernel above: sums their pieces, normalises, writes the rows (CHECK: and the verdicts).
-// One workgroup per item, a wavefront for each 64 rows, lane layout of the accumulators as above.  Memory bound: SPLIT_FLOATS
-// * 4 bytes read per piece.
+// A wavefront for each 64 rows, lane layout of the accumulators as above.  Memory bound: SPLIT_FLOATS * 4 bytes read per piece.
+// Four workgroups per item, one for each query block (CHECK: one, which leaves the wavefronts' verdicts), on the item's XCD: with
+// one for all four a launch of 48 items read 0.5 MB per workgroup and nothing beside it.
 template <bool CHECK>
 __global__ __launch_bounds__(256) void attn_fwd_bf16_merge_kernel(const AttnKernArgs a) {
+  constexpr int SHARES = MERGE_SHARES<CHECK>;
   __shared__ int s_sel[LOCATE_WORDS];
   if (gate_closed(a)) return;
   const int tid = threadIdx.x, l = tid & 63, n = l & 15, g = l >> 4;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const WorkItem wi = locate_work(a, 256, tid, s_sel, blockIdx.x + 8u * a.split_from);
+  const unsigned share = (blockIdx.x >> 3) % SHARES, item = ((blockIdx.x >> 3) / SHARES << 3) | (blockIdx.x & 7u);
+  const WorkItem wi = locate_work(a, 256, tid, s_sel, item + 8u * a.split_from);
   const int row0 = wi.q0 + 64 * w;
   if (!wi.valid || wi.ke <= wi.ks) return;  // (nothing there, or without keys: done)
   if (row0 >= wi.qe) {
     if (CHECK && l == 0) a.verdict[4 * (long)wi.item + w] = 0;
     return;
   }
-  const float* const base = a.partial + (long)blockIdx.x * a.split_pieces * SPLIT_FLOATS;
+  const float* const base = a.partial + (long)item * a.split_pieces * SPLIT_FLOATS;
   const int pieces = (int)a.split_pieces;
   bool bad = false;
 #pragma unroll
-  for (int qb = 0; qb < 4; ++qb) {
+  for (int k = 0; k < 4 / SHARES; ++k) {
+    const int qb = CHECK ? k : (int)share;
     const float* p = base;
     float s = 0.f;
     f32x4v o[8];
@@ -755,7 +763,7 @@ void launch_merge(const AttnKernArgs& a, hipStream_t stream) {
   if (const unsigned items = split_items(a)) {
     AttnKernArgs m = a;
     m.flags &= ~ATTN_ZERO_GAPS;  // (the rows no range covers are clear by now)
-    hipLaunchKernelGGL(attn_fwd_bf16_merge_kernel<CHECK>, dim3(8u * items), dim3(256), 0, stream, m);
+    hipLaunchKernelGGL(attn_fwd_bf16_merge_kernel<CHECK>, dim3(8u * items * MERGE_SHARES<CHECK>), dim3(256), 0, stream, m);
   }
 }
 }  // namespace

@@ -33,10 +33,24 @@ constexpr int BM = 32 * NW;
 constexpr int LOADS = 8 / NW;  // direct loads per wave per matrix per tile (8 rows each)
 constexpr float P_SHIFT = 8.f;
 
-// acc * inv as bf16 rows wi.q0 + row0 .. + 31 of out; acc in the lane layout of the PV MFMAs.
-// A lane holds four consecutive features per (mb, b), its partner in the other half wave the next four: the
-// halves trade the odd-b registers of the lower half for the even-b registers of the upper one, after which
-// every lane owns eight consecutive features and stores 16 bytes at a time.  (The row address is derived from
+// acc * inv as bf16, features 32 mb .. +31 of this lane's row (op: the row's bytes + 16 g); acc in the lane layout of the PV MFMAs.
+// A lane holds four consecutive features per b, its partner in the other half wave the next four: the halves trade the odd-b
+// registers of the lower half for the even-b registers of the upper one, after which every lane owns eight consecutive features
+// and stores 16 bytes at a time.
+__device__ __forceinline__ void store_block(bool row_ok, char* op, int mb, const f32x16& acc, float inv) {
+#pragma unroll
+  for (int bp = 0; bp < 2; ++bp) {
+    unsigned ev[2], od[2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      ev[e] = pack_bf16x2(acc[8 * bp + 2 * e] * inv, acc[8 * bp + 2 * e + 1] * inv);
+      od[e] = pack_bf16x2(acc[8 * bp + 4 + 2 * e] * inv, acc[8 * bp + 4 + 2 * e + 1] * inv);
+      half_swap(ev[e], od[e]);  // lower half: (own even, partner's even); upper half: (partner's odd, own odd)
+    }
+    if (row_ok) *(u32x4*)(op + (32 * mb + 16 * bp) * 2) = u32x4{ev[0], ev[1], od[0], od[1]};
+  }
+}
+// acc * inv as bf16 rows wi.q0 + row0 .. + 31 of out.  (The row address is derived from
 // an opaque copy of the lane index so that it is computed here and not carried through the main loop.)
 __device__ __forceinline__ void store_rows(const AttnKernArgs& a, const WorkItem& wi, int row0, int l, const f32x16 (&acc)[4], float inv) {
   int lane_e = l;
@@ -44,18 +58,7 @@ __device__ __forceinline__ void store_rows(const AttnKernArgs& a, const WorkItem
   const bool row_ok = wi.q0 + row0 + (l & 31) < wi.qe;
   char* const op = a.out + (long)(wi.q0 + row0 + (lane_e & 31)) * a.os_t + wi.o_head + 16 * (lane_e >> 5);
 #pragma unroll
-  for (int mb = 0; mb < 4; ++mb)
-#pragma unroll
-    for (int bp = 0; bp < 2; ++bp) {
-      unsigned ev[2], od[2];
-#pragma unroll
-      for (int e = 0; e < 2; ++e) {
-        ev[e] = pack_bf16x2(acc[mb][8 * bp + 2 * e] * inv, acc[mb][8 * bp + 2 * e + 1] * inv);
-        od[e] = pack_bf16x2(acc[mb][8 * bp + 4 + 2 * e] * inv, acc[mb][8 * bp + 4 + 2 * e + 1] * inv);
-        half_swap(ev[e], od[e]);  // lower half: (own even, partner's even); upper half: (partner's odd, own odd)
-      }
-      if (row_ok) *(u32x4*)(op + (32 * mb + 16 * bp) * 2) = u32x4{ev[0], ev[1], od[0], od[1]};
-    }
+  for (int mb = 0; mb < 4; ++mb) store_block(row_ok, op, mb, acc[mb], inv);
 }
 
 // FASTP (with POW2): the probabilities come from a piecewise-linear exp2 built on the matrix pipe's scaling
@@ -477,39 +480,38 @@ __global__ __launch_bounds__(64 * NW, 3) void attn_fwd_fp8_kernel(const AttnKern
 }
 
 // The split items of a launch of the kernel above (a.split_*): brings the pieces' sums to a common maximum, adds them in the order
-// of the keys, normalises, writes the rows.  One workgroup per item, lanes and wavefronts as there.  Memory bound.
+// of the keys, normalises, writes the rows.  Lanes and wavefronts as there, four workgroups per item, one for each 32 features, on the
+// item's XCD.  Memory bound.
 __global__ __launch_bounds__(64 * NW) void attn_fwd_fp8_merge_kernel(const AttnKernArgs a) {
   __shared__ int s_sel[LOCATE_WORDS];
   const int tid = threadIdx.x, l = tid & 63, i = l & 31, g = l >> 5;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const WorkItem wi = locate_work(a, BM, tid, s_sel, blockIdx.x + 8u * a.split_from);
+  const int mb = (int)(blockIdx.x >> 3) & 3;
+  const unsigned item = (blockIdx.x >> 5 << 3) | (blockIdx.x & 7u);
+  const WorkItem wi = locate_work(a, BM, tid, s_sel, item + 8u * a.split_from);
   if (!wi.valid || wi.ke <= wi.ks || wi.q0 + 32 * w >= wi.qe) return;
   const int pieces = (int)a.split_pieces, row = 32 * w + i;
-  const float* const base = a.partial + (long)blockIdx.x * pieces * SPLIT_FLOATS_FP8;
+  const float* const base = a.partial + (long)item * pieces * SPLIT_FLOATS_FP8;
   float m = -__builtin_inff();
   for (int p = 0; p < pieces; ++p) m = fmaxf(m, base[(long)p * SPLIT_FLOATS_FP8 + 128 * 128 + 128 + row]);
   float sum = 0.f;
-  f32x16 o[4];
+  f32x16 o;
 #pragma unroll
-  for (int mb = 0; mb < 4; ++mb)
-#pragma unroll
-    for (int v = 0; v < 16; ++v) o[mb][v] = 0.f;
+  for (int v = 0; v < 16; ++v) o[v] = 0.f;
   for (int p = 0; p < pieces; ++p) {
     const float* const src = base + (long)p * SPLIT_FLOATS_FP8;
     const float f = __builtin_amdgcn_exp2f(src[128 * 128 + 128 + row] - m);
     sum += src[128 * 128 + row] * f;
     const f32x4* const acc = (const f32x4*)src + w * 1024 + l;
 #pragma unroll
-    for (int mb = 0; mb < 4; ++mb)
+    for (int b = 0; b < 4; ++b) {
+      const f32x4 x = acc[(4 * mb + b) * 64];
 #pragma unroll
-      for (int b = 0; b < 4; ++b) {
-        const f32x4 x = acc[(4 * mb + b) * 64];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) o[mb][4 * b + e] += x[e] * f;
-      }
+      for (int e = 0; e < 4; ++e) o[4 * b + e] += x[e] * f;
+    }
   }
-  store_rows(a, wi, 32 * w, l, o, 1.f / sum);
-  if (a.lse && g == 0 && wi.q0 + row < wi.qe) a.lse[(long)wi.h * a.total_q + wi.q0 + row] = (m + __builtin_amdgcn_logf(sum)) * 0.6931471805599453f;
+  store_block(wi.q0 + row < wi.qe, a.out + (long)(wi.q0 + row) * a.os_t + wi.o_head + 16 * g, mb, o, 1.f / sum);
+  if (a.lse && mb == 0 && g == 0 && wi.q0 + row < wi.qe) a.lse[(long)wi.h * a.total_q + wi.q0 + row] = (m + __builtin_amdgcn_logf(sum)) * 0.6931471805599453f;
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -674,7 +676,7 @@ hipError_t launch_attn_fwd_fp8(const AttnKernArgs& a, hipStream_t stream) {
   if (const unsigned items = split_items(a)) {
     AttnKernArgs m = a;
     m.flags &= ~ATTN_ZERO_GAPS;  // (the rows no range covers are clear by now)
-    hipLaunchKernelGGL(attn_fwd_fp8_merge_kernel, dim3(8u * items), dim3(64 * NW), 0, stream, m);
+    hipLaunchKernelGGL(attn_fwd_fp8_merge_kernel, dim3(32u * items), dim3(64 * NW), 0, stream, m);
   }
   return hipGetLastError();
 }
