@@ -67,6 +67,51 @@ def _dtype_code(t: torch.Tensor) -> int:
     raise TypeError(f"unsupported dtype {t.dtype}: bf16 or float8_e4m3fn")
 
 
+def range_count(q_ranges: torch.Tensor, k_ranges: torch.Tensor, mode: int) -> int:
+    """The number of ranges of a pair of device-side lists, refused where a launch could not read them."""
+    if q_ranges.dtype != torch.int32 or k_ranges.dtype != torch.int32:
+        raise TypeError("q_ranges / k_ranges must be int32")
+    if not (q_ranges.is_cuda and k_ranges.is_cuda):
+        raise ValueError("q_ranges / k_ranges must live on the device")
+    if mode == L.MAGI_RANGES_PAIRS:
+        if q_ranges.shape != k_ranges.shape or q_ranges.dim() != 2 or q_ranges.shape[1] != 2:
+            raise ValueError("q_ranges / k_ranges must both be [n, 2]")
+        return q_ranges.shape[0]
+    if q_ranges.numel() != k_ranges.numel():
+        raise ValueError("cu_seqlens_q / cu_seqlens_k must have the same length")
+    return q_ranges.numel() - 1
+
+
+def covered_by_launch(n: int, max_seqlen_q: int, rows: int) -> bool:
+    """Rows that no range covers are zeros (lse -inf).  Where the ranges can cover the rows, the attention launch takes care
+    of the few that are left; a clearing pass over the whole output only where it would have to write most of it."""
+    return 1 <= n <= 64 and max_seqlen_q > 0 and n * max_seqlen_q >= rows
+
+
+def launch_bounded_attention(dev: torch.device, q: int, q_row: int, rows: int, Hq: int, kv: int, side: int, k_split: int, total_k: int,
+                             kv_row: int, Hkv: int, q_ranges: torch.Tensor, k_ranges: torch.Tensor, n: int, mode: int, max_seqlen_q: int,
+                             max_seqlen_k: int, out: int, o_row: int, group_heads: int, o_group: int, clear: bool, bound: float,
+                             q_norm: Optional[tuple] = None) -> None:
+    """range_attention for a caller that has made its tensors itself and knows them to be sound: bf16 rows by address (strides in
+    elements, heads 128 apart), K | V interleaved per head at kv, those from k_split on at `side` (0: none), scores bounded (0 <
+    bound <= MAGI_SCORE_BOUND_MAX).  q carries the softmax scale, or is raw with q_norm = (gamma, beta, eps) by address.  clear: rows no
+    range covers become zeros (the caller has cleared `out` unless covered_by_launch).  Shares keys as range_attention does."""
+    max_seqlen_q, max_seqlen_k = int(max_seqlen_q), int(max_seqlen_k)
+    split, split_bytes = None, 0
+    if max_seqlen_k >= 512:
+        split_bytes = L.lib().magi_attn_split_bytes(Hq, Hkv, max(n, 0), max_seqlen_q, max_seqlen_k, L.MAGI_DTYPE_BF16)
+        if split_bytes:
+            split = torch.empty(split_bytes, dtype=torch.uint8, device=dev)
+    q_ranges, k_ranges = q_ranges.contiguous(), k_ranges.contiguous()
+    gamma, beta, eps = (0, 0, 0.0) if q_norm is None else q_norm
+    flags = (L.MAGI_ATTN_Q_PRESCALED if q_norm is None else 0) | (L.MAGI_ATTN_ZERO_UNCOVERED if clear and covered_by_launch(n, max_seqlen_q, rows) else 0)
+    _launch_packed(
+        dev, "magi_attn_fwd", L.AttnArgs, q, kv, kv + 256, side, side + 256 if side else 0, out, 0, q_ranges.data_ptr(), k_ranges.data_ptr(), 0, 0, 0,
+        q_row, 128, kv_row, 256, kv_row, 256, o_row, 128, rows, total_k, k_split, max(n, 0), mode, max_seqlen_q, max_seqlen_k, Hq, Hkv, 128,
+        L.MAGI_DTYPE_BF16, 0, 0.0, flags, group_heads, o_group, bound, 0, gamma, beta, eps, L.MAGI_NORM_LAYERNORM_1P, 0, 0, 0, 0, 0, 0,
+        0 if split is None else split.data_ptr(), split_bytes)
+
+
 def range_attention(
     q: torch.Tensor,
     k: torch.Tensor,
@@ -150,23 +195,10 @@ def range_attention(
             raise ValueError("k2 / v2 must have the strides of k / v")
         if k_split is None or not (0 <= k_split <= k.shape[0]):
             raise ValueError("k_split must lie inside k")
-    if q_ranges.dtype != torch.int32 or k_ranges.dtype != torch.int32:
-        raise TypeError("q_ranges / k_ranges must be int32")
-    if not (q_ranges.is_cuda and k_ranges.is_cuda):
-        raise ValueError("q_ranges / k_ranges must live on the device")
+    n = range_count(q_ranges, k_ranges, ranges_mode)
     q_ranges = q_ranges.contiguous()
     k_ranges = k_ranges.contiguous()
-    if ranges_mode == L.MAGI_RANGES_PAIRS:
-        n = q_ranges.shape[0]
-        if q_ranges.shape != k_ranges.shape or q_ranges.dim() != 2 or q_ranges.shape[1] != 2:
-            raise ValueError("q_ranges / k_ranges must both be [n, 2]")
-    else:
-        n = q_ranges.numel() - 1
-        if q_ranges.numel() != k_ranges.numel():
-            raise ValueError("cu_seqlens_q / cu_seqlens_k must have the same length")
-    # Rows that no range covers are zeros (lse -inf).  Where the ranges can cover the rows, the attention launch takes care
-    # of the few that are left; a clearing pass over the whole output only where it would have to write most of it.
-    by_kernel = out is None and 1 <= n <= 64 and max_seqlen_q > 0 and n * max_seqlen_q >= Tq
+    by_kernel = out is None and covered_by_launch(n, max_seqlen_q, Tq)
     zero_gaps = by_kernel and (zero_init or return_lse)
     if out is None:
         new = torch.zeros if zero_init and not by_kernel else torch.empty
@@ -503,6 +535,11 @@ def _rows(t: torch.Tensor, name: str) -> None:
         raise ValueError(f"{name} must be a 2-D bf16 device tensor with contiguous rows")
 
 
+def launch_small_projections(dev: torch.device, *fields) -> None:
+    """magi_small_projections with the fields of its argument struct behind struct_size, in order."""
+    _launch_packed(dev, "magi_small_projections", L.SmallProjArgs, *fields)
+
+
 def small_projections(x: Optional[torch.Tensor], w: Optional[torch.Tensor], rope, gq, bq, gk, bk, *, Hq: int, Hkv: int, Hqx: int = 0,
                       ln: Optional[tuple] = None, eps: float = 1e-6, batch: int = 1, q_premul: float = 1.0,
                       kv_out: Optional[torch.Tensor] = None, n_cache_rows: Optional[int] = None,
@@ -565,8 +602,8 @@ def small_projections(x: Optional[torch.Tensor], w: Optional[torch.Tensor], rope
         text_kv = torch.empty((T, Hkv, 2 * D), dtype=torch.bfloat16, device=dev)
     if dev is None:
         raise ValueError("neither x nor text given")
-    _launch_packed(
-        dev, "magi_small_projections", L.SmallProjArgs, _ptr(x), _ptr(w) if x is not None else 0, ln_w, ln_b,
+    launch_small_projections(
+        dev, _ptr(x), _ptr(w) if x is not None else 0, ln_w, ln_b,
         x.stride(0) if S > 1 else K, S, K, ln_fp32, ln_eps, Hq, Hkv, Hqx, R2, _ptr(rope) if R2 else 0, _ptr(gq), _ptr(bq), _ptr(gk),
         _ptr(bk), eps, batch, q_premul,
         n_cache_rows or 0, _ptr(q), _ptr(kv_out), _ptr(kv_tail),

@@ -34,7 +34,7 @@ import torch
 
 from . import _lib as L
 from .cache import Fp8KVCache, OffloadedKVCache
-from .functional import _measuring_a_bound_pays
+from .functional import _measuring_a_bound_pays, covered_by_launch, launch_bounded_attention, launch_small_projections, range_count
 from .functional import (div_clamp_to, head_norm, layer_norm, layer_norm_div_clamp, pow2_scale_for, qk_prologue, qk_prologue_fp8, qkv_proj_prologue,
                          quantize_fp8_split,
                          range_attention, small_projections)
@@ -225,12 +225,12 @@ def _compute_units(device: torch.device) -> int:
 
 def _projects_in_one_launch(rows: int, heads: int, text_rows: int, text_heads: int, K: int, cus: int) -> bool:
     """Whether a layer's projections run as one launch of small_projections: where its workgroups (32 rows x one head each, 64 rows up
-    to K = 768) are one round, or two of the taller ones.  In one round the launch takes less time than the norm, the library's two
-    products, the prologue and the text's head norm (240 + 24 rows at K = 768, 20 + 4 heads, 12.7 against 22 us; 672 rows 19.4
-    against 26), in two about 10 us more (1344 rows 36 against 29), and the host issues it 60 us sooner, which such a layer is waiting
-    for: 840 rows behind 1120, 167 against 105 us for the layer."""
+    to K = 768) are one round, or up to four of the taller ones.  In one round the launch takes less time than the norm, the library's
+    two products, the prologue and the text's head norm (240 + 24 rows at K = 768, 20 + 4 heads, 12.7 against 22 us; 672 rows 19.4
+    against 26), in several more (1344 rows 36 against 29, 2048 39 against 32), but the host issues the layer 100 us sooner, and such
+    layers wait for it: 840 rows behind 1120 167 / 105 us in all, 2048 rows over 6144 keys 154 / 130.  The rest is not measured."""
     tile = lambda n: ((rows + n - 1) // n) * heads + ((text_rows + n - 1) // n) * text_heads  # noqa: E731
-    return tile(64) <= 2 * cus if K <= 768 else tile(32) <= cus
+    return tile(64) <= 4 * cus if K <= 768 else tile(32) <= cus
 
 
 def _text_in_one_launch(flop: float, rows: int, heads: int, K: int, cus: int) -> bool:
@@ -815,25 +815,26 @@ class FullyParallelAttention(torch.nn.Module):
 
     def _cross_attention_fused(self, qx_raw: torch.Tensor, sq: int, b: int, key_value_states: torch.Tensor,
                                cross_attn_params: PackedCrossAttnParams, out: Optional[torch.Tensor],
-                               bound: float, text_kv: Optional[torch.Tensor] = None, own_text: bool = False) -> Optional[torch.Tensor]:
+                               bound: float, own_text: bool = False) -> Optional[torch.Tensor]:
         """Cross attention on the RAW qx projection [sq * b, Hq*D].  Batch 1: the attention kernel applies q_layernorm_xattn
         while it loads q (no normalised copy of q in memory) and, the scores of normed q and k being bounded, runs without a
         running maximum; returns None when that path does not apply (then the caller takes get_xqkv + cross_attention).
         Batch > 1: head norm and online softmax, the arithmetic of get_xqkv + cross_attention bit for bit, on the [position,
         batch] rows where they are (no copy to batch-major order and back: 230 MB each way at the 480p unconditional pass).
-        text_kv: the K | V rows of the text tokens [Ty, Hkv, 2D], K normed, where the caller has them.  own_text: they come from small_projections where it takes the states (else the library's GEMM and a head norm).
+        own_text: the text's K | V rows come from small_projections where it takes the states (else the library's GEMM and a head norm).
         -> [sq, b, Hq, D] contiguous (or `out`, batch 1 only)."""
         if b == 1 and not (0.0 < bound <= L.MAGI_SCORE_BOUND_MAX):
             return None
         D = self.hidden_size_per_attention_head
         q = qx_raw.view(sq * b, -1, D)  # row-strided view of the projection
         m = self._modules
-        if text_kv is None and own_text:
+        text_kv = None
+        if own_text:
             w = _param(m["linear_kv_xattn"], "weight")
             if _plain_rows(key_value_states, w):
                 gk, bk = m["k_layernorm_xattn"].gamma_beta_fp32()
                 text_kv = small_projections(None, None, None, None, None, None, None, Hq=0, Hkv=self.num_query_groups_per_partition,
-                                            eps=self.eps, text=(key_value_states, w.detach(), gk, bk))[4]
+                                            eps=self.eps, text=(key_value_states, w, gk, bk))[4]
         if text_kv is not None:
             kx, v_ = _halves(text_kv, text_kv.shape[0])
         else:
@@ -861,34 +862,118 @@ class FullyParallelAttention(torch.nn.Module):
         x = m.forward_ln(hidden_states)
         return tuple(t.reshape(-1, t.shape[-1]) for t in m.forward_qkvx(x)), x
 
-    def _small_layer(self, hidden_states: torch.Tensor, key_value_states: torch.Tensor):
-        """Batch 1, bf16: what small_projections needs of a small layer whose projections are the library's own: a callable
-        (destinations as keywords) -> its results.  None where the separate launches run: other projections, larger layers, tensors of
-        other types or layouts."""
-        S, _, K = hidden_states.shape
-        if K > 1024 or key_value_states.dim() != 2 or not hidden_states.is_cuda:
+    def _tail_rows(self, rows: int, cache: torch.Tensor) -> torch.Tensor:
+        """Side buffer for the K | V rows that must not be persisted, kept between calls."""
+        tail = getattr(self, "_kv_tail", None)
+        if (tail is None or tail.shape[0] < rows or tail.shape[1:] != cache.shape[1:] or tail.dtype != cache.dtype
+                or tail.device != cache.device):
+            tail = torch.empty(rows, cache.shape[1], cache.shape[2], dtype=cache.dtype, device=cache.device)
+            self._kv_tail = tail
+        return tail[:rows]
+
+    def _forward_small(self, hidden_states: torch.Tensor, key_value_states: torch.Tensor, inference_params: Optional[InferenceParams],
+                       rope: torch.Tensor, meta_args: ModelMetaArgs, proj_layout: bool, bound_core: float, bound_cross: float):
+        """forward() of a small bf16 layer at batch 1 with both score bounds in force, whose projections are the library's own: three
+        launches (magi_small_projections, core attention, cross attention) with their arguments put together in one go.  None, before
+        anything has changed, where forward() goes on with the separate launches: other projections or caches, larger layers, tensors
+        of other types or layouts.
+
+        Such a layer waits for the host: 240 + 24 rows, 20 + 4 heads, 87 us through the callables, 51 this way.  There
+        each launch brings its own checks, allocations and views with it."""
+        S, b, K = hidden_states.shape
+        if K > 1024 or b != 1 or key_value_states.dim() != 2 or not hidden_states.is_cuda or self.fused_projection:
             return None
-        Hq, Hkv, (T, Kt) = self.num_attention_heads, self.num_query_groups_per_partition, key_value_states.shape
-        if Kt > 1024 or not _projects_in_one_launch(S, 2 * (Hq + Hkv), T, 2 * Hkv, max(K, Kt), _compute_units(hidden_states.device)):
+        dev = hidden_states.device
+        Hq, Hkv, D, (T, Kt) = self.num_attention_heads, self.num_query_groups_per_partition, 128, key_value_states.shape
+        if Kt > 1024 or not _projects_in_one_launch(S, 2 * (Hq + Hkv), T, 2 * Hkv, max(K, Kt), _compute_units(dev)):
             return None
         m = self._modules
         lin = m["linear_qkv"]
-        if lin.__dict__.get("fp8_quant", True) or self.fused_projection or not hidden_states.is_contiguous():
+        if lin.__dict__.get("fp8_quant", True) or not hidden_states.is_contiguous() or rope.shape[-1] % 16 or rope.shape[-1] > D:
             return None
         if not (_is_own(lin, _OWN_PROJECTIONS) and _is_own(self, _OWN_CROSS)):
             return None
-        x = hidden_states.view(S, K)
         w, wt, ln = lin.fused_weight(), _param(m["linear_kv_xattn"], "weight"), lin._modules["layer_norm"]
         lw, lb = _param(ln, "weight"), _param(ln, "bias")
-        if not (_plain_rows(x, w) and _plain_rows(key_value_states, wt)) or lw is None or lb is None or lw.dtype is not lb.dtype:
+        if not (_plain_rows(hidden_states[:, 0], w) and _plain_rows(key_value_states, wt)) or lw is None or lb is None:
             return None
-        if lw.dtype not in (torch.bfloat16, torch.float32) or not (lw.is_contiguous() and lb.is_contiguous()) or (
-                lw.data_ptr() | lb.data_ptr()) % 16:
+        if lw.dtype is not lb.dtype or lw.dtype not in (torch.bfloat16, torch.float32) or not (lw.is_contiguous() and lb.is_contiguous()) or (
+                lw.shape[0] != K or lb.shape[0] != K or (lw.data_ptr() | lb.data_ptr()) % 16 or lw.device != dev or key_value_states.device != dev):
             return None
-        par = m["q_layernorm"].gamma_beta_fp32() + m["k_layernorm"].gamma_beta_fp32()
-        text = (key_value_states, wt.detach()) + m["k_layernorm_xattn"].gamma_beta_fp32()
-        return lambda rope, **dst: small_projections(x, w, rope, *par, Hq=Hq, Hkv=Hkv, Hqx=Hq, ln=(lw.detach(), lb.detach(), ln.eps), eps=self.eps,
-                                                     q_premul=self._q_premul, text=text, **dst)
+        cache = tail = offloaded = None
+        start = n_keep = persisted = 0
+        if inference_params is not None and (meta_args.extract_prefix_video_feature or meta_args.fwd_extra_1st_chunk or meta_args.slice_point > 0):
+            if inference_params.max_batch_size != 1:
+                return None
+            cache = self._cache(inference_params, hidden_states.dtype)
+            if isinstance(cache, OffloadedKVCache):
+                offloaded, cache = cache, cache.arena.stages[0]  # (they are all alike; the one in use comes from stage() below)
+            if not isinstance(cache, torch.Tensor) or cache.dtype is not torch.bfloat16 or cache.stride()[1:] != (2 * D, 1) or (
+                    cache.shape[1:] != (Hkv, 2 * D) or cache.stride(0) % 8 or cache.data_ptr() % 16 or cache.device != dev):
+                return None
+            start = meta_args.slice_point * meta_args.clip_token_nums
+            if inference_params.update_kv_cache:
+                n_keep = S - meta_args.clip_token_nums if meta_args.distill_nearly_clean_chunk else S
+            if n_keep < 0 or start + n_keep > cache.shape[0]:
+                return None  # (forward() refuses it)
+            if n_keep < S:
+                tail = self._tail_rows(S - n_keep, cache)
+                if tail.stride() != cache.stride():
+                    return None
+        p, cp = meta_args.core_attn_params, meta_args.cross_attn_params
+        if rope.dim() != 2 or rope.shape[0] != S:
+            raise ValueError("rope must be a contiguous fp32 [S / batch, 2*R2] tensor")
+        core_n = range_count(p.q_range, p.k_range, L.MAGI_RANGES_PAIRS)
+        cross_n = range_count(cp.cu_seqlens_q, cp.cu_seqlens_kv, L.MAGI_RANGES_CU)
+        gq, bq = m["q_layernorm"].gamma_beta_fp32()
+        gk, bk = m["k_layernorm"].gamma_beta_fp32()
+        gx, bx = m["q_layernorm_xattn"].gamma_beta_fp32()
+        gkx, bkx = m["k_layernorm_xattn"].gamma_beta_fp32()
+        # one buffer for q, the raw cross-attention q, the text's K | V rows, and K | V without a cache
+        ws = torch.empty(D * (2 * Hq * S + 2 * Hkv * (T + (S if cache is None else 0))), dtype=torch.bfloat16, device=dev)
+        q = ws.data_ptr()
+        qx = q + 2 * D * Hq * S
+        text_kv = qx + 2 * D * Hq * S
+        row = 2 * D * Hkv  # elements of a K | V row
+        side = 0 if tail is None else tail.data_ptr()
+        if proj_layout and Hq % PROJ_GROUPS == 0:
+            # (rows that no q range / cu_seqlens segment covers are left as allocated: the pipeline's ranges cover
+            # every row, dit_model.py:220-222, 246)
+            out = torch.empty(S, 1, 2 * Hq * D, dtype=torch.bfloat16, device=dev)
+            per = Hq // PROJ_GROUPS
+            core_out = out.data_ptr()
+            cross_out, o_row, groups, o_group, clear = core_out + 2 * per * D, 2 * Hq * D, per, 2 * per * D, False
+        else:
+            core, cross = torch.empty(S, 1, Hq * D, dtype=torch.bfloat16, device=dev), torch.empty(S, 1, Hq * D, dtype=torch.bfloat16, device=dev)
+            core_out, cross_out, o_row, groups, o_group, clear = core.data_ptr(), cross.data_ptr(), Hq * D, 0, 0, True
+            for t, n, most in ((core, core_n, p.max_seqlen_q), (cross, cross_n, cp.max_seqlen_q)):
+                if not covered_by_launch(n, most, S):
+                    t.zero_()
+        if offloaded is not None:  # kv_offload: the prefix comes through a device staging buffer
+            cache = offloaded.stage(start)
+        try:
+            if cache is None:
+                kv, kv_row, new, kept, total = text_kv + 2 * row * T, row, text_kv + 2 * row * T, S, S
+            else:
+                kv, kv_row, kept, total = cache.data_ptr(), cache.stride(0), n_keep, start + S
+                new = kv + 2 * kv_row * start
+            launch_small_projections(
+                dev, hidden_states.data_ptr(), w.data_ptr(), lw.data_ptr(), lb.data_ptr(), K, S, K, int(lw.dtype is torch.float32), ln.eps, Hq,
+                Hkv, Hq, rope.shape[1] // 2, rope.data_ptr(), gq.data_ptr(), bq.data_ptr(), gk.data_ptr(), bk.data_ptr(), self.eps, 1,
+                self._q_premul, kept, q, new, side, kv_row, kv_row, qx, key_value_states.data_ptr(), wt.data_ptr(),
+                key_value_states.stride(0) if T > 1 else Kt, T, Kt, gkx.data_ptr(), bkx.data_ptr(), text_kv)
+            launch_bounded_attention(dev, q, Hq * D, S, Hq, kv, side, start + kept, total, kv_row, Hkv, p.q_range, p.k_range, core_n,
+                                     L.MAGI_RANGES_PAIRS, p.max_seqlen_q, p.max_seqlen_k, core_out, o_row, groups, o_group, clear, bound_core)
+            persisted = n_keep
+        finally:
+            if offloaded is not None:  # the persisted rows go back to the host behind the attention launch
+                offloaded.release(start, persisted)
+        launch_bounded_attention(dev, qx, Hq * D, S, Hq, text_kv, 0, T, T, row, Hkv, cp.cu_seqlens_q, cp.cu_seqlens_kv, cross_n, L.MAGI_RANGES_CU,
+                                 cp.max_seqlen_q, cp.max_seqlen_kv, cross_out, o_row, groups, o_group, clear, bound_cross,
+                                 (gx.data_ptr(), bx.data_ptr(), self.eps))
+        if clear is False:
+            return out
+        return attn_linear_proj_input(core, cross) if proj_layout else (core, cross)
 
     # ------------------------------------------------------------------ forward
     def forward(self, hidden_states: torch.Tensor, key_value_states: torch.Tensor,
@@ -918,27 +1003,22 @@ class FullyParallelAttention(torch.nn.Module):
                 measured = _measuring_a_bound_pays(shape_q, shape_k, p_.q_range.shape[0], p_.max_seqlen_q, p_.max_seqlen_k)
             if measured:
                 core_bound_kw = {"auto_bound": True}
-        # which attention kernels this forward selects (diagnostics; the choice follows from the norm parameters)
-        bounded = lambda b: "bounded-score, 64 rows per wavefront" if 0.0 < b <= L.MAGI_SCORE_BOUND_MAX \
-            else "online softmax, 32 rows per wavefront"
-        self.__dict__["last_forward_kernels"] = {
-            "core": "fp8" if self.attention_dtype == "fp8" else
-            ("measured bound: bounded-score or online softmax, chosen on the device" if measured else bounded(bound_core)),
-            "core_score_bound": bound_core,
-            "cross": bounded(bound_cross if hidden_states.shape[1] == 1 else float("inf")),
-            "cross_score_bound": bound_cross}
         bs = hidden_states.shape[1]
         sq = hidden_states.shape[0]
         D = self.hidden_size_per_attention_head
+        # which attention kernels this forward selects (diagnostics; the choice follows from the norm parameters)
+        core_bounded, cross_bounded = 0.0 < bound_core <= L.MAGI_SCORE_BOUND_MAX, bs == 1 and 0.0 < bound_cross <= L.MAGI_SCORE_BOUND_MAX
+        self.__dict__["last_forward_kernels"] = {
+            "core": "fp8" if self.attention_dtype == "fp8" else
+            ("measured bound: bounded-score or online softmax, chosen on the device" if measured else _KERNEL_NAMES[core_bounded]),
+            "core_score_bound": bound_core, "cross": _KERNEL_NAMES[cross_bounded], "cross_score_bound": bound_cross}
+        if core_bounded and cross_bounded and self.attention_dtype == "bf16":
+            small = self._forward_small(hidden_states, key_value_states, inference_params, rope, meta_args, proj_layout, bound_core, bound_cross)
+            if small is not None:
+                return small
         one_launch = (self.fused_projection and self.attention_dtype == "bf16" and bs == 1
                       and rope.shape[-1] == 96 and hidden_states.shape[-1] % 64 == 0)
-        small = None
-        text_kv = None
-        if bs == 1 and self.attention_dtype == "bf16" and 0.0 < bound_cross <= L.MAGI_SCORE_BOUND_MAX:
-            small = self._small_layer(hidden_states, key_value_states) if rope.shape[-1] % 16 == 0 and rope.shape[-1] <= D else None
-        if small is not None:
-            mixed_qqkv, raw, qx_raw = hidden_states, None, None
-        elif one_launch:
+        if one_launch:
             # projections + prologue in one launch: nothing raw reaches memory (qx leaves unnormalised, as the
             # cross-attention kernel takes it)
             mixed_qqkv = self.linear_qkv.forward_ln(hidden_states)
@@ -953,10 +1033,6 @@ class FullyParallelAttention(torch.nn.Module):
 
         def project(kv_out=None, n_cache_rows=None, kv_tail=None):
             """-> (q [S, Hq, D] carrying the softmax scale, kv destination(s), qx_raw [sq * b, Hq*D])"""
-            nonlocal text_kv
-            if small is not None:
-                q_, kv_, tail_, qx_, text_kv = small(rope, kv_out=kv_out, n_cache_rows=n_cache_rows, kv_tail=kv_tail)
-                return q_, (kv_ if tail_ is None else (kv_, tail_)), qx_.view(sq, -1)
             if not one_launch:
                 q_, kv_ = self._fused_qkv(mixed_qqkv, None, None, kv_out=kv_out, n_cache_rows=n_cache_rows,
                                           kv_tail=kv_tail, raw=raw, q_premul=self._q_premul, rope=rope)
@@ -973,11 +1049,10 @@ class FullyParallelAttention(torch.nn.Module):
             if bs > 1 and not own_cross:  # (a replaced cross attention runs; at batch 1 with a bound in force it never did)
                 return None
             flop = 512.0 * sq * Hq * (hidden_states.shape[2] + p.max_seqlen_k)
-            own_text = (bs == 1 and text_kv is None and key_value_states.dim() == 2 and hidden_states.is_cuda and _text_in_one_launch(
+            own_text = (bs == 1 and key_value_states.dim() == 2 and hidden_states.is_cuda and _text_in_one_launch(
                 flop, key_value_states.shape[0], 2 * self.num_query_groups_per_partition, key_value_states.shape[1],
                 _compute_units(hidden_states.device)))
-            return self._cross_attention_fused(qx_raw, sq, bs, key_value_states, meta_args.cross_attn_params, dst, bound_cross, text_kv,
-                                               own_text)
+            return self._cross_attention_fused(qx_raw, sq, bs, key_value_states, meta_args.cross_attn_params, dst, bound_cross, own_text)
 
         get_xqkv = lambda m, y: self.get_xqkv(m, y, qx_raw=qx_raw.view(sq, bs, -1))
         p = meta_args.core_attn_params
@@ -1018,14 +1093,7 @@ class FullyParallelAttention(torch.nn.Module):
                 if offloaded is not None:
                     offloaded.release()
                 raise ValueError("KV cache overflow")
-            tail = None
-            if n_keep < S:  # side buffer for the rows that must not be persisted, kept between calls
-                tail = getattr(self, "_kv_tail", None)
-                if (tail is None or tail.shape[0] < S - n_keep or tail.shape[1:] != cache.shape[1:]
-                        or tail.dtype != cache.dtype or tail.device != cache.device):
-                    tail = torch.empty(S - n_keep, cache.shape[1], cache.shape[2], dtype=cache.dtype, device=cache.device)
-                    self._kv_tail = tail
-                tail = tail[:S - n_keep]
+            tail = self._tail_rows(S - n_keep, cache) if n_keep < S else None
             persisted = 0
             try:
                 q, _, qx_raw = project(kv_out=cache[start:], n_cache_rows=n_keep, kv_tail=tail)
@@ -1058,6 +1126,7 @@ class FullyParallelAttention(torch.nn.Module):
         return core_attn_out, xattn_out
 
 
+_KERNEL_NAMES = ("online softmax, 32 rows per wavefront", "bounded-score, 64 rows per wavefront")  # by: a bound is in force
 # the methods whose work forward() does in another shape, as long as they are these
 _OWN_FP8_LINEAR = {"forward": PerTensorQuantizedFp8Linear.forward}
 _OWN_PROJECTIONS = {"forward_ln": CustomLayerNormLinear.forward_ln, "forward_qkvx": CustomLayerNormLinear.forward_qkvx}

@@ -6,6 +6,7 @@ land on the neighbouring bf16, as in any product summed in another order: the 2-
 rounding to bf16 that the expected values do without (2^-9 / sqrt(3) = 1.1e-3 uniformly, 1.7e-3 at the low end of a binade), bar
 2.5e-3, and no element is further off than 2^-6 of its row's largest."""
 import ctypes as C
+import dataclasses
 import os
 import subprocess
 
@@ -167,12 +168,30 @@ def test_small_layer_gives_what_the_separate_launches_give(dev, monkeypatch, hid
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("ranges", ["a gap behind each", "one of three"])
+def test_rows_outside_the_ranges_of_a_small_layer_are_zeros(dev, ranges):
+    """By the attention launch where the ranges can cover the rows, by a clearing pass where they cannot."""
+    layer, _, (hs, y, meta, rope) = _layer_case(dev, 256, 1, 5, 9, 3, 0, "none", False, [8, 3, 1])
+    p = meta.core_attn_params
+    if ranges == "one of three":
+        q, k, covered = p.q_range[1:2].contiguous(), p.k_range[1:2].contiguous(), torch.arange(135, device=dev) // 45 == 1
+    else:
+        q, k, covered = p.q_range - torch.tensor([0, 4], dtype=torch.int32, device=dev), p.k_range, torch.arange(135, device=dev) % 45 < 41
+    with torch.no_grad():
+        whole = layer(hs, y, None, rope, meta)[0]
+        layer(hs * 3, y, None, rope, meta)  # (so that freshly allocated outputs hold something)
+        part = layer(hs, y, None, rope, dataclasses.replace(meta, core_attn_params=dataclasses.replace(p, q_range=q, k_range=k)))[0]
+    assert (part[~covered] == 0).all() and torch.equal(part[covered], whole[covered])
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("what", ["patched forward_ln", "hidden rows apart", "text rows backwards", "fp32 text", "autocast", "above the bound", "batch"])
 def test_layers_that_the_one_launch_does_not_take(dev, monkeypatch, what):
     """Replaced projections are called; other layouts, types and modes go where they went."""
     layer, run, (hs, y, meta, rope) = _layer_case(dev, 256, 1, 4, 6, 2, 1, "none", False, [8, 5])
     taken = []
-    monkeypatch.setattr(MOD, "small_projections", lambda *a, **k: taken.append(1) or M.small_projections(*a, **k))
+    for name in ("small_projections", "launch_small_projections"):
+        monkeypatch.setattr(MOD, name, lambda *a, _f=getattr(MOD, name), **k: taken.append(1) or _f(*a, **k))
     call = lambda h, t: layer(h, t, None, rope, meta)  # noqa: E731
     with torch.no_grad():
         want = call(hs, y)
@@ -211,7 +230,7 @@ def test_layers_that_the_one_launch_does_not_take(dev, monkeypatch, what):
 def test_which_layers_take_the_one_launch():
     cus = 256
     one = MOD._projects_in_one_launch
-    assert one(240, 20, 48, 4, 768, cus) and one(1600, 20, 0, 4, 768, cus) and not one(1633, 20, 40, 4, 768, cus)
+    assert one(240, 20, 48, 4, 768, cus) and one(2048, 20, 1600, 4, 768, cus) and not one(3265, 20, 40, 4, 768, cus)
     assert one(380, 20, 100, 4, 1024, cus) and not one(400, 20, 100, 4, 1024, cus)  # (no taller workgroups there: one round)
     text = MOD._text_in_one_launch
     assert text(6e10, 512, 16, 3072, cus) and not text(6e10, 513, 16, 3072, cus) and text(6e10, 2048, 4, 768, cus)
