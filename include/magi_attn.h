@@ -231,7 +231,8 @@ typedef struct magi_attn_args {
   int64_t split_workspace_bytes;
 } magi_attn_args;
 
-/* Bytes of split_workspace that a call of these sizes makes use of (dtype: MAGI_DTYPE_*); 0: such a call is not split. */
+/* Bytes of split_workspace that a call of these sizes may make use of (dtype: MAGI_DTYPE_*); 0: such a call is not split.  (Where
+ * smaller workgroups fill the chip better, only MAGI_ATTN_CHECKED does.) */
 int64_t magi_attn_split_bytes(int32_t Hq, int32_t Hkv, int32_t n_ranges, int32_t max_seqlen_q, int32_t max_seqlen_k, int32_t dtype);
 
 int magi_attn_fwd(const magi_attn_args* args, void* stream);

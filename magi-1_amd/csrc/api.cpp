@@ -160,6 +160,35 @@ SplitPlan split_plan(unsigned items, int n_ranges, int max_seqlen_q, int max_seq
   return s;
 }
 
+// How a launch of the 64-rows-per-wavefront kernel without a running maximum is cut: workgroups of 256 rows, their last round's
+// items sharing keys where that pays and the caller has brought the memory, or workgroups of 128 rows
+// (32 per wavefront; a row's bits are the same).  Those fetch and read every tile for half the rows, so they are only for launches
+// that leave two of them per CU a CU of their own or nearly: a tile of 64 keys then takes 1.15 us alone on its CU, 1.75 beside
+// another, against 1.75 and 2.5 to 3.0 of 256 rows.  Measured, 24 / 8 heads, 256 rows whole / in pieces / 128 rows: up to one
+// workgroup per CU 240 rows over 960 keys 32.1 / - / 21.5 us, 900 over 2000 61 / 45 / 42, text of 183 rows for 468 15.1 / - / 10.5;
+// up to two 1300 over 1300 43.5 / - / 37.3, 2600 over 13000 502 / 404 / 366, four ranges of 288 over 1152 to 2016 61 / - / 45; beyond
+// 972 x 4 over 972 to 3888 130 / - / 123, but 3800 over 3800 168 / - / 172 and 1000 x 3 over 3000 to 5000 161 / 148 / 173.  Few items
+// with long keys are better off in pieces, which cost about 12 us and 0.3 per piece of an XCD: 240 rows over 3000 keys 86 / 33 / 56,
+// 1300 over 4000 113 / 81 / 97.
+struct TilePlan {
+  int rows;
+  SplitPlan split;
+};
+TilePlan tile_plan(int Hq, int Hkv, int n_ranges, int max_seqlen_q, int max_seqlen_k, int64_t split_bytes) {
+  auto items = [&](int rows) { return items_per_xcd(Hq, Hkv, n_ranges, max_seqlen_q / rows + (max_seqlen_q % rows != 0)); };
+  const SplitPlan none = {UINT32_MAX, 1, 1, 1, false};
+  const unsigned cus = (unsigned)compute_units() / 8, whole = items(256), half = items(128);
+  TilePlan t = {256, split_bytes > 0 ? split_plan(whole, n_ranges, max_seqlen_q, max_seqlen_k, false) : none};
+  if (t.split.bytes(whole) > split_bytes) t.split = none;
+  if (half > 2 * cus) return t;
+  if (t.split.from < whole) {  // (without a whole round ahead of them: all items are in pieces)
+    const unsigned pieces = whole * t.split.pieces;
+    const double tiles = (max_seqlen_k + 63) / 64, in_pieces = tiles * t.split.num / t.split.den * (pieces <= cus ? 1.75 : 2.6) + 12.0 + 0.3 * pieces;
+    if (in_pieces <= tiles * (half <= cus ? 1.15 : 1.75)) return t;
+  }
+  return {128, none};
+}
+
 int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace);
 
 // the caller's struct as this version lays it out: itself, or `full` filled from the shorter one of version 103
@@ -399,7 +428,10 @@ int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace) {
     if (p->dtype == MAGI_DTYPE_BF16) {
       const double wg384 = (double)p->Hq * p->n_ranges * ((p->max_seqlen_q + 383) / 384);
       const bool long_keys = p->max_seqlen_k == 0 || p->max_seqlen_k >= 4096;  // (0 = not stated)
-      if (bounded)
+      if (bounded && !checked && !mfma32)
+        a.block_m = tile_plan(p->Hq, p->Hkv, p->n_ranges, p->max_seqlen_q, p->max_seqlen_k,
+                              p->split_workspace ? p->split_workspace_bytes : 0).rows;
+      else if (bounded)
         a.block_m = 256;  // (512-row workgroups fetch half the tiles and measure 1 % slower: their two waves per SIMD march in step)
       else if (wg384 >= 9.0 * compute_units() && long_keys)
         a.block_m = 384;
@@ -434,7 +466,7 @@ int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace) {
       e = magi::launch_attn_fwd_fp8(a, static_cast<hipStream_t>(stream));
     else if (checked)
       e = magi::launch_attn_fwd_bf16_checked(a, compute_units(), static_cast<hipStream_t>(stream));
-    else if (bounded && a.block_m == 256 && !mfma32)
+    else if (bounded && a.block_m <= 256 && !mfma32)
       e = magi::launch_attn_fwd_bf16_x16(a, static_cast<hipStream_t>(stream));
     else if (bounded)
       e = magi::launch_attn_fwd_bf16_w64(a, static_cast<hipStream_t>(stream));

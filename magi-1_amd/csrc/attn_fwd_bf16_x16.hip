@@ -101,10 +101,13 @@ __device__ __forceinline__ void store_partial_zero(float* out, int w, int l) {
   out[256 * 128 + 64 * w + l] = 0.f;
 }
 
-template <int QMODE>
+// QB: query blocks of 16 rows per wavefront: 4, or 2 for launches that are better dealt in smaller pieces (tile_rows in api.cpp).
+// A row's result does not depend on it, bit for bit.
+template <int QMODE, int QB = 4>
 __global__ __launch_bounds__(256, 2) void attn_fwd_bf16_x16_kernel(const AttnKernArgs a) {
   constexpr bool CHECK = QMODE == Q_CHECK;
-  constexpr int NW = 4, BM = 64 * NW;
+  constexpr int NW = 4, WROWS = 16 * QB, BM = WROWS * NW;
+  static_assert(QB == 4 || (QB == 2 && !CHECK), "two query blocks: no verdicts, no shared keys");
   constexpr int LOADS = BN / (4 * NW);  // direct loads per wave per matrix per tile (4 rows each)
   constexpr int RING = 4;               // operand fragments in flight between LDS and the MFMAs
   // K and V double buffered in four separate LDS objects that are only named statically (an operand read then
@@ -120,7 +123,8 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_bf16_x16_kernel(const AttnKer
   const int tid = threadIdx.x;
   if (CHECK && tid == 0) s_over = 0;
   unsigned block = blockIdx.x;
-  const SplitPiece sp = split_piece<SPLIT_FLOATS>(a, block);
+  SplitPiece sp = {nullptr, 0u};
+  if constexpr (QB == 4) sp = split_piece<SPLIT_FLOATS>(a, block);
   const WorkItem wi = locate_work(a, BM, tid, s_sel, block);
   if (!wi.valid) return;
   const int qe = wi.qe;
@@ -128,10 +132,10 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_bf16_x16_kernel(const AttnKer
 
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l = tid & 63, n = l & 15, g = l >> 4;
-  const int row0 = wi.q0 + 64 * w;  // first row of this wave
+  const int row0 = wi.q0 + WROWS * w;  // first row of this wave
   if (ke <= ks) {
 #pragma unroll
-    for (int b = 0; b < 2; ++b)
+    for (int b = 0; b < QB / 2; ++b)
       if (row0 + 32 * b + (l & 31) < qe) store_empty_row(a, wi, row0 + 32 * b + (l & 31), l >> 5);
     if (CHECK && l == 0) a.verdict[4 * (long)wi.item + w] = 0;
     return;
@@ -212,9 +216,9 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_bf16_x16_kernel(const AttnKer
   issue_mat(ks + last * BN, sV0, true);
 
   // ---- Q fragments (B operand of S^T = K Q^T): lane (n, g) holds Q[row 16 qb + n][32 kk + 8 g .. +8] ----
-  bf16x8 qf[4][4];
+  bf16x8 qf[QB][4];
 #pragma unroll
-  for (int qb = 0; qb < 4; ++qb) {
+  for (int qb = 0; qb < QB; ++qb) {
     const int qr = min(row0 + 16 * qb + n, qe - 1);
     const char* qp = a.q + row_offset(a, qr, a.qs_t, a.qs_b) + (long)wi.h * a.qs_h + g * 16;
 #pragma unroll
@@ -223,7 +227,7 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_bf16_x16_kernel(const AttnKer
   if constexpr (QMODE == Q_SCALE) {
     const float cs = a.scale_log2;
 #pragma unroll
-    for (int qb = 0; qb < 4; ++qb)
+    for (int qb = 0; qb < QB; ++qb)
 #pragma unroll
       for (int kk = 0; kk < 4; ++kk)
 #pragma unroll
@@ -234,9 +238,9 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_bf16_x16_kernel(const AttnKer
     // one rounding to bf16.  A row's features are spread over the four lanes (n, 0..3): 32 each, feature
     // 32 kk + 8 g + e in fragment kk, element e.
     const float inv_d = 1.f / 128.f;
-    float mean[4], rstd[4];
+    float mean[QB], rstd[QB];
 #pragma unroll
-    for (int qb = 0; qb < 4; ++qb) {
+    for (int qb = 0; qb < QB; ++qb) {
       float sum = 0.f;
 #pragma unroll
       for (int kk = 0; kk < 4; ++kk)
@@ -270,7 +274,7 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_bf16_x16_kernel(const AttnKer
         b1 = bp[1];
       }
 #pragma unroll
-      for (int qb = 0; qb < 4; ++qb)
+      for (int qb = 0; qb < QB; ++qb)
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
           const float gm = (e < 4 ? g0[e & 3] : g1[e & 3]) + 1.f;
@@ -294,8 +298,8 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_bf16_x16_kernel(const AttnKer
   const int r4 = n >> 2, c4 = n & 3;
   const int base_v = g * V_GROUP + r4 * ROW_BYTES + (r4 << 5) + (c4 << 3);
 
-  f32x4v o_acc[8][4];  // [d block][query block]; zeroed below, right ahead of the first tile
-  float l_run[4] = {0.f, 0.f, 0.f, 0.f};  // this lane's share of the row sums, per query block
+  f32x4v o_acc[8][QB];  // [d block][query block]; zeroed below, right ahead of the first tile
+  float l_run[QB] = {};  // this lane's share of the row sums, per query block
   const bool wave_on = row0 < qe;
   const f32x4v zero4 = {0.f, 0.f, 0.f, 0.f};
 
@@ -317,8 +321,8 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_bf16_x16_kernel(const AttnKer
     static_for<0, RD>([&](auto oc) __attribute__((always_inline)) { ring[decltype(oc)::value] = read_op(oc); });
     __builtin_amdgcn_sched_barrier(0);
 
-    f32x4v sc[2][4];  // scores of the current half: [key block][query block]
-    u32x4 pf[4];      // their probabilities as the B operand of the PV MFMAs, per query block
+    f32x4v sc[2][QB];  // scores of the current half: [key block][query block]
+    u32x4 pf[QB];     // their probabilities as the B operand of the PV MFMAs, per query block
     auto consume = [&](auto oc) __attribute__((always_inline)) {
       constexpr int o = decltype(oc)::value;
       constexpr int t = o >> 4, j = o & 15;
@@ -337,7 +341,7 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_bf16_x16_kernel(const AttnKer
         pf[qb][2 * kb + 1] = pack_bf16x2(p2, p3);
       };
       if constexpr (j == 8) {
-        static_for<0, 4>([&](auto qc) __attribute__((always_inline)) {
+        static_for<0, QB>([&](auto qc) __attribute__((always_inline)) {
           soft(std::integral_constant<int, 0>{}, qc);
           soft(std::integral_constant<int, 1>{}, qc);
         });
@@ -362,13 +366,13 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_bf16_x16_kernel(const AttnKer
           for (int r = 0; r < 4; ++r) c0[r] = r < left ? 0.f : (CHECK ? -__builtin_inff() : -1.0e4f);
         }
 #pragma unroll
-        for (int qb = 0; qb < 4; ++qb)
+        for (int qb = 0; qb < QB; ++qb)
           sc[kb][qb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ring[o % RD], qf[qb][kk], kk == 0 ? c0 : sc[kb][qb], 0, 0, 0);
       } else {
         // O^T[d][q] += V^T[d][key] P^T[key][q]
         constexpr int db = v_block(j - 8);
 #pragma unroll
-        for (int qb = 0; qb < 4; ++qb)
+        for (int qb = 0; qb < QB; ++qb)
           o_acc[db][qb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ring[o % RD], __builtin_bit_cast(bf16x8, pf[qb]), o_acc[db][qb], 0, 0, 0);
       }
       // refill the slot just consumed with the fragment RD ahead; the first RD V^T fragments of a half are requested
@@ -396,13 +400,16 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_bf16_x16_kernel(const AttnKer
   // there, a round trip to scratch memory for every workgroup.  (Here, behind the q fragments, so that the 128
   // registers are not held while q is loaded and normalised: the statement below pins the finished q fragments
   // ahead of them, or the compiler sinks the norm arithmetic to its first use, behind the zeros.)
-  asm volatile("" ::"v"(qf[0][0]), "v"(qf[0][1]), "v"(qf[0][2]), "v"(qf[0][3]), "v"(qf[1][0]), "v"(qf[1][1]), "v"(qf[1][2]),
+  if constexpr (QB == 2)
+    asm volatile("" ::"v"(qf[0][0]), "v"(qf[0][1]), "v"(qf[0][2]), "v"(qf[0][3]), "v"(qf[1][0]), "v"(qf[1][1]), "v"(qf[1][2]), "v"(qf[1][3]));
+  if constexpr (QB == 4)
+    asm volatile("" ::"v"(qf[0][0]), "v"(qf[0][1]), "v"(qf[0][2]), "v"(qf[0][3]), "v"(qf[1][0]), "v"(qf[1][1]), "v"(qf[1][2]),
                "v"(qf[1][3]), "v"(qf[2][0]), "v"(qf[2][1]), "v"(qf[2][2]), "v"(qf[2][3]), "v"(qf[3][0]), "v"(qf[3][1]),
                "v"(qf[3][2]), "v"(qf[3][3]));
 #pragma unroll
   for (int db = 0; db < 8; ++db)
 #pragma unroll
-    for (int qb = 0; qb < 4; ++qb) {
+    for (int qb = 0; qb < QB; ++qb) {
       o_acc[db][qb] = f32x4v{0.f, 0.f, 0.f, 0.f};
       asm volatile("" : "+v"(o_acc[db][qb]));
     }
@@ -425,7 +432,7 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_bf16_x16_kernel(const AttnKer
     // may still grow; an overflow is final).
     bool over = false;
 #pragma unroll
-    for (int qb = 0; qb < 4; ++qb) over |= !(l_run[qb] <= SUM_MAX);
+    for (int qb = 0; qb < QB; ++qb) over |= !(l_run[qb] <= SUM_MAX);
     if (wave_on && over) s_over = 1;
     __syncthreads();
     if (__builtin_amdgcn_readfirstlane(s_over) != 0) {
@@ -445,7 +452,7 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_bf16_x16_kernel(const AttnKer
     if (!wave_on) return;
     f32x4v* const dst = (f32x4v*)sp.out + w * 2048 + l;
 #pragma unroll
-    for (int qb = 0; qb < 4; ++qb) {
+    for (int qb = 0; qb < QB; ++qb) {
       float s = l_run[qb];
       s += __shfl_xor(s, 16);
       s += __shfl_xor(s, 32);
@@ -458,7 +465,7 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_bf16_x16_kernel(const AttnKer
   }
 
   // ---- epilogue: normalise, transpose through LDS, store whole rows ----
-  __syncthreads();  // every wave is done with the tile slots: wave w takes slot w as its 64 x 256-byte staging area
+  __syncthreads();  // every wave is done with the tile slots: wave w takes slot w as its staging area of 256 bytes a row
   if (!wave_on) {
     if (CHECK && l == 0) a.verdict[4 * (long)wi.item + w] = 0;
     return;
@@ -469,7 +476,7 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_bf16_x16_kernel(const AttnKer
   const int ne = lane_e & 15, ge = lane_e >> 4;
   bool bad = false;
 #pragma unroll
-  for (int qb = 0; qb < 4; ++qb) {
+  for (int qb = 0; qb < QB; ++qb) {
     float s = l_run[qb];
     s += __shfl_xor(s, 16);
     s += __shfl_xor(s, 32);
@@ -505,7 +512,7 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_bf16_x16_kernel(const AttnKer
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   // 16 lanes x 16 bytes = one row; the wave stores four rows per instruction
 #pragma unroll
-  for (int it = 0; it < 16; ++it) {
+  for (int it = 0; it < 4 * QB; ++it) {
     const int r = 4 * it + ge;
     const u32x4 v = *LDS_PTR(const u32x4, stage + r * ROW_BYTES + ((ne ^ (r & 15)) << 4));
     const int q_row = row0 + r;
@@ -770,6 +777,15 @@ void launch_merge(const AttnKernArgs& a, hipStream_t stream) {
 
 hipError_t launch_attn_fwd_bf16_x16(const AttnKernArgs& a, hipStream_t stream) {
   const dim3 grid(split_grid(a));
+  if (a.block_m == 128) {
+    if (a.q_norm_gamma)
+      hipLaunchKernelGGL((attn_fwd_bf16_x16_kernel<Q_NORM, 2>), grid, dim3(256), 0, stream, a);
+    else if (a.flags & ATTN_SCALE_Q)
+      hipLaunchKernelGGL((attn_fwd_bf16_x16_kernel<Q_SCALE, 2>), grid, dim3(256), 0, stream, a);
+    else
+      hipLaunchKernelGGL((attn_fwd_bf16_x16_kernel<Q_AS_IS, 2>), grid, dim3(256), 0, stream, a);
+    return hipGetLastError();
+  }
   if (a.q_norm_gamma)  // raw q, normalised while it is loaded (cross attention)
     hipLaunchKernelGGL(attn_fwd_bf16_x16_kernel<Q_NORM>, grid, dim3(256), 0, stream, a);
   else if (a.flags & ATTN_SCALE_Q)  // unscaled q, scaled while it is loaded (the reference-shaped callables)
