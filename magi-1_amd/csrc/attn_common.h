@@ -60,6 +60,14 @@ __device__ __forceinline__ void wait_vmcnt() {
   asm volatile("" ::: "memory");
 }
 
+// Workgroup barrier that leaves this wavefront's direct loads into LDS in flight (__syncthreads() waits for every one of them,
+// s_waitcnt vmcnt(0)); its LDS reads and writes are over.
+__device__ __forceinline__ void barrier_loads_in_flight() {
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
 // p0 + p1 + acc for a packed pair of bf16 values
 __device__ __forceinline__ float pair_sum(unsigned pk, float acc) {
   const bf16x2 one = {(__bf16)1.0f, (__bf16)1.0f};

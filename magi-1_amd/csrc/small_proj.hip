@@ -5,10 +5,11 @@
 //
 // What bounds it: latency.  Below about a thousand rows the library's GEMM, the norm ahead of it and the prologue behind it
 // each live for little more than a launch and a few trips to memory, and a library call costs the host 18 us to issue.
-// So: many small workgroups.  A workgroup of four wavefronts forms 32 rows x one head (128 columns); the weight rows stream
-// through LDS in steps of 64 elements of K, three stages filled by direct global->LDS loads, 128 bytes of a row per eight lanes
-// (operands loaded straight into registers, 16 bytes per lane from 16 rows at a time, move 16 bytes per clock and CU: 33 us
-// for 400 text tokens at K = 3072), one barrier per step.  The product is formed transposed, W X^T on
+// So: many small workgroups.  A workgroup of four wavefronts forms 32 or 64 rows x one head (128 columns); the weight rows stream
+// through LDS in steps of 64 elements of K, three to six stages filled by direct global->LDS loads, 128 bytes of a row per eight
+// lanes, which stay in flight over the barriers (__syncthreads() would wait for them: layers of 768 rows 121 against 116 us, of 840
+// rows 158 against 148) (operands loaded straight into registers, 16 bytes per lane from 16 rows at a time, move 16 bytes per clock and CU: 33 us
+// for 400 text tokens at K = 3072, 16 so).  The product is formed transposed, W X^T on
 // v_mfma_f32_16x16x32_bf16 with the weight rows as the A operand: register r of lane (n, g) of a result block is column 4 g + r
 // of the block, row n; it goes through LDS to eight lanes per row, which do with it what the prologue does.
 // RES: the workgroup's rows are in LDS whole (K up to 1024), normalised ahead of the product; their statistics are merged from
@@ -130,15 +131,16 @@ __device__ __forceinline__ void store_rows32(const SmallProjKernArgs& a, const R
 
 // RES: the rows whole in LDS ahead of the product, normalised on the way there; else they stream beside the weights, as they are
 template <bool RES, int ROWS>
-__global__ __launch_bounds__(64 * NW, RES ? 1 : 2) void small_proj_kernel(const SmallProjKernArgs a) {
-  constexpr int NST = RES && ROWS == 64 ? 3 : 4;  // stages
-  constexpr int TB = ROWS / 16;                   // blocks of 16 rows
+__global__ __launch_bounds__(64 * NW, 1) void small_proj_kernel(const SmallProjKernArgs a) {
+  constexpr int NST = RES ? (ROWS == 64 ? 3 : 4) : 6;  // stages
+  constexpr int TB = ROWS / 16;                        // blocks of 16 rows
   constexpr int STAGE_X = RES ? 16 : ROWS * BK * 2;
   // the stages, named statically (an operand read then does not wait for the loads in flight to another stage)
-  __shared__ __attribute__((aligned(1024))) unsigned char sW0[STAGE_W], sW1[STAGE_W], sW2[STAGE_W], sW3[NST > 3 ? STAGE_W : 16];
-  __shared__ __attribute__((aligned(1024))) unsigned char sX0[STAGE_X], sX1[STAGE_X], sX2[STAGE_X], sX3[STAGE_X];
+  __shared__ __attribute__((aligned(1024))) unsigned char sW0[STAGE_W], sW1[STAGE_W], sW2[STAGE_W], sW3[NST > 3 ? STAGE_W : 16],
+      sW4[NST > 4 ? STAGE_W : 16], sW5[NST > 5 ? STAGE_W : 16];
+  __shared__ __attribute__((aligned(1024))) unsigned char sX0[STAGE_X], sX1[STAGE_X], sX2[STAGE_X], sX3[STAGE_X], sX4[STAGE_X], sX5[STAGE_X];
   __shared__ __attribute__((aligned(1024))) unsigned char sR[RES ? ROWS * (2 * res_max_k<ROWS>() + 16) : 16];
-  static_assert((RES ? 0 : 4 * STAGE_X) + NST * STAGE_W + (RES ? (int)sizeof(sR) : 0) <= (RES ? LDS_MAX : LDS_MAX / 2), "LDS");
+  static_assert(NST * (STAGE_X + STAGE_W) + (int)sizeof(sR) <= LDS_MAX - 512, "LDS");
   const int tid = threadIdx.x;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l = tid & 63, n = l & 15, g = l >> 4;
@@ -163,23 +165,33 @@ __global__ __launch_bounds__(64 * NW, RES ? 1 : 2) void small_proj_kernel(const 
   const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void*)wt, 0, 0x7fffffff, 0x00020000);
   const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((void*)(x + (long)row0 * xs), 0, 0x7fffffff, 0x00020000);
   const unsigned vw = (unsigned)(8 * w + lr) * (unsigned)(K * 2) + 16u * (unsigned)chunk;
-  static_assert(RES || ROWS == 32, "one load of x per wavefront and stage");
   const unsigned vx = (unsigned)min(8 * w + lr, rows - 1 - row0) * (unsigned)xs + 16u * (unsigned)chunk;
-  constexpr int LOADS = RES ? 4 : 5;  // per wavefront and stage
+  const unsigned vx2 = (unsigned)min(8 * w + lr + 32, rows - 1 - row0) * (unsigned)xs + 16u * (unsigned)chunk;
+  constexpr int LOADS = RES ? 4 : 4 + ROWS / 32;  // per wavefront and stage
+  // Streaming workgroups walk K from different places (three stages on per workgroup of an XCD): in step, all of them would be at the
+  // same bytes of rows that are a multiple of the caches' interleave apart, i.e. on one or two channels, and behind the same
+  // misses.  100 to 400 rows, 16 heads, K = 6144: 47 to 49 us in step, 28 to 29 so.
+  const int first = RES ? 0 : (int)((3u * (blockIdx.x >> 3)) % (unsigned)steps);
   auto load = [&](int step, unsigned char* W, unsigned char* X) __attribute__((always_inline)) {
     if (step >= steps) return;
+    step += first;
+    if (!RES && step >= steps) step -= steps;
 #pragma unroll
     for (int j = 0; j < 4; ++j)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, LDS_PTR(void, W + (w + 4 * j) * 1024), 16, vw,
                                                (int)((unsigned)step * (BK * 2) + (unsigned)(32 * j) * (unsigned)(K * 2)), 0, 0);
-    if constexpr (!RES)
+    if constexpr (!RES) {
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, LDS_PTR(void, X + w * 1024), 16, vx, (int)((unsigned)step * (BK * 2)), 0, 0);
+      if constexpr (ROWS == 64)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, LDS_PTR(void, X + (w + 4) * 1024), 16, vx2, (int)((unsigned)step * (BK * 2)), 0, 0);
+    }
   };
   RowParams<ROWS / 32> params;
   load_row_params(a, params, text, head, row0, rows, tid);
   load(0, sW0, sX0);
   load(1, sW1, sX1);
   if constexpr (NST > 3) load(2, sW2, sX2);
+  if constexpr (!RES) load(3, sW3, sX3);
 
   // ---- RES: the workgroup's rows, their statistics and norm, eight lanes a row ----
   const int x_row = resident_row(K);
@@ -256,43 +268,87 @@ __global__ __launch_bounds__(64 * NW, RES ? 1 : 2) void small_proj_kernel(const 
   for (int fb = 0; fb < 2; ++fb)
 #pragma unroll
     for (int tb = 0; tb < TB; ++tb) acc[fb][tb] = f32x4{0.f, 0.f, 0.f, 0.f};
-  auto step = [&](int s, const unsigned char* W, const unsigned char* X, unsigned char* Wn, unsigned char* Xn) __attribute__((always_inline)) {
-    if (s >= steps) return;
-    // (the loads of the stages behind this one may be outstanding; RES: the barrier also publishes the rows)
-    const int behind = steps - 1 - s;
-    if (behind >= NST - 2)
-      wait_vmcnt<LOADS * (NST - 2)>();
-    else if (NST > 3 && behind == 1)
-      wait_vmcnt<LOADS>();
-    else
-      wait_vmcnt<0>();
-    __syncthreads();
-    load(s + NST - 1, Wn, Xn);
+  struct Operands {
+    bf16x8 w[2][2], x[2][TB];
+  };
+  auto read = [&](Operands& o, int s, const unsigned char* W, const unsigned char* X) __attribute__((always_inline)) {
 #pragma unroll
     for (int kk = 0; kk < 2; ++kk) {
-      bf16x8 wf[2], xf[TB];
 #pragma unroll
-      for (int fb = 0; fb < 2; ++fb) wf[fb] = *LDS_PTR(const bf16x8, W + ((base_w + ((64 * kk) ^ sh)) + fb * 16 * (BK * 2)));
+      for (int fb = 0; fb < 2; ++fb) o.w[kk][fb] = *LDS_PTR(const bf16x8, W + ((base_w + ((64 * kk) ^ sh)) + fb * 16 * (BK * 2)));
 #pragma unroll
       for (int tb = 0; tb < TB; ++tb)
-        xf[tb] = RES ? *LDS_PTR(const bf16x8, sR + (base_x + tb * 16 * x_row + s * (BK * 2) + 64 * kk))
-                     : *LDS_PTR(const bf16x8, X + ((base_x + ((64 * kk) ^ sh)) + tb * 16 * (BK * 2)));
+        o.x[kk][tb] = RES ? *LDS_PTR(const bf16x8, sR + (base_x + tb * 16 * x_row + s * (BK * 2) + 64 * kk))
+                          : *LDS_PTR(const bf16x8, X + ((base_x + ((64 * kk) ^ sh)) + tb * 16 * (BK * 2)));
+    }
+  };
+  auto multiply = [&](const Operands& o) __attribute__((always_inline)) {
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
       for (int fb = 0; fb < 2; ++fb)
 #pragma unroll
-        for (int tb = 0; tb < TB; ++tb) acc[fb][tb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[fb], xf[tb], acc[fb][tb], 0, 0, 0);
-    }
+        for (int tb = 0; tb < TB; ++tb)
+          acc[fb][tb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(o.w[kk][fb], o.x[kk][tb], acc[fb][tb], 0, 0, 0);
   };
-  for (int s = 0; s < steps; s += NST) {
-    if constexpr (NST == 4) {
-      step(s, sW0, sX0, sW3, sX3);
-      step(s + 1, sW1, sX1, sW0, sX0);
-      step(s + 2, sW2, sX2, sW1, sX1);
-      step(s + 3, sW3, sX3, sW2, sX2);
-    } else {
-      step(s, sW0, sX0, sW2, sX2);
-      step(s + 1, sW1, sX1, sW0, sX0);
-      step(s + 2, sW2, sX2, sW1, sX1);
+  if constexpr (RES) {
+    auto step = [&](int s, const unsigned char* W, unsigned char* Wn) __attribute__((always_inline)) {
+      if (s >= steps) return;
+      // (the loads of the stages behind this one may be outstanding; the barrier also publishes the rows)
+      const int behind = steps - 1 - s;
+      if (behind >= NST - 2)
+        wait_vmcnt<LOADS * (NST - 2)>();
+      else if (NST > 3 && behind == 1)
+        wait_vmcnt<LOADS>();
+      else
+        wait_vmcnt<0>();
+      barrier_loads_in_flight();
+      load(s + NST - 1, Wn, nullptr);
+      Operands o;
+      read(o, s, W, nullptr);
+      __builtin_amdgcn_sched_barrier(0);  // (all reads of a stage ahead of its products: their latency once; 1.5 % of a layer of 768 rows)
+      multiply(o);
+    };
+    for (int s = 0; s < steps; s += NST) {
+      if constexpr (NST == 4) {
+        step(s, sW0, sW3);
+        step(s + 1, sW1, sW0);
+        step(s + 2, sW2, sW1);
+        step(s + 3, sW3, sW2);
+      } else {
+        step(s, sW0, sW2);
+        step(s + 1, sW1, sW0);
+        step(s + 2, sW2, sW1);
+      }
+    }
+  } else {
+    // Two stages per barrier, the four behind them on the way (their bytes arrive at 130 GB/s per CU, what the direct path holds).  A
+    // last stage without a partner is multiplied by itself.
+    auto pair = [&](int s, const unsigned char* Wa, const unsigned char* Xa, const unsigned char* Wb, const unsigned char* Xb, unsigned char* Wan,
+                    unsigned char* Xan, unsigned char* Wbn, unsigned char* Xbn) __attribute__((always_inline)) {
+      if (s >= steps) return;
+      const int behind = steps - 2 - s;
+      if (behind >= 2)
+        wait_vmcnt<LOADS * 2>();
+      else if (behind == 1)
+        wait_vmcnt<LOADS>();
+      else
+        wait_vmcnt<0>();
+      barrier_loads_in_flight();
+      load(s + 4, Wan, Xan);
+      load(s + 5, Wbn, Xbn);
+      Operands o;
+      read(o, s, Wa, Xa);
+      multiply(o);
+      if (s + 1 < steps) {
+        read(o, s + 1, Wb, Xb);
+        multiply(o);
+      }
+    };
+    for (int s = 0; s < steps; s += 6) {
+      pair(s, sW0, sX0, sW1, sX1, sW4, sX4, sW5, sX5);
+      pair(s + 2, sW2, sX2, sW3, sX3, sW0, sX0, sW1, sX1);
+      pair(s + 4, sW4, sX4, sW5, sX5, sW2, sX2, sW3, sX3);
     }
   }
   // 32 rows at a time through LDS: 512 bytes a row, its 16-byte chunk c at c ^ (row % 16)
@@ -318,10 +374,12 @@ hipError_t launch_small_proj(const SmallProjKernArgs& a_in, int compute_units, h
   auto blocks = [&](int rows) { return ((a.S + rows - 1) / rows) * heads + ((a.T + rows - 1) / rows) * 2 * a.Hkv; };
   if (blocks(32) == 0) return hipSuccess;
   const int K = (a.S > 0 && a.K > a.Kt) || a.T == 0 ? a.K : a.Kt;  // the longer rows
-  const bool res = K <= res_max_k<32>(), tall = K <= res_max_k<64>() && blocks(32) > compute_units;
+  const bool res = K <= res_max_k<32>(), tall = (!res || K <= res_max_k<64>()) && blocks(32) > compute_units;
   a.hidden_blocks = (tall ? (a.S + 63) / 64 : (a.S + 31) / 32) * heads;
   const dim3 grid((unsigned)blocks(tall ? 64 : 32)), threads(64 * NW);
-  if (!res)
+  if (!res && tall)
+    hipLaunchKernelGGL((small_proj_kernel<false, 64>), grid, threads, 0, stream, a);
+  else if (!res)
     hipLaunchKernelGGL((small_proj_kernel<false, 32>), grid, threads, 0, stream, a);
   else if (tall)
     hipLaunchKernelGGL((small_proj_kernel<true, 64>), grid, threads, 0, stream, a);

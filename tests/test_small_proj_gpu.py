@@ -49,7 +49,8 @@ def _rotate(x, rope, batch, R2):
     (1, 64, 1, 64, 2, 1, 1, 1, "bf16", True, 48), (31, 128, 33, 192, 6, 2, 1, 0, "fp32", True, 48), (33, 192, 65, 64, 3, 3, 3, 20, "bf16", False, 48),
     (64, 256, 31, 320, 6, 2, 2, 64, None, True, 32), (240, 768, 24, 768, 6, 2, 1, 120, "bf16", True, 48), (97, 1024, 40, 1024, 4, 2, 1, 97, "bf16", True, 0),
     (1313, 256, 129, 256, 6, 2, 1, 700, "bf16", True, 48), (700, 768, 63, 704, 6, 2, 1, 699, "fp32", False, 48), (1281, 64, 0, 0, 6, 2, 1, 1281, "bf16", True, 64),
-    (65, 1088, 33, 3072, 2, 2, 1, 1, None, True, 48), (0, 0, 402, 3072, 0, 8, 1, 0, None, True, 0), (0, 0, 1, 1088, 0, 1, 1, 0, None, False, 0)])
+    (65, 1088, 33, 3072, 2, 2, 1, 1, None, True, 48), (0, 0, 402, 3072, 0, 8, 1, 0, None, True, 0), (0, 0, 1, 1088, 0, 1, 1, 0, None, False, 0),
+    (0, 0, 97, 1152, 0, 40, 1, 0, None, True, 0), (150, 1088, 0, 0, 26, 3, 1, 150, None, True, 48), (0, 0, 800, 3072, 0, 8, 1, 0, None, True, 0)])
 def test_small_projections_against_float64(dev, S, K, T, Kt, Hq, Hkv, batch, kept, ln, beta, R2):
     g = torch.Generator(device=dev).manual_seed(S + T + K)
     rnd = lambda *s: torch.randn(*s, device=dev, generator=g)  # noqa: E731
