@@ -239,9 +239,9 @@ def _text_in_one_launch(flop: float, rows: int, heads: int, K: int, cus: int) ->
     norm against this launch (K = 3072, 16 heads): 20 rows 10.5 / 15.3 us, 100 rows 12.2 / 15.4, 200 rows 16.0 / 15.6, 400 rows
     18.3 / 16.3, 800 rows 23.7 / 21.9; K = 768, 4 heads: 1500 rows 10.4 / 10.7.  The host takes 8.5 instead of 29 us, which counts where
     the layer is waiting for it: whole layers of 24 heads, 468 rows over 2340 keys (3.1e10 flop) 163 / 145 us, 840 over 3360 (6.6e10)
-    167 / 160, but 924 over 4620 in fp8 (8.7e10) 191 / 198; beyond that only from 200 rows on: layers of 24 heads, two
-    chunks of 648 rows with 200 text rows each 192 / 189 us, 1710 rows over 13680 keys with 402 372 / 369, 2550 over 10200 with 60 439 / 445.  At K = 6144 the product is the
-    faster one (400 rows 25 / 29 us)."""
+    167 / 160, but 924 over 4620 in fp8 (8.7e10) 191 / 198; beyond that only from 200 text rows on: layers of 24 heads, two chunks of
+    648 rows with 200 text rows each 192 / 189 us, 1710 rows over 13680 keys with 402 372 / 369, 2550 over 10200 with 60 439 / 445.
+    At K = 6144 the product is the faster one (400 rows 25 / 29 us)."""
     tile = 64 if K > 1024 else 32
     return (flop < 7e10 or rows >= 200) and K <= 3072 and (rows + tile - 1) // tile * heads <= cus
 
