@@ -234,8 +234,7 @@ def test_which_layers_take_the_one_launch():
     assert one(240, 20, 48, 4, 768, cus) and one(2048, 20, 1600, 4, 768, cus) and not one(3265, 20, 40, 4, 768, cus)
     assert one(380, 20, 100, 4, 1024, cus) and not one(400, 20, 100, 4, 1024, cus)  # (no taller workgroups there: one round)
     text = MOD._text_in_one_launch
-    assert text(6e10, 1024, 16, 3072, cus) and not text(6e10, 1025, 16, 3072, cus) and text(6e10, 2048, 4, 768, cus)
-    assert text(6e10, 512, 16, 1024, cus) and not text(6e10, 513, 16, 1024, cus)  # (32 rows a workgroup there)
+    assert text(6e10, 512, 16, 3072, cus) and not text(6e10, 513, 16, 3072, cus) and text(6e10, 2048, 4, 768, cus)
     assert not text(6e10, 100, 16, 6144, cus) and not text(8e10, 199, 16, 3072, cus) and text(8e10, 200, 16, 3072, cus)
 
 
