@@ -235,9 +235,9 @@ def _projects_in_one_launch(rows: int, heads: int, text_rows: int, text_heads: i
 
 def _text_in_one_launch(flop: float, rows: int, heads: int, K: int, cus: int) -> bool:
     """Whether the K | V projection of the text rows and the K norm run as one launch of small_projections rather than as the library's
-    product and a head norm.  In one round of its workgroups (32 rows x one of the `heads`), product and norm against this launch (K = 3072, 16 heads): 20 rows 10.5 / 15.3 us, 100 rows 12.2 / 15.4, 200 rows 16.0 / 15.6, 400 rows
-    18.3 / 16.3; K = 768, 4 heads: 1500 rows 10.4 / 10.7.  The host takes 8.5 instead of 29 us, which counts where
-    the layer is waiting for it: whole layers of 24 heads, 468 rows over 2340 keys (3.1e10 flop) 163 / 145 us, 840 over 3360 (6.6e10)
+    product and a head norm.  In one round of its workgroups (32 rows x one of the `heads`), product and norm against this
+    launch (K = 3072, 16 heads): 20 rows 10.5 / 15.3 us, 100 rows 12.2 / 15.4, 200 rows 16.0 / 15.6, 400 rows 18.3 / 16.3; K = 768, 4 heads:
+    1500 rows 10.4 / 10.7.  The host takes 8.5 instead of 29 us, which counts where the layer is waiting for it: whole layers of 24 heads, 468 rows over 2340 keys (3.1e10 flop) 163 / 145 us, 840 over 3360 (6.6e10)
     167 / 160, but 924 over 4620 in fp8 (8.7e10) 191 / 198; beyond that only from 200 text rows on: layers of 24 heads, two chunks of
     648 rows with 200 text rows each 192 / 189 us, 1710 rows over 13680 keys with 402 372 / 369, 2550 over 10200 with 60 439 / 445.
     More rows (64 a workgroup then) gain nothing once the weights come from memory: four chunks of 1170 rows with 674 in all 374 / 376.  At K = 6144 the
