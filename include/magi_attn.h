@@ -357,6 +357,7 @@ int magi_qkv_proj_prologue(const magi_qkv_proj_args* args, void* stream);
  * Text rows (T > 0): text [T, Kt] bf16 -> columns [kv head][K | V] of w_text [2 Hkv 128, Kt] -> text_out [T, Hkv, 256], the K
  * halves normed with gkx / bkx (LayerNorm-1p, eps).
  * K and Kt: multiples of 64, with ln_w at most 1024.  Strides in elements, rows 16-byte aligned.
+ * A row's result depends on that row and the weights alone, bit for bit: the products are fp32 sums over K from first to last.
  */
 typedef struct magi_small_proj_args {
   uint32_t struct_size; /* sizeof(magi_small_proj_args) */

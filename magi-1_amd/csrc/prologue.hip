@@ -122,14 +122,7 @@ __global__ __launch_bounds__(THREADS) void prologue_kernel(const PrologueKernArg
       unpack8(va, x);
       unpack8(vb, x + 8);
       norm16(x, s_par[2 * kind], s_par[2 * kind + 1], ea, eb, a.norm_kind, a.eps, true);
-      if (rot_lane && a.rope) {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          const float x1 = x[i], x2 = x[8 + i];
-          x[i] = x1 * cs[i] - x2 * sn[i];
-          x[8 + i] = x1 * sn[i] + x2 * cs[i];
-        }
-      }
+      if (rot_lane && a.rope) rotate8(x, [&](int i) { return sn[i]; }, [&](int i) { return cs[i]; });
       if (kind == 0 && a.q_premul != 1.f) {  // e.g. softmax_scale * log2(e), ahead of the one rounding to bf16
 #pragma unroll
         for (int i = 0; i < 16; ++i) x[i] *= a.q_premul;

@@ -60,28 +60,45 @@ __device__ __forceinline__ float wave_sum(float x) {
   return x;
 }
 
-// Normalise the 16 values of this lane (8 lanes = one row of 128) in place.
-__device__ __forceinline__ void norm16(float* x, const float* gam, const float* bet, int ea, int eb, int kind, float eps,
-                                       bool has_beta) {
+// Normalise the 16 values of this lane (8 lanes = one row of 128) in place; gam(i), bet(i): the parameters of its value i.  The
+// roundings are spelled out (no contraction that the compiler is free to choose), so that every kernel that norms heads gives
+// the same bits.
+template <class G, class B>
+__device__ __forceinline__ void norm16_by(float* x, G gam, B bet, int kind, float eps, bool has_beta) {
+#pragma clang fp contract(off)
   if (kind == 2) return;
   float s = 0.f;
 #pragma unroll
   for (int i = 0; i < 16; ++i) s += x[i];
   float mean = 0.f;
   if (kind == 0) mean = group8_sum(s) * (1.f / D);
-  float q = 0.f;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) x[i] -= mean;
+  float q = __builtin_fmaf(x[0], x[0], x[1] * x[1]);
+#pragma unroll
+  for (int i = 2; i < 16; ++i) q = __builtin_fmaf(x[i], x[i], q);
+  const float rstd = __builtin_amdgcn_rsqf(__builtin_fmaf(group8_sum(q), 1.f / D, eps));
 #pragma unroll
   for (int i = 0; i < 16; ++i) {
-    const float d = x[i] - mean;
-    q += d * d;
-  }
-  const float rstd = __builtin_amdgcn_rsqf(group8_sum(q) * (1.f / D) + eps);
-#pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const int e = (i < 8) ? ea + i : eb + (i - 8);
-    float y = (x[i] - mean) * rstd * (gam[e] + 1.f);
-    if (kind == 0 && has_beta) y += bet[e];
+    float y = x[i] * rstd * (gam(i) + 1.f);
+    if (kind == 0 && has_beta) y += bet(i);
     x[i] = y;
+  }
+}
+__device__ __forceinline__ void norm16(float* x, const float* gam, const float* bet, int ea, int eb, int kind, float eps,
+                                       bool has_beta) {
+  auto at = [&](int i) { return i < 8 ? ea + i : eb + (i - 8); };
+  norm16_by(x, [&](int i) { return gam[at(i)]; }, [&](int i) { return bet[at(i)]; }, kind, eps, has_beta);
+}
+// Rotate the eight pairs (x[i], x[8 + i]), with the roundings spelled out as above
+template <class S, class C>
+__device__ __forceinline__ void rotate8(float* x, S sn, C cs) {
+#pragma clang fp contract(off)
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const float x1 = x[i], x2 = x[8 + i];
+    x[i] = __builtin_fmaf(x1, cs(i), -(x2 * sn(i)));
+    x[8 + i] = __builtin_fmaf(x1, sn(i), x2 * cs(i));
   }
 }
 

@@ -1,7 +1,10 @@
 // The projections of a small layer with everything around them, in one launch, for gfx950: LayerNorm of the layer input,
 // q | k | v | qx projections, per-head norm, rotary, cast, KV-cache append; and for the text tokens the K | V projection with
-// the K norm.  Every rounding to bf16 that the separate launches make is made here too (the normalised input, the raw
-// projections, the results), sums are in fp32.
+// the K norm.  Every rounding that the separate launches make is made here too, in fp32 and to bf16 (the normalised input, the raw
+// projections, the results): norms and rotary in their arithmetic and order of sums, the products as one fp32 sum over K from its
+// first element to its last, 32 at a time, whatever the row's place.  That is the library's order as well wherever it does not cut
+// K in pieces: the same bits for 32 rows and more at K up to 1024, for more than 2^17 results above (700 drawn shapes; with fewer
+// rows one result of some thousand is the neighbouring bf16).
 //
 // What bounds it: latency.  Below about a thousand rows the library's GEMM, the norm ahead of it and the prologue behind it
 // each live for little more than a launch and a few trips to memory, and a library call costs the host 18 us to issue.
@@ -12,8 +15,10 @@
 // for 400 text tokens at K = 3072, 16 so).  The product is formed transposed, W X^T on
 // v_mfma_f32_16x16x32_bf16 with the weight rows as the A operand: register r of lane (n, g) of a result block is column 4 g + r
 // of the block, row n; it goes through LDS to eight lanes per row, which do with it what the prologue does.
-// RES: the workgroup's rows are in LDS whole (K up to 1024), normalised ahead of the product; their statistics are merged from
-// pieces of eight elements, which is as exact as two passes.  Otherwise the rows, not to be normalised, stream beside the weights.
+// RES: the workgroup's rows are in LDS whole (K up to 1024), normalised ahead of the product.  Otherwise the rows, not to be
+// normalised, stream beside the weights.  (Streaming workgroups that start at different places of K, so that they are not all at
+// the same bytes of rows a multiple of the caches' interleave apart: 300 rows x 16 heads at K = 3072 out of memory 21.7 / 17.8 us,
+// but then the order of a row's sums depends on its place among the rows.)
 #include "attn_common.h"
 #include "row_ops.h"
 
@@ -98,35 +103,73 @@ __device__ __forceinline__ void store_rows32(const SmallProjKernArgs& a, const R
   } else {
     dst = a.qx_out + ((long)s * a.Hqx + (head - a.Hq - 2 * a.Hkv)) * (D * 2);
   }
-  if (p.normed) {  // (as norm16)
-    float sum = 0.f, sq = 0.f;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) sum += v[i];
-    const float mean = group8_sum(sum) * (1.f / D);
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const float d = v[i] - mean;
-      sq += d * d;
-    }
-    const float rstd = __builtin_amdgcn_rsqf(group8_sum(sq) * (1.f / D) + a.eps);
-#pragma unroll
-    for (int i = 0; i < 16; ++i) v[i] = (v[i] - mean) * rstd * (p.gam[i >> 2][i & 3] + 1.f) + p.bet[i >> 2][i & 3];
-  }
-  if (p.rot) {
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const float sn = p.sin_cos[half][i >> 2][i & 3], cs = p.sin_cos[half][2 + (i >> 2)][i & 3];
-      const float x1 = v[i], x2 = v[8 + i];
-      v[i] = x1 * cs - x2 * sn;
-      v[8 + i] = x1 * sn + x2 * cs;
-    }
-  }
+  // (the arithmetic of the prologue and, for the text, of the head norm: the bits of the separate launches)
+  if (p.normed) norm16_by(v, [&](int i) { return p.gam[i >> 2][i & 3]; }, [&](int i) { return p.bet[i >> 2][i & 3]; }, 0, a.eps, !text || a.bkx);
+  if (p.rot)
+    rotate8(v, [&](int i) { return p.sin_cos[half][i >> 2][i & 3]; }, [&](int i) { return p.sin_cos[half][2 + (i >> 2)][i & 3]; });
   if (mul != 1.f) {
 #pragma unroll
     for (int i = 0; i < 16; ++i) v[i] *= mul;
   }
   *(u32x4*)(dst + p.ea * 2) = pack8(v);
   *(u32x4*)(dst + p.eb * 2) = pack8(v + 8);
+}
+
+// x of the lane whose number differs in bit M (1, 2 or 4)
+template <int M>
+__device__ __forceinline__ float lane_xor(float x) {
+  int v = __builtin_bit_cast(int, x);
+  if constexpr (M == 4) v = __builtin_amdgcn_mov_dpp(v, 0x141, 0xf, 0xf, true);  // row_half_mirror: lane ^ 7
+  constexpr int QUAD = M == 1 ? 0xb1 : M == 2 ? 0x4e : 0x1b;                     // quad_perm: lane ^ 1, ^ 2, ^ 3
+  return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(v, QUAD, 0xf, 0xf, true));
+}
+// The sum over a wavefront's 64 lanes of wave_sum, for eight lanes that stand for them: x[p] of lane j is lane 8 p + j's.  Same pairs in
+// the same order, so the same bits: the lanes' bits 1, 2, 4 first (each step a lane hands on the half of the sums that it does not
+// keep, and lane j is left with that of p = j), then the bits of p.
+__device__ __forceinline__ float wave_sum8(const float (&x)[8], int j) {
+  float y[4], z[2];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) y[i] = (j & 1 ? x[2 * i + 1] : x[2 * i]) + lane_xor<1>(j & 1 ? x[2 * i] : x[2 * i + 1]);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) z[i] = (j & 2 ? y[2 * i + 1] : y[2 * i]) + lane_xor<2>(j & 2 ? y[2 * i] : y[2 * i + 1]);
+  float s = (j & 4 ? z[1] : z[0]) + lane_xor<4>(j & 4 ? z[0] : z[1]);
+  s += lane_xor<1>(s);
+  s += lane_xor<2>(s);
+  return s + lane_xor<4>(s);
+}
+// Mean and reciprocal standard deviation of a row that eight lanes hold packed, pieces j, j + 8, ... of eight elements in lane j's raw
+// (nv of them), as row_stats of the layer norm's kernel forms them: its wavefront has piece 64 i + l in lane l, so lane j here
+// stands for lanes j, j + 8, ... j + 56 with up to two pieces each.
+template <int NV>
+__device__ __forceinline__ void row_stats8(const u32x4 (&raw)[NV], int j, int nv, float inv_n, float eps, float& mean, float& rstd) {
+#pragma clang fp contract(off)
+  static_assert(NV <= 16, "two pieces per lane of a wavefront");
+  float part[8];
+#pragma unroll
+  for (int p = 0; p < 8; ++p) part[p] = 0.f;
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {  // (zeros past the end)
+    float f[8];
+    unpack8(raw[i], f);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) part[i & 7] += f[e];
+  }
+  mean = wave_sum8(part, j) * inv_n;
+#pragma unroll
+  for (int p = 0; p < 8; ++p) part[p] = 0.f;
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    if (i >= nv) continue;
+    float f[8];
+    unpack8(raw[i], f);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) f[e] -= mean;
+    float q = i < 8 ? __builtin_fmaf(f[0], f[0], f[1] * f[1]) : __builtin_fmaf(f[1], f[1], __builtin_fmaf(f[0], f[0], part[i & 7]));
+#pragma unroll
+    for (int e = 2; e < 8; ++e) q = __builtin_fmaf(f[e], f[e], q);
+    part[i & 7] = q;
+  }
+  rstd = __builtin_amdgcn_rsqf(__builtin_fmaf(inv_n, wave_sum8(part, j), eps));
 }
 
 // RES: the rows whole in LDS ahead of the product, normalised on the way there; else they stream beside the weights, as they are
@@ -168,14 +211,8 @@ __global__ __launch_bounds__(64 * NW, 1) void small_proj_kernel(const SmallProjK
   const unsigned vx = (unsigned)min(8 * w + lr, rows - 1 - row0) * (unsigned)xs + 16u * (unsigned)chunk;
   const unsigned vx2 = (unsigned)min(8 * w + lr + 32, rows - 1 - row0) * (unsigned)xs + 16u * (unsigned)chunk;
   constexpr int LOADS = RES ? 4 : 4 + ROWS / 32;  // per wavefront and stage
-  // Streaming workgroups walk K from different places (three stages on per workgroup of an XCD): in step, all of them would be at the
-  // same bytes of rows that are a multiple of the caches' interleave apart, i.e. on one or two channels, and behind the same
-  // misses.  100 to 400 rows, 16 heads, K = 6144: 47 to 49 us in step, 28 to 29 so.
-  const int first = RES ? 0 : (int)((3u * (blockIdx.x >> 3)) % (unsigned)steps);
   auto load = [&](int step, unsigned char* W, unsigned char* X) __attribute__((always_inline)) {
     if (step >= steps) return;
-    step += first;
-    if (!RES && step >= steps) step -= steps;
 #pragma unroll
     for (int j = 0; j < 4; ++j)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, LDS_PTR(void, W + (w + 4 * j) * 1024), 16, vw,
@@ -213,30 +250,8 @@ __global__ __launch_bounds__(64 * NW, 1) void small_proj_kernel(const SmallProjK
         lnb[i] = i < nv ? *(const u32x4*)(a.ln_b + (8 * i + j) * 16) : u32x4{0u, 0u, 0u, 0u};
       }
     }
-    float mean = 0.f, m2 = 0.f;
-#pragma unroll
-    for (int i = 0; i < NV; ++i) {
-      if (i >= nv) continue;
-      float f[8], s = 0.f, q = 0.f;
-      unpack8(raw[i], f);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) s += f[e];
-      s *= 0.125f;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) q += (f[e] - s) * (f[e] - s);
-      const float d = s - mean, share = 1.f / (float)(i + 1);  // 8 i elements so far, 8 more
-      m2 += q + d * d * (8.f * (float)i * share);
-      mean += d * share;
-    }
-    float cnt = 8.f * (float)nv;  // per lane; all lanes of a row hold as many
-#pragma unroll
-    for (int m = 1; m < 8; m <<= 1) {
-      const float mo = __shfl_xor(mean, m), d = mo - mean;
-      m2 += __shfl_xor(m2, m) + d * d * (0.5f * cnt);
-      mean = 0.5f * (mean + mo);
-      cnt *= 2.f;
-    }
-    const float rstd = __builtin_amdgcn_rsqf(m2 / (float)K + a.ln_eps);
+    float mean = 0.f, rstd = 1.f;
+    if (ln) row_stats8<NV>(raw, j, nv, 1.f / (float)K, a.ln_eps, mean, rstd);
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
       if (i >= nv) continue;
@@ -254,7 +269,7 @@ __global__ __launch_bounds__(64 * NW, 1) void small_proj_kernel(const SmallProjK
         unpack8(lnb[i], bf);
       }
 #pragma unroll
-      for (int e = 0; e < 8; ++e) f[e] = (f[e] - mean) * rstd * wf[e] + bf[e];
+      for (int e = 0; e < 8; ++e) f[e] = __builtin_fmaf((f[e] - mean) * rstd, wf[e], bf[e]);
       *LDS_PTR(u32x4, sR + r * x_row + (8 * i + j) * 16) = pack8(f);
     }
    }

@@ -235,14 +235,16 @@ def _projects_in_one_launch(rows: int, heads: int, text_rows: int, text_heads: i
 
 def _text_in_one_launch(flop: float, rows: int, heads: int, K: int, cus: int) -> bool:
     """Whether the K | V projection of the text rows and the K norm run as one launch of small_projections rather than as the library's
-    product and a head norm.  In one round of its workgroups (32 rows x one of the `heads`), product and norm against this
-    launch (K = 3072, 16 heads): 20 rows 10.5 / 15.3 us, 100 rows 12.2 / 15.4, 200 rows 16.0 / 15.6, 400 rows 18.3 / 16.3; K = 768, 4 heads:
-    1500 rows 10.4 / 10.7.  The host takes 8.5 instead of 29 us, which counts where the layer is waiting for it: whole layers of 24 heads, 468 rows over 2340 keys (3.1e10 flop) 163 / 145 us, 840 over 3360 (6.6e10)
-    167 / 160, but 924 over 4620 in fp8 (8.7e10) 191 / 198; beyond that only from 200 text rows on: layers of 24 heads, two chunks of
-    648 rows with 200 text rows each 192 / 189 us, 1710 rows over 13680 keys with 402 372 / 369, 2550 over 10200 with 60 439 / 445.
-    More rows (64 a workgroup then) gain nothing once the weights come from memory: four chunks of 1170 rows with 674 in all 374 / 376.  At K = 6144 the
-    product is the faster one (400 rows 25 / 29 us)."""
-    return (flop < 7e10 or rows >= 200) and K <= 3072 and (rows + 31) // 32 * heads <= cus
+    product and a head norm.  The host takes 8.5 instead of 29 us for it, which counts where the layer is waiting for it; on the device
+    (K = 3072, 16 heads, weights out of memory, norm and product / this launch) 100 rows take 14.7 / 20.5 us, 200 rows 19.9 / 21.1, 300
+    rows 21.1 / 21.8, 512 rows 21.3 / 23.3.  Whole layers of 24 heads: 468 rows over 2340 keys (3.1e10 flop) 151 / 132 us, two chunks of 648 rows
+    with 348 text rows (9e10) 162 / 160, 900 rows over 4500 keys in fp8 with 300 (8.4e10) 268 / 247; from 7e10 on with fewer than 200 text rows
+    924 over 4620 in fp8 191 / 198; 1710 rows over 13680 keys with 302 356 / 356.  In one round of its workgroups (32 rows x one of the
+    `heads`): more rows (64 a workgroup then) gain nothing, four chunks of 1170 rows with 674 in all 374 / 376.  At K = 6144 the
+    product is the faster one (400 rows 25 / 29 us).
+    Up to 2^17 results of a long sum the library cuts K in pieces (64 rows at 16 heads, 128 at 8): another order of the sums, other bits.
+    Those layers keep the library's."""
+    return (flop < 7e10 or rows >= 200) and K <= 3072 and (K <= 1024 or rows * heads > 1024) and (rows + 31) // 32 * heads <= cus
 
 
 def _global_hooks() -> bool:

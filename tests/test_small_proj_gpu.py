@@ -168,6 +168,41 @@ def test_small_layer_gives_what_the_separate_launches_give(dev, monkeypatch, hid
         assert a.shape == b.shape and float(x @ y / (x.norm() * y.norm())) >= 0.9999 and float((x - y).abs().max()) <= 2e-2 * max(1.0, float(y.abs().max()))
 
 
+# K: one piece for a part of the norm's 64 lanes, for all of them, two pieces; 32 and 64 rows a workgroup; rows that stream
+@pytest.mark.gpu
+@pytest.mark.parametrize("S,K,T,Kt,Hq,Hkv,ln,beta", [
+    (32, 64, 32, 128, 2, 1, "bf16", True), (97, 448, 40, 512, 6, 2, "fp32", True), (240, 768, 45, 768, 6, 2, "bf16", True), (96, 1024, 33, 1024, 4, 4, "bf16", False),
+    (1344, 768, 131, 768, 6, 2, "fp32", False), (0, 0, 65, 3072, 0, 8, None, True), (0, 0, 300, 3072, 0, 8, None, False), (0, 0, 800, 1088, 0, 8, None, True)])
+def test_bits_are_those_of_the_separate_launches(dev, S, K, T, Kt, Hq, Hkv, ln, beta):
+    """Norm, projections, prologue and head norm one after the other give every bit of the one launch, at sizes where the library's
+    product does not cut K in pieces; and a row's bits do not depend on where it lies."""
+    g = torch.Generator(device=dev).manual_seed(S + T + K)
+    rnd = lambda *s: torch.randn(*s, device=dev, generator=g)  # noqa: E731
+    par = [rnd(D) * 0.2 for _ in range(6)]
+    if not beta:
+        par[1] = par[3] = par[5] = None
+    linear, kw, x, w, rope = torch.nn.functional.linear, {}, None, None, None
+    if S:
+        x, w = (rnd(S, K) * 2 + 0.5).bfloat16(), (rnd(2 * (Hq + Hkv) * D, K) * K ** -0.5).bfloat16()
+        dt = torch.float32 if ln == "fp32" else torch.bfloat16
+        kw["ln"] = ((1 + 0.1 * rnd(K)).to(dt), (0.1 * rnd(K)).to(dt), 1e-6)
+        angle = torch.rand(S, 48, device=dev, generator=g) * 60
+        rope = torch.cat([angle.sin(), angle.cos()], -1)
+    y, wt = rnd(T, Kt).bfloat16(), (rnd(2 * Hkv * D, Kt) * Kt ** -0.5).bfloat16()
+    one = lambda x, rope, y: M.small_projections(x, w, rope, *par[:4], Hq=Hq, Hkv=Hkv, Hqx=Hq, q_premul=0.1275,  # noqa: E731
+                                                 text=(y, wt, par[4], par[5]), **kw)
+    q, kv, _, qx, text_kv = one(x, rope, y)
+    if S:
+        rq, rk, rv, rx = linear(M.layer_norm(x, *kw["ln"]), w).split((Hq * D, Hkv * D, Hkv * D, Hq * D), -1)
+        want_q, want_kv, _ = M.qk_prologue(rq, rk, rv, rope, *par[:4], Hq=Hq, Hkv=Hkv, q_premul=0.1275)
+        assert torch.equal(qx.view(S, -1), rx) and torch.equal(kv, want_kv) and torch.equal(q, want_q)
+    raw = linear(y, wt).view(T, Hkv, 2 * D)
+    assert torch.equal(text_kv[..., D:], raw[..., D:]) and torch.equal(text_kv[..., :D], M.head_norm(raw[..., :D], par[4], par[5]))
+    turned = one(None if x is None else x.flip(0).contiguous(), None if rope is None else rope.flip(0).contiguous(), y.flip(0).contiguous())
+    for a, b in zip((q, kv, qx, text_kv), (turned[0], turned[1], turned[3], turned[4])):
+        assert a is None or torch.equal(a, b.flip(0))
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("ranges", ["a gap behind each", "one of three"])
 def test_rows_outside_the_ranges_of_a_small_layer_are_zeros(dev, ranges):
@@ -235,6 +270,7 @@ def test_which_layers_take_the_one_launch():
     assert one(380, 20, 100, 4, 1024, cus) and not one(400, 20, 100, 4, 1024, cus)  # (no taller workgroups there: one round)
     text = MOD._text_in_one_launch
     assert text(6e10, 512, 16, 3072, cus) and not text(6e10, 513, 16, 3072, cus) and text(6e10, 2048, 4, 768, cus)
+    assert text(6e10, 65, 16, 3072, cus) and not text(6e10, 64, 16, 3072, cus) and text(6e10, 3, 4, 1024, cus)  # (where the library cuts K)
     assert not text(6e10, 100, 16, 6144, cus) and not text(8e10, 199, 16, 3072, cus) and text(8e10, 200, 16, 3072, cus)
 
 
