@@ -201,10 +201,10 @@ def _linear_in_whole_rounds(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return torch.nn.functional.linear(x, w)
 
 
-def _plain_rows(x: torch.Tensor, w: torch.Tensor) -> bool:
-    """Whether x [rows, K] and the weight w [n, K] are as small_projections takes them: bf16 rows of the same device, aligned, of a
+def _plain_rows(x: torch.Tensor, w: torch.Tensor, heads: int) -> bool:
+    """Whether x [rows, K] and the weight w [heads * 128, K] are as small_projections takes them: bf16 rows of the same device, aligned, of a
     multiple of 64 elements, and no autocast that would have the library's product convert them."""
-    if x.dim() != 2 or x.dtype is not torch.bfloat16 or w.dtype is not torch.bfloat16 or torch.is_autocast_enabled():
+    if w.shape[0] != 128 * heads or x.dim() != 2 or x.dtype is not torch.bfloat16 or w.dtype is not torch.bfloat16 or torch.is_autocast_enabled():
         return False
     K = x.shape[1]
     if K % 64 or w.dim() != 2 or w.shape[1] != K or not w.is_contiguous() or x.shape[0] == 0 or not x.is_cuda or w.device != x.device:
@@ -835,7 +835,7 @@ class FullyParallelAttention(torch.nn.Module):
         text_kv = None
         if own_text:
             w = _param(m["linear_kv_xattn"], "weight")
-            if _plain_rows(key_value_states, w):
+            if _plain_rows(key_value_states, w, 2 * self.num_query_groups_per_partition):  # (others have as many heads as the weight)
                 gk, bk = m["k_layernorm_xattn"].gamma_beta_fp32()
                 text_kv = small_projections(None, None, None, None, None, None, None, Hq=0, Hkv=self.num_query_groups_per_partition,
                                             eps=self.eps, text=(key_value_states, w, gk, bk))[4]
@@ -899,7 +899,10 @@ class FullyParallelAttention(torch.nn.Module):
             return None
         w, wt, ln = lin.fused_weight(), _param(m["linear_kv_xattn"], "weight"), lin._modules["layer_norm"]
         lw, lb = _param(ln, "weight"), _param(ln, "bias")
-        if not (_plain_rows(hidden_states[:, 0], w) and _plain_rows(key_value_states, wt)) or lw is None or lb is None:
+        if not (_plain_rows(hidden_states[:, 0], w, 2 * (Hq + Hkv)) and _plain_rows(key_value_states, wt, 2 * Hkv)) or lw is None or lb is None:
+            return None
+        pq, pk = lin._projections()[:2]
+        if _param(pq, "weight").shape[0] != Hq * D or _param(pk, "weight").shape[0] != Hkv * D:
             return None
         if lw.dtype is not lb.dtype or lw.dtype not in (torch.bfloat16, torch.float32) or not (lw.is_contiguous() and lb.is_contiguous()) or (
                 lw.shape[0] != K or lb.shape[0] != K or (lw.data_ptr() | lb.data_ptr()) % 16 or lw.device != dev or key_value_states.device != dev):

@@ -263,6 +263,24 @@ def test_layers_that_the_one_launch_does_not_take(dev, monkeypatch, what):
             assert float((a.float() - b.float()).abs().max()) <= 2e-2 * max(1.0, float(b.abs().max()))
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads", [1, 4, 8])
+@pytest.mark.parametrize("small", [True, False])
+def test_text_weight_with_other_heads_than_the_layer(dev, monkeypatch, small, heads):
+    """The text has as many key heads as linear_kv_xattn's weight (the layer has two), in a small layer and where the text alone
+    would go in one launch."""
+    layer, run, _ = _layer_case(dev, 256, 1, 5, 9, 2, 1, "append", False, [33, 20])
+    layer.linear_kv_xattn = torch.nn.Linear(256, 2 * heads * D, bias=False, device=dev, dtype=torch.bfloat16)
+    if not small:
+        monkeypatch.setattr(MOD, "_projects_in_one_launch", lambda *a: False)
+    got, _ = run()
+    for name in ("_projects_in_one_launch", "_text_in_one_launch"):
+        monkeypatch.setattr(MOD, name, lambda *a: False)
+    want, _ = run()
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
+
+
 def test_which_layers_take_the_one_launch():
     cus = 256
     one = MOD._projects_in_one_launch
