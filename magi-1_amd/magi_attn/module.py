@@ -895,7 +895,7 @@ class FullyParallelAttention(torch.nn.Module):
         lin = m["linear_qkv"]
         if lin.__dict__.get("fp8_quant", True) or not hidden_states.is_contiguous() or rope.shape[-1] % 16 or rope.shape[-1] > D:
             return None
-        if not (_is_own(lin, _OWN_PROJECTIONS) and _is_own(self, _OWN_CROSS)):
+        if not (_is_own(lin, _OWN_SMALL_PROJECTIONS) and _is_own(self, _OWN_SMALL)):
             return None
         w, wt, ln = lin.fused_weight(), _param(m["linear_kv_xattn"], "weight"), lin._modules["layer_norm"]
         lw, lb = _param(ln, "weight"), _param(ln, "bias")
@@ -909,7 +909,11 @@ class FullyParallelAttention(torch.nn.Module):
             return None
         cache = tail = offloaded = None
         start = n_keep = persisted = 0
-        if inference_params is not None and (meta_args.extract_prefix_video_feature or meta_args.fwd_extra_1st_chunk or meta_args.slice_point > 0):
+        use_cache = inference_params is not None and (
+            meta_args.extract_prefix_video_feature or meta_args.fwd_extra_1st_chunk or meta_args.slice_point > 0)
+        if not use_cache and not _is_own(self, _OWN_CORE):
+            return None
+        if use_cache:
             if inference_params.max_batch_size != 1:
                 return None
             cache = self._cache(inference_params, hidden_states.dtype)
@@ -1056,10 +1060,11 @@ class FullyParallelAttention(torch.nn.Module):
             if bs > 1 and not own_cross:  # (a replaced cross attention runs; at batch 1 with a bound in force it never did)
                 return None
             flop = 512.0 * sq * Hq * (hidden_states.shape[2] + p.max_seqlen_k)
-            own_text = (bs == 1 and key_value_states.dim() == 2 and hidden_states.is_cuda and _text_in_one_launch(
+            own_text = (bs == 1 and key_value_states.dim() == 2 and hidden_states.is_cuda and _is_own(self, _OWN_SMALL) and _text_in_one_launch(
                 flop, key_value_states.shape[0], 2 * self.num_query_groups_per_partition, key_value_states.shape[1],
                 _compute_units(hidden_states.device)))
-            return self._cross_attention_fused(qx_raw, sq, bs, key_value_states, meta_args.cross_attn_params, dst, bound_cross, own_text)
+            more = {"own_text": True} if own_text else {}  # (one put in its place may not know it)
+            return self._cross_attention_fused(qx_raw, sq, bs, key_value_states, meta_args.cross_attn_params, dst, bound_cross, **more)
 
         get_xqkv = lambda m, y: self.get_xqkv(m, y, qx_raw=qx_raw.view(sq, bs, -1))
         p = meta_args.core_attn_params
@@ -1137,4 +1142,9 @@ _KERNEL_NAMES = ("online softmax, 32 rows per wavefront", "bounded-score, 64 row
 # the methods whose work forward() does in another shape, as long as they are these
 _OWN_FP8_LINEAR = {"forward": PerTensorQuantizedFp8Linear.forward}
 _OWN_PROJECTIONS = {"forward_ln": CustomLayerNormLinear.forward_ln, "forward_qkvx": CustomLayerNormLinear.forward_qkvx}
+_OWN_SMALL_PROJECTIONS = {**_OWN_PROJECTIONS, "forward_ln_qkvx_rows": CustomLayerNormLinear.forward_ln_qkvx_rows,
+                          "_split": CustomLayerNormLinear._split}
+_OWN_CORE = {"core_attention": FullyParallelAttention.core_attention}  # (called without a cache)
 _OWN_CROSS = {"get_xqkv": FullyParallelAttention.get_xqkv, "cross_attention": FullyParallelAttention.cross_attention}
+_OWN_SMALL = {**_OWN_CROSS, "_project_rows": FullyParallelAttention._project_rows, "_fused_qkv": FullyParallelAttention._fused_qkv,
+              "_cross_attention_fused": FullyParallelAttention._cross_attention_fused}

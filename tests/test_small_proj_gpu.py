@@ -264,6 +264,31 @@ def test_layers_that_the_one_launch_does_not_take(dev, monkeypatch, what):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("how", ["instance", "subclass"])
+@pytest.mark.parametrize("on,name", [("layer", "core_attention"), ("layer", "_fused_qkv"), ("layer", "_cross_attention_fused"),
+                                     ("layer", "_project_rows"), ("linear_qkv", "forward_ln_qkvx_rows"), ("linear_qkv", "forward_ln")])
+def test_replaced_methods_of_a_small_layer_are_called(dev, on, name, how):
+    """Whatever the separate launches call runs in small layers too where it is not the library's own; core_attention without a cache
+    only, as ever.  One put in its place may have the arguments of before the text's own launch."""
+    for cache in ("none", "append"):
+        layer, run, _ = _layer_case(dev, 256, 1, 5, 9, 2, 1, cache, False, [33, 20])
+        want, n_small = run()
+        m, calls = layer if on == "layer" else layer.linear_qkv, []
+        own = getattr(type(m), name)
+        new = lambda self, *a, **k: calls.append(k) or own(self, *a, **k)  # noqa: E731
+        if name == "_cross_attention_fused":
+            new = lambda self, qx, sq, b, kvs, p, dst, bound: calls.append(1) or own(self, qx, sq, b, kvs, p, dst, bound)  # noqa: E731
+        if how == "instance":
+            m.__dict__[name] = new.__get__(m)
+        else:
+            m.__class__ = type("Other", (type(m),), {name: new})
+        got, n = run()
+        assert bool(calls) == (name != "core_attention" or cache == "none")
+        assert (n > n_small) == bool(calls)
+        assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("heads", [1, 4, 8])
 @pytest.mark.parametrize("small", [True, False])
 def test_text_weight_with_other_heads_than_the_layer(dev, monkeypatch, small, heads):
