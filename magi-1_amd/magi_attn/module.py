@@ -925,7 +925,7 @@ class FullyParallelAttention(torch.nn.Module):
             start = meta_args.slice_point * meta_args.clip_token_nums
             if inference_params.update_kv_cache:
                 n_keep = S - meta_args.clip_token_nums if meta_args.distill_nearly_clean_chunk else S
-            if n_keep < 0 or start + n_keep > cache.shape[0]:
+            if start < 0 or n_keep < 0 or start + n_keep > cache.shape[0]:
                 return None  # (forward() refuses it)
             if n_keep < S:
                 tail = self._tail_rows(S - n_keep, cache)

@@ -289,6 +289,20 @@ def test_replaced_methods_of_a_small_layer_are_called(dev, on, name, how):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("slice_point", [-1, 3, 5])
+def test_positions_outside_the_cache_are_refused_in_small_layers(dev, monkeypatch, slice_point):
+    """Ahead of and behind the cached rows, before anything is launched by address."""
+    layer, _, (hs, y, meta, rope) = _layer_case(dev, 256, 1, 5, 9, 2, 1, "append", False, [33, 20])
+    monkeypatch.setattr(MOD, "launch_small_projections", lambda *a: pytest.fail("launched"))
+    ip = P.InferenceParams(1, 4 * 45)
+    ip.key_value_memory_dict[1] = torch.full((4 * 45, 2, 2 * D), 7.0, dtype=torch.bfloat16, device=dev)
+    ip.update_kv_cache = True
+    with torch.no_grad(), pytest.raises(ValueError):
+        layer(hs, y, ip, rope, dataclasses.replace(meta, slice_point=slice_point, extract_prefix_video_feature=True))
+    assert (ip.key_value_memory_dict[1] == 7).all()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("heads", [1, 4, 8])
 @pytest.mark.parametrize("small", [True, False])
 def test_text_weight_with_other_heads_than_the_layer(dev, monkeypatch, small, heads):
