@@ -201,10 +201,13 @@ def _linear_in_whole_rounds(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return torch.nn.functional.linear(x, w)
 
 
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
+
+
 def _plain_rows(x: torch.Tensor, w: torch.Tensor, heads: int) -> bool:
     """Whether x [rows, K] and the weight w [heads * 128, K] are as small_projections takes them: bf16 rows of the same device, aligned, of a
-    multiple of 64 elements, and no autocast that would have the library's product convert them."""
-    if w.shape[0] != 128 * heads or x.dim() != 2 or x.dtype is not torch.bfloat16 or w.dtype is not torch.bfloat16 or torch.is_autocast_enabled():
+    multiple of 64 elements, no subclass of tensors with a product of its own, no autocast that would have the library's convert them."""
+    if type(x) not in _PLAIN or type(w) not in _PLAIN or w.shape[0] != 128 * heads or x.dim() != 2 or x.dtype is not torch.bfloat16 or w.dtype is not torch.bfloat16 or torch.is_autocast_enabled():
         return False
     K = x.shape[1]
     if K % 64 or w.dim() != 2 or w.shape[1] != K or not w.is_contiguous() or x.shape[0] == 0 or not x.is_cuda or w.device != x.device:

@@ -288,6 +288,29 @@ def test_replaced_methods_of_a_small_layer_are_called(dev, on, name, how):
         assert all(torch.equal(a, b) for a, b in zip(got, want))
 
 
+class _TwiceTheProduct(torch.Tensor):
+    """A weight with a product of its own, as quantised or sharded ones have."""
+
+    @classmethod
+    def __torch_function__(cls, func, types, args=(), kwargs=None):
+        out = super().__torch_function__(func, types, args, kwargs or {})
+        return out.as_subclass(torch.Tensor) * 2 if func is torch.nn.functional.linear else out
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("small", [True, False])
+def test_text_weight_with_a_product_of_its_own(dev, monkeypatch, small):
+    """Is asked for it, not read: the values (not normed) and so the cross attention come out twice as large."""
+    layer, run, _ = _layer_case(dev, 256, 1, 5, 9, 2, 1, "none", False, [33, 20])
+    if not small:
+        monkeypatch.setattr(MOD, "_projects_in_one_launch", lambda *a: False)
+    want, _ = run()
+    layer.linear_kv_xattn.weight = torch.nn.Parameter(layer.linear_kv_xattn.weight.detach().as_subclass(_TwiceTheProduct), requires_grad=False)
+    got, _ = run()
+    assert torch.equal(got[0], want[0])
+    assert float((got[1].float() - 2 * want[1].float()).abs().max()) <= 2e-2 * float(want[1].abs().max())
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("slice_point", [-1, 3, 5])
 def test_positions_outside_the_cache_are_refused_in_small_layers(dev, monkeypatch, slice_point):
