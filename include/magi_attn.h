@@ -231,9 +231,14 @@ typedef struct magi_attn_args {
   int64_t split_workspace_bytes;
 } magi_attn_args;
 
-/* Bytes of split_workspace that a call of these sizes may make use of (dtype: MAGI_DTYPE_*); 0: such a call is not split.  (Where
- * smaller workgroups fill the chip better, only MAGI_ATTN_CHECKED does.) */
+/* Bytes of split_workspace that a call of these sizes makes use of in 256-row (fp8: 128-row) workgroups (dtype: MAGI_DTYPE_*); 0: such
+ * a call is not split. */
 int64_t magi_attn_split_bytes(int32_t Hq, int32_t Hkv, int32_t n_ranges, int32_t max_seqlen_q, int32_t max_seqlen_k, int32_t dtype);
+
+/* Rows per workgroup that a bf16 call of these sizes takes with a score_bound in force (or measured and in force), q_tile_rows 0, no
+ * MAGI_ATTN_CHECKED and this much split_workspace: 256, or 128 where these fill the chip better, which make no use of that memory.  A row's
+ * bits are those of 256-row workgroups without it. */
+int32_t magi_attn_tile_rows(int32_t Hq, int32_t Hkv, int32_t n_ranges, int32_t max_seqlen_q, int32_t max_seqlen_k, int64_t split_workspace_bytes);
 
 int magi_attn_fwd(const magi_attn_args* args, void* stream);
 

@@ -170,23 +170,17 @@ SplitPlan split_plan(unsigned items, int n_ranges, int max_seqlen_q, int max_seq
 // 972 x 4 over 972 to 3888 130 / - / 123, but 3800 over 3800 168 / - / 172 and 1000 x 3 over 3000 to 5000 161 / 148 / 173.  Few items
 // with long keys are better off in pieces, which cost about 12 us and 0.3 per piece of an XCD: 240 rows over 3000 keys 86 / 33 / 56,
 // 1300 over 4000 113 / 81 / 97.
-struct TilePlan {
-  int rows;
-  SplitPlan split;
-};
-TilePlan tile_plan(int Hq, int Hkv, int n_ranges, int max_seqlen_q, int max_seqlen_k, int64_t split_bytes) {
+int tile_rows(int Hq, int Hkv, int n_ranges, int max_seqlen_q, int max_seqlen_k, int64_t split_bytes) {
   auto items = [&](int rows) { return items_per_xcd(Hq, Hkv, n_ranges, max_seqlen_q / rows + (max_seqlen_q % rows != 0)); };
-  const SplitPlan none = {UINT32_MAX, 1, 1, 1, false};
   const unsigned cus = (unsigned)compute_units() / 8, whole = items(256), half = items(128);
-  TilePlan t = {256, split_bytes > 0 ? split_plan(whole, n_ranges, max_seqlen_q, max_seqlen_k, false) : none};
-  if (t.split.bytes(whole) > split_bytes) t.split = none;
-  if (half > 2 * cus) return t;
-  if (t.split.from < whole) {  // (without a whole round ahead of them: all items are in pieces)
-    const unsigned pieces = whole * t.split.pieces;
-    const double tiles = (max_seqlen_k + 63) / 64, in_pieces = tiles * t.split.num / t.split.den * (pieces <= cus ? 1.75 : 2.6) + 12.0 + 0.3 * pieces;
-    if (in_pieces <= tiles * (half <= cus ? 1.15 : 1.75)) return t;
-  }
-  return {128, none};
+  if (half > 2 * cus) return 256;
+  if (split_bytes <= 0) return 128;
+  const SplitPlan s = split_plan(whole, n_ranges, max_seqlen_q, max_seqlen_k, false);
+  if (s.from >= whole || s.bytes(whole) > split_bytes) return 128;
+  // (without a whole round ahead of them: all items are in pieces)
+  const unsigned pieces = whole * s.pieces;
+  const double tiles = (max_seqlen_k + 63) / 64, in_pieces = tiles * s.num / s.den * (pieces <= cus ? 1.75 : 2.6) + 12.0 + 0.3 * pieces;
+  return in_pieces <= tiles * (half <= cus ? 1.15 : 1.75) ? 256 : 128;
 }
 
 int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace);
@@ -219,6 +213,13 @@ int64_t magi_attn_split_bytes(int32_t Hq, int32_t Hkv, int32_t n_ranges, int32_t
   if ((double)Hq * n_ranges * tiles > 2.0e9) return 0;
   const unsigned items = items_per_xcd(Hq, Hkv, n_ranges, tiles);
   return split_plan(items, n_ranges, max_seqlen_q, max_seqlen_k, fp8).bytes(items);
+}
+
+int32_t magi_attn_tile_rows(int32_t Hq, int32_t Hkv, int32_t n_ranges, int32_t max_seqlen_q, int32_t max_seqlen_k,
+                            int64_t split_workspace_bytes) {
+  if (Hq <= 0 || Hkv <= 0 || Hq % Hkv || n_ranges <= 0 || max_seqlen_q <= 0) return 256;
+  if ((double)Hq * n_ranges * (max_seqlen_q / 128 + 1) > 2.0e9) return 256;
+  return tile_rows(Hq, Hkv, n_ranges, max_seqlen_q, max_seqlen_k, split_workspace_bytes);
 }
 
 int magi_attn_fwd(const magi_attn_args* p, void* stream) {
@@ -423,14 +424,14 @@ int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace) {
   auto launch = [&](bool bounded) -> int {
     // a bound stated for unscaled q (what the reference's callers pass): the kernel applies the softmax scale while
     // it loads q, after which the scores are exp2 exponents as with MAGI_ATTN_Q_PRESCALED
+    const int64_t split_bytes = p->split_workspace ? p->split_workspace_bytes : 0;
     const bool scale_q = bounded && !q_norm && !checked && !(p->flags & MAGI_ATTN_Q_PRESCALED);
     a.block_m = 128;
     if (p->dtype == MAGI_DTYPE_BF16) {
       const double wg384 = (double)p->Hq * p->n_ranges * ((p->max_seqlen_q + 383) / 384);
       const bool long_keys = p->max_seqlen_k == 0 || p->max_seqlen_k >= 4096;  // (0 = not stated)
       if (bounded && !checked && !mfma32)
-        a.block_m = tile_plan(p->Hq, p->Hkv, p->n_ranges, p->max_seqlen_q, p->max_seqlen_k,
-                              p->split_workspace ? p->split_workspace_bytes : 0).rows;
+        a.block_m = tile_rows(p->Hq, p->Hkv, p->n_ranges, p->max_seqlen_q, p->max_seqlen_k, split_bytes);
       else if (bounded)
         a.block_m = 256;  // (512-row workgroups fetch half the tiles and measure 1 % slower: their two waves per SIMD march in step)
       else if (wg384 >= 9.0 * compute_units() && long_keys)
@@ -451,9 +452,9 @@ int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace) {
     a.per_xcd = items_per_xcd(p->Hq, p->Hkv, p->n_ranges, a.tiles_per_range);
     a.split_from = UINT32_MAX;
     const bool fp8 = p->dtype == MAGI_DTYPE_FP8_E4M3;
-    if ((fp8 || (bounded && a.block_m == 256 && !mfma32)) && p->split_workspace) {
+    if ((fp8 || (bounded && a.block_m == 256 && !mfma32)) && split_bytes > 0) {
       const SplitPlan s = split_plan(a.per_xcd, p->n_ranges, p->max_seqlen_q, p->max_seqlen_k, fp8);
-      if (s.from < a.per_xcd && s.bytes(a.per_xcd) <= p->split_workspace_bytes) {
+      if (s.from < a.per_xcd && s.bytes(a.per_xcd) <= split_bytes) {
         a.partial = static_cast<float*>(p->split_workspace);
         a.split_from = s.from;
         a.split_pieces = s.pieces;
