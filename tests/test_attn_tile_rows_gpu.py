@@ -15,6 +15,19 @@ def _rows(g, dev, *shape):
     return torch.nn.functional.layer_norm(x, (D,))
 
 
+def _kernels(call):
+    """What call() returns, and the names of the attention kernels that ran in it."""
+    from torch.profiler import ProfilerActivity, profile
+
+    with profile(activities=[ProfilerActivity.CUDA]) as prof:
+        out = call()
+        torch.cuda.synchronize()
+    names = [e.name for e in prof.events() if "attn_fwd_bf16" in e.name]
+    if not names:
+        pytest.skip("the profiler records no kernels here: nothing says which of them ran")
+    return out, names
+
+
 # rows around 32 (a wavefront), 128 and 256 (a workgroup); keys around half a tile and a tile; one and several ranges, an empty one,
 # rows that no range covers, ranges in another order, a key axis in two pieces
 @pytest.mark.gpu
@@ -42,8 +55,12 @@ def test_rows_of_the_smaller_workgroups_have_the_same_bits(dev, mode, Hq, Hkv, T
         k, v = k[:k_split], v[:k_split]
     most_q, most_k = max(e - b for b, e in q_ranges), max(e - b for b, e in k_ranges)
     call = lambda rows, **o: M.range_attention(q, k, v, qr, kr, most_q, most_k, q_tile_rows=rows, split_keys=False, **kw, **o)  # noqa: E731
-    (a, la), (b, lb) = call(0), call(256)
+    (a, la), ran = _kernels(lambda: call(0))
+    (b, lb), ran_256 = _kernels(lambda: call(256))
     assert torch.equal(a, b) and torch.equal(la, lb)
+    form = {"as it is": 0, "normed": 1, "scaled": 2}[mode]
+    for names, blocks in ((ran, 2), (ran_256, 4)):  # (query blocks of 16 rows per wavefront: the two forms that were compared)
+        assert len(names) == 1 and f"attn_fwd_bf16_x16_kernel<{form}, {blocks}>" in names[0], names
     if Hq % 2 == 0:  # grouped outputs
         o = [torch.full((Tq, 2, 2, Hq // 2, D), 3.0, device=dev, dtype=torch.bfloat16) for _ in range(2)]
         call(0, out=o[0][:, :, 1])
@@ -62,21 +79,13 @@ def test_rows_of_the_smaller_workgroups_have_the_same_bits(dev, mode, Hq, Hkv, T
     (240, 1, 13, 24, 8, False, True), (2600, 1, 4, 24, 8, True, True), (1300, 1, 3, 24, 8, True, False), (1000, 3, 2, 24, 8, True, False)])
 def test_which_launches_take_the_smaller_workgroups(dev, rows, n, prefix, Hq, Hkv, split, smaller):
     """By the name of the kernel that runs; no launch behind it that adds pieces up."""
-    from torch.profiler import ProfilerActivity, profile
-
     q, kv = (torch.randn(r, h, 2 * D, device=dev, dtype=torch.bfloat16) * 0.1 for r, h in ((n * rows, Hq), ((n + prefix) * rows, Hkv)))
     qr = torch.tensor([[i * rows, (i + 1) * rows] for i in range(n)], dtype=torch.int32, device=dev)
     kr = torch.tensor([[0, (prefix + i + 1) * rows] for i in range(n)], dtype=torch.int32, device=dev)
-    call = lambda: M.range_attention(q[..., :D], kv[..., :D], kv[..., D:], qr, kr, rows, (n + prefix) * rows, q_prescaled=True,  # noqa: E731
-                                     score_bound=60.0, split_keys=split, return_lse=False)
-    call()
-    with profile(activities=[ProfilerActivity.CUDA]) as prof:
-        call()
-        torch.cuda.synchronize()
-    names = [e.name for e in prof.events() if "attn_fwd_bf16" in e.name]
-    if names:  # (nothing recorded: the bits above are the check)
-        assert any("x16_kernel<0, 2>" in x for x in names) == smaller, names
-        assert not (smaller and any("merge" in x for x in names)), names
+    _, names = _kernels(lambda: M.range_attention(q[..., :D], kv[..., :D], kv[..., D:], qr, kr, rows, (n + prefix) * rows, q_prescaled=True,
+                                                  score_bound=60.0, split_keys=split, return_lse=False))
+    assert any("x16_kernel<0, 2>" in x for x in names) == smaller, names
+    assert not (smaller and any("merge" in x for x in names)), names
 
 
 # rows per range, ranges, cached ranges, with scratch memory: as above
