@@ -226,14 +226,15 @@ def _compute_units(device: torch.device) -> int:
     return n
 
 
-def _projects_in_one_launch(rows: int, heads: int, text_rows: int, text_heads: int, K: int, cus: int) -> bool:
+def _projects_in_one_launch(rows: int, heads: int, text_rows: int, text_heads: int, K: int, cus: int, captured: bool = False) -> bool:
     """Whether a layer's projections run as one launch of small_projections: where its workgroups (32 rows x one head each, 64 rows up
     to K = 768) are one round, or up to four of the taller ones.  In one round the launch takes less time than the norm, the library's
-    two products, the prologue and the text's head norm (240 + 24 rows at K = 768, 20 + 4 heads, 12.7 against 22 us; 672 rows 19.4
-    against 26), in several more (1344 rows 36 against 29, 2048 39 against 32), but the host issues the layer 100 us sooner, and such
-    layers wait for it: 840 rows behind 1120 167 / 105 us in all, 2048 rows over 6144 keys 154 / 130.  The rest is not measured."""
+    two products, the prologue and the text's head norm (K = 768, 20 + 4 heads, 24 text rows: 240 rows 11.6 / 22.1 us, 768 rows 17.8 / 25.7), in
+    several more (840 rows 29.6 / 26.9, 1344 32.7 / 30.4, 2048 48.1 / 35.7), but the host issues the layer 80 us sooner and such layers wait
+    for it: 840 rows over 1260 keys 68 / 150 us in all, 1344 over 2688 76 / 154, 2048 over 6144 118 / 154.
+    captured: into a graph, where no host is waited for: one round only (the same layers replayed 70 / 71, 79 / 77, 120 / 108 us)."""
     tile = lambda n: ((rows + n - 1) // n) * heads + ((text_rows + n - 1) // n) * text_heads  # noqa: E731
-    return tile(64) <= 4 * cus if K <= 768 else tile(32) <= cus
+    return tile(64) <= (1 if captured else 4) * cus if K <= 768 else tile(32) <= cus
 
 
 def _text_in_one_launch(flop: float, rows: int, heads: int, K: int, cus: int) -> bool:
@@ -246,7 +247,8 @@ def _text_in_one_launch(flop: float, rows: int, heads: int, K: int, cus: int) ->
     `heads`): more rows (64 a workgroup then) gain nothing, four chunks of 1170 rows with 674 in all 374 / 376.  At K = 6144 the
     product is the faster one (400 rows 25 / 29 us).
     Up to 2^17 results of a long sum the library cuts K in pieces (64 rows at 16 heads, 128 at 8): another order of the sums, other bits.
-    Those layers keep the library's."""
+    Those layers keep the library's, and so do those captured into a graph, which wait for no host, unless K is at most 1024 (100 rows at
+    K = 768 and 4 heads 10.3 / 7.7 us, 300 at 1024 and 16 12.6 / 9.3)."""
     return (flop < 7e10 or rows >= 200) and K <= 3072 and (K <= 1024 or rows * heads > 1024) and (rows + 31) // 32 * heads <= cus
 
 
@@ -892,7 +894,8 @@ class FullyParallelAttention(torch.nn.Module):
             return None
         dev = hidden_states.device
         Hq, Hkv, D, (T, Kt) = self.num_attention_heads, self.num_query_groups_per_partition, 128, key_value_states.shape
-        if Kt > 1024 or not _projects_in_one_launch(S, 2 * (Hq + Hkv), T, 2 * Hkv, max(K, Kt), _compute_units(dev)):
+        size = (S, 2 * (Hq + Hkv), T, 2 * Hkv, max(K, Kt), _compute_units(dev))
+        if Kt > 1024 or not _projects_in_one_launch(*size) or (not _projects_in_one_launch(*size, True) and torch.cuda.is_current_stream_capturing()):
             return None
         m = self._modules
         lin = m["linear_qkv"]
@@ -1065,7 +1068,7 @@ class FullyParallelAttention(torch.nn.Module):
             flop = 512.0 * sq * Hq * (hidden_states.shape[2] + p.max_seqlen_k)
             own_text = (bs == 1 and key_value_states.dim() == 2 and hidden_states.is_cuda and _is_own(self, _OWN_SMALL) and _text_in_one_launch(
                 flop, key_value_states.shape[0], 2 * self.num_query_groups_per_partition, key_value_states.shape[1],
-                _compute_units(hidden_states.device)))
+                _compute_units(hidden_states.device)) and (key_value_states.shape[1] <= 1024 or not torch.cuda.is_current_stream_capturing()))
             more = {"own_text": True} if own_text else {}  # (one put in its place may not know it)
             return self._cross_attention_fused(qx_raw, sq, bs, key_value_states, meta_args.cross_attn_params, dst, bound_cross, **more)
 
