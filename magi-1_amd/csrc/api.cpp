@@ -381,7 +381,8 @@ int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace) {
   //    wavefront; 256-row workgroups (4 waves, two per CU: the two waves of a SIMD belong to different workgroups
   //    and drift out of step, so one computes scores while the other is in its softmax) on v_mfma_f32_16x16x32
   //    (the part is power limited and that shape takes less energy per FLOP; measured +3 % on the 720p layer,
-  //    between 0 and +6 % from box to box); the 32x32x16 form on request and for 512-row workgroups.
+  //    between 0 and +6 % from box to box), 128-row ones with 32 rows per wavefront where that leaves at most two of them per CU
+  //    (tile_rows); the 32x32x16 form on request and for 512-row workgroups.
   //  * Otherwise 32 rows per wavefront with the online softmax: 384-row workgroups (12 waves, one workgroup per CU,
   //    every K / V tile fetched once for three times as many rows and one barrier per tile) pay on grids of many
   //    rounds with long key ranges (measured: +3 % at 43 rounds, +1 % at 9.4, -3 % at 5.3); small grids and short
@@ -670,7 +671,8 @@ int magi_small_projections(const magi_small_proj_args* p, void* stream) {
     if (!p->x || !p->w) return fail(MAGI_EINVAL, "magi_small_projections: NULL x / w");
     if (p->x_stride < p->K || p->x_stride % 8 || !aligned16(p->x) || !aligned16(p->w))
       return fail(MAGI_EINVAL, "magi_small_projections: rows of x and w must be 16-byte aligned and at least K long");
-    // (32-bit byte offsets: 32 rows of x, the 128 weight rows of a head)
+    // (32-bit byte offsets within the descriptors' 2^31 - 1: row 63 of a workgroup's 64 rows of x, 2^25 bytes apart at most, which nearly
+    // fills them; the 128 weight rows of a head)
     if (p->x_stride > (1 << 24) || p->K > (1 << 22)) return fail(MAGI_ENOSYS, "magi_small_projections: rows above 2^22 elements are not implemented");
     if (p->ln_w && (p->K > 1024 || (text && p->Kt > 1024)))
       return fail(MAGI_ENOSYS, "magi_small_projections: the input norm is implemented for K (and Kt) up to 1024");

@@ -10,11 +10,12 @@
 // each live for little more than a launch and a few trips to memory, and a library call costs the host 18 us to issue.
 // So: many small workgroups.  A workgroup of four wavefronts forms 32 or 64 rows x one head (128 columns); the weight rows stream
 // through LDS in steps of 64 elements of K, three to six stages filled by direct global->LDS loads, 128 bytes of a row per eight
-// lanes, which stay in flight over the barriers (__syncthreads() would wait for them: layers of 768 rows 121 against 116 us, of 840
-// rows 158 against 148) (operands loaded straight into registers, 16 bytes per lane from 16 rows at a time, move 16 bytes per clock and CU: 33 us
-// for 400 text tokens at K = 3072, 16 so).  The product is formed transposed, W X^T on
-// v_mfma_f32_16x16x32_bf16 with the weight rows as the A operand: register r of lane (n, g) of a result block is column 4 g + r
-// of the block, row n; it goes through LDS to eight lanes per row, which do with it what the prologue does.
+// lanes.  (Operands loaded straight into registers, 16 bytes per lane from 16 rows at a time, move 16 bytes per clock and CU: 33 us
+// for 400 text tokens at K = 3072, 16 so.)  The loads stay in flight over the barriers; __syncthreads() would wait for them (layers of 768
+// rows 121 against 116 us, of 840 rows 158 against 148).
+// The product is formed transposed, W X^T on v_mfma_f32_16x16x32_bf16 with the weight rows as the A operand: register r of lane
+// (n, g) of a result block is column 4 g + r of the block, row n; it goes through LDS to eight lanes per row, which do with it
+// what the prologue does.
 // RES: the workgroup's rows are in LDS whole (K up to 1024), normalised ahead of the product.  Otherwise the rows, not to be
 // normalised, stream beside the weights.  (Streaming workgroups that start at different places of K, so that they are not all at
 // the same bytes of rows a multiple of the caches' interleave apart: 300 rows x 16 heads at K = 3072 out of memory 21.7 / 17.8 us,
@@ -31,7 +32,8 @@ constexpr int STAGE_W = D * BK * 2;
 constexpr int LDS_MAX = 160 * 1024;
 // bytes per resident row: 16 more than its elements, so that the 16 rows of an operand read fall on different banks
 __device__ __forceinline__ int resident_row(int K) { return 2 * K + 16; }
-// Resident rows (RES): how long they may be, beside three stages of weights
+// Resident rows (RES): how long they may be, beside the stages of weights.  (64 rows of 832 elements would fit too; they would be a
+// thirteenth piece per lane for a width that no layer here has.)
 template <int ROWS>
 constexpr int res_max_k() { return ROWS == 32 ? 1024 : 768; }
 
@@ -235,44 +237,44 @@ __global__ __launch_bounds__(64 * NW, 1) void small_proj_kernel(const SmallProjK
   if constexpr (RES) {
 #pragma unroll
     for (int half = 0; half < ROWS / 32; ++half) {
-    const int r = 32 * half + (tid >> 3), j = tid & 7;
-    const char* const rp = x + (long)min(row0 + r, rows - 1) * xs;
-    constexpr int NV = res_max_k<ROWS>() / 64;  // pieces of eight elements per lane: j, j + 8, ...
-    const int nv = K >> 6;
-    u32x4 raw[NV];
+      const int r = 32 * half + (tid >> 3), j = tid & 7;
+      const char* const rp = x + (long)min(row0 + r, rows - 1) * xs;
+      constexpr int NV = res_max_k<ROWS>() / 64;  // pieces of eight elements per lane: j, j + 8, ...
+      const int nv = K >> 6;
+      u32x4 raw[NV];
 #pragma unroll
-    for (int i = 0; i < NV; ++i) raw[i] = i < nv ? *(const u32x4*)(rp + (8 * i + j) * 16) : u32x4{0u, 0u, 0u, 0u};
-    u32x4 lnw[NV], lnb[NV];  // bf16 parameters, requested with the rows
-    if (ln && !a.ln_fp32) {
+      for (int i = 0; i < NV; ++i) raw[i] = i < nv ? *(const u32x4*)(rp + (8 * i + j) * 16) : u32x4{0u, 0u, 0u, 0u};
+      u32x4 lnw[NV], lnb[NV];  // bf16 parameters, requested with the rows
+      if (ln && !a.ln_fp32) {
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+          lnw[i] = i < nv ? *(const u32x4*)(a.ln_w + (8 * i + j) * 16) : u32x4{0u, 0u, 0u, 0u};
+          lnb[i] = i < nv ? *(const u32x4*)(a.ln_b + (8 * i + j) * 16) : u32x4{0u, 0u, 0u, 0u};
+        }
+      }
+      float mean = 0.f, rstd = 1.f;
+      if (ln) row_stats8<NV>(raw, j, nv, 1.f / (float)K, a.ln_eps, mean, rstd);
 #pragma unroll
       for (int i = 0; i < NV; ++i) {
-        lnw[i] = i < nv ? *(const u32x4*)(a.ln_w + (8 * i + j) * 16) : u32x4{0u, 0u, 0u, 0u};
-        lnb[i] = i < nv ? *(const u32x4*)(a.ln_b + (8 * i + j) * 16) : u32x4{0u, 0u, 0u, 0u};
+        if (i >= nv) continue;
+        float f[8], wf[8], bf[8];
+        unpack8(raw[i], f);
+        if (!ln) {
+          *LDS_PTR(u32x4, sR + r * x_row + (8 * i + j) * 16) = raw[i];
+          continue;
+        }
+        if (a.ln_fp32) {
+          param8<true>(a.ln_w, 8 * i + j, wf);
+          param8<true>(a.ln_b, 8 * i + j, bf);
+        } else {
+          unpack8(lnw[i], wf);
+          unpack8(lnb[i], bf);
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) f[e] = __builtin_fmaf((f[e] - mean) * rstd, wf[e], bf[e]);
+        *LDS_PTR(u32x4, sR + r * x_row + (8 * i + j) * 16) = pack8(f);
       }
     }
-    float mean = 0.f, rstd = 1.f;
-    if (ln) row_stats8<NV>(raw, j, nv, 1.f / (float)K, a.ln_eps, mean, rstd);
-#pragma unroll
-    for (int i = 0; i < NV; ++i) {
-      if (i >= nv) continue;
-      float f[8], wf[8], bf[8];
-      unpack8(raw[i], f);
-      if (!ln) {
-        *LDS_PTR(u32x4, sR + r * x_row + (8 * i + j) * 16) = raw[i];
-        continue;
-      }
-      if (a.ln_fp32) {
-        param8<true>(a.ln_w, 8 * i + j, wf);
-        param8<true>(a.ln_b, 8 * i + j, bf);
-      } else {
-        unpack8(lnw[i], wf);
-        unpack8(lnb[i], bf);
-      }
-#pragma unroll
-      for (int e = 0; e < 8; ++e) f[e] = __builtin_fmaf((f[e] - mean) * rstd, wf[e], bf[e]);
-      *LDS_PTR(u32x4, sR + r * x_row + (8 * i + j) * 16) = pack8(f);
-    }
-   }
   }
 
   // ---- operand reads: lane (n, g) holds elements 32 kk + 8 g .. +8 of weight row 32 w + 16 fb + n and of row 16 tb + n ----
@@ -369,16 +371,16 @@ __global__ __launch_bounds__(64 * NW, 1) void small_proj_kernel(const SmallProjK
   // 32 rows at a time through LDS: 512 bytes a row, its 16-byte chunk c at c ^ (row % 16)
   float* const out = (float*)sW0;
 #pragma unroll
- for (int half = 0; half < ROWS / 32; ++half) {
-  __syncthreads();
+  for (int half = 0; half < ROWS / 32; ++half) {
+    __syncthreads();
 #pragma unroll
-  for (int fb = 0; fb < 2; ++fb)
+    for (int fb = 0; fb < 2; ++fb)
 #pragma unroll
-    for (int tb = 0; tb < 2; ++tb)
-      *LDS_PTR(f32x4, out + (16 * tb + n) * D + (((8 * w + 4 * fb + g) ^ n) << 2)) = acc[fb][2 * half + tb];
-  __syncthreads();
-  store_rows32(a, params, half, out, text, head, row0 + 32 * half, rows, tid);
- }
+      for (int tb = 0; tb < 2; ++tb)
+        *LDS_PTR(f32x4, out + (16 * tb + n) * D + (((8 * w + 4 * fb + g) ^ n) << 2)) = acc[fb][2 * half + tb];
+    __syncthreads();
+    store_rows32(a, params, half, out, text, head, row0 + 32 * half, rows, tid);
+  }
 }
 
 }  // namespace

@@ -884,8 +884,8 @@ class FullyParallelAttention(torch.nn.Module):
                        rope: torch.Tensor, meta_args: ModelMetaArgs, proj_layout: bool, bound_core: float, bound_cross: float):
         """forward() of a small bf16 layer at batch 1 with both score bounds in force, whose projections are the library's own: three
         launches (magi_small_projections, core attention, cross attention) with their arguments put together in one go.  None, before
-        anything has changed, where forward() goes on with the separate launches: other projections or caches, larger layers, tensors
-        of other types or layouts.
+        anything is launched or written, where forward() goes on with the separate launches: other methods, projections or caches, larger
+        layers, tensors of other types or layouts.  (The layer's cache and its side buffer may have been allocated by then, as forward() would.)
 
         Such a layer waits for the host: 240 + 24 rows, 20 + 4 heads, 87 us through the callables, 51 this way.  There
         each launch brings its own checks, allocations and views with it."""
@@ -1144,7 +1144,7 @@ class FullyParallelAttention(torch.nn.Module):
         return core_attn_out, xattn_out
 
 
-_KERNEL_NAMES = ("online softmax, 32 rows per wavefront", "bounded-score, 64 rows per wavefront")  # by: a bound is in force
+_KERNEL_NAMES = ("online softmax, 32 rows per wavefront", "bounded-score, 64 rows per wavefront (32 in small launches)")  # by: a bound is in force
 # the methods whose work forward() does in another shape, as long as they are these
 _OWN_FP8_LINEAR = {"forward": PerTensorQuantizedFp8Linear.forward}
 _OWN_PROJECTIONS = {"forward_ln": CustomLayerNormLinear.forward_ln, "forward_qkvx": CustomLayerNormLinear.forward_qkvx}
