@@ -28,6 +28,7 @@ from typing import Callable, Optional, Tuple
 
 import itertools
 import math
+import operator
 import os
 
 import torch
@@ -204,16 +205,21 @@ def _linear_in_whole_rounds(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 _PLAIN = (torch.Tensor, torch.nn.Parameter)
 
 
+def _plain_weight(w: torch.Tensor, heads: int, K: int, device: torch.device) -> bool:
+    """Whether w is as small_projections takes a weight: plain bf16 rows [heads * 128, K], K a multiple of 64, aligned, on the device;
+    no subclass of tensors with a product of its own, no autocast that would have the library's product convert it."""
+    return (type(w) in _PLAIN and w.shape == (128 * heads, K) and w.dtype is torch.bfloat16 and K % 64 == 0 and w.is_contiguous()
+            and w.device == device and w.data_ptr() % 16 == 0 and not torch.is_autocast_enabled())
+
+
 def _plain_rows(x: torch.Tensor, w: torch.Tensor, heads: int) -> bool:
-    """Whether x [rows, K] and the weight w [heads * 128, K] are as small_projections takes them: bf16 rows of the same device, aligned, of a
-    multiple of 64 elements, no subclass of tensors with a product of its own, no autocast that would have the library's convert them."""
-    if type(x) not in _PLAIN or type(w) not in _PLAIN or w.shape[0] != 128 * heads or x.dim() != 2 or x.dtype is not torch.bfloat16 or w.dtype is not torch.bfloat16 or torch.is_autocast_enabled():
+    """The same of the rows x [rows, K] and their weight w."""
+    if type(x) not in _PLAIN or x.dim() != 2 or x.dtype is not torch.bfloat16 or not x.is_cuda:
         return False
-    K = x.shape[1]
-    if K % 64 or w.dim() != 2 or w.shape[1] != K or not w.is_contiguous() or x.shape[0] == 0 or not x.is_cuda or w.device != x.device:
-        return False
+    rows, K = x.shape
     st = x.stride()
-    return st[1] == 1 and K <= st[0] <= 1 << 24 and st[0] % 8 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+    return (rows > 0 and st[1] == 1 and K <= st[0] <= 1 << 24 and st[0] % 8 == 0 and x.data_ptr() % 16 == 0
+            and _plain_weight(w, heads, K, x.device))
 
 
 _CUS = {}  # compute units by device index
@@ -257,14 +263,17 @@ def _global_hooks() -> bool:
     return bool(torch.nn.modules.module._has_any_global_hook())
 
 
-def _is_own(m: torch.nn.Module, own: dict) -> bool:
-    """Whether calling these methods of m runs the library's code as it stands here ({name: function}): no subclass, no patch of
-    the class and none of the instance replaces one."""
-    t, state = type(m), m.__dict__
-    for name, f in own.items():
-        if getattr(t, name, None) is not f or name in state:
-            return False
-    return True
+class _Own:
+    """The library's functions of these names in a class of modules.  of(m): whether calling them on m runs the library's code as it
+    stands here, no other class, no patch of the class and none of the instance replaces one."""
+
+    def __init__(self, cls: type, *names: str):
+        self.cls, self.names = cls, names
+        self.get = operator.attrgetter(*names) if len(names) > 1 else lambda t, _get=operator.attrgetter(*names): (_get(t),)
+        self.functions = self.get(cls)
+
+    def of(self, m: torch.nn.Module) -> bool:
+        return isinstance(m, self.cls) and self.get(type(m)) == self.functions and m.__dict__.keys().isdisjoint(self.names)
 
 
 class PerTensorQuantizedFp8Linear(torch.nn.Module):
@@ -378,7 +387,7 @@ class CustomLayerNormLinear(torch.nn.Module):
         """Whether the fused norm may hand m its quantised input: m is the fp8 linear itself (another class has its own
         attributes and its own idea of the input), nothing watches or replaces its call, and its input_scale is as
         layer_norm_div_clamp takes it."""
-        if type(m) is not PerTensorQuantizedFp8Linear or not _is_own(m, _OWN_FP8_LINEAR):
+        if type(m) is not PerTensorQuantizedFp8Linear or not _OWN_FP8_LINEAR.of(m):
             return False
         if m._forward_hooks or m._forward_pre_hooks or _global_hooks():
             return False
@@ -866,7 +875,7 @@ class FullyParallelAttention(torch.nn.Module):
         """-> (q, k, v, qx) of the normalised input as [tokens, out] rows, and that input where it exists: with the library's
         own projections only the rows are formed, others have their forward_ln and forward_qkvx called."""
         m = self._modules["linear_qkv"]
-        if _is_own(m, _OWN_PROJECTIONS):
+        if _OWN_PROJECTIONS.of(m):
             return m.forward_ln_qkvx_rows(hidden_states), None
         x = m.forward_ln(hidden_states)
         return tuple(t.reshape(-1, t.shape[-1]) for t in m.forward_qkvx(x)), x
@@ -895,30 +904,28 @@ class FullyParallelAttention(torch.nn.Module):
         dev = hidden_states.device
         Hq, Hkv, D, (T, Kt) = self.num_attention_heads, self.num_query_groups_per_partition, 128, key_value_states.shape
         size = (S, 2 * (Hq + Hkv), T, 2 * Hkv, max(K, Kt), _compute_units(dev))
-        if Kt > 1024 or not _projects_in_one_launch(*size) or (not _projects_in_one_launch(*size, True) and torch.cuda.is_current_stream_capturing()):
+        if Kt > 1024 or not (_projects_in_one_launch(*size, True) or (_projects_in_one_launch(*size) and not torch.cuda.is_current_stream_capturing())):
             return None
         m = self._modules
         lin = m["linear_qkv"]
         if lin.__dict__.get("fp8_quant", True) or not hidden_states.is_contiguous() or rope.shape[-1] % 16 or rope.shape[-1] > D:
             return None
-        if not (_is_own(lin, _OWN_SMALL_PROJECTIONS) and _is_own(self, _OWN_SMALL)):
+        use_cache = inference_params is not None and (
+            meta_args.extract_prefix_video_feature or meta_args.fwd_extra_1st_chunk or meta_args.slice_point > 0)
+        if not (_OWN_SMALL_PROJECTIONS.of(lin) and (_OWN_SMALL if use_cache else _OWN_SMALL_UNCACHED).of(self)):
             return None
         w, wt, ln = lin.fused_weight(), _param(m["linear_kv_xattn"], "weight"), lin._modules["layer_norm"]
         lw, lb = _param(ln, "weight"), _param(ln, "bias")
-        if not (_plain_rows(hidden_states[:, 0], w, 2 * (Hq + Hkv)) and _plain_rows(key_value_states, wt, 2 * Hkv)) or lw is None or lb is None:
+        if (hidden_states.dtype is not torch.bfloat16 or type(hidden_states) not in _PLAIN or S == 0 or hidden_states.data_ptr() % 16
+                or not _plain_weight(w, 2 * (Hq + Hkv), K, dev) or not _plain_rows(key_value_states, wt, 2 * Hkv) or lw is None or lb is None):
             return None
-        pq, pk = lin._projections()[:2]
-        if _param(pq, "weight").shape[0] != Hq * D or _param(pk, "weight").shape[0] != Hkv * D:
+        if _param(lin._modules["q"], "weight").shape[0] != Hq * D or _param(lin._modules["k"], "weight").shape[0] != Hkv * D:
             return None
         if lw.dtype is not lb.dtype or lw.dtype not in (torch.bfloat16, torch.float32) or not (lw.is_contiguous() and lb.is_contiguous()) or (
                 lw.shape[0] != K or lb.shape[0] != K or (lw.data_ptr() | lb.data_ptr()) % 16 or lw.device != dev or key_value_states.device != dev):
             return None
         cache = tail = offloaded = None
         start = n_keep = persisted = 0
-        use_cache = inference_params is not None and (
-            meta_args.extract_prefix_video_feature or meta_args.fwd_extra_1st_chunk or meta_args.slice_point > 0)
-        if not use_cache and not _is_own(self, _OWN_CORE):
-            return None
         if use_cache:
             if inference_params.max_batch_size != 1:
                 return None
@@ -1044,7 +1051,7 @@ class FullyParallelAttention(torch.nn.Module):
             # all four projections in one GEMM; q / k / v feed the fused prologue as row-strided views of its result
             (q_raw, k_raw, v_raw, qx_raw), mixed_qqkv = self._project_rows(hidden_states)
             raw = (q_raw, k_raw, v_raw)
-        own_cross = _is_own(self, _OWN_CROSS)
+        own_cross = _OWN_CROSS.of(self)
         if mixed_qqkv is None:  # (the library's own methods use its shape only: every projection is in hand)
             mixed_qqkv = hidden_states if own_cross else self.linear_qkv.forward_ln(hidden_states)
 
@@ -1066,7 +1073,7 @@ class FullyParallelAttention(torch.nn.Module):
             if bs > 1 and not own_cross:  # (a replaced cross attention runs; at batch 1 with a bound in force it never did)
                 return None
             flop = 512.0 * sq * Hq * (hidden_states.shape[2] + p.max_seqlen_k)
-            own_text = (bs == 1 and key_value_states.dim() == 2 and hidden_states.is_cuda and _is_own(self, _OWN_SMALL) and _text_in_one_launch(
+            own_text = (bs == 1 and key_value_states.dim() == 2 and hidden_states.is_cuda and _OWN_SMALL.of(self) and _text_in_one_launch(
                 flop, key_value_states.shape[0], 2 * self.num_query_groups_per_partition, key_value_states.shape[1],
                 _compute_units(hidden_states.device)) and (key_value_states.shape[1] <= 1024 or not torch.cuda.is_current_stream_capturing()))
             more = {"own_text": True} if own_text else {}  # (one put in its place may not know it)
@@ -1146,11 +1153,9 @@ class FullyParallelAttention(torch.nn.Module):
 
 _KERNEL_NAMES = ("online softmax, 32 rows per wavefront", "bounded-score, 64 rows per wavefront (32 in small launches)")  # by: a bound is in force
 # the methods whose work forward() does in another shape, as long as they are these
-_OWN_FP8_LINEAR = {"forward": PerTensorQuantizedFp8Linear.forward}
-_OWN_PROJECTIONS = {"forward_ln": CustomLayerNormLinear.forward_ln, "forward_qkvx": CustomLayerNormLinear.forward_qkvx}
-_OWN_SMALL_PROJECTIONS = {**_OWN_PROJECTIONS, "forward_ln_qkvx_rows": CustomLayerNormLinear.forward_ln_qkvx_rows,
-                          "_split": CustomLayerNormLinear._split}
-_OWN_CORE = {"core_attention": FullyParallelAttention.core_attention}  # (called without a cache)
-_OWN_CROSS = {"get_xqkv": FullyParallelAttention.get_xqkv, "cross_attention": FullyParallelAttention.cross_attention}
-_OWN_SMALL = {**_OWN_CROSS, "_project_rows": FullyParallelAttention._project_rows, "_fused_qkv": FullyParallelAttention._fused_qkv,
-              "_cross_attention_fused": FullyParallelAttention._cross_attention_fused}
+_OWN_FP8_LINEAR = _Own(PerTensorQuantizedFp8Linear, "forward")
+_OWN_PROJECTIONS = _Own(CustomLayerNormLinear, "forward_ln", "forward_qkvx")
+_OWN_SMALL_PROJECTIONS = _Own(CustomLayerNormLinear, "forward_ln", "forward_qkvx", "forward_ln_qkvx_rows", "_split")
+_OWN_CROSS = _Own(FullyParallelAttention, "get_xqkv", "cross_attention")
+_OWN_SMALL = _Own(FullyParallelAttention, "_project_rows", "_fused_qkv", "_cross_attention_fused")
+_OWN_SMALL_UNCACHED = _Own(FullyParallelAttention, "_project_rows", "_fused_qkv", "_cross_attention_fused", "core_attention")
