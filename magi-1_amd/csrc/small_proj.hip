@@ -17,9 +17,11 @@
 // (n, g) of a result block is column 4 g + r of the block, row n; it goes through LDS to eight lanes per row, which do with it
 // what the prologue does.
 // RES: the workgroup's rows are in LDS whole (K up to 1024), normalised ahead of the product.  Otherwise the rows, not to be
-// normalised, stream beside the weights.  (Streaming workgroups that start at different places of K, so that they are not all at
-// the same bytes of rows a multiple of the caches' interleave apart: 300 rows x 16 heads at K = 3072 out of memory 21.7 / 17.8 us,
-// but then the order of a row's sums depends on its place among the rows.)
+// normalised, stream beside the weights.  All workgroups then walk K in step, at the same bytes of weight rows that are a multiple
+// of the caches' interleave apart, i.e. on one or two channels; so the workgroups of a head first touch a piece of K each of its weights
+// (they are on one XCD: its L2 then has or awaits the lines, from all channels): 300 rows x 16 heads at K = 3072, weights out of memory,
+// 21.7 -> 17.7 us, 100 rows 20.5 -> 19.4, out of L2 the same 15.5.  (Walking K from different places gains as much, 17.8, but the order of
+// a row's sums then depends on its place among the rows.)
 #include "attn_common.h"
 #include "row_ops.h"
 
@@ -185,7 +187,8 @@ __global__ __launch_bounds__(64 * NW, 1) void small_proj_kernel(const SmallProjK
       sW4[NST > 4 ? STAGE_W : 16], sW5[NST > 5 ? STAGE_W : 16];
   __shared__ __attribute__((aligned(1024))) unsigned char sX0[STAGE_X], sX1[STAGE_X], sX2[STAGE_X], sX3[STAGE_X], sX4[STAGE_X], sX5[STAGE_X];
   __shared__ __attribute__((aligned(1024))) unsigned char sR[RES ? ROWS * (2 * res_max_k<ROWS>() + 16) : 16];
-  static_assert(NST * (STAGE_X + STAGE_W) + (int)sizeof(sR) <= LDS_MAX - 512, "LDS");
+  __shared__ __attribute__((aligned(1024))) unsigned char sT[RES ? 16 : NW * 256];
+  static_assert(NST * (STAGE_X + STAGE_W) + (int)sizeof(sR) + (int)sizeof(sT) <= LDS_MAX - 512, "LDS");
   const int tid = threadIdx.x;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l = tid & 63, n = l & 15, g = l >> 4;
@@ -225,6 +228,13 @@ __global__ __launch_bounds__(64 * NW, 1) void small_proj_kernel(const SmallProjK
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, LDS_PTR(void, X + (w + 4) * 1024), 16, vx2, (int)((unsigned)step * (BK * 2)), 0, 0);
     }
   };
+  if constexpr (!RES) {  // the touches: four bytes of each row and stage, a line per lane, into LDS that nothing reads
+    const int tiles = (rows + ROWS - 1) / ROWS, end = (int)((long)steps * (tile + 1) / tiles);
+    for (int st = (int)((long)steps * tile / tiles) + w; st < end; st += NW)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, LDS_PTR(void, sT + w * 256), 4, (unsigned)(64 * j + l) * (unsigned)(K * 2), st * (BK * 2), 0, 0);
+  }
   RowParams<ROWS / 32> params;
   load_row_params(a, params, text, head, row0, rows, tid);
   load(0, sW0, sX0);
