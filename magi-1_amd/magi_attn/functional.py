@@ -88,16 +88,6 @@ def covered_by_launch(n: int, max_seqlen_q: int, rows: int) -> bool:
     return 1 <= n <= 64 and max_seqlen_q > 0 and n * max_seqlen_q >= rows
 
 
-def split_scratch_bytes(Hq: int, Hkv: int, n: int, max_seqlen_q: int, max_seqlen_k: int, dtype: int, whole_tiles: bool = False) -> int:
-    """Scratch memory with which a launch of these sizes shares keys among workgroups, 0 where it does not: bf16 launches in 128-row
-    workgroups make no use of it (whole_tiles: the launch is in 256-row ones whatever its sizes)."""
-    n = max(n, 0)
-    need = L.lib().magi_attn_split_bytes(Hq, Hkv, n, max_seqlen_q, max_seqlen_k, dtype)
-    if need and dtype == L.MAGI_DTYPE_BF16 and not whole_tiles and L.lib().magi_attn_tile_rows(Hq, Hkv, n, max_seqlen_q, max_seqlen_k, need) == 128:
-        return 0
-    return need
-
-
 def launch_bounded_attention(dev: torch.device, q: int, q_row: int, rows: int, Hq: int, kv: int, side: int, k_split: int, total_k: int,
                              kv_row: int, Hkv: int, q_ranges: torch.Tensor, k_ranges: torch.Tensor, n: int, mode: int, max_seqlen_q: int,
                              max_seqlen_k: int, out: int, o_row: int, group_heads: int, o_group: int, clear: bool, bound: float,
@@ -109,7 +99,9 @@ def launch_bounded_attention(dev: torch.device, q: int, q_row: int, rows: int, H
     max_seqlen_q, max_seqlen_k = int(max_seqlen_q), int(max_seqlen_k)
     split, split_bytes = None, 0
     if max_seqlen_k >= 512:
-        split_bytes = split_scratch_bytes(Hq, Hkv, n, max_seqlen_q, max_seqlen_k, L.MAGI_DTYPE_BF16)
+        split_bytes = L.lib().magi_attn_split_bytes(Hq, Hkv, max(n, 0), max_seqlen_q, max_seqlen_k, L.MAGI_DTYPE_BF16)
+        if split_bytes and L.lib().magi_attn_tile_rows(Hq, Hkv, n, max_seqlen_q, max_seqlen_k, split_bytes) == 128:
+            split_bytes = 0  # (in 128-row workgroups the launch makes no use of it)
         if split_bytes:
             split = torch.empty(split_bytes, dtype=torch.uint8, device=dev)
     q_ranges, k_ranges = q_ranges.contiguous(), k_ranges.contiguous()
@@ -259,7 +251,10 @@ def range_attention(
     split, split_bytes = None, 0
     if split_keys and not static_scratch and max_seqlen_k >= 512 and (
             checked or auto_bound or 0.0 < score_bound <= L.MAGI_SCORE_BOUND_MAX or q.dtype is torch.float8_e4m3fn):
-        split_bytes = split_scratch_bytes(Hq, Hkv, n, int(max_seqlen_q), int(max_seqlen_k), _dtype_code(q), checked or bool(q_tile_rows))
+        split_bytes = L.lib().magi_attn_split_bytes(Hq, Hkv, max(n, 0), int(max_seqlen_q), int(max_seqlen_k), _dtype_code(q))
+        if split_bytes and not (checked or q_tile_rows) and q.dtype is torch.bfloat16 and L.lib().magi_attn_tile_rows(
+                Hq, Hkv, n, int(max_seqlen_q), int(max_seqlen_k), split_bytes) == 128:
+            split_bytes = 0  # (in 128-row workgroups the launch makes no use of it)
         if split_bytes:  # (no going on without it where memory is short: the same call would give other bits then)
             split = torch.empty(split_bytes, dtype=torch.uint8, device=q.device)
     gamma = beta = None  # (alive until the launch is enqueued)

@@ -245,17 +245,21 @@ def _projects_in_one_launch(rows: int, heads: int, text_rows: int, text_heads: i
 
 def _text_in_one_launch(flop: float, rows: int, heads: int, K: int, cus: int) -> bool:
     """Whether the K | V projection of the text rows and the K norm run as one launch of small_projections rather than as the library's
-    product and a head norm.  The host takes 8.5 instead of 29 us for it, which counts where the layer is waiting for it; on the device
-    (K = 3072, 16 heads, weights out of memory, norm and product / this launch) 100 rows take 14.7 / 20.5 us, 200 rows 19.9 / 21.1, 300
-    rows 21.1 / 21.8, 512 rows 21.3 / 23.3.  Whole layers of 24 heads: 468 rows over 2340 keys (3.1e10 flop) 151 / 132 us, two chunks of 648 rows
-    with 348 text rows (9e10) 162 / 160, 900 rows over 4500 keys in fp8 with 300 (8.4e10) 268 / 247; from 7e10 on with fewer than 200 text rows
-    924 over 4620 in fp8 191 / 198; 1710 rows over 13680 keys with 302 356 / 356.  In one round of its workgroups (32 rows x one of the
-    `heads`): more rows (64 a workgroup then) gain nothing, four chunks of 1170 rows with 674 in all 374 / 376.  At K = 6144 the
-    product is the faster one (400 rows 25 / 29 us).
+    product and a head norm.  The host takes 8.5 instead of 29 us for it, which counts where the layer is waiting for it: whole layers of
+    24 heads, 468 rows over 2340 keys (3.1e10 flop) 151 / 132 us, two chunks of 648 rows with 348 text rows (9e10) 162 / 160, 900 rows over 4500
+    keys in fp8 with 300 (8.4e10) 268 / 247; from 7e10 on with fewer than 200 text rows 924 over 4620 in fp8 191 / 198.  In one round of its
+    workgroups (32 rows x one of the `heads`): more rows (64 a workgroup then) gain nothing, four chunks of 1170 rows with 674 in
+    all 374 / 376.  At K = 6144 the product is the faster one (400 rows 25 / 29 us).
     Up to 2^17 results of a long sum the library cuts K in pieces (64 rows at 16 heads, 128 at 8): another order of the sums, other bits.
-    Those layers keep the library's, and so do those captured into a graph, which wait for no host, unless K is at most 1024 (100 rows at
-    K = 768 and 4 heads 10.3 / 7.7 us, 300 at 1024 and 16 12.6 / 9.3)."""
+    Those layers keep the library's."""
     return (flop < 7e10 or rows >= 200) and K <= 3072 and (K <= 1024 or rows * heads > 1024) and (rows + 31) // 32 * heads <= cus
+
+
+def _text_waits_for_the_host(rows: int, heads: int, K: int) -> bool:
+    """Whether it is for the host alone that the text rows are better off in one launch; a captured stream waits for no host.  On the device,
+    weights out of memory, norm and product / one launch: K = 768 and 4 heads 10.3 / 7.7 us with 100 rows; K = 3072 and 16 heads 14.5 / 19.4
+    with 100, 19.8 / 18.6 with 130, 21.1 / 17.7 with 300, 8 heads 14.1 / 17.6 with 200 and 19.0 / 17.1 with 300: up to 2^18 results."""
+    return K > 1024 and rows * heads <= 2048
 
 
 def _global_hooks() -> bool:
@@ -1073,9 +1077,12 @@ class FullyParallelAttention(torch.nn.Module):
             if bs > 1 and not own_cross:  # (a replaced cross attention runs; at batch 1 with a bound in force it never did)
                 return None
             flop = 512.0 * sq * Hq * (hidden_states.shape[2] + p.max_seqlen_k)
-            own_text = (bs == 1 and key_value_states.dim() == 2 and hidden_states.is_cuda and _OWN_SMALL.of(self) and _text_in_one_launch(
-                flop, key_value_states.shape[0], 2 * self.num_query_groups_per_partition, key_value_states.shape[1],
-                _compute_units(hidden_states.device)) and (key_value_states.shape[1] <= 1024 or not torch.cuda.is_current_stream_capturing()))
+            text_rows, heads = key_value_states.shape[0], 2 * self.num_query_groups_per_partition
+            own_text = (bs == 1 and key_value_states.dim() == 2 and hidden_states.is_cuda
+                        and "_cross_attention_fused" not in self.__dict__ and type(self)._cross_attention_fused is _CROSS_FUSED
+                        and _text_in_one_launch(flop, text_rows, heads, key_value_states.shape[1], _compute_units(hidden_states.device)))
+            if own_text and _text_waits_for_the_host(text_rows, heads, key_value_states.shape[1]) and torch.cuda.is_current_stream_capturing():
+                own_text = False
             more = {"own_text": True} if own_text else {}  # (one put in its place may not know it)
             return self._cross_attention_fused(qx_raw, sq, bs, key_value_states, meta_args.cross_attn_params, dst, bound_cross, **more)
 
@@ -1157,5 +1164,6 @@ _OWN_FP8_LINEAR = _Own(PerTensorQuantizedFp8Linear, "forward")
 _OWN_PROJECTIONS = _Own(CustomLayerNormLinear, "forward_ln", "forward_qkvx")
 _OWN_SMALL_PROJECTIONS = _Own(CustomLayerNormLinear, "forward_ln", "forward_qkvx", "forward_ln_qkvx_rows", "_split")
 _OWN_CROSS = _Own(FullyParallelAttention, "get_xqkv", "cross_attention")
+_CROSS_FUSED = FullyParallelAttention._cross_attention_fused
 _OWN_SMALL = _Own(FullyParallelAttention, "_project_rows", "_fused_qkv", "_cross_attention_fused")
 _OWN_SMALL_UNCACHED = _Own(FullyParallelAttention, "_project_rows", "_fused_qkv", "_cross_attention_fused", "core_attention")

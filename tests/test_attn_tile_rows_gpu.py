@@ -5,7 +5,6 @@ import torch
 
 import magi_attn as M
 from magi_attn import _lib as L
-from magi_attn import functional as F
 
 D, PRE = 128, 128 ** -0.5 * 1.4426950408889634
 
@@ -88,27 +87,27 @@ def test_which_launches_take_the_smaller_workgroups(dev, rows, n, prefix, Hq, Hk
     assert not (smaller and any("merge" in x for x in names)), names
 
 
-# rows per range, ranges, cached ranges, with scratch memory: as above
-@pytest.mark.parametrize("rows,n,prefix,Hq,Hkv,split,smaller", [
-    (240, 2, 2, 6, 2, True, True), (2600, 1, 0, 24, 8, True, True), (3800, 1, 0, 24, 8, True, False), (240, 1, 13, 24, 8, True, False),
-    (240, 1, 13, 24, 8, False, True), (2600, 1, 4, 24, 8, True, True), (1300, 1, 3, 24, 8, True, False), (1000, 3, 2, 24, 8, True, False)])
-def test_smaller_workgroups_come_without_scratch_memory(rows, n, prefix, Hq, Hkv, split, smaller):
-    if torch.cuda.is_available() and torch.cuda.get_device_properties(0).multi_processor_count != 256:
-        pytest.skip("the sizes are chosen for 256 CUs")
-    size = (Hq, Hkv, n, rows, (n + prefix) * rows)
-    asked = L.lib().magi_attn_split_bytes(*size, L.MAGI_DTYPE_BF16)
-    assert (L.lib().magi_attn_tile_rows(*size, asked if split else 0) == 128) == smaller
-    assert F.split_scratch_bytes(*size, L.MAGI_DTYPE_BF16) == (0 if smaller and split else asked)
-    assert F.split_scratch_bytes(*size, L.MAGI_DTYPE_BF16, whole_tiles=True) == asked  # (checked, or the workgroups stated)
-
-
 @pytest.mark.gpu
-def test_a_launch_of_smaller_workgroups_allocates_its_output_only(dev, monkeypatch):
-    rows, Tk = 2600, 13000  # (70 MB in pieces of 256-row workgroups)
-    q, kv = (torch.randn(r, h, 2 * D, device=dev, dtype=torch.bfloat16) * 0.1 for r, h in ((rows, 24), (Tk, 8)))
+@pytest.mark.parametrize("rows,n,prefix,Hq,Hkv,smaller", [(2600, 1, 4, 24, 8, True), (1300, 1, 3, 24, 8, False)])
+def test_launches_of_smaller_workgroups_allocate_no_scratch_memory(dev, monkeypatch, rows, n, prefix, Hq, Hkv, smaller):
+    """As the library says which they are; checked launches, in 256-row workgroups always, do."""
+    if torch.cuda.get_device_properties(dev).multi_processor_count != 256:
+        pytest.skip("the sizes are chosen for 256 CUs")
+    Tk = (n + prefix) * rows
+    size = (Hq, Hkv, n, rows, Tk)
+    asked = L.lib().magi_attn_split_bytes(*size, L.MAGI_DTYPE_BF16)
+    assert asked > 0 and (L.lib().magi_attn_tile_rows(*size, asked) == 128) == smaller and L.lib().magi_attn_tile_rows(*size, 0) == 128
+    q, kv = (torch.randn(r, h, 2 * D, device=dev, dtype=torch.bfloat16) * 0.1 for r, h in ((rows, Hq), (Tk, Hkv)))
     qr, kr = (torch.tensor([[0, e]], dtype=torch.int32, device=dev) for e in (rows, Tk))
-    call = lambda **kw: M.range_attention(q[..., :D], kv[..., :D], kv[..., D:], qr, kr, rows, Tk, q_prescaled=True, score_bound=60.0,  # noqa: E731
-                                          return_lse=False, **kw)[0]
-    want, real = call(split_keys=False), torch.empty
-    monkeypatch.setattr(torch, "empty", lambda *a, **kw: pytest.fail("scratch memory") if kw.get("dtype") is torch.uint8 else real(*a, **kw))
-    assert torch.equal(call(), want)
+    call = lambda **kw: M.range_attention(q[..., :D], kv[..., :D], kv[..., D:], qr, kr, rows, Tk, return_lse=False, **kw)[0]  # noqa: E731
+    whole, real, got = call(split_keys=False, score_bound=60.0), torch.empty, []
+
+    def empty(*a, **kw):
+        if kw.get("dtype") is torch.uint8:
+            got.append(a[0])
+        return real(*a, **kw)
+
+    monkeypatch.setattr(torch, "empty", empty)
+    assert torch.equal(call(score_bound=60.0), whole) == smaller and got == ([] if smaller else [asked])
+    call(checked=True)
+    assert got[-1] == asked

@@ -381,6 +381,8 @@ def test_which_layers_take_the_one_launch():
     text = MOD._text_in_one_launch
     assert text(6e10, 512, 16, 3072, cus) and not text(6e10, 513, 16, 3072, cus) and text(6e10, 2048, 4, 768, cus)
     assert text(6e10, 65, 16, 3072, cus) and not text(6e10, 64, 16, 3072, cus) and text(6e10, 3, 4, 1024, cus)  # (where the library cuts K)
+    waits = MOD._text_waits_for_the_host
+    assert waits(128, 16, 3072) and not waits(129, 16, 3072) and not waits(3, 4, 1024)
     assert not text(6e10, 100, 16, 6144, cus) and not text(8e10, 199, 16, 3072, cus) and text(8e10, 200, 16, 3072, cus)
 
 
