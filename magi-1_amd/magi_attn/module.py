@@ -232,15 +232,17 @@ def _compute_units(device: torch.device) -> int:
     return n
 
 
-def _projects_in_one_launch(rows: int, heads: int, text_rows: int, text_heads: int, K: int, cus: int, captured: bool = False) -> bool:
+def _projects_in_one_launch(rows: int, heads: int, text_rows: int, text_heads: int, K: int, cus: int) -> bool:
     """Whether a layer's projections run as one launch of small_projections: where its workgroups (32 rows x one head each, 64 rows up
     to K = 768) are one round, or up to four of the taller ones.  In one round the launch takes less time than the norm, the library's
     two products, the prologue and the text's head norm (K = 768, 20 + 4 heads, 24 text rows: 240 rows 11.6 / 22.1 us, 768 rows 17.8 / 25.7), in
     several more (840 rows 29.6 / 26.9, 1344 32.7 / 30.4, 2048 48.1 / 35.7), but the host issues the layer 80 us sooner and such layers wait
     for it: 840 rows over 1260 keys 68 / 150 us in all, 1344 over 2688 76 / 154, 2048 over 6144 118 / 154.
-    captured: into a graph, where no host is waited for: one round only (the same layers replayed 70 / 71, 79 / 77, 120 / 108 us)."""
+    Replayed from a graph, which waits for no host, the same layers take 70 / 71, 79 / 77, 120 / 108 us.  The choice does not look at whether the
+    stream is being captured all the same: an eager pass ahead of the capture would not have brought the library's product up, and
+    bringing it up is not permitted in a capture."""
     tile = lambda n: ((rows + n - 1) // n) * heads + ((text_rows + n - 1) // n) * text_heads  # noqa: E731
-    return tile(64) <= (1 if captured else 4) * cus if K <= 768 else tile(32) <= cus
+    return tile(64) <= 4 * cus if K <= 768 else tile(32) <= cus
 
 
 def _text_in_one_launch(flop: float, rows: int, heads: int, K: int, cus: int) -> bool:
@@ -251,15 +253,11 @@ def _text_in_one_launch(flop: float, rows: int, heads: int, K: int, cus: int) ->
     workgroups (32 rows x one of the `heads`): more rows (64 a workgroup then) gain nothing, four chunks of 1170 rows with 674 in
     all 374 / 376.  At K = 6144 the product is the faster one (400 rows 25 / 29 us).
     Up to 2^17 results of a long sum the library cuts K in pieces (64 rows at 16 heads, 128 at 8): another order of the sums, other bits.
-    Those layers keep the library's."""
+    Those layers keep the library's.
+    On the device, weights out of memory, norm and product / this launch: K = 768 and 4 heads 10.3 / 7.7 us with 100 rows; K = 3072 and 16 heads
+    14.5 / 19.4 with 100, 19.8 / 18.6 with 130, 21.1 / 17.7 with 300, 8 heads 14.1 / 17.6 with 200 and 19.0 / 17.1 with 300: it is the
+    host's time that decides up to 2^18 results, in a captured stream too (see _projects_in_one_launch)."""
     return (flop < 7e10 or rows >= 200) and K <= 3072 and (K <= 1024 or rows * heads > 1024) and (rows + 31) // 32 * heads <= cus
-
-
-def _text_waits_for_the_host(rows: int, heads: int, K: int) -> bool:
-    """Whether it is for the host alone that the text rows are better off in one launch; a captured stream waits for no host.  On the device,
-    weights out of memory, norm and product / one launch: K = 768 and 4 heads 10.3 / 7.7 us with 100 rows; K = 3072 and 16 heads 14.5 / 19.4
-    with 100, 19.8 / 18.6 with 130, 21.1 / 17.7 with 300, 8 heads 14.1 / 17.6 with 200 and 19.0 / 17.1 with 300: up to 2^18 results."""
-    return K > 1024 and rows * heads <= 2048
 
 
 def _global_hooks() -> bool:
@@ -907,8 +905,7 @@ class FullyParallelAttention(torch.nn.Module):
             return None
         dev = hidden_states.device
         Hq, Hkv, D, (T, Kt) = self.num_attention_heads, self.num_query_groups_per_partition, 128, key_value_states.shape
-        size = (S, 2 * (Hq + Hkv), T, 2 * Hkv, max(K, Kt), _compute_units(dev))
-        if Kt > 1024 or not (_projects_in_one_launch(*size, True) or (_projects_in_one_launch(*size) and not torch.cuda.is_current_stream_capturing())):
+        if Kt > 1024 or not _projects_in_one_launch(S, 2 * (Hq + Hkv), T, 2 * Hkv, max(K, Kt), _compute_units(dev)):
             return None
         m = self._modules
         lin = m["linear_qkv"]
@@ -1081,8 +1078,6 @@ class FullyParallelAttention(torch.nn.Module):
             own_text = (bs == 1 and key_value_states.dim() == 2 and hidden_states.is_cuda
                         and "_cross_attention_fused" not in self.__dict__ and type(self)._cross_attention_fused is _CROSS_FUSED
                         and _text_in_one_launch(flop, text_rows, heads, key_value_states.shape[1], _compute_units(hidden_states.device)))
-            if own_text and _text_waits_for_the_host(text_rows, heads, key_value_states.shape[1]) and torch.cuda.is_current_stream_capturing():
-                own_text = False
             more = {"own_text": True} if own_text else {}  # (one put in its place may not know it)
             return self._cross_attention_fused(qx_raw, sq, bs, key_value_states, meta_args.cross_attn_params, dst, bound_cross, **more)
 
