@@ -235,6 +235,10 @@ typedef struct magi_attn_args {
  * a call is not split. */
 int64_t magi_attn_split_bytes(int32_t Hq, int32_t Hkv, int32_t n_ranges, int32_t max_seqlen_q, int32_t max_seqlen_k, int32_t dtype);
 
+/* The same for a bf16 call of these sizes that runs the online softmax in 128-row workgroups (no score_bound in force, no
+ * MAGI_ATTN_AUTO_BOUND, no MAGI_ATTN_CHECKED, no MAGI_ATTN_Q_PRESCALED, q_tile_rows 0 or 128). */
+int64_t magi_attn_online_split_bytes(int32_t Hq, int32_t Hkv, int32_t n_ranges, int32_t max_seqlen_q, int32_t max_seqlen_k);
+
 /* Rows per workgroup that a bf16 call of these sizes takes with a score_bound in force (or measured and in force), q_tile_rows 0, no
  * MAGI_ATTN_CHECKED and this much split_workspace: 256, or 128 where these fill the chip better, which make no use of that memory.  A row's
  * bits are those of 256-row workgroups without it. */

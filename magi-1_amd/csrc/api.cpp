@@ -160,6 +160,78 @@ SplitPlan split_plan(unsigned items, int n_ranges, int max_seqlen_q, int max_seq
   return s;
 }
 
+// Whether and how a launch of the online softmax in 128-row workgroups shares the keys of its items (AttnKernArgs::share_*): every
+// item in pieces of the same number of tiles, a workgroup each, and a launch behind it that brings them together.
+struct SharePlan {
+  unsigned pieces, tiles;  // of the longest item, of a piece
+  int64_t bytes(unsigned per_xcd) const { return pieces > 1 ? 4ll * magi::ONLINE_PARTIAL_FLOATS * 8 * per_xcd * pieces : 0; }
+};
+// What a launch in pieces of `cut` tiles takes, in us.  A tile of 64 keys takes a workgroup 1.36 us alone on its CU, 1.9 beside
+// another, 2.55 beside two; a launch 9 us besides; bringing pieces together 5 us and 18 ns each (their way through memory).  Workgroups
+// that fit the chip at once run side by side until the shortest are done, and so on; more of them keep it full but for the end.
+double share_us(unsigned items, const unsigned* lengths, int n_ranges, unsigned cut, unsigned cus) {
+  unsigned len[2 * 16], count[2 * 16];  // the pieces, by length
+  int kinds = 0;
+  auto add = [&](unsigned l, unsigned c) {
+    int i = 0;
+    while (i < kinds && len[i] < l) ++i;
+    if (i < kinds && len[i] == l) {
+      count[i] += c;
+      return;
+    }
+    for (int k = kinds++; k > i; --k) len[k] = len[k - 1], count[k] = count[k - 1];
+    len[i] = l, count[i] = c;
+  };
+  const unsigned each = items / (unsigned)n_ranges;
+  double all = 0, parts = 0, work = 0;
+  for (int r = 0; r < n_ranges; ++r) {
+    const unsigned whole = lengths[r] / cut, rest = lengths[r] % cut;
+    if (whole) add(cut, whole * each);
+    if (rest) add(rest, each);
+    const unsigned n = whole + (rest != 0);
+    all += (double)n * each;
+    work += (double)lengths[r] * each;
+    if (n > 1) parts += (double)n * each;
+  }
+  auto tile_us = [](double on_a_cu) {
+    return on_a_cu <= 1 ? 1.36 : on_a_cu <= 2 ? 1.36 + 0.54 * (on_a_cu - 1) : on_a_cu <= 3 ? 1.9 + 0.65 * (on_a_cu - 2) : 2.55;
+  };
+  double t = 9.0;
+  if (all > 3.0 * cus) {
+    t += 2.55 * (work / (3.0 * cus) + 0.25 * cut);
+  } else {
+    double left = all;
+    for (int i = 0; i < kinds; left -= count[i++])
+      t += (len[i] - (i ? len[i - 1] : 0)) * tile_us(i + 1 < kinds ? left / cus : std::ceil(left / cus));
+  }
+  return parts > 0 ? t + 5.0 + 0.018 * parts : t;
+}
+// Measured, whole / in pieces: 24 items over 127 tiles 181 / 41 us, 126 over 332 455 / 186, 180 over 592 and less 795 / 428, 240 over 180 257
+// / 195, 336 over 136 265 / 210, 576 over 378 981 / 846; not cut, 384 over 16 and 32 57 / 62, 528 over 44 and 66 151 / 159, 864 over 24 to
+// 72 178 / 193, 1728 over 54 to 108 543 / 565.  The host does not know the ranges' lengths: taken are ranges that end a chunk of
+// max_seqlen_q keys apart, or all of max_seqlen_k keys where that does not go.  Only where the estimate is 6 % shorter, 10 % behind a whole round
+// (864 items over 86 to 111 tiles 402 / 410), and from 20 tiles on: max_seqlen_k of text is the padded length, of which a call may fill a fraction.
+SharePlan share_plan(unsigned per_xcd, int n_ranges, int max_seqlen_q, int max_seqlen_k) {
+  SharePlan best = {1, 0};
+  const unsigned cus = (unsigned)compute_units(), longest = (unsigned)(max_seqlen_k + 63) / 64, items = 8 * per_xcd;
+  if (max_seqlen_k <= 0 || longest < 20 || n_ranges < 1 || n_ranges > 16 || items == 0 || items > 6 * cus) return best;
+  unsigned lengths[16];
+  const bool apart = max_seqlen_k > (int64_t)(n_ranges - 1) * max_seqlen_q;
+  for (int r = 0; r < n_ranges; ++r) lengths[r] = apart ? (unsigned)(max_seqlen_k - r * max_seqlen_q + 63) / 64 : longest;
+  double least = (items > 3 * cus ? 0.90 : 0.94) * share_us(items, lengths, n_ranges, longest, cus);
+  static const unsigned char tried[] = {2, 3, 4, 5, 6, 8, 10, 12, 16};
+  for (unsigned pieces : tried) {
+    const unsigned cut = (longest + pieces - 1) / pieces;
+    if (cut < 3 || (double)items * pieces > 8.0 * cus) break;
+    const double us = share_us(items, lengths, n_ranges, cut, cus);
+    if (us < least) {
+      least = us;
+      best = {(longest + cut - 1) / cut, cut};
+    }
+  }
+  return best;
+}
+
 // How a launch of the 64-rows-per-wavefront kernel without a running maximum is cut: workgroups of 256 rows, their last round's
 // items sharing keys where that pays and the caller has brought the memory, or workgroups of 128 rows
 // (32 per wavefront; a row's bits are the same).  Those fetch and read every tile for half the rows, so they are only for launches
@@ -213,6 +285,13 @@ int64_t magi_attn_split_bytes(int32_t Hq, int32_t Hkv, int32_t n_ranges, int32_t
   if ((double)Hq * n_ranges * tiles > 2.0e9) return 0;
   const unsigned items = items_per_xcd(Hq, Hkv, n_ranges, tiles);
   return split_plan(items, n_ranges, max_seqlen_q, max_seqlen_k, fp8).bytes(items);
+}
+
+int64_t magi_attn_online_split_bytes(int32_t Hq, int32_t Hkv, int32_t n_ranges, int32_t max_seqlen_q, int32_t max_seqlen_k) {
+  if (Hq <= 0 || Hkv <= 0 || Hq % Hkv || n_ranges <= 0 || max_seqlen_q <= 0) return 0;
+  if ((double)Hq * n_ranges * (max_seqlen_q / 128 + 1) > 2.0e9) return 0;
+  const unsigned items = items_per_xcd(Hq, Hkv, n_ranges, max_seqlen_q / 128 + (max_seqlen_q % 128 != 0));
+  return share_plan(items, n_ranges, max_seqlen_q, max_seqlen_k).bytes(items);
 }
 
 int32_t magi_attn_tile_rows(int32_t Hq, int32_t Hkv, int32_t n_ranges, int32_t max_seqlen_q, int32_t max_seqlen_k,
@@ -463,6 +542,19 @@ int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace) {
         a.split_den = s.den;
       }
     }
+    // The online softmax on unscaled q, 128 rows a workgroup: the 16x16x32 form for launches of more workgroups than run at a time
+    // (three per CU) and for shared keys, the 32x32x16 form for the others.  Measured, 32x32x16 / 16x16x32: 9360 rows x 2
+    // chunks x 24 heads over 28080 and 37440 keys 6604 / 6407 us, 93600 x 24 text cross attention 612 / 600, over 20 keys 223 / 202,
+    // 4580 x 48 over 3435 to 6870 555 / 545; 700 x 24 over 700 22.3 / 23.2, 700 x 48 over 1400 48.5 / 50.7, 2000 x 24 57 / 58.
+    const bool online128 = !fp8 && !bounded && a.block_m == 128 && !(p->flags & MAGI_ATTN_Q_PRESCALED);
+    if (online128 && !a.gate && split_bytes > 0) {
+      const SharePlan s = share_plan(a.per_xcd, p->n_ranges, p->max_seqlen_q, p->max_seqlen_k);
+      if (s.pieces > 1 && s.bytes(a.per_xcd) <= split_bytes) {
+        a.partial = static_cast<float*>(p->split_workspace);
+        a.share_pieces = s.pieces;
+        a.share_tiles = s.tiles;
+      }
+    }
     hipError_t e;
     if (p->dtype != MAGI_DTYPE_BF16)
       e = magi::launch_attn_fwd_fp8(a, static_cast<hipStream_t>(stream));
@@ -472,10 +564,12 @@ int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace) {
       e = magi::launch_attn_fwd_bf16_x16(a, static_cast<hipStream_t>(stream));
     else if (bounded)
       e = magi::launch_attn_fwd_bf16_w64(a, static_cast<hipStream_t>(stream));
+    else if (online128 && (a.share_pieces > 1 || 8.0 * a.per_xcd > 3.0 * compute_units()))
+      e = magi::launch_attn_fwd_bf16_online16(a, static_cast<hipStream_t>(stream));
     else
       e = magi::launch_attn_fwd_bf16(a, static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return hip_fail(e, "magi_attn_fwd launch");
-    g_launches.fetch_add((checked ? 2 : 1) + (a.split_from < a.per_xcd), std::memory_order_relaxed);
+    g_launches.fetch_add((checked ? 2 : 1) + (a.split_from < a.per_xcd) + (a.share_pieces > 1), std::memory_order_relaxed);
     return MAGI_OK;
   };
 

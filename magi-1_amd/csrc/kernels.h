@@ -53,7 +53,12 @@ struct AttnKernArgs {
   // p - 1) / split_den of the item's key range, piece 0 at tile 0.  `partial`: SPLIT_FLOATS floats per piece.
   float* partial;
   unsigned split_from, split_pieces, split_num, split_den;  // split_from: UINT_MAX = nothing is split
+  // Online softmax, 128-row workgroups: the keys of every item in up to share_pieces pieces of share_tiles tiles each (0 or 1:
+  // whole; `partial`: ONLINE_PARTIAL_FLOATS floats per item and piece).
+  unsigned share_pieces, share_tiles;
 };
+// online softmax: 128 rows x 128 accumulators, 128 row sums, 128 row maxima
+constexpr int ONLINE_PARTIAL_FLOATS = 128 * 128 + 256;
 // 256 rows x 128 accumulators, and the 256 row sums behind them
 constexpr int SPLIT_FLOATS = 256 * 128 + 256;
 // fp8: 128 rows x 128 accumulators, 128 row sums, 128 row maxima
@@ -74,6 +79,7 @@ constexpr int ATTN_SCALE_Q = 1 << 9;
 constexpr int ATTN_ZERO_GAPS = 32;
 
 hipError_t launch_attn_fwd_bf16(const AttnKernArgs& a, hipStream_t stream);
+hipError_t launch_attn_fwd_bf16_online16(const AttnKernArgs& a, hipStream_t stream);
 hipError_t launch_attn_fwd_bf16_w64(const AttnKernArgs& a, hipStream_t stream);
 // (with items to split: and behind it the launch that adds their pieces up)
 hipError_t launch_attn_fwd_bf16_x16(const AttnKernArgs& a, hipStream_t stream);

@@ -255,8 +255,11 @@ def range_attention(
         if split_bytes and not (checked or q_tile_rows) and q.dtype is torch.bfloat16 and L.lib().magi_attn_tile_rows(
                 Hq, Hkv, n, int(max_seqlen_q), int(max_seqlen_k), split_bytes) == 128:
             split_bytes = 0  # (in 128-row workgroups the launch makes no use of it)
-        if split_bytes:  # (no going on without it where memory is short: the same call would give other bits then)
-            split = torch.empty(split_bytes, dtype=torch.uint8, device=q.device)
+    elif (split_keys and not static_scratch and max_seqlen_k >= 512 and q.dtype is torch.bfloat16 and not (auto_bound or q_prescaled)
+          and q_tile_rows in (0, 128)):
+        split_bytes = L.lib().magi_attn_online_split_bytes(Hq, Hkv, max(n, 0), int(max_seqlen_q), int(max_seqlen_k))
+    if split_bytes:  # (no going on without it where memory is short: the same call would give other bits then)
+        split = torch.empty(split_bytes, dtype=torch.uint8, device=q.device)
     gamma = beta = None  # (alive until the launch is enqueued)
     norm_eps, norm_kind = 0.0, 0
     if q_norm is not None:
