@@ -3,11 +3,11 @@
 // What attn_fwd_bf16.hip's 4-wave form computes, on unscaled q: 128-row workgroups, three per CU, 64-key tiles, two K slots and one
 // V slot filled by direct global->LDS loads.  The MFMA shape, its operand layouts and the layout of the tiles in LDS are those of
 // attn_fwd_bf16_x16.hip (there: why that shape, and the reads' banks), with two query blocks of 16 per wavefront instead of four.
-// 162 registers.  What bounds it: per tile and wavefront the matrix pipe has 1024 cycles of work, the LDS 32 KB of operand reads,
+// 164 registers.  What bounds it: per tile and wavefront the matrix pipe has 1024 cycles of work, the LDS 32 KB of operand reads,
 // the vector pipe 32 exponentials and 100 other instructions, about as long each; long launches run at the power limit, where the
 // 16x16x32 shape takes less energy per FLOP: 9360 rows x 2 chunks x 24 heads over 28080 and 37440 keys 6407 us against the 6604 of the
 // 32x32x16 form (1.18 PFLOP/s).  Whole rows go out through LDS, 16 lanes a row: 74880 x 24 rows over 20 keys, which is mostly the way
-// of q and out, 223 -> 202 us.
+// of q and out, 223 -> 202 us, and 174 with the first tile requested ahead of q.
 //
 // Shared keys (SHARE).  A launch of few items leaves most of the chip idle: 24 items over 127 tiles take 127 tiles in a row, 181 us.
 // Their keys are cut in pieces of a.share_tiles tiles, a workgroup each; a piece leaves unnormalised accumulators, row sums
@@ -145,7 +145,12 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_bf16_online16_kernel(const At
     }
   };
 
-  issue_mat(ks, sK0, false);
+  // The LAST tile of the range goes first: it may be ragged, so it has a copy of the tile's code of its own, which also knows that there
+  // is no maximum yet, and the others' code has neither.  It is on its way into LDS, V too, while q is loaded.  (The text cross attention,
+  // a few tiles: 93600 x 24 rows 511 -> 509 us, 42196 x 24 over 115 keys 137 -> 133, 74880 x 24 over 64 keys 194 -> 187, over 20 191 -> 174.)
+  const int last = (ke - ks - 1) / BN;
+  issue_mat(ks + last * BN, sK0, false);
+  issue_mat(ks + last * BN, sV, true);
 
   // ---- Q fragments (B operand of S^T = K Q^T): lane (n, g) holds Q[row 16 qb + n][32 kk + 8 g .. +8] ----
   bf16x8 qf[QB][4];
@@ -170,8 +175,10 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_bf16_online16_kernel(const At
   float m_run[QB] = {-__builtin_inff(), -__builtin_inff()};  // running maxima of the raw scores
   const float c = a.scale_log2;
   const f32x4v zero4 = {0.f, 0.f, 0.f, 0.f};
+  const f32x4v none4 = {-__builtin_inff(), -__builtin_inff(), -__builtin_inff(), -__builtin_inff()};
 
-  auto compute_tile = [&](const unsigned char* Kt, const unsigned char* Vt, int k0, auto before_pv) __attribute__((always_inline)) {
+  auto compute_tile = [&](const unsigned char* Kt, const unsigned char* Vt, int k0, auto first, auto before_pv) __attribute__((always_inline)) {
+    constexpr bool FIRST = decltype(first)::value;
     // scores, S^T[key][q]: fragment o = (half t, kk, kb of the half), so that four accumulators are in turn
     auto read_kf = [&](auto oc) __attribute__((always_inline)) -> bf16x8 {
       constexpr int o = decltype(oc)::value;
@@ -183,9 +190,10 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_bf16_online16_kernel(const At
     };
     bf16x8 ring[RD];
     f32x4v sc[4][QB];
+    const bool half = FIRST && ke - k0 <= BN / 2;  // no key in the second half
     static_for<0, RD>([&](auto oc) __attribute__((always_inline)) { ring[decltype(oc)::value] = read_kf(oc); });
     __builtin_amdgcn_sched_barrier(0);
-    static_for<0, 16>([&](auto oc) __attribute__((always_inline)) {
+    auto scores = [&](auto oc) __attribute__((always_inline)) {
       constexpr int o = decltype(oc)::value;
       constexpr int kb = 2 * (o >> 3) + (o & 1), kk = (o >> 1) & 3;
 #pragma unroll
@@ -193,8 +201,15 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_bf16_online16_kernel(const At
         sc[kb][qb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ring[o % RD], qf[qb][kk], kk == 0 ? zero4 : sc[kb][qb], 0, 0, 0);
       if constexpr (o + RD < 16) ring[o % RD] = read_kf(std::integral_constant<int, o + RD>{});
       __builtin_amdgcn_sched_barrier(0);
-    });
-    if (k0 + BN > ke) {  // ragged last tile: keys >= ke do not exist
+    };
+    static_for<0, 8>(scores);
+    if (!half) {
+      static_for<8, 16>(scores);
+    } else {
+#pragma unroll
+      for (int qb = 0; qb < QB; ++qb) sc[2][qb] = sc[3][qb] = none4;
+    }
+    if (FIRST && k0 + BN > ke) {  // ragged: keys >= ke do not exist
 #pragma unroll
       for (int kb = 0; kb < 4; ++kb)
 #pragma unroll
@@ -219,7 +234,10 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_bf16_online16_kernel(const At
     }
     quad_max2(mx[0], mx[1]);
     const float m0 = fmaxf(m_run[0], mx[0]), m1 = fmaxf(m_run[1], mx[1]);
-    if (__builtin_amdgcn_ballot_w64(m0 != m_run[0] || m1 != m_run[1]) != 0) {  // some row of this wave saw a new maximum
+    if constexpr (FIRST) {
+      m_run[0] = m0;
+      m_run[1] = m1;
+    } else if (__builtin_amdgcn_ballot_w64(m0 != m_run[0] || m1 != m_run[1]) != 0) {  // some row of this wave saw a new maximum
       const float a0 = __builtin_amdgcn_exp2f((m_run[0] - m0) * c), a1 = __builtin_amdgcn_exp2f((m_run[1] - m1) * c);
       m_run[0] = m0;
       m_run[1] = m1;
@@ -249,7 +267,7 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_bf16_online16_kernel(const At
     // O^T[d][q] += V^T[d][key] P^T[key][q]
     static_for<0, RD>([&](auto oc) __attribute__((always_inline)) { ring[decltype(oc)::value] = read_vf(oc); });
     __builtin_amdgcn_sched_barrier(0);
-    static_for<0, 16>([&](auto oc) __attribute__((always_inline)) {
+    auto products = [&](auto oc) __attribute__((always_inline)) {
       constexpr int o = decltype(oc)::value;
       constexpr int db = v_block(o & 7);
 #pragma unroll
@@ -257,27 +275,33 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_bf16_online16_kernel(const At
         o_acc[db][qb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ring[o % RD], __builtin_bit_cast(bf16x8, pf[o >> 3][qb]), o_acc[db][qb], 0, 0, 0);
       if constexpr (o + RD < 16) ring[o % RD] = read_vf(std::integral_constant<int, o + RD>{});
       __builtin_amdgcn_sched_barrier(0);
-    });
+    };
+    static_for<0, 8>(products);
+    if (!half) static_for<8, 16>(products);
   };
 
-  auto step = [&](int k0, auto bc) __attribute__((always_inline)) {
+  // one tile (`nxt`: the one behind it, if below `last`): the last one in K slot 0, then tile j in slot (j + 1) & 1
+  auto step = [&](int cur, int nxt, auto bc, auto first) __attribute__((always_inline)) {
     constexpr int B = decltype(bc)::value;
     wait_vmcnt<0>();
     barrier_loads_in_flight();  // the K tile landed in everybody's view; the other K slot and the V slot are free
-    issue_mat(k0, sV, true);
-    if (k0 + BN < ke) issue_mat(k0 + BN, B ? sK0 : sK1, false);
-    compute_tile(B ? sK1 : sK0, sV, k0, [&]() __attribute__((always_inline)) {
-      if (k0 + BN < ke)
+    if constexpr (!decltype(first)::value) issue_mat(ks + cur * BN, sV, true);
+    if (nxt < last) issue_mat(ks + nxt * BN, B ? sK0 : sK1, false);
+    compute_tile(B ? sK1 : sK0, sV, ks + cur * BN, first, [&]() __attribute__((always_inline)) {
+      if (nxt < last)
         wait_vmcnt<LOADS>();  // the V tile landed, the next K tile stays in flight
       else
         wait_vmcnt<0>();
       barrier_loads_in_flight();
     });
   };
-  for (int k0 = ks; k0 < ke; k0 += 2 * BN) {
-    step(k0, std::integral_constant<int, 0>{});
-    if (k0 + BN >= ke) break;
-    step(k0 + BN, std::integral_constant<int, 1>{});
+  const std::integral_constant<int, 0> slot0;
+  const std::integral_constant<int, 1> slot1;
+  step(last, 0, slot0, std::true_type{});
+  for (int j = 0; j < last; j += 2) {
+    step(j, j + 1, slot1, std::false_type{});
+    if (j + 1 >= last) break;
+    step(j + 1, j + 2, slot0, std::false_type{});
   }
 
   if (row0 >= qe) return;
