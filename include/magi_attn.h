@@ -404,6 +404,13 @@ typedef struct magi_small_proj_args {
 int magi_small_projections(const magi_small_proj_args* args, void* stream);
 
 /*
+ * The same for e4m3 attention: q_out [S, Hq, 128] and the K rows that go to kv_out / kv_tail [rows, Hkv, 128] (strides in elements, that
+ * is bytes) leave as e4m3, divided by the constants q_quant_scale (q times q_premul) and k_quant_scale, as magi_qk_prologue's do;
+ * v goes to v_out [S, Hkv, 128] bf16, where magi_quantize_fp8_split takes its scales from it.
+ */
+int magi_small_projections_e4m3(const magi_small_proj_args* args, float q_quant_scale, float k_quant_scale, void* v_out, void* stream);
+
+/*
  * LayerNorm of the layer input over its last axis: x [rows, cols] bf16 -> y [rows, cols] bf16 with fp32
  * statistics, y = (x - mean) / sqrt(var + eps) * weight + bias (plain weight, not the "+1" form).
  * Stands in for torch.nn.LayerNorm in CustomLayerNormLinear.forward_ln (dit_module.py:401, 412-413;

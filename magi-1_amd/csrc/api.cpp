@@ -601,6 +601,112 @@ int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace) {
 
 }  // namespace
 
+namespace {
+
+// magi_small_projections, and with `e4m3` magi_small_projections_e4m3
+struct SmallProjE4m3 {
+  float q_scale, k_scale;
+  void* v_out;
+};
+int small_projections_impl(const magi_small_proj_args* p, const SmallProjE4m3* e4m3, void* stream) {
+  if (!p) return fail(MAGI_EINVAL, "magi_small_projections: args is NULL");
+  MAGI_CHECK_LAYOUT("magi_small_projections", p);
+  if (p->S < 0 || p->T < 0 || p->Hq < 0 || p->Hkv < 0 || p->Hqx < 0 || p->batch < 0)
+    return fail(MAGI_EINVAL, "magi_small_projections: negative size");
+  const bool hidden = p->S > 0 && p->Hq + p->Hkv + p->Hqx > 0, text = p->T > 0 && p->Hkv > 0;
+  if (!hidden && !text) return MAGI_OK;
+  if ((double)(p->S / 32 + 1) * (p->Hq + 2.0 * p->Hkv + p->Hqx) + (double)(p->T / 32 + 1) * 2 * p->Hkv > 2.0e9)
+    return fail(MAGI_ENOSYS, "magi_small_projections: too many rows");
+  if (!(p->eps >= 0.f)) return fail(MAGI_EINVAL, "magi_small_projections: eps");
+  magi::SmallProjKernArgs a;
+  std::memset(&a, 0, sizeof(a));
+  a.Hq = p->Hq;
+  a.Hkv = p->Hkv;
+  a.Hqx = p->Hqx;
+  a.eps = p->eps;
+  a.batch = p->batch > 1 ? p->batch : 1;
+  if (hidden) {
+    if (p->K <= 0 || p->K % 64) return fail(MAGI_ENOSYS, "magi_small_projections: K=%d is not a multiple of 64", p->K);
+    if (!p->x || !p->w) return fail(MAGI_EINVAL, "magi_small_projections: NULL x / w");
+    if (p->x_stride < p->K || p->x_stride % 8 || !aligned16(p->x) || !aligned16(p->w))
+      return fail(MAGI_EINVAL, "magi_small_projections: rows of x and w must be 16-byte aligned and at least K long");
+    // (32-bit byte offsets within the descriptors' 2^31 - 1: row 63 of a workgroup's 64 rows of x, 2^25 bytes apart at most, which nearly
+    // fills them; the 128 weight rows of a head)
+    if (p->x_stride > (1 << 24) || p->K > (1 << 22)) return fail(MAGI_ENOSYS, "magi_small_projections: rows above 2^22 elements are not implemented");
+    if (p->ln_w && (p->K > 1024 || (text && p->Kt > 1024)))
+      return fail(MAGI_ENOSYS, "magi_small_projections: the input norm is implemented for K (and Kt) up to 1024");
+    if ((p->ln_w != nullptr) != (p->ln_b != nullptr) || !aligned16(p->ln_w) || !aligned16(p->ln_b) || (p->ln_w && !(p->ln_eps >= 0.f)))
+      return fail(MAGI_EINVAL, "magi_small_projections: ln_w and ln_b come together, 16-byte aligned, with ln_eps >= 0");
+    if (p->R2 < 0 || p->R2 % 8 || 2 * p->R2 > 128) return fail(MAGI_EINVAL, "magi_small_projections: R2=%d must be a multiple of 8 up to 64", p->R2);
+    if ((p->Hq > 0 && (!p->q_out || !p->gq)) || (p->Hkv > 0 && !p->gk) || (p->Hqx > 0 && !p->qx_out))
+      return fail(MAGI_EINVAL, "magi_small_projections: NULL output or norm parameter");
+    if (p->n_cache_rows < 0 || p->n_cache_rows > p->S)
+      return fail(MAGI_EINVAL, "magi_small_projections: n_cache_rows %d outside [0, S=%d]", p->n_cache_rows, p->S);
+    if (p->Hkv > 0 && ((p->n_cache_rows > 0 && !p->kv_out) || (p->n_cache_rows < p->S && !p->kv_tail)))
+      return fail(MAGI_EINVAL, "magi_small_projections: NULL kv_out / kv_tail");
+    if (p->kv_stride_t % 8 || p->kv_tail_stride_t % 8 || !aligned16(p->q_out) || !aligned16(p->kv_out) || !aligned16(p->kv_tail) ||
+        !aligned16(p->qx_out) || !aligned16(p->rope) || !aligned16(p->gq) || !aligned16(p->bq) || !aligned16(p->gk) || !aligned16(p->bk))
+      return fail(MAGI_EINVAL, "magi_small_projections: buffers must be 16-byte aligned");
+    if (!std::isfinite(p->q_premul)) return fail(MAGI_EINVAL, "magi_small_projections: q_premul is not finite");
+    a.x = static_cast<const char*>(p->x);
+    a.w = static_cast<const char*>(p->w);
+    a.ln_w = static_cast<const char*>(p->ln_w);
+    a.ln_b = static_cast<const char*>(p->ln_b);
+    a.x_stride = p->x_stride * 2;
+    a.S = p->S;
+    a.K = p->K;
+    a.ln_fp32 = p->ln_params_fp32 != 0;
+    a.ln_eps = p->ln_eps;
+    a.rope = p->R2 > 0 ? p->rope : nullptr;
+    a.R2 = a.rope ? p->R2 : 0;
+    a.gq = p->gq;
+    a.bq = p->bq;
+    a.gk = p->gk;
+    a.bk = p->bk;
+    a.q_premul = p->q_premul == 0.f ? 1.f : p->q_premul;
+    a.n_cache_rows = p->n_cache_rows;
+    a.q_out = static_cast<char*>(p->q_out);
+    a.kv_out = static_cast<char*>(p->kv_out);
+    a.kv_tail = static_cast<char*>(p->kv_tail);
+    a.kv_stride_t = p->kv_stride_t * 2;
+    a.kv_tail_stride_t = p->kv_tail_stride_t * 2;
+    a.qx_out = static_cast<char*>(p->qx_out);
+    if (e4m3) {
+      if ((p->Hq > 0 && !(e4m3->q_scale > 0.f && std::isfinite(e4m3->q_scale))) ||
+          (p->Hkv > 0 && (!(e4m3->k_scale > 0.f && std::isfinite(e4m3->k_scale)) || !e4m3->v_out || !aligned16(e4m3->v_out))))
+        return fail(MAGI_EINVAL, "magi_small_projections_e4m3: q_quant_scale and k_quant_scale must be positive and finite, v_out 16-byte aligned");
+      a.out_fp8 = 1;
+      a.q_inv_scale = 1.f / e4m3->q_scale;
+      a.k_inv_scale = 1.f / e4m3->k_scale;
+      a.v_out = static_cast<char*>(e4m3->v_out);
+      a.kv_stride_t = p->kv_stride_t;
+      a.kv_tail_stride_t = p->kv_tail_stride_t;
+    }
+  }
+  if (text) {
+    if (p->Kt <= 0 || p->Kt % 64) return fail(MAGI_ENOSYS, "magi_small_projections: Kt=%d is not a multiple of 64", p->Kt);
+    if (!p->text || !p->w_text || !p->text_out || !p->gkx) return fail(MAGI_EINVAL, "magi_small_projections: NULL text / w_text / text_out / gkx");
+    if (p->text_stride < p->Kt || p->text_stride % 8 || !aligned16(p->text) || !aligned16(p->w_text) || !aligned16(p->text_out) ||
+        !aligned16(p->gkx) || !aligned16(p->bkx))
+      return fail(MAGI_EINVAL, "magi_small_projections: rows of text and w_text must be 16-byte aligned and at least Kt long");
+    if (p->text_stride > (1 << 24) || p->Kt > (1 << 22)) return fail(MAGI_ENOSYS, "magi_small_projections: rows above 2^22 elements are not implemented");
+    a.text = static_cast<const char*>(p->text);
+    a.w_text = static_cast<const char*>(p->w_text);
+    a.text_stride = p->text_stride * 2;
+    a.T = p->T;
+    a.Kt = p->Kt;
+    a.gkx = p->gkx;
+    a.bkx = p->bkx;
+    a.text_out = static_cast<char*>(p->text_out);
+  }
+  hipError_t e = magi::launch_small_proj(a, compute_units(), static_cast<hipStream_t>(stream));
+  if (e != hipSuccess) return hip_fail(e, "magi_small_projections launch");
+  g_launches.fetch_add(1, std::memory_order_relaxed);
+  return MAGI_OK;
+}
+
+}  // namespace
+
 extern "C" {
 
 int magi_qk_prologue(const magi_prologue_args* p, void* stream) {
@@ -743,90 +849,11 @@ int magi_qkv_proj_prologue(const magi_qkv_proj_args* p, void* stream) {
   return MAGI_OK;
 }
 
-int magi_small_projections(const magi_small_proj_args* p, void* stream) {
-  if (!p) return fail(MAGI_EINVAL, "magi_small_projections: args is NULL");
-  MAGI_CHECK_LAYOUT("magi_small_projections", p);
-  if (p->S < 0 || p->T < 0 || p->Hq < 0 || p->Hkv < 0 || p->Hqx < 0 || p->batch < 0)
-    return fail(MAGI_EINVAL, "magi_small_projections: negative size");
-  const bool hidden = p->S > 0 && p->Hq + p->Hkv + p->Hqx > 0, text = p->T > 0 && p->Hkv > 0;
-  if (!hidden && !text) return MAGI_OK;
-  if ((double)(p->S / 32 + 1) * (p->Hq + 2.0 * p->Hkv + p->Hqx) + (double)(p->T / 32 + 1) * 2 * p->Hkv > 2.0e9)
-    return fail(MAGI_ENOSYS, "magi_small_projections: too many rows");
-  if (!(p->eps >= 0.f)) return fail(MAGI_EINVAL, "magi_small_projections: eps");
-  magi::SmallProjKernArgs a;
-  std::memset(&a, 0, sizeof(a));
-  a.Hq = p->Hq;
-  a.Hkv = p->Hkv;
-  a.Hqx = p->Hqx;
-  a.eps = p->eps;
-  a.batch = p->batch > 1 ? p->batch : 1;
-  if (hidden) {
-    if (p->K <= 0 || p->K % 64) return fail(MAGI_ENOSYS, "magi_small_projections: K=%d is not a multiple of 64", p->K);
-    if (!p->x || !p->w) return fail(MAGI_EINVAL, "magi_small_projections: NULL x / w");
-    if (p->x_stride < p->K || p->x_stride % 8 || !aligned16(p->x) || !aligned16(p->w))
-      return fail(MAGI_EINVAL, "magi_small_projections: rows of x and w must be 16-byte aligned and at least K long");
-    // (32-bit byte offsets within the descriptors' 2^31 - 1: row 63 of a workgroup's 64 rows of x, 2^25 bytes apart at most, which nearly
-    // fills them; the 128 weight rows of a head)
-    if (p->x_stride > (1 << 24) || p->K > (1 << 22)) return fail(MAGI_ENOSYS, "magi_small_projections: rows above 2^22 elements are not implemented");
-    if (p->ln_w && (p->K > 1024 || (text && p->Kt > 1024)))
-      return fail(MAGI_ENOSYS, "magi_small_projections: the input norm is implemented for K (and Kt) up to 1024");
-    if ((p->ln_w != nullptr) != (p->ln_b != nullptr) || !aligned16(p->ln_w) || !aligned16(p->ln_b) || (p->ln_w && !(p->ln_eps >= 0.f)))
-      return fail(MAGI_EINVAL, "magi_small_projections: ln_w and ln_b come together, 16-byte aligned, with ln_eps >= 0");
-    if (p->R2 < 0 || p->R2 % 8 || 2 * p->R2 > 128) return fail(MAGI_EINVAL, "magi_small_projections: R2=%d must be a multiple of 8 up to 64", p->R2);
-    if ((p->Hq > 0 && (!p->q_out || !p->gq)) || (p->Hkv > 0 && !p->gk) || (p->Hqx > 0 && !p->qx_out))
-      return fail(MAGI_EINVAL, "magi_small_projections: NULL output or norm parameter");
-    if (p->n_cache_rows < 0 || p->n_cache_rows > p->S)
-      return fail(MAGI_EINVAL, "magi_small_projections: n_cache_rows %d outside [0, S=%d]", p->n_cache_rows, p->S);
-    if (p->Hkv > 0 && ((p->n_cache_rows > 0 && !p->kv_out) || (p->n_cache_rows < p->S && !p->kv_tail)))
-      return fail(MAGI_EINVAL, "magi_small_projections: NULL kv_out / kv_tail");
-    if (p->kv_stride_t % 8 || p->kv_tail_stride_t % 8 || !aligned16(p->q_out) || !aligned16(p->kv_out) || !aligned16(p->kv_tail) ||
-        !aligned16(p->qx_out) || !aligned16(p->rope) || !aligned16(p->gq) || !aligned16(p->bq) || !aligned16(p->gk) || !aligned16(p->bk))
-      return fail(MAGI_EINVAL, "magi_small_projections: buffers must be 16-byte aligned");
-    if (!std::isfinite(p->q_premul)) return fail(MAGI_EINVAL, "magi_small_projections: q_premul is not finite");
-    a.x = static_cast<const char*>(p->x);
-    a.w = static_cast<const char*>(p->w);
-    a.ln_w = static_cast<const char*>(p->ln_w);
-    a.ln_b = static_cast<const char*>(p->ln_b);
-    a.x_stride = p->x_stride * 2;
-    a.S = p->S;
-    a.K = p->K;
-    a.ln_fp32 = p->ln_params_fp32 != 0;
-    a.ln_eps = p->ln_eps;
-    a.rope = p->R2 > 0 ? p->rope : nullptr;
-    a.R2 = a.rope ? p->R2 : 0;
-    a.gq = p->gq;
-    a.bq = p->bq;
-    a.gk = p->gk;
-    a.bk = p->bk;
-    a.q_premul = p->q_premul == 0.f ? 1.f : p->q_premul;
-    a.n_cache_rows = p->n_cache_rows;
-    a.q_out = static_cast<char*>(p->q_out);
-    a.kv_out = static_cast<char*>(p->kv_out);
-    a.kv_tail = static_cast<char*>(p->kv_tail);
-    a.kv_stride_t = p->kv_stride_t * 2;
-    a.kv_tail_stride_t = p->kv_tail_stride_t * 2;
-    a.qx_out = static_cast<char*>(p->qx_out);
-  }
-  if (text) {
-    if (p->Kt <= 0 || p->Kt % 64) return fail(MAGI_ENOSYS, "magi_small_projections: Kt=%d is not a multiple of 64", p->Kt);
-    if (!p->text || !p->w_text || !p->text_out || !p->gkx) return fail(MAGI_EINVAL, "magi_small_projections: NULL text / w_text / text_out / gkx");
-    if (p->text_stride < p->Kt || p->text_stride % 8 || !aligned16(p->text) || !aligned16(p->w_text) || !aligned16(p->text_out) ||
-        !aligned16(p->gkx) || !aligned16(p->bkx))
-      return fail(MAGI_EINVAL, "magi_small_projections: rows of text and w_text must be 16-byte aligned and at least Kt long");
-    if (p->text_stride > (1 << 24) || p->Kt > (1 << 22)) return fail(MAGI_ENOSYS, "magi_small_projections: rows above 2^22 elements are not implemented");
-    a.text = static_cast<const char*>(p->text);
-    a.w_text = static_cast<const char*>(p->w_text);
-    a.text_stride = p->text_stride * 2;
-    a.T = p->T;
-    a.Kt = p->Kt;
-    a.gkx = p->gkx;
-    a.bkx = p->bkx;
-    a.text_out = static_cast<char*>(p->text_out);
-  }
-  hipError_t e = magi::launch_small_proj(a, compute_units(), static_cast<hipStream_t>(stream));
-  if (e != hipSuccess) return hip_fail(e, "magi_small_projections launch");
-  g_launches.fetch_add(1, std::memory_order_relaxed);
-  return MAGI_OK;
+int magi_small_projections(const magi_small_proj_args* p, void* stream) { return small_projections_impl(p, nullptr, stream); }
+
+int magi_small_projections_e4m3(const magi_small_proj_args* p, float q_quant_scale, float k_quant_scale, void* v_out, void* stream) {
+  const SmallProjE4m3 e4m3 = {q_quant_scale, k_quant_scale, v_out};
+  return small_projections_impl(p, &e4m3, stream);
 }
 
 int magi_layer_norm(const void* x, int64_t x_stride, const void* weight, const void* bias, int32_t params_fp32,

@@ -170,6 +170,10 @@ struct SmallProjKernArgs {
   int Hq, Hkv, Hqx, R2;
   int ln_fp32, batch;
   float ln_eps, eps, q_premul;
+  // out_fp8: q and k leave as e4m3 (kv_out / kv_tail then hold K rows only, strides in bytes), v as it is in rows of v_out [S, Hkv, 128] bf16
+  int out_fp8;
+  float q_inv_scale, k_inv_scale;  // out_fp8: 1 / the constant scale of q (after q_premul) and of k
+  char* v_out;
   int hidden_blocks;  // filled by the launcher
 };
 hipError_t launch_small_proj(const SmallProjKernArgs& a, int compute_units, hipStream_t stream);

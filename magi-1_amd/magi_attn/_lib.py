@@ -131,7 +131,7 @@ EXPORTS = ("magi_version", "magi_last_error", "magi_launch_count", "magi_attn_fw
            "magi_attn_split_bytes", "magi_attn_online_split_bytes", "magi_attn_tile_rows",
            "magi_qk_prologue", "magi_head_norm",
            "magi_apply_rotary", "magi_quantize_fp8", "magi_quantize_fp8_split", "magi_layer_norm", "magi_qkv_proj_prologue", "magi_div_clamp_to_e4m3",
-           "magi_layer_norm_e4m3", "magi_small_projections")
+           "magi_layer_norm_e4m3", "magi_small_projections", "magi_small_projections_e4m3")
 
 _lib = None
 
@@ -185,6 +185,8 @@ def lib() -> C.CDLL:
         l.magi_qkv_proj_prologue.restype = C.c_int
         l.magi_small_projections.argtypes = [C.POINTER(SmallProjArgs), C.c_void_p]
         l.magi_small_projections.restype = C.c_int
+        l.magi_small_projections_e4m3.argtypes = [C.POINTER(SmallProjArgs), C.c_float, C.c_float, C.c_void_p, C.c_void_p]
+        l.magi_small_projections_e4m3.restype = C.c_int
         l.magi_quantize_fp8_split.argtypes = [C.POINTER(QuantizeArgs), C.c_void_p]
         l.magi_quantize_fp8_split.restype = C.c_int
         _lib = l
@@ -192,28 +194,28 @@ def lib() -> C.CDLL:
 
 
 class PackedCall:
-    """A C-ABI entry point `int f(const args*, void* stream)` called with its argument struct packed in one go
+    """A C-ABI entry point `int f(const args*, [more,] void* stream)` called with its argument struct packed in one go
     (struct.pack over all fields in declaration order, NULL = 0) instead of field by field through ctypes: a small
     launch costs the host less than its struct did."""
 
     _CODES = {C.c_uint32: "I", C.c_int32: "i", C.c_int64: "q", C.c_void_p: "P", C.c_float: "f"}
 
-    def __init__(self, name: str, args: type):
+    def __init__(self, name: str, args: type, *more: type):
         layout = struct.Struct("@" + "".join(self._CODES[t] for _, t in args._fields_) + "0q")
         if layout.size != C.sizeof(args):
             raise RuntimeError(f"{args.__name__}: {layout.size} packed bytes for a struct of {C.sizeof(args)}")
         self.size, self.pack = layout.size, layout.pack
         self.fn = lib()[name]  # (a handle of its own: the shared one takes a pointer to the struct)
-        self.fn.argtypes, self.fn.restype = [C.c_char_p, C.c_void_p], C.c_int
+        self.fn.argtypes, self.fn.restype = [C.c_char_p, *more, C.c_void_p], C.c_int
 
 
 _packed = {}
 
 
-def packed(name: str, args: type) -> PackedCall:
+def packed(name: str, args: type, *more: type) -> PackedCall:
     call = _packed.get(name)
     if call is None:
-        call = _packed[name] = PackedCall(name, args)
+        call = _packed[name] = PackedCall(name, args, *more)
     return call
 
 

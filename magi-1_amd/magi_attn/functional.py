@@ -548,6 +548,41 @@ def launch_small_projections(dev: torch.device, *fields) -> None:
     _launch_packed(dev, "magi_small_projections", L.SmallProjArgs, *fields)
 
 
+def launch_small_projections_e4m3(dev: torch.device, q_scale: float, k_scale: float, v_out: int, *fields) -> None:
+    """magi_small_projections_e4m3, the fields of the struct as above."""
+    call = L.packed("magi_small_projections_e4m3", L.SmallProjArgs, C.c_float, C.c_float, C.c_void_p)
+    _launch(dev, call.fn, call.pack(call.size, *fields), q_scale, k_scale, v_out)
+
+
+def launch_quantize_fp8_split(dev: torch.device, *fields) -> None:
+    """magi_quantize_fp8_split with the fields of its argument struct behind struct_size, in order."""
+    _launch_packed(dev, "magi_quantize_fp8_split", L.QuantizeArgs, *fields)
+
+
+def launch_fp8_attention(dev: torch.device, q: int, rows: int, Hq: int, k: int, v: int, k_side: int, v_side: int, k_split: int, total_k: int,
+                         Hkv: int, scales: tuple, chunk_tokens: int, q_ranges: torch.Tensor, k_ranges: torch.Tensor, n: int, max_seqlen_q: int,
+                         max_seqlen_k: int, out: int, o_row: int, group_heads: int, o_group: int, clear: bool, fast_exp2: bool) -> None:
+    """launch_bounded_attention for e4m3 rows with power-of-two scales, heads and rows contiguous: K and V rows at k / v, those from
+    k_split on at k_side / v_side (0: none); scales: the tables of q, k, v, and of k and v there (0: none) by address.  Shares keys as
+    range_attention does."""
+    max_seqlen_q, max_seqlen_k = int(max_seqlen_q), int(max_seqlen_k)
+    split, split_bytes = None, 0
+    if max_seqlen_k >= 512:
+        split_bytes = L.lib().magi_attn_split_bytes(Hq, Hkv, max(n, 0), max_seqlen_q, max_seqlen_k, L.MAGI_DTYPE_FP8_E4M3)
+        if split_bytes:
+            split = torch.empty(split_bytes, dtype=torch.uint8, device=dev)
+    q_ranges, k_ranges = q_ranges.contiguous(), k_ranges.contiguous()
+    qs, ks, vs, k2s, v2s = scales
+    flags = (L.MAGI_ATTN_FP8_POW2_PRESCALED | (L.MAGI_ATTN_FP8_FAST_EXP2 if fast_exp2 else 0)
+             | (L.MAGI_ATTN_ZERO_UNCOVERED if clear and covered_by_launch(n, max_seqlen_q, rows) else 0))
+    row = Hkv * 128
+    _launch_packed(
+        dev, "magi_attn_fwd", L.AttnArgs, q, k, v, k_side, v_side, out, 0, q_ranges.data_ptr(), k_ranges.data_ptr(), qs, ks, vs, Hq * 128, 128, row, 128,
+        row, 128, o_row, 128, rows, total_k, k_split, max(n, 0), L.MAGI_RANGES_PAIRS, max_seqlen_q, max_seqlen_k, Hq, Hkv, 128,
+        L.MAGI_DTYPE_FP8_E4M3, chunk_tokens, 0.0, flags, group_heads, o_group, 0.0, 0, 0, 0, 0.0, 0, k2s, v2s, 0, 0, 0, 0,
+        0 if split is None else split.data_ptr(), split_bytes)
+
+
 def small_projections(x: Optional[torch.Tensor], w: Optional[torch.Tensor], rope, gq, bq, gk, bk, *, Hq: int, Hkv: int, Hqx: int = 0,
                       ln: Optional[tuple] = None, eps: float = 1e-6, batch: int = 1, q_premul: float = 1.0,
                       kv_out: Optional[torch.Tensor] = None, n_cache_rows: Optional[int] = None,

@@ -35,7 +35,8 @@ import torch
 
 from . import _lib as L
 from .cache import Fp8KVCache, OffloadedKVCache
-from .functional import _measuring_a_bound_pays, covered_by_launch, launch_bounded_attention, launch_small_projections, range_count
+from .functional import (_measuring_a_bound_pays, covered_by_launch, launch_bounded_attention, launch_fp8_attention, launch_quantize_fp8_split,
+                         launch_small_projections, launch_small_projections_e4m3, range_count)
 from .functional import (div_clamp_to, head_norm, layer_norm, layer_norm_div_clamp, pow2_scale_for, qk_prologue, qk_prologue_fp8, qkv_proj_prologue,
                          quantize_fp8_split,
                          range_attention, small_projections)
@@ -358,19 +359,28 @@ class CustomLayerNormLinear(torch.nn.Module):
             row += w.shape[0]
         return fused
 
-    def fused_weight(self) -> torch.Tensor:
-        """The [q | k | v | qx] weight as one tensor (rebuilt first if the parameters no longer share a buffer)."""
-        ws = [_param(m, "weight") for m in self._projections()]
-        base = ws[0]
-        ptr, rows = base.data_ptr(), 0
-        row_bytes = base.shape[1] * base.element_size()
-        for w in ws:
+    def _fused_rows(self) -> Tuple[torch.Tensor, int]:
+        """(the first parameter of the shared buffer, the rows of all four), 0 rows where they do not share one."""
+        base, ptr, rows = None, 0, 0
+        for m in self._projections():
+            w = _param(m, "weight")
+            if base is None:
+                base, ptr = w, w.data_ptr()
+                row_bytes = w.shape[1] * w.element_size()
             if w.data_ptr() != ptr or w.dtype is not base.dtype or not w.is_contiguous():
-                return self._fuse_weights()
-            ptr += w.shape[0] * row_bytes
-            rows += w.shape[0]
+                return base, 0
+            n = w.shape[0]
+            ptr += n * row_bytes
+            rows += n
         # back to back, and all of it inside the first one's allocation
         if base.untyped_storage().nbytes() - base.storage_offset() * base.element_size() < rows * row_bytes:
+            return base, 0
+        return base, rows
+
+    def fused_weight(self) -> torch.Tensor:
+        """The [q | k | v | qx] weight as one tensor (rebuilt first if the parameters no longer share a buffer)."""
+        base, rows = self._fused_rows()
+        if rows == 0:
             return self._fuse_weights()
         return base.data.as_strided((rows, base.shape[1]), (base.shape[1], 1))
 
@@ -891,15 +901,17 @@ class FullyParallelAttention(torch.nn.Module):
             self._kv_tail = tail
         return tail[:rows]
 
-    def _forward_small(self, hidden_states: torch.Tensor, key_value_states: torch.Tensor, inference_params: Optional[InferenceParams],
-                       rope: torch.Tensor, meta_args: ModelMetaArgs, proj_layout: bool, bound_core: float, bound_cross: float):
-        """forward() of a small bf16 layer at batch 1 with both score bounds in force, whose projections are the library's own: three
-        launches (magi_small_projections, core attention, cross attention) with their arguments put together in one go.  None, before
-        anything is launched or written, where forward() goes on with the separate launches: other methods, projections or caches, larger
-        layers, tensors of other types or layouts.  (The layer's cache and its side buffer may have been allocated by then, as forward() would.)
+    def _norm_parameters(self):
+        """gamma_beta_fp32() of the four head norms, which forward() has had converted or checked by now (score_bounds)."""
+        m = self._modules
+        lns = (m["q_layernorm"], m["k_layernorm"], m["q_layernorm_xattn"], m["k_layernorm_xattn"])
+        if FusedLayerNorm.gamma_beta_fp32 is not _GAMMA_BETA:
+            return [ln.gamma_beta_fp32() for ln in lns]
+        return [d["_gb"] if type(ln) is FusedLayerNorm and "gamma_beta_fp32" not in (d := ln.__dict__) else ln.gamma_beta_fp32() for ln in lns]
 
-        Such a layer waits for the host: 240 + 24 rows, 20 + 4 heads, 87 us through the callables, 51 this way.  There
-        each launch brings its own checks, allocations and views with it."""
+    def _small_layer_weights(self, hidden_states: torch.Tensor, key_value_states: torch.Tensor, rope: torch.Tensor, own: "_Own"):
+        """(w, wt, ln, lw, lb): the parameter that the weight of the four projections starts with, the text's weight, the input norm and its parameters, of a small layer
+        at batch 1 whose projections are the library's own and whose tensors are as magi_small_projections takes them; else None."""
         S, b, K = hidden_states.shape
         if K > 1024 or b != 1 or key_value_states.dim() != 2 or not hidden_states.is_cuda or self.fused_projection:
             return None
@@ -911,20 +923,58 @@ class FullyParallelAttention(torch.nn.Module):
         lin = m["linear_qkv"]
         if lin.__dict__.get("fp8_quant", True) or not hidden_states.is_contiguous() or rope.shape[-1] % 16 or rope.shape[-1] > D:
             return None
-        use_cache = inference_params is not None and (
-            meta_args.extract_prefix_video_feature or meta_args.fwd_extra_1st_chunk or meta_args.slice_point > 0)
-        if not (_OWN_SMALL_PROJECTIONS.of(lin) and (_OWN_SMALL if use_cache else _OWN_SMALL_UNCACHED).of(self)):
+        if not (_OWN_SMALL_PROJECTIONS.of(lin) and own.of(self)):
             return None
-        w, wt, ln = lin.fused_weight(), _param(m["linear_kv_xattn"], "weight"), lin._modules["layer_norm"]
+        w, rows = lin._fused_rows()
+        if rows == 0:
+            w = lin._fuse_weights()
+            rows = w.shape[0]
+        wt, ln = _param(m["linear_kv_xattn"], "weight"), lin._modules["layer_norm"]
         lw, lb = _param(ln, "weight"), _param(ln, "bias")
         if (hidden_states.dtype is not torch.bfloat16 or type(hidden_states) not in _PLAIN or S == 0 or hidden_states.data_ptr() % 16
-                or not _plain_weight(w, 2 * (Hq + Hkv), K, dev) or not _plain_rows(key_value_states, wt, 2 * Hkv) or lw is None or lb is None):
+                or rows != 2 * (Hq + Hkv) * D or not _plain_weight(w, w.shape[0] // D, K, dev) or not _plain_rows(key_value_states, wt, 2 * Hkv)
+                or lw is None or lb is None):
             return None
         if _param(lin._modules["q"], "weight").shape[0] != Hq * D or _param(lin._modules["k"], "weight").shape[0] != Hkv * D:
             return None
         if lw.dtype is not lb.dtype or lw.dtype not in (torch.bfloat16, torch.float32) or not (lw.is_contiguous() and lb.is_contiguous()) or (
                 lw.shape[0] != K or lb.shape[0] != K or (lw.data_ptr() | lb.data_ptr()) % 16 or lw.device != dev or key_value_states.device != dev):
             return None
+        return w, wt, ln, lw, lb
+
+    def _small_layer_outputs(self, S: int, dev: torch.device, proj_layout: bool, core_n: int, core_most: int, cross_n: int, cross_most: int):
+        """-> (tensors, address of core's rows, of cross's, row stride, heads per group, group stride, whether rows that no range covers are
+        cleared): one tensor in linear_proj's layout or two, as forward() returns them."""
+        Hq, D = self.num_attention_heads, 128
+        if proj_layout and Hq % PROJ_GROUPS == 0:
+            # (rows that no q range / cu_seqlens segment covers are left as allocated: the pipeline's ranges cover
+            # every row, dit_model.py:220-222, 246)
+            out = torch.empty(S, 1, 2 * Hq * D, dtype=torch.bfloat16, device=dev)
+            per = Hq // PROJ_GROUPS
+            return (out,), out.data_ptr(), out.data_ptr() + 2 * per * D, 2 * Hq * D, per, 2 * per * D, False
+        core, cross = torch.empty(S, 1, Hq * D, dtype=torch.bfloat16, device=dev), torch.empty(S, 1, Hq * D, dtype=torch.bfloat16, device=dev)
+        for t, n, most in ((core, core_n, core_most), (cross, cross_n, cross_most)):
+            if not covered_by_launch(n, most, S):
+                t.zero_()
+        return (core, cross), core.data_ptr(), cross.data_ptr(), Hq * D, 0, 0, True
+
+    def _forward_small(self, hidden_states: torch.Tensor, key_value_states: torch.Tensor, inference_params: Optional[InferenceParams],
+                       rope: torch.Tensor, meta_args: ModelMetaArgs, proj_layout: bool, bound_core: float, bound_cross: float):
+        """forward() of a small bf16 layer at batch 1 with both score bounds in force, whose projections are the library's own: three
+        launches (magi_small_projections, core attention, cross attention) with their arguments put together in one go.  None, before
+        anything is launched or written, where forward() goes on with the separate launches: other methods, projections or caches, larger
+        layers, tensors of other types or layouts.  (The layer's cache and its side buffer may have been allocated by then, as forward() would.)
+
+        Such a layer waits for the host: 240 + 45 rows, 20 + 4 heads, 87 us through the callables, 48 this way.  There
+        each launch brings its own checks, allocations and views with it."""
+        use_cache = inference_params is not None and (
+            meta_args.extract_prefix_video_feature or meta_args.fwd_extra_1st_chunk or meta_args.slice_point > 0)
+        parts = self._small_layer_weights(hidden_states, key_value_states, rope, _OWN_SMALL if use_cache else _OWN_SMALL_UNCACHED)
+        if parts is None:
+            return None
+        w, wt, ln, lw, lb = parts
+        (S, _, K), dev, m = hidden_states.shape, hidden_states.device, self._modules
+        Hq, Hkv, D, (T, Kt) = self.num_attention_heads, self.num_query_groups_per_partition, 128, key_value_states.shape
         cache = tail = offloaded = None
         start = n_keep = persisted = 0
         if use_cache:
@@ -950,10 +1000,7 @@ class FullyParallelAttention(torch.nn.Module):
             raise ValueError("rope must be a contiguous fp32 [S / batch, 2*R2] tensor")
         core_n = range_count(p.q_range, p.k_range, L.MAGI_RANGES_PAIRS)
         cross_n = range_count(cp.cu_seqlens_q, cp.cu_seqlens_kv, L.MAGI_RANGES_CU)
-        gq, bq = m["q_layernorm"].gamma_beta_fp32()
-        gk, bk = m["k_layernorm"].gamma_beta_fp32()
-        gx, bx = m["q_layernorm_xattn"].gamma_beta_fp32()
-        gkx, bkx = m["k_layernorm_xattn"].gamma_beta_fp32()
+        (gq, bq), (gk, bk), (gx, bx), (gkx, bkx) = self._norm_parameters()
         # one buffer for q, the raw cross-attention q, the text's K | V rows, and K | V without a cache
         ws = torch.empty(D * (2 * Hq * S + 2 * Hkv * (T + (S if cache is None else 0))), dtype=torch.bfloat16, device=dev)
         q = ws.data_ptr()
@@ -961,19 +1008,8 @@ class FullyParallelAttention(torch.nn.Module):
         text_kv = qx + 2 * D * Hq * S
         row = 2 * D * Hkv  # elements of a K | V row
         side = 0 if tail is None else tail.data_ptr()
-        if proj_layout and Hq % PROJ_GROUPS == 0:
-            # (rows that no q range / cu_seqlens segment covers are left as allocated: the pipeline's ranges cover
-            # every row, dit_model.py:220-222, 246)
-            out = torch.empty(S, 1, 2 * Hq * D, dtype=torch.bfloat16, device=dev)
-            per = Hq // PROJ_GROUPS
-            core_out = out.data_ptr()
-            cross_out, o_row, groups, o_group, clear = core_out + 2 * per * D, 2 * Hq * D, per, 2 * per * D, False
-        else:
-            core, cross = torch.empty(S, 1, Hq * D, dtype=torch.bfloat16, device=dev), torch.empty(S, 1, Hq * D, dtype=torch.bfloat16, device=dev)
-            core_out, cross_out, o_row, groups, o_group, clear = core.data_ptr(), cross.data_ptr(), Hq * D, 0, 0, True
-            for t, n, most in ((core, core_n, p.max_seqlen_q), (cross, cross_n, cp.max_seqlen_q)):
-                if not covered_by_launch(n, most, S):
-                    t.zero_()
+        outs, core_out, cross_out, o_row, groups, o_group, clear = self._small_layer_outputs(S, dev, proj_layout, core_n, p.max_seqlen_q, cross_n,
+                                                                                             cp.max_seqlen_q)
         if offloaded is not None:  # kv_offload: the prefix comes through a device staging buffer
             cache = offloaded.stage(start)
         try:
@@ -996,9 +1032,82 @@ class FullyParallelAttention(torch.nn.Module):
         launch_bounded_attention(dev, qx, Hq * D, S, Hq, text_kv, 0, T, T, row, Hkv, cp.cu_seqlens_q, cp.cu_seqlens_kv, cross_n, L.MAGI_RANGES_CU,
                                  cp.max_seqlen_q, cp.max_seqlen_kv, cross_out, o_row, groups, o_group, clear, bound_cross,
                                  (gx.data_ptr(), bx.data_ptr(), self.eps))
-        if clear is False:
-            return out
-        return attn_linear_proj_input(core, cross) if proj_layout else (core, cross)
+        return outs[0] if len(outs) == 1 else attn_linear_proj_input(*outs) if proj_layout else outs
+
+    def _forward_small_fp8(self, hidden_states: torch.Tensor, key_value_states: torch.Tensor, inference_params: Optional[InferenceParams],
+                           rope: torch.Tensor, meta_args: ModelMetaArgs, proj_layout: bool, bound_cross: float):
+        """_forward_small for e4m3 attention (the text's scores bounded): magi_small_projections_e4m3, the quantiser of V, core attention,
+        cross attention.  None where forward() goes on with the separate launches, or refuses the call.  240 + 45 rows, 20 + 4
+        heads: 153 us through the callables, 66 this way."""
+        use_cache = inference_params is not None and (
+            meta_args.extract_prefix_video_feature or meta_args.fwd_extra_1st_chunk or meta_args.slice_point > 0)
+        parts = self._small_layer_weights(hidden_states, key_value_states, rope, _OWN_SMALL_FP8)
+        if parts is None:
+            return None
+        w, wt, ln, lw, lb = parts
+        (S, _, K), dev, m = hidden_states.shape, hidden_states.device, self._modules
+        Hq, Hkv, D, (T, Kt) = self.num_attention_heads, self.num_query_groups_per_partition, 128, key_value_states.shape
+        Lc, row = meta_args.clip_token_nums, Hkv * D  # bytes of a K or V row
+        start = n_keep = 0
+        cache = None
+        if use_cache:
+            if inference_params.max_batch_size != 1 or Lc <= 0:
+                return None
+            cache = self._cache_fp8(inference_params, Lc)
+            start = meta_args.slice_point * Lc
+            if inference_params.update_kv_cache:
+                n_keep = S - Lc if meta_args.distill_nearly_clean_chunk else S
+            if type(cache) is not Fp8KVCache or S % Lc or start < 0 or n_keep < 0 or start + n_keep > cache.max_sequence_length:
+                return None
+            chunks = (start + n_keep) // Lc
+            for t, dtype, heads, rows in ((cache.k, torch.float8_e4m3fn, (Hkv, D), start + n_keep), (cache.v, torch.float8_e4m3fn, (Hkv, D), start + n_keep),
+                                          (cache.k_scale, torch.float32, (Hkv,), chunks), (cache.v_scale, torch.float32, (Hkv,), chunks)):
+                if (type(t) is not torch.Tensor or t.dtype is not dtype or t.shape[1:] != heads or t.shape[0] < rows or not t.is_contiguous()
+                        or t.device != dev or t.data_ptr() % 16):
+                    return None
+        if Lc <= 0:
+            return None
+        p, cp = meta_args.core_attn_params, meta_args.cross_attn_params
+        if rope.dim() != 2 or rope.shape[0] != S:
+            raise ValueError("rope must be a contiguous fp32 [S / batch, 2*R2] tensor")
+        core_n = range_count(p.q_range, p.k_range, L.MAGI_RANGES_PAIRS)
+        cross_n = range_count(cp.cu_seqlens_q, cp.cu_seqlens_kv, L.MAGI_RANGES_CU)
+        q_scale, k_scale = self.fp8_operand_scales()
+        (gq, bq), (gk, bk), (gx, bx), (gkx, bkx) = self._norm_parameters()
+        n_side = S - n_keep  # rows that must not be persisted (all of them without a cache), in chunks of their own
+        side_chunks = (n_side + Lc - 1) // Lc
+        # one buffer: raw cross-attention q, v, the text's K | V rows (bf16), the e4m3 q, K and V rows that are not kept and the latter's scales
+        sizes = (2 * D * Hq * S, 2 * row * S, 4 * row * T, D * Hq * S, row * n_side, row * n_side, 4 * side_chunks * Hkv)
+        at = list(itertools.accumulate(((n + 255) // 256 * 256 for n in sizes), initial=0))
+        ws = torch.empty(at[-1], dtype=torch.uint8, device=dev)
+        qx, v_raw, text_kv, q8, k_side, v_side, vs_side = (ws.data_ptr() + o for o in at[:-1])
+        tables = self._const_scale_table(q_scale, (S + Lc - 1) // Lc, Hq, dev)
+        side_ks = self._const_scale_table(k_scale, max(side_chunks, 1), Hkv, dev)
+        outs, core_out, cross_out, o_row, groups, o_group, clear = self._small_layer_outputs(S, dev, proj_layout, core_n, p.max_seqlen_q, cross_n,
+                                                                                             cp.max_seqlen_q)
+        if cache is None:  # everything in the one buffer
+            k_new, v_new, vs_new, kept, k_tail, v_tail, vs_tail = k_side, v_side, vs_side, S, 0, 0, 0
+            k_all, v_all, scales, split, total = k_side, v_side, (tables.data_ptr(), side_ks.data_ptr(), vs_side, 0, 0), S, S
+        else:
+            if n_keep:
+                cache.note_constant_k_scale(k_scale, start // Lc, n_keep // Lc)
+            k_all, v_all = cache.k.data_ptr(), cache.v.data_ptr()
+            k_new, v_new, vs_new, kept = k_all + start * row, v_all + start * row, cache.v_scale.data_ptr() + 4 * Hkv * (start // Lc), n_keep
+            k_tail, v_tail, vs_tail = (k_side, v_side, vs_side) if n_side else (0, 0, 0)
+            scales = (tables.data_ptr(), cache.k_scale.data_ptr(), cache.v_scale.data_ptr()) + ((side_ks.data_ptr(), vs_side) if n_side else (0, 0))
+            split, total = start + n_keep, start + S
+        launch_small_projections_e4m3(
+            dev, q_scale, k_scale, v_raw, hidden_states.data_ptr(), w.data_ptr(), lw.data_ptr(), lb.data_ptr(), K, S, K, int(lw.dtype is torch.float32),
+            ln.eps, Hq, Hkv, Hq, rope.shape[1] // 2, rope.data_ptr(), gq.data_ptr(), bq.data_ptr(), gk.data_ptr(), bk.data_ptr(), self.eps, 1,
+            self._q_premul, kept, q8, k_new, k_tail, row, row, qx, key_value_states.data_ptr(), wt.data_ptr(),
+            key_value_states.stride(0) if T > 1 else Kt, T, Kt, gkx.data_ptr(), bkx.data_ptr(), text_kv)
+        launch_quantize_fp8_split(dev, v_raw, row, D, S, Hkv, D, Lc, 1.0, 1, v_new if kept else 0, vs_new if kept else 0, kept, v_tail, vs_tail)
+        launch_fp8_attention(dev, q8, S, Hq, k_all, v_all, k_tail, v_tail, split, total, Hkv, scales, Lc, p.q_range, p.k_range, core_n,
+                             p.max_seqlen_q, p.max_seqlen_k, core_out, o_row, groups, o_group, clear, self.fp8_fast_exp2)
+        launch_bounded_attention(dev, qx, Hq * D, S, Hq, text_kv, 0, T, T, 2 * row, Hkv, cp.cu_seqlens_q, cp.cu_seqlens_kv, cross_n, L.MAGI_RANGES_CU,
+                                 cp.max_seqlen_q, cp.max_seqlen_kv, cross_out, o_row, groups, o_group, clear, bound_cross,
+                                 (gx.data_ptr(), bx.data_ptr(), self.eps))
+        return outs[0] if len(outs) == 1 else attn_linear_proj_input(*outs) if proj_layout else outs
 
     # ------------------------------------------------------------------ forward
     def forward(self, hidden_states: torch.Tensor, key_value_states: torch.Tensor,
@@ -1039,6 +1148,10 @@ class FullyParallelAttention(torch.nn.Module):
             "core_score_bound": bound_core, "cross": _KERNEL_NAMES[cross_bounded], "cross_score_bound": bound_cross}
         if core_bounded and cross_bounded and self.attention_dtype == "bf16":
             small = self._forward_small(hidden_states, key_value_states, inference_params, rope, meta_args, proj_layout, bound_core, bound_cross)
+            if small is not None:
+                return small
+        if cross_bounded and self.attention_dtype == "fp8":
+            small = self._forward_small_fp8(hidden_states, key_value_states, inference_params, rope, meta_args, proj_layout, bound_cross)
             if small is not None:
                 return small
         one_launch = (self.fused_projection and self.attention_dtype == "bf16" and bs == 1
@@ -1157,8 +1270,10 @@ _KERNEL_NAMES = ("online softmax, 32 rows per wavefront", "bounded-score, 64 row
 # the methods whose work forward() does in another shape, as long as they are these
 _OWN_FP8_LINEAR = _Own(PerTensorQuantizedFp8Linear, "forward")
 _OWN_PROJECTIONS = _Own(CustomLayerNormLinear, "forward_ln", "forward_qkvx")
-_OWN_SMALL_PROJECTIONS = _Own(CustomLayerNormLinear, "forward_ln", "forward_qkvx", "forward_ln_qkvx_rows", "_split")
+_OWN_SMALL_PROJECTIONS = _Own(CustomLayerNormLinear, "forward_ln", "forward_qkvx", "forward_ln_qkvx_rows", "_split", "fused_weight")
 _OWN_CROSS = _Own(FullyParallelAttention, "get_xqkv", "cross_attention")
 _CROSS_FUSED = FullyParallelAttention._cross_attention_fused
 _OWN_SMALL = _Own(FullyParallelAttention, "_project_rows", "_fused_qkv", "_cross_attention_fused")
 _OWN_SMALL_UNCACHED = _Own(FullyParallelAttention, "_project_rows", "_fused_qkv", "_cross_attention_fused", "core_attention")
+_OWN_SMALL_FP8 = _Own(FullyParallelAttention, "_project_rows", "_core_attention_fp8", "_cross_attention_fused")
+_GAMMA_BETA = FusedLayerNorm.gamma_beta_fp32
