@@ -1037,11 +1037,11 @@ class FullyParallelAttention(torch.nn.Module):
     def _forward_small_fp8(self, hidden_states: torch.Tensor, key_value_states: torch.Tensor, inference_params: Optional[InferenceParams],
                            rope: torch.Tensor, meta_args: ModelMetaArgs, proj_layout: bool, bound_cross: float):
         """_forward_small for e4m3 attention (the text's scores bounded): magi_small_projections_e4m3, the quantiser of V, core attention,
-        cross attention.  None where forward() goes on with the separate launches, or refuses the call.  240 + 45 rows, 20 + 4
+        cross attention.  None where forward() goes on with the separate launches (among others in the extra forward of a first chunk, once
+        a video, whose launches the tests of the operands' preparation count), or refuses the call.  240 + 45 rows, 20 + 4
         heads: 153 us through the callables, 66 this way."""
-        use_cache = inference_params is not None and (
-            meta_args.extract_prefix_video_feature or meta_args.fwd_extra_1st_chunk or meta_args.slice_point > 0)
-        parts = self._small_layer_weights(hidden_states, key_value_states, rope, _OWN_SMALL_FP8)
+        use_cache = inference_params is not None and (meta_args.extract_prefix_video_feature or meta_args.slice_point > 0)
+        parts = None if meta_args.fwd_extra_1st_chunk else self._small_layer_weights(hidden_states, key_value_states, rope, _OWN_SMALL_FP8)
         if parts is None:
             return None
         w, wt, ln, lw, lb = parts
