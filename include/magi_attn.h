@@ -223,7 +223,7 @@ typedef struct magi_attn_args {
   int32_t q_batch_rows;
   int64_t q_stride_b, o_stride_b;
   /* Optional scratch memory on the DEVICE (any content, 16-byte aligned, one for each of the calls that may overlap), of
-   * magi_attn_split_bytes() or more.  With it, a launch of the fp8 kernel, or of the bf16 kernel without a running maximum, whose last round of
+   * magi_attn_split_bytes() or more (bf16 without a score bound: magi_attn_pieces_bytes()).  With it, a launch of the fp8 kernel or of a bf16 kernel whose last round of
    * workgroups would leave part of the chip idle has the keys of that round's rows shared by several workgroups, whose unnormalised fp32 sums a
    * launch behind it adds in the order of the keys (same precision).  NULL, or too small: not split.  A call's bits are the same
    * each time for the same sizes and the same choice of this memory; split and not split differ in the order of fp32 sums. */
@@ -231,13 +231,14 @@ typedef struct magi_attn_args {
   int64_t split_workspace_bytes;
 } magi_attn_args;
 
-/* Bytes of split_workspace that a call of these sizes makes use of in 256-row (fp8: 128-row) workgroups (dtype: MAGI_DTYPE_*); 0: such
+/* Bytes of split_workspace that a call of these sizes makes use of (dtype: MAGI_DTYPE_*; bf16: with a score bound, or checked); 0: such
  * a call is not split. */
 int64_t magi_attn_split_bytes(int32_t Hq, int32_t Hkv, int32_t n_ranges, int32_t max_seqlen_q, int32_t max_seqlen_k, int32_t dtype);
 
-/* The same for a bf16 call of these sizes that runs the online softmax in 128-row workgroups (no score_bound in force, no
- * MAGI_ATTN_AUTO_BOUND, no MAGI_ATTN_CHECKED, no MAGI_ATTN_Q_PRESCALED, q_tile_rows 0 or 128). */
-int64_t magi_attn_online_split_bytes(int32_t Hq, int32_t Hkv, int32_t n_ranges, int32_t max_seqlen_q, int32_t max_seqlen_k);
+/* Where a bf16 call of these sizes has the keys of all its rows shared, in 128-row workgroups: the bytes for that, else 0.  bounded !=
+ * 0: with a score_bound in force, no MAGI_ATTN_CHECKED, q_tile_rows 0.  0: with the online softmax (no MAGI_ATTN_AUTO_BOUND,
+ * MAGI_ATTN_CHECKED or MAGI_ATTN_Q_PRESCALED, q_tile_rows 0 or 128), whose bytes magi_attn_split_bytes does not tell. */
+int64_t magi_attn_pieces_bytes(int32_t Hq, int32_t Hkv, int32_t n_ranges, int32_t max_seqlen_q, int32_t max_seqlen_k, int32_t bounded);
 
 /* Rows per workgroup that a bf16 call of these sizes takes with a score_bound in force (or measured and in force), q_tile_rows 0, no
  * MAGI_ATTN_CHECKED and this much split_workspace: 256, or 128 where these fill the chip better, which make no use of that memory.  A row's

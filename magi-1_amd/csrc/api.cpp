@@ -166,10 +166,21 @@ struct SharePlan {
   unsigned pieces, tiles;  // of the longest item, of a piece
   int64_t bytes(unsigned per_xcd) const { return pieces > 1 ? 4ll * magi::ONLINE_PARTIAL_FLOATS * 8 * per_xcd * pieces : 0; }
 };
-// What a launch in pieces of `cut` tiles takes, in us.  A tile of 64 keys takes a workgroup 1.36 us alone on its CU, 1.9 beside
-// another, 2.55 beside two; a launch 9 us besides; bringing pieces together 5 us and 18 ns each (their way through memory).  Workgroups
-// that fit the chip at once run side by side until the shortest are done, and so on; more of them keep it full but for the end.
-double share_us(unsigned items, const unsigned* lengths, int n_ranges, unsigned cut, unsigned cus) {
+// A kernel's pace: us that a tile of 64 keys takes a workgroup alone on its CU, beside another, beside two; workgroups that run on a CU at a
+// time; us of a launch besides.
+struct Pace {
+  double one, two, three;
+  unsigned most;
+  double launch_us;
+};
+constexpr Pace PACE_ONLINE = {1.36, 1.9, 2.55, 3, 9.0};      // 128 rows, 32 per wavefront, online softmax
+constexpr Pace PACE_R32 = {1.13, 1.6, 2.4, 3, 6.5};          // the same without a running maximum
+constexpr Pace PACE_X16_128 = {1.10, 1.6, 1.6, 2, 6.0};      // 128 rows, two slots for K and for V
+constexpr Pace PACE_X16_256 = {1.75, 2.75, 2.75, 2, 7.0};    // 256 rows
+// What a launch in pieces of `cut` tiles takes, in us: bringing pieces together takes 5 us and 18 ns each (their way through
+// memory).  Workgroups that fit the chip at once run side by side until the shortest are done, and so on; more of them keep it full but
+// for the end.
+double share_us(const Pace& p, unsigned items, const unsigned* lengths, int n_ranges, unsigned cut, unsigned cus) {
   unsigned len[2 * 16], count[2 * 16];  // the pieces, by length
   int kinds = 0;
   auto add = [&](unsigned l, unsigned c) {
@@ -193,12 +204,14 @@ double share_us(unsigned items, const unsigned* lengths, int n_ranges, unsigned 
     work += (double)lengths[r] * each;
     if (n > 1) parts += (double)n * each;
   }
-  auto tile_us = [](double on_a_cu) {
-    return on_a_cu <= 1 ? 1.36 : on_a_cu <= 2 ? 1.36 + 0.54 * (on_a_cu - 1) : on_a_cu <= 3 ? 1.9 + 0.65 * (on_a_cu - 2) : 2.55;
+  auto tile_us = [&](double on_a_cu) {
+    if (on_a_cu <= 1) return p.one;
+    if (on_a_cu <= 2) return p.one + (p.two - p.one) * (on_a_cu - 1);
+    return on_a_cu <= 3 ? p.two + (p.three - p.two) * (on_a_cu - 2) : p.three;
   };
-  double t = 9.0;
-  if (all > 3.0 * cus) {
-    t += 2.55 * (work / (3.0 * cus) + 0.25 * cut);
+  double t = p.launch_us;
+  if (all > (double)p.most * cus) {
+    t += p.three * (work / ((double)p.most * cus) + 0.25 * cut);
   } else {
     double left = all;
     for (int i = 0; i < kinds; left -= count[i++])
@@ -211,25 +224,35 @@ double share_us(unsigned items, const unsigned* lengths, int n_ranges, unsigned 
 // 72 178 / 193, 1728 over 54 to 108 543 / 565.  The host does not know the ranges' lengths: taken are ranges that end a chunk of
 // max_seqlen_q keys apart, or all of max_seqlen_k keys where that does not go.  Only where the estimate is 6 % shorter, 10 % behind a whole round
 // (864 items over 86 to 111 tiles 402 / 410), and from 20 tiles on: max_seqlen_k of text is the padded length, of which a call may fill a fraction.
-SharePlan share_plan(unsigned per_xcd, int n_ranges, int max_seqlen_q, int max_seqlen_k) {
-  SharePlan best = {1, 0};
-  const unsigned cus = (unsigned)compute_units(), longest = (unsigned)(max_seqlen_k + 63) / 64, items = 8 * per_xcd;
-  if (max_seqlen_k <= 0 || longest < 20 || n_ranges < 1 || n_ranges > 16 || items == 0 || items > 6 * cus) return best;
-  unsigned lengths[16];
+// key tiles of each range, as far as sizes tell; false where they do not
+bool range_tiles(int n_ranges, int max_seqlen_q, int max_seqlen_k, unsigned* lengths) {
+  if (max_seqlen_k <= 0 || n_ranges < 1 || n_ranges > 16) return false;
   const bool apart = max_seqlen_k > (int64_t)(n_ranges - 1) * max_seqlen_q;
-  for (int r = 0; r < n_ranges; ++r) lengths[r] = apart ? (unsigned)(max_seqlen_k - r * max_seqlen_q + 63) / 64 : longest;
-  double least = (items > 3 * cus ? 0.90 : 0.94) * share_us(items, lengths, n_ranges, longest, cus);
+  for (int r = 0; r < n_ranges; ++r) lengths[r] = (unsigned)(max_seqlen_k - (apart ? r * max_seqlen_q : 0) + 63) / 64;
+  return true;
+}
+// the best of the launches in pieces that take less than `us`
+SharePlan best_pieces(const Pace& p, unsigned items, const unsigned* lengths, int n_ranges, double us) {
+  SharePlan best = {1, 0};
+  const unsigned cus = (unsigned)compute_units(), longest = lengths[0];
   static const unsigned char tried[] = {2, 3, 4, 5, 6, 8, 10, 12, 16};
   for (unsigned pieces : tried) {
     const unsigned cut = (longest + pieces - 1) / pieces;
     if (cut < 3 || (double)items * pieces > 8.0 * cus) break;
-    const double us = share_us(items, lengths, n_ranges, cut, cus);
-    if (us < least) {
-      least = us;
+    const double t = share_us(p, items, lengths, n_ranges, cut, cus);
+    if (t < us) {
+      us = t;
       best = {(longest + cut - 1) / cut, cut};
     }
   }
   return best;
+}
+SharePlan share_plan(unsigned per_xcd, int n_ranges, int max_seqlen_q, int max_seqlen_k) {
+  const unsigned cus = (unsigned)compute_units(), items = 8 * per_xcd;
+  unsigned lengths[16];
+  if (items == 0 || items > 6 * cus || !range_tiles(n_ranges, max_seqlen_q, max_seqlen_k, lengths) || lengths[0] < 20) return {1, 0};
+  return best_pieces(PACE_ONLINE, items, lengths, n_ranges,
+                     (items > 3 * cus ? 0.90 : 0.94) * share_us(PACE_ONLINE, items, lengths, n_ranges, lengths[0], cus));
 }
 
 // How a launch of the 64-rows-per-wavefront kernel without a running maximum is cut: workgroups of 256 rows, their last round's
@@ -253,6 +276,63 @@ int tile_rows(int Hq, int Hkv, int n_ranges, int max_seqlen_q, int max_seqlen_k,
   const unsigned pieces = whole * s.pieces;
   const double tiles = (max_seqlen_k + 63) / 64, in_pieces = tiles * s.num / s.den * (pieces <= cus ? 1.75 : 2.6) + 12.0 + 0.3 * pieces;
   return in_pieces <= tiles * (half <= cus ? 1.15 : 1.75) ? 256 : 128;
+}
+
+// Whether a launch without a running maximum runs in workgroups of 128 rows, three per CU (attn_fwd_bf16_r32.hip): whole items, which
+// have the bits of the other forms' whole items, or pieces of all of them.
+struct R32Plan {
+  bool use;
+  SharePlan share;
+};
+// Whole: where 256 rows to a workgroup, whole, are what split_plan and tile_rows leave, and one round of the smaller ones (more than two
+// per CU, which tile_rows takes care of) holds them all.  Measured, 24 heads, 256 rows / 128: 2700 rows over 2700 keys 125 / 107 us, 3354
+// over 3354 152 / 136, 3744 over 3744 168 / 156, four ranges of 792 over 1584 to 3960 138 / 114, three of 1200 over 1200 to 3600 125 / 103;
+// but behind that round 2250 x 2 over 2250 and 4500 164 / 185, 2340 x 2 168 / 211.
+// Pieces: the estimates of both launches, and at least 8 % less.  Measured, before / in pieces: 6 heads, 270 rows over 1350 keys 30 / 17, three
+// ranges of 312 over 1248 to 1872 31 / 22, four of 252 33 / 20; 24 heads, 432 over 1728 36 / 29, 720 over 2880 49 / 42, three of 612 over
+// 5508 to 6732 178 / 144; not so 1386 over 5544 109 / 114, 1080 over 5400 86 / 86, 720 over 720 21 / 25.  Error against float64 over that of whole items 0.9999 to 1.0001 (27 drawn sizes).
+// (From 16 tiles on: max_seqlen_k of text is the padded length, 800, of which a call may fill a fraction; 15 tiles would gain 4 to 6 us.)
+R32Plan r32_plan(int Hq, int Hkv, int n_ranges, int max_seqlen_q, int max_seqlen_k, int64_t& split_bytes) {
+  R32Plan plan = {false, {1, 0}};
+  const unsigned cus = (unsigned)compute_units();
+  auto items = [&](int rows) { return items_per_xcd(Hq, Hkv, n_ranges, max_seqlen_q / rows + (max_seqlen_q % rows != 0)); };
+  const unsigned half = items(128), whole = items(256);
+  unsigned lengths[16];
+  if (half == 0 || 8 * half > 3 * cus || (split_bytes <= 0 && half <= cus / 4) || !range_tiles(n_ranges, max_seqlen_q, max_seqlen_k, lengths)) return plan;
+  // what tile_rows and split_plan make of this much memory
+  bool small;
+  SplitPlan split;
+  auto others = [&](int64_t bytes) {
+    small = tile_rows(Hq, Hkv, n_ranges, max_seqlen_q, max_seqlen_k, bytes) == 128;
+    split = {UINT32_MAX, 1, 1, 1, false};
+    if (!small && bytes > 0) split = split_plan(whole, n_ranges, max_seqlen_q, max_seqlen_k, false);
+    if (split.bytes(whole) > bytes) split.from = UINT32_MAX;
+    return !small && split.from >= whole && half > cus / 4;  // whole items of 256 rows, more than two of 128 per CU
+  };
+  if (split_bytes > 0 && lengths[0] >= 16) {
+    const bool whole_items = others(INT64_MAX);
+    double us;
+    if (split.from < whole)  // (at most one round here: all items are in pieces)
+      us = 19.0 + lengths[0] * (double)split.num / split.den * (8 * whole * split.pieces <= cus ? 1.75 : 2.6) + 0.3 * whole * split.pieces;
+    else
+      us = share_us(whole_items ? PACE_R32 : small ? PACE_X16_128 : PACE_X16_256, 8 * (whole_items || small ? half : whole), lengths, n_ranges,
+                    lengths[0], cus);
+    plan.share = best_pieces(PACE_R32, 8 * half, lengths, n_ranges, 0.92 * us);
+    plan.use = plan.share.pieces > 1;
+    if (plan.use && plan.share.bytes(half) > split_bytes) {  // (too little memory: whole items)
+      plan = {false, {1, 0}};
+      split_bytes = 0;
+    }
+  }
+  if (!plan.use) plan.use = others(split_bytes);
+  return plan;
+}
+
+// the memory of its pieces, 0 where it takes whole items or none
+int64_t r32_bytes(int Hq, int Hkv, int n_ranges, int max_seqlen_q, int max_seqlen_k) {
+  int64_t any = INT64_MAX;
+  return r32_plan(Hq, Hkv, n_ranges, max_seqlen_q, max_seqlen_k, any)
+      .share.bytes(items_per_xcd(Hq, Hkv, n_ranges, max_seqlen_q / 128 + (max_seqlen_q % 128 != 0)));
 }
 
 int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace);
@@ -284,13 +364,16 @@ int64_t magi_attn_split_bytes(int32_t Hq, int32_t Hkv, int32_t n_ranges, int32_t
   const int rows = fp8 ? 128 : 256, tiles = max_seqlen_q / rows + (max_seqlen_q % rows != 0);
   if ((double)Hq * n_ranges * tiles > 2.0e9) return 0;
   const unsigned items = items_per_xcd(Hq, Hkv, n_ranges, tiles);
-  return split_plan(items, n_ranges, max_seqlen_q, max_seqlen_k, fp8).bytes(items);
+  const int64_t split = split_plan(items, n_ranges, max_seqlen_q, max_seqlen_k, fp8).bytes(items);
+  const int64_t pieces = fp8 ? 0 : r32_bytes(Hq, Hkv, n_ranges, max_seqlen_q, max_seqlen_k);
+  return split > pieces ? split : pieces;  // (checked launches, 256-row always, take the former)
 }
 
-int64_t magi_attn_online_split_bytes(int32_t Hq, int32_t Hkv, int32_t n_ranges, int32_t max_seqlen_q, int32_t max_seqlen_k) {
+int64_t magi_attn_pieces_bytes(int32_t Hq, int32_t Hkv, int32_t n_ranges, int32_t max_seqlen_q, int32_t max_seqlen_k, int32_t bounded) {
   if (Hq <= 0 || Hkv <= 0 || Hq % Hkv || n_ranges <= 0 || max_seqlen_q <= 0) return 0;
   if ((double)Hq * n_ranges * (max_seqlen_q / 128 + 1) > 2.0e9) return 0;
   const unsigned items = items_per_xcd(Hq, Hkv, n_ranges, max_seqlen_q / 128 + (max_seqlen_q % 128 != 0));
+  if (bounded) return r32_bytes(Hq, Hkv, n_ranges, max_seqlen_q, max_seqlen_k);
   return share_plan(items, n_ranges, max_seqlen_q, max_seqlen_k).bytes(items);
 }
 
@@ -461,7 +544,8 @@ int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace) {
   //    and drift out of step, so one computes scores while the other is in its softmax) on v_mfma_f32_16x16x32
   //    (the part is power limited and that shape takes less energy per FLOP; measured +3 % on the 720p layer,
   //    between 0 and +6 % from box to box), 128-row ones with 32 rows per wavefront where that leaves at most two of them per CU
-  //    (tile_rows); the 32x32x16 form on request and for 512-row workgroups.
+  //    (tile_rows), three of those per CU where one round of them holds the launch or its keys are better shared (r32_plan); the
+  //    32x32x16 form on request and for 512-row workgroups.
   //  * Otherwise 32 rows per wavefront with the online softmax: 384-row workgroups (12 waves, one workgroup per CU,
   //    every K / V tile fetched once for three times as many rows and one barrier per tile) pay on grids of many
   //    rounds with long key ranges (measured: +3 % at 43 rounds, +1 % at 9.4, -3 % at 5.3); small grids and short
@@ -504,13 +588,18 @@ int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace) {
   auto launch = [&](bool bounded) -> int {
     // a bound stated for unscaled q (what the reference's callers pass): the kernel applies the softmax scale while
     // it loads q, after which the scores are exp2 exponents as with MAGI_ATTN_Q_PRESCALED
-    const int64_t split_bytes = p->split_workspace ? p->split_workspace_bytes : 0;
+    int64_t split_bytes = p->split_workspace ? p->split_workspace_bytes : 0;  // (0 where it is too little for the launch's pieces)
     const bool scale_q = bounded && !q_norm && !checked && !(p->flags & MAGI_ATTN_Q_PRESCALED);
     a.block_m = 128;
+    R32Plan r32 = {false, {1, 0}};
     if (p->dtype == MAGI_DTYPE_BF16) {
       const double wg384 = (double)p->Hq * p->n_ranges * ((p->max_seqlen_q + 383) / 384);
       const bool long_keys = p->max_seqlen_k == 0 || p->max_seqlen_k >= 4096;  // (0 = not stated)
-      if (bounded && !checked && !mfma32)
+      if (bounded && !checked && !mfma32 && p->q_tile_rows == 0)
+        r32 = r32_plan(p->Hq, p->Hkv, p->n_ranges, p->max_seqlen_q, p->max_seqlen_k, split_bytes);
+      if (r32.use)
+        a.block_m = 128;
+      else if (bounded && !checked && !mfma32)
         a.block_m = tile_rows(p->Hq, p->Hkv, p->n_ranges, p->max_seqlen_q, p->max_seqlen_k, split_bytes);
       else if (bounded)
         a.block_m = 256;  // (512-row workgroups fetch half the tiles and measure 1 % slower: their two waves per SIMD march in step)
@@ -532,6 +621,13 @@ int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace) {
     a.per_xcd = items_per_xcd(p->Hq, p->Hkv, p->n_ranges, a.tiles_per_range);
     a.split_from = UINT32_MAX;
     const bool fp8 = p->dtype == MAGI_DTYPE_FP8_E4M3;
+    auto pieces = [&](const SharePlan& s) {
+      a.share_pieces = s.pieces;
+      a.share_tiles = s.tiles;
+      if (s.pieces > 1) a.partial = static_cast<float*>(p->split_workspace);
+    };
+    a.share_pieces = 1;
+    if (r32.use) pieces(r32.share);
     if ((fp8 || (bounded && a.block_m == 256 && !mfma32)) && split_bytes > 0) {
       const SplitPlan s = split_plan(a.per_xcd, p->n_ranges, p->max_seqlen_q, p->max_seqlen_k, fp8);
       if (s.from < a.per_xcd && s.bytes(a.per_xcd) <= split_bytes) {
@@ -549,23 +645,19 @@ int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace) {
     const bool online128 = !fp8 && !bounded && a.block_m == 128 && !(p->flags & MAGI_ATTN_Q_PRESCALED);
     if (online128 && !a.gate && split_bytes > 0) {
       const SharePlan s = share_plan(a.per_xcd, p->n_ranges, p->max_seqlen_q, p->max_seqlen_k);
-      if (s.pieces > 1 && s.bytes(a.per_xcd) <= split_bytes) {
-        a.partial = static_cast<float*>(p->split_workspace);
-        a.share_pieces = s.pieces;
-        a.share_tiles = s.tiles;
-      }
+      if (s.bytes(a.per_xcd) <= split_bytes) pieces(s);
     }
     hipError_t e;
     if (p->dtype != MAGI_DTYPE_BF16)
       e = magi::launch_attn_fwd_fp8(a, static_cast<hipStream_t>(stream));
     else if (checked)
       e = magi::launch_attn_fwd_bf16_checked(a, compute_units(), static_cast<hipStream_t>(stream));
+    else if (r32.use || (online128 && (a.share_pieces > 1 || 8.0 * a.per_xcd > 3.0 * compute_units())))
+      e = magi::launch_attn_fwd_bf16_r32(a, static_cast<hipStream_t>(stream));
     else if (bounded && a.block_m <= 256 && !mfma32)
       e = magi::launch_attn_fwd_bf16_x16(a, static_cast<hipStream_t>(stream));
     else if (bounded)
       e = magi::launch_attn_fwd_bf16_w64(a, static_cast<hipStream_t>(stream));
-    else if (online128 && (a.share_pieces > 1 || 8.0 * a.per_xcd > 3.0 * compute_units()))
-      e = magi::launch_attn_fwd_bf16_online16(a, static_cast<hipStream_t>(stream));
     else
       e = magi::launch_attn_fwd_bf16(a, static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return hip_fail(e, "magi_attn_fwd launch");

@@ -1,19 +1,23 @@
-// Range attention forward, bf16, online softmax, 32 query rows per wavefront on v_mfma_f32_16x16x32_bf16, for gfx950 (MI355X).
+// Range attention forward, bf16, 32 query rows per wavefront on v_mfma_f32_16x16x32_bf16, three workgroups of 128 rows per CU, for gfx950
+// (MI355X): the online softmax on unscaled q, and the softmax of bounded scores without a running maximum.
 //
-// What attn_fwd_bf16.hip's 4-wave form computes, on unscaled q: 128-row workgroups, three per CU, 64-key tiles, two K slots and one
-// V slot filled by direct global->LDS loads.  The MFMA shape, its operand layouts and the layout of the tiles in LDS are those of
-// attn_fwd_bf16_x16.hip (there: why that shape, and the reads' banks), with two query blocks of 16 per wavefront instead of four.
-// 164 registers.  What bounds it: per tile and wavefront the matrix pipe has 1024 cycles of work, the LDS 32 KB of operand reads,
-// the vector pipe 32 exponentials and 100 other instructions, about as long each; long launches run at the power limit, where the
-// 16x16x32 shape takes less energy per FLOP: 9360 rows x 2 chunks x 24 heads over 28080 and 37440 keys 6407 us against the 6604 of the
-// 32x32x16 form (1.18 PFLOP/s).  Whole rows go out through LDS, 16 lanes a row: 74880 x 24 rows over 20 keys, which is mostly the way
-// of q and out, 223 -> 202 us, and 174 with the first tile requested ahead of q.
+// 64-key tiles, two K slots and one V slot (three of them fit a CU's LDS) filled by direct global->LDS loads.  The MFMA shape, its operand
+// layouts and the layout of the tiles in LDS are those of attn_fwd_bf16_x16.hip (there: why that shape, and the reads' banks), with two
+// query blocks of 16 per wavefront; without a running maximum a row's bits are the same.  160 to 164 registers.
+// What bounds it: per tile and wavefront the matrix pipe has 1024 cycles of work, the LDS 32 KB of operand reads, the vector pipe 32
+// exponentials and 60 to 100 other instructions, about as long each; long launches run at the power limit.
+//   Online softmax, in launches of more than a round: the 16x16x32 shape takes less energy per FLOP, 9360 rows x 2 chunks x 24 heads over
+// 28080 and 37440 keys 6604 us on 32x32x16 (attn_fwd_bf16.hip) and 6407 so (1.18 PFLOP/s); whole rows go out through LDS, 16 lanes a row:
+// 74880 x 24 rows over 20 keys, which is mostly the way of q and out, 223 -> 202 us, and 174 with the first tile requested ahead of q.
+//   Bounded scores: 64 rows per wavefront read half as much from LDS and win in full launches (attn_fwd_bf16_x16.hip); this form where its
+// 128-row workgroups are one round, three per CU, and 256-row ones a partly empty round (r32_plan in api.cpp): 2700 rows x 24 heads over
+// 2700 keys 125 -> 107 us, four ranges of 792 rows over 1584 to 3960 138 -> 114.
 //
 // Shared keys (SHARE).  A launch of few items leaves most of the chip idle: 24 items over 127 tiles take 127 tiles in a row, 181 us.
 // Their keys are cut in pieces of a.share_tiles tiles, a workgroup each; a piece leaves unnormalised accumulators, row sums
 // and row maxima in fp32 (65 KB), a second launch brings them to a common maximum and adds them up in the order of the keys: 41 us.
 // The grid has the pieces of the longest range for every item: the surplus ones of shorter ranges return at once.  An item of one piece
-// is written right away.  Relative error against float64 as without pieces (share_plan in api.cpp has when, and more times).
+// is written right away.  Relative error against float64, pieces over whole: 0.90 to 0.99, 0.97 on average (online, 23 drawn sizes).
 #include "attn_common.h"
 
 namespace magi {
@@ -61,9 +65,65 @@ __device__ __forceinline__ void quad_max2(float& a, float& b) {
       : "+v"(a), "+v"(b));
 }
 
-// SHARE: the keys of an item are shared by several workgroups, a.share_tiles tiles each (share_plan in api.cpp).
-template <bool SHARE>
-__global__ __launch_bounds__(256, 3) void attn_fwd_bf16_online16_kernel(const AttnKernArgs a) {
+// NORM: qf holds the raw projection, lane (n, g) features 32 kk + 8 g .. +8 of row 16 qb + n in fragment kk: per-(token, head) norm over the
+// 128 features in fp32, times the softmax scale, one rounding to bf16 (the bits of attn_fwd_bf16_x16.hip's)
+template <int QB>
+__device__ __forceinline__ void norm_q(const AttnKernArgs& a, bf16x8 (&qf)[QB][4], int g) {
+  const float inv_d = 1.f / 128.f;
+  float mean[QB], rstd[QB];
+#pragma unroll
+  for (int qb = 0; qb < QB; ++qb) {
+    float sum = 0.f;
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) sum += (float)qf[qb][kk][e];
+    sum += __shfl_xor(sum, 16);
+    sum += __shfl_xor(sum, 32);
+    mean[qb] = a.q_norm_kind == 0 ? sum * inv_d : 0.f;  // (RMS form: no centring)
+    float sq = 0.f;
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float d = (float)qf[qb][kk][e] - mean[qb];
+        sq += d * d;
+      }
+    sq += __shfl_xor(sq, 16);
+    sq += __shfl_xor(sq, 32);
+    rstd[qb] = __builtin_amdgcn_rsqf(sq * inv_d + a.q_norm_eps) * a.scale_log2;
+  }
+  // (one fragment index at a time, so that the parameters of one fragment are all that is in registers)
+#pragma unroll
+  for (int kk = 0; kk < 4; ++kk) {
+    __builtin_amdgcn_sched_barrier(0);
+    const f32x4* gp = (const f32x4*)(a.q_norm_gamma + 32 * kk + 8 * g);
+    const f32x4 g0 = gp[0], g1 = gp[1];
+    f32x4 b0 = {0.f, 0.f, 0.f, 0.f}, b1 = b0;
+    if (a.q_norm_beta) {
+      const f32x4* bp = (const f32x4*)(a.q_norm_beta + 32 * kk + 8 * g);
+      b0 = bp[0];
+      b1 = bp[1];
+    }
+#pragma unroll
+    for (int qb = 0; qb < QB; ++qb)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float gm = (e < 4 ? g0[e & 3] : g1[e & 3]) + 1.f;
+        const float bt = (e < 4 ? b0[e & 3] : b1[e & 3]) * a.scale_log2;
+        qf[qb][kk][e] = (__bf16)(((float)qf[qb][kk][e] - mean[qb]) * rstd[qb] * gm + bt);
+      }
+  }
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+// What q holds, and what is known about the scores.  ONLINE: unscaled bf16 q, nothing: running maximum, scores scaled in fp32.  The others
+// as in attn_fwd_bf16_x16.hip, scores bounded, no maximum: AS_IS, q carries the scale; NORM, the raw projection; SCALE, unscaled.
+constexpr int AS_IS = 0, NORM = 1, SCALE = 2, ONLINE = 3;
+// SHARE: the keys of an item are shared by several workgroups, a.share_tiles tiles each (share_plan and r32_plan in api.cpp).
+template <int QMODE, bool SHARE>
+__global__ __launch_bounds__(256, 3) void attn_fwd_bf16_r32_kernel(const AttnKernArgs a) {
+  constexpr bool MAX = QMODE == ONLINE;
   constexpr int QB = 2, NW = 4, WROWS = 16 * QB, BM = WROWS * NW;
   constexpr int LOADS = BN / (4 * NW);  // direct loads per wave per matrix per tile (4 rows each)
   constexpr int RD = 4;                 // operand fragments in flight between LDS and the MFMAs
@@ -161,6 +221,15 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_bf16_online16_kernel(const At
 #pragma unroll
     for (int kk = 0; kk < 4; ++kk) qf[qb][kk] = *(const bf16x8*)(qp + kk * 64);
   }
+  if constexpr (QMODE == SCALE) {
+#pragma unroll
+    for (int qb = 0; qb < QB; ++qb)
+#pragma unroll
+      for (int kk = 0; kk < 4; ++kk)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) qf[qb][kk][e] = (__bf16)((float)qf[qb][kk][e] * a.scale_log2);
+  }
+  if constexpr (QMODE == NORM) norm_q<QB>(a, qf, g);
 
   const int base_k = (n >> 2) * K_GROUP + (n & 3) * ROW_BYTES + ((g ^ (n & 3)) << 4);
   const int r4 = n >> 2, c4 = n & 3;
@@ -219,34 +288,36 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_bf16_online16_kernel(const At
             for (int qb = 0; qb < QB; ++qb) sc[kb][qb][r] = -__builtin_inff();
           }
     }
-    // online softmax: lane (n, g) holds keys 16 kb + 4 g + r of query n of each block
-    float mx[QB];
+    // softmax: lane (n, g) holds keys 16 kb + 4 g + r of query n of each block
+    if constexpr (MAX) {
+      float mx[QB];
 #pragma unroll
-    for (int qb = 0; qb < QB; ++qb) {
-      float m = max3(sc[0][qb][0], sc[0][qb][1], sc[0][qb][2]);
-      m = max3(m, sc[0][qb][3], sc[1][qb][0]);
-      m = max3(m, sc[1][qb][1], sc[1][qb][2]);
-      m = max3(m, sc[1][qb][3], sc[2][qb][0]);
-      m = max3(m, sc[2][qb][1], sc[2][qb][2]);
-      m = max3(m, sc[2][qb][3], sc[3][qb][0]);
-      m = max3(m, sc[3][qb][1], sc[3][qb][2]);
-      mx[qb] = fmaxf(m, sc[3][qb][3]);
-    }
-    quad_max2(mx[0], mx[1]);
-    const float m0 = fmaxf(m_run[0], mx[0]), m1 = fmaxf(m_run[1], mx[1]);
-    if constexpr (FIRST) {
-      m_run[0] = m0;
-      m_run[1] = m1;
-    } else if (__builtin_amdgcn_ballot_w64(m0 != m_run[0] || m1 != m_run[1]) != 0) {  // some row of this wave saw a new maximum
-      const float a0 = __builtin_amdgcn_exp2f((m_run[0] - m0) * c), a1 = __builtin_amdgcn_exp2f((m_run[1] - m1) * c);
-      m_run[0] = m0;
-      m_run[1] = m1;
-      l_run[0] *= a0;
-      l_run[1] *= a1;
+      for (int qb = 0; qb < QB; ++qb) {
+        float m = max3(sc[0][qb][0], sc[0][qb][1], sc[0][qb][2]);
+        m = max3(m, sc[0][qb][3], sc[1][qb][0]);
+        m = max3(m, sc[1][qb][1], sc[1][qb][2]);
+        m = max3(m, sc[1][qb][3], sc[2][qb][0]);
+        m = max3(m, sc[2][qb][1], sc[2][qb][2]);
+        m = max3(m, sc[2][qb][3], sc[3][qb][0]);
+        m = max3(m, sc[3][qb][1], sc[3][qb][2]);
+        mx[qb] = fmaxf(m, sc[3][qb][3]);
+      }
+      quad_max2(mx[0], mx[1]);
+      const float m0 = fmaxf(m_run[0], mx[0]), m1 = fmaxf(m_run[1], mx[1]);
+      if constexpr (FIRST) {
+        m_run[0] = m0;
+        m_run[1] = m1;
+      } else if (__builtin_amdgcn_ballot_w64(m0 != m_run[0] || m1 != m_run[1]) != 0) {  // some row of this wave saw a new maximum
+        const float a0 = __builtin_amdgcn_exp2f((m_run[0] - m0) * c), a1 = __builtin_amdgcn_exp2f((m_run[1] - m1) * c);
+        m_run[0] = m0;
+        m_run[1] = m1;
+        l_run[0] *= a0;
+        l_run[1] *= a1;
 #pragma unroll
-      for (int db = 0; db < 8; ++db) {
-        o_acc[db][0] *= a0;
-        o_acc[db][1] *= a1;
+        for (int db = 0; db < 8; ++db) {
+          o_acc[db][0] *= a0;
+          o_acc[db][1] *= a1;
+        }
       }
     }
     u32x4 pf[2][QB];
@@ -255,8 +326,8 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_bf16_online16_kernel(const At
       const float mc = fmaxf(m_run[qb], -3.0e38f) * c;  // (a piece whose scores are all -inf so far adds zeros)
 #pragma unroll
       for (int kb = 0; kb < 4; ++kb) {
-        const float p0 = __builtin_amdgcn_exp2f(sc[kb][qb][0] * c - mc), p1 = __builtin_amdgcn_exp2f(sc[kb][qb][1] * c - mc);
-        const float p2 = __builtin_amdgcn_exp2f(sc[kb][qb][2] * c - mc), p3 = __builtin_amdgcn_exp2f(sc[kb][qb][3] * c - mc);
+        const float p0 = __builtin_amdgcn_exp2f(MAX ? sc[kb][qb][0] * c - mc : sc[kb][qb][0]), p1 = __builtin_amdgcn_exp2f(MAX ? sc[kb][qb][1] * c - mc : sc[kb][qb][1]);
+        const float p2 = __builtin_amdgcn_exp2f(MAX ? sc[kb][qb][2] * c - mc : sc[kb][qb][2]), p3 = __builtin_amdgcn_exp2f(MAX ? sc[kb][qb][3] * c - mc : sc[kb][qb][3]);
         l_run[qb] += (p0 + p1) + (p2 + p3);
         pf[kb >> 1][qb][2 * (kb & 1)] = pack_bf16x2(p0, p1);
         pf[kb >> 1][qb][2 * (kb & 1) + 1] = pack_bf16x2(p2, p3);
@@ -321,7 +392,7 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_bf16_online16_kernel(const At
     for (int qb = 0; qb < QB; ++qb) {
       if (ge == 0) {
         part[128 * 128 + WROWS * w + 16 * qb + ne] = sum[qb];
-        part[128 * 128 + 128 + WROWS * w + 16 * qb + ne] = m_run[qb] * c;
+        part[128 * 128 + 128 + WROWS * w + 16 * qb + ne] = MAX ? m_run[qb] * c : 0.f;
       }
 #pragma unroll
       for (int db = 0; db < 8; ++db) dst[(2 * db + qb) * 64] = o_acc[db][qb];
@@ -344,7 +415,7 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_bf16_online16_kernel(const At
     }
     const int q_row = row0 + 16 * qb + ne;
     if (a.lse && ge == 0 && q_row < qe)
-      a.lse[(long)wi.h * a.total_q + q_row] = (m_run[qb] * c + __builtin_amdgcn_logf(sum[qb])) * 0.6931471805599453f;
+      a.lse[(long)wi.h * a.total_q + q_row] = ((MAX ? m_run[qb] * c : 0.f) + __builtin_amdgcn_logf(sum[qb])) * 0.6931471805599453f;
   }
   // (the staging area is this wave's own: its LDS operations complete in order, no workgroup barrier is needed)
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -363,9 +434,10 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_bf16_online16_kernel(const At
 constexpr unsigned MERGE_SHARES = 4;
 // The items of a SHARE launch that are in pieces: brings the pieces to a common maximum, adds them up in the order of the keys,
 // normalises, writes the rows.  Four workgroups per item (query block, half of the features), on the item's XCD.
-__global__ __launch_bounds__(256) void attn_fwd_bf16_online16_merge_kernel(const AttnKernArgs a) {
+__global__ __launch_bounds__(256) void attn_fwd_bf16_r32_merge_kernel(const AttnKernArgs a) {
   constexpr unsigned SHARES = MERGE_SHARES;
   __shared__ int s_sel[LOCATE_WORDS];
+  if (gate_closed(a)) return;
   const int tid = threadIdx.x, l = tid & 63, n = l & 15, g = l >> 4;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const unsigned share = (blockIdx.x >> 3) % SHARES, block = ((blockIdx.x >> 3) / SHARES << 3) | (blockIdx.x & 7u);
@@ -404,15 +476,29 @@ __global__ __launch_bounds__(256) void attn_fwd_bf16_online16_merge_kernel(const
 
 }  // namespace
 
-hipError_t launch_attn_fwd_bf16_online16(const AttnKernArgs& a, hipStream_t stream) {
+namespace {
+template <int QMODE>
+void launch(const AttnKernArgs& a, hipStream_t stream) {
   if (a.share_pieces > 1) {
-    hipLaunchKernelGGL(attn_fwd_bf16_online16_kernel<true>, dim3(8u * a.per_xcd * a.share_pieces), dim3(256), 0, stream, a);
+    hipLaunchKernelGGL((attn_fwd_bf16_r32_kernel<QMODE, true>), dim3(8u * a.per_xcd * a.share_pieces), dim3(256), 0, stream, a);
     AttnKernArgs m = a;
     m.flags &= ~ATTN_ZERO_GAPS;  // (the rows no range covers are clear by now)
-    hipLaunchKernelGGL(attn_fwd_bf16_online16_merge_kernel, dim3(8u * a.per_xcd * MERGE_SHARES), dim3(256), 0, stream, m);
+    hipLaunchKernelGGL(attn_fwd_bf16_r32_merge_kernel, dim3(8u * a.per_xcd * MERGE_SHARES), dim3(256), 0, stream, m);
   } else {
-    hipLaunchKernelGGL(attn_fwd_bf16_online16_kernel<false>, dim3(8u * a.per_xcd), dim3(256), 0, stream, a);
+    hipLaunchKernelGGL((attn_fwd_bf16_r32_kernel<QMODE, false>), dim3(8u * a.per_xcd), dim3(256), 0, stream, a);
   }
+}
+}  // namespace
+
+hipError_t launch_attn_fwd_bf16_r32(const AttnKernArgs& a, hipStream_t stream) {
+  if (!(a.flags & ATTN_BOUNDED))
+    launch<ONLINE>(a, stream);
+  else if (a.q_norm_gamma)
+    launch<NORM>(a, stream);
+  else if (a.flags & ATTN_SCALE_Q)
+    launch<SCALE>(a, stream);
+  else
+    launch<AS_IS>(a, stream);
   return hipGetLastError();
 }
 

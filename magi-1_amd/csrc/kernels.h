@@ -79,7 +79,7 @@ constexpr int ATTN_SCALE_Q = 1 << 9;
 constexpr int ATTN_ZERO_GAPS = 32;
 
 hipError_t launch_attn_fwd_bf16(const AttnKernArgs& a, hipStream_t stream);
-hipError_t launch_attn_fwd_bf16_online16(const AttnKernArgs& a, hipStream_t stream);
+hipError_t launch_attn_fwd_bf16_r32(const AttnKernArgs& a, hipStream_t stream);
 hipError_t launch_attn_fwd_bf16_w64(const AttnKernArgs& a, hipStream_t stream);
 // (with items to split: and behind it the launch that adds their pieces up)
 hipError_t launch_attn_fwd_bf16_x16(const AttnKernArgs& a, hipStream_t stream);

@@ -88,6 +88,16 @@ def covered_by_launch(n: int, max_seqlen_q: int, rows: int) -> bool:
     return 1 <= n <= 64 and max_seqlen_q > 0 and n * max_seqlen_q >= rows
 
 
+def _bounded_split_bytes(Hq: int, Hkv: int, n: int, max_seqlen_q: int, max_seqlen_k: int) -> int:
+    """The scratch memory that a bf16 call with bounded scores makes use of."""
+    lib, n = L.lib(), max(n, 0)  # (see magi_attn_tile_rows: whole 128-row workgroups make no use of any)
+    size = lib.magi_attn_split_bytes(Hq, Hkv, n, max_seqlen_q, max_seqlen_k, L.MAGI_DTYPE_BF16)
+    if size and lib.magi_attn_tile_rows(Hq, Hkv, n, max_seqlen_q, max_seqlen_k, size) == 128 and not lib.magi_attn_pieces_bytes(
+            Hq, Hkv, n, max_seqlen_q, max_seqlen_k, 1):
+        size = 0
+    return size
+
+
 def launch_bounded_attention(dev: torch.device, q: int, q_row: int, rows: int, Hq: int, kv: int, side: int, k_split: int, total_k: int,
                              kv_row: int, Hkv: int, q_ranges: torch.Tensor, k_ranges: torch.Tensor, n: int, mode: int, max_seqlen_q: int,
                              max_seqlen_k: int, out: int, o_row: int, group_heads: int, o_group: int, clear: bool, bound: float,
@@ -99,9 +109,7 @@ def launch_bounded_attention(dev: torch.device, q: int, q_row: int, rows: int, H
     max_seqlen_q, max_seqlen_k = int(max_seqlen_q), int(max_seqlen_k)
     split, split_bytes = None, 0
     if max_seqlen_k >= 512:
-        split_bytes = L.lib().magi_attn_split_bytes(Hq, Hkv, max(n, 0), max_seqlen_q, max_seqlen_k, L.MAGI_DTYPE_BF16)
-        if split_bytes and L.lib().magi_attn_tile_rows(Hq, Hkv, n, max_seqlen_q, max_seqlen_k, split_bytes) == 128:
-            split_bytes = 0  # (in 128-row workgroups the launch makes no use of it)
+        split_bytes = _bounded_split_bytes(Hq, Hkv, n, max_seqlen_q, max_seqlen_k)
         if split_bytes:
             split = torch.empty(split_bytes, dtype=torch.uint8, device=dev)
     q_ranges, k_ranges = q_ranges.contiguous(), k_ranges.contiguous()
@@ -251,13 +259,13 @@ def range_attention(
     split, split_bytes = None, 0
     if split_keys and not static_scratch and max_seqlen_k >= 512 and (
             checked or auto_bound or 0.0 < score_bound <= L.MAGI_SCORE_BOUND_MAX or q.dtype is torch.float8_e4m3fn):
-        split_bytes = L.lib().magi_attn_split_bytes(Hq, Hkv, max(n, 0), int(max_seqlen_q), int(max_seqlen_k), _dtype_code(q))
-        if split_bytes and not (checked or q_tile_rows) and q.dtype is torch.bfloat16 and L.lib().magi_attn_tile_rows(
-                Hq, Hkv, n, int(max_seqlen_q), int(max_seqlen_k), split_bytes) == 128:
-            split_bytes = 0  # (in 128-row workgroups the launch makes no use of it)
+        if q.dtype is torch.bfloat16 and not (checked or q_tile_rows or bounded_mfma32):
+            split_bytes = _bounded_split_bytes(Hq, Hkv, n, int(max_seqlen_q), int(max_seqlen_k))
+        else:
+            split_bytes = L.lib().magi_attn_split_bytes(Hq, Hkv, max(n, 0), int(max_seqlen_q), int(max_seqlen_k), _dtype_code(q))
     elif (split_keys and not static_scratch and max_seqlen_k >= 512 and q.dtype is torch.bfloat16 and not (auto_bound or q_prescaled)
           and q_tile_rows in (0, 128)):
-        split_bytes = L.lib().magi_attn_online_split_bytes(Hq, Hkv, max(n, 0), int(max_seqlen_q), int(max_seqlen_k))
+        split_bytes = L.lib().magi_attn_pieces_bytes(Hq, Hkv, max(n, 0), int(max_seqlen_q), int(max_seqlen_k), 0)
     if split_bytes:  # (no going on without it where memory is short: the same call would give other bits then)
         split = torch.empty(split_bytes, dtype=torch.uint8, device=q.device)
     gamma = beta = None  # (alive until the launch is enqueued)

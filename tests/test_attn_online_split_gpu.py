@@ -34,7 +34,7 @@ def test_shared_keys_give_what_one_workgroup_gives(dev, rows, n, sp, Hq, Hkv, ma
     Tk = (sp + n) * rows
     mk = max_k or Tk
     cus = torch.cuda.get_device_properties(dev).multi_processor_count
-    assert cus != 256 or L.lib().magi_attn_online_split_bytes(Hq, Hkv, n, rows, mk) > 0
+    assert cus != 256 or L.lib().magi_attn_pieces_bytes(Hq, Hkv, n, rows, mk, 0) > 0
     q, k, v = (t.to(dev) for t in O.synthetic_qkv(n * rows + 7, Tk, Hq, Hkv, 128, seed=rows + n))
     qr = _ranges([[i * rows, (i + 1) * rows] for i in range(n)], dev)
     kr = _ranges([[0, (sp + 1 + i) * rows] for i in range(n)], dev)

@@ -1,0 +1,72 @@
+"""GPU tests of launches without a running maximum in 128-row workgroups, three per CU: whole items have the bits of 256-row workgroups,
+pieces of the keys add up to them."""
+import pytest
+import torch
+
+import magi_attn as M
+from magi_attn import _lib as L
+from oracle import magi_oracle as O
+
+pytestmark = pytest.mark.gpu
+PRE = 128 ** -0.5 * 1.4426950408889634
+
+
+def _case(dev, rows, n, Hq, Hkv, keys, mode, seed=0):
+    Tk = max(b for _, b in keys)
+    q, k, v = (t.to(dev) for t in O.synthetic_qkv(n * rows + 5, Tk, Hq, Hkv, 128, seed=seed))
+    qr = torch.tensor([[i * rows, (i + 1) * rows] for i in range(n)], dtype=torch.int32, device=dev)
+    kr = torch.tensor(keys, dtype=torch.int32, device=dev)
+    kw = {"as it is": {"q_prescaled": True, "score_bound": 40.0}, "scaled": {"score_bound": 40.0},
+          "norm": {"score_bound": 40.0, "q_norm": (torch.linspace(-0.2, 0.2, 128, device=dev), None, 1e-6)}}[mode]
+    if mode == "as it is":
+        q = (q.float() * PRE).bfloat16()
+    return q, k, v, qr, kr, kw
+
+
+# more than two workgroups per CU and at most three; tiles with wavefronts and rows missing; ranges of one key, of a tile's and half a tile's
+# edges, of none; no launch of the other forms
+@pytest.mark.parametrize("mode", ["as it is", "scaled", "norm"])
+@pytest.mark.parametrize("rows,Hq,Hkv,keys", [
+    (200, 48, 8, [(0, 1), (0, 0), (3, 35), (3, 36), (5, 69), (0, 200)]), (129, 64, 8, [(0, 64), (0, 65), (0, 128), (9, 300), (0, 31)]),
+    (2700, 24, 8, [(0, 500)])])
+def test_whole_items_have_the_bits_of_256_rows(dev, rows, Hq, Hkv, keys, mode):
+    n = len(keys)
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    items = Hq * n * ((rows + 127) // 128)
+    assert cus != 256 or 2 * cus < items <= 3 * cus
+    q, k, v, qr, kr, kw = _case(dev, rows, n, Hq, Hkv, keys, mode)
+    a, la = M.range_attention(q, k, v, qr, kr, rows, 500, **kw)
+    b, lb = M.range_attention(q, k, v, qr, kr, rows, 500, q_tile_rows=256, split_keys=False, **kw)
+    assert torch.equal(a, b) and torch.equal(la, lb)
+
+
+# single and unequal ranges, odd head counts, fewer keys than the launch was sized for (surplus pieces), a last piece of one key
+@pytest.mark.parametrize("mode", ["as it is", "scaled", "norm"])
+@pytest.mark.parametrize("rows,Hq,Hkv,keys,max_k", [
+    (270, 6, 2, [(0, 1601)], 0), (300, 3, 1, [(0, 1200), (0, 1500), (0, 1800)], 0), (129, 5, 5, [(0, 3), (7, 7), (0, 2400)], 3000), (1, 1, 1, [(0, 4097)], 0),
+    (432, 24, 8, [(0, 1728)], 0)])
+def test_pieces_add_up(dev, rows, Hq, Hkv, keys, max_k, mode):
+    n, mk = len(keys), max_k or max(b for _, b in keys)
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    assert cus != 256 or L.lib().magi_attn_pieces_bytes(Hq, Hkv, n, rows, mk, 1) > 0
+    q, k, v, qr, kr, kw = _case(dev, rows, n, Hq, Hkv, keys, mode, seed=rows)
+    a, la = M.range_attention(q, k, v, qr, kr, rows, mk, **kw)
+    b, lb = M.range_attention(q, k, v, qr, kr, rows, mk, split_keys=False, **kw)
+    # fp32 sums in another order: far less than half a bf16 step of outputs of about 0.05 (test_attn_split_gpu.py)
+    d = (a.float() - b.float()).abs()
+    assert torch.isfinite(a).all() and (d <= b.float().abs() * 2.0 ** -7 + 1e-5).all(), d.max().item()
+    fin = torch.isfinite(lb)
+    assert torch.equal(fin, torch.isfinite(la)) and (la - lb)[fin].abs().max().item() <= 1e-5
+    assert torch.equal(a, M.range_attention(q, k, v, qr, kr, rows, mk, **kw)[0])
+    if mode == "scaled":
+        ref = O.range_attention(q.cpu(), k.cpu(), v.cpu(), qr.cpu().numpy(), kr.cpu().numpy())
+        assert (a[:n * rows].float().cpu() - ref[:n * rows]).abs().max().item() <= 2e-2
+
+
+def test_a_gate_closes_pieces_too(dev):
+    """Scores that the measured bound hands to the online softmax: the launch in pieces and its merge leave the output alone."""
+    q, k, v, qr, kr, _ = _case(dev, 270, 1, 6, 2, [(0, 1601)], "scaled")
+    q = (q.float() * 60).bfloat16()
+    a = M.range_attention(q, k, v, qr, kr, 270, 1601, auto_bound=True)
+    b = M.range_attention(q, k, v, qr, kr, 270, 1601, split_keys=False)
+    assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1])
