@@ -412,6 +412,62 @@ int magi_small_projections(const magi_small_proj_args* args, void* stream);
 int magi_small_projections_e4m3(const magi_small_proj_args* args, float q_quant_scale, float k_quant_scale, void* v_out, void* stream);
 
 /*
+ * The three launches of a small bf16 layer at batch 1 with bounded scores in one call: magi_small_projections (norm, q | k | v | qx, text K | V),
+ * the core attention of the rows q over [kv[:k_split] | kv_side], the cross attention of the rows qx over text_kv.  What it stands for
+ * in those calls' structs: strides in elements; heads 128 apart; K | V interleaved per head, kv_row elements a row, the new rows to kv_new (kept of
+ * them) and kv_side; q, qx [S, Hq, 128], text_kv [T, Hkv, 256]; pairs for core, cumulative lengths for cross; split workspaces of their own.
+ * parts: 1 = the first two, 2 = the last, 3 = all.  A refusal of one of the three is this call's, what is ahead of it has been launched.
+ */
+typedef struct magi_small_layer_args {
+  uint32_t struct_size; /* sizeof(magi_small_layer_args) */
+  int32_t parts;
+  const void* x;
+  const void* w;
+  const void* ln_w;
+  const void* ln_b;
+  const float* rope;
+  const float* gq;
+  const float* bq;
+  const float* gk;
+  const float* bk;
+  const void* text;
+  const void* w_text;
+  const float* gkx;
+  const float* bkx;
+  const float* gqx;
+  const float* bqx;
+  int64_t text_stride;
+  int32_t S, K, ln_params_fp32, T, Kt, Hq, Hkv, R2;
+  float ln_eps, eps, q_premul;
+  void* q;
+  void* qx;
+  void* text_kv;
+  void* kv;
+  void* kv_new;
+  void* kv_side;
+  int64_t kv_row;
+  int32_t kept, k_split, total_k;
+  int32_t out_group_heads;
+  int64_t o_stride_t, o_stride_g;
+  const int32_t* q_ranges;
+  const int32_t* k_ranges;
+  int32_t n_core, max_core_q, max_core_k, core_flags; /* MAGI_ATTN_ZERO_UNCOVERED or 0 */
+  float core_bound;
+  void* core_out;
+  void* core_split;
+  int64_t core_split_bytes;
+  const int32_t* cu_q;
+  const int32_t* cu_k;
+  int32_t n_cross, max_cross_q, max_cross_k, cross_flags;
+  float cross_bound;
+  void* cross_out;
+  void* cross_split;
+  int64_t cross_split_bytes;
+} magi_small_layer_args;
+
+int magi_small_layer(const magi_small_layer_args* args, void* stream);
+
+/*
  * LayerNorm of the layer input over its last axis: x [rows, cols] bf16 -> y [rows, cols] bf16 with fp32
  * statistics, y = (x - mean) / sqrt(var + eps) * weight + bias (plain weight, not the "+1" form).
  * Stands in for torch.nn.LayerNorm in CustomLayerNormLinear.forward_ln (dit_module.py:401, 412-413;

@@ -948,6 +948,110 @@ int magi_small_projections_e4m3(const magi_small_proj_args* p, float q_quant_sca
   return small_projections_impl(p, &e4m3, stream);
 }
 
+int magi_small_layer(const magi_small_layer_args* p, void* stream) {
+  if (!p) return fail(MAGI_EINVAL, "magi_small_layer: args is NULL");
+  MAGI_CHECK_LAYOUT("magi_small_layer", p);
+  if (p->parts < 1 || p->parts > 3) return fail(MAGI_EINVAL, "magi_small_layer: parts %d", p->parts);
+  auto at = [](void* base, int64_t elements) -> const void* { return base ? static_cast<char*>(base) + 2 * elements : nullptr; };
+  magi_attn_args a;
+  std::memset(&a, 0, sizeof(a));
+  a.struct_size = sizeof(a);
+  a.q_stride_t = (int64_t)p->Hq * 128;
+  a.q_stride_h = a.o_stride_h = a.D = 128;
+  a.k_stride_h = a.v_stride_h = 256;
+  a.total_q = p->S;
+  a.Hq = p->Hq;
+  a.Hkv = p->Hkv;
+  a.dtype = MAGI_DTYPE_BF16;
+  a.o_stride_t = p->o_stride_t;
+  a.o_stride_g = p->o_stride_g;
+  a.out_group_heads = p->out_group_heads;
+  if (p->parts & 1) {
+    magi_small_proj_args s;
+    std::memset(&s, 0, sizeof(s));
+    s.struct_size = sizeof(s);
+    s.x = p->x;
+    s.w = p->w;
+    s.ln_w = p->ln_w;
+    s.ln_b = p->ln_b;
+    s.x_stride = s.K = p->K;
+    s.S = p->S;
+    s.ln_params_fp32 = p->ln_params_fp32;
+    s.ln_eps = p->ln_eps;
+    s.Hq = s.Hqx = p->Hq;
+    s.Hkv = p->Hkv;
+    s.R2 = p->R2;
+    s.rope = p->rope;
+    s.gq = p->gq;
+    s.bq = p->bq;
+    s.gk = p->gk;
+    s.bk = p->bk;
+    s.eps = p->eps;
+    s.batch = 1;
+    s.q_premul = p->q_premul;
+    s.n_cache_rows = p->kept;
+    s.q_out = p->q;
+    s.kv_out = p->kv_new;
+    s.kv_tail = p->kv_side;
+    s.kv_stride_t = s.kv_tail_stride_t = p->kv_row;
+    s.qx_out = p->qx;
+    s.text = p->text;
+    s.w_text = p->w_text;
+    s.text_stride = p->text_stride;
+    s.T = p->T;
+    s.Kt = p->Kt;
+    s.gkx = p->gkx;
+    s.bkx = p->bkx;
+    s.text_out = p->text_kv;
+    if (const int rc = small_projections_impl(&s, nullptr, stream)) return rc;
+    a.q = p->q;
+    a.k = p->kv;
+    a.v = at(p->kv, 128);
+    a.k2 = p->kv_side;
+    a.v2 = at(p->kv_side, 128);
+    a.k_stride_t = a.v_stride_t = p->kv_row;
+    a.total_k = p->total_k;
+    a.k_split = p->k_split;
+    a.q_ranges = p->q_ranges;
+    a.k_ranges = p->k_ranges;
+    a.n_ranges = p->n_core;
+    a.ranges_mode = MAGI_RANGES_PAIRS;
+    a.max_seqlen_q = p->max_core_q;
+    a.max_seqlen_k = p->max_core_k;
+    a.flags = MAGI_ATTN_Q_PRESCALED | p->core_flags;
+    a.score_bound = p->core_bound;
+    a.out = p->core_out;
+    a.split_workspace = p->core_split;
+    a.split_workspace_bytes = p->core_split_bytes;
+    if (const int rc = attn_fwd_impl(&a, stream, nullptr)) return rc;
+  }
+  if (p->parts & 2) {
+    a.q = p->qx;
+    a.k = p->text_kv;
+    a.v = at(p->text_kv, 128);
+    a.k2 = a.v2 = nullptr;
+    a.k_stride_t = a.v_stride_t = (int64_t)p->Hkv * 256;
+    a.total_k = a.k_split = p->T;
+    a.q_ranges = p->cu_q;
+    a.k_ranges = p->cu_k;
+    a.n_ranges = p->n_cross;
+    a.ranges_mode = MAGI_RANGES_CU;
+    a.max_seqlen_q = p->max_cross_q;
+    a.max_seqlen_k = p->max_cross_k;
+    a.flags = p->cross_flags;
+    a.score_bound = p->cross_bound;
+    a.out = p->cross_out;
+    a.split_workspace = p->cross_split;
+    a.split_workspace_bytes = p->cross_split_bytes;
+    a.q_norm_gamma = p->gqx;
+    a.q_norm_beta = p->bqx;
+    a.q_norm_eps = p->eps;
+    a.q_norm_kind = MAGI_NORM_LAYERNORM_1P;
+    return attn_fwd_impl(&a, stream, nullptr);
+  }
+  return MAGI_OK;
+}
+
 int magi_layer_norm(const void* x, int64_t x_stride, const void* weight, const void* bias, int32_t params_fp32,
                     void* y, int64_t y_stride, int64_t rows, int32_t cols, float eps, void* stream) {
   if (rows < 0 || cols < 0) return fail(MAGI_EINVAL, "magi_layer_norm: negative size");

@@ -125,13 +125,32 @@ class SmallProjArgs(_SizedStructure):
     ]
 
 
+class SmallLayerArgs(_SizedStructure):
+    _fields_ = [
+        ("struct_size", C.c_uint32), ("parts", C.c_int32), ("x", C.c_void_p), ("w", C.c_void_p), ("ln_w", C.c_void_p),
+        ("ln_b", C.c_void_p), ("rope", C.c_void_p), ("gq", C.c_void_p), ("bq", C.c_void_p), ("gk", C.c_void_p), ("bk", C.c_void_p),
+        ("text", C.c_void_p), ("w_text", C.c_void_p), ("gkx", C.c_void_p), ("bkx", C.c_void_p), ("gqx", C.c_void_p), ("bqx", C.c_void_p),
+        ("text_stride", C.c_int64), ("S", C.c_int32), ("K", C.c_int32), ("ln_params_fp32", C.c_int32), ("T", C.c_int32), ("Kt", C.c_int32),
+        ("Hq", C.c_int32), ("Hkv", C.c_int32), ("R2", C.c_int32), ("ln_eps", C.c_float), ("eps", C.c_float), ("q_premul", C.c_float),
+        ("q", C.c_void_p), ("qx", C.c_void_p), ("text_kv", C.c_void_p), ("kv", C.c_void_p), ("kv_new", C.c_void_p),
+        ("kv_side", C.c_void_p), ("kv_row", C.c_int64), ("kept", C.c_int32), ("k_split", C.c_int32), ("total_k", C.c_int32),
+        ("out_group_heads", C.c_int32), ("o_stride_t", C.c_int64), ("o_stride_g", C.c_int64), ("q_ranges", C.c_void_p),
+        ("k_ranges", C.c_void_p), ("n_core", C.c_int32), ("max_core_q", C.c_int32), ("max_core_k", C.c_int32), ("core_flags", C.c_int32),
+        ("core_bound", C.c_float), ("core_out", C.c_void_p), ("core_split", C.c_void_p), ("core_split_bytes", C.c_int64),
+        ("cu_q", C.c_void_p), ("cu_k", C.c_void_p), ("n_cross", C.c_int32), ("max_cross_q", C.c_int32), ("max_cross_k", C.c_int32),
+        ("cross_flags", C.c_int32), ("cross_bound", C.c_float), ("cross_out", C.c_void_p), ("cross_split", C.c_void_p),
+        ("cross_split_bytes", C.c_int64),
+    ]
+
+
 ABI_VERSION = 104  # magi_version() of the library these mirrors were written for
 
 EXPORTS = ("magi_version", "magi_last_error", "magi_launch_count", "magi_attn_fwd", "magi_attn_fwd_static_scratch",
            "magi_attn_split_bytes", "magi_attn_pieces_bytes", "magi_attn_tile_rows",
            "magi_qk_prologue", "magi_head_norm",
            "magi_apply_rotary", "magi_quantize_fp8", "magi_quantize_fp8_split", "magi_layer_norm", "magi_qkv_proj_prologue", "magi_div_clamp_to_e4m3",
-           "magi_layer_norm_e4m3", "magi_small_projections", "magi_small_projections_e4m3")
+           "magi_layer_norm_e4m3", "magi_small_projections", "magi_small_projections_e4m3",
+           "magi_small_layer")
 
 _lib = None
 
@@ -185,6 +204,8 @@ def lib() -> C.CDLL:
         l.magi_qkv_proj_prologue.restype = C.c_int
         l.magi_small_projections.argtypes = [C.POINTER(SmallProjArgs), C.c_void_p]
         l.magi_small_projections.restype = C.c_int
+        l.magi_small_layer.argtypes = [C.POINTER(SmallLayerArgs), C.c_void_p]
+        l.magi_small_layer.restype = C.c_int
         l.magi_small_projections_e4m3.argtypes = [C.POINTER(SmallProjArgs), C.c_float, C.c_float, C.c_void_p, C.c_void_p]
         l.magi_small_projections_e4m3.restype = C.c_int
         l.magi_quantize_fp8_split.argtypes = [C.POINTER(QuantizeArgs), C.c_void_p]

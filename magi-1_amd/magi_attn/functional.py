@@ -562,6 +562,20 @@ def launch_small_projections_e4m3(dev: torch.device, q_scale: float, k_scale: fl
     _launch(dev, call.fn, call.pack(call.size, *fields), q_scale, k_scale, v_out)
 
 
+def launch_small_layer(dev: torch.device, parts: int, *fields) -> None:
+    """magi_small_layer with the fields of its argument struct behind parts, in order."""
+    _launch_packed(dev, "magi_small_layer", L.SmallLayerArgs, parts, *fields)
+
+
+def split_memory(dev: torch.device, Hq: int, Hkv: int, n: int, max_seqlen_q: int, max_seqlen_k: int):
+    """(the scratch memory that a bf16 call with bounded scores makes use of or None, its address, its bytes)"""
+    size = _bounded_split_bytes(Hq, Hkv, n, max_seqlen_q, max_seqlen_k) if max_seqlen_k >= 512 else 0
+    if not size:
+        return None, 0, 0
+    t = torch.empty(size, dtype=torch.uint8, device=dev)
+    return t, t.data_ptr(), size
+
+
 def launch_quantize_fp8_split(dev: torch.device, *fields) -> None:
     """magi_quantize_fp8_split with the fields of its argument struct behind struct_size, in order."""
     _launch_packed(dev, "magi_quantize_fp8_split", L.QuantizeArgs, *fields)
