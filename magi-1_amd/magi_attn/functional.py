@@ -152,6 +152,7 @@ def range_attention(
     checked: bool = False,
     static_scratch: bool = False,
     q_norm: Optional[tuple] = None,
+    clear_out: bool = False,
     out: Optional[torch.Tensor] = None,
     return_lse: bool = True,
     zero_init: bool = True,
@@ -190,6 +191,8 @@ def range_attention(
     [rows, batch, Hq, D] transposed.  Needs a score_bound (math.inf: the online softmax).
     q_norm: (gamma, beta or None, eps[, norm_kind]): q is the raw projection, normalised per (token, head) row inside
     the kernel (fp32, zero-centred gamma) and scaled by softmax_scale * log2(e); needs score_bound.
+    clear_out: rows of a given `out` that no range covers become zeros too.  A batched q's `out` may be [batch, rows, groups,
+    Hq / groups, D], as a 4-D one otherwise.
     """
     batched = q.dim() == 4
     _check_thd(q[0] if batched else q, "q")
@@ -208,8 +211,10 @@ def range_attention(
     n = range_count(q_ranges, k_ranges, ranges_mode)
     q_ranges = q_ranges.contiguous()
     k_ranges = k_ranges.contiguous()
-    by_kernel = out is None and covered_by_launch(n, max_seqlen_q, Tq)
-    zero_gaps = by_kernel and (zero_init or return_lse)
+    by_kernel = (out is None or clear_out) and covered_by_launch(n, max_seqlen_q, Tq)
+    zero_gaps = by_kernel and (zero_init or return_lse or clear_out)
+    if clear_out and out is not None and not by_kernel:
+        out.zero_()
     if out is None:
         new = torch.zeros if zero_init and not by_kernel else torch.empty
         out = new((q.shape[1], q.shape[0], Hq, D), dtype=torch.bfloat16, device=q.device).transpose(0, 1) if batched else \
@@ -239,14 +244,17 @@ def range_attention(
     q_stride, o_stride = q.stride(), out.stride()
     group_heads = o_stride_g = batch_rows = q_stride_b = o_stride_b = 0
     if batched:
-        if out.shape != q.shape or o_stride[3] != 1:
+        if len(o_stride) == 5 and out.shape[:2] == q.shape[:2] and out.shape[2] * out.shape[3] == Hq and out.shape[4] == D and o_stride[4] == 1:
+            o_stride_g, group_heads, o_stride_t = o_stride[2], out.shape[3], o_stride[1]
+        elif out.shape != q.shape or o_stride[3] != 1:
             raise ValueError("out must have the shape of a batched q, with contiguous rows")
         batch_rows, q_stride_b, o_stride_b = q.shape[1], q_stride[0], o_stride[0]
     elif len(o_stride) == 4:  # [Tq, groups, heads per group, D]: two-level head addressing
         if out.shape[0] != Tq or out.shape[1] * out.shape[2] != Hq or out.shape[3] != D or o_stride[3] != 1:
             raise ValueError("a 4-D out must be [Tq, groups, Hq / groups, D] with contiguous rows")
         o_stride_g, group_heads = o_stride[1], out.shape[2]
-    o_stride_t = o_stride[0] if group_heads else o_stride[-3]
+    if not (batched and group_heads):
+        o_stride_t = o_stride[0] if group_heads else o_stride[-3]
     flags = ((L.MAGI_ATTN_FP8_POW2_PRESCALED if fp8_pow2_prescaled else 0) | (L.MAGI_ATTN_Q_PRESCALED if q_prescaled else 0)
              | (L.MAGI_ATTN_FP8_FAST_EXP2 if fp8_fast_exp2 else 0) | (L.MAGI_ATTN_BOUNDED_MFMA32 if bounded_mfma32 else 0)
              | (L.MAGI_ATTN_AUTO_BOUND if auto_bound else 0) | (L.MAGI_ATTN_ZERO_UNCOVERED if zero_gaps else 0)

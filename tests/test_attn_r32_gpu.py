@@ -70,3 +70,21 @@ def test_a_gate_closes_pieces_too(dev):
     a = M.range_attention(q, k, v, qr, kr, 270, 1601, auto_bound=True)
     b = M.range_attention(q, k, v, qr, kr, 270, 1601, split_keys=False)
     assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1])
+
+
+@pytest.mark.parametrize("batch", [2, 3])
+def test_batched_rows_in_groups_of_heads(dev, batch):
+    rows, Hq, Hkv, n = 150, 8, 2, 90
+    torch.manual_seed(batch)
+    q = torch.randn(rows, batch, Hq, 128, device=dev).bfloat16().transpose(0, 1)
+    kv = torch.randn(n, Hkv, 256, device=dev).bfloat16()
+    cq = torch.tensor([0, rows], dtype=torch.int32, device=dev)  # (the other batch rows are covered by no range)
+    ck = torch.tensor([0, n], dtype=torch.int32, device=dev)
+    for bound in (60.0, float("inf")):
+        kw = dict(ranges_mode=L.MAGI_RANGES_CU, return_lse=False, score_bound=bound)
+        want, _ = M.range_attention(q, kv[..., :128], kv[..., 128:], cq, ck, batch * rows, n, **kw)
+        store = torch.full((rows, batch, 4, 2, 2, 128), float("nan"), dtype=torch.bfloat16, device=dev)
+        out = store[:, :, :, 1].transpose(0, 1)
+        got, _ = M.range_attention(q, kv[..., :128], kv[..., 128:], cq, ck, batch * rows, n, out=out, clear_out=True, **kw)
+        assert got is out and torch.equal(out.reshape(batch, rows, Hq, 128), want)
+        assert torch.isnan(store[:, :, :, 0]).all()
