@@ -241,8 +241,9 @@ int64_t magi_attn_split_bytes(int32_t Hq, int32_t Hkv, int32_t n_ranges, int32_t
 int64_t magi_attn_pieces_bytes(int32_t Hq, int32_t Hkv, int32_t n_ranges, int32_t max_seqlen_q, int32_t max_seqlen_k, int32_t bounded);
 
 /* Rows per workgroup that a bf16 call of these sizes takes with a score_bound in force (or measured and in force), q_tile_rows 0, no
- * MAGI_ATTN_CHECKED and this much split_workspace: 256, or 128 where these fill the chip better, which make no use of that memory.  A row's
- * bits are those of 256-row workgroups without it. */
+ * MAGI_ATTN_CHECKED and this much split_workspace, where the keys of all rows are not shared (magi_attn_pieces_bytes): 128 where two of these per
+ * CU or less fill the chip better, which make no use of that memory, else 256 (or up to three of 128 per CU instead of whole ones
+ * of 256 in a partly empty round).  A row's bits are the same in all of these, without that memory. */
 int32_t magi_attn_tile_rows(int32_t Hq, int32_t Hkv, int32_t n_ranges, int32_t max_seqlen_q, int32_t max_seqlen_k, int64_t split_workspace_bytes);
 
 int magi_attn_fwd(const magi_attn_args* args, void* stream);

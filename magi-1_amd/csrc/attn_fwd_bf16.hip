@@ -23,7 +23,8 @@
 // shallow operand prefetch):
 //   * 4 waves per workgroup, three workgroups per CU, 48 KB of LDS each (64-key tiles, K double
 //     buffered, ONE V slot that is refilled under the score MFMAs and the softmax of the same tile,
-//     two barriers per tile, slots named statically): small grids and short key ranges;
+//     two barriers per tile, slots named statically): small grids and short key ranges.  Unscaled q in launches of more than a
+//     round, or with the keys of an item shared, runs in attn_fwd_bf16_r32.hip instead (why: its head and magi_attn_fwd's dispatch);
 //   * 12 waves per workgroup (DB), ONE workgroup per CU, 64 KB of LDS (K and V double buffered in
 //     four statically named slots, one barrier per tile, the tile loads issued by four of the
 //     waves, one per SIMD): every K / V tile is fetched from L2 once
