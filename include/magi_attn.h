@@ -78,6 +78,10 @@ extern "C" {
  * MAGI_ATTN_BOUNDED_MFMA32 or MAGI_ATTN_AUTO_BOUND. */
 #define MAGI_ATTN_CHECKED 64
 
+/* bf16: a row's bits depend on its own range alone, not on how many rows the launch has besides.  The online softmax then keeps to one order of
+ * the keys (that of small launches) in all sizes; with a score_bound they do not anyhow.  Without split_workspace. */
+#define MAGI_ATTN_ROW_BITS 128
+
 #define MAGI_RANGES_PAIRS 0 /* int32 [n, 2]: range i = [r[2i], r[2i+1])          */
 #define MAGI_RANGES_CU 1    /* int32 [n + 1] cumulative: range i = [r[i], r[i+1]) */
 

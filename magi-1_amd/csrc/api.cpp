@@ -475,6 +475,8 @@ int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace) {
     if (!workspace || !aligned16(workspace))
       return fail(MAGI_EINVAL, "magi_attn_fwd: MAGI_ATTN_AUTO_BOUND needs a 16-byte workspace on the device, 16-byte aligned");
   }
+  if ((p->flags & MAGI_ATTN_ROW_BITS) && (p->split_workspace || p->dtype != MAGI_DTYPE_BF16))
+    return fail(MAGI_EINVAL, "magi_attn_fwd: MAGI_ATTN_ROW_BITS goes with bf16 and without split_workspace");
   const bool checked = (p->flags & MAGI_ATTN_CHECKED) != 0;
   if (checked) {
     if (p->dtype != MAGI_DTYPE_BF16 || p->score_bound > 0.f || q_norm || p->q_tile_rows != 0 ||
@@ -642,7 +644,8 @@ int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace) {
     // (three per CU) and for shared keys, the 32x32x16 form for the others.  Measured, 32x32x16 / 16x16x32: 9360 rows x 2
     // chunks x 24 heads over 28080 and 37440 keys 6604 / 6407 us, 93600 x 24 text cross attention 612 / 600, over 20 keys 223 / 202,
     // 4580 x 48 over 3435 to 6870 555 / 545; 700 x 24 over 700 22.3 / 23.2, 700 x 48 over 1400 48.5 / 50.7, 2000 x 24 57 / 58.
-    const bool online128 = !fp8 && !bounded && a.block_m == 128 && !(p->flags & MAGI_ATTN_Q_PRESCALED);
+    // (MAGI_ATTN_ROW_BITS: the 32x32x16 forms in all sizes, whose order of the keys is one.)
+    const bool online128 = !fp8 && !bounded && a.block_m == 128 && !(p->flags & (MAGI_ATTN_Q_PRESCALED | MAGI_ATTN_ROW_BITS));
     if (online128 && !a.gate && split_bytes > 0) {
       const SharePlan s = share_plan(a.per_xcd, p->n_ranges, p->max_seqlen_q, p->max_seqlen_k);
       if (s.bytes(a.per_xcd) <= split_bytes) pieces(s);

@@ -26,6 +26,7 @@ MAGI_ATTN_BOUNDED_MFMA32 = 8
 MAGI_ATTN_AUTO_BOUND = 16
 MAGI_ATTN_ZERO_UNCOVERED = 32
 MAGI_ATTN_CHECKED = 64
+MAGI_ATTN_ROW_BITS = 128
 MAGI_SCORE_BOUND_MAX = 64.0
 
 

@@ -185,7 +185,8 @@ def range_attention(
     softmax where the workgroups fill the chip, and its results are further from the exact ones (see _unbounded_mode).
     split_keys: False keeps the library from sharing the keys of a row among workgroups where that fills the chip better
     (magi_attn_args.split_workspace, up to 135 MB of scratch memory for the call; the fp32 sums are then added in another
-    order).  Whether it does follows from the sizes of the launch alone.  Needs max_seqlen_k.
+    order).  Whether it does follows from the sizes of the launch alone.  Needs max_seqlen_k.  Without it a bf16 row's bits depend on its
+    own range alone (MAGI_ATTN_ROW_BITS).
     q may be [batch, rows, Hq, D] with any batch stride (batch of activations laid out [position, batch, ...]): its rows
     count as batch * rows tokens for the ranges, out is (or comes back as) a tensor of q's shape, by default
     [rows, batch, Hq, D] transposed.  Needs a score_bound (math.inf: the online softmax).
@@ -258,7 +259,7 @@ def range_attention(
     flags = ((L.MAGI_ATTN_FP8_POW2_PRESCALED if fp8_pow2_prescaled else 0) | (L.MAGI_ATTN_Q_PRESCALED if q_prescaled else 0)
              | (L.MAGI_ATTN_FP8_FAST_EXP2 if fp8_fast_exp2 else 0) | (L.MAGI_ATTN_BOUNDED_MFMA32 if bounded_mfma32 else 0)
              | (L.MAGI_ATTN_AUTO_BOUND if auto_bound else 0) | (L.MAGI_ATTN_ZERO_UNCOVERED if zero_gaps else 0)
-             | (L.MAGI_ATTN_CHECKED if checked else 0))
+             | (L.MAGI_ATTN_CHECKED if checked else 0) | (0 if split_keys or q.dtype is not torch.bfloat16 else L.MAGI_ATTN_ROW_BITS))
     workspace = None
     if checked:
         workspace = torch.empty(max(4 * Hq * max(n, 0) * ((int(max_seqlen_q) + 255) // 256), 4), dtype=torch.int32, device=q.device)

@@ -88,3 +88,24 @@ def test_batched_rows_in_groups_of_heads(dev, batch):
         got, _ = M.range_attention(q, kv[..., :128], kv[..., 128:], cq, ck, batch * rows, n, out=out, clear_out=True, **kw)
         assert got is out and torch.equal(out.reshape(batch, rows, Hq, 128), want)
         assert torch.isnan(store[:, :, :, 0]).all()
+
+
+@pytest.mark.parametrize("rows,Hq,Hkv", [(1536, 24, 8), (130, 256, 32), (3500, 24, 8)])
+def test_rows_have_the_bits_of_their_range_alone(dev, rows, Hq, Hkv):
+    """Without shared keys, where all ranges are a launch of more than three workgroups per CU (and one range is not, or is in the larger
+    workgroups of many rounds): the online softmax keeps to one order of the keys."""
+    torch.manual_seed(rows)
+    n = 3
+    q = torch.randn(n * rows, Hq, 128, device=dev).bfloat16()
+    k, v = (torch.randn(n * rows, Hkv, 128, device=dev).bfloat16() for _ in range(2))
+    qr = torch.tensor([[i * rows, (i + 1) * rows] for i in range(n)], dtype=torch.int32, device=dev)
+    kr = torch.tensor([[0, (i + 1) * rows] for i in range(n)], dtype=torch.int32, device=dev)
+    all_rows, _ = M.range_attention(q, k, v, qr, kr, rows, n * rows, split_keys=False)
+    for i in range(n):
+        one, _ = M.range_attention(q[i * rows:(i + 1) * rows], k, v, qr[:1], kr[i:i + 1], rows, n * rows, split_keys=False)
+        assert torch.equal(one, all_rows[i * rows:(i + 1) * rows]), i
+    with pytest.raises(M.MagiError, match="ROW_BITS"):  # (nor with memory for shared keys)
+        a = L.AttnArgs(dtype=L.MAGI_DTYPE_BF16, D=128, Hq=1, Hkv=1, total_q=1, total_k=0, n_ranges=1, max_seqlen_q=1, flags=L.MAGI_ATTN_ROW_BITS,
+                       q=q.data_ptr(), out=q.data_ptr(), q_ranges=qr.data_ptr(), k_ranges=kr.data_ptr(), split_workspace=q.data_ptr(),
+                       split_workspace_bytes=16, **{"%s_stride_%s" % (x, y): 128 for x in "qkvo" for y in "th"})
+        L.check(L.lib().magi_attn_fwd(a, None))
