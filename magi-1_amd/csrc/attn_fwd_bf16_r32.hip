@@ -154,7 +154,8 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_bf16_r32_kernel(const AttnKer
   }
   float* part = nullptr;
   if constexpr (SHARE) {
-    const int first = ks + (int)(piece * a.share_tiles) * BN, end = first + (int)a.share_tiles * BN;
+    // (the last piece takes what is left: ranges may be longer than the max_seqlen_k that the pieces were planned with)
+    const int first = ks + (int)(piece * a.share_tiles) * BN, end = piece + 1 < a.share_pieces ? first + (int)a.share_tiles * BN : ke;
     if (first >= ke) return;
     if (piece != 0 || end < ke) part = a.partial + ((long)block * a.share_pieces + piece) * ONLINE_PARTIAL_FLOATS;
     ks = first;
@@ -444,7 +445,7 @@ __global__ __launch_bounds__(256) void attn_fwd_bf16_r32_merge_kernel(const Attn
   const int qb = (int)(share >> 1), half = (int)(share & 1);
   const WorkItem wi = locate_work(a, 128, tid, s_sel, block);
   if (!wi.valid || wi.ke <= wi.ks) return;
-  const int tiles = (wi.ke - wi.ks + BN - 1) / BN, pieces = (int)(((unsigned)tiles + a.share_tiles - 1) / a.share_tiles);
+  const int tiles = (wi.ke - wi.ks + BN - 1) / BN, pieces = (int)min(((unsigned)tiles + a.share_tiles - 1) / a.share_tiles, a.share_pieces);
   if (pieces < 2) return;
   const int q_row = wi.q0 + 32 * w + 16 * qb + n;
   if (wi.q0 + 32 * w >= wi.qe) return;  // (wavefronts without rows leave nothing)

@@ -109,3 +109,21 @@ def test_rows_have_the_bits_of_their_range_alone(dev, rows, Hq, Hkv):
                        q=q.data_ptr(), out=q.data_ptr(), q_ranges=qr.data_ptr(), k_ranges=kr.data_ptr(), split_workspace=q.data_ptr(),
                        split_workspace_bytes=16, **{"%s_stride_%s" % (x, y): 128 for x in "qkvo" for y in "th"})
         L.check(L.lib().magi_attn_fwd(a, None))
+
+
+@pytest.mark.parametrize("bounded", [False, True])
+@pytest.mark.parametrize("stated", [2000, 1920, 5000])
+def test_ranges_that_are_not_as_long_as_stated(dev, stated, bounded):
+    """max_seqlen_k plans the pieces and no more: the last one of a longer range takes the rest, a shorter one has fewer."""
+    rows, n, Hq, Hkv = 200, 4321, 6, 2
+    assert L.lib().magi_attn_pieces_bytes(Hq, Hkv, 2, rows, stated, int(bounded)) > 0
+    q, k, v = (t.to(dev) for t in O.synthetic_qkv(2 * rows, n, Hq, Hkv, 128, seed=stated))
+    qr = torch.tensor([[0, rows], [rows, 2 * rows]], dtype=torch.int32, device=dev)
+    kr = torch.tensor([[0, n], [17, 17 + n // 3]], dtype=torch.int32, device=dev)
+    kw = dict(score_bound=30.0) if bounded else {}
+    got, lse = M.range_attention(q, k, v, qr, kr, rows, stated, **kw)
+    want, want_lse = M.range_attention(q, k, v, qr, kr, rows, stated, split_keys=False, **kw)
+    size = M.range_attention(q, k, v.abs(), qr, kr, rows, stated, split_keys=False, **kw)[0].float()
+    # (bf16 probabilities and results on both sides, as in test_attn_online_split_gpu.py)
+    assert ((got.float() - want.float()).abs() <= 2.0 ** -6 * size + 1e-6).all()
+    assert (lse - want_lse).abs().max() < 1e-4
