@@ -1124,7 +1124,7 @@ class FullyParallelAttention(torch.nn.Module):
 
         With proj_layout=True the return value is ONE tensor [sq, b, 2*Hq*D] already in the "(hn n hd)" order
         that linear_proj consumes (what attn_linear_proj builds with concat + rearrange, dit_module.py:1332-1340):
-        at batch 1 both attention launches write straight into it."""
+        both attention launches write straight into it (of a batch where both are the library's own methods)."""
         if rotary_pos_emb is None:
             raise ValueError("FullyParallelAttention needs rotary_pos_emb")
         # the incoming table already is the [sin | cos] layout the prologue takes
