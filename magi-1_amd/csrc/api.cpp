@@ -292,9 +292,8 @@ struct R32Plan {
 // ranges of 312 over 1248 to 1872 31 / 22, four of 252 33 / 20; 24 heads, 432 over 1728 36 / 29, 720 over 2880 49 / 42, three of 612 over
 // 5508 to 6732 178 / 144; not so 1386 over 5544 109 / 114, 1080 over 5400 86 / 86, 720 over 720 21 / 25.  Error against float64 over that of whole items 0.9999 to 1.0001 (27 drawn sizes).
 // (From 16 tiles on: max_seqlen_k of text is the padded length, 800, of which a call may fill a fraction; 15 tiles would gain 4 to 6 us.)
-R32Plan r32_plan(int Hq, int Hkv, int n_ranges, int max_seqlen_q, int max_seqlen_k, int64_t& split_bytes) {
+R32Plan make_r32_plan(int Hq, int Hkv, int n_ranges, int max_seqlen_q, int max_seqlen_k, unsigned cus, int64_t& split_bytes) {
   R32Plan plan = {false, {1, 0}};
-  const unsigned cus = (unsigned)compute_units();
   auto items = [&](int rows) { return items_per_xcd(Hq, Hkv, n_ranges, max_seqlen_q / rows + (max_seqlen_q % rows != 0)); };
   const unsigned half = items(128), whole = items(256);
   unsigned lengths[16];
@@ -326,6 +325,31 @@ R32Plan r32_plan(int Hq, int Hkv, int n_ranges, int max_seqlen_q, int max_seqlen
   }
   if (!plan.use) plan.use = others(split_bytes);
   return plan;
+}
+
+// (Asked for twice or three times for a launch, for its memory and for itself, and again by the next layer; 1 to 2 us each, which layers that
+// wait for the host have not got.  A thread's last eight are kept by their sizes.)
+R32Plan r32_plan(int Hq, int Hkv, int n_ranges, int max_seqlen_q, int max_seqlen_k, int64_t& split_bytes) {
+  struct Kept {
+    int sizes[5];
+    unsigned cus;
+    int64_t given, left;
+    R32Plan plan;
+  };
+  static thread_local Kept kept[8];  // (cus 0: none)
+  static thread_local unsigned next = 0;
+  const unsigned cus = (unsigned)compute_units();
+  for (const Kept& e : kept)
+    if (e.cus == cus && e.given == split_bytes && e.sizes[0] == Hq && e.sizes[1] == Hkv && e.sizes[2] == n_ranges && e.sizes[3] == max_seqlen_q &&
+        e.sizes[4] == max_seqlen_k) {
+      split_bytes = e.left;
+      return e.plan;
+    }
+  Kept& e = kept[next++ % 8];
+  const int64_t given = split_bytes;
+  e.plan = make_r32_plan(Hq, Hkv, n_ranges, max_seqlen_q, max_seqlen_k, cus, split_bytes);
+  e = {{Hq, Hkv, n_ranges, max_seqlen_q, max_seqlen_k}, cus, given, split_bytes, e.plan};
+  return e.plan;
 }
 
 // the memory of its pieces, 0 where it takes whole items or none
