@@ -180,7 +180,8 @@ constexpr Pace PACE_X16_256 = {1.75, 2.75, 2.75, 2, 7.0};    // 256 rows
 // What a launch in pieces of `cut` tiles takes, in us: bringing pieces together takes 5 us and 18 ns each (their way through
 // memory).  Workgroups that fit the chip at once run side by side until the shortest are done, and so on; more of them keep it full but
 // for the end.
-double share_us(const Pace& p, unsigned items, const unsigned* lengths, int n_ranges, unsigned cut, unsigned cus) {
+// even: pieces of nearly the same length end together, so a CU that has one more than the others keeps it to the end.
+double share_us(const Pace& p, unsigned items, const unsigned* lengths, int n_ranges, unsigned cut, unsigned cus, bool even = false) {
   unsigned len[2 * 16], count[2 * 16];  // the pieces, by length
   int kinds = 0;
   auto add = [&](unsigned l, unsigned c) {
@@ -215,7 +216,7 @@ double share_us(const Pace& p, unsigned items, const unsigned* lengths, int n_ra
   } else {
     double left = all;
     for (int i = 0; i < kinds; left -= count[i++])
-      t += (len[i] - (i ? len[i - 1] : 0)) * tile_us(i + 1 < kinds ? left / cus : std::ceil(left / cus));
+      t += (len[i] - (i ? len[i - 1] : 0)) * tile_us(i + 1 < kinds && !(even && 8 * len[i] >= 7 * len[kinds - 1]) ? left / cus : std::ceil(left / cus));
   }
   return parts > 0 ? t + 5.0 + 0.018 * parts : t;
 }
@@ -232,14 +233,17 @@ bool range_tiles(int n_ranges, int max_seqlen_q, int max_seqlen_k, unsigned* len
   return true;
 }
 // the best of the launches in pieces that take less than `us`
-SharePlan best_pieces(const Pace& p, unsigned items, const unsigned* lengths, int n_ranges, double us) {
+SharePlan best_pieces(const Pace& p, unsigned items, const unsigned* lengths, int n_ranges, double us, bool one_round = false) {
   SharePlan best = {1, 0};
   const unsigned cus = (unsigned)compute_units(), longest = lengths[0];
   static const unsigned char tried[] = {2, 3, 4, 5, 6, 8, 10, 12, 16};
   for (unsigned pieces : tried) {
     const unsigned cut = (longest + pieces - 1) / pieces;
     if (cut < 3 || (double)items * pieces > 8.0 * cus) break;
-    const double t = share_us(p, items, lengths, n_ranges, cut, cus);
+    unsigned parts = 0;
+    for (int r = 0; r < n_ranges; ++r) parts += (lengths[r] + cut - 1) / cut;
+    if (one_round && (double)items / n_ranges * parts > (double)p.most * cus) continue;
+    const double t = share_us(p, items, lengths, n_ranges, cut, cus, one_round);
     if (t < us) {
       us = t;
       best = {(longest + cut - 1) / cut, cut};
@@ -288,9 +292,11 @@ struct R32Plan {
 // per CU, which tile_rows takes care of) holds them all.  Measured, 24 heads, 256 rows / 128: 2700 rows over 2700 keys 125 / 107 us, 3354
 // over 3354 152 / 136, 3744 over 3744 168 / 156, four ranges of 792 over 1584 to 3960 138 / 114, three of 1200 over 1200 to 3600 125 / 103;
 // but behind that round 2250 x 2 over 2250 and 4500 164 / 185, 2340 x 2 168 / 211.
-// Pieces: the estimates of both launches, and at least 8 % less.  Measured, before / in pieces: 6 heads, 270 rows over 1350 keys 30 / 17, three
+// Pieces: the estimates of both launches, and at least 5 % less, where all pieces run at a time; pieces of one length
+// take as long as the CU that has most of them (264 items in two each, three on 16 CUs: 1386 rows over 6930 and 13860 keys 121 / 140, 197 / 236).  Measured, before / in pieces: 6 heads, 270 rows over 1350 keys 30 / 17, three
 // ranges of 312 over 1248 to 1872 31 / 22, four of 252 33 / 20; 24 heads, 432 over 1728 36 / 29, 720 over 2880 49 / 42, three of 612 over
-// 5508 to 6732 178 / 144; not so 1386 over 5544 109 / 114, 1080 over 5400 86 / 86, 720 over 720 21 / 25.  Error against float64 over that of whole items 0.9999 to 1.0001 (27 drawn sizes).
+// 5508 to 6732 178 / 144; not so 1080 over 5400 86 / 86, 720 over 720 21 / 25, 660 over 5940 63 / 70, 48 heads 105 / 123,
+// two of 660 over 5280 and 5940 113 / 123, four over 1980 to 3960 112 / 116 (256 rows in pieces all: their time by the mean length of the ranges).  Error against float64 over that of whole items 0.9999 to 1.0001 (27 drawn sizes).
 // (From 16 tiles on: max_seqlen_k of text is the padded length, 800, of which a call may fill a fraction; 15 tiles would gain 4 to 6 us.)
 R32Plan make_r32_plan(int Hq, int Hkv, int n_ranges, int max_seqlen_q, int max_seqlen_k, unsigned cus, int64_t& split_bytes) {
   R32Plan plan = {false, {1, 0}};
@@ -310,13 +316,14 @@ R32Plan make_r32_plan(int Hq, int Hkv, int n_ranges, int max_seqlen_q, int max_s
   };
   if (split_bytes > 0 && lengths[0] >= 16) {
     const bool whole_items = others(INT64_MAX);
-    double us;
+    double us, tiles = 0;  // (tiles: of all ranges)
+    for (int r = 0; r < n_ranges; ++r) tiles += lengths[r];
     if (split.from < whole)  // (at most one round here: all items are in pieces)
-      us = 19.0 + lengths[0] * (double)split.num / split.den * (8 * whole * split.pieces <= cus ? 1.75 : 2.6) + 0.3 * whole * split.pieces;
+      us = 16.0 + tiles / n_ranges * (double)split.num / split.den * (8 * whole * split.pieces <= cus ? 1.75 : 2.6) + 0.18 * whole * split.pieces;
     else
       us = share_us(whole_items ? PACE_R32 : small ? PACE_X16_128 : PACE_X16_256, 8 * (whole_items || small ? half : whole), lengths, n_ranges,
                     lengths[0], cus);
-    plan.share = best_pieces(PACE_R32, 8 * half, lengths, n_ranges, 0.92 * us);
+    plan.share = best_pieces(PACE_R32, 8 * half, lengths, n_ranges, 0.95 * us, true);
     plan.use = plan.share.pieces > 1;
     if (plan.use && plan.share.bytes(half) > split_bytes) {  // (too little memory: whole items)
       plan = {false, {1, 0}};
