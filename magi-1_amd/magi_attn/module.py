@@ -904,12 +904,14 @@ class FullyParallelAttention(torch.nn.Module):
         return tail[:rows]
 
     def _norm_parameters(self):
-        """gamma_beta_fp32() of the four head norms, which forward() has had converted or checked by now (score_bounds)."""
+        """gamma_beta_fp32() of the four head norms.  Where they and score_bounds() are the library's own, forward() has just had the
+        parameters converted or checked (score_bounds asks each norm for its parameter_epoch)."""
         m = self._modules
         lns = (m["q_layernorm"], m["k_layernorm"], m["q_layernorm_xattn"], m["k_layernorm_xattn"])
-        if FusedLayerNorm.gamma_beta_fp32 is not _GAMMA_BETA:
+        if not _OWN_BOUNDS.of(self) or _NORM_FORMS(FusedLayerNorm) != _OWN_NORM_FORMS:
             return [ln.gamma_beta_fp32() for ln in lns]
-        return [d["_gb"] if type(ln) is FusedLayerNorm and "gamma_beta_fp32" not in (d := ln.__dict__) else ln.gamma_beta_fp32() for ln in lns]
+        return [d["_gb"] if type(ln) is FusedLayerNorm and "gamma_beta_fp32" not in (d := ln.__dict__) and "parameter_epoch" not in d
+                else ln.gamma_beta_fp32() for ln in lns]
 
     def _small_layer_weights(self, hidden_states: torch.Tensor, key_value_states: torch.Tensor, rope: torch.Tensor, own: "_Own"):
         """(w, wt, ln, lw, lb): the parameter that the weight of the four projections starts with, the text's weight, the input norm and its parameters, of a small layer
@@ -1290,5 +1292,7 @@ _CROSS_FUSED = FullyParallelAttention._cross_attention_fused
 _OWN_SMALL = _Own(FullyParallelAttention, "_project_rows", "_fused_qkv", "_cross_attention_fused")
 _OWN_SMALL_UNCACHED = _Own(FullyParallelAttention, "_project_rows", "_fused_qkv", "_cross_attention_fused", "core_attention")
 _OWN_SMALL_FP8 = _Own(FullyParallelAttention, "_project_rows", "_core_attention_fp8", "_cross_attention_fused")
-_GAMMA_BETA = FusedLayerNorm.gamma_beta_fp32
+_OWN_BOUNDS = _Own(FullyParallelAttention, "score_bounds")
+_NORM_FORMS = operator.attrgetter("gamma_beta_fp32", "parameter_epoch")
+_OWN_NORM_FORMS = _NORM_FORMS(FusedLayerNorm)
 _OWN_BATCH = _Own(FullyParallelAttention, "core_attention", "_cross_attention_fused")
