@@ -154,12 +154,14 @@ __global__ __launch_bounds__(256, 3) void attn_fwd_bf16_r32_kernel(const AttnKer
   }
   float* part = nullptr;
   if constexpr (SHARE) {
-    // (the last piece takes what is left: ranges may be longer than the max_seqlen_k that the pieces were planned with)
-    const int first = ks + (int)(piece * a.share_tiles) * BN, end = piece + 1 < a.share_pieces ? first + (int)a.share_tiles * BN : ke;
-    if (first >= ke) return;
-    if (piece != 0 || end < ke) part = a.partial + ((long)block * a.share_pieces + piece) * ONLINE_PARTIAL_FLOATS;
-    ks = first;
-    ke = min(ke, end);
+    // (the last piece takes what is left: ranges may be longer than the max_seqlen_k that the pieces were planned with; counted from
+    // the range's first key, unsigned: a stated max_seqlen_k of up to 2^31 - 1 puts pieces behind the last key that an int could name)
+    const unsigned keys = (unsigned)(ke - ks), per = a.share_tiles * BN, first = piece * per;
+    if (first >= keys) return;
+    const unsigned end = piece + 1 < a.share_pieces ? min(first + per, keys) : keys;
+    if (piece != 0 || end < keys) part = a.partial + ((long)block * a.share_pieces + piece) * ONLINE_PARTIAL_FLOATS;
+    ke = ks + (int)end;
+    ks += (int)first;
   }
 
   const long ks_t = a.ks_t, vs_t = a.vs_t;

@@ -127,3 +127,24 @@ def test_ranges_that_are_not_as_long_as_stated(dev, stated, bounded):
     # (bf16 probabilities and results on both sides, as in test_attn_online_split_gpu.py)
     assert ((got.float() - want.float()).abs() <= 2.0 ** -6 * size + 1e-6).all()
     assert (lse - want_lse).abs().max() < 1e-4
+
+
+@pytest.mark.parametrize("bounded", [False, True])
+@pytest.mark.parametrize("stated", [1500, 2 ** 31 - 1])
+def test_pieces_of_a_range_far_along_the_key_axis(dev, stated, bounded):
+    """Keys 2e9 .. 2e9 + 1500 of an axis whose first segment is never looked at: pieces are counted from the range's first key, those
+    behind its end, at positions beyond 2^31 with the largest stated length, leave nothing."""
+    rows, n, far, Hq, Hkv = 200, 1500, 2_000_000_000, 6, 2
+    size = L.lib().magi_attn_pieces_bytes(Hq, Hkv, 1, rows, stated, int(bounded))
+    assert size > 0
+    q, k, v = (t.to(dev) for t in O.synthetic_qkv(rows, n, Hq, Hkv, 128, seed=5))
+    kw = dict(score_bound=30.0) if bounded else {}
+    want, _ = M.range_attention(q, k, v, *(torch.tensor([[0, m]], dtype=torch.int32, device=dev) for m in (rows, n)), rows, stated, **kw)
+    out, scratch = torch.empty_like(q), torch.empty(size, dtype=torch.uint8, device=dev)
+    qr, kr = torch.tensor([[0, rows]], dtype=torch.int32, device=dev), torch.tensor([[far, far + n]], dtype=torch.int32, device=dev)
+    a = L.AttnArgs(dtype=L.MAGI_DTYPE_BF16, D=128, Hq=Hq, Hkv=Hkv, total_q=rows, total_k=far + n, n_ranges=1, max_seqlen_q=rows, max_seqlen_k=stated,
+                   q=q.data_ptr(), k=k.data_ptr(), v=v.data_ptr(), k2=k.data_ptr(), v2=v.data_ptr(), k_split=far, out=out.data_ptr(),
+                   q_ranges=qr.data_ptr(), k_ranges=kr.data_ptr(), split_workspace=scratch.data_ptr(), split_workspace_bytes=size, **kw,
+                   **{"%s_stride_t" % x: (Hkv if x in "kv" else Hq) * 128 for x in "qkvo"}, **{"%s_stride_h" % x: 128 for x in "qkvo"})
+    L.check(L.lib().magi_attn_fwd(a, torch.cuda.current_stream().cuda_stream))
+    assert torch.equal(out, want)
