@@ -92,7 +92,9 @@ extern "C" {
 
 /* 100 * major + minor.  The layout of the argument structs below belongs to the version; every struct also starts
  * with its own size as the caller compiled it (struct_size = sizeof(the struct)), and an entry point that is handed
- * another size returns MAGI_EINVAL instead of reading fields the caller never wrote. */
+ * another size returns MAGI_EINVAL instead of reading fields the caller never wrote.
+ * 105: the structs of 104; new are MAGI_ATTN_ROW_BITS (a library of 104 would ignore it), magi_attn_pieces_bytes,
+ * magi_small_projections_e4m3 and magi_small_layer. */
 int magi_version(void);
 const char* magi_last_error(void);
 /* Diagnostics: the number of kernel launches the library has issued in this process so far (all threads, all

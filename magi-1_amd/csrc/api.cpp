@@ -382,7 +382,7 @@ const magi_attn_args* current_layout(const magi_attn_args* p, magi_attn_args* fu
 
 extern "C" {
 
-int magi_version(void) { return 104; }
+int magi_version(void) { return 105; }
 
 uint64_t magi_launch_count(void) { return g_launches.load(std::memory_order_relaxed); }
 

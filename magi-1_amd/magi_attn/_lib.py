@@ -144,7 +144,7 @@ class SmallLayerArgs(_SizedStructure):
     ]
 
 
-ABI_VERSION = 104  # magi_version() of the library these mirrors were written for
+ABI_VERSION = 105  # magi_version() of the library these mirrors were written for
 
 EXPORTS = ("magi_version", "magi_last_error", "magi_launch_count", "magi_attn_fwd", "magi_attn_fwd_static_scratch",
            "magi_attn_split_bytes", "magi_attn_pieces_bytes", "magi_attn_tile_rows",
@@ -169,6 +169,9 @@ def lib() -> C.CDLL:
         if l.magi_version() != ABI_VERSION:
             raise RuntimeError(f"{LIB_PATH} reports version {l.magi_version()}, this package binds version {ABI_VERSION}: "
                                "rebuild the library (`make -C magi-1_amd/csrc`)")
+        missing = [name for name in EXPORTS if not hasattr(l, name)]
+        if missing:
+            raise RuntimeError(f"{LIB_PATH} has no {', '.join(missing)}: rebuild the library (`make -C magi-1_amd/csrc`)")
         l.magi_launch_count.restype = C.c_uint64
         l.magi_last_error.restype = C.c_char_p
         l.magi_attn_split_bytes.argtypes = [C.c_int32] * 6

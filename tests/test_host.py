@@ -593,3 +593,17 @@ def test_copying_form_of_the_cache_update_matches_the_reference_semantics():
             assert torch.equal(ip.key_value_memory_dict[2][:written], model.mem[:written])
         k, v = layer.adjust_key_and_value_for_inference(kv, None, meta)
         assert torch.equal(k, kv[..., :D]) and torch.equal(v, kv[..., D:])
+
+
+@pytest.mark.parametrize("version,exports", [(104, ()), (L.ABI_VERSION, ("magi_attn_fwd",))])
+def test_a_library_of_another_version_or_without_an_entry_point_is_refused(tmp_path, monkeypatch, version, exports):
+    """Version 104 had neither MAGI_ATTN_ROW_BITS, which it would ignore, nor the entry points that came with it."""
+    import subprocess
+
+    src, so = tmp_path / "old.c", tmp_path / "old.so"
+    src.write_text("int magi_version(void) { return %d; }\n" % version + "".join("int %s(void) { return 0; }\n" % n for n in exports))
+    subprocess.run(["gcc", "-shared", "-fPIC", str(src), "-o", str(so)], check=True)
+    monkeypatch.setattr(L, "_lib", None)
+    monkeypatch.setattr(L, "LIB_PATH", str(so))
+    with pytest.raises(RuntimeError, match="rebuild the library"):
+        L.lib()
