@@ -1210,15 +1210,15 @@ class FullyParallelAttention(torch.nn.Module):
         core_dst = cross_dst = None
         if proj_layout and bs == 1 and Hq % PROJ_GROUPS == 0:
             # (rows that no q range / cu_seqlens segment covers are left as allocated: the pipeline's ranges cover
-            # every row, dit_model.py:220-222, 246)
-            fused = torch.empty(sq, 1, 2 * Hq * D, dtype=hidden_states.dtype, device=hidden_states.device)
+            # every row, dit_model.py:220-222, 246; bf16, what the launches write, whatever hidden_states is)
+            fused = torch.empty(sq, 1, 2 * Hq * D, dtype=torch.bfloat16, device=hidden_states.device)
             grouped = fused.view(sq, PROJ_GROUPS, 2, Hq // PROJ_GROUPS, D)
             core_dst, cross_dst = grouped[:, :, 0], grouped[:, :, 1]
         elif (proj_layout and bs > 1 and Hq % PROJ_GROUPS == 0 and own_cross and _OWN_BATCH.of(self) and self.attention_dtype == "bf16"
               and hidden_states.is_cuda):
             # (batch rows are further groups of heads to the core attention: position, batch, group, core | cross, head.  Without the copy that
             # put the two together: two rows of 13824 tokens, 24 heads, 4.59 -> 4.33 ms; three of 3420, 48 heads, 2.52 -> 2.30)
-            fused = torch.empty(sq, bs, 2 * Hq * D, dtype=hidden_states.dtype, device=hidden_states.device)
+            fused = torch.empty(sq, bs, 2 * Hq * D, dtype=torch.bfloat16, device=hidden_states.device)
             grouped = fused.view(sq, bs, PROJ_GROUPS, 2, Hq // PROJ_GROUPS, D)
             core_dst, cross_dst = grouped.view(sq, bs * PROJ_GROUPS, 2, Hq // PROJ_GROUPS, D)[:, :, 0], grouped[:, :, :, 1]
 
