@@ -85,6 +85,9 @@ unsigned items_per_xcd(int Hq, int Hkv, int n_ranges, int tiles_per_range) {
   return (unsigned)((Hkv / 8) * per_head + (left * per_head + 7) / 8);
 }
 
+// tiles of 64 keys; unsigned, since the stated max_seqlen_k may be anything up to 2^31 - 1
+unsigned key_tiles(int keys) { return ((unsigned)keys + 63) / 64; }
+
 // Which items of a 256-row launch without a running maximum have their keys shared by several workgroups (AttnKernArgs::split_*).
 struct SplitPlan {
   unsigned from, pieces, num, den;
@@ -125,7 +128,7 @@ SplitPlan split_plan(unsigned items, int n_ranges, int max_seqlen_q, int max_seq
   SplitPlan s = {UINT32_MAX, 1, 1, 1, fp8};
   const unsigned cus = (unsigned)compute_units() / 8, slots = cus * (fp8 ? 3 : 2);  // of one XCD
   if (slots == 0 || max_seqlen_k <= 0) return s;
-  const unsigned rounds = items / slots, left = items % slots, tiles = (unsigned)(max_seqlen_k + 63) / 64;
+  const unsigned rounds = items / slots, left = items % slots, tiles = key_tiles(max_seqlen_k);
   if (left == 0 || rounds >= 8 || (fp8 && rounds == 0)) return s;
   if (n_ranges > 1 && max_seqlen_k > max_seqlen_q) {
     const int64_t shortest = max_seqlen_k - (int64_t)(n_ranges - 1) * max_seqlen_q;
@@ -229,7 +232,7 @@ double share_us(const Pace& p, unsigned items, const unsigned* lengths, int n_ra
 bool range_tiles(int n_ranges, int max_seqlen_q, int max_seqlen_k, unsigned* lengths) {
   if (max_seqlen_k <= 0 || n_ranges < 1 || n_ranges > 16) return false;
   const bool apart = max_seqlen_k > (int64_t)(n_ranges - 1) * max_seqlen_q;
-  for (int r = 0; r < n_ranges; ++r) lengths[r] = (unsigned)(max_seqlen_k - (apart ? r * max_seqlen_q : 0) + 63) / 64;
+  for (int r = 0; r < n_ranges; ++r) lengths[r] = key_tiles(max_seqlen_k - (apart ? r * max_seqlen_q : 0));
   return true;
 }
 // the best of the launches in pieces that take less than `us`
@@ -278,7 +281,7 @@ int tile_rows(int Hq, int Hkv, int n_ranges, int max_seqlen_q, int max_seqlen_k,
   if (s.from >= whole || s.bytes(whole) > split_bytes) return 128;
   // (without a whole round ahead of them: all items are in pieces)
   const unsigned pieces = whole * s.pieces;
-  const double tiles = (max_seqlen_k + 63) / 64, in_pieces = tiles * s.num / s.den * (pieces <= cus ? 1.75 : 2.6) + 12.0 + 0.3 * pieces;
+  const double tiles = key_tiles(max_seqlen_k), in_pieces = tiles * s.num / s.den * (pieces <= cus ? 1.75 : 2.6) + 12.0 + 0.3 * pieces;
   return in_pieces <= tiles * (half <= cus ? 1.15 : 1.75) ? 256 : 128;
 }
 

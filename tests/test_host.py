@@ -607,3 +607,14 @@ def test_a_library_of_another_version_or_without_an_entry_point_is_refused(tmp_p
     monkeypatch.setattr(L, "LIB_PATH", str(so))
     with pytest.raises(RuntimeError, match="rebuild the library"):
         L.lib()
+
+
+@pytest.mark.parametrize("size", [(6, 2, 1, 200), (24, 8, 1, 1300), (24, 8, 4, 288)])
+def test_plans_of_the_longest_stated_key_ranges(size):
+    """A max_seqlen_k as large as the type: the plan is that of one that differs by less than a tile of 64 keys in 2^25."""
+    lib, longest, near = L.lib(), 2 ** 31 - 1, 2 ** 31 - 128
+    memory = lib.magi_attn_split_bytes(*size, near, L.MAGI_DTYPE_BF16)
+    assert memory > 0 and memory == lib.magi_attn_split_bytes(*size, longest, L.MAGI_DTYPE_BF16)
+    assert lib.magi_attn_tile_rows(*size, near, memory) == lib.magi_attn_tile_rows(*size, longest, memory)
+    for bounded in (0, 1):
+        assert lib.magi_attn_pieces_bytes(*size, near, bounded) == lib.magi_attn_pieces_bytes(*size, longest, bounded)
