@@ -93,8 +93,8 @@ extern "C" {
 /* 100 * major + minor.  The layout of the argument structs below belongs to the version; every struct also starts
  * with its own size as the caller compiled it (struct_size = sizeof(the struct)), and an entry point that is handed
  * another size returns MAGI_EINVAL instead of reading fields the caller never wrote.
- * 105: the structs of 104; new are MAGI_ATTN_ROW_BITS (a library of 104 would ignore it), magi_attn_pieces_bytes,
- * magi_small_projections_e4m3 and magi_small_layer. */
+ * 105: the structs of 104; new are MAGI_ATTN_ROW_BITS (a library of 104 would ignore it), magi_attn_split_bytes_256,
+ * magi_attn_pieces_bytes, magi_small_projections_e4m3 and magi_small_layer. */
 int magi_version(void);
 const char* magi_last_error(void);
 /* Diagnostics: the number of kernel launches the library has issued in this process so far (all threads, all
@@ -237,9 +237,13 @@ typedef struct magi_attn_args {
   int64_t split_workspace_bytes;
 } magi_attn_args;
 
-/* Bytes of split_workspace that a call of these sizes makes use of (dtype: MAGI_DTYPE_*; bf16: with a score bound, or checked); 0: such
+/* Bytes of split_workspace that a call of these sizes makes use of (dtype: MAGI_DTYPE_*; bf16: with a score bound); 0: such
  * a call is not split. */
 int64_t magi_attn_split_bytes(int32_t Hq, int32_t Hkv, int32_t n_ranges, int32_t max_seqlen_q, int32_t max_seqlen_k, int32_t dtype);
+
+/* The same for a bf16 call in 256-row workgroups whatever its sizes: MAGI_ATTN_CHECKED, or q_tile_rows 256 with a score bound.  At most the
+ * above, which also has to hold the pieces of magi_attn_pieces_bytes; MAGI_ATTN_BOUNDED_MFMA32 and q_tile_rows 512 make use of none. */
+int64_t magi_attn_split_bytes_256(int32_t Hq, int32_t Hkv, int32_t n_ranges, int32_t max_seqlen_q, int32_t max_seqlen_k);
 
 /* Where a bf16 call of these sizes has the keys of all its rows shared, in 128-row workgroups: the bytes for that, else 0.  bounded !=
  * 0: with a score_bound in force, no MAGI_ATTN_CHECKED, q_tile_rows 0.  0: with the online softmax (no MAGI_ATTN_AUTO_BOUND,

@@ -400,7 +400,15 @@ int64_t magi_attn_split_bytes(int32_t Hq, int32_t Hkv, int32_t n_ranges, int32_t
   const unsigned items = items_per_xcd(Hq, Hkv, n_ranges, tiles);
   const int64_t split = split_plan(items, n_ranges, max_seqlen_q, max_seqlen_k, fp8).bytes(items);
   const int64_t pieces = fp8 ? 0 : r32_bytes(Hq, Hkv, n_ranges, max_seqlen_q, max_seqlen_k);
-  return split > pieces ? split : pieces;  // (checked launches, 256-row always, take the former)
+  return split > pieces ? split : pieces;
+}
+
+int64_t magi_attn_split_bytes_256(int32_t Hq, int32_t Hkv, int32_t n_ranges, int32_t max_seqlen_q, int32_t max_seqlen_k) {
+  if (Hq <= 0 || Hkv <= 0 || Hq % Hkv || n_ranges <= 0 || max_seqlen_q <= 0) return 0;
+  const int tiles = max_seqlen_q / 256 + (max_seqlen_q % 256 != 0);
+  if ((double)Hq * n_ranges * tiles > 2.0e9) return 0;
+  const unsigned items = items_per_xcd(Hq, Hkv, n_ranges, tiles);
+  return split_plan(items, n_ranges, max_seqlen_q, max_seqlen_k, false).bytes(items);
 }
 
 int64_t magi_attn_pieces_bytes(int32_t Hq, int32_t Hkv, int32_t n_ranges, int32_t max_seqlen_q, int32_t max_seqlen_k, int32_t bounded) {

@@ -147,7 +147,7 @@ class SmallLayerArgs(_SizedStructure):
 ABI_VERSION = 105  # magi_version() of the library these mirrors were written for
 
 EXPORTS = ("magi_version", "magi_last_error", "magi_launch_count", "magi_attn_fwd", "magi_attn_fwd_static_scratch",
-           "magi_attn_split_bytes", "magi_attn_pieces_bytes", "magi_attn_tile_rows",
+           "magi_attn_split_bytes", "magi_attn_split_bytes_256", "magi_attn_pieces_bytes", "magi_attn_tile_rows",
            "magi_qk_prologue", "magi_head_norm",
            "magi_apply_rotary", "magi_quantize_fp8", "magi_quantize_fp8_split", "magi_layer_norm", "magi_qkv_proj_prologue", "magi_div_clamp_to_e4m3",
            "magi_layer_norm_e4m3", "magi_small_projections", "magi_small_projections_e4m3",
@@ -176,6 +176,8 @@ def lib() -> C.CDLL:
         l.magi_last_error.restype = C.c_char_p
         l.magi_attn_split_bytes.argtypes = [C.c_int32] * 6
         l.magi_attn_split_bytes.restype = C.c_int64
+        l.magi_attn_split_bytes_256.argtypes = [C.c_int32] * 5
+        l.magi_attn_split_bytes_256.restype = C.c_int64
         l.magi_attn_pieces_bytes.argtypes = [C.c_int32] * 6
         l.magi_attn_pieces_bytes.restype = C.c_int64
         l.magi_attn_tile_rows.argtypes = [C.c_int32] * 5 + [C.c_int64]

@@ -268,10 +268,12 @@ def range_attention(
     split, split_bytes = None, 0
     if split_keys and not static_scratch and max_seqlen_k >= 512 and (
             checked or auto_bound or 0.0 < score_bound <= L.MAGI_SCORE_BOUND_MAX or q.dtype is torch.float8_e4m3fn):
-        if q.dtype is torch.bfloat16 and not (checked or q_tile_rows or bounded_mfma32):
-            split_bytes = _bounded_split_bytes(Hq, Hkv, n, int(max_seqlen_q), int(max_seqlen_k))
-        else:
+        if q.dtype is not torch.bfloat16:
             split_bytes = L.lib().magi_attn_split_bytes(Hq, Hkv, max(n, 0), int(max_seqlen_q), int(max_seqlen_k), _dtype_code(q))
+        elif checked or q_tile_rows == 256:
+            split_bytes = 0 if bounded_mfma32 else L.lib().magi_attn_split_bytes_256(Hq, Hkv, max(n, 0), int(max_seqlen_q), int(max_seqlen_k))
+        elif not (q_tile_rows or bounded_mfma32):  # (those make no use of any)
+            split_bytes = _bounded_split_bytes(Hq, Hkv, n, int(max_seqlen_q), int(max_seqlen_k))
     elif (split_keys and not static_scratch and max_seqlen_k >= 512 and q.dtype is torch.bfloat16 and not (auto_bound or q_prescaled)
           and q_tile_rows in (0, 128)):
         split_bytes = L.lib().magi_attn_pieces_bytes(Hq, Hkv, max(n, 0), int(max_seqlen_q), int(max_seqlen_k), 0)

@@ -148,3 +148,29 @@ def test_pieces_of_a_range_far_along_the_key_axis(dev, stated, bounded):
                    **{"%s_stride_t" % x: (Hkv if x in "kv" else Hq) * 128 for x in "qkvo"}, **{"%s_stride_h" % x: 128 for x in "qkvo"})
     L.check(L.lib().magi_attn_fwd(a, torch.cuda.current_stream().cuda_stream))
     assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize("size", [(24, 8, 1, 432, 1728), (6, 2, 1, 270, 1350), (6, 2, 1, 270, 1601)])
+def test_forms_without_pieces_take_no_memory_for_them(dev, monkeypatch, size):
+    """Workgroups of 256 rows whatever the sizes take what their last round's items need, the 32x32x16 form and 512 rows nothing."""
+    if torch.cuda.get_device_properties(dev).multi_processor_count != 256:
+        pytest.skip("the sizes are chosen for 256 CUs")
+    Hq, Hkv, n, rows, mk = size
+    lib = L.lib()
+    split, pieces = lib.magi_attn_split_bytes_256(*size), lib.magi_attn_pieces_bytes(*size, 1)
+    assert max(split, pieces) == lib.magi_attn_split_bytes(*size, L.MAGI_DTYPE_BF16) and split < pieces
+    q, k, v, qr, kr, kw = _case(dev, rows, n, Hq, Hkv, [(0, mk)] * n, "as it is")
+    real, got = torch.empty, []
+
+    def empty(*a, **o):
+        if o.get("dtype") is torch.uint8:
+            got.append(a[0])
+        return real(*a, **o)
+
+    monkeypatch.setattr(torch, "empty", empty)
+    for form, want in (({}, [pieces]), ({"q_tile_rows": 256}, [split] * (split > 0)), ({"q_tile_rows": 512}, []), ({"bounded_mfma32": True}, [])):
+        M.range_attention(q, k, v, qr, kr, rows, mk, **kw, **form)
+        assert got == want, form
+        got.clear()
+    M.range_attention(q, k, v, qr, kr, rows, mk, checked=True)
+    assert got == [split] * (split > 0)

@@ -618,3 +618,9 @@ def test_plans_of_the_longest_stated_key_ranges(size):
     assert lib.magi_attn_tile_rows(*size, near, memory) == lib.magi_attn_tile_rows(*size, longest, memory)
     for bounded in (0, 1):
         assert lib.magi_attn_pieces_bytes(*size, near, bounded) == lib.magi_attn_pieces_bytes(*size, longest, bounded)
+
+
+def test_memory_of_256_row_workgroups_is_part_of_what_a_bounded_call_asks_for():
+    for size in ((24, 8, 1, 432, 1728), (6, 2, 1, 270, 1350), (24, 8, 1, 720, 2880), (24, 8, 4, 288, 2016), (0, 1, 1, 1, 1), (3, 2, 1, 1, 1), (6, 2, 0, 1, 1)):
+        whole, pieces = L.lib().magi_attn_split_bytes(*size, L.MAGI_DTYPE_BF16), L.lib().magi_attn_pieces_bytes(*size, 1)
+        assert max(L.lib().magi_attn_split_bytes_256(*size), pieces) == whole
