@@ -184,9 +184,9 @@ def range_attention(
     bounded, and a second launch repeats the blocks of rows where they were not, MAGI_ATTN_CHECKED.  Faster than the online
     softmax where the workgroups fill the chip, and its results are further from the exact ones (see _unbounded_mode).
     split_keys: False keeps the library from sharing the keys of a row among workgroups where that fills the chip better
-    (magi_attn_args.split_workspace, up to 135 MB of scratch memory for the call; the fp32 sums are then added in another
-    order).  Whether it does follows from the sizes of the launch alone.  Needs max_seqlen_k.  Without it a bf16 row's bits depend on its
-    own range alone (MAGI_ATTN_ROW_BITS).
+    (magi_attn_args.split_workspace, up to 137 MB of scratch memory for the call; the fp32 sums are then added in another
+    order).  Whether it does follows from the sizes of the launch alone, except that the online softmax runs without where there is no such
+    memory to be had (the others raise).  Needs max_seqlen_k.  Without it a bf16 row's bits depend on its own range alone (MAGI_ATTN_ROW_BITS).
     q may be [batch, rows, Hq, D] with any batch stride (batch of activations laid out [position, batch, ...]): its rows
     count as batch * rows tokens for the ranges, out is (or comes back as) a tensor of q's shape, by default
     [rows, batch, Hq, D] transposed.  Needs a score_bound (math.inf: the online softmax).
@@ -265,7 +265,7 @@ def range_attention(
         workspace = torch.empty(max(4 * Hq * max(n, 0) * ((int(max_seqlen_q) + 255) // 256), 4), dtype=torch.int32, device=q.device)
     if auto_bound and not static_scratch:
         workspace = torch.empty(4, dtype=torch.float32, device=q.device)  # (alive until the launches are enqueued)
-    split, split_bytes = None, 0
+    split, split_bytes, online = None, 0, False
     if split_keys and not static_scratch and max_seqlen_k >= 512 and (
             checked or auto_bound or 0.0 < score_bound <= L.MAGI_SCORE_BOUND_MAX or q.dtype is torch.float8_e4m3fn):
         if q.dtype is not torch.bfloat16:
@@ -276,9 +276,14 @@ def range_attention(
             split_bytes = _bounded_split_bytes(Hq, Hkv, n, int(max_seqlen_q), int(max_seqlen_k))
     elif (split_keys and not static_scratch and max_seqlen_k >= 512 and q.dtype is torch.bfloat16 and not (auto_bound or q_prescaled)
           and q_tile_rows in (0, 128)):
-        split_bytes = L.lib().magi_attn_pieces_bytes(Hq, Hkv, max(n, 0), int(max_seqlen_q), int(max_seqlen_k), 0)
-    if split_bytes:  # (no going on without it where memory is short: the same call would give other bits then)
-        split = torch.empty(split_bytes, dtype=torch.uint8, device=q.device)
+        split_bytes, online = L.lib().magi_attn_pieces_bytes(Hq, Hkv, max(n, 0), int(max_seqlen_q), int(max_seqlen_k), 0), True
+    if split_bytes:
+        try:
+            split = torch.empty(split_bytes, dtype=torch.uint8, device=q.device)
+        except torch.OutOfMemoryError:
+            if not online:  # (no going on without it: the same call would give other bits then)
+                raise
+            split_bytes = 0  # (a reference-shaped call, which promises nothing about its scores, needs no memory but its output's)
     gamma = beta = None  # (alive until the launch is enqueued)
     norm_eps, norm_kind = 0.0, 0
     if q_norm is not None:

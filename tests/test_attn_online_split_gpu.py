@@ -116,3 +116,26 @@ def test_more_whole_items_than_run_at_a_time(dev):
         want = s.logsumexp(1) if c else torch.full((rows,), float("-inf"))
         assert torch.allclose(lse[9, i * rows:(i + 1) * rows].cpu(), want, atol=2e-5)
     assert torch.isinf(lse[:, n * rows:]).all()
+
+
+@pytest.mark.parametrize("call", ["flex", "varlen"])
+def test_without_memory_for_the_pieces_the_items_stay_whole(dev, monkeypatch, call):
+    """The rebound callables need no memory but their output's: where there is none to share the keys with, they run as they do without."""
+    rows, Hq, Hkv, Tk = 300, 6, 2, 4000
+    q, k, v = (t.to(dev) for t in O.synthetic_qkv(rows, Tk, Hq, Hkv, 128, seed=3))
+    qr, kr = _ranges([[0, rows]], dev), _ranges([[0, Tk]], dev)
+    want = M.range_attention(q, k, v, qr, kr, rows, Tk, split_keys=False)[0]
+    real, refused = torch.empty, []
+
+    def empty(*size, dtype=None, **kw):
+        if dtype is torch.uint8:
+            refused.append(size)
+            raise torch.OutOfMemoryError("no scratch memory")
+        return real(*size, dtype=dtype, **kw)
+
+    monkeypatch.setattr(torch, "empty", empty)
+    if call == "flex":
+        got = M.flex_flash_attn_func(q, k, v, qr, kr, rows, Tk)[0]
+    else:
+        got = M.flash_attn_varlen_func(q, k, v, qr[0], kr[0], rows, Tk)
+    assert torch.equal(got, want) and (refused or torch.cuda.get_device_properties(dev).multi_processor_count != 256)
