@@ -79,7 +79,9 @@ extern "C" {
 #define MAGI_ATTN_CHECKED 64
 
 /* bf16: a row's bits depend on its own range alone, not on how many rows the launch has besides.  The online softmax then keeps to one order of
- * the keys (that of small launches) in all sizes; with a score_bound they do not anyhow.  Without split_workspace. */
+ * the keys (that of small launches) in all sizes; with a score_bound they do not anyhow.  Without split_workspace.  With
+ * MAGI_ATTN_AUTO_BOUND this holds of each of the two kernels; which of them runs, for all rows of the launch, follows from the longest
+ * rows of q and of k in it, those of other ranges included: for a row's bits whatever the launch, state a score_bound or none. */
 #define MAGI_ATTN_ROW_BITS 128
 
 #define MAGI_RANGES_PAIRS 0 /* int32 [n, 2]: range i = [r[2i], r[2i+1])          */

@@ -186,7 +186,8 @@ def range_attention(
     split_keys: False keeps the library from sharing the keys of a row among workgroups where that fills the chip better
     (magi_attn_args.split_workspace, up to 137 MB of scratch memory for the call; the fp32 sums are then added in another
     order).  Whether it does follows from the sizes of the launch alone, except that the online softmax runs without where there is no such
-    memory to be had (the others raise).  Needs max_seqlen_k.  Without it a bf16 row's bits depend on its own range alone (MAGI_ATTN_ROW_BITS).
+    memory to be had (the others raise).  Needs max_seqlen_k.  Without it a bf16 row's bits depend on its own range alone (MAGI_ATTN_ROW_BITS); with
+    auto_bound also on which of the two kernels the longest rows of the whole call select.
     q may be [batch, rows, Hq, D] with any batch stride (batch of activations laid out [position, batch, ...]): its rows
     count as batch * rows tokens for the ranges, out is (or comes back as) a tensor of q's shape, by default
     [rows, batch, Hq, D] transposed.  Needs a score_bound (math.inf: the online softmax).

@@ -780,7 +780,7 @@ class FullyParallelAttention(torch.nn.Module):
         destination view, possibly in the grouped layout of range_attention (bs > 1: [sq, bs * groups, heads, D]).  q_prescaled: query carries
         softmax_scale * log2(e); score_bound, auto_bound: see range_attention.  split_keys: whether the keys of a row may
         be shared among workgroups, the sums added in an order that depends on what else the launch holds; without it a
-        row's bits are those of full_attention on its range alone."""
+        row's bits are those of full_attention on its range alone (with auto_bound, where the measured bound does not hold)."""
         p = meta_args.core_attn_params
         if bs == 1:
             out, _ = range_attention(query, key, value, p.q_range, p.k_range, p.max_seqlen_q, p.max_seqlen_k,

@@ -149,3 +149,17 @@ def test_auto_bound_argument_checks(dev):
     a.n_ranges, a.max_seqlen_q, a.Hq, a.Hkv, a.D = 1, 8, 2, 2, 128
     a.flags = L.MAGI_ATTN_AUTO_BOUND
     assert L.lib().magi_attn_fwd(a, None) == -22 and b"workspace" in L.lib().magi_last_error()
+
+
+def test_one_kernel_for_all_rows_whatever_their_ranges(dev):
+    """Without shared keys a row has the bits of its range alone in the kernel that runs; one long row of another range decides which."""
+    rows, Hq, Hkv = 300, 4, 2
+    g = torch.Generator(device=dev).manual_seed(3)
+    q, k, v = (torch.randn(2 * rows, h, 128, device=dev, generator=g).bfloat16() for h in (Hq, Hkv, Hkv))
+    qr = torch.tensor([[0, rows], [rows, 2 * rows]], dtype=torch.int32, device=dev)
+    call = lambda x, r, **kw: M.range_attention(x, k, v, r, r, rows, rows, split_keys=False, return_lse=False, **kw)[0][:rows]  # noqa: E731
+    online, bounded = call(q, qr[:1]), call(q, qr[:1], score_bound=60.0)
+    assert not torch.equal(online, bounded)
+    assert torch.equal(call(q, qr, auto_bound=True), bounded)
+    q[rows + 7] *= 100
+    assert torch.equal(call(q, qr, auto_bound=True), online) and torch.equal(call(q, qr), online)
