@@ -98,30 +98,6 @@ def _bounded_split_bytes(Hq: int, Hkv: int, n: int, max_seqlen_q: int, max_seqle
     return size
 
 
-def launch_bounded_attention(dev: torch.device, q: int, q_row: int, rows: int, Hq: int, kv: int, side: int, k_split: int, total_k: int,
-                             kv_row: int, Hkv: int, q_ranges: torch.Tensor, k_ranges: torch.Tensor, n: int, mode: int, max_seqlen_q: int,
-                             max_seqlen_k: int, out: int, o_row: int, group_heads: int, o_group: int, clear: bool, bound: float,
-                             q_norm: Optional[tuple] = None) -> None:
-    """range_attention for a caller that has made its tensors itself and knows them to be sound: bf16 rows by address (strides in
-    elements, heads 128 apart), K | V interleaved per head at kv, those from k_split on at `side` (0: none), scores bounded (0 <
-    bound <= MAGI_SCORE_BOUND_MAX).  q carries the softmax scale, or is raw with q_norm = (gamma, beta, eps) by address.  clear: rows no
-    range covers become zeros (the caller has cleared `out` unless covered_by_launch).  Shares keys as range_attention does."""
-    max_seqlen_q, max_seqlen_k = int(max_seqlen_q), int(max_seqlen_k)
-    split, split_bytes = None, 0
-    if max_seqlen_k >= 512:
-        split_bytes = _bounded_split_bytes(Hq, Hkv, n, max_seqlen_q, max_seqlen_k)
-        if split_bytes:
-            split = torch.empty(split_bytes, dtype=torch.uint8, device=dev)
-    q_ranges, k_ranges = q_ranges.contiguous(), k_ranges.contiguous()
-    gamma, beta, eps = (0, 0, 0.0) if q_norm is None else q_norm
-    flags = (L.MAGI_ATTN_Q_PRESCALED if q_norm is None else 0) | (L.MAGI_ATTN_ZERO_UNCOVERED if clear and covered_by_launch(n, max_seqlen_q, rows) else 0)
-    _launch_packed(
-        dev, "magi_attn_fwd", L.AttnArgs, q, kv, kv + 256, side, side + 256 if side else 0, out, 0, q_ranges.data_ptr(), k_ranges.data_ptr(), 0, 0, 0,
-        q_row, 128, kv_row, 256, kv_row, 256, o_row, 128, rows, total_k, k_split, max(n, 0), mode, max_seqlen_q, max_seqlen_k, Hq, Hkv, 128,
-        L.MAGI_DTYPE_BF16, 0, 0.0, flags, group_heads, o_group, bound, 0, gamma, beta, eps, L.MAGI_NORM_LAYERNORM_1P, 0, 0, 0, 0, 0, 0,
-        0 if split is None else split.data_ptr(), split_bytes)
-
-
 def range_attention(
     q: torch.Tensor,
     k: torch.Tensor,
@@ -598,12 +574,30 @@ def launch_quantize_fp8_split(dev: torch.device, *fields) -> None:
     _launch_packed(dev, "magi_quantize_fp8_split", L.QuantizeArgs, *fields)
 
 
+def launch_text_attention(dev: torch.device, q: int, rows: int, Hq: int, kv: int, total_k: int, Hkv: int, cu_q: torch.Tensor, cu_k: torch.Tensor,
+                          n: int, max_seqlen_q: int, max_seqlen_k: int, out: int, o_row: int, group_heads: int, o_group: int, clear: bool,
+                          bound: float, gamma: int, beta: int, eps: float) -> None:
+    """range_attention for a caller that has made its tensors itself and knows them to be sound: raw bf16 q rows by address, normalised
+    with gamma, beta and eps (rows and heads contiguous, as K | V interleaved per head at kv), cumulative lengths, scores bounded (0 <
+    bound <= MAGI_SCORE_BOUND_MAX).  clear: rows no range covers become zeros (the caller has cleared `out` unless covered_by_launch).
+    Shares keys as range_attention does."""
+    max_seqlen_q, max_seqlen_k = int(max_seqlen_q), int(max_seqlen_k)
+    split, split_at, split_bytes = split_memory(dev, Hq, Hkv, n, max_seqlen_q, max_seqlen_k)
+    cu_q, cu_k = cu_q.contiguous(), cu_k.contiguous()
+    flags = L.MAGI_ATTN_ZERO_UNCOVERED if clear and covered_by_launch(n, max_seqlen_q, rows) else 0
+    kv_row = Hkv * 256
+    _launch_packed(
+        dev, "magi_attn_fwd", L.AttnArgs, q, kv, kv + 256, 0, 0, out, 0, cu_q.data_ptr(), cu_k.data_ptr(), 0, 0, 0,
+        Hq * 128, 128, kv_row, 256, kv_row, 256, o_row, 128, rows, total_k, total_k, max(n, 0), L.MAGI_RANGES_CU, max_seqlen_q, max_seqlen_k, Hq, Hkv,
+        128, L.MAGI_DTYPE_BF16, 0, 0.0, flags, group_heads, o_group, bound, 0, gamma, beta, eps, L.MAGI_NORM_LAYERNORM_1P, 0, 0, 0, 0, 0, 0,
+        split_at, split_bytes)
+
+
 def launch_fp8_attention(dev: torch.device, q: int, rows: int, Hq: int, k: int, v: int, k_side: int, v_side: int, k_split: int, total_k: int,
                          Hkv: int, scales: tuple, chunk_tokens: int, q_ranges: torch.Tensor, k_ranges: torch.Tensor, n: int, max_seqlen_q: int,
                          max_seqlen_k: int, out: int, o_row: int, group_heads: int, o_group: int, clear: bool, fast_exp2: bool) -> None:
-    """launch_bounded_attention for e4m3 rows with power-of-two scales, heads and rows contiguous: K and V rows at k / v, those from
-    k_split on at k_side / v_side (0: none); scales: the tables of q, k, v, and of k and v there (0: none) by address.  Shares keys as
-    range_attention does."""
+    """The same for the core attention of e4m3 rows with power-of-two scales, heads and rows contiguous, ranges in pairs: K and V rows at
+    k / v, those from k_split on at k_side / v_side (0: none); scales: the tables of q, k, v, and of k and v there (0: none) by address."""
     max_seqlen_q, max_seqlen_k = int(max_seqlen_q), int(max_seqlen_k)
     split, split_bytes = None, 0
     if max_seqlen_k >= 512:

@@ -35,9 +35,9 @@ import torch
 
 from . import _lib as L
 from .cache import Fp8KVCache, OffloadedKVCache
-from .functional import (_measuring_a_bound_pays, covered_by_launch, launch_bounded_attention, launch_fp8_attention, launch_quantize_fp8_split,
-                         launch_small_projections_e4m3, range_count, split_memory)
-from .functional import launch_small_layer as launch_small_projections  # (by its first launch: what callers and tests know and watch)
+from .functional import (_measuring_a_bound_pays, covered_by_launch, launch_fp8_attention, launch_quantize_fp8_split,
+                         launch_small_projections_e4m3, launch_text_attention, range_count, split_memory)
+from .functional import launch_small_layer as launch_small_projections  # (named by the first of the launches it stands for)
 from .functional import (div_clamp_to, head_norm, layer_norm, layer_norm_div_clamp, pow2_scale_for, qk_prologue, qk_prologue_fp8, qkv_proj_prologue,
                          quantize_fp8_split,
                          range_attention, small_projections)
@@ -1046,8 +1046,8 @@ class FullyParallelAttention(torch.nn.Module):
     def _forward_small_fp8(self, hidden_states: torch.Tensor, key_value_states: torch.Tensor, inference_params: Optional[InferenceParams],
                            rope: torch.Tensor, meta_args: ModelMetaArgs, proj_layout: bool, bound_cross: float):
         """_forward_small for e4m3 attention (the text's scores bounded): magi_small_projections_e4m3, the quantiser of V, core attention,
-        cross attention.  None where forward() goes on with the separate launches (among others in the extra forward of a first chunk, once
-        a video, whose launches the tests of the operands' preparation count), or refuses the call.  240 + 45 rows, 20 + 4
+        cross attention.  None where forward() goes on with the separate launches (among others in the extra forward of a first chunk,
+        which runs once a video and not once a step), or refuses the call.  240 + 45 rows, 20 + 4
         heads: 153 us through the callables, 66 this way."""
         use_cache = inference_params is not None and (meta_args.extract_prefix_video_feature or meta_args.slice_point > 0)
         parts = None if meta_args.fwd_extra_1st_chunk else self._small_layer_weights(hidden_states, key_value_states, rope, _OWN_SMALL_FP8)
@@ -1113,9 +1113,8 @@ class FullyParallelAttention(torch.nn.Module):
         launch_quantize_fp8_split(dev, v_raw, row, D, S, Hkv, D, Lc, 1.0, 1, v_new if kept else 0, vs_new if kept else 0, kept, v_tail, vs_tail)
         launch_fp8_attention(dev, q8, S, Hq, k_all, v_all, k_tail, v_tail, split, total, Hkv, scales, Lc, p.q_range, p.k_range, core_n,
                              p.max_seqlen_q, p.max_seqlen_k, core_out, o_row, groups, o_group, clear, self.fp8_fast_exp2)
-        launch_bounded_attention(dev, qx, Hq * D, S, Hq, text_kv, 0, T, T, 2 * row, Hkv, cp.cu_seqlens_q, cp.cu_seqlens_kv, cross_n, L.MAGI_RANGES_CU,
-                                 cp.max_seqlen_q, cp.max_seqlen_kv, cross_out, o_row, groups, o_group, clear, bound_cross,
-                                 (gx.data_ptr(), bx.data_ptr(), self.eps))
+        launch_text_attention(dev, qx, S, Hq, text_kv, T, Hkv, cp.cu_seqlens_q, cp.cu_seqlens_kv, cross_n, cp.max_seqlen_q, cp.max_seqlen_kv,
+                              cross_out, o_row, groups, o_group, clear, bound_cross, gx.data_ptr(), bx.data_ptr(), self.eps)
         return outs[0] if len(outs) == 1 else attn_linear_proj_input(*outs) if proj_layout else outs
 
     # ------------------------------------------------------------------ forward
