@@ -686,7 +686,7 @@ def test_batched_cross_attention_is_the_reference_shaped_composition_bit_for_bit
 def test_layer_output_in_linear_proj_layout(dev):
     """proj_layout=True: both attention launches write into the "(hn n hd)" buffer that linear_proj consumes
     (dit_module.py:1336-1339).  Same kernels, other store addresses: bit-identical to re-ordering the two
-    separate outputs, with and without the KV cache, and through the torch fallback at batch > 1."""
+    separate outputs, with and without the KV cache, and at batch > 1."""
     hidden, Hq, Hkv, D = 256, 16, 8, 128
     fr, H, W = 1, 3, 5
     L = fr * H * W
@@ -716,7 +716,7 @@ def test_layer_output_in_linear_proj_layout(dev):
         assert fused.shape == (S, 1, 2 * Hq * D)
         assert torch.equal(fused.cpu(), O.attn_linear_proj_input(core.cpu(), xo.cpu()))
         assert torch.count_nonzero(xo[L:]).item() == 0  # the chunk without text
-    # batch > 1: no single-stride destination exists, the module re-orders with torch
+    # batch > 1: the batch rows are further groups of heads to the core attention
     B = 2
     hs = torch.randn(L, B, hidden, generator=g).bfloat16().to(dev)
     lens = torch.tensor([4, 8])
