@@ -908,7 +908,8 @@ class FullyParallelAttention(torch.nn.Module):
         parameters converted or checked (score_bounds asks each norm for its parameter_epoch)."""
         m = self._modules
         lns = (m["q_layernorm"], m["k_layernorm"], m["q_layernorm_xattn"], m["k_layernorm_xattn"])
-        if not _OWN_BOUNDS.of(self) or _NORM_FORMS(FusedLayerNorm) != _OWN_NORM_FORMS:
+        if (type(self).score_bounds is not _SCORE_BOUNDS or "score_bounds" in self.__dict__ or FusedLayerNorm.gamma_beta_fp32 is not _GAMMA_BETA
+                or FusedLayerNorm.parameter_epoch is not _PARAMETER_EPOCH):
             return [ln.gamma_beta_fp32() for ln in lns]
         return [d["_gb"] if type(ln) is FusedLayerNorm and "gamma_beta_fp32" not in (d := ln.__dict__) and "parameter_epoch" not in d
                 else ln.gamma_beta_fp32() for ln in lns]
@@ -1291,7 +1292,6 @@ _CROSS_FUSED = FullyParallelAttention._cross_attention_fused
 _OWN_SMALL = _Own(FullyParallelAttention, "_project_rows", "_fused_qkv", "_cross_attention_fused")
 _OWN_SMALL_UNCACHED = _Own(FullyParallelAttention, "_project_rows", "_fused_qkv", "_cross_attention_fused", "core_attention")
 _OWN_SMALL_FP8 = _Own(FullyParallelAttention, "_project_rows", "_core_attention_fp8", "_cross_attention_fused")
-_OWN_BOUNDS = _Own(FullyParallelAttention, "score_bounds")
-_NORM_FORMS = operator.attrgetter("gamma_beta_fp32", "parameter_epoch")
-_OWN_NORM_FORMS = _NORM_FORMS(FusedLayerNorm)
+_SCORE_BOUNDS = FullyParallelAttention.score_bounds
+_GAMMA_BETA, _PARAMETER_EPOCH = FusedLayerNorm.gamma_beta_fp32, FusedLayerNorm.parameter_epoch
 _OWN_BATCH = _Own(FullyParallelAttention, "core_attention", "_cross_attention_fused")
