@@ -223,11 +223,6 @@ double share_us(const Pace& p, unsigned items, const unsigned* lengths, int n_ra
   }
   return parts > 0 ? t + 5.0 + 0.018 * parts : t;
 }
-// Measured, whole / in pieces: 24 items over 127 tiles 181 / 41 us, 126 over 332 455 / 186, 180 over 592 and less 795 / 428, 240 over 180 257
-// / 195, 336 over 136 265 / 210, 576 over 378 981 / 846; not cut, 384 over 16 and 32 57 / 62, 528 over 44 and 66 151 / 159, 864 over 24 to
-// 72 178 / 193, 1728 over 54 to 108 543 / 565.  The host does not know the ranges' lengths: taken are ranges that end a chunk of
-// max_seqlen_q keys apart, or all of max_seqlen_k keys where that does not go.  Only where the estimate is 6 % shorter, 10 % behind a whole round
-// (864 items over 86 to 111 tiles 402 / 410), and from 20 tiles on: max_seqlen_k of text is the padded length, of which a call may fill a fraction.
 // key tiles of each range, as far as sizes tell; false where they do not
 bool range_tiles(int n_ranges, int max_seqlen_q, int max_seqlen_k, unsigned* lengths) {
   if (max_seqlen_k <= 0 || n_ranges < 1 || n_ranges > 16) return false;
@@ -254,6 +249,12 @@ SharePlan best_pieces(const Pace& p, unsigned items, const unsigned* lengths, in
   }
   return best;
 }
+// Measured, whole / in pieces: 24 items over 127 tiles 181 / 41 us, 126 over 332 455 / 186, 180 over 592 and less 795 / 428, 240 over 180 257
+// / 195, 336 over 136 265 / 210, 576 over 378 981 / 846; not cut, 384 over 16 and 32 57 / 62, 528 over 44 and 66 151 / 159, 864 over 24 to
+// 72 178 / 193, 1728 over 54 to 108 543 / 565.  The host does not know the ranges' lengths: taken are ranges that end a chunk of
+// max_seqlen_q keys apart, or all of max_seqlen_k keys where that does not go.  Only where the estimate is 6 % shorter, 10 % behind a whole round
+// (864 items over 86 to 111 tiles 402 / 410), and from 20 tiles on: max_seqlen_k of text is the padded length, of which a call may fill a fraction.  Ranges far
+// shorter than stated lose 3 to 4 us (24 heads, 240 rows over 60 keys, 2000 stated: 6.9 / 11.0).  All drawn launches: profiles/launches_below_a_round_sweep.txt.
 SharePlan share_plan(unsigned per_xcd, int n_ranges, int max_seqlen_q, int max_seqlen_k) {
   const unsigned cus = (unsigned)compute_units(), items = 8 * per_xcd;
   unsigned lengths[16];
@@ -299,7 +300,7 @@ struct R32Plan {
 // take as long as the CU that has most of them (264 items in two each, three on 16 CUs: 1386 rows over 6930 and 13860 keys 121 / 140, 197 / 236).  Measured, before / in pieces: 6 heads, 270 rows over 1350 keys 30 / 17, three
 // ranges of 312 over 1248 to 1872 31 / 22, four of 252 33 / 20; 24 heads, 432 over 1728 36 / 29, 720 over 2880 49 / 42, three of 612 over
 // 5508 to 6732 178 / 144; not so 1080 over 5400 86 / 86, 720 over 720 21 / 25, 660 over 5940 63 / 70, 48 heads 105 / 123,
-// two of 660 over 5280 and 5940 113 / 123, four over 1980 to 3960 112 / 116 (256 rows in pieces all: their time by the mean length of the ranges).  Error against float64 over that of whole items 0.9999 to 1.0001 (27 drawn sizes).
+// two of 660 over 5280 and 5940 113 / 123, four over 1980 to 3960 112 / 116 (256 rows in pieces all: their time by the mean length of the ranges).  Error against float64 over that of whole items 1.0000 to 1.0001 (27 drawn sizes).
 // (From 16 tiles on: max_seqlen_k of text is the padded length, 800, of which a call may fill a fraction; 15 tiles would gain 4 to 6 us.)
 R32Plan make_r32_plan(int Hq, int Hkv, int n_ranges, int max_seqlen_q, int max_seqlen_k, unsigned cus, int64_t& split_bytes) {
   R32Plan plan = {false, {1, 0}};
