@@ -113,6 +113,33 @@ def test_norm_and_quantisers_in_one_launch_give_the_same_bytes(dev, rows, cols, 
         assert torch.equal(bytes_[~nan], want[~nan]) and bool(((bytes_[nan] & 0x7f) == 0x7f).all())
 
 
+def test_rows_of_whole_rounds_ahead_of_the_rest(dev, monkeypatch):
+    """forward_quantized cuts the rows behind whole rounds of tiles in two calls of the library: the bits of one call (256 CUs: 16384 rows
+    are one round at 1024 columns), and one call where the rest is long, a gradient is asked for or the tensor is another class."""
+    K, N, rows = 1024, 1024, 16384 + 300
+    m = MOD.PerTensorQuantizedFp8Linear(K, N, device=dev)
+    m.weight.data = (torch.randn(1, N, K, device=dev) * 40).clamp(-448, 448).to(torch.float8_e4m3fn)
+    m.weight_scale.data.fill_(0.02)
+    m.input_scale.data.fill_(0.01)
+    x8 = (torch.randn(rows, K, device=dev) * 40).clamp(-448, 448).to(torch.float8_e4m3fn)
+    calls, product = [], torch._scaled_mm
+    monkeypatch.setattr(torch, "_scaled_mm", lambda x, *a, **k: calls.append(x.shape[0]) or product(x, *a, **k))
+    monkeypatch.setattr(MOD, "_compute_units", lambda device: 256)
+    y = m.forward_quantized(x8)
+    assert calls == [16384, 300] and y.shape == (rows, N) and y.dtype == torch.bfloat16
+    want = product(x8, m.weight[0].t(), scale_a=m.input_scale[:1], scale_b=m.weight_scale, out_dtype=torch.bfloat16)
+    assert torch.equal(y, want)
+    calls.clear()
+    assert torch.equal(m.forward_quantized(x8.view(2, rows // 2, K)), want.view(2, rows // 2, N)) and calls == [16384, 300]
+    calls.clear()
+    m.forward_quantized(x8[:16384])
+    m.weight_scale.requires_grad_(True)
+    m.forward_quantized(x8)
+    with torch.no_grad():
+        m.forward_quantized(x8)
+    assert calls == [16384, rows, 16384, 300]
+
+
 def test_projections_hold_no_more_memory_than_norm_and_quantisers_apart(dev):
     """The e4m3 inputs of the four linears are given back one by one: the most that is held is below the outputs, the norm's
     bf16 rows and one e4m3 input, which is what separate calls hold."""

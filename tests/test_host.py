@@ -405,6 +405,19 @@ def test_projection_rows_are_cut_only_where_a_round_of_tiles_is_left_partly_empt
         assert _rows_ahead(9360, cols_, depth, cus) == 0
 
 
+@pytest.mark.parametrize("cols,whole", [(1024, 16384), (3072, 16384), (6144, 8192), (8192, 2048), (256, 65536), (5120, 16384)])
+def test_e4m3_rows_are_cut_behind_rounds_that_are_whole_to_the_last_tile(cols, whole):
+    from magi_attn.module import _rows_ahead_e4m3
+
+    for n in (0, 1, 2, 7, 9):
+        for rest in (0, 1, n * whole // 7, n * whole // 7 + 1, whole - 1):
+            if rest >= whole:
+                continue
+            assert _rows_ahead_e4m3(n * whole + rest, cols, 1024, 256) == (n * whole if 0 < rest and 7 * rest <= n * whole else 0), (n, rest)
+    for cols_, depth, cus in ((1024, 1016, 256), (1000, 3072, 256), (0, 3072, 256), (131072, 3072, 256)):
+        assert _rows_ahead_e4m3(16974, cols_, depth, cus) == 0
+
+
 def test_replaced_projection_methods_are_called(monkeypatch):
     """forward() projects through linear_qkv.forward_ln and .forward_qkvx where these are not the library's own: another module
     that offers the two, a subclass, a method patched onto the instance."""
