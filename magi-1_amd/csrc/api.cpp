@@ -30,6 +30,16 @@ int hip_fail(hipError_t e, const char* what) {
 
 std::atomic<uint64_t> g_launches{0};
 
+// Counts n launches, and touches thread-local storage of this library.  The C library's table of a thread's storage (the DTV) is brought up to
+// date only by an access to a module that was loaded behind the last update, and until then every access of every older module, torch's and HIP's
+// on each call, takes the long way.  This library is among the last to be loaded.  Issued calls, 240 rows of rotary 7.14 -> 6.30 us, online softmax of
+// 128 rows 13.9 -> 12.0, of one text segment 12.1 -> 10.4.  (Bounded launches touched it before, by their kept plans.)
+thread_local volatile unsigned g_touched = 0;
+void count_launches(uint64_t n) {
+  g_touched = 1;
+  g_launches.fetch_add(n, std::memory_order_relaxed);
+}
+
 // the caller's view of an argument struct must be this library's
 template <class T>
 bool same_layout(const T* p) { return p->struct_size == sizeof(T); }
@@ -707,7 +717,7 @@ int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace) {
     else
       e = magi::launch_attn_fwd_bf16(a, static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return hip_fail(e, "magi_attn_fwd launch");
-    g_launches.fetch_add((checked ? 2 : 1) + (a.split_from < a.per_xcd) + (a.share_pieces > 1), std::memory_order_relaxed);
+    count_launches((checked ? 2 : 1) + (a.split_from < a.per_xcd) + (a.share_pieces > 1));
     return MAGI_OK;
   };
 
@@ -728,7 +738,7 @@ int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace) {
   if (e == hipSuccess && p->total_k > k_split)
     e = magi::launch_row_norm_max(a.k2, a.ks_t, a.ks_h, p->total_k - k_split, p->Hkv, ws + 1, st);
   if (e != hipSuccess) return hip_fail(e, "magi_attn_fwd bound measurement");
-  g_launches.fetch_add(2 + (k_split > 0) + (p->total_k > k_split), std::memory_order_relaxed);
+  count_launches(2 + (k_split > 0) + (p->total_k > k_split));
   a.gate = workspace;
   a.gate_want = 1;
   int rc = launch(true);
@@ -839,7 +849,7 @@ int small_projections_impl(const magi_small_proj_args* p, const SmallProjE4m3* e
   }
   hipError_t e = magi::launch_small_proj(a, compute_units(), static_cast<hipStream_t>(stream));
   if (e != hipSuccess) return hip_fail(e, "magi_small_projections launch");
-  g_launches.fetch_add(1, std::memory_order_relaxed);
+  count_launches(1);
   return MAGI_OK;
 }
 
@@ -914,7 +924,7 @@ int magi_qk_prologue(const magi_prologue_args* p, void* stream) {
   a.q_premul = p->q_premul == 0.f ? 1.f : p->q_premul;
   hipError_t e = magi::launch_prologue(a, static_cast<hipStream_t>(stream));
   if (e != hipSuccess) return hip_fail(e, "magi_qk_prologue launch");
-  g_launches.fetch_add(1, std::memory_order_relaxed);
+  count_launches(1);
   return MAGI_OK;
 }
 
@@ -983,7 +993,7 @@ int magi_qkv_proj_prologue(const magi_qkv_proj_args* p, void* stream) {
   a.q_premul = p->q_premul == 0.f ? 1.f : p->q_premul;
   hipError_t e = magi::launch_qkv_gemm_prologue(a, static_cast<hipStream_t>(stream));
   if (e != hipSuccess) return hip_fail(e, "magi_qkv_proj_prologue launch");
-  g_launches.fetch_add(1, std::memory_order_relaxed);
+  count_launches(1);
   return MAGI_OK;
 }
 
@@ -1114,7 +1124,7 @@ int magi_layer_norm(const void* x, int64_t x_stride, const void* weight, const v
                                          static_cast<char*>(y), y_stride * 2, rows, cols, eps,
                                          static_cast<hipStream_t>(stream));
   if (e != hipSuccess) return hip_fail(e, "magi_layer_norm launch");
-  g_launches.fetch_add(1, std::memory_order_relaxed);
+  count_launches(1);
   return MAGI_OK;
 }
 
@@ -1150,7 +1160,7 @@ int magi_layer_norm_e4m3(const void* x, int64_t x_stride, const void* weight, co
   a.eps = eps;
   hipError_t e = magi::launch_layer_norm_quant(a, params_fp32 != 0, compute_units(), static_cast<hipStream_t>(stream));
   if (e != hipSuccess) return hip_fail(e, "magi_layer_norm_e4m3 launch");
-  g_launches.fetch_add(1, std::memory_order_relaxed);
+  count_launches(1);
   return MAGI_OK;
 }
 
@@ -1170,7 +1180,7 @@ int magi_div_clamp_to_e4m3(const void* x, int64_t x_stride, const float* scale, 
   hipError_t e = magi::launch_div_clamp(static_cast<const char*>(x), x_stride * 2, scale, scale_len != 1,
                                         static_cast<char*>(y), y_stride, rows, cols, static_cast<hipStream_t>(stream));
   if (e != hipSuccess) return hip_fail(e, "magi_div_clamp_to_e4m3 launch");
-  g_launches.fetch_add(1, std::memory_order_relaxed);
+  count_launches(1);
   return MAGI_OK;
 }
 
@@ -1187,7 +1197,7 @@ int magi_head_norm(const void* x, int64_t x_stride_t, int64_t x_stride_h, const 
   hipError_t e = magi::launch_head_norm(static_cast<const char*>(x), x_stride_t * 2, x_stride_h * 2, gamma, beta,
                                         static_cast<char*>(y), S, H, norm_kind, eps, static_cast<hipStream_t>(stream));
   if (e != hipSuccess) return hip_fail(e, "magi_head_norm launch");
-  g_launches.fetch_add(1, std::memory_order_relaxed);
+  count_launches(1);
   return MAGI_OK;
 }
 
@@ -1199,7 +1209,7 @@ int magi_apply_rotary(const void* x, const float* cos, const float* sin, void* y
   if (!x || !y || (R2 > 0 && (!cos || !sin))) return fail(MAGI_EINVAL, "magi_apply_rotary: NULL pointer");
   hipError_t e = magi::launch_rotary(x, cos, sin, y, B, S, H, D, R2, is_bf16, static_cast<hipStream_t>(stream));
   if (e != hipSuccess) return hip_fail(e, "magi_apply_rotary launch");
-  g_launches.fetch_add(1, std::memory_order_relaxed);
+  count_launches(1);
   return MAGI_OK;
 }
 
@@ -1228,7 +1238,7 @@ static int quantize_impl(const magi_quantize_args* p, void* stream, bool always_
                                            p->pow2_scales, p->n_rows_first, static_cast<char*>(p->y2), p->scales2,
                                            always_one_launch, compute_units(), static_cast<hipStream_t>(stream), &n_launches);
   if (e != hipSuccess) return hip_fail(e, "magi_quantize_fp8 launch");
-  g_launches.fetch_add((uint64_t)n_launches, std::memory_order_relaxed);
+  count_launches((uint64_t)n_launches);
   return MAGI_OK;
 }
 
