@@ -83,6 +83,11 @@ extern "C" {
  * MAGI_ATTN_AUTO_BOUND this holds of each of the two kernels; which of them runs, for all rows of the launch, follows from the longest
  * rows of q and of k in it, those of other ranges included: for a row's bits whatever the launch, state a score_bound or none. */
 #define MAGI_ATTN_ROW_BITS 128
+/* bf16 with a score_bound in force: the keys of a row may be shared by the wavefronts of a workgroup where the launch is so small that
+ * it waits for its longest row (32 rows to a workgroup, about one workgroup per CU; from max_seqlen_k, which has to be stated, and the other
+ * sizes alone).  The fp32 sums are then added in another order, as with split_workspace; no memory is needed.  Ignored elsewhere; not
+ * with MAGI_ATTN_ROW_BITS. */
+#define MAGI_ATTN_SHARE_WAVES 1024
 
 #define MAGI_RANGES_PAIRS 0 /* int32 [n, 2]: range i = [r[2i], r[2i+1])          */
 #define MAGI_RANGES_CU 1    /* int32 [n + 1] cumulative: range i = [r[i], r[i+1]) */
@@ -96,7 +101,8 @@ extern "C" {
  * with its own size as the caller compiled it (struct_size = sizeof(the struct)), and an entry point that is handed
  * another size returns MAGI_EINVAL instead of reading fields the caller never wrote.
  * 105: the structs of 104; new are MAGI_ATTN_ROW_BITS (a library of 104 would ignore it), magi_attn_split_bytes_256,
- * magi_attn_pieces_bytes, magi_small_projections_e4m3 and magi_small_layer. */
+ * magi_attn_pieces_bytes, magi_small_projections_e4m3 and magi_small_layer.
+ * 106: the structs of 105; new are MAGI_ATTN_SHARE_WAVES, magi_attn_waves and magi_attn_fwd_two. */
 int magi_version(void);
 const char* magi_last_error(void);
 /* Diagnostics: the number of kernel launches the library has issued in this process so far (all threads, all
@@ -258,7 +264,16 @@ int64_t magi_attn_pieces_bytes(int32_t Hq, int32_t Hkv, int32_t n_ranges, int32_
  * of 256 in a partly empty round).  A row's bits are the same in all of these, without that memory. */
 int32_t magi_attn_tile_rows(int32_t Hq, int32_t Hkv, int32_t n_ranges, int32_t max_seqlen_q, int32_t max_seqlen_k, int64_t split_workspace_bytes);
 
+/* Wavefronts that share the keys of a row where such a call has MAGI_ATTN_SHARE_WAVES and a score_bound in force, no split_workspace's use
+ * then; 0: it takes the other forms. */
+int32_t magi_attn_waves(int32_t Hq, int32_t Hkv, int32_t n_ranges, int32_t ranges_mode, int32_t max_seqlen_q, int32_t max_seqlen_k);
+
 int magi_attn_fwd(const magi_attn_args* args, void* stream);
+
+/* magi_attn_fwd of two calls that do not depend on each other and write different outputs (a layer's core and text attention): in one
+ * launch where both take the form of MAGI_ATTN_SHARE_WAVES, else one after the other; the same bits as two calls.  A refusal of the
+ * second is this call's, the first has been launched by then. */
+int magi_attn_fwd_two(const magi_attn_args* first, const magi_attn_args* second, void* stream);
 
 /*
  * magi_attn_fwd for callers that cannot hand over a workspace and must not allocate one (code under HIP graph
@@ -425,11 +440,11 @@ int magi_small_projections(const magi_small_proj_args* args, void* stream);
 int magi_small_projections_e4m3(const magi_small_proj_args* args, float q_quant_scale, float k_quant_scale, void* v_out, void* stream);
 
 /*
- * The three launches of a small bf16 layer at batch 1 with bounded scores in one call: magi_small_projections (norm, q | k | v | qx, text K | V),
+ * The launches of a small bf16 layer at batch 1 with bounded scores in one call: magi_small_projections (norm, q | k | v | qx, text K | V),
  * the core attention of the rows q over [kv[:k_split] | kv_side], the cross attention of the rows qx over text_kv.  What it stands for
  * in those calls' structs: strides in elements; heads 128 apart; K | V interleaved per head, kv_row elements a row, the new rows to kv_new (kept of
  * them) and kv_side; q, qx [S, Hq, 128], text_kv [T, Hkv, 256]; pairs for core, cumulative lengths for cross; split workspaces of their own.
- * parts: 1 = the first two, 2 = the last, 3 = all.  A refusal of one of the three is this call's, what is ahead of it has been launched.
+ * parts: 1 = the first two, 2 = the last, 3 = all, the two attention calls as magi_attn_fwd_two makes them.  A refusal of one of the three is this call's, what is ahead of it has been launched.
  */
 typedef struct magi_small_layer_args {
   uint32_t struct_size; /* sizeof(magi_small_layer_args) */

@@ -380,7 +380,30 @@ int64_t r32_bytes(int Hq, int Hkv, int n_ranges, int max_seqlen_q, int max_seqle
       .share.bytes(items_per_xcd(Hq, Hkv, n_ranges, max_seqlen_q / 128 + (max_seqlen_q % 128 != 0)));
 }
 
-int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace);
+// Whether a launch without a running maximum whose caller permits it (MAGI_ATTN_SHARE_WAVES) has the keys of 32 rows shared by the wavefronts of
+// a workgroup (attn_fwd_bf16_waves.hip): how many wavefronts, 0: not.
+// Eight, a workgroup per CU, or four, two of them.  Measured, 128 and 256 rows to a workgroup (in pieces where that was the better) / this form, drawn sizes
+// (profiles/launches_below_a_round_sweep.txt): up to one workgroup of 32 rows per CU 120 launches 0.94 to 1.76 times as fast, 1.23 on average (12
+// workgroups over 519 keys 14.9 / 11.5 us, 48 over 480 13.4 / 9.1, 192 over 945 21.5 / 12.7, 216 over 5040 35.9 / 30.9, 240 over 7632 43.5 / 44.5);
+// four wavefronts up to 1024 keys (96 over 691 18.2 / 12.7 with either) and for more than a workgroup per CU: 288 over 594 15.5 / 12.7, 360 over 1600 27.8 / 19.5, 416 over 4040
+// 45.6 / 39.3, but 288 over 5085 40.8 / 47.1, 312 over 8100 52.7 / 72.6; beyond two per CU 576 over 1050 23.6 / 27.3.  max_seqlen_k of text is the padded
+// length: 288 workgroups over 39 of 800 keys 7.6 / 8.0, 504 over 184 10.4 / 12.5, so cumulative lengths only up to one per CU.
+int waves_plan(int Hq, int Hkv, int n_ranges, int ranges_mode, int max_seqlen_q, int max_seqlen_k) {
+  if ((double)Hq * n_ranges * (max_seqlen_q / 32 + 1) > 2.0e9) return 0;
+  const double items = 8.0 * items_per_xcd(Hq, Hkv, n_ranges, max_seqlen_q / 32 + (max_seqlen_q % 32 != 0));
+  const int cus = compute_units();
+  if (max_seqlen_k <= 0 || items > (ranges_mode == MAGI_RANGES_CU ? 1 : 2) * cus) return 0;
+  if (max_seqlen_k <= 1024) return 4;
+  if (items <= cus) return max_seqlen_k <= 8192 ? 8 : 0;
+  return max_seqlen_k <= 4096 ? 4 : 0;
+}
+
+// held: where the call takes the form that may share a launch with another, its arguments instead of the launch; HELD is returned then
+constexpr int HELD = 1;
+int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace, magi::AttnKernArgs* held = nullptr);
+// one or two held calls in one launch
+int launch_held(const magi::AttnPairArgs& pair, void* stream);
+int attn_fwd_two(const magi_attn_args* first, const magi_attn_args* second, void* stream);
 
 // the caller's struct as this version lays it out: itself, or `full` filled from the shorter one of version 103
 const magi_attn_args* current_layout(const magi_attn_args* p, magi_attn_args* full) {
@@ -396,7 +419,7 @@ const magi_attn_args* current_layout(const magi_attn_args* p, magi_attn_args* fu
 
 extern "C" {
 
-int magi_version(void) { return 105; }
+int magi_version(void) { return 106; }
 
 uint64_t magi_launch_count(void) { return g_launches.load(std::memory_order_relaxed); }
 
@@ -430,6 +453,11 @@ int64_t magi_attn_pieces_bytes(int32_t Hq, int32_t Hkv, int32_t n_ranges, int32_
   return share_plan(items, n_ranges, max_seqlen_q, max_seqlen_k).bytes(items);
 }
 
+int32_t magi_attn_waves(int32_t Hq, int32_t Hkv, int32_t n_ranges, int32_t ranges_mode, int32_t max_seqlen_q, int32_t max_seqlen_k) {
+  if (Hq <= 0 || Hkv <= 0 || Hq % Hkv || n_ranges <= 0 || max_seqlen_q <= 0) return 0;
+  return waves_plan(Hq, Hkv, n_ranges, ranges_mode, max_seqlen_q, max_seqlen_k);
+}
+
 int32_t magi_attn_tile_rows(int32_t Hq, int32_t Hkv, int32_t n_ranges, int32_t max_seqlen_q, int32_t max_seqlen_k,
                             int64_t split_workspace_bytes) {
   if (Hq <= 0 || Hkv <= 0 || Hq % Hkv || n_ranges <= 0 || max_seqlen_q <= 0) return 256;
@@ -443,6 +471,13 @@ int magi_attn_fwd(const magi_attn_args* p, void* stream) {
   p = current_layout(p, &full);
   MAGI_CHECK_LAYOUT("magi_attn_fwd", p);
   return attn_fwd_impl(p, stream, p->workspace);
+}
+
+int magi_attn_fwd_two(const magi_attn_args* first, const magi_attn_args* second, void* stream) {
+  if (!first || !second) return fail(MAGI_EINVAL, "magi_attn_fwd_two: args is NULL");
+  MAGI_CHECK_LAYOUT("magi_attn_fwd_two", first);
+  MAGI_CHECK_LAYOUT("magi_attn_fwd_two", second);
+  return attn_fwd_two(first, second, stream);
 }
 
 int magi_attn_fwd_static_scratch(const magi_attn_args* p, void* stream) {
@@ -463,7 +498,26 @@ int magi_attn_fwd_static_scratch(const magi_attn_args* p, void* stream) {
 
 namespace {
 
-int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace) {
+int launch_held(const magi::AttnPairArgs& pair, void* stream) {
+  const hipError_t e = magi::launch_attn_fwd_bf16_waves(pair, static_cast<hipStream_t>(stream));
+  if (e != hipSuccess) return hip_fail(e, "magi_attn_fwd launch");
+  count_launches(1);
+  return MAGI_OK;
+}
+
+// first, then second, which do not depend on each other: in one launch where both take the form for it
+int attn_fwd_two(const magi_attn_args* first, const magi_attn_args* second, void* stream) {
+  magi::AttnPairArgs pair;
+  const int one = attn_fwd_impl(first, stream, first->workspace, &pair.job[0]);
+  if (one < 0) return one;
+  const int two = attn_fwd_impl(second, stream, second->workspace, &pair.job[one == HELD ? 1 : 0]);
+  if (one != HELD && two != HELD) return two;
+  if ((one == HELD) != (two == HELD)) pair.job[1].per_xcd = 0;
+  const int rc = launch_held(pair, stream);
+  return two < 0 ? two : rc;
+}
+
+int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace, magi::AttnKernArgs* held) {
   if (p->D != 128) return fail(MAGI_ENOSYS, "magi_attn_fwd: head_dim %d not implemented (128 only)", p->D);
   if (p->dtype != MAGI_DTYPE_BF16 && p->dtype != MAGI_DTYPE_FP8_E4M3)
     return fail(MAGI_EINVAL, "magi_attn_fwd: unknown dtype %d", p->dtype);
@@ -528,6 +582,8 @@ int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace) {
     if (!workspace || !aligned16(workspace))
       return fail(MAGI_EINVAL, "magi_attn_fwd: MAGI_ATTN_AUTO_BOUND needs a 16-byte workspace on the device, 16-byte aligned");
   }
+  if ((p->flags & MAGI_ATTN_ROW_BITS) && (p->flags & MAGI_ATTN_SHARE_WAVES))
+    return fail(MAGI_EINVAL, "magi_attn_fwd: MAGI_ATTN_ROW_BITS and MAGI_ATTN_SHARE_WAVES exclude each other");
   if ((p->flags & MAGI_ATTN_ROW_BITS) && (p->split_workspace || p->dtype != MAGI_DTYPE_BF16))
     return fail(MAGI_EINVAL, "magi_attn_fwd: MAGI_ATTN_ROW_BITS goes with bf16 and without split_workspace");
   const bool checked = (p->flags & MAGI_ATTN_CHECKED) != 0;
@@ -650,9 +706,13 @@ int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace) {
     if (p->dtype == MAGI_DTYPE_BF16) {
       const double wg384 = (double)p->Hq * p->n_ranges * ((p->max_seqlen_q + 383) / 384);
       const bool long_keys = p->max_seqlen_k == 0 || p->max_seqlen_k >= 4096;  // (0 = not stated)
-      if (bounded && !checked && !mfma32 && p->q_tile_rows == 0)
+      if (bounded && !checked && !auto_bound && !mfma32 && p->q_tile_rows == 0 && (p->flags & MAGI_ATTN_SHARE_WAVES))
+        a.waves = waves_plan(p->Hq, p->Hkv, p->n_ranges, p->ranges_mode, p->max_seqlen_q, p->max_seqlen_k);
+      if (bounded && !checked && !mfma32 && p->q_tile_rows == 0 && !a.waves)
         r32 = r32_plan(p->Hq, p->Hkv, p->n_ranges, p->max_seqlen_q, p->max_seqlen_k, split_bytes);
-      if (r32.use)
+      if (a.waves)
+        a.block_m = 32;
+      else if (r32.use)
         a.block_m = 128;
       else if (bounded && !checked && !mfma32)
         a.block_m = tile_rows(p->Hq, p->Hkv, p->n_ranges, p->max_seqlen_q, p->max_seqlen_k, split_bytes);
@@ -682,6 +742,16 @@ int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace) {
       if (s.pieces > 1) a.partial = static_cast<float*>(p->split_workspace);
     };
     a.share_pieces = 1;
+    if (a.waves) {
+      magi::AttnPairArgs pair;
+      if (held) {
+        *held = a;
+        return HELD;
+      }
+      pair.job[0] = a;
+      pair.job[1].per_xcd = 0;
+      return launch_held(pair, stream);
+    }
     if (r32.use) pieces(r32.share);
     if ((fp8 || (bounded && a.block_m == 256 && !mfma32)) && split_bytes > 0) {
       const SplitPlan s = split_plan(a.per_xcd, p->n_ranges, p->max_seqlen_q, p->max_seqlen_k, fp8);
@@ -1074,13 +1144,14 @@ int magi_small_layer(const magi_small_layer_args* p, void* stream) {
     a.ranges_mode = MAGI_RANGES_PAIRS;
     a.max_seqlen_q = p->max_core_q;
     a.max_seqlen_k = p->max_core_k;
-    a.flags = MAGI_ATTN_Q_PRESCALED | p->core_flags;
+    a.flags = MAGI_ATTN_Q_PRESCALED | MAGI_ATTN_SHARE_WAVES | p->core_flags;
     a.score_bound = p->core_bound;
     a.out = p->core_out;
     a.split_workspace = p->core_split;
     a.split_workspace_bytes = p->core_split_bytes;
-    if (const int rc = attn_fwd_impl(&a, stream, nullptr)) return rc;
+    if (p->parts == 1) return attn_fwd_impl(&a, stream, nullptr);
   }
+  const magi_attn_args core = a;
   if (p->parts & 2) {
     a.q = p->qx;
     a.k = p->text_kv;
@@ -1094,7 +1165,7 @@ int magi_small_layer(const magi_small_layer_args* p, void* stream) {
     a.ranges_mode = MAGI_RANGES_CU;
     a.max_seqlen_q = p->max_cross_q;
     a.max_seqlen_k = p->max_cross_k;
-    a.flags = p->cross_flags;
+    a.flags = MAGI_ATTN_SHARE_WAVES | p->cross_flags;
     a.score_bound = p->cross_bound;
     a.out = p->cross_out;
     a.split_workspace = p->cross_split;
@@ -1103,7 +1174,7 @@ int magi_small_layer(const magi_small_layer_args* p, void* stream) {
     a.q_norm_beta = p->bqx;
     a.q_norm_eps = p->eps;
     a.q_norm_kind = MAGI_NORM_LAYERNORM_1P;
-    return attn_fwd_impl(&a, stream, nullptr);
+    return p->parts == 3 ? attn_fwd_two(&core, &a, stream) : attn_fwd_impl(&a, stream, nullptr);
   }
   return MAGI_OK;
 }

@@ -56,6 +56,7 @@ struct AttnKernArgs {
   // Online softmax, 128-row workgroups: the keys of every item in up to share_pieces pieces of share_tiles tiles each (0 or 1:
   // whole; `partial`: ONLINE_PARTIAL_FLOATS floats per item and piece).
   unsigned share_pieces, share_tiles;
+  int waves;  // attn_fwd_bf16_waves.hip: wavefronts that share the keys of a workgroup's rows, 4 or 8
 };
 // online softmax: 128 rows x 128 accumulators, 128 row sums, 128 row maxima
 constexpr int ONLINE_PARTIAL_FLOATS = 128 * 128 + 256;
@@ -80,6 +81,11 @@ constexpr int ATTN_ZERO_GAPS = 32;
 
 hipError_t launch_attn_fwd_bf16(const AttnKernArgs& a, hipStream_t stream);
 hipError_t launch_attn_fwd_bf16_r32(const AttnKernArgs& a, hipStream_t stream);
+// One or two calls (job[1].per_xcd = 0: one), bounded scores, block_m 32: the wavefronts of a workgroup share the keys of 32 rows
+struct AttnPairArgs {
+  AttnKernArgs job[2];
+};
+hipError_t launch_attn_fwd_bf16_waves(const AttnPairArgs& p, hipStream_t stream);
 hipError_t launch_attn_fwd_bf16_w64(const AttnKernArgs& a, hipStream_t stream);
 // (with items to split: and behind it the launch that adds their pieces up)
 hipError_t launch_attn_fwd_bf16_x16(const AttnKernArgs& a, hipStream_t stream);

@@ -27,6 +27,7 @@ MAGI_ATTN_AUTO_BOUND = 16
 MAGI_ATTN_ZERO_UNCOVERED = 32
 MAGI_ATTN_CHECKED = 64
 MAGI_ATTN_ROW_BITS = 128
+MAGI_ATTN_SHARE_WAVES = 1024
 MAGI_SCORE_BOUND_MAX = 64.0
 
 
@@ -144,9 +145,9 @@ class SmallLayerArgs(_SizedStructure):
     ]
 
 
-ABI_VERSION = 105  # magi_version() of the library these mirrors were written for
+ABI_VERSION = 106  # magi_version() of the library these mirrors were written for
 
-EXPORTS = ("magi_version", "magi_last_error", "magi_launch_count", "magi_attn_fwd", "magi_attn_fwd_static_scratch",
+EXPORTS = ("magi_version", "magi_last_error", "magi_launch_count", "magi_attn_fwd", "magi_attn_fwd_two", "magi_attn_waves", "magi_attn_fwd_static_scratch",
            "magi_attn_split_bytes", "magi_attn_split_bytes_256", "magi_attn_pieces_bytes", "magi_attn_tile_rows",
            "magi_qk_prologue", "magi_head_norm",
            "magi_apply_rotary", "magi_quantize_fp8", "magi_quantize_fp8_split", "magi_layer_norm", "magi_qkv_proj_prologue", "magi_div_clamp_to_e4m3",
@@ -182,8 +183,12 @@ def lib() -> C.CDLL:
         l.magi_attn_pieces_bytes.restype = C.c_int64
         l.magi_attn_tile_rows.argtypes = [C.c_int32] * 5 + [C.c_int64]
         l.magi_attn_tile_rows.restype = C.c_int32
+        l.magi_attn_waves.argtypes = [C.c_int32] * 6
+        l.magi_attn_waves.restype = C.c_int32
         l.magi_attn_fwd.argtypes = [C.POINTER(AttnArgs), C.c_void_p]
         l.magi_attn_fwd.restype = C.c_int
+        l.magi_attn_fwd_two.argtypes = [C.POINTER(AttnArgs), C.POINTER(AttnArgs), C.c_void_p]
+        l.magi_attn_fwd_two.restype = C.c_int
         l.magi_attn_fwd_static_scratch.argtypes = [C.POINTER(AttnArgs), C.c_void_p]
         l.magi_attn_fwd_static_scratch.restype = C.c_int
         l.magi_qk_prologue.argtypes = [C.POINTER(PrologueArgs), C.c_void_p]
@@ -236,7 +241,23 @@ class PackedCall:
         self.fn.argtypes, self.fn.restype = [C.c_char_p, *more, C.c_void_p], C.c_int
 
 
+class PackedPair:
+    """The same for an entry point of two packed structs of one kind."""
+
+    def __init__(self, name: str):
+        self.fn = lib()[name]
+        self.fn.argtypes, self.fn.restype = [C.c_char_p, C.c_char_p, C.c_void_p], C.c_int
+
+
 _packed = {}
+
+
+def packed_pair(name: str) -> PackedPair:
+    call = _packed.get(name)
+    if call is None:
+        call = _packed[name] = PackedPair(name)
+    return call
+
 
 
 def packed(name: str, args: type, *more: type) -> PackedCall:

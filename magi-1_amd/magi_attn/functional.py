@@ -133,6 +133,8 @@ def range_attention(
     return_lse: bool = True,
     zero_init: bool = True,
     split_keys: bool = True,
+    share_waves: bool = False,
+    held: Optional[list] = None,
 ) -> Tuple[torch.Tensor, Optional[torch.Tensor]]:
     """out[q_range_i] = softmax(q k^T * scale) v over k[k_range_i]; see magi_attn_fwd.
 
@@ -164,6 +166,9 @@ def range_attention(
     order).  Whether it does follows from the sizes of the launch alone, except that the online softmax runs without where there is no such
     memory to be had (the others raise).  Needs max_seqlen_k.  Without it a bf16 row's bits depend on its own range alone (MAGI_ATTN_ROW_BITS); with
     auto_bound also on which of the two kernels the longest rows of the whole call select.
+    share_waves (with split_keys, a score_bound and max_seqlen_k): in launches of a few rows the wavefronts of a workgroup may share the keys of
+    a row, MAGI_ATTN_SHARE_WAVES.
+    held: the call is appended here instead of launched; launch_held() then launches one or two of them.
     q may be [batch, rows, Hq, D] with any batch stride (batch of activations laid out [position, batch, ...]): its rows
     count as batch * rows tokens for the ranges, out is (or comes back as) a tensor of q's shape, by default
     [rows, batch, Hq, D] transposed.  Needs a score_bound (math.inf: the online softmax).
@@ -236,14 +241,17 @@ def range_attention(
     flags = ((L.MAGI_ATTN_FP8_POW2_PRESCALED if fp8_pow2_prescaled else 0) | (L.MAGI_ATTN_Q_PRESCALED if q_prescaled else 0)
              | (L.MAGI_ATTN_FP8_FAST_EXP2 if fp8_fast_exp2 else 0) | (L.MAGI_ATTN_BOUNDED_MFMA32 if bounded_mfma32 else 0)
              | (L.MAGI_ATTN_AUTO_BOUND if auto_bound else 0) | (L.MAGI_ATTN_ZERO_UNCOVERED if zero_gaps else 0)
-             | (L.MAGI_ATTN_CHECKED if checked else 0) | (0 if split_keys or q.dtype is not torch.bfloat16 else L.MAGI_ATTN_ROW_BITS))
+             | (L.MAGI_ATTN_CHECKED if checked else 0) | (L.MAGI_ATTN_SHARE_WAVES if share_waves and split_keys else 0) | (0 if split_keys or q.dtype is not torch.bfloat16 else L.MAGI_ATTN_ROW_BITS))
     workspace = None
     if checked:
         workspace = torch.empty(max(4 * Hq * max(n, 0) * ((int(max_seqlen_q) + 255) // 256), 4), dtype=torch.int32, device=q.device)
     if auto_bound and not static_scratch:
         workspace = torch.empty(4, dtype=torch.float32, device=q.device)  # (alive until the launches are enqueued)
     split, split_bytes, online = None, 0, False
-    if split_keys and not static_scratch and max_seqlen_k >= 512 and (
+    if (share_waves and split_keys and q.dtype is torch.bfloat16 and 0.0 < score_bound <= L.MAGI_SCORE_BOUND_MAX and not (q_tile_rows or bounded_mfma32)
+            and attention_waves(Hq, Hkv, n, ranges_mode, max_seqlen_q, max_seqlen_k)):
+        pass  # (keys shared without memory)
+    elif split_keys and not static_scratch and max_seqlen_k >= 512 and (
             checked or auto_bound or 0.0 < score_bound <= L.MAGI_SCORE_BOUND_MAX or q.dtype is torch.float8_e4m3fn):
         if q.dtype is not torch.bfloat16:
             split_bytes = L.lib().magi_attn_split_bytes(Hq, Hkv, max(n, 0), int(max_seqlen_q), int(max_seqlen_k), _dtype_code(q))
@@ -268,16 +276,32 @@ def range_attention(
         norm_eps = float(q_norm[2])
         norm_kind = int(q_norm[3]) if len(q_norm) > 3 else L.MAGI_NORM_LAYERNORM_1P
     k_stride, v_stride = k.stride(), v.stride()
-    _launch_packed(
-        q.device, "magi_attn_fwd_static_scratch" if static_scratch else "magi_attn_fwd", L.AttnArgs,
-        q.data_ptr(), k.data_ptr(), v.data_ptr(), _ptr(k2), _ptr(v2), out.data_ptr(), _ptr(lse), q_ranges.data_ptr(),
+    call = L.packed("magi_attn_fwd_static_scratch" if static_scratch else "magi_attn_fwd", L.AttnArgs)
+    args = call.pack(
+        call.size, q.data_ptr(), k.data_ptr(), v.data_ptr(), _ptr(k2), _ptr(v2), out.data_ptr(), _ptr(lse), q_ranges.data_ptr(),
         k_ranges.data_ptr(), _ptr(q_scale), _ptr(k_scale), _ptr(v_scale), q_stride[-3], q_stride[-2], k_stride[0], k_stride[1],
         v_stride[0], v_stride[1], o_stride_t, o_stride[-2], Tq, total_k, total_k if k2 is None else int(k_split), max(n, 0),
         ranges_mode, int(max_seqlen_q), int(max_seqlen_k), Hq, Hkv, D, _dtype_code(q), int(scale_chunk_tokens),
         0.0 if softmax_scale is None else float(softmax_scale), flags, group_heads, o_stride_g,
         min(float(score_bound), 3e38), int(q_tile_rows), _ptr(gamma), _ptr(beta), norm_eps, norm_kind, _ptr(k2_scale),
         _ptr(v2_scale), _ptr(workspace), batch_rows, q_stride_b, o_stride_b, _ptr(split), split_bytes)
+    if held is None:
+        _launch(q.device, call.fn, args)
+    else:  # (with everything it reads and writes)
+        held.append((q.device, call.fn, args, (q, k, v, k2, v2, q_ranges, k_ranges, q_scale, k_scale, v_scale, k2_scale, v2_scale, gamma, beta, workspace,
+                                               split, out, lse)))
     return out, lse
+
+
+def launch_held(calls: list) -> None:
+    """The calls that range_attention(held=calls) left, on the current stream: two that do not depend on each other in one launch where their
+    sizes are for it (magi_attn_fwd_two).  Empties the list."""
+    if len(calls) == 2 and calls[0][0] == calls[1][0]:
+        _launch(calls[0][0], L.packed_pair("magi_attn_fwd_two").fn, calls[0][2], calls[1][2])
+    else:
+        for dev, fn, args, _ in calls:
+            _launch(dev, fn, args)
+    calls.clear()
 
 
 def qk_norm_score_bound(q_norm_bound: float, k_norm_bound: float, head_dim: int = 128,
@@ -560,9 +584,16 @@ def launch_small_layer(dev: torch.device, parts: int, *fields) -> None:
     _launch_packed(dev, "magi_small_layer", L.SmallLayerArgs, parts, *fields)
 
 
-def split_memory(dev: torch.device, Hq: int, Hkv: int, n: int, max_seqlen_q: int, max_seqlen_k: int):
-    """(the scratch memory that a bf16 call with bounded scores makes use of or None, its address, its bytes)"""
-    size = _bounded_split_bytes(Hq, Hkv, n, max_seqlen_q, max_seqlen_k) if max_seqlen_k >= 512 else 0
+def attention_waves(Hq: int, Hkv: int, n: int, mode: int, max_seqlen_q: int, max_seqlen_k: int) -> int:
+    """The wavefronts that share a row's keys where range_attention(share_waves=True) with a bound in force does not take another form; else 0."""
+    return L.lib().magi_attn_waves(Hq, Hkv, max(n, 0), mode, int(max_seqlen_q), int(max_seqlen_k))
+
+
+def split_memory(dev: torch.device, Hq: int, Hkv: int, n: int, mode: int, max_seqlen_q: int, max_seqlen_k: int):
+    """(the scratch memory that a bf16 call with bounded scores and MAGI_ATTN_SHARE_WAVES makes use of or None, its address, its bytes)"""
+    size = 0
+    if max_seqlen_k >= 512 and not attention_waves(Hq, Hkv, n, mode, max_seqlen_q, max_seqlen_k):
+        size = _bounded_split_bytes(Hq, Hkv, n, max_seqlen_q, max_seqlen_k)
     if not size:
         return None, 0, 0
     t = torch.empty(size, dtype=torch.uint8, device=dev)
@@ -582,9 +613,9 @@ def launch_text_attention(dev: torch.device, q: int, rows: int, Hq: int, kv: int
     bound <= MAGI_SCORE_BOUND_MAX).  clear: rows no range covers become zeros (the caller has cleared `out` unless covered_by_launch).
     Shares keys as range_attention does."""
     max_seqlen_q, max_seqlen_k = int(max_seqlen_q), int(max_seqlen_k)
-    split, split_at, split_bytes = split_memory(dev, Hq, Hkv, n, max_seqlen_q, max_seqlen_k)
+    split, split_at, split_bytes = split_memory(dev, Hq, Hkv, n, L.MAGI_RANGES_CU, max_seqlen_q, max_seqlen_k)
     cu_q, cu_k = cu_q.contiguous(), cu_k.contiguous()
-    flags = L.MAGI_ATTN_ZERO_UNCOVERED if clear and covered_by_launch(n, max_seqlen_q, rows) else 0
+    flags = L.MAGI_ATTN_SHARE_WAVES | (L.MAGI_ATTN_ZERO_UNCOVERED if clear and covered_by_launch(n, max_seqlen_q, rows) else 0)
     kv_row = Hkv * 256
     _launch_packed(
         dev, "magi_attn_fwd", L.AttnArgs, q, kv, kv + 256, 0, 0, out, 0, cu_q.data_ptr(), cu_k.data_ptr(), 0, 0, 0,

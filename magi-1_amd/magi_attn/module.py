@@ -37,6 +37,7 @@ from . import _lib as L
 from .cache import Fp8KVCache, OffloadedKVCache
 from .functional import (_measuring_a_bound_pays, covered_by_launch, launch_fp8_attention, launch_quantize_fp8_split,
                          launch_small_projections_e4m3, launch_text_attention, range_count, split_memory)
+from .functional import attention_waves, launch_held
 from .functional import launch_small_layer as launch_small_projections  # (named by the first of the launches it stands for)
 from .functional import (div_clamp_to, head_norm, layer_norm, layer_norm_div_clamp, pow2_scale_for, qk_prologue, qk_prologue_fp8, qkv_proj_prologue,
                          quantize_fp8_split,
@@ -800,18 +801,19 @@ class FullyParallelAttention(torch.nn.Module):
     def core_attention(self, query: torch.Tensor, key: torch.Tensor, value: torch.Tensor, bs: int,
                        meta_args: ModelMetaArgs, out: Optional[torch.Tensor] = None,
                        q_prescaled: bool = False, score_bound: float = 0.0, auto_bound: bool = False,
-                       split_keys: bool = False) -> torch.Tensor:
+                       split_keys: bool = False, held: Optional[list] = None) -> torch.Tensor:
         """query [(sq b), Hq, D], key / value [(sk b), Hkv, D] -> [(sq b), Hq, D]; dit_module.py:1023-1066.
         bs > 1 only occurs with one range per batch row (asserted there too).  `out` is a
         destination view, possibly in the grouped layout of range_attention (bs > 1: [sq, bs * groups, heads, D]).  q_prescaled: query carries
         softmax_scale * log2(e); score_bound, auto_bound: see range_attention.  split_keys: whether the keys of a row may
-        be shared among workgroups, the sums added in an order that depends on what else the launch holds; without it a
-        row's bits are those of full_attention on its range alone (with auto_bound, where the measured bound does not hold)."""
+        be shared among workgroups and wavefronts, the sums added in an order that depends on what else the launch holds; without it a
+        row's bits are those of full_attention on its range alone (with auto_bound, where the measured bound does not hold).  held (bs 1):
+        see range_attention."""
         p = meta_args.core_attn_params
         if bs == 1:
             out, _ = range_attention(query, key, value, p.q_range, p.k_range, p.max_seqlen_q, p.max_seqlen_k,
                                      out=out, return_lse=False, q_prescaled=q_prescaled, score_bound=score_bound,
-                                     auto_bound=auto_bound, split_keys=split_keys)
+                                     auto_bound=auto_bound, split_keys=split_keys, share_waves=split_keys, held=held)
             return out
         if meta_args.denoising_range_num > 1:
             raise ValueError("bs > 1 with several denoising ranges is not a layout the pipeline produces")
@@ -872,13 +874,14 @@ class FullyParallelAttention(torch.nn.Module):
 
     def _cross_attention_fused(self, qx_raw: torch.Tensor, sq: int, b: int, key_value_states: torch.Tensor,
                                cross_attn_params: PackedCrossAttnParams, out: Optional[torch.Tensor],
-                               bound: float, own_text: bool = False) -> Optional[torch.Tensor]:
+                               bound: float, own_text: bool = False, held: Optional[list] = None) -> Optional[torch.Tensor]:
         """Cross attention on the RAW qx projection [sq * b, Hq*D].  Batch 1: the attention kernel applies q_layernorm_xattn
         while it loads q (no normalised copy of q in memory) and, the scores of normed q and k being bounded, runs without a
         running maximum; returns None when that path does not apply (then the caller takes get_xqkv + cross_attention).
         Batch > 1: head norm and online softmax, the arithmetic of get_xqkv + cross_attention bit for bit, on the [position,
         batch] rows where they are (no copy to batch-major order and back: 230 MB each way at the 480p unconditional pass).
         own_text: the text's K | V rows come from small_projections where it takes the states (else the library's GEMM and a head norm).
+        held (batch 1): see range_attention.
         -> [sq, b, Hq, D] contiguous, or `out` (batch > 1: [sq, b, groups, heads, D])."""
         if b == 1 and not (0.0 < bound <= L.MAGI_SCORE_BOUND_MAX):
             return None
@@ -901,7 +904,7 @@ class FullyParallelAttention(torch.nn.Module):
             kx = head_norm(k_, gk, bk, self.eps)
         gq, bq = m["q_layernorm_xattn"].gamma_beta_fp32()
         if b == 1:
-            q_kw = {"score_bound": bound, "q_norm": (gq, bq, self.eps)}
+            q_kw = {"score_bound": bound, "q_norm": (gq, bq, self.eps), "share_waves": True, "held": held}
         else:
             q = head_norm(q, gq, bq, self.eps).view(sq, b, -1, D).transpose(0, 1)
             q_kw = {"score_bound": math.inf, "clear_out": True}
@@ -991,8 +994,8 @@ class FullyParallelAttention(torch.nn.Module):
 
     def _forward_small(self, hidden_states: torch.Tensor, key_value_states: torch.Tensor, inference_params: Optional[InferenceParams],
                        rope: torch.Tensor, meta_args: ModelMetaArgs, proj_layout: bool, bound_core: float, bound_cross: float):
-        """forward() of a small bf16 layer at batch 1 with both score bounds in force, whose projections are the library's own: three
-        launches (magi_small_projections, core attention, cross attention) with their arguments put together in one go.  None, before
+        """forward() of a small bf16 layer at batch 1 with both score bounds in force, whose projections are the library's own:
+        magi_small_projections, core attention and cross attention (in one launch where both are small) with their arguments put together in one go.  None, before
         anything is launched or written, where forward() goes on with the separate launches: other methods, projections or caches, larger
         layers, tensors of other types or layouts.  (The layer's cache and its side buffer may have been allocated by then, as forward() would.)
 
@@ -1051,7 +1054,8 @@ class FullyParallelAttention(torch.nn.Module):
                 new = kv + 2 * kv_row * start
             core_q, core_k, cross_q, cross_k = int(p.max_seqlen_q), int(p.max_seqlen_k), int(cp.max_seqlen_q), int(cp.max_seqlen_kv)
             zero = L.MAGI_ATTN_ZERO_UNCOVERED if clear else 0
-            core_split, cross_split = split_memory(dev, Hq, Hkv, core_n, core_q, core_k), split_memory(dev, Hq, Hkv, cross_n, cross_q, cross_k)
+            core_split = split_memory(dev, Hq, Hkv, core_n, L.MAGI_RANGES_PAIRS, core_q, core_k)
+            cross_split = split_memory(dev, Hq, Hkv, cross_n, L.MAGI_RANGES_CU, cross_q, cross_k)
             ranges = [t.contiguous() for t in (p.q_range, p.k_range, cp.cu_seqlens_q, cp.cu_seqlens_kv)]
             fields = (
                 hidden_states.data_ptr(), w.data_ptr(), lw.data_ptr(), lb.data_ptr(), rope.data_ptr(), gq.data_ptr(), bq.data_ptr(), gk.data_ptr(),
@@ -1226,7 +1230,9 @@ class FullyParallelAttention(torch.nn.Module):
             own_text = (bs == 1 and key_value_states.dim() == 2 and hidden_states.is_cuda
                         and "_cross_attention_fused" not in self.__dict__ and type(self)._cross_attention_fused is _CROSS_FUSED
                         and _text_in_one_launch(flop, text_rows, heads, key_value_states.shape[1], _compute_units(hidden_states.device)))
-            more = {"own_text": True} if own_text else {}  # (one put in its place may not know it)
+            more = {"own_text": True} if own_text else {}  # (one put in its place may not know these)
+            if held is not None:
+                more["held"] = held
             return self._cross_attention_fused(qx_raw, sq, bs, key_value_states, meta_args.cross_attn_params, dst, bound_cross, **more)
 
         get_xqkv = lambda m, y: self.get_xqkv(m, y, qx_raw=qx_raw.view(sq, bs, -1))
@@ -1234,6 +1240,14 @@ class FullyParallelAttention(torch.nn.Module):
         Hq = self.num_attention_heads
         fused = None
         core_dst = cross_dst = None
+        # core and text attention, which do not depend on each other, go into one launch behind the text's projection where both take the form for it
+        # (others are issued as soon as they can be: the device is not to wait for what the host does for the text)
+        held = None
+        if core_bounded and cross_bounded and self.attention_dtype == "bf16" and sq * Hq <= 32 * _compute_units(hidden_states.device) and _OWN_CROSS_FUSED.of(self):
+            cp, Hkv = meta_args.cross_attn_params, self.num_query_groups_per_partition
+            if attention_waves(Hq, Hkv, p.q_range.shape[0], L.MAGI_RANGES_PAIRS, p.max_seqlen_q, p.max_seqlen_k) and attention_waves(
+                    Hq, Hkv, cp.cu_seqlens_q.numel() - 1, L.MAGI_RANGES_CU, cp.max_seqlen_q, cp.max_seqlen_kv):
+                held = []
         if proj_layout and bs == 1 and Hq % PROJ_GROUPS == 0:
             # (rows that no q range / cu_seqlens segment covers are left as allocated: the pipeline's ranges cover
             # every row, dit_model.py:220-222, 246; bf16, what the launches write, whatever hidden_states is)
@@ -1256,8 +1270,10 @@ class FullyParallelAttention(torch.nn.Module):
             core = self._core_attention_fp8(raw, rope, inference_params, meta_args, use_cache, core_dst)
         elif not use_cache:
             q, kv, qx_raw = project()
+            if not _OWN_CORE.of(self):
+                held = None
             core = self.core_attention(q, *_halves(kv, kv.shape[0]), bs, meta_args, out=core_dst, q_prescaled=True,
-                                       split_keys=True, **core_bound_kw)
+                                       split_keys=True, **core_bound_kw, **({} if held is None else {"held": held}))
         else:
             if bs != 1 or inference_params.max_batch_size != 1:
                 raise ValueError("the cached path runs at batch 1 (as the reference pipeline does)")
@@ -1266,6 +1282,7 @@ class FullyParallelAttention(torch.nn.Module):
             S = sq
             offloaded = cache if isinstance(cache, OffloadedKVCache) else None
             if offloaded is not None:  # kv_offload: the prefix comes through a device staging buffer
+                held = None
                 cache = offloaded.stage(start)
             if inference_params.update_kv_cache:
                 n_keep = S - meta_args.clip_token_nums if meta_args.distill_nearly_clean_chunk else S
@@ -1283,12 +1300,12 @@ class FullyParallelAttention(torch.nn.Module):
                 kc, vc = _halves(cache, split)
                 if tail is None:
                     core, _ = range_attention(q, kc, vc, p.q_range, p.k_range, p.max_seqlen_q, p.max_seqlen_k,
-                                              out=core_dst, return_lse=False, q_prescaled=True, **core_bound_kw)
+                                              out=core_dst, return_lse=False, q_prescaled=True, share_waves=True, held=held, **core_bound_kw)
                 else:
                     k2, v2 = _halves(tail, tail.shape[0])
                     core, _ = range_attention(q, kc, vc, p.q_range, p.k_range, p.max_seqlen_q, p.max_seqlen_k,
                                               k2=k2, v2=v2, k_split=split, out=core_dst,
-                                              return_lse=False, q_prescaled=True, **core_bound_kw)
+                                              return_lse=False, q_prescaled=True, share_waves=True, held=held, **core_bound_kw)
                 persisted = n_keep
             finally:
                 if offloaded is not None:  # the persisted rows go back to the host behind the attention launch
@@ -1296,9 +1313,13 @@ class FullyParallelAttention(torch.nn.Module):
         if fused is not None:
             if cross_fused(cross_dst) is None:
                 self.cross_attention(mixed_qqkv, key_value_states, meta_args.cross_attn_params, get_xqkv, out=cross_dst)
+            if held is not None:
+                launch_held(held)
             return fused
         core_attn_out = core.view(sq, bs, -1)
         xo = cross_fused(None)
+        if held is not None:
+            launch_held(held)
         if xo is not None:
             xattn_out = xo.reshape(sq, bs, -1)
         else:
@@ -1315,6 +1336,8 @@ _OWN_PROJECTIONS = _Own(CustomLayerNormLinear, "forward_ln", "forward_qkvx")
 _OWN_SMALL_PROJECTIONS = _Own(CustomLayerNormLinear, "forward_ln", "forward_qkvx", "forward_ln_qkvx_rows", "_split", "fused_weight")
 _OWN_CROSS = _Own(FullyParallelAttention, "get_xqkv", "cross_attention")
 _CROSS_FUSED = FullyParallelAttention._cross_attention_fused
+_OWN_CROSS_FUSED = _Own(FullyParallelAttention, "_cross_attention_fused")
+_OWN_CORE = _Own(FullyParallelAttention, "core_attention")
 _OWN_SMALL = _Own(FullyParallelAttention, "_project_rows", "_fused_qkv", "_cross_attention_fused")
 _OWN_SMALL_UNCACHED = _Own(FullyParallelAttention, "_project_rows", "_fused_qkv", "_cross_attention_fused", "core_attention")
 _OWN_SMALL_FP8 = _Own(FullyParallelAttention, "_project_rows", "_core_attention_fp8", "_cross_attention_fused")
