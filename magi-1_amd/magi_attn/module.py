@@ -215,7 +215,7 @@ def _rows_ahead_e4m3(rows: int, cols: int, depth: int, cus: int) -> int:
     depth 3072: 21600 rows 61 / 65, 28080 67 / 71; behind rounds that end within a row of tiles, 6144 columns: 14155 rows 362 / 469).  The
     same bits in all of them."""
     tiles = cols // 256
-    if cols % 256 or not 0 < tiles <= cus or depth < 1024:
+    if rows * cols < 65536 * cus or cols % 256 or not 0 < tiles <= cus or depth < 1024:  # (less than one round, ...)
         return 0
     whole = 256 * (cus // math.gcd(cus, tiles))
     head = rows // whole * whole
@@ -335,11 +335,9 @@ class PerTensorQuantizedFp8Linear(torch.nn.Module):
         """The GEMM alone, on an input that is already div_clamp_to(input, self.input_scale)."""
         x2 = x8 if x8.dim() == 2 else x8.reshape(-1, self.in_features)
         w, scale_a, scale_b = _param(self, "weight"), _param(self, "input_scale").reshape(-1)[:1], _param(self, "weight_scale").reshape(-1)[:1]
-        head = 0
-        if (type(x2) in _PLAIN and type(w) in _PLAIN and x2.is_cuda and x2.is_contiguous()
-                and not (torch.is_grad_enabled() and any(t.requires_grad for t in (x2, w, scale_a, scale_b)))):
-            head = _rows_ahead_e4m3(x2.shape[0], self.out_features, self.in_features, _compute_units(x2.device))
-        if head:
+        head = _rows_ahead_e4m3(x2.shape[0], self.out_features, self.in_features, _compute_units(x2.device)) if x2.is_cuda else 0
+        if head and (type(x2) in _PLAIN and type(w) in _PLAIN and x2.is_contiguous()
+                     and not (torch.is_grad_enabled() and any(t.requires_grad for t in (x2, w, scale_a, scale_b)))):
             y = torch.empty((x2.shape[0], self.out_features), dtype=self.output_dtype, device=x2.device)
             for rows in (slice(0, head), slice(head, None)):
                 torch._scaled_mm(x2[rows], w[0].t(), scale_a=scale_a, scale_b=scale_b, out_dtype=self.output_dtype, out=y[rows])
