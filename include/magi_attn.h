@@ -271,8 +271,9 @@ int32_t magi_attn_waves(int32_t Hq, int32_t Hkv, int32_t n_ranges, int32_t range
 int magi_attn_fwd(const magi_attn_args* args, void* stream);
 
 /* magi_attn_fwd of two calls that do not depend on each other and write different outputs (a layer's core and text attention): in one
- * launch where both take the form of MAGI_ATTN_SHARE_WAVES, else one after the other; the same bits as two calls.  A refusal of the
- * second is this call's, the first has been launched by then. */
+ * launch where both take the form of MAGI_ATTN_SHARE_WAVES, or both 256 rows per workgroup (magi_attn_tile_rows) with q pre-scaled or raw,
+ * a score_bound and no keys of the second shared; else one after the other.  The same bits as two calls.  A refusal of the second is this
+ * call's, the first has been launched by then. */
 int magi_attn_fwd_two(const magi_attn_args* first, const magi_attn_args* second, void* stream);
 
 /*

@@ -398,11 +398,11 @@ int waves_plan(int Hq, int Hkv, int n_ranges, int ranges_mode, int max_seqlen_q,
   return max_seqlen_k <= 4096 ? 4 : 0;
 }
 
-// held: where the call takes the form that may share a launch with another, its arguments instead of the launch; HELD is returned then
+// held: where the call takes a form that may share a launch with another, its arguments instead of the launch; HELD is returned then
 constexpr int HELD = 1;
 int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace, magi::AttnKernArgs* held = nullptr);
-// one or two held calls in one launch
-int launch_held(const magi::AttnPairArgs& pair, void* stream);
+// a held call by itself
+int launch_held(const magi::AttnKernArgs& a, void* stream);
 int attn_fwd_two(const magi_attn_args* first, const magi_attn_args* second, void* stream);
 
 // the caller's struct as this version lays it out: itself, or `full` filled from the shorter one of version 103
@@ -498,23 +498,34 @@ int magi_attn_fwd_static_scratch(const magi_attn_args* p, void* stream) {
 
 namespace {
 
-int launch_held(const magi::AttnPairArgs& pair, void* stream) {
-  const hipError_t e = magi::launch_attn_fwd_bf16_waves(pair, static_cast<hipStream_t>(stream));
+// Held calls: 32 rows to a workgroup, whose wavefronts share keys; or 256 rows of q as it is or raw.  count of them, in one launch.
+int launch_held(magi::AttnPairArgs& pair, int count, void* stream) {
+  const hipStream_t st = static_cast<hipStream_t>(stream);
+  const magi::AttnKernArgs& a = pair.job[0];
+  if (count == 1) pair.job[1].per_xcd = 0;
+  const hipError_t e = a.block_m == 32 ? magi::launch_attn_fwd_bf16_waves(pair, st)
+                       : count == 2    ? magi::launch_attn_fwd_bf16_x16_pair(pair, st)
+                                       : magi::launch_attn_fwd_bf16_x16(a, st);
   if (e != hipSuccess) return hip_fail(e, "magi_attn_fwd launch");
-  count_launches(1);
+  count_launches(1 + (a.block_m != 32 && a.split_from < a.per_xcd));
   return MAGI_OK;
+}
+int launch_held(const magi::AttnKernArgs& a, void* stream) {
+  magi::AttnPairArgs pair;
+  pair.job[0] = a;
+  return launch_held(pair, 1, stream);
 }
 
 // first, then second, which do not depend on each other: in one launch where both take the form for it
 int attn_fwd_two(const magi_attn_args* first, const magi_attn_args* second, void* stream) {
   magi::AttnPairArgs pair;
   const int one = attn_fwd_impl(first, stream, first->workspace, &pair.job[0]);
-  if (one < 0) return one;
-  const int two = attn_fwd_impl(second, stream, second->workspace, &pair.job[one == HELD ? 1 : 0]);
-  if (one != HELD && two != HELD) return two;
-  if ((one == HELD) != (two == HELD)) pair.job[1].per_xcd = 0;
-  const int rc = launch_held(pair, stream);
-  return two < 0 ? two : rc;
+  if (one != HELD) return one < 0 ? one : attn_fwd_impl(second, stream, second->workspace);
+  const int two = attn_fwd_impl(second, stream, second->workspace, &pair.job[1]);
+  const magi::AttnKernArgs &a = pair.job[0], &b = pair.job[1];
+  if (two == HELD && a.block_m == b.block_m && (b.block_m == 32 || b.split_from >= b.per_xcd)) return launch_held(pair, 2, stream);
+  const int rc = launch_held(a, stream);
+  return rc < 0 ? rc : two == HELD ? launch_held(b, stream) : two;
 }
 
 int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace, magi::AttnKernArgs* held) {
@@ -743,14 +754,9 @@ int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace, magi:
     };
     a.share_pieces = 1;
     if (a.waves) {
-      magi::AttnPairArgs pair;
-      if (held) {
-        *held = a;
-        return HELD;
-      }
-      pair.job[0] = a;
-      pair.job[1].per_xcd = 0;
-      return launch_held(pair, stream);
+      if (!held) return launch_held(a, stream);
+      *held = a;
+      return HELD;
     }
     if (r32.use) pieces(r32.share);
     if ((fp8 || (bounded && a.block_m == 256 && !mfma32)) && split_bytes > 0) {
@@ -772,6 +778,11 @@ int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace, magi:
     if (online128 && !a.gate && split_bytes > 0) {
       const SharePlan s = share_plan(a.per_xcd, p->n_ranges, p->max_seqlen_q, p->max_seqlen_k);
       if (s.bytes(a.per_xcd) <= split_bytes) pieces(s);
+    }
+    // (of the other forms the one of large launches: in the smaller ones the core's rows or keys are dealt out over the whole chip as it is)
+    if (held && bounded && a.block_m == 256 && !checked && !mfma32 && !auto_bound && !scale_q) {
+      *held = a;
+      return HELD;
     }
     hipError_t e;
     if (p->dtype != MAGI_DTYPE_BF16)

@@ -84,11 +84,14 @@ hipError_t launch_attn_fwd_bf16_r32(const AttnKernArgs& a, hipStream_t stream);
 // One or two calls (job[1].per_xcd = 0: one), bounded scores, block_m 32: the wavefronts of a workgroup share the keys of 32 rows
 struct AttnPairArgs {
   AttnKernArgs job[2];
+  unsigned ahead;  // attn_fwd_bf16_x16.hip: workgroups of the first per XCD
 };
 hipError_t launch_attn_fwd_bf16_waves(const AttnPairArgs& p, hipStream_t stream);
 hipError_t launch_attn_fwd_bf16_w64(const AttnKernArgs& a, hipStream_t stream);
 // (with items to split: and behind it the launch that adds their pieces up)
 hipError_t launch_attn_fwd_bf16_x16(const AttnKernArgs& a, hipStream_t stream);
+// two such calls in 256-row workgroups, the second without items to split, q as it is or raw
+hipError_t launch_attn_fwd_bf16_x16_pair(const AttnPairArgs& p, hipStream_t stream);
 // the bounded-score kernel without a promise, and behind it the launch that repeats what it could not be trusted with
 hipError_t launch_attn_fwd_bf16_checked(const AttnKernArgs& a, int compute_units, hipStream_t stream);
 hipError_t launch_attn_fwd_fp8(const AttnKernArgs& a, hipStream_t stream);

@@ -1,5 +1,5 @@
-"""Bounded scores in launches of a few rows: the wavefronts of a workgroup share the keys of 32 rows (MAGI_ATTN_SHARE_WAVES), one call or two
-(magi_attn_fwd_two)."""
+"""Bounded scores in launches of a few rows: the wavefronts of a workgroup share the keys of 32 rows (MAGI_ATTN_SHARE_WAVES); two calls in one
+launch (magi_attn_fwd_two), in this form or in 256-row workgroups."""
 import pytest
 import torch
 
@@ -81,6 +81,40 @@ def test_two_calls_have_the_bits_of_each(dev, first, second, launches):
     assert not held and (M.lib().magi_launch_count() - n0 == launches or torch.cuda.get_device_properties(dev).multi_processor_count != 256)
     for (a, la), (b, lb) in zip(got, want):
         assert torch.equal(a, b) and torch.equal(la, lb)
+
+
+# 256 rows to a workgroup in both: whole items; the last round's keys shared in the first (a launch more, for the sums), in the second (two calls);
+# ranges without keys, rows in no range, two key segments; q as it is, raw or (no form for two) unscaled; the smaller one ahead; both orders of q's kinds
+@pytest.mark.parametrize("first,second,modes,launches", [
+    ((24, 8, [(0, 4200)], [(0, 700)], 4200), (24, 8, [(0, 4190)], [(0, 70)], 4190), ("as it is", "normed"), 1),
+    ((24, 8, [(0, 4200)], [(0, 700)], 4201, 130), (24, 8, [(5, 4190)], [(3, 70)], 4195), ("normed", "as it is"), 1),
+    ((24, 8, [(0, 3000), (3000, 6000)], [(0, 1500), (0, 3000)], 6000), (24, 8, [(0, 3000), (3000, 6001)], [(0, 1), (9, 9)], 6003), ("as it is", "normed"), 2),
+    ((4, 1, [(0, 20000)], [(0, 300)], 20000), (24, 8, [(0, 3000), (3000, 6000)], [(0, 1500), (0, 3000)], 6000), ("normed", "as it is"), 3),
+    ((24, 8, [(0, 4200)], [(0, 700)], 4200), (24, 8, [(0, 4190)], [(0, 70)], 4190), ("scaled", "normed"), 2),
+    ((24, 8, [(0, 4200)], [(0, 700)], 4200), (24, 8, [(0, 4190)], [(0, 70)], 4190), ("as it is", "scaled"), 2),
+    ((24, 8, [(0, 4200)], [(0, 700)], 4200), (6, 2, [(0, 300)], [(0, 70)], 300), ("as it is", "normed"), 2)])
+def test_two_large_calls_have_the_bits_of_each(dev, first, second, modes, launches):
+    calls = [_case(dev, *c, mode=m)[0] for c, m in zip((first, second), modes)]
+    want = [call() for call in calls]
+    held = []
+    got = [call(held=held) for call in calls]
+    n0 = M.lib().magi_launch_count()
+    F.launch_held(held)
+    assert M.lib().magi_launch_count() - n0 == launches or torch.cuda.get_device_properties(dev).multi_processor_count != 256
+    for (a, la), (b, lb) in zip(got, want):
+        assert torch.equal(a, b) and torch.equal(la, lb)
+    del want
+    graph, held = torch.cuda.CUDAGraph(), []
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        again = [call(return_lse=False, held=held)[0] for call in calls]
+        F.launch_held(held)
+    for _ in range(3):
+        for t in again:
+            t.fill_(7.0)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, (b, _) in zip(again, got))
 
 
 def test_a_refused_second_call_raises_and_the_first_has_run(dev):
