@@ -102,7 +102,8 @@ extern "C" {
  * another size returns MAGI_EINVAL instead of reading fields the caller never wrote.
  * 105: the structs of 104; new are MAGI_ATTN_ROW_BITS (a library of 104 would ignore it), magi_attn_split_bytes_256,
  * magi_attn_pieces_bytes, magi_small_projections_e4m3 and magi_small_layer.
- * 106: the structs of 105; new are MAGI_ATTN_SHARE_WAVES, magi_attn_waves and magi_attn_fwd_two. */
+ * 106: the structs of 105; new are MAGI_ATTN_SHARE_WAVES, magi_attn_waves and magi_attn_fwd_two.
+ * 107: the structs of 106; new are magi_qk_prologue_row_max and magi_quantize_fp8_row_max. */
 int magi_version(void);
 const char* magi_last_error(void);
 /* Diagnostics: the number of kernel launches the library has issued in this process so far (all threads, all
@@ -342,6 +343,9 @@ typedef struct magi_prologue_args {
 } magi_prologue_args;
 
 int magi_qk_prologue(const magi_prologue_args* args, void* stream);
+/* The same with e4m3 outputs, and v_row_max [Hkv, S] (2 bytes each) receives the largest magnitude of each row of v_raw as the bits of that
+ * bf16 number, which is what magi_quantize_fp8_row_max takes its scales from. */
+int magi_qk_prologue_row_max(const magi_prologue_args* args, void* v_row_max, void* stream);
 
 /*
  * The four projections of the attention layer and the prologue in one launch: a bf16 GEMM
@@ -583,6 +587,8 @@ typedef struct magi_quantize_args {
 } magi_quantize_args;
 
 int magi_quantize_fp8_split(const magi_quantize_args* args, void* stream);
+/* The same bytes and scales, the absmax of a group from row_max [H, T] (see magi_qk_prologue_row_max) instead of a pass over its rows. */
+int magi_quantize_fp8_row_max(const magi_quantize_args* args, const void* row_max, void* stream);
 
 #ifdef __cplusplus
 }

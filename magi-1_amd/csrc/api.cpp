@@ -419,7 +419,7 @@ const magi_attn_args* current_layout(const magi_attn_args* p, magi_attn_args* fu
 
 extern "C" {
 
-int magi_version(void) { return 106; }
+int magi_version(void) { return 107; }
 
 uint64_t magi_launch_count(void) { return g_launches.load(std::memory_order_relaxed); }
 
@@ -936,9 +936,7 @@ int small_projections_impl(const magi_small_proj_args* p, const SmallProjE4m3* e
 
 }  // namespace
 
-extern "C" {
-
-int magi_qk_prologue(const magi_prologue_args* p, void* stream) {
+static int prologue_impl(const magi_prologue_args* p, void* v_row_max, void* stream) {
   if (!p) return fail(MAGI_EINVAL, "magi_qk_prologue: args is NULL");
   MAGI_CHECK_LAYOUT("magi_qk_prologue", p);
   if (p->D != 128) return fail(MAGI_ENOSYS, "magi_qk_prologue: head_dim %d not implemented (128 only)", p->D);
@@ -967,7 +965,7 @@ int magi_qk_prologue(const magi_prologue_args* p, void* stream) {
   if (p->q_raw_stride_t % 8 || p->k_raw_stride_t % 8 || p->v_raw_stride_t % 8 || p->kv_stride_t % 8 ||
       p->kv_tail_stride_t % 8)
     return fail(MAGI_EINVAL, "magi_qk_prologue: strides must keep rows 16-byte aligned");
-  if (!aligned16(p->q_raw) || !aligned16(p->k_raw) || (!out8 && !aligned16(p->v_raw)) || !aligned16(p->q_out) ||
+  if (!aligned16(p->q_raw) || !aligned16(p->k_raw) || ((!out8 || v_row_max) && !aligned16(p->v_raw)) || !aligned16(p->q_out) ||
       !aligned16(p->kv_out) || !aligned16(p->kv_tail))
     return fail(MAGI_EINVAL, "magi_qk_prologue: buffers must be 16-byte aligned");
 
@@ -1003,10 +1001,23 @@ int magi_qk_prologue(const magi_prologue_args* p, void* stream) {
   if (!(p->q_premul == p->q_premul) || std::fabs(p->q_premul) > 1e30f)
     return fail(MAGI_EINVAL, "magi_qk_prologue: q_premul is not finite");
   a.q_premul = p->q_premul == 0.f ? 1.f : p->q_premul;
+  a.v_row_max = static_cast<unsigned short*>(v_row_max);
   hipError_t e = magi::launch_prologue(a, static_cast<hipStream_t>(stream));
   if (e != hipSuccess) return hip_fail(e, "magi_qk_prologue launch");
   count_launches(1);
   return MAGI_OK;
+}
+
+extern "C" {
+
+int magi_qk_prologue(const magi_prologue_args* p, void* stream) { return prologue_impl(p, nullptr, stream); }
+
+int magi_qk_prologue_row_max(const magi_prologue_args* p, void* v_row_max, void* stream) {
+  if (p && p->struct_size == sizeof(*p) && p->S > 0 && p->Hkv > 0) {  // (the rest is prologue_impl's to refuse)
+    if (p->out_dtype != MAGI_DTYPE_FP8_E4M3) return fail(MAGI_EINVAL, "magi_qk_prologue_row_max: e4m3 outputs only");
+    if (!p->v_raw || !v_row_max) return fail(MAGI_EINVAL, "magi_qk_prologue_row_max: NULL v_raw/v_row_max");
+  }
+  return prologue_impl(p, v_row_max, stream);
 }
 
 int magi_qkv_proj_prologue(const magi_qkv_proj_args* p, void* stream) {
@@ -1295,7 +1306,7 @@ int magi_apply_rotary(const void* x, const float* cos, const float* sin, void* y
   return MAGI_OK;
 }
 
-static int quantize_impl(const magi_quantize_args* p, void* stream, bool always_one_launch) {
+static int quantize_impl(const magi_quantize_args* p, void* stream, bool always_one_launch, const void* row_max = nullptr) {
   if (!p) return fail(MAGI_EINVAL, "magi_quantize_fp8: args is NULL");
   MAGI_CHECK_LAYOUT("magi_quantize_fp8", p);
   if (p->D != 128) return fail(MAGI_ENOSYS, "magi_quantize_fp8: head_dim %d not implemented (128 only)", p->D);
@@ -1314,6 +1325,16 @@ static int quantize_impl(const magi_quantize_args* p, void* stream, bool always_
     return fail(MAGI_EINVAL, "magi_quantize_fp8: y2 / scales2 needed for rows >= n_rows_first");
   if (p->x_stride_t % 8 || p->x_stride_h % 8 || !aligned16(p->x) || !aligned16(p->y) || !aligned16(p->y2))
     return fail(MAGI_EINVAL, "magi_quantize_fp8: rows must be 16-byte aligned");
+  if (row_max) {
+    hipError_t e = magi::launch_quantize_fp8_row_max(static_cast<const char*>(p->x), p->x_stride_t * 2, p->x_stride_h * 2,
+                                                     static_cast<char*>(p->y), p->scales, p->T, p->H, p->chunk_tokens, p->premul,
+                                                     p->pow2_scales, p->n_rows_first, static_cast<char*>(p->y2), p->scales2,
+                                                     static_cast<const unsigned short*>(row_max), compute_units(),
+                                                     static_cast<hipStream_t>(stream));
+    if (e != hipSuccess) return hip_fail(e, "magi_quantize_fp8_row_max launch");
+    count_launches(1);
+    return MAGI_OK;
+  }
   int n_launches = 0;
   hipError_t e = magi::launch_quantize_fp8(static_cast<const char*>(p->x), p->x_stride_t * 2, p->x_stride_h * 2,
                                            static_cast<char*>(p->y), p->scales, p->T, p->H, p->chunk_tokens, p->premul,
@@ -1325,6 +1346,11 @@ static int quantize_impl(const magi_quantize_args* p, void* stream, bool always_
 }
 
 int magi_quantize_fp8_split(const magi_quantize_args* p, void* stream) { return quantize_impl(p, stream, true); }
+
+int magi_quantize_fp8_row_max(const magi_quantize_args* p, const void* row_max, void* stream) {
+  if (!row_max) return fail(MAGI_EINVAL, "magi_quantize_fp8_row_max: NULL row_max");
+  return quantize_impl(p, stream, true, row_max);
+}
 
 int magi_quantize_fp8(const void* x, int64_t x_stride_t, int64_t x_stride_h, void* y, float* scales, int32_t T,
                       int32_t H, int32_t D, int32_t chunk_tokens, float premul, int32_t pow2_scales, void* stream) {

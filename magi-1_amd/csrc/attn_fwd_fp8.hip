@@ -672,6 +672,52 @@ __global__ __launch_bounds__(QT1) void quantize_groups_kernel(const char* x, lon
     *(u32x2*)(ycol + (long)t * H * 128) = quantize8(*(const u32x4*)(xcol + (long)t * xs_t), premul, sc);
 }
 
+// The quantiser with the largest magnitude of each row in hand (row_max [H, T], bf16 bits): a workgroup takes its group's scale from two
+// bytes per row and quantises its slice, whose first rows are requested ahead of that.  Bound by HBM, below some thousand
+// rows by two trips to memory.  Out of memory, a pass over the rows first / this: [9360, 8] in one group per head 46 / 11 us, [3000, 8] 13.5 / 7.3,
+// [37440, 8] in four 61 / 31, [86400, 8] in four 142 / 59 (4.5 TB/s); the prologue pays 5, 1, 16 and 13 us for the maxima.
+constexpr int UNK = 4;  // rows in flight per lane
+__global__ __launch_bounds__(QT1) void quantize_row_max_kernel(const char* x, long xs_t, long xs_h, char* y, float* scales, int T, int H,
+                                                               int chunk_tokens, float premul, int pow2, int n_first, char* y2,
+                                                               float* scales2, const unsigned short* row_max) {
+  __shared__ unsigned s_red[QT1 / 64];
+  const int h = blockIdx.x, c = blockIdx.y;
+  const int t_begin = c * chunk_tokens, t_end = (int)min((long)T, (long)t_begin + chunk_tokens);
+  const int per = (t_end - t_begin + (int)gridDim.z - 1) / (int)gridDim.z;  // rows of a workgroup's slice
+  const int s_begin = t_begin + (int)blockIdx.z * per, s_end = min(t_end, s_begin + per);
+  if (s_begin >= s_end) return;  // (never slice 0, which writes the scale)
+  const int lane16 = threadIdx.x & 15, sub = threadIdx.x >> 4;
+  const char* const xcol = x + (long)h * xs_h + lane16 * 16;
+  u32x4 v[UNK];
+  auto request = [&](int t) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < UNK; ++u) v[u] = *(const u32x4*)(xcol + (long)min(t + u * QROWS, s_end - 1) * xs_t);
+  };
+  request(s_begin + sub);
+  const unsigned short* const rm = row_max + (long)h * T;
+  unsigned m = 0u;
+#pragma unroll 8
+  for (int t = t_begin + (int)threadIdx.x; t < t_end; t += QT1) m = max(m, (unsigned)rm[t]);
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) m = max(m, (unsigned)__shfl_xor((int)m, o));
+  if ((threadIdx.x & 63) == 0) s_red[threadIdx.x >> 6] = m;
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < QT1 / 64; ++j) m = max(m, s_red[j]);
+  const float sc = scale_of_absmax(__builtin_bit_cast(float, m << 16), premul, pow2);
+  const bool second = t_begin >= n_first;
+  const int t_off = second ? n_first : 0;
+  if (threadIdx.x == 0 && blockIdx.z == 0) (second ? scales2 : scales)[(long)(c - t_off / chunk_tokens) * H + h] = sc;
+  char* const ycol = (second ? y2 : y) + (long)h * 128 + lane16 * 8 - (long)t_off * H * 128;
+  for (int t = s_begin + sub;; t += UNK * QROWS) {
+#pragma unroll
+    for (int u = 0; u < UNK; ++u)
+      if (t + u * QROWS < s_end) *(u32x2*)(ycol + (long)(t + u * QROWS) * H * 128) = quantize8(v[u], premul, sc);
+    if (t + UNK * QROWS >= s_end) break;
+    request(t + UNK * QROWS);
+  }
+}
+
 }  // namespace
 
 hipError_t launch_attn_fwd_fp8(const AttnKernArgs& a, hipStream_t stream) {
@@ -727,6 +773,20 @@ hipError_t launch_quantize_fp8(const char* x, long x_stride_t, long x_stride_h, 
   hipLaunchKernelGGL(quantize_kernel, dim3((unsigned)((threads + QT - 1) / QT)), dim3(QT), 0, stream, x, x_stride_t,
                      x_stride_h, y, scales, T, H, chunk_tokens, premul);
   *n_launches = 4;
+  return hipGetLastError();
+}
+
+hipError_t launch_quantize_fp8_row_max(const char* x, long x_stride_t, long x_stride_h, char* y, float* scales, int T, int H,
+                                       int chunk_tokens, float premul, int pow2_scales, int n_first, char* y2, float* scales2,
+                                       const unsigned short* row_max, int compute_units, hipStream_t stream) {
+  if (T <= 0 || H <= 0) return hipSuccess;
+  const int n_chunks = (int)(((long)T + chunk_tokens - 1) / chunk_tokens);
+  if (n_chunks > 65535) return hipErrorInvalidValue;
+  // two workgroups per CU over the launch, each slice at least one pass long
+  const long n = (long)n_chunks * H;
+  const int share = (int)max(1L, min((2L * compute_units + n - 1) / n, (long)min(chunk_tokens, T) / QROWS));
+  hipLaunchKernelGGL(quantize_row_max_kernel, dim3(H, n_chunks, share), dim3(QT1), 0, stream, x, x_stride_t, x_stride_h, y, scales, T,
+                     H, chunk_tokens, premul, pow2_scales, n_first, y2, scales2, row_max);
   return hipGetLastError();
 }
 

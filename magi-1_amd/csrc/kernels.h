@@ -124,6 +124,7 @@ struct PrologueKernArgs {
   float q_premul;  // factor on q before the bf16 rounding (1 = none)
   int out_fp8;     // q and k leave as e4m3 (kv_out / kv_tail then hold K rows only, strides in bytes); v untouched
   float q_inv_scale, k_inv_scale;  // out_fp8: 1 / the constant scale of q (after q_premul) and of k
+  unsigned short* v_row_max;       // out_fp8, or nullptr: [Hkv, S] receives the largest magnitude of each row of v, as bf16 bits
 };
 hipError_t launch_prologue(const PrologueKernArgs& a, hipStream_t stream);
 
@@ -216,5 +217,9 @@ hipError_t launch_rotary(const void* x, const float* cos, const float* sin, void
 hipError_t launch_quantize_fp8(const char* x, long x_stride_t, long x_stride_h, char* y, float* scales, int T, int H,
                                int chunk_tokens, float premul, int pow2_scales, int n_first, char* y2, float* scales2,
                                bool one_launch, int compute_units, hipStream_t stream, int* n_launches);
+// The same with the largest magnitude of each row in hand: row_max [H, T], bf16 bits
+hipError_t launch_quantize_fp8_row_max(const char* x, long x_stride_t, long x_stride_h, char* y, float* scales, int T, int H,
+                                       int chunk_tokens, float premul, int pow2_scales, int n_first, char* y2, float* scales2,
+                                       const unsigned short* row_max, int compute_units, hipStream_t stream);
 
 }  // namespace magi

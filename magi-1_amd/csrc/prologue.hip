@@ -18,7 +18,9 @@ constexpr int THREADS = 256;
 constexpr int GROUPS = THREADS / 8;  // rows in flight per workgroup
 
 // TPB: tokens that share a workgroup (1, 2, 4 or 8).  OUT8: q and k leave as e4m3 bytes (q_out [S, Hq, D],
-// K rows [*, Hkv, D] at kv_out / kv_tail), each multiplied by its constant inverse scale; v is not touched.
+// K rows [*, Hkv, D] at kv_out / kv_tail), each multiplied by its constant inverse scale; v is not touched, but for the largest
+// magnitude of each of its rows where a.v_row_max asks for them: its quantiser then finds a group's scale in two bytes per row
+// ([9360, 24 + 8 heads], out of memory: 32 -> 37 us here, 46 -> 11 there).
 template <int TPB, bool OUT8>
 __global__ __launch_bounds__(THREADS) void prologue_kernel(const PrologueKernArgs a) {
   __shared__ float s_par[4][D];  // gq, bq, gk, bk
@@ -45,7 +47,7 @@ __global__ __launch_bounds__(THREADS) void prologue_kernel(const PrologueKernArg
   const bool rot_lane = j < nr;
   const int ea = rot_lane ? 8 * j : 2 * a.R2 + 16 * (j - nr);  // first element of vector A
   const int eb = rot_lane ? a.R2 + 8 * j : ea + 8;             // first element of vector B
-  const int U = a.Hq + (OUT8 ? 1 : 2) * a.Hkv;
+  const int U = a.Hq + (OUT8 && !a.v_row_max ? 1 : 2) * a.Hkv;
   constexpr int ES = OUT8 ? 1 : 2;  // bytes per output element
 
   const int s = blockIdx.x * TPB + team;
@@ -114,7 +116,21 @@ __global__ __launch_bounds__(THREADS) void prologue_kernel(const PrologueKernArg
       va_n = *(const u32x4*)(src_n + ea * 2);
       vb_n = *(const u32x4*)(src_n + eb * 2);
     }
-    if (kind == 2) {
+    if (OUT8 && kind == 2) {
+      // (two magnitudes per word, which order like unsigned 16-bit integers, a NaN above all)
+      typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+      u16x2 mp = {0, 0};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        mp = __builtin_elementwise_max(mp, __builtin_bit_cast(u16x2, va[i] & 0x7fff7fffu));
+        mp = __builtin_elementwise_max(mp, __builtin_bit_cast(u16x2, vb[i] & 0x7fff7fffu));
+      }
+      unsigned m = max(mp[0], mp[1]);
+      m = max(m, (unsigned)__shfl_xor((int)m, 1));
+      m = max(m, (unsigned)__shfl_xor((int)m, 2));
+      m = max(m, (unsigned)__shfl_xor((int)m, 4));
+      if (j == 0) a.v_row_max[(long)(u - a.Hq - a.Hkv) * a.S + sc] = (unsigned short)m;
+    } else if (kind == 2) {
       *(u32x4*)(dst + ea * 2) = va;
       *(u32x4*)(dst + eb * 2) = vb;
     } else {
@@ -586,7 +602,7 @@ hipError_t launch_div_clamp(const char* x, long x_stride, const float* scale, in
 hipError_t launch_prologue(const PrologueKernArgs& a_in, hipStream_t stream) {
   if (a_in.S <= 0) return hipSuccess;
   const PrologueKernArgs& a = a_in;
-  const int rows = a.Hq + (a.out_fp8 ? 1 : 2) * a.Hkv;
+  const int rows = a.Hq + (a.out_fp8 && !a.v_row_max ? 1 : 2) * a.Hkv;
   int tpb = 1;
   while (tpb < 8 && 2 * tpb * rows <= GROUPS) tpb *= 2;
   const dim3 grid((unsigned)((a.S + tpb - 1) / tpb)), block(THREADS);

@@ -145,12 +145,12 @@ class SmallLayerArgs(_SizedStructure):
     ]
 
 
-ABI_VERSION = 106  # magi_version() of the library these mirrors were written for
+ABI_VERSION = 107  # magi_version() of the library these mirrors were written for
 
 EXPORTS = ("magi_version", "magi_last_error", "magi_launch_count", "magi_attn_fwd", "magi_attn_fwd_two", "magi_attn_waves", "magi_attn_fwd_static_scratch",
            "magi_attn_split_bytes", "magi_attn_split_bytes_256", "magi_attn_pieces_bytes", "magi_attn_tile_rows",
-           "magi_qk_prologue", "magi_head_norm",
-           "magi_apply_rotary", "magi_quantize_fp8", "magi_quantize_fp8_split", "magi_layer_norm", "magi_qkv_proj_prologue", "magi_div_clamp_to_e4m3",
+           "magi_qk_prologue", "magi_qk_prologue_row_max", "magi_head_norm",
+           "magi_apply_rotary", "magi_quantize_fp8", "magi_quantize_fp8_split", "magi_quantize_fp8_row_max", "magi_layer_norm", "magi_qkv_proj_prologue", "magi_div_clamp_to_e4m3",
            "magi_layer_norm_e4m3", "magi_small_projections", "magi_small_projections_e4m3",
            "magi_small_layer")
 
@@ -193,6 +193,8 @@ def lib() -> C.CDLL:
         l.magi_attn_fwd_static_scratch.restype = C.c_int
         l.magi_qk_prologue.argtypes = [C.POINTER(PrologueArgs), C.c_void_p]
         l.magi_qk_prologue.restype = C.c_int
+        l.magi_qk_prologue_row_max.argtypes = [C.POINTER(PrologueArgs), C.c_void_p, C.c_void_p]
+        l.magi_qk_prologue_row_max.restype = C.c_int
         l.magi_head_norm.argtypes = [C.c_void_p, C.c_int64, C.c_int64, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int32,
                                      C.c_int32, C.c_int32, C.c_int32, C.c_float, C.c_void_p]
         l.magi_head_norm.restype = C.c_int
@@ -221,6 +223,8 @@ def lib() -> C.CDLL:
         l.magi_small_projections_e4m3.restype = C.c_int
         l.magi_quantize_fp8_split.argtypes = [C.POINTER(QuantizeArgs), C.c_void_p]
         l.magi_quantize_fp8_split.restype = C.c_int
+        l.magi_quantize_fp8_row_max.argtypes = [C.POINTER(QuantizeArgs), C.c_void_p, C.c_void_p]
+        l.magi_quantize_fp8_row_max.restype = C.c_int
         _lib = l
     return _lib
 

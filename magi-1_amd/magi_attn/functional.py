@@ -467,12 +467,14 @@ def qk_prologue(q_raw, k_raw, v_raw, rope, gq, bq, gk, bk, *, Hq: int, Hkv: int,
 def qk_prologue_fp8(q_raw, k_raw, rope, gq, bq, gk, bk, *, Hq: int, Hkv: int, q_scale: float, k_scale: float,
                     eps: float = 1e-6, norm_kind: int = L.MAGI_NORM_LAYERNORM_1P, k_out: Optional[torch.Tensor] = None,
                     n_cache_rows: Optional[int] = None, k_tail: Optional[torch.Tensor] = None,
-                    q_out: Optional[torch.Tensor] = None, batch: int = 1, q_premul: float = 1.0):
+                    q_out: Optional[torch.Tensor] = None, batch: int = 1, q_premul: float = 1.0, v_raw: Optional[torch.Tensor] = None,
+                    v_row_max: Optional[torch.Tensor] = None):
     """qk_prologue with e4m3 outputs (magi_prologue_args.out_dtype): q [S, Hq, D] = sat_e4m3(q * q_premul / q_scale)
     and K rows [*, Hkv, D] = sat_e4m3(k / k_scale) straight from the norm + rotary pass, with the two constant
     scales of the call (powers of two; see pow2_scale_for).  k_out takes the first n_cache_rows tokens (a view of
     an fp8 cache's K rows at the write position), k_tail the rest; with neither a fresh [S, Hkv, D] tensor.
-    V is not part of this pass (quantize_fp8_split takes it from the raw projection).
+    V is not part of this pass (quantize_fp8_split takes it from the raw projection); with v_raw [S, Hkv*D] and v_row_max, an int16
+    [Hkv, S] tensor, the latter receives the largest magnitude of each row, which quantize_fp8_split takes the scales from.
     Returns (q8, k_out, k_tail)."""
     S = q_raw.shape[0]
     D = 128
@@ -487,9 +489,12 @@ def qk_prologue_fp8(q_raw, k_raw, rope, gq, bq, gk, bk, *, Hq: int, Hkv: int, q_
         n_cache_rows = S
     if n_cache_rows is None:
         n_cache_rows = S if k_tail is None else 0
-    for name, t in (("q_raw", q_raw), ("k_raw", k_raw)):
-        if t.dtype != torch.bfloat16 or t.stride(-1) != 1 or t.dim() != 2:
+    for name, t in (("q_raw", q_raw), ("k_raw", k_raw)) + ((("v_raw", v_raw),) if v_row_max is not None else ()):
+        if t is None or t.dtype != torch.bfloat16 or t.stride(-1) != 1 or t.dim() != 2:
             raise ValueError(f"{name} must be a 2-D bf16 tensor with contiguous rows")
+    if v_row_max is not None and (v_row_max.dtype != torch.int16 or tuple(v_row_max.shape) != (Hkv, S) or not v_row_max.is_contiguous()
+                                  or tuple(v_raw.shape) != (S, Hkv * D) or v_raw.device != dev or v_row_max.device != dev):
+        raise ValueError("v_row_max must be a contiguous int16 [Hkv, S] tensor, v_raw [S, Hkv * 128], on q_raw's device")
     for name, t in (("k_out", k_out), ("k_tail", k_tail)):
         if t is not None and (t.dtype != f8 or t.dim() != 3 or t.shape[1:] != (Hkv, D) or t.stride(2) != 1
                               or t.stride(1) != D):
@@ -504,11 +509,14 @@ def qk_prologue_fp8(q_raw, k_raw, rope, gq, bq, gk, bk, *, Hq: int, Hkv: int, q_
         if rope.dtype != torch.float32 or rope.dim() != 2 or rope.shape[0] * max(batch, 1) != S or not rope.is_contiguous():
             raise ValueError("rope must be a contiguous fp32 [S / batch, 2*R2] tensor")
         R2 = rope.shape[1] // 2
-    _launch_packed(dev, "magi_qk_prologue", L.PrologueArgs, q_raw.data_ptr(), k_raw.data_ptr(), 0, _ptr(rope), _ptr(gq), _ptr(bq),
-                   _ptr(gk), _ptr(bk), q_out.data_ptr(), _ptr(k_out), _ptr(k_tail), q_raw.stride(0), k_raw.stride(0), 0,
-                   0 if k_out is None else k_out.stride(0), 0 if k_tail is None else k_tail.stride(0), S, int(n_cache_rows), Hq,
-                   Hkv, D, R2, int(norm_kind), float(eps), int(batch), float(q_premul), L.MAGI_DTYPE_FP8_E4M3, float(q_scale),
-                   float(k_scale))
+    more = v_row_max is not None
+    call = L.packed("magi_qk_prologue_row_max", L.PrologueArgs, C.c_void_p) if more else L.packed("magi_qk_prologue", L.PrologueArgs)
+    args = call.pack(call.size, q_raw.data_ptr(), k_raw.data_ptr(), v_raw.data_ptr() if more else 0, _ptr(rope), _ptr(gq), _ptr(bq), _ptr(gk),
+                     _ptr(bk), q_out.data_ptr(), _ptr(k_out), _ptr(k_tail), q_raw.stride(0), k_raw.stride(0), v_raw.stride(0) if more else 0,
+                     0 if k_out is None else k_out.stride(0), 0 if k_tail is None else k_tail.stride(0), S, int(n_cache_rows), Hq,
+                     Hkv, D, R2, int(norm_kind), float(eps), int(batch), float(q_premul), L.MAGI_DTYPE_FP8_E4M3, float(q_scale),
+                     float(k_scale))
+    _launch(dev, call.fn, args, *((v_row_max.data_ptr(),) if more else ()))
     return q_out, k_out, k_tail
 
 
@@ -865,12 +873,14 @@ def quantize_fp8(x: torch.Tensor, chunk_tokens: int, premul: float = 1.0, pow2_s
 
 def quantize_fp8_split(x: torch.Tensor, chunk_tokens: int, n_rows_first: int, out: Optional[torch.Tensor],
                        scales_out: Optional[torch.Tensor], out2: Optional[torch.Tensor],
-                       scales2_out: Optional[torch.Tensor], premul: float = 1.0, pow2_scales: bool = False) -> None:
+                       scales2_out: Optional[torch.Tensor], premul: float = 1.0, pow2_scales: bool = False,
+                       row_max: Optional[torch.Tensor] = None) -> None:
     """quantize_fp8 in ONE launch with two destinations (magi_quantize_fp8_split): tokens below n_rows_first (a
     multiple of chunk_tokens unless it is T) go to out / scales_out, e.g. the rows of an fp8 KV cache at the write
     position and the matching rows of its scale table; the others to out2 / scales2_out, indexed from
     n_rows_first.  Destinations are contiguous and at least as long as their share; a share of zero rows may
-    pass None."""
+    pass None.  row_max: the largest magnitudes of x's rows as qk_prologue_fp8 leaves them (int16 [H, T]), instead of a pass over x for
+    them; the same bytes."""
     _check_thd(x, "x")
     if x.dtype != torch.bfloat16:
         raise TypeError("x must be bf16")
@@ -888,5 +898,12 @@ def quantize_fp8_split(x: torch.Tensor, chunk_tokens: int, n_rows_first: int, ou
         if (sc is None or sc.dtype != torch.float32 or sc.dim() != 2 or sc.shape[0] < chunks or sc.shape[1] != H
                 or not sc.is_contiguous() or sc.device != x.device):
             raise ValueError(f"the scales of {name} must be a contiguous fp32 [>= {chunks}, H] tensor on x's device")
-    _launch_packed(x.device, "magi_quantize_fp8_split", L.QuantizeArgs, x.data_ptr(), x.stride(0), x.stride(1), T, H, D,
-                   int(chunk_tokens), float(premul), int(pow2_scales), _ptr(out), _ptr(scales_out), n1, _ptr(out2), _ptr(scales2_out))
+    fields = (x.data_ptr(), x.stride(0), x.stride(1), T, H, D, int(chunk_tokens), float(premul), int(pow2_scales), _ptr(out),
+              _ptr(scales_out), n1, _ptr(out2), _ptr(scales2_out))
+    if row_max is None:
+        _launch_packed(x.device, "magi_quantize_fp8_split", L.QuantizeArgs, *fields)
+        return
+    if row_max.dtype != torch.int16 or tuple(row_max.shape) != (H, T) or not row_max.is_contiguous() or row_max.device != x.device:
+        raise ValueError("row_max must be a contiguous int16 [H, T] tensor on x's device")
+    call = L.packed("magi_quantize_fp8_row_max", L.QuantizeArgs, C.c_void_p)
+    _launch(x.device, call.fn, call.pack(call.size, *fields), row_max.data_ptr())

@@ -615,7 +615,8 @@ class FullyParallelAttention(torch.nn.Module):
                             meta_args: ModelMetaArgs, use_cache: bool, out: Optional[torch.Tensor]) -> torch.Tensor:
         """Self-attention on e4m3 operands, three launches from the raw projections (q_raw, k_raw, v_raw) on: the
         prologue writes q and k as e4m3 with the constant scales of fp8_operand_scales(), k straight into the
-        cache rows; one quantiser launch takes v's per-(chunk, head) absmax scales and writes v; the attention.
+        cache rows, and leaves the largest magnitude of each row of v; one quantiser launch takes v's per-(chunk, head) absmax
+        scales from those and writes v; the attention.
         Scale chunks are video chunks (clip_token_nums tokens), so the cache rules of the bf16 path
         (dit_module.py:905-931: append at slice_point, keep nothing when update_kv_cache is False, keep all but
         the last chunk under distill_nearly_clean_chunk) carry over chunk by chunk."""
@@ -631,7 +632,8 @@ class FullyParallelAttention(torch.nn.Module):
         qs_c, ks_c = self.fp8_operand_scales()
         gq, bq = self.q_layernorm.gamma_beta_fp32()
         gk, bk = self.k_layernorm.gamma_beta_fp32()
-        pro = dict(Hq=Hq, Hkv=Hkv, q_scale=qs_c, k_scale=ks_c, eps=self.eps, q_premul=self._q_premul)
+        row_max = torch.empty((Hkv, S), dtype=torch.int16, device=dev)  # of v, from the prologue to the quantiser
+        pro = dict(Hq=Hq, Hkv=Hkv, q_scale=qs_c, k_scale=ks_c, eps=self.eps, q_premul=self._q_premul, v_raw=v_raw, v_row_max=row_max)
         kw = dict(q_scale=self._const_scale_table(qs_c, n_chunks, Hq, dev), scale_chunk_tokens=Lc,
                   fp8_pow2_prescaled=True, fp8_fast_exp2=self.fp8_fast_exp2, out=out, return_lse=False)
         f8 = torch.float8_e4m3fn
@@ -639,7 +641,7 @@ class FullyParallelAttention(torch.nn.Module):
             q8, k8, _ = qk_prologue_fp8(q_raw, k_raw, rope, gq, bq, gk, bk, **pro)
             v8 = torch.empty((S, Hkv, D), dtype=f8, device=dev)
             vs = torch.empty((n_chunks, Hkv), dtype=torch.float32, device=dev)
-            quantize_fp8_split(v3, Lc, S, v8, vs, None, None, pow2_scales=True)
+            quantize_fp8_split(v3, Lc, S, v8, vs, None, None, pow2_scales=True, row_max=row_max)
             o, _ = range_attention(q8, k8, v8, p.q_range, p.k_range, p.max_seqlen_q, p.max_seqlen_k,
                                    k_scale=self._const_scale_table(ks_c, n_chunks, Hkv, dev), v_scale=vs, **kw)
             return o
@@ -664,7 +666,7 @@ class FullyParallelAttention(torch.nn.Module):
             cache.note_constant_k_scale(ks_c, c0, n_keep // Lc)
         q8, _, _ = qk_prologue_fp8(q_raw, k_raw, rope, gq, bq, gk, bk, k_out=cache.k[start:], n_cache_rows=n_keep,
                                    k_tail=k_side, **pro)
-        quantize_fp8_split(v3, Lc, n_keep, cache.v[start:], cache.v_scale[c0:], v_side, vs_side, pow2_scales=True)
+        quantize_fp8_split(v3, Lc, n_keep, cache.v[start:], cache.v_scale[c0:], v_side, vs_side, pow2_scales=True, row_max=row_max)
         split = start + n_keep
         if not n_side:
             o, _ = range_attention(q8, cache.k[:split], cache.v[:split], p.q_range, p.k_range, p.max_seqlen_q,
