@@ -273,8 +273,9 @@ int magi_attn_fwd(const magi_attn_args* args, void* stream);
 
 /* magi_attn_fwd of two calls that do not depend on each other and write different outputs (a layer's core and text attention): in one
  * launch where both take the form of MAGI_ATTN_SHARE_WAVES, or both 256 rows per workgroup (magi_attn_tile_rows) with q pre-scaled or raw,
- * a score_bound and no keys of the second shared; else one after the other.  The same bits as two calls.  A refusal of the second is this
- * call's, the first has been launched by then. */
+ * a score_bound and no keys of the second shared, or the first has e4m3 rows with MAGI_ATTN_FP8_POW2_PRESCALED and the second raw q
+ * (q_norm_gamma) and a score_bound; else one after the other.  The same bits as two calls, the second of them, behind e4m3 rows, without
+ * a split_workspace.  A refusal of the second is this call's, the first has been launched by then. */
 int magi_attn_fwd_two(const magi_attn_args* first, const magi_attn_args* second, void* stream);
 
 /*

@@ -400,7 +400,8 @@ int waves_plan(int Hq, int Hkv, int n_ranges, int ranges_mode, int max_seqlen_q,
 
 // held: where the call takes a form that may share a launch with another, its arguments instead of the launch; HELD is returned then
 constexpr int HELD = 1;
-int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace, magi::AttnKernArgs* held = nullptr);
+// (text: beside a call of e4m3 rows, where every form of raw q with bounded scores is one, but those whose keys are shared)
+int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace, magi::AttnKernArgs* held = nullptr, bool text = false);
 // a held call by itself
 int launch_held(const magi::AttnKernArgs& a, void* stream);
 int attn_fwd_two(const magi_attn_args* first, const magi_attn_args* second, void* stream);
@@ -521,6 +522,22 @@ int attn_fwd_two(const magi_attn_args* first, const magi_attn_args* second, void
   magi::AttnPairArgs pair;
   const int one = attn_fwd_impl(first, stream, first->workspace, &pair.job[0]);
   if (one != HELD) return one < 0 ? one : attn_fwd_impl(second, stream, second->workspace);
+  if (first->dtype == MAGI_DTYPE_FP8_E4M3) {
+    const hipStream_t st = static_cast<hipStream_t>(stream);
+    magi::AttnKernArgs &a = pair.job[0], &b = pair.job[1];
+    const int two = attn_fwd_impl(second, stream, second->workspace, &b, true);
+    const bool together = two == HELD && b.block_m != 32 && (double)b.Hq * b.n_ranges * second->max_seqlen_q < 1e11;  // (a grid that fits)
+    if (together) {
+      b.block_m = 128;
+      b.tiles_per_range = (second->max_seqlen_q + 127) / 128;
+      b.per_xcd = items_per_xcd(b.Hq, b.Hkv, b.n_ranges, b.tiles_per_range);
+      b.split_from = UINT32_MAX;
+    }
+    const hipError_t e = together ? magi::launch_attn_fwd_fp8_text(pair, st) : magi::launch_attn_fwd_fp8(a, st);
+    if (e != hipSuccess) return hip_fail(e, "magi_attn_fwd launch");
+    count_launches(1 + (a.split_from < a.per_xcd));
+    return together || two != HELD ? (two < 0 ? two : MAGI_OK) : launch_held(b, stream);
+  }
   const int two = attn_fwd_impl(second, stream, second->workspace, &pair.job[1]);
   const magi::AttnKernArgs &a = pair.job[0], &b = pair.job[1];
   if (two == HELD && a.block_m == b.block_m && (b.block_m == 32 || b.split_from >= b.per_xcd)) return launch_held(pair, 2, stream);
@@ -528,7 +545,7 @@ int attn_fwd_two(const magi_attn_args* first, const magi_attn_args* second, void
   return rc < 0 ? rc : two == HELD ? launch_held(b, stream) : two;
 }
 
-int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace, magi::AttnKernArgs* held) {
+int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace, magi::AttnKernArgs* held, bool text) {
   if (p->D != 128) return fail(MAGI_ENOSYS, "magi_attn_fwd: head_dim %d not implemented (128 only)", p->D);
   if (p->dtype != MAGI_DTYPE_BF16 && p->dtype != MAGI_DTYPE_FP8_E4M3)
     return fail(MAGI_EINVAL, "magi_attn_fwd: unknown dtype %d", p->dtype);
@@ -780,7 +797,12 @@ int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace, magi:
       if (s.bytes(a.per_xcd) <= split_bytes) pieces(s);
     }
     // (of the other forms the one of large launches: in the smaller ones the core's rows or keys are dealt out over the whole chip as it is)
-    if (held && bounded && a.block_m == 256 && !checked && !mfma32 && !auto_bound && !scale_q) {
+    if (held && bounded && a.block_m == 256 && !checked && !mfma32 && !auto_bound && !scale_q && (!text || q_norm)) {
+      *held = a;
+      return HELD;
+    }
+    if (held && (text ? bounded && q_norm && a.block_m == 128 && a.share_pieces <= 1 && !checked && !auto_bound
+                      : fp8 && (p->flags & MAGI_ATTN_FP8_POW2_PRESCALED))) {
       *held = a;
       return HELD;
     }

@@ -84,7 +84,7 @@ hipError_t launch_attn_fwd_bf16_r32(const AttnKernArgs& a, hipStream_t stream);
 // One or two calls (job[1].per_xcd = 0: one), bounded scores, block_m 32: the wavefronts of a workgroup share the keys of 32 rows
 struct AttnPairArgs {
   AttnKernArgs job[2];
-  unsigned ahead;  // attn_fwd_bf16_x16.hip: workgroups of the first per XCD
+  unsigned ahead;  // attn_fwd_bf16_x16.hip, attn_fwd_fp8_text.hip: workgroups of the first per XCD
 };
 hipError_t launch_attn_fwd_bf16_waves(const AttnPairArgs& p, hipStream_t stream);
 hipError_t launch_attn_fwd_bf16_w64(const AttnKernArgs& a, hipStream_t stream);
@@ -95,6 +95,9 @@ hipError_t launch_attn_fwd_bf16_x16_pair(const AttnPairArgs& p, hipStream_t stre
 // the bounded-score kernel without a promise, and behind it the launch that repeats what it could not be trusted with
 hipError_t launch_attn_fwd_bf16_checked(const AttnKernArgs& a, int compute_units, hipStream_t stream);
 hipError_t launch_attn_fwd_fp8(const AttnKernArgs& a, hipStream_t stream);
+void launch_fp8_merge(const AttnKernArgs& a, hipStream_t stream);  // the launch behind one with items to split
+// a call of e4m3 rows with power-of-two scales and one of bf16 rows in 128-row tiles, bounded scores, raw q, nothing to split
+hipError_t launch_attn_fwd_fp8_text(const AttnPairArgs& p, hipStream_t stream);
 // ws[0..3] = 0 (a kernel, not a memset: the call may be under graph capture)
 hipError_t launch_gate_init(unsigned* ws, hipStream_t stream);
 // *out_bits = max(*out_bits, bit pattern of the largest sum of squares over a [T, H, 128] bf16 tensor's rows);

@@ -612,7 +612,7 @@ class FullyParallelAttention(torch.nn.Module):
         return t[:shape[0]]
 
     def _core_attention_fp8(self, raw, rope: torch.Tensor, inference_params: Optional[InferenceParams],
-                            meta_args: ModelMetaArgs, use_cache: bool, out: Optional[torch.Tensor]) -> torch.Tensor:
+                            meta_args: ModelMetaArgs, use_cache: bool, out: Optional[torch.Tensor], held: Optional[list] = None) -> torch.Tensor:
         """Self-attention on e4m3 operands, three launches from the raw projections (q_raw, k_raw, v_raw) on: the
         prologue writes q and k as e4m3 with the constant scales of fp8_operand_scales(), k straight into the
         cache rows, and leaves the largest magnitude of each row of v; one quantiser launch takes v's per-(chunk, head) absmax
@@ -639,7 +639,7 @@ class FullyParallelAttention(torch.nn.Module):
         if row_max is not None:
             pro.update(v_raw=v_raw, v_row_max=row_max)
         kw = dict(q_scale=self._const_scale_table(qs_c, n_chunks, Hq, dev), scale_chunk_tokens=Lc,
-                  fp8_pow2_prescaled=True, fp8_fast_exp2=self.fp8_fast_exp2, out=out, return_lse=False)
+                  fp8_pow2_prescaled=True, fp8_fast_exp2=self.fp8_fast_exp2, out=out, return_lse=False, held=held)
         f8 = torch.float8_e4m3fn
         if not use_cache:
             q8, k8, _ = qk_prologue_fp8(q_raw, k_raw, rope, gq, bq, gk, bk, **pro)
@@ -1259,6 +1259,10 @@ class FullyParallelAttention(torch.nn.Module):
                     held = []
             elif rows_per_cu >= 512:
                 held = []
+        elif cross_bounded and self.attention_dtype == "fp8" and _OWN_CROSS_FUSED.of(self) and _OWN_CORE_FP8.of(self):
+            # (e4m3 core: the text beside it in a form of its own, attn_fwd_fp8_text.hip.  40 drawn layers from 122 rows per CU on 1.006 to 1.096
+            # times as fast, 86400 rows 1.001; up to 71 rows per CU 0.997 to 1.004: their core and text do not fill the chip together)
+            held = [] if sq * Hq >= 64 * _compute_units(hidden_states.device) else None
         if proj_layout and bs == 1 and Hq % PROJ_GROUPS == 0:
             # (rows that no q range / cu_seqlens segment covers are left as allocated: the pipeline's ranges cover
             # every row, dit_model.py:220-222, 246; bf16, what the launches write, whatever hidden_states is)
@@ -1278,7 +1282,7 @@ class FullyParallelAttention(torch.nn.Module):
         if self.attention_dtype == "fp8":
             if bs != 1 or (use_cache and inference_params.max_batch_size != 1):
                 raise ValueError("the fp8 self-attention runs at batch 1")
-            core = self._core_attention_fp8(raw, rope, inference_params, meta_args, use_cache, core_dst)
+            core = self._core_attention_fp8(raw, rope, inference_params, meta_args, use_cache, core_dst, **({} if held is None else {"held": held}))
         elif not use_cache:
             q, kv, qx_raw = project()
             if not _OWN_CORE.of(self):
@@ -1349,6 +1353,7 @@ _OWN_CROSS = _Own(FullyParallelAttention, "get_xqkv", "cross_attention")
 _CROSS_FUSED = FullyParallelAttention._cross_attention_fused
 _OWN_CROSS_FUSED = _Own(FullyParallelAttention, "_cross_attention_fused")
 _OWN_CORE = _Own(FullyParallelAttention, "core_attention")
+_OWN_CORE_FP8 = _Own(FullyParallelAttention, "_core_attention_fp8")
 _OWN_SMALL = _Own(FullyParallelAttention, "_project_rows", "_fused_qkv", "_cross_attention_fused")
 _OWN_SMALL_UNCACHED = _Own(FullyParallelAttention, "_project_rows", "_fused_qkv", "_cross_attention_fused", "core_attention")
 _OWN_SMALL_FP8 = _Own(FullyParallelAttention, "_project_rows", "_core_attention_fp8", "_cross_attention_fused")
