@@ -538,7 +538,8 @@ int attn_fwd_two(const magi_attn_args* first, const magi_attn_args* second, void
     count_launches(1 + (a.split_from < a.per_xcd));
     return together || two != HELD ? (two < 0 ? two : MAGI_OK) : launch_held(b, stream);
   }
-  const int two = attn_fwd_impl(second, stream, second->workspace, &pair.job[1]);
+  const bool rows8 = second->dtype == MAGI_DTYPE_FP8_E4M3;  // (shares a launch as the first of the two only)
+  const int two = attn_fwd_impl(second, stream, second->workspace, rows8 ? nullptr : &pair.job[1]);
   const magi::AttnKernArgs &a = pair.job[0], &b = pair.job[1];
   if (two == HELD && a.block_m == b.block_m && (b.block_m == 32 || b.split_from >= b.per_xcd)) return launch_held(pair, 2, stream);
   const int rc = launch_held(a, stream);

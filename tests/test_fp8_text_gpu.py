@@ -56,8 +56,11 @@ def test_the_bits_of_the_two_launches(dev, chunks, Lc, prefix, Hq, Hkv, text, fa
     assert M.lib().magi_launch_count() == before and len(held) == 2
     launch_held(held)
     assert not held and 1 <= M.lib().magi_launch_count() - before <= 4
-    for a, b in zip(together, one_by_one):
-        assert torch.equal(a, b) and bool(torch.isfinite(a.float()).all())
+    turned = calls(held)
+    held.reverse()  # (the text first: two launches)
+    launch_held(held)
+    for a, b, c in zip(together, one_by_one, turned):
+        assert torch.equal(a, b) and torch.equal(c, b) and bool(torch.isfinite(a.float()).all())
 
 
 def test_a_held_call_by_itself(dev):
