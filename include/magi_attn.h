@@ -103,7 +103,7 @@ extern "C" {
  * 105: the structs of 104; new are MAGI_ATTN_ROW_BITS (a library of 104 would ignore it), magi_attn_split_bytes_256,
  * magi_attn_pieces_bytes, magi_small_projections_e4m3 and magi_small_layer.
  * 106: the structs of 105; new are MAGI_ATTN_SHARE_WAVES, magi_attn_waves and magi_attn_fwd_two.
- * 107: the structs of 106; new are magi_qk_prologue_row_max and magi_quantize_fp8_row_max. */
+ * 107: the structs of 106; new are magi_qk_prologue_row_max, magi_quantize_fp8_row_max, magi_attn_fwd_begin and magi_attn_fwd_end. */
 int magi_version(void);
 const char* magi_last_error(void);
 /* Diagnostics: the number of kernel launches the library has issued in this process so far (all threads, all
@@ -277,6 +277,14 @@ int magi_attn_fwd(const magi_attn_args* args, void* stream);
  * (q_norm_gamma) and a score_bound; else one after the other.  The same bits as two calls, the second of them, behind e4m3 rows, without
  * a split_workspace.  A refusal of the second is this call's, the first has been launched by then. */
 int magi_attn_fwd_two(const magi_attn_args* first, const magi_attn_args* second, void* stream);
+
+/* magi_attn_fwd in two halves.  begin returns MAGI_OK where the call is done, and 1 where it has left pieces in split_workspace (bounded
+ * scores, keys of 256-row items shared): its output is then written by magi_attn_fwd_end with the same arguments on the same stream, and
+ * split_workspace is kept until that.  end takes a second call with it (or NULL) that does not depend on the first's output, a text attention:
+ * in one launch where it has raw q (q_norm_gamma) and a score_bound, else behind it.  The same bits as two calls, the second without a
+ * split_workspace.  A refusal of the second is this call's, the first is done all the same. */
+int magi_attn_fwd_begin(const magi_attn_args* args, void* stream);
+int magi_attn_fwd_end(const magi_attn_args* first, const magi_attn_args* second, void* stream);
 
 /*
  * magi_attn_fwd for callers that cannot hand over a workspace and must not allocate one (code under HIP graph

@@ -400,11 +400,14 @@ int waves_plan(int Hq, int Hkv, int n_ranges, int ranges_mode, int max_seqlen_q,
 
 // held: where the call takes a form that may share a launch with another, its arguments instead of the launch; HELD is returned then
 constexpr int HELD = 1;
-// (text: beside a call of e4m3 rows, where every form of raw q with bounded scores is one, but those whose keys are shared)
-int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace, magi::AttnKernArgs* held = nullptr, bool text = false);
+// TEXT: beside something else, where every form of raw q with bounded scores is one, but those whose keys are shared.  BEGIN: items whose keys
+// are shared leave their pieces (HELD then), others are done; PIECES: the arguments that left them.
+enum Held { ALIKE, TEXT, BEGIN, PIECES };
+int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace, magi::AttnKernArgs* held = nullptr, Held how = ALIKE);
 // a held call by itself
 int launch_held(const magi::AttnKernArgs& a, void* stream);
 int attn_fwd_two(const magi_attn_args* first, const magi_attn_args* second, void* stream);
+int attn_fwd_end(const magi_attn_args* first, const magi_attn_args* second, void* stream);
 
 // the caller's struct as this version lays it out: itself, or `full` filled from the shorter one of version 103
 const magi_attn_args* current_layout(const magi_attn_args* p, magi_attn_args* full) {
@@ -481,6 +484,20 @@ int magi_attn_fwd_two(const magi_attn_args* first, const magi_attn_args* second,
   return attn_fwd_two(first, second, stream);
 }
 
+int magi_attn_fwd_begin(const magi_attn_args* p, void* stream) {
+  if (!p) return fail(MAGI_EINVAL, "magi_attn_fwd_begin: args is NULL");
+  MAGI_CHECK_LAYOUT("magi_attn_fwd_begin", p);
+  magi::AttnKernArgs left;
+  return attn_fwd_impl(p, stream, p->workspace, &left, BEGIN);
+}
+
+int magi_attn_fwd_end(const magi_attn_args* first, const magi_attn_args* second, void* stream) {
+  if (!first) return fail(MAGI_EINVAL, "magi_attn_fwd_end: args is NULL");
+  MAGI_CHECK_LAYOUT("magi_attn_fwd_end", first);
+  if (second) MAGI_CHECK_LAYOUT("magi_attn_fwd_end", second);
+  return attn_fwd_end(first, second, stream);
+}
+
 int magi_attn_fwd_static_scratch(const magi_attn_args* p, void* stream) {
   if (!p) return fail(MAGI_EINVAL, "magi_attn_fwd_static_scratch: args is NULL");
   magi_attn_args full;
@@ -517,6 +534,31 @@ int launch_held(const magi::AttnKernArgs& a, void* stream) {
   return launch_held(pair, 1, stream);
 }
 
+// a held text call as attn_text_rows.h takes it: 128-row tiles, whole items; false where it is another kind, or the grid would not fit
+bool text_in_128_rows(magi::AttnKernArgs& b, int max_seqlen_q) {
+  if (b.block_m == 32 || (double)b.Hq * b.n_ranges * max_seqlen_q >= 1e11) return false;
+  b.block_m = 128;
+  b.tiles_per_range = (max_seqlen_q + 127) / 128;
+  b.per_xcd = items_per_xcd(b.Hq, b.Hkv, b.n_ranges, b.tiles_per_range);
+  b.split_from = UINT32_MAX;
+  return true;
+}
+
+// the second half of magi_attn_fwd_begin(first), beside second
+int attn_fwd_end(const magi_attn_args* first, const magi_attn_args* second, void* stream) {
+  const hipStream_t st = static_cast<hipStream_t>(stream);
+  magi::AttnPairArgs pair;
+  magi::AttnKernArgs &a = pair.job[0], &b = pair.job[1];
+  const int one = attn_fwd_impl(first, stream, first->workspace, &a, PIECES);
+  if (one != HELD) return one < 0 ? one : fail(MAGI_EINVAL, "magi_attn_fwd_end: an empty call leaves no pieces");
+  const int two = second ? attn_fwd_impl(second, stream, second->workspace, &b, TEXT) : MAGI_OK;
+  const bool together = two == HELD && text_in_128_rows(b, second->max_seqlen_q);
+  const hipError_t e = together ? magi::launch_attn_text_merge(pair, st) : magi::launch_attn_fwd_bf16_merge(a, st);
+  if (e != hipSuccess) return hip_fail(e, "magi_attn_fwd_end launch");
+  count_launches(1);
+  return together ? MAGI_OK : two == HELD ? launch_held(b, stream) : two;
+}
+
 // first, then second, which do not depend on each other: in one launch where both take the form for it
 int attn_fwd_two(const magi_attn_args* first, const magi_attn_args* second, void* stream) {
   magi::AttnPairArgs pair;
@@ -525,14 +567,8 @@ int attn_fwd_two(const magi_attn_args* first, const magi_attn_args* second, void
   if (first->dtype == MAGI_DTYPE_FP8_E4M3) {
     const hipStream_t st = static_cast<hipStream_t>(stream);
     magi::AttnKernArgs &a = pair.job[0], &b = pair.job[1];
-    const int two = attn_fwd_impl(second, stream, second->workspace, &b, true);
-    const bool together = two == HELD && b.block_m != 32 && (double)b.Hq * b.n_ranges * second->max_seqlen_q < 1e11;  // (a grid that fits)
-    if (together) {
-      b.block_m = 128;
-      b.tiles_per_range = (second->max_seqlen_q + 127) / 128;
-      b.per_xcd = items_per_xcd(b.Hq, b.Hkv, b.n_ranges, b.tiles_per_range);
-      b.split_from = UINT32_MAX;
-    }
+    const int two = attn_fwd_impl(second, stream, second->workspace, &b, TEXT);
+    const bool together = two == HELD && text_in_128_rows(b, second->max_seqlen_q);
     const hipError_t e = together ? magi::launch_attn_fwd_fp8_text(pair, st) : magi::launch_attn_fwd_fp8(a, st);
     if (e != hipSuccess) return hip_fail(e, "magi_attn_fwd launch");
     count_launches(1 + (a.split_from < a.per_xcd));
@@ -546,7 +582,7 @@ int attn_fwd_two(const magi_attn_args* first, const magi_attn_args* second, void
   return rc < 0 ? rc : two == HELD ? launch_held(b, stream) : two;
 }
 
-int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace, magi::AttnKernArgs* held, bool text) {
+int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace, magi::AttnKernArgs* held, Held how) {
   if (p->D != 128) return fail(MAGI_ENOSYS, "magi_attn_fwd: head_dim %d not implemented (128 only)", p->D);
   if (p->dtype != MAGI_DTYPE_BF16 && p->dtype != MAGI_DTYPE_FP8_E4M3)
     return fail(MAGI_EINVAL, "magi_attn_fwd: unknown dtype %d", p->dtype);
@@ -772,7 +808,7 @@ int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace, magi:
     };
     a.share_pieces = 1;
     if (a.waves) {
-      if (!held) return launch_held(a, stream);
+      if (!held || how == BEGIN) return launch_held(a, stream);
       *held = a;
       return HELD;
     }
@@ -798,12 +834,18 @@ int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace, magi:
       if (s.bytes(a.per_xcd) <= split_bytes) pieces(s);
     }
     // (of the other forms the one of large launches: in the smaller ones the core's rows or keys are dealt out over the whole chip as it is)
-    if (held && bounded && a.block_m == 256 && !checked && !mfma32 && !auto_bound && !scale_q && (!text || q_norm)) {
+    const bool x16 = bounded && a.block_m == 256 && !checked && !mfma32 && !auto_bound;
+    if (how == PIECES || (how == BEGIN && x16 && a.split_from < a.per_xcd)) {
+      if (!x16 || a.split_from >= a.per_xcd) return fail(MAGI_EINVAL, "magi_attn_fwd_end: not what magi_attn_fwd_begin left pieces of");
       *held = a;
+      if (how == PIECES) return HELD;
+      const hipError_t e = magi::launch_attn_fwd_bf16_x16(a, static_cast<hipStream_t>(stream), false);
+      if (e != hipSuccess) return hip_fail(e, "magi_attn_fwd_begin launch");
+      count_launches(1);
       return HELD;
     }
-    if (held && (text ? bounded && q_norm && a.block_m == 128 && a.share_pieces <= 1 && !checked && !auto_bound
-                      : fp8 && (p->flags & MAGI_ATTN_FP8_POW2_PRESCALED))) {
+    if (how == ALIKE ? held && ((x16 && !scale_q) || (fp8 && (p->flags & MAGI_ATTN_FP8_POW2_PRESCALED)))
+                     : how == TEXT && q_norm && (x16 || (bounded && a.block_m == 128 && a.share_pieces <= 1 && !checked && !auto_bound))) {
       *held = a;
       return HELD;
     }

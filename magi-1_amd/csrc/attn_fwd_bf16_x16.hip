@@ -28,7 +28,7 @@
 // The epilogue goes through LDS (the tile slots are free by then): every wave writes its 64 x 128 normalised
 // outputs as bf16 rows and reads them back 16 bytes per lane, so that 16 consecutive lanes store one whole 256-byte
 // row: every global store instruction writes four complete rows.
-#include "attn_common.h"
+#include "attn_bf16_merge.h"
 
 namespace magi {
 namespace {
@@ -82,8 +82,6 @@ constexpr int v_block(int i) { return (i >> 1) + 4 * (i & 1); }
 // Q_EITHER: as it is, or raw where the call has norm parameters (a launch of two calls).
 constexpr int Q_AS_IS = 0, Q_NORM = 1, Q_SCALE = 2, Q_CHECK = 3, Q_EITHER = 4;
 
-// Row sums that the kernel without a running maximum can be trusted with (CHECK, below).
-constexpr float SUM_MIN = 0x1p-16f, SUM_MAX = 0x1p64f;
 
 // CHECK (QMODE Q_CHECK): nobody has promised that the scores are bounded.  The kernel computes as if they were, and each wavefront
 // leaves a verdict on its 64 rows in a.verdict[4 * item + wavefront]: they are good where SUM_MIN <= row sum <= SUM_MAX
@@ -128,68 +126,12 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_bf16_x16_pair_kernel(const At
 }
 #undef X16_BLOCK
 
-// workgroups per item of the kernel below
-template <bool CHECK>
-constexpr int MERGE_SHARES = CHECK ? 1 : 4;
-
-// The split items of a launch of the kernel above: sums their pieces, normalises, writes the rows (CHECK: and the verdicts).
-// A wavefront for each 64 rows, lane layout of the accumulators as above.  Memory bound: SPLIT_FLOATS * 4 bytes read per piece.
-// Four workgroups per item, one for each query block (CHECK: one, which leaves the wavefronts' verdicts), on the item's XCD: with
-// one for all four a launch of 48 items read 0.5 MB per workgroup and nothing beside it.
+// (see attn_bf16_merge.h)
 template <bool CHECK>
 __global__ __launch_bounds__(256) void attn_fwd_bf16_merge_kernel(const AttnKernArgs a) {
-  constexpr int SHARES = MERGE_SHARES<CHECK>;
   __shared__ int s_sel[LOCATE_WORDS];
   if (gate_closed(a)) return;
-  const int tid = threadIdx.x, l = tid & 63, n = l & 15, g = l >> 4;
-  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const unsigned share = (blockIdx.x >> 3) % SHARES, item = ((blockIdx.x >> 3) / SHARES << 3) | (blockIdx.x & 7u);
-  const WorkItem wi = locate_work(a, 256, tid, s_sel, item + 8u * a.split_from);
-  const int row0 = wi.q0 + 64 * w;
-  if (!wi.valid || wi.ke <= wi.ks) return;  // (nothing there, or without keys: done)
-  if (row0 >= wi.qe) {
-    if (CHECK && l == 0) a.verdict[4 * (long)wi.item + w] = 0;
-    return;
-  }
-  const float* const base = a.partial + (long)item * a.split_pieces * SPLIT_FLOATS;
-  const int pieces = (int)a.split_pieces;
-  bool bad = false;
-#pragma unroll
-  for (int k = 0; k < 4 / SHARES; ++k) {
-    const int qb = CHECK ? k : (int)share;
-    const float* p = base;
-    float s = 0.f;
-    f32x4v o[8];
-#pragma unroll
-    for (int db = 0; db < 8; ++db) o[db] = f32x4v{0.f, 0.f, 0.f, 0.f};
-    for (int i = 0; i < pieces; ++i, p += SPLIT_FLOATS) {
-      const f32x4v* const src = (const f32x4v*)p + w * 2048 + l;
-#pragma unroll
-      for (int db = 0; db < 8; ++db) o[db] += src[(4 * db + qb) * 64];
-      s += p[256 * 128 + 64 * w + 16 * qb + n];
-    }
-    if constexpr (CHECK) {
-      float fine = 0.f;
-#pragma unroll
-      for (int db = 0; db < 8; ++db)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) fine = __builtin_fmaf(o[db][r], 0.f, fine);
-      bad |= !(s >= SUM_MIN && s <= SUM_MAX) || fine != fine;
-    }
-    const int q_row = row0 + 16 * qb + n;
-    if (q_row >= wi.qe) continue;
-    const float inv = 1.f / s;
-    char* const op = a.out + row_offset(a, q_row, a.os_t, a.os_b) + wi.o_head + 8 * g;
-#pragma unroll
-    for (int db = 0; db < 8; ++db)
-      *(u32x2*)(op + 32 * db) = u32x2{pack_bf16x2(o[db][0] * inv, o[db][1] * inv), pack_bf16x2(o[db][2] * inv, o[db][3] * inv)};
-    if (a.lse && g == 0) a.lse[(long)wi.h * a.total_q + q_row] = __builtin_amdgcn_logf(s) * 0.6931471805599453f;
-  }
-  if constexpr (CHECK) {
-    // (rows beyond the range repeat its last row, as in the kernel that left the pieces: they raise no flag of their own)
-    const bool any = __builtin_amdgcn_ballot_w64(bad) != 0;
-    if (l == 0) a.verdict[4 * (long)wi.item + w] = any ? 1 : 0;
-  }
+  merge_pieces<CHECK>(a, blockIdx.x, s_sel);
 }
 
 // The rows that a CHECK launch of the kernels above could not be trusted with, again, with a running maximum: same ranges,
@@ -383,7 +325,7 @@ void launch_merge(const AttnKernArgs& a, hipStream_t stream) {
 }
 }  // namespace
 
-hipError_t launch_attn_fwd_bf16_x16(const AttnKernArgs& a, hipStream_t stream) {
+hipError_t launch_attn_fwd_bf16_x16(const AttnKernArgs& a, hipStream_t stream, bool merge) {
   const dim3 grid(split_grid(a));
   if (a.block_m == 128) {
     if (a.q_norm_gamma)
@@ -400,6 +342,11 @@ hipError_t launch_attn_fwd_bf16_x16(const AttnKernArgs& a, hipStream_t stream) {
     hipLaunchKernelGGL(attn_fwd_bf16_x16_kernel<Q_SCALE>, grid, dim3(256), 0, stream, a);
   else
     hipLaunchKernelGGL(attn_fwd_bf16_x16_kernel<Q_AS_IS>, grid, dim3(256), 0, stream, a);
+  if (merge) launch_merge<false>(a, stream);
+  return hipGetLastError();
+}
+
+hipError_t launch_attn_fwd_bf16_merge(const AttnKernArgs& a, hipStream_t stream) {
   launch_merge<false>(a, stream);
   return hipGetLastError();
 }

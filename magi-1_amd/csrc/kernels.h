@@ -89,7 +89,10 @@ struct AttnPairArgs {
 hipError_t launch_attn_fwd_bf16_waves(const AttnPairArgs& p, hipStream_t stream);
 hipError_t launch_attn_fwd_bf16_w64(const AttnKernArgs& a, hipStream_t stream);
 // (with items to split: and behind it the launch that adds their pieces up)
-hipError_t launch_attn_fwd_bf16_x16(const AttnKernArgs& a, hipStream_t stream);
+hipError_t launch_attn_fwd_bf16_x16(const AttnKernArgs& a, hipStream_t stream, bool merge = true);
+hipError_t launch_attn_fwd_bf16_merge(const AttnKernArgs& a, hipStream_t stream);  // that launch by itself
+// and it beside a call in 128-row tiles, bounded scores, raw q, nothing to split
+hipError_t launch_attn_text_merge(const AttnPairArgs& p, hipStream_t stream);
 // two such calls in 256-row workgroups, the second without items to split, q as it is or raw
 hipError_t launch_attn_fwd_bf16_x16_pair(const AttnPairArgs& p, hipStream_t stream);
 // the bounded-score kernel without a promise, and behind it the launch that repeats what it could not be trusted with

@@ -23,7 +23,7 @@ import torch
 from . import _lib as L
 
 
-def _launch(dev: torch.device, fn, *args) -> None:
+def _launch(dev: torch.device, fn, *args) -> int:
     """fn(*args, stream) with `dev` current, on its current stream; raises on a negative code."""
     index = dev.index
     if torch._C._cuda_getDevice() == index:
@@ -31,8 +31,16 @@ def _launch(dev: torch.device, fn, *args) -> None:
     else:
         with torch.cuda.device(dev):
             code = fn(*args, torch._C._cuda_getCurrentRawStream(index))
-    if code != 0:
+    if code < 0:
         L.check(code)
+    return code
+
+
+class BegunCalls(list):
+    """A list for range_attention's `held` whose first call is launched at once but for what brings its pieces together, where it
+    leaves any (magi_attn_fwd_begin); launch_held() then launches that and the second call as one where it can."""
+
+    begin = True  # the next call is the first
 
 
 def _launch_packed(dev: torch.device, name: str, args: type, *fields) -> None:
@@ -287,6 +295,10 @@ def range_attention(
         _ptr(v2_scale), _ptr(workspace), batch_rows, q_stride_b, o_stride_b, _ptr(split), split_bytes)
     if held is None:
         _launch(q.device, call.fn, args)
+    elif type(held) is BegunCalls and held.begin:
+        held.begin = False
+        if _launch(q.device, L.packed("magi_attn_fwd_begin", L.AttnArgs).fn, args):
+            held.append((q.device, None, args, (q, k, v, k2, v2, q_ranges, k_ranges, gamma, beta, split, out, lse)))
     else:  # (with everything it reads and writes)
         held.append((q.device, call.fn, args, (q, k, v, k2, v2, q_ranges, k_ranges, q_scale, k_scale, v_scale, k2_scale, v2_scale, gamma, beta, workspace,
                                                split, out, lse)))
@@ -296,7 +308,13 @@ def range_attention(
 def launch_held(calls: list) -> None:
     """The calls that range_attention(held=calls) left, on the current stream: two that do not depend on each other in one launch where their
     sizes are for it (magi_attn_fwd_two).  Empties the list."""
-    if len(calls) == 2 and calls[0][0] == calls[1][0]:
+    if calls and calls[0][1] is None:  # (begun)
+        alone = len(calls) == 1 or calls[0][0] != calls[1][0]
+        _launch(calls[0][0], L.packed_pair("magi_attn_fwd_end").fn, calls[0][2], None if alone else calls[1][2])
+        if alone:
+            for dev, fn, args, _ in calls[1:]:
+                _launch(dev, fn, args)
+    elif len(calls) == 2 and calls[0][0] == calls[1][0]:
         _launch(calls[0][0], L.packed_pair("magi_attn_fwd_two").fn, calls[0][2], calls[1][2])
     else:
         for dev, fn, args, _ in calls:

@@ -37,7 +37,7 @@ from . import _lib as L
 from .cache import Fp8KVCache, OffloadedKVCache
 from .functional import (_measuring_a_bound_pays, covered_by_launch, launch_fp8_attention, launch_quantize_fp8_split,
                          launch_small_projections_e4m3, launch_text_attention, range_count, split_memory)
-from .functional import attention_waves, launch_held
+from .functional import BegunCalls, attention_waves, launch_held
 from .functional import launch_small_layer as launch_small_projections  # (named by the first of the launches it stands for)
 from .functional import (div_clamp_to, head_norm, layer_norm, layer_norm_div_clamp, pow2_scale_for, qk_prologue, qk_prologue_fp8, qkv_proj_prologue,
                          quantize_fp8_split,
@@ -1248,7 +1248,9 @@ class FullyParallelAttention(torch.nn.Module):
         # for it: few rows (waves), or two rounds of 256-row workgroups.  There the text's workgroups run beside the core's last ones: 2 to 4 %
         # of a layer of 3120 to 16200 rows and 24 or 48 heads (1233 -> 1197 us, 2215 -> 2183, 6414 -> 6264, 7670 -> 7426), 0.6 % of
         # 21600 rows x 2 chunks (29.7 -> 29.5 ms).  Between the two the core is issued as soon as it can be: its keys are in pieces that fill
-        # the chip anyway, and the device would wait for what the host does for the text (one round and below: 0.90 to 1.04 of the speed).
+        # the chip anyway, and the device would wait for what the host does for the text (one round and below: 0.90 to 1.04 of the speed);
+        # what brings the pieces together then goes beside the text: 30 drawn layers of 148 to 504 rows per CU 0.994 to 1.037 times as fast
+        # (2112 rows 390 -> 381 us, 2964 403 -> 389), the ones without pieces the same; from 44 to 83 rows per CU, which wait for the host, 0.985 to 1.026.
         held = None
         if core_bounded and cross_bounded and self.attention_dtype == "bf16" and _OWN_CROSS_FUSED.of(self):
             rows_per_cu = sq * Hq / _compute_units(hidden_states.device)  # of all heads
@@ -1259,6 +1261,8 @@ class FullyParallelAttention(torch.nn.Module):
                     held = []
             elif rows_per_cu >= 512:
                 held = []
+            elif rows_per_cu >= 128:
+                held = BegunCalls()
         elif cross_bounded and self.attention_dtype == "fp8" and _OWN_CROSS_FUSED.of(self) and _OWN_CORE_FP8.of(self):
             # (e4m3 core: the text beside it in a form of its own, attn_fwd_fp8_text.hip.  40 drawn layers from 122 rows per CU on 1.006 to 1.096
             # times as fast, 86400 rows 1.001; up to 71 rows per CU 0.997 to 1.004: their core and text do not fill the chip together)

@@ -1,0 +1,76 @@
+"""The core attention in two halves, the second beside the text attention: the bits and the number of launches of the calls one by one."""
+import pytest
+import torch
+
+import magi_attn as M
+from magi_attn import _lib as L
+from magi_attn.functional import BegunCalls, attention_waves, launch_held, range_attention
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def dev():
+    assert torch.cuda.is_available()
+    return torch.device("cuda")
+
+
+# keys in pieces: less than a round of 256-row workgroups, a round and a part; ranges of two lengths; text around the 32- and 64-key tiles, of
+# which one segment has none; a core without pieces (done by its first half); text in a launch of its own (few rows)
+@pytest.mark.parametrize("chunks,Lc,prefix,Hq,Hkv,text,pieces", [
+    (1, 1350, 7, 24, 8, (468,), True), (1, 672, 5, 48, 8, (33,), True), (3, 1134, 8, 48, 8, (0, 259, 800), True), (2, 1440, 1, 24, 8, (31, 65), True),
+    (1, 9360, 0, 24, 8, (400,), True), (1, 2310, 2, 24, 8, (97,), True), (4, 384, 4, 24, 8, (162, 1, 32, 64), False),
+    (4, 336, 3, 48, 8, (72, 5, 0, 96), False), (1, 240, 12, 24, 8, (45,), False)])
+def test_the_bits_of_the_calls_one_by_one(dev, chunks, Lc, prefix, Hq, Hkv, text, pieces):
+    g = torch.Generator(device=dev).manual_seed(Lc + Hq)
+    D, S, K, T = 128, chunks * Lc, (chunks + prefix) * Lc, sum(text)
+    rows = lambda *s: torch.nn.functional.layer_norm(torch.randn(*s, D, device=dev, generator=g), (D,)).bfloat16()
+    q = (rows(S, Hq).float() * (D ** -0.5 * 1.4426950408889634)).bfloat16()
+    cache = torch.randn(K, Hkv, 2 * D, device=dev, generator=g, dtype=torch.bfloat16)
+    cache[..., :D] = rows(K, Hkv)
+    q_ranges = torch.tensor([[i * Lc, (i + 1) * Lc] for i in range(chunks)], dtype=torch.int32, device=dev)
+    k_ranges = torch.tensor([[0, (prefix + i + 1) * Lc] for i in range(chunks)], dtype=torch.int32, device=dev)
+    qx = torch.randn(S, 2 * Hq, D, device=dev, generator=g, dtype=torch.bfloat16)[:, Hq:]  # a view of the projection
+    kv = torch.randn(T, Hkv, 2 * D, device=dev, generator=g, dtype=torch.bfloat16)
+    kv[..., :D] = rows(T, Hkv)
+    gamma, beta = torch.randn(D, device=dev, generator=g) * 0.1, torch.randn(D, device=dev, generator=g) * 0.1
+    cu_q = torch.arange(0, S + 1, Lc, dtype=torch.int32, device=dev)
+    cu_k = torch.tensor((0,) + text, dtype=torch.int32, device=dev).cumsum(0).to(torch.int32)
+    waves = attention_waves(Hq, Hkv, chunks, L.MAGI_RANGES_CU, Lc, 800)
+
+    def core(held):
+        return range_attention(q, cache[..., :D], cache[..., D:], q_ranges, k_ranges, Lc, K, return_lse=False, q_prescaled=True, score_bound=17.0,
+                               share_waves=True, held=held)[0]
+
+    def cross(held, split=True):
+        return range_attention(qx, kv[..., :D], kv[..., D:], cu_q, cu_k, Lc, 800, ranges_mode=L.MAGI_RANGES_CU, return_lse=False, score_bound=30.0,
+                               q_norm=(gamma, beta, 1e-6), share_waves=True, held=held, split_keys=split)[0]
+
+    n = M.lib().magi_launch_count
+    n0 = n()
+    want = core(None)
+    n1 = n()
+    want_x = cross(None, split=not pieces or bool(waves))  # (beside the merge the text's own items are whole)
+    assert n1 - n0 == 1 + int(pieces)
+    held, n0 = BegunCalls(), n()
+    got = core(held)
+    assert n() - n0 == 1 and len(held) == int(pieces)
+    got_x = cross(held)
+    launch_held(held)
+    assert not held and torch.equal(got, want) and torch.equal(got_x, want_x)
+    assert bool(torch.isfinite(got.float()).all()) and bool(torch.isfinite(got_x.float()).all())
+    if pieces:
+        assert n() - n0 == 2  # the core; its merge and the text
+        held = BegunCalls()
+        alone = core(held)
+        launch_held(held)  # (nothing beside it)
+        assert torch.equal(alone, want)
+
+
+def test_an_end_without_pieces_is_refused(dev):
+    q = torch.randn(64, 4, 128, device=dev, dtype=torch.bfloat16)
+    r = torch.tensor([[0, 64]], dtype=torch.int32, device=dev)
+    held = []
+    range_attention(q, q, q, r, r, 64, 64, held=held, return_lse=False)
+    with pytest.raises(M.MagiError):
+        launch_held([(held[0][0], None) + held[0][2:]])
