@@ -36,9 +36,19 @@ def _launch(dev: torch.device, fn, *args) -> int:
     return code
 
 
+_CUS = {}  # compute units by device index
+
+
+def _compute_units(device: torch.device) -> int:
+    n = _CUS.get(device.index)
+    if n is None:
+        n = _CUS[device.index] = torch.cuda.get_device_properties(device).multi_processor_count
+    return n
+
+
 class BegunCalls(list):
-    """A list for range_attention's `held` whose first call is launched at once but for what brings its pieces together, where it
-    leaves any (magi_attn_fwd_begin); launch_held() then launches that and the second call as one where it can."""
+    """A list for range_attention's `held` whose first call is begun at once (magi_attn_fwd_begin): done, or launched but for what brings its
+    pieces together, or held where nothing is in pieces; launch_held() then launches what is left and the second call as one where it can."""
 
     begin = True  # the next call is the first
 
@@ -257,6 +267,7 @@ def range_attention(
         workspace = torch.empty(4, dtype=torch.float32, device=q.device)  # (alive until the launches are enqueued)
     split, split_bytes, online = None, 0, False
     if (share_waves and split_keys and q.dtype is torch.bfloat16 and 0.0 < score_bound <= L.MAGI_SCORE_BOUND_MAX and not (q_tile_rows or bounded_mfma32)
+            and Hq * n * max_seqlen_q <= 64 * _compute_units(q.device)  # (two workgroups of 32 rows per CU: magi_attn_waves says no beyond)
             and attention_waves(Hq, Hkv, n, ranges_mode, max_seqlen_q, max_seqlen_k)):
         pass  # (keys shared without memory)
     elif split_keys and not static_scratch and max_seqlen_k >= 512 and (

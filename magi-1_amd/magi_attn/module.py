@@ -37,7 +37,7 @@ from . import _lib as L
 from .cache import Fp8KVCache, OffloadedKVCache
 from .functional import (_measuring_a_bound_pays, covered_by_launch, launch_fp8_attention, launch_quantize_fp8_split,
                          launch_small_projections_e4m3, launch_text_attention, range_count, split_memory)
-from .functional import BegunCalls, attention_waves, launch_held
+from .functional import BegunCalls, _compute_units, attention_waves, launch_held
 from .functional import launch_small_layer as launch_small_projections  # (named by the first of the launches it stands for)
 from .functional import (div_clamp_to, head_norm, layer_norm, layer_norm_div_clamp, pow2_scale_for, qk_prologue, qk_prologue_fp8, qkv_proj_prologue,
                          quantize_fp8_split,
@@ -242,14 +242,6 @@ def _plain_rows(x: torch.Tensor, w: torch.Tensor, heads: int) -> bool:
             and _plain_weight(w, heads, K, x.device))
 
 
-_CUS = {}  # compute units by device index
-
-
-def _compute_units(device: torch.device) -> int:
-    n = _CUS.get(device.index)
-    if n is None:
-        n = _CUS[device.index] = torch.cuda.get_device_properties(device).multi_processor_count
-    return n
 
 
 def _projects_in_one_launch(rows: int, heads: int, text_rows: int, text_heads: int, K: int, cus: int) -> bool:
@@ -335,7 +327,9 @@ class PerTensorQuantizedFp8Linear(torch.nn.Module):
         """The GEMM alone, on an input that is already div_clamp_to(input, self.input_scale)."""
         x2 = x8 if x8.dim() == 2 else x8.reshape(-1, self.in_features)
         w, scale_a, scale_b = _param(self, "weight"), _param(self, "input_scale").reshape(-1)[:1], _param(self, "weight_scale").reshape(-1)[:1]
-        head = _rows_ahead_e4m3(x2.shape[0], self.out_features, self.in_features, _compute_units(x2.device)) if x2.is_cuda else 0
+        head = 0
+        if x2.shape[0] * self.out_features >= 1 << 24 and x2.is_cuda:  # (a round of 256 CUs: four calls a layer that may wait for the host)
+            head = _rows_ahead_e4m3(x2.shape[0], self.out_features, self.in_features, _compute_units(x2.device))
         if head and (type(x2) in _PLAIN and type(w) in _PLAIN and x2.is_contiguous()
                      and not (torch.is_grad_enabled() and any(t.requires_grad for t in (x2, w, scale_a, scale_b)))):
             y = torch.empty((x2.shape[0], self.out_features), dtype=self.output_dtype, device=x2.device)
@@ -634,8 +628,8 @@ class FullyParallelAttention(torch.nn.Module):
         gk, bk = self.k_layernorm.gamma_beta_fp32()
         pro = dict(Hq=Hq, Hkv=Hkv, q_scale=qs_c, k_scale=ks_c, eps=self.eps, q_premul=self._q_premul)
         # The largest magnitudes of v's rows, from the prologue to the quantiser.  Not in chunks that a workgroup of the quantiser has in
-        # flight as a whole or nearly (400 rows 9.3 -> 7.3 us, 200 rows 7.1 -> 7.5, the host's time for it 1.5 us).
-        row_max = torch.empty((Hkv, S), dtype=torch.int16, device=dev) if min(Lc, S) > 256 else None
+        # flight as a whole or nearly (400 rows 9.3 -> 7.3 us, 200 rows 7.1 -> 7.5), nor in layers of few rows, which wait for the host (3 us).
+        row_max = torch.empty((Hkv, S), dtype=torch.int16, device=dev) if min(Lc, S) > 256 and S * Hq >= 64 * _compute_units(dev) else None
         if row_max is not None:
             pro.update(v_raw=v_raw, v_row_max=row_max)
         kw = dict(q_scale=self._const_scale_table(qs_c, n_chunks, Hq, dev), scale_chunk_tokens=Lc,
@@ -1249,8 +1243,9 @@ class FullyParallelAttention(torch.nn.Module):
         # of a layer of 3120 to 16200 rows and 24 or 48 heads (1233 -> 1197 us, 2215 -> 2183, 6414 -> 6264, 7670 -> 7426), 0.6 % of
         # 21600 rows x 2 chunks (29.7 -> 29.5 ms).  Between the two the core is issued as soon as it can be: its keys are in pieces that fill
         # the chip anyway, and the device would wait for what the host does for the text (one round and below: 0.90 to 1.04 of the speed);
-        # what brings the pieces together then goes beside the text: 30 drawn layers of 148 to 504 rows per CU 0.994 to 1.037 times as fast
-        # (2112 rows 390 -> 381 us, 2964 403 -> 389), the ones without pieces the same; from 44 to 83 rows per CU, which wait for the host, 0.985 to 1.026.
+        # what brings the pieces together then goes beside the text, and a core of whole 256-row items into the text's launch after all: 54 drawn
+        # layers of 128 to 512 rows per CU 0.994 to 1.097 times as fast (2112 rows 390 -> 381 us, 2964 403 -> 389; whole 3888 373 -> 340,
+        # 4176 505 -> 480), cores of other forms the same; from 44 to 83 rows per CU, which wait for the host, 0.985 to 1.026.
         held = None
         if core_bounded and cross_bounded and self.attention_dtype == "bf16" and _OWN_CROSS_FUSED.of(self):
             rows_per_cu = sq * Hq / _compute_units(hidden_states.device)  # of all heads
@@ -1263,10 +1258,11 @@ class FullyParallelAttention(torch.nn.Module):
                 held = []
             elif rows_per_cu >= 128:
                 held = BegunCalls()
-        elif cross_bounded and self.attention_dtype == "fp8" and _OWN_CROSS_FUSED.of(self) and _OWN_CORE_FP8.of(self):
+        elif (cross_bounded and self.attention_dtype == "fp8" and sq * Hq >= 64 * _compute_units(hidden_states.device) and _OWN_CROSS_FUSED.of(self)
+              and _OWN_CORE_FP8.of(self)):
             # (e4m3 core: the text beside it in a form of its own, attn_fwd_fp8_text.hip.  40 drawn layers from 122 rows per CU on 1.006 to 1.096
             # times as fast, 86400 rows 1.001; up to 71 rows per CU 0.997 to 1.004: their core and text do not fill the chip together)
-            held = [] if sq * Hq >= 64 * _compute_units(hidden_states.device) else None
+            held = []
         if proj_layout and bs == 1 and Hq % PROJ_GROUPS == 0:
             # (rows that no q range / cu_seqlens segment covers are left as allocated: the pipeline's ranges cover
             # every row, dit_model.py:220-222, 246; bf16, what the launches write, whatever hidden_states is)
@@ -1329,6 +1325,8 @@ class FullyParallelAttention(torch.nn.Module):
             finally:
                 if offloaded is not None:  # the persisted rows go back to the host behind the attention launch
                     offloaded.release(start, persisted)
+        if type(held) is BegunCalls and not held:  # (the core is done: nothing for the text to go with)
+            held = None
         if fused is not None:
             if cross_fused(cross_dst) is None:
                 self.cross_attention(mixed_qqkv, key_value_states, meta_args.cross_attn_params, get_xqkv, out=cross_dst)
