@@ -278,9 +278,9 @@ int magi_attn_fwd(const magi_attn_args* args, void* stream);
  * a split_workspace.  A refusal of the second is this call's, the first has been launched by then. */
 int magi_attn_fwd_two(const magi_attn_args* first, const magi_attn_args* second, void* stream);
 
-/* magi_attn_fwd in two halves.  begin returns MAGI_OK where the call is done, and 1 where it has left pieces in split_workspace (bounded
- * scores, keys of 256-row items shared): its output is then written by magi_attn_fwd_end with the same arguments on the same stream, and
- * split_workspace is kept until that.  end takes a second call with it (or NULL) that does not depend on the first's output, a text attention:
+/* magi_attn_fwd in two halves.  begin returns MAGI_OK where the call is done, and 1 where magi_attn_fwd_end, with the same arguments on the
+ * same stream, has to finish it (bounded scores, 256 rows per workgroup): it has left pieces in split_workspace, or not started yet.  Inputs and
+ * split_workspace are kept until that.  end takes a second call with it (or NULL) that does not depend on the first's output, a text attention:
  * in one launch where it has raw q (q_norm_gamma) and a score_bound, else behind it.  The same bits as two calls, the second without a
  * split_workspace.  A refusal of the second is this call's, the first is done all the same. */
 int magi_attn_fwd_begin(const magi_attn_args* args, void* stream);

@@ -400,9 +400,10 @@ int waves_plan(int Hq, int Hkv, int n_ranges, int ranges_mode, int max_seqlen_q,
 
 // held: where the call takes a form that may share a launch with another, its arguments instead of the launch; HELD is returned then
 constexpr int HELD = 1;
-// TEXT: beside something else, where every form of raw q with bounded scores is one, but those whose keys are shared.  BEGIN: items whose keys
-// are shared leave their pieces (HELD then), others are done; PIECES: the arguments that left them.
-enum Held { ALIKE, TEXT, BEGIN, PIECES };
+// TEXT: beside something else, where every form of raw q with bounded scores is one, but those whose keys are shared.  BEGIN: of 256-row items some
+// with shared keys leave their pieces, and a launch of whole ones waits for the second call (HELD both times); others are done; END: the
+// arguments of such a call.
+enum Held { ALIKE, TEXT, BEGIN, END };
 int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace, magi::AttnKernArgs* held = nullptr, Held how = ALIKE);
 // a held call by itself
 int launch_held(const magi::AttnKernArgs& a, void* stream);
@@ -534,11 +535,11 @@ int launch_held(const magi::AttnKernArgs& a, void* stream) {
   return launch_held(pair, 1, stream);
 }
 
-// a held text call as attn_text_rows.h takes it: 128-row tiles, whole items; false where it is another kind, or the grid would not fit
-bool text_in_128_rows(magi::AttnKernArgs& b, int max_seqlen_q) {
+// a held text call in tiles of 128 (as attn_text_rows.h takes it) or 256 rows, whole items; false where it is another kind, or the grid would not fit
+bool text_in_rows(magi::AttnKernArgs& b, int max_seqlen_q, int rows) {
   if (b.block_m == 32 || (double)b.Hq * b.n_ranges * max_seqlen_q >= 1e11) return false;
-  b.block_m = 128;
-  b.tiles_per_range = (max_seqlen_q + 127) / 128;
+  b.block_m = rows;
+  b.tiles_per_range = (max_seqlen_q + rows - 1) / rows;
   b.per_xcd = items_per_xcd(b.Hq, b.Hkv, b.n_ranges, b.tiles_per_range);
   b.split_from = UINT32_MAX;
   return true;
@@ -549,11 +550,13 @@ int attn_fwd_end(const magi_attn_args* first, const magi_attn_args* second, void
   const hipStream_t st = static_cast<hipStream_t>(stream);
   magi::AttnPairArgs pair;
   magi::AttnKernArgs &a = pair.job[0], &b = pair.job[1];
-  const int one = attn_fwd_impl(first, stream, first->workspace, &a, PIECES);
-  if (one != HELD) return one < 0 ? one : fail(MAGI_EINVAL, "magi_attn_fwd_end: an empty call leaves no pieces");
+  const int one = attn_fwd_impl(first, stream, first->workspace, &a, END);
+  if (one != HELD) return one < 0 ? one : fail(MAGI_EINVAL, "magi_attn_fwd_end: an empty call leaves nothing");
+  const bool whole = a.split_from >= a.per_xcd;
   const int two = second ? attn_fwd_impl(second, stream, second->workspace, &b, TEXT) : MAGI_OK;
-  const bool together = two == HELD && text_in_128_rows(b, second->max_seqlen_q);
-  const hipError_t e = together ? magi::launch_attn_text_merge(pair, st) : magi::launch_attn_fwd_bf16_merge(a, st);
+  const bool together = two == HELD && text_in_rows(b, second->max_seqlen_q, whole ? 256 : 128);
+  const hipError_t e = whole ? (together ? magi::launch_attn_fwd_bf16_x16_pair(pair, st) : magi::launch_attn_fwd_bf16_x16(a, st))
+                             : (together ? magi::launch_attn_text_merge(pair, st) : magi::launch_attn_fwd_bf16_merge(a, st));
   if (e != hipSuccess) return hip_fail(e, "magi_attn_fwd_end launch");
   count_launches(1);
   return together ? MAGI_OK : two == HELD ? launch_held(b, stream) : two;
@@ -568,7 +571,7 @@ int attn_fwd_two(const magi_attn_args* first, const magi_attn_args* second, void
     const hipStream_t st = static_cast<hipStream_t>(stream);
     magi::AttnKernArgs &a = pair.job[0], &b = pair.job[1];
     const int two = attn_fwd_impl(second, stream, second->workspace, &b, TEXT);
-    const bool together = two == HELD && text_in_128_rows(b, second->max_seqlen_q);
+    const bool together = two == HELD && text_in_rows(b, second->max_seqlen_q, 128);
     const hipError_t e = together ? magi::launch_attn_fwd_fp8_text(pair, st) : magi::launch_attn_fwd_fp8(a, st);
     if (e != hipSuccess) return hip_fail(e, "magi_attn_fwd launch");
     count_launches(1 + (a.split_from < a.per_xcd));
@@ -835,10 +838,10 @@ int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace, magi:
     }
     // (of the other forms the one of large launches: in the smaller ones the core's rows or keys are dealt out over the whole chip as it is)
     const bool x16 = bounded && a.block_m == 256 && !checked && !mfma32 && !auto_bound;
-    if (how == PIECES || (how == BEGIN && x16 && a.split_from < a.per_xcd)) {
-      if (!x16 || a.split_from >= a.per_xcd) return fail(MAGI_EINVAL, "magi_attn_fwd_end: not what magi_attn_fwd_begin left pieces of");
+    if (how == END || (how == BEGIN && x16 && !scale_q)) {
+      if (!x16 || scale_q) return fail(MAGI_EINVAL, "magi_attn_fwd_end: not a call that magi_attn_fwd_begin leaves anything of");
       *held = a;
-      if (how == PIECES) return HELD;
+      if (how == END || a.split_from >= a.per_xcd) return HELD;
       const hipError_t e = magi::launch_attn_fwd_bf16_x16(a, static_cast<hipStream_t>(stream), false);
       if (e != hipSuccess) return hip_fail(e, "magi_attn_fwd_begin launch");
       count_launches(1);

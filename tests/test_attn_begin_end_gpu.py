@@ -16,8 +16,10 @@ def dev():
 
 
 # keys in pieces: less than a round of 256-row workgroups, a round and a part; ranges of two lengths; text around the 32- and 64-key tiles, of
-# which one segment has none; a core without pieces (done by its first half); text in a launch of its own (few rows)
+# which one segment has none; 256-row items all whole ("whole": both in one launch; text of 128-row items, in pieces by itself); a core of another
+# form (done by its first half); text in a launch of its own (few rows)
 @pytest.mark.parametrize("chunks,Lc,prefix,Hq,Hkv,text,pieces", [
+    (3, 1296, 0, 24, 8, (660, 1, 129), "whole"), (4, 660, 0, 48, 8, (577, 0, 96, 32), "whole"), (3, 1392, 2, 24, 8, (732, 70, 31), "whole"),
     (1, 1350, 7, 24, 8, (468,), True), (1, 672, 5, 48, 8, (33,), True), (3, 1134, 8, 48, 8, (0, 259, 800), True), (2, 1440, 1, 24, 8, (31, 65), True),
     (1, 9360, 0, 24, 8, (400,), True), (1, 2310, 2, 24, 8, (97,), True), (4, 384, 4, 24, 8, (162, 1, 32, 64), False),
     (4, 336, 3, 48, 8, (72, 5, 0, 96), False), (1, 240, 12, 24, 8, (45,), False)])
@@ -51,16 +53,16 @@ def test_the_bits_of_the_calls_one_by_one(dev, chunks, Lc, prefix, Hq, Hkv, text
     want = core(None)
     n1 = n()
     want_x = cross(None, split=not pieces or bool(waves))  # (beside the merge the text's own items are whole)
-    assert n1 - n0 == 1 + int(pieces)
+    assert n1 - n0 == (2 if pieces is True else 1)
     held, n0 = BegunCalls(), n()
     got = core(held)
-    assert n() - n0 == 1 and len(held) == int(pieces)
+    assert n() - n0 == int(pieces != "whole") and len(held) == int(bool(pieces))
     got_x = cross(held)
     launch_held(held)
     assert not held and torch.equal(got, want) and torch.equal(got_x, want_x)
     assert bool(torch.isfinite(got.float()).all()) and bool(torch.isfinite(got_x.float()).all())
     if pieces:
-        assert n() - n0 == 2  # the core; its merge and the text
+        assert n() - n0 == (1 if pieces == "whole" else 2)  # (the core;) its merge, or all of it, and the text
         held = BegunCalls()
         alone = core(held)
         launch_held(held)  # (nothing beside it)
