@@ -76,3 +76,41 @@ def test_an_end_without_pieces_is_refused(dev):
     range_attention(q, q, q, r, r, 64, 64, held=held, return_lse=False)
     with pytest.raises(M.MagiError):
         launch_held([(held[0][0], None) + held[0][2:]])
+
+
+@pytest.mark.parametrize("chunks,Lc,prefix,text", [(1, 1350, 2, (468,)), (3, 1296, 0, (660, 1, 129))])  # in pieces; whole items
+def test_captured_in_a_graph(dev, chunks, Lc, prefix, text):
+    g = torch.Generator(device=dev).manual_seed(Lc)
+    Hq, Hkv, D, S, K, T = 24, 8, 128, chunks * Lc, (chunks + prefix) * Lc, sum(text)
+    norm = lambda t: torch.nn.functional.layer_norm(t.float(), (D,))
+    draw = lambda *s: torch.randn(*s, D, device=dev, generator=g, dtype=torch.bfloat16)
+    q, qx, v, vx = draw(S, Hq), draw(S, Hq), draw(K, Hkv), draw(T, Hkv)
+    k, kx = norm(draw(K, Hkv)).bfloat16(), norm(draw(T, Hkv)).bfloat16()
+    q_ranges = torch.tensor([[i * Lc, (i + 1) * Lc] for i in range(chunks)], dtype=torch.int32, device=dev)
+    k_ranges = torch.tensor([[0, (prefix + i + 1) * Lc] for i in range(chunks)], dtype=torch.int32, device=dev)
+    gamma = torch.randn(D, device=dev, generator=g) * 0.1
+    cu_q = torch.arange(0, S + 1, Lc, dtype=torch.int32, device=dev)
+    cu_k = torch.tensor((0,) + text, dtype=torch.int32, device=dev).cumsum(0).to(torch.int32)
+
+    def both():
+        held = BegunCalls()
+        a, _ = range_attention(q, k, v, q_ranges, k_ranges, Lc, K, return_lse=False, q_prescaled=True, score_bound=17.0, held=held)
+        b, _ = range_attention(qx, kx, vx, cu_q, cu_k, Lc, 800, ranges_mode=L.MAGI_RANGES_CU, return_lse=False, score_bound=30.0,
+                               q_norm=(gamma, None, 1e-6), held=held)
+        launch_held(held)
+        return a, b
+
+    fill = lambda: (q.copy_(norm(draw(S, Hq)) * (D ** -0.5 * 1.4426950408889634)), qx.copy_(draw(S, Hq)))
+    fill()
+    both()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = both()
+    for _ in range(3):
+        fill()
+        want = both()
+        graph.replay()
+        torch.cuda.synchronize()
+        for x, y in zip(out, want):
+            assert torch.equal(x, y)
