@@ -628,8 +628,9 @@ class FullyParallelAttention(torch.nn.Module):
         gk, bk = self.k_layernorm.gamma_beta_fp32()
         pro = dict(Hq=Hq, Hkv=Hkv, q_scale=qs_c, k_scale=ks_c, eps=self.eps, q_premul=self._q_premul)
         # The largest magnitudes of v's rows, from the prologue to the quantiser.  Not in chunks that a workgroup of the quantiser has in
-        # flight as a whole or nearly (400 rows 9.3 -> 7.3 us, 200 rows 7.1 -> 7.5), nor in layers of few rows, which wait for the host (3 us).
-        row_max = torch.empty((Hkv, S), dtype=torch.int16, device=dev) if min(Lc, S) > 256 and S * Hq >= 64 * _compute_units(dev) else None
+        # flight as a whole or nearly (400 rows 9.3 -> 7.3 us, 200 rows 7.1 -> 7.5), nor below 256 rows per CU (of all heads), where the two launches
+        # gain 2 to 7 us together and layers with e4m3 products wait for the host, which pays 3 (1536 rows x 24 heads 264 / 270).
+        row_max = torch.empty((Hkv, S), dtype=torch.int16, device=dev) if min(Lc, S) > 256 and S * Hq >= 256 * _compute_units(dev) else None
         if row_max is not None:
             pro.update(v_raw=v_raw, v_row_max=row_max)
         kw = dict(q_scale=self._const_scale_table(qs_c, n_chunks, Hq, dev), scale_chunk_tokens=Lc,
