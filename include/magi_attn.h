@@ -274,14 +274,16 @@ int magi_attn_fwd(const magi_attn_args* args, void* stream);
 /* magi_attn_fwd of two calls that do not depend on each other and write different outputs (a layer's core and text attention): in one
  * launch where both take the form of MAGI_ATTN_SHARE_WAVES, or both 256 rows per workgroup (magi_attn_tile_rows) with q pre-scaled or raw,
  * a score_bound and no keys of the second shared, or the first has e4m3 rows with MAGI_ATTN_FP8_POW2_PRESCALED and the second raw q
- * (q_norm_gamma) and a score_bound; else one after the other.  The same bits as two calls, the second of them, behind e4m3 rows, without
- * a split_workspace.  A refusal of the second is this call's, the first has been launched by then. */
+ * (q_norm_gamma), a score_bound and no keys shared among 128-row workgroups; else the second behind the first, both of which may have the same
+ * split_workspace.  The same bits as two calls, but that a second one in a launch with e4m3 rows makes no use of its split_workspace.  A
+ * refusal of the second is this call's, the first has been launched by then. */
 int magi_attn_fwd_two(const magi_attn_args* first, const magi_attn_args* second, void* stream);
 
 /* magi_attn_fwd in two halves.  begin returns MAGI_OK where the call is done, and 1 where magi_attn_fwd_end, with the same arguments on the
  * same stream, has to finish it (bounded scores, 256 rows per workgroup): it has left pieces in split_workspace, or not started yet.  Inputs and
- * split_workspace are kept until that.  end takes a second call with it (or NULL) that does not depend on the first's output, a text attention:
- * in one launch where it has raw q (q_norm_gamma) and a score_bound, else behind it.  The same bits as two calls, the second without a
+ * split_workspace are kept until that.  end takes a second call with it (or NULL) that does not depend on the first's output, a text attention: in
+ * one launch where it has raw q (q_norm_gamma), a score_bound and no keys shared among 128-row workgroups or by wavefronts, else behind all of the
+ * first, whose split_workspace it may have too.  The same bits as two calls, but that a second one in one launch makes no use of its
  * split_workspace.  A refusal of the second is this call's, the first is done all the same. */
 int magi_attn_fwd_begin(const magi_attn_args* args, void* stream);
 int magi_attn_fwd_end(const magi_attn_args* first, const magi_attn_args* second, void* stream);

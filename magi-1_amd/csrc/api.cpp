@@ -398,13 +398,14 @@ int waves_plan(int Hq, int Hkv, int n_ranges, int ranges_mode, int max_seqlen_q,
   return max_seqlen_k <= 4096 ? 4 : 0;
 }
 
-// held: where the call takes a form that may share a launch with another, its arguments instead of the launch; HELD is returned then
-constexpr int HELD = 1;
-// TEXT: beside something else, where every form of raw q with bounded scores is one, but those whose keys are shared.  BEGIN: of 256-row items some
-// with shared keys leave their pieces, and a launch of whole ones waits for the second call (HELD both times); others are done; END: the
-// arguments of such a call.
-enum Held { ALIKE, TEXT, BEGIN, END };
-int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace, magi::AttnKernArgs* held = nullptr, Held how = ALIKE);
+// HELD: the call takes a form that may share a launch with another, `held` has its arguments and nothing is launched; ALONE: it does not, and
+// nothing is launched either.  FIRST, SECOND of two alike: wavefronts that share keys, or 256-row workgroups; a first call of another form is
+// launched (MAGI_OK), a second one is ALONE, as it must not run ahead of the first.  TEXT, a second call beside something else: every form of raw q
+// with bounded scores, but those whose keys are shared.  BEGIN: of 256-row items some with shared keys leave their pieces, and a launch of whole
+// ones waits for the second call (HELD both times); others are launched; END: the arguments of such a call.
+constexpr int HELD = 1, ALONE = 2;
+enum Held { NOW, FIRST, SECOND, TEXT, BEGIN, END };
+int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace, magi::AttnKernArgs* held = nullptr, Held how = NOW);
 // a held call by itself
 int launch_held(const magi::AttnKernArgs& a, void* stream);
 int attn_fwd_two(const magi_attn_args* first, const magi_attn_args* second, void* stream);
@@ -545,6 +546,11 @@ bool text_in_rows(magi::AttnKernArgs& b, int max_seqlen_q, int rows) {
   return true;
 }
 
+// a second call that did not go with the first, which has been launched: `two` is what attn_fwd_impl returned for it, b its arguments where HELD
+int launch_behind(int two, const magi::AttnKernArgs& b, const magi_attn_args* second, void* stream) {
+  return two == HELD ? launch_held(b, stream) : two == ALONE ? attn_fwd_impl(second, stream, second->workspace) : two;
+}
+
 // the second half of magi_attn_fwd_begin(first), beside second
 int attn_fwd_end(const magi_attn_args* first, const magi_attn_args* second, void* stream) {
   const hipStream_t st = static_cast<hipStream_t>(stream);
@@ -559,30 +565,28 @@ int attn_fwd_end(const magi_attn_args* first, const magi_attn_args* second, void
                              : (together ? magi::launch_attn_text_merge(pair, st) : magi::launch_attn_fwd_bf16_merge(a, st));
   if (e != hipSuccess) return hip_fail(e, "magi_attn_fwd_end launch");
   count_launches(1);
-  return together ? MAGI_OK : two == HELD ? launch_held(b, stream) : two;
+  return together ? MAGI_OK : launch_behind(two, b, second, stream);
 }
 
 // first, then second, which do not depend on each other: in one launch where both take the form for it
 int attn_fwd_two(const magi_attn_args* first, const magi_attn_args* second, void* stream) {
   magi::AttnPairArgs pair;
-  const int one = attn_fwd_impl(first, stream, first->workspace, &pair.job[0]);
+  magi::AttnKernArgs &a = pair.job[0], &b = pair.job[1];
+  const int one = attn_fwd_impl(first, stream, first->workspace, &a, FIRST);
   if (one != HELD) return one < 0 ? one : attn_fwd_impl(second, stream, second->workspace);
   if (first->dtype == MAGI_DTYPE_FP8_E4M3) {
     const hipStream_t st = static_cast<hipStream_t>(stream);
-    magi::AttnKernArgs &a = pair.job[0], &b = pair.job[1];
     const int two = attn_fwd_impl(second, stream, second->workspace, &b, TEXT);
     const bool together = two == HELD && text_in_rows(b, second->max_seqlen_q, 128);
     const hipError_t e = together ? magi::launch_attn_fwd_fp8_text(pair, st) : magi::launch_attn_fwd_fp8(a, st);
     if (e != hipSuccess) return hip_fail(e, "magi_attn_fwd launch");
     count_launches(1 + (a.split_from < a.per_xcd));
-    return together || two != HELD ? (two < 0 ? two : MAGI_OK) : launch_held(b, stream);
+    return together ? MAGI_OK : launch_behind(two, b, second, stream);
   }
-  const bool rows8 = second->dtype == MAGI_DTYPE_FP8_E4M3;  // (shares a launch as the first of the two only)
-  const int two = attn_fwd_impl(second, stream, second->workspace, rows8 ? nullptr : &pair.job[1]);
-  const magi::AttnKernArgs &a = pair.job[0], &b = pair.job[1];
+  const int two = attn_fwd_impl(second, stream, second->workspace, &b, SECOND);
   if (two == HELD && a.block_m == b.block_m && (b.block_m == 32 || b.split_from >= b.per_xcd)) return launch_held(pair, 2, stream);
   const int rc = launch_held(a, stream);
-  return rc < 0 ? rc : two == HELD ? launch_held(b, stream) : two;
+  return rc < 0 ? rc : launch_behind(two, b, second, stream);
 }
 
 int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace, magi::AttnKernArgs* held, Held how) {
@@ -838,20 +842,22 @@ int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace, magi:
     }
     // (of the other forms the one of large launches: in the smaller ones the core's rows or keys are dealt out over the whole chip as it is)
     const bool x16 = bounded && a.block_m == 256 && !checked && !mfma32 && !auto_bound;
-    if (how == END || (how == BEGIN && x16 && !scale_q)) {
-      if (!x16 || scale_q) return fail(MAGI_EINVAL, "magi_attn_fwd_end: not a call that magi_attn_fwd_begin leaves anything of");
+    const bool plain = x16 && !scale_q;
+    // (raw q is bounded, in 128- or 256-row workgroups)
+    const bool hold = how == FIRST  ? plain || (fp8 && (p->flags & MAGI_ATTN_FP8_POW2_PRESCALED))
+                      : how == TEXT ? q_norm && a.share_pieces <= 1
+                                    : how != NOW && plain;
+    if (hold) {
       *held = a;
-      if (how == END || a.split_from >= a.per_xcd) return HELD;
-      const hipError_t e = magi::launch_attn_fwd_bf16_x16(a, static_cast<hipStream_t>(stream), false);
-      if (e != hipSuccess) return hip_fail(e, "magi_attn_fwd_begin launch");
-      count_launches(1);
+      if (how == BEGIN && a.split_from < a.per_xcd) {
+        const hipError_t e = magi::launch_attn_fwd_bf16_x16(a, static_cast<hipStream_t>(stream), false);
+        if (e != hipSuccess) return hip_fail(e, "magi_attn_fwd_begin launch");
+        count_launches(1);
+      }
       return HELD;
     }
-    if (how == ALIKE ? held && ((x16 && !scale_q) || (fp8 && (p->flags & MAGI_ATTN_FP8_POW2_PRESCALED)))
-                     : how == TEXT && q_norm && (x16 || (bounded && a.block_m == 128 && a.share_pieces <= 1 && !checked && !auto_bound))) {
-      *held = a;
-      return HELD;
-    }
+    if (how == END) return fail(MAGI_EINVAL, "magi_attn_fwd_end: not a call that magi_attn_fwd_begin leaves anything of");
+    if (how == SECOND || how == TEXT) return ALONE;
     hipError_t e;
     if (p->dtype != MAGI_DTYPE_BF16)
       e = magi::launch_attn_fwd_fp8(a, static_cast<hipStream_t>(stream));
@@ -875,6 +881,8 @@ int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace, magi:
     return launch(true);
   }
   if (!auto_bound) return launch(promised);
+  if (how == SECOND || how == TEXT) return ALONE;
+  if (how == END) return fail(MAGI_EINVAL, "magi_attn_fwd_end: not a call that magi_attn_fwd_begin leaves anything of");
 
   // No promise about the scores: measure one.  Two streaming passes leave the largest squared length of a q row and
   // of a k row in the workspace (|q . k| <= |q| |k|); both attention kernels are launched behind them, each tests

@@ -69,6 +69,34 @@ def test_the_bits_of_the_calls_one_by_one(dev, chunks, Lc, prefix, Hq, Hkv, text
         assert torch.equal(alone, want)
 
 
+# a second call of 128-row items whose keys are shared; one of the online softmax; one that joins the merge
+@pytest.mark.parametrize("rows,keys,raw", [(480, 4000, True), (480, 4000, False), (2112, 400, True)])
+def test_one_scratch_buffer_for_both(dev, rows, keys, raw):
+    """A caller that keeps one split_workspace per stream: the second call may not leave its pieces there ahead of the first one's merge."""
+    g = torch.Generator(device=dev).manual_seed(rows)
+    D, Hq, Hkv, S, K = 128, 24, 8, 2112, 14784
+    draw = lambda *s: torch.randn(*s, D, device=dev, generator=g, dtype=torch.bfloat16)
+    norm = lambda t: torch.nn.functional.layer_norm(t.float(), (D,))
+    q, k, v = (norm(draw(S, Hq)) * (D ** -0.5 * 1.4426950408889634)).bfloat16(), norm(draw(K, Hkv)).bfloat16(), draw(K, Hkv)
+    qx, kx, vx = draw(rows, Hq), norm(draw(keys, Hkv)).bfloat16(), draw(keys, Hkv)
+    ranges = lambda n: torch.tensor([[0, n]], dtype=torch.int32, device=dev)
+    more = dict(score_bound=30.0, q_norm=(torch.randn(D, device=dev, generator=g) * 0.1, None, 1e-6)) if raw else {}
+    core = lambda held: range_attention(q, k, v, ranges(S), ranges(K), S, K, return_lse=False, q_prescaled=True, score_bound=17.0, held=held)[0]
+    cross = lambda held: range_attention(qx, kx, vx, ranges(rows), ranges(keys), rows, keys, return_lse=False, held=held, **more)[0]
+    want, want_x = core(None), cross(None)
+    held = []
+    got, got_x = core(held), cross(held)
+    calls = [L.AttnArgs.from_buffer_copy(c[2]) for c in held]
+    assert calls[0].split_workspace and (calls[1].split_workspace or rows > 480)
+    scratch = torch.empty(max(c.split_workspace_bytes for c in calls), dtype=torch.uint8, device=dev)
+    for c in calls:
+        c.split_workspace, c.split_workspace_bytes = scratch.data_ptr(), scratch.numel()
+    stream = torch.cuda.current_stream().cuda_stream
+    lib = L.lib()
+    assert lib.magi_attn_fwd_begin(calls[0], stream) == 1 and lib.magi_attn_fwd_end(calls[0], calls[1], stream) == 0
+    assert torch.equal(got, want) and torch.equal(got_x, want_x)
+
+
 def test_an_end_without_pieces_is_refused(dev):
     q = torch.randn(64, 4, 128, device=dev, dtype=torch.bfloat16)
     r = torch.tensor([[0, 64]], dtype=torch.int32, device=dev)
