@@ -589,6 +589,8 @@ int attn_fwd_two(const magi_attn_args* first, const magi_attn_args* second, void
   return rc < 0 ? rc : launch_behind(two, b, second, stream);
 }
 
+int not_begun() { return fail(MAGI_EINVAL, "magi_attn_fwd_end: not a call that magi_attn_fwd_begin leaves anything of"); }
+
 int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace, magi::AttnKernArgs* held, Held how) {
   if (p->D != 128) return fail(MAGI_ENOSYS, "magi_attn_fwd: head_dim %d not implemented (128 only)", p->D);
   if (p->dtype != MAGI_DTYPE_BF16 && p->dtype != MAGI_DTYPE_FP8_E4M3)
@@ -815,6 +817,7 @@ int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace, magi:
     };
     a.share_pieces = 1;
     if (a.waves) {
+      if (how == END) return not_begun();
       if (!held || how == BEGIN) return launch_held(a, stream);
       *held = a;
       return HELD;
@@ -856,7 +859,7 @@ int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace, magi:
       }
       return HELD;
     }
-    if (how == END) return fail(MAGI_EINVAL, "magi_attn_fwd_end: not a call that magi_attn_fwd_begin leaves anything of");
+    if (how == END) return not_begun();
     if (how == SECOND || how == TEXT) return ALONE;
     hipError_t e;
     if (p->dtype != MAGI_DTYPE_BF16)
@@ -882,7 +885,7 @@ int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace, magi:
   }
   if (!auto_bound) return launch(promised);
   if (how == SECOND || how == TEXT) return ALONE;
-  if (how == END) return fail(MAGI_EINVAL, "magi_attn_fwd_end: not a call that magi_attn_fwd_begin leaves anything of");
+  if (how == END) return not_begun();
 
   // No promise about the scores: measure one.  Two streaming passes leave the largest squared length of a q row and
   // of a k row in the workspace (|q . k| <= |q| |k|); both attention kernels are launched behind them, each tests

@@ -122,3 +122,17 @@ def test_a_refused_second_call_leaves_the_first_done(api):
         assert call(C.byref(first), C.byref(second), None) < 0 and b"head_dim" in api.magi_last_error()
         got = _launches(api)
         assert len(got) == 1 and [out for out, _, _ in got[0][1]] == [0x100]
+
+
+@pytest.mark.parametrize("kind,rows,keys", [("as it is, wavefronts", 96, 400), ("raw, wavefronts", 96, 400), ("as it is", 480, 4000), ("unscaled", 2112, 14784),
+                                            ("online", 2112, 14784), ("measured", 2112, 14784), ("checked", 2112, 14784), ("e4m3", 2112, 14784), ("raw", 0, 400)])
+def test_an_end_of_what_was_not_begun_is_refused(api, kind, rows, keys):
+    """A form that the first half launches as a whole: the second half launches nothing of it, and nothing beside it."""
+    first, second = _call(0x100, rows, keys, kind.split(",")[0]), _call(0x200, 480, 400, "raw")
+    if "wavefronts" in kind:
+        first.flags |= L.MAGI_ATTN_SHARE_WAVES
+    assert api.magi_attn_fwd_begin(C.byref(first), None) == 0
+    _launches(api)
+    for beside in (None, C.byref(second)):
+        assert api.magi_attn_fwd_end(C.byref(first), beside, None) == -22 and b"magi_attn_fwd_end" in api.magi_last_error()
+    assert not _launches(api)
