@@ -536,12 +536,20 @@ int launch_held(const magi::AttnKernArgs& a, void* stream) {
   return launch_held(pair, 1, stream);
 }
 
-// a held text call in tiles of 128 (as attn_text_rows.h takes it) or 256 rows, whole items; false where it is another kind, or the grid would not fit
-bool text_in_rows(magi::AttnKernArgs& b, int max_seqlen_q, int rows) {
-  if (b.block_m == 32 || (double)b.Hq * b.n_ranges * max_seqlen_q >= 1e11) return false;
+// Whether so many workgroups of 256 threads are a launch: HIP takes less than 2^32 threads.  (Two calls may fit apart and not together: ranges of
+// a long max_seqlen_q have most of their tiles beyond their rows.)
+bool fits(uint64_t workgroups) { return workgroups * 256 <= UINT32_MAX; }
+
+// a held text call in tiles of 128 (as attn_text_rows.h takes it) or 256 rows, whole items, beside so many other workgroups; false, and b as it was,
+// where it is another kind or the launch would not fit
+bool text_in_rows(magi::AttnKernArgs& b, int max_seqlen_q, int rows, uint64_t others) {
+  const int tiles = max_seqlen_q / rows + (max_seqlen_q % rows != 0);
+  if (b.block_m == 32 || (double)b.Hq * b.n_ranges * tiles > 2.0e9) return false;
+  const unsigned per_xcd = items_per_xcd(b.Hq, b.Hkv, b.n_ranges, tiles);
+  if (!fits(others + 8ull * per_xcd)) return false;
   b.block_m = rows;
-  b.tiles_per_range = (max_seqlen_q + rows - 1) / rows;
-  b.per_xcd = items_per_xcd(b.Hq, b.Hkv, b.n_ranges, b.tiles_per_range);
+  b.tiles_per_range = tiles;
+  b.per_xcd = per_xcd;
   b.split_from = UINT32_MAX;
   return true;
 }
@@ -560,7 +568,9 @@ int attn_fwd_end(const magi_attn_args* first, const magi_attn_args* second, void
   if (one != HELD) return one < 0 ? one : fail(MAGI_EINVAL, "magi_attn_fwd_end: an empty call leaves nothing");
   const bool whole = a.split_from >= a.per_xcd;
   const int two = second ? attn_fwd_impl(second, stream, second->workspace, &b, TEXT) : MAGI_OK;
-  const bool together = two == HELD && text_in_rows(b, second->max_seqlen_q, whole ? 256 : 128);
+  // (beside the workgroups of the first, or the four of each of its items that bring the pieces together)
+  const uint64_t others = whole ? split_grid(a) : 32ull * split_items(a);
+  const bool together = two == HELD && text_in_rows(b, second->max_seqlen_q, whole ? 256 : 128, others);
   const hipError_t e = whole ? (together ? magi::launch_attn_fwd_bf16_x16_pair(pair, st) : magi::launch_attn_fwd_bf16_x16(a, st))
                              : (together ? magi::launch_attn_text_merge(pair, st) : magi::launch_attn_fwd_bf16_merge(a, st));
   if (e != hipSuccess) return hip_fail(e, "magi_attn_fwd_end launch");
@@ -577,14 +587,16 @@ int attn_fwd_two(const magi_attn_args* first, const magi_attn_args* second, void
   if (first->dtype == MAGI_DTYPE_FP8_E4M3) {
     const hipStream_t st = static_cast<hipStream_t>(stream);
     const int two = attn_fwd_impl(second, stream, second->workspace, &b, TEXT);
-    const bool together = two == HELD && text_in_rows(b, second->max_seqlen_q, 128);
+    const bool together = two == HELD && text_in_rows(b, second->max_seqlen_q, 128, split_grid(a));
     const hipError_t e = together ? magi::launch_attn_fwd_fp8_text(pair, st) : magi::launch_attn_fwd_fp8(a, st);
     if (e != hipSuccess) return hip_fail(e, "magi_attn_fwd launch");
     count_launches(1 + (a.split_from < a.per_xcd));
     return together ? MAGI_OK : launch_behind(two, b, second, stream);
   }
   const int two = attn_fwd_impl(second, stream, second->workspace, &b, SECOND);
-  if (two == HELD && a.block_m == b.block_m && (b.block_m == 32 || b.split_from >= b.per_xcd)) return launch_held(pair, 2, stream);
+  // (of 32 rows there is at most a workgroup or two per CU)
+  if (two == HELD && a.block_m == b.block_m && (b.block_m == 32 || (b.split_from >= b.per_xcd && fits(split_grid(a) + 8ull * b.per_xcd))))
+    return launch_held(pair, 2, stream);
   const int rc = launch_held(a, stream);
   return rc < 0 ? rc : launch_behind(two, b, second, stream);
 }

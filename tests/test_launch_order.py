@@ -136,3 +136,33 @@ def test_an_end_of_what_was_not_begun_is_refused(api, kind, rows, keys):
     for beside in (None, C.byref(second)):
         assert api.magi_attn_fwd_end(C.byref(first), beside, None) == -22 and b"magi_attn_fwd_end" in api.magi_last_error()
     assert not _launches(api)
+
+
+@pytest.mark.parametrize("first,entry", [(("as it is", 5400, 7000, 1), "two"), (("e4m3", 5400, 9000, 1), "two"), (("as it is", 1296, 3888, 3), "end"),
+                                         (("as it is", 2112, 14784, 1), "end")])
+def test_launches_that_fit_apart_only_are_launched_apart(api, first, entry):
+    """HIP takes less than 2^32 threads in a launch: 16777215 workgroups of 256.  A long max_seqlen_q, whose tiles lie beyond the rows mostly, is
+    just within that by itself (with e4m3 rows and beside pieces in tiles of 128 rows, twice as many), and not with the first call."""
+    kind, rows, keys, n = first
+    most = 16777215
+    calls = [_call(0x100, rows, keys, kind, n), _call(0x200, 4096, 400, "raw")]
+
+    def launches(max_q):
+        calls[1].max_seqlen_q = max_q
+        if entry == "end":
+            assert api.magi_attn_fwd_begin(C.byref(calls[0]), None) == 1
+        _launches(api)
+        assert getattr(api, "magi_attn_fwd_" + entry)(C.byref(calls[0]), C.byref(calls[1]), None) == 0
+        got = _launches(api)
+        assert all(w <= most for _, _, w in got) and sum(len(jobs) for _, jobs, _ in got) == 2
+        return got
+
+    per_tile = 24  # (workgroups of all heads)
+    tile = 128 if kind == "e4m3" or rows == 2112 else 256
+    whole = launches(256 * (most // per_tile - 100))
+    assert len(whole) == (2 if tile == 128 else 1)
+    others = launches(256 * 1024)[0][2] - 1024 * (256 // tile) * per_tile  # of the first call
+    edge = (most - others) // per_tile
+    got = launches(tile * edge)
+    assert len(got) == 1 and got[0][2] == others + edge * per_tile
+    assert len(launches(tile * edge + 1)) == 2
