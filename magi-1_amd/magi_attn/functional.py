@@ -319,17 +319,13 @@ def range_attention(
 def launch_held(calls: list) -> None:
     """The calls that range_attention(held=calls) left, on the current stream: two that do not depend on each other in one launch where their
     sizes are for it (magi_attn_fwd_two).  Empties the list."""
-    if calls and calls[0][1] is None:  # (begun)
-        alone = len(calls) == 1 or calls[0][0] != calls[1][0]
-        _launch(calls[0][0], L.packed_pair("magi_attn_fwd_end").fn, calls[0][2], None if alone else calls[1][2])
-        if alone:
-            for dev, fn, args, _ in calls[1:]:
-                _launch(dev, fn, args)
-    elif len(calls) == 2 and calls[0][0] == calls[1][0]:
-        _launch(calls[0][0], L.packed_pair("magi_attn_fwd_two").fn, calls[0][2], calls[1][2])
-    else:
-        for dev, fn, args, _ in calls:
-            _launch(dev, fn, args)
+    begun, rest = bool(calls) and calls[0][1] is None, calls
+    pair = (len(calls) == 2 or (begun and len(calls) > 2)) and calls[0][0] == calls[1][0]
+    if begun or pair:
+        _launch(calls[0][0], L.packed_pair("magi_attn_fwd_end" if begun else "magi_attn_fwd_two").fn, calls[0][2], calls[1][2] if pair else None)
+        rest = calls[2 if pair else 1:]
+    for dev, fn, args, _ in rest:
+        _launch(dev, fn, args)
     calls.clear()
 
 

@@ -405,6 +405,23 @@ def test_projection_rows_are_cut_only_where_a_round_of_tiles_is_left_partly_empt
         assert _rows_ahead(9360, cols_, depth, cus) == 0
 
 
+@pytest.mark.parametrize("begun", [False, True])
+@pytest.mark.parametrize("devices", ["0", "00", "01", "000", "010", "0000"])
+def test_every_held_call_is_launched_once(monkeypatch, begun, devices):
+    from magi_attn import functional as F
+
+    done = []
+    monkeypatch.setattr(F, "_launch", lambda dev, fn, *args: done.append((dev, fn, args)))
+    names = [f"call {i}" for i in range(len(devices))]
+    held = [(dev, None if begun and i == 0 else "fwd", name, ()) for i, (dev, name) in enumerate(zip(devices, names))]
+    F.launch_held(held)
+    assert not held and [a for _, _, args in done for a in args if a] == names  # each once, in their order
+    together = [args for _, _, args in done if len(args) == 2 and args[1]]
+    assert together == ([tuple(names[:2])] if devices[:2] == "00" and (begun or len(devices) == 2) else [])
+    for dev, _, args in done:
+        assert all(devices[names.index(a)] == dev for a in args if a)
+
+
 @pytest.mark.parametrize("cols,whole", [(1024, 16384), (3072, 16384), (6144, 8192), (8192, 2048), (256, 65536), (5120, 16384)])
 def test_e4m3_rows_are_cut_behind_rounds_that_are_whole_to_the_last_tile(cols, whole):
     from magi_attn.module import _rows_ahead_e4m3
