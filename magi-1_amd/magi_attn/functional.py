@@ -186,7 +186,7 @@ def range_attention(
     auto_bound also on which of the two kernels the longest rows of the whole call select.
     share_waves (with split_keys, a score_bound and max_seqlen_k): in launches of a few rows the wavefronts of a workgroup may share the keys of
     a row, MAGI_ATTN_SHARE_WAVES.
-    held: the call is appended here instead of launched; launch_held() then launches one or two of them.
+    held: the call is appended here instead of launched; launch_held() then launches what is in it, two of them as one where it can.
     q may be [batch, rows, Hq, D] with any batch stride (batch of activations laid out [position, batch, ...]): its rows
     count as batch * rows tokens for the ranges, out is (or comes back as) a tensor of q's shape, by default
     [rows, batch, Hq, D] transposed.  Needs a score_bound (math.inf: the online softmax).
@@ -304,10 +304,12 @@ def range_attention(
         0.0 if softmax_scale is None else float(softmax_scale), flags, group_heads, o_stride_g,
         min(float(score_bound), 3e38), int(q_tile_rows), _ptr(gamma), _ptr(beta), norm_eps, norm_kind, _ptr(k2_scale),
         _ptr(v2_scale), _ptr(workspace), batch_rows, q_stride_b, o_stride_b, _ptr(split), split_bytes)
+    begin = type(held) is BegunCalls and held.begin
+    if begin:
+        held.begin = False
     if held is None:
         _launch(q.device, call.fn, args)
-    elif type(held) is BegunCalls and held.begin:
-        held.begin = False
+    elif begin and not static_scratch:
         if _launch(q.device, L.packed("magi_attn_fwd_begin", L.AttnArgs).fn, args):
             held.append((q.device, None, args, (q, k, v, k2, v2, q_ranges, k_ranges, gamma, beta, split, out, lse)))
     else:  # (with everything it reads and writes)
@@ -320,7 +322,10 @@ def launch_held(calls: list) -> None:
     """The calls that range_attention(held=calls) left, on the current stream: two that do not depend on each other in one launch where their
     sizes are for it (magi_attn_fwd_two).  Empties the list."""
     begun, rest = bool(calls) and calls[0][1] is None, calls
-    pair = (len(calls) == 2 or (begun and len(calls) > 2)) and calls[0][0] == calls[1][0]
+    # (calls with static scratch memory have an entry point of their own: the ones for two would ask them for a workspace)
+    fwd = L.packed("magi_attn_fwd", L.AttnArgs).fn
+    pair = ((len(calls) == 2 or (begun and len(calls) > 2)) and calls[0][0] == calls[1][0] and calls[1][1] is fwd
+            and (begun or calls[0][1] is fwd))
     if begun or pair:
         _launch(calls[0][0], L.packed_pair("magi_attn_fwd_end" if begun else "magi_attn_fwd_two").fn, calls[0][2], calls[1][2] if pair else None)
         rest = calls[2 if pair else 1:]

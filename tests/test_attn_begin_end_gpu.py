@@ -97,6 +97,24 @@ def test_one_scratch_buffer_for_both(dev, rows, keys, raw):
     assert torch.equal(got, want) and torch.equal(got_x, want_x)
 
 
+@pytest.mark.parametrize("static", ["first", "second", "both"])
+@pytest.mark.parametrize("calls", [list, BegunCalls])
+def test_held_calls_with_static_scratch_memory(dev, calls, static):
+    """They take no workspace, which the entry points for two calls and for two halves would ask a measured bound for."""
+    g = torch.Generator(device=dev).manual_seed(5)
+    t = torch.randn(4200, 24, 128, device=dev, generator=g, dtype=torch.bfloat16) * 0.25  # (256-row items, which a first half leaves)
+    r = torch.tensor([[0, 4200]], dtype=torch.int32, device=dev)
+
+    def call(i, held):
+        kw = {"auto_bound": True, "static_scratch": True} if static in ("both", ("first", "second")[i]) else {"score_bound": 60.0, "q_prescaled": True}
+        return range_attention(t, t[:, i::3], t[:, i::3], r, r, 4200, 4200, return_lse=False, held=held, **kw)[0]
+
+    want, held = [call(i, None) for i in (0, 1)], calls()
+    got = [call(i, held) for i in (0, 1)]
+    launch_held(held)
+    assert not held and all(torch.equal(a, b) for a, b in zip(got, want))
+
+
 def test_an_end_without_pieces_is_refused(dev):
     q = torch.randn(64, 4, 128, device=dev, dtype=torch.bfloat16)
     r = torch.tensor([[0, 64]], dtype=torch.int32, device=dev)

@@ -408,12 +408,13 @@ def test_projection_rows_are_cut_only_where_a_round_of_tiles_is_left_partly_empt
 @pytest.mark.parametrize("begun", [False, True])
 @pytest.mark.parametrize("devices", ["0", "00", "01", "000", "010", "0000"])
 def test_every_held_call_is_launched_once(monkeypatch, begun, devices):
+    from magi_attn import _lib as L
     from magi_attn import functional as F
 
     done = []
     monkeypatch.setattr(F, "_launch", lambda dev, fn, *args: done.append((dev, fn, args)))
-    names = [f"call {i}" for i in range(len(devices))]
-    held = [(dev, None if begun and i == 0 else "fwd", name, ()) for i, (dev, name) in enumerate(zip(devices, names))]
+    names, fwd = [f"call {i}" for i in range(len(devices))], L.packed("magi_attn_fwd", L.AttnArgs).fn
+    held = [(dev, None if begun and i == 0 else fwd, name, ()) for i, (dev, name) in enumerate(zip(devices, names))]
     F.launch_held(held)
     assert not held and [a for _, _, args in done for a in args if a] == names  # each once, in their order
     together = [args for _, _, args in done if len(args) == 2 and args[1]]
