@@ -166,6 +166,13 @@ def qk_score_bound(q_norm: FusedLayerNorm, k_norm: FusedLayerNorm, rotary_half: 
     return float(bound.item())
 
 
+def _transformed() -> bool:
+    """Whether what is called is recorded or transformed (torch.compile, jit.trace, dispatch modes, vmap and the other function transforms,
+    forward-mode derivatives): row counts of its own and out= are not for those."""
+    return (torch.compiler.is_compiling() or torch._C._is_tracing() or torch._C._len_torch_dispatch_stack() > 0
+            or torch._C._functorch.maybe_current_level() is not None or torch.autograd.forward_ad._current_level >= 0)
+
+
 def _rows_ahead(rows: int, cols: int, depth: int, cus: int) -> int:
     """How many rows of a [rows, depth] x [cols, depth]^T product to run in a call of their own, 0: none.
 
@@ -193,10 +200,10 @@ def _linear_in_whole_rounds(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """torch.nn.functional.linear(x, w), the rows cut in two where that suits the library's tiles better (_rows_ahead)."""
     cols, depth = w.shape
     if (depth >= 1024 and cols % 256 == 0 and x.is_cuda and x.is_contiguous() and x.dtype is w.dtype
-            and not torch.is_autocast_enabled() and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad))):
+            and not torch.is_autocast_enabled() and not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad)) and not torch._C._is_tracing()):
         rows = x.numel() // depth
         head = _rows_ahead(rows, cols, depth, _compute_units(x.device))
-        if head:
+        if head and not _transformed():
             x2, wt = x.view(rows, depth), w.t()
             y = torch.empty((rows, cols), dtype=x.dtype, device=x.device)
             torch.mm(x2[:head], wt, out=y[:head])
@@ -328,7 +335,8 @@ class PerTensorQuantizedFp8Linear(torch.nn.Module):
         x2 = x8 if x8.dim() == 2 else x8.reshape(-1, self.in_features)
         w, scale_a, scale_b = _param(self, "weight"), _param(self, "input_scale").reshape(-1)[:1], _param(self, "weight_scale").reshape(-1)[:1]
         head = 0
-        if x2.shape[0] * self.out_features >= 1 << 24 and x2.is_cuda:  # (a round of 256 CUs: four calls a layer that may wait for the host)
+        # (a round of 256 CUs: four calls a layer that may wait for the host)
+        if x2.shape[0] * self.out_features >= 1 << 24 and x2.is_cuda and not _transformed():
             head = _rows_ahead_e4m3(x2.shape[0], self.out_features, self.in_features, _compute_units(x2.device))
         if head and (type(x2) in _PLAIN and type(w) in _PLAIN and x2.is_contiguous()
                      and not (torch.is_grad_enabled() and any(t.requires_grad for t in (x2, w, scale_a, scale_b)))):

@@ -140,6 +140,30 @@ def test_rows_of_whole_rounds_ahead_of_the_rest(dev, monkeypatch):
     assert calls == [16384, rows, 16384, 300]
 
 
+@pytest.mark.parametrize("how", ["vmap", "jit.trace", "make_fx"])
+def test_products_that_are_cut_under_transforms(dev, how):
+    """vmap has no batched form of a product with out=, and a recorded one is run with other numbers of rows: one call for all rows there.
+    (Of 1024 terms in another order, fp32 sums: 2^-14 of their size at most, and a bf16 step.)"""
+    K, N, rows = 1024, 1024, 16384 + 300
+    m = MOD.PerTensorQuantizedFp8Linear(K, N, device=dev)
+    m.weight.data = (torch.randn(1, N, K, device=dev) * 40).clamp(-448, 448).to(torch.float8_e4m3fn)
+    x8 = (torch.randn(2, rows, K, device=dev) * 40).clamp(-448, 448).to(torch.float8_e4m3fn)
+    w = torch.randn(2048, K, device=dev, dtype=torch.bfloat16)  # (8 columns of tiles: 8192 rows are a round)
+    for f, x in ((lambda t: m.forward_quantized(t), x8), (lambda t: MOD._linear_in_whole_rounds(t, w), torch.randn(2, 8192 + 300, K, device=dev, dtype=torch.bfloat16))):
+        with torch.no_grad():
+            want = torch.stack([f(x[0]), f(x[1])])
+            if how == "vmap":
+                got = torch.vmap(f)(x)
+            else:
+                from torch.fx.experimental.proxy_tensor import make_fx
+                recorded = torch.jit.trace(f, (x[0],), check_trace=False) if how == "jit.trace" else make_fx(f)(x[0])
+                got = torch.stack([recorded(t) for t in x])
+                for n in (96, x.shape[1] + 96):
+                    more = x.reshape(-1, K)[:n]
+                    assert torch.allclose(recorded(more).float(), f(more).float(), rtol=2.0 ** -7, atol=2.0 ** -14 * want.float().abs().max().item())
+        assert torch.allclose(got.float(), want.float(), rtol=2.0 ** -7, atol=2.0 ** -14 * want.float().abs().max().item())
+
+
 def test_projections_hold_no_more_memory_than_norm_and_quantisers_apart(dev):
     """The e4m3 inputs of the four linears are given back one by one: the most that is held is below the outputs, the norm's
     bf16 rows and one e4m3 input, which is what separate calls hold."""
