@@ -85,8 +85,8 @@ extern "C" {
 #define MAGI_ATTN_ROW_BITS 128
 /* bf16 with a score_bound in force: the keys of a row may be shared by the wavefronts of a workgroup where the launch is so small that
  * it waits for its longest row (32 rows to a workgroup, about one workgroup per CU; from max_seqlen_k, which has to be stated, and the other
- * sizes alone).  The fp32 sums are then added in another order, as with split_workspace; no memory is needed.  Ignored elsewhere; not
- * with MAGI_ATTN_ROW_BITS. */
+ * sizes alone).  The fp32 sums are then added in another order, as with split_workspace; no memory is needed.  Ignored elsewhere, and below
+ * 32 keys but for magi_attn_fwd_two; not with MAGI_ATTN_ROW_BITS. */
 #define MAGI_ATTN_SHARE_WAVES 1024
 
 #define MAGI_RANGES_PAIRS 0 /* int32 [n, 2]: range i = [r[2i], r[2i+1])          */
@@ -266,7 +266,7 @@ int64_t magi_attn_pieces_bytes(int32_t Hq, int32_t Hkv, int32_t n_ranges, int32_
 int32_t magi_attn_tile_rows(int32_t Hq, int32_t Hkv, int32_t n_ranges, int32_t max_seqlen_q, int32_t max_seqlen_k, int64_t split_workspace_bytes);
 
 /* Wavefronts that share the keys of a row where such a call has MAGI_ATTN_SHARE_WAVES and a score_bound in force, no split_workspace's use
- * then; 0: it takes the other forms. */
+ * then (max_seqlen_k below 32: in a launch with another call only, the same bits); 0: it takes the other forms. */
 int32_t magi_attn_waves(int32_t Hq, int32_t Hkv, int32_t n_ranges, int32_t ranges_mode, int32_t max_seqlen_q, int32_t max_seqlen_k);
 
 int magi_attn_fwd(const magi_attn_args* args, void* stream);

@@ -383,11 +383,16 @@ int64_t r32_bytes(int Hq, int Hkv, int n_ranges, int max_seqlen_q, int max_seqle
 // Whether a launch without a running maximum whose caller permits it (MAGI_ATTN_SHARE_WAVES) has the keys of 32 rows shared by the wavefronts of
 // a workgroup (attn_fwd_bf16_waves.hip): how many wavefronts, 0: not.
 // Eight, a workgroup per CU, or four, two of them.  Measured, 128 and 256 rows to a workgroup (in pieces where that was the better) / this form, drawn sizes
-// (profiles/launches_below_a_round_sweep.txt): up to one workgroup of 32 rows per CU 120 launches 0.94 to 1.76 times as fast, 1.23 on average (12
-// workgroups over 519 keys 14.9 / 11.5 us, 48 over 480 13.4 / 9.1, 192 over 945 21.5 / 12.7, 216 over 5040 35.9 / 30.9, 240 over 7632 43.5 / 44.5);
-// four wavefronts up to 1024 keys (96 over 691 18.2 / 12.7 with either) and for more than a workgroup per CU: 288 over 594 15.5 / 12.7, 360 over 1600 27.8 / 19.5, 416 over 4040
-// 45.6 / 39.3, but 288 over 5085 40.8 / 47.1, 312 over 8100 52.7 / 72.6; beyond two per CU 576 over 1050 23.6 / 27.3.  max_seqlen_k of text is the padded
-// length: 288 workgroups over 39 of 800 keys 7.6 / 8.0, 504 over 184 10.4 / 12.5, so cumulative lengths only up to one per CU.
+// (those it takes: profiles/launches_below_a_round_sweep.txt): up to one workgroup of 32 rows per CU, from 65 keys on, 77 launches 0.95 to 1.72 times as fast, 1.23 on average (12
+// workgroups over 423 keys 12.1 / 9.7 us, 48 over 480 13.4 / 9.1, 240 over 1113 18.2 / 12.7, 228 over 5930 41.1 / 34.5); four wavefronts up to 1024 keys
+// and for more than a workgroup per CU: 288 over 600 15.8 / 12.3, 480 over 1460 30.3 / 22.7, 360 over 4570 41.5 / 40.6, but 288 over 5085 40.8 / 47.1, 312 over
+// 8100 52.7 / 72.6; beyond two per CU 576 over 1050 23.6 / 27.3.  max_seqlen_k of text is the padded length: 288 workgroups over 39 of 800 keys
+// 7.6 / 8.0, 504 over 184 10.4 / 12.5, so cumulative lengths only up to one per CU.
+// Below a SLAB of keys there is nothing to share: by itself such a launch takes the other forms (21 drawn ones of 1 to 31 keys 0.86 to 1.02 of
+// their time in this one, 0.94 on average; the same bits), beside another small call this one, a launch less (31 and 20 keys 11.6 us one by one, 7.2
+// together).  Above, by themselves: 32 keys 1.00 to 1.12, 33 to 64 0.90 to 1.04, 0.97 on average (their sums are in another order here, which a
+// call beside another one has too).
+constexpr int SLAB = 32;
 int waves_plan(int Hq, int Hkv, int n_ranges, int ranges_mode, int max_seqlen_q, int max_seqlen_k) {
   if ((double)Hq * n_ranges * (max_seqlen_q / 32 + 1) > 2.0e9) return 0;
   const double items = 8.0 * items_per_xcd(Hq, Hkv, n_ranges, max_seqlen_q / 32 + (max_seqlen_q % 32 != 0));
@@ -406,8 +411,7 @@ int waves_plan(int Hq, int Hkv, int n_ranges, int ranges_mode, int max_seqlen_q,
 constexpr int HELD = 1, ALONE = 2;
 enum Held { NOW, FIRST, SECOND, TEXT, BEGIN, END };
 int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace, magi::AttnKernArgs* held = nullptr, Held how = NOW);
-// a held call by itself
-int launch_held(const magi::AttnKernArgs& a, void* stream);
+int launch_waves(const magi::AttnKernArgs& a, void* stream);
 int attn_fwd_two(const magi_attn_args* first, const magi_attn_args* second, void* stream);
 int attn_fwd_end(const magi_attn_args* first, const magi_attn_args* second, void* stream);
 
@@ -518,22 +522,25 @@ int magi_attn_fwd_static_scratch(const magi_attn_args* p, void* stream) {
 
 namespace {
 
-// Held calls: 32 rows to a workgroup, whose wavefronts share keys; or 256 rows of q as it is or raw.  count of them, in one launch.
-int launch_held(magi::AttnPairArgs& pair, int count, void* stream) {
+// a call of wavefronts that share keys by itself
+int launch_waves(const magi::AttnKernArgs& a, void* stream) {
+  magi::AttnPairArgs pair;
+  pair.job[0] = a;
+  pair.job[1].per_xcd = 0;
+  const hipError_t e = magi::launch_attn_fwd_bf16_waves(pair, static_cast<hipStream_t>(stream));
+  if (e != hipSuccess) return hip_fail(e, "magi_attn_fwd launch");
+  count_launches(1);
+  return MAGI_OK;
+}
+
+// two held calls of one form in one launch: 32 rows to a workgroup, whose wavefronts share keys; or 256 rows of q as it is or raw
+int launch_alike(const magi::AttnPairArgs& pair, void* stream) {
   const hipStream_t st = static_cast<hipStream_t>(stream);
   const magi::AttnKernArgs& a = pair.job[0];
-  if (count == 1) pair.job[1].per_xcd = 0;
-  const hipError_t e = a.block_m == 32 ? magi::launch_attn_fwd_bf16_waves(pair, st)
-                       : count == 2    ? magi::launch_attn_fwd_bf16_x16_pair(pair, st)
-                                       : magi::launch_attn_fwd_bf16_x16(a, st);
+  const hipError_t e = a.block_m == 32 ? magi::launch_attn_fwd_bf16_waves(pair, st) : magi::launch_attn_fwd_bf16_x16_pair(pair, st);
   if (e != hipSuccess) return hip_fail(e, "magi_attn_fwd launch");
   count_launches(1 + (a.block_m != 32 && a.split_from < a.per_xcd));
   return MAGI_OK;
-}
-int launch_held(const magi::AttnKernArgs& a, void* stream) {
-  magi::AttnPairArgs pair;
-  pair.job[0] = a;
-  return launch_held(pair, 1, stream);
 }
 
 // Whether so many workgroups of 256 threads are a launch: HIP takes less than 2^32 threads.  (Two calls may fit apart and not together: ranges of
@@ -541,10 +548,10 @@ int launch_held(const magi::AttnKernArgs& a, void* stream) {
 bool fits(uint64_t workgroups) { return workgroups * 256 <= UINT32_MAX; }
 
 // a held text call in tiles of 128 (as attn_text_rows.h takes it) or 256 rows, whole items, beside so many other workgroups; false, and b as it was,
-// where it is another kind or the launch would not fit
+// where the launch would not fit
 bool text_in_rows(magi::AttnKernArgs& b, int max_seqlen_q, int rows, uint64_t others) {
   const int tiles = max_seqlen_q / rows + (max_seqlen_q % rows != 0);
-  if (b.block_m == 32 || (double)b.Hq * b.n_ranges * tiles > 2.0e9) return false;
+  if ((double)b.Hq * b.n_ranges * tiles > 2.0e9) return false;
   const unsigned per_xcd = items_per_xcd(b.Hq, b.Hkv, b.n_ranges, tiles);
   if (!fits(others + 8ull * per_xcd)) return false;
   b.block_m = rows;
@@ -554,9 +561,9 @@ bool text_in_rows(magi::AttnKernArgs& b, int max_seqlen_q, int rows, uint64_t ot
   return true;
 }
 
-// a second call that did not go with the first, which has been launched: `two` is what attn_fwd_impl returned for it, b its arguments where HELD
-int launch_behind(int two, const magi::AttnKernArgs& b, const magi_attn_args* second, void* stream) {
-  return two == HELD ? launch_held(b, stream) : two == ALONE ? attn_fwd_impl(second, stream, second->workspace) : two;
+// a second call that did not go with the first, which has been launched: `two` is what attn_fwd_impl returned for it
+int launch_behind(int two, const magi_attn_args* second, void* stream) {
+  return two == HELD || two == ALONE ? attn_fwd_impl(second, stream, second->workspace) : two;
 }
 
 // the second half of magi_attn_fwd_begin(first), beside second
@@ -575,7 +582,7 @@ int attn_fwd_end(const magi_attn_args* first, const magi_attn_args* second, void
                              : (together ? magi::launch_attn_text_merge(pair, st) : magi::launch_attn_fwd_bf16_merge(a, st));
   if (e != hipSuccess) return hip_fail(e, "magi_attn_fwd_end launch");
   count_launches(1);
-  return together ? MAGI_OK : launch_behind(two, b, second, stream);
+  return together ? MAGI_OK : launch_behind(two, second, stream);
 }
 
 // first, then second, which do not depend on each other: in one launch where both take the form for it
@@ -591,14 +598,14 @@ int attn_fwd_two(const magi_attn_args* first, const magi_attn_args* second, void
     const hipError_t e = together ? magi::launch_attn_fwd_fp8_text(pair, st) : magi::launch_attn_fwd_fp8(a, st);
     if (e != hipSuccess) return hip_fail(e, "magi_attn_fwd launch");
     count_launches(1 + (a.split_from < a.per_xcd));
-    return together ? MAGI_OK : launch_behind(two, b, second, stream);
+    return together ? MAGI_OK : launch_behind(two, second, stream);
   }
   const int two = attn_fwd_impl(second, stream, second->workspace, &b, SECOND);
   // (of 32 rows there is at most a workgroup or two per CU)
   if (two == HELD && a.block_m == b.block_m && (b.block_m == 32 || (b.split_from >= b.per_xcd && fits(split_grid(a) + 8ull * b.per_xcd))))
-    return launch_held(pair, 2, stream);
-  const int rc = launch_held(a, stream);
-  return rc < 0 ? rc : launch_behind(two, b, second, stream);
+    return launch_alike(pair, stream);
+  const int rc = attn_fwd_impl(first, stream, first->workspace);
+  return rc < 0 ? rc : launch_behind(two, second, stream);
 }
 
 int not_begun() { return fail(MAGI_EINVAL, "magi_attn_fwd_end: not a call that magi_attn_fwd_begin leaves anything of"); }
@@ -793,7 +800,9 @@ int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace, magi:
       const double wg384 = (double)p->Hq * p->n_ranges * ((p->max_seqlen_q + 383) / 384);
       const bool long_keys = p->max_seqlen_k == 0 || p->max_seqlen_k >= 4096;  // (0 = not stated)
       if (bounded && !checked && !auto_bound && !mfma32 && p->q_tile_rows == 0 && (p->flags & MAGI_ATTN_SHARE_WAVES))
-        a.waves = waves_plan(p->Hq, p->Hkv, p->n_ranges, p->ranges_mode, p->max_seqlen_q, p->max_seqlen_k);
+        a.waves = p->max_seqlen_k >= SLAB || how == FIRST || how == SECOND
+                      ? waves_plan(p->Hq, p->Hkv, p->n_ranges, p->ranges_mode, p->max_seqlen_q, p->max_seqlen_k)
+                      : 0;
       if (bounded && !checked && !mfma32 && p->q_tile_rows == 0 && !a.waves)
         r32 = r32_plan(p->Hq, p->Hkv, p->n_ranges, p->max_seqlen_q, p->max_seqlen_k, split_bytes);
       if (a.waves)
@@ -830,7 +839,8 @@ int attn_fwd_impl(const magi_attn_args* p, void* stream, float* workspace, magi:
     a.share_pieces = 1;
     if (a.waves) {
       if (how == END) return not_begun();
-      if (!held || how == BEGIN) return launch_held(a, stream);
+      if (how == TEXT) return ALONE;
+      if (!held || how == BEGIN) return launch_waves(a, stream);
       *held = a;
       return HELD;
     }

@@ -2,9 +2,10 @@
 // gfx950 (MI355X).  One or two calls in a launch (a layer's core and text attention, which do not depend on each other).
 //
 // What bounds such launches is latency: 12 items of 128 rows over 480 keys are eight tiles in a row on twelve CUs, 14.3 us, while the rest
-// of the chip waits, and the text attention behind it lives for 7.8 us of launch and trips to memory.  So: workgroups of 32 rows x eight
-// wavefronts, each wavefront every eighth slab of 32 keys, with LDS slots of its own (no barriers in the loop); without a running maximum
-// the wavefronts' accumulators and row sums simply add up, through LDS.  MFMA shape, operand layouts and the layout of keys in LDS are those
+// of the chip waits, and the text attention behind it lives for 7.8 us of launch and trips to memory.  So: workgroups of 32 rows x four
+// wavefronts (up to 1024 keys, and more than a workgroup per CU) or eight, each wavefront every fourth or eighth slab of 32 keys, with LDS slots
+// of its own (no barriers in the loop); without a running maximum the wavefronts' accumulators and row sums simply add up, through LDS.
+// The two calls in one launch 10.1 us.  MFMA shape, operand layouts and the layout of keys in LDS are those
 // of attn_fwd_bf16_r32.hip.  A slab is fetched for 32 rows only, four times the bytes per row of a 128-row workgroup: 130 GB/s and CU, what
 // direct loads hold, are 1 us per 256 keys, so this is for launches of about one workgroup per CU (waves_plan in api.cpp).
 #include "attn_bf16_tiles.h"

@@ -65,6 +65,23 @@ def test_shared_keys_give_what_the_other_forms_give(dev, mode, Hq, Hkv, Tq, q_ra
         assert torch.equal(o[:, :, 1].reshape(Tq, Hq, D), got) and (o[:, :, 0] == 3.0).all()
 
 
+# one key, a few, a whole slab; rows around a workgroup's 32 and two of them; a range without keys; rows in no range; two key segments
+@pytest.mark.parametrize("mode", ["as it is", "scaled", "normed"])
+@pytest.mark.parametrize("Hq,Hkv,Tq,q_ranges,k_ranges,k_split", [
+    (1, 1, 1, [(0, 1)], [(0, 1)], None), (6, 2, 33, [(0, 33)], [(3, 34)], 20), (24, 8, 70, [(2, 66)], [(0, 32)], None), (6, 2, 65, [(0, 32), (32, 65)], [(7, 7), (0, 9)], 4)])
+def test_one_slab_of_keys_has_the_bits_of_the_other_forms(dev, mode, Hq, Hkv, Tq, q_ranges, k_ranges, k_split):
+    """By itself such a call takes those; in one launch with another one a wavefront of its workgroup has all of the keys, in the same order."""
+    call, _, waves = _case(dev, Hq, Hkv, q_ranges, k_ranges, Tq, k_split, mode)
+    want = call(split_keys=False)
+    held = []
+    one, got, other = call(share_waves=True), call(share_waves=True, held=held), call(share_waves=True, held=held)
+    n0 = M.lib().magi_launch_count()
+    F.launch_held(held)
+    assert not waves or M.lib().magi_launch_count() - n0 == 1
+    for o, lse in (one, got, other):
+        assert torch.equal(o, want[0]) and torch.equal(lse, want[1])
+
+
 # both small (four wavefronts; four and eight), one of them or both in other forms; the number of launches
 @pytest.mark.parametrize("first,second,launches", [
     ((6, 2, [(0, 120), (120, 240)], [(0, 360), (0, 480)], 240), (6, 2, [(0, 240)], [(0, 30)], 240), 1),

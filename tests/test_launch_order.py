@@ -166,3 +166,21 @@ def test_launches_that_fit_apart_only_are_launched_apart(api, first, entry):
     got = launches(tile * edge)
     assert len(got) == 1 and got[0][2] == others + edge * per_tile
     assert len(launches(tile * edge + 1)) == 2
+
+
+@pytest.mark.parametrize("keys", [1, 31, 32, 33])
+def test_less_than_a_slab_of_keys_is_shared_beside_another_small_call_only(api, keys):
+    waves = lambda out, n, kind: _call(out, 96, n, kind, flags=L.MAGI_ATTN_SHARE_WAVES | (L.MAGI_ATTN_Q_PRESCALED if kind == "as it is" else 0))
+    core, text = waves(0x100, keys, "as it is"), waves(0x200, keys, "raw")
+    name = lambda: [(f[0], len(f[1])) for f in _launches(api)]
+    of_one = [("launch_attn_fwd_bf16_x16" if keys < 32 else "launch_attn_fwd_bf16_waves", 1)]
+    both = [("launch_attn_fwd_bf16_waves", 2)]
+    name()
+    for call in (core, text):
+        assert api.magi_attn_fwd(C.byref(call), None) == 0 and name() == of_one
+    assert api.magi_attn_fwd_begin(C.byref(core), None) == 0 and name() == of_one
+    for a, b in ((core, text), (core, waves(0x200, 400, "raw")), (waves(0x100, 400, "as it is"), text)):
+        assert api.magi_attn_fwd_two(C.byref(a), C.byref(b), None) == 0 and name() == both
+    large = _call(0x300, 4200, 3000, "as it is")
+    for a, b in ((core, large), (large, core)):  # (and no other call in the launch)
+        assert api.magi_attn_fwd_two(C.byref(a), C.byref(b), None) == 0 and sorted(name()) == sorted(of_one + [("launch_attn_fwd_bf16_x16", 1)])
