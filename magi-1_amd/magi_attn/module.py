@@ -1256,17 +1256,17 @@ class FullyParallelAttention(torch.nn.Module):
         # layers of 128 to 512 rows per CU 0.994 to 1.097 times as fast (2112 rows 390 -> 381 us, 2964 403 -> 389; whole 3888 373 -> 340,
         # 4176 505 -> 480), cores of other forms the same; from 44 to 83 rows per CU, which wait for the host, 0.985 to 1.026.
         held = None
-        if core_bounded and cross_bounded and self.attention_dtype == "bf16" and _OWN_CROSS_FUSED.of(self):
+        if core_bounded and cross_bounded and self.attention_dtype == "bf16":
             rows_per_cu = sq * Hq / _compute_units(hidden_states.device)  # of all heads
-            if rows_per_cu <= 32:
+            if 32 < rows_per_cu < 128 or not _OWN_CROSS_FUSED.of(self):
+                pass
+            elif rows_per_cu <= 32:
                 cp, Hkv = meta_args.cross_attn_params, self.num_query_groups_per_partition
                 if attention_waves(Hq, Hkv, p.q_range.shape[0], L.MAGI_RANGES_PAIRS, p.max_seqlen_q, p.max_seqlen_k) and attention_waves(
                         Hq, Hkv, cp.cu_seqlens_q.numel() - 1, L.MAGI_RANGES_CU, cp.max_seqlen_q, cp.max_seqlen_kv):
                     held = []
-            elif rows_per_cu >= 512:
-                held = []
-            elif rows_per_cu >= 128:
-                held = BegunCalls()
+            else:
+                held = [] if rows_per_cu >= 512 else BegunCalls()
         elif (cross_bounded and self.attention_dtype == "fp8" and sq * Hq >= 64 * _compute_units(hidden_states.device) and _OWN_CROSS_FUSED.of(self)
               and _OWN_CORE_FP8.of(self)):
             # (e4m3 core: the text beside it in a form of its own, attn_fwd_fp8_text.hip.  40 drawn layers from 122 rows per CU on 1.006 to 1.096
