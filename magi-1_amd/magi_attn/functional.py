@@ -259,15 +259,17 @@ def range_attention(
     flags = ((L.MAGI_ATTN_FP8_POW2_PRESCALED if fp8_pow2_prescaled else 0) | (L.MAGI_ATTN_Q_PRESCALED if q_prescaled else 0)
              | (L.MAGI_ATTN_FP8_FAST_EXP2 if fp8_fast_exp2 else 0) | (L.MAGI_ATTN_BOUNDED_MFMA32 if bounded_mfma32 else 0)
              | (L.MAGI_ATTN_AUTO_BOUND if auto_bound else 0) | (L.MAGI_ATTN_ZERO_UNCOVERED if zero_gaps else 0)
-             | (L.MAGI_ATTN_CHECKED if checked else 0) | (L.MAGI_ATTN_SHARE_WAVES if share_waves and split_keys else 0) | (0 if split_keys or q.dtype is not torch.bfloat16 else L.MAGI_ATTN_ROW_BITS))
+             | (L.MAGI_ATTN_CHECKED if checked else 0) | (L.MAGI_ATTN_SHARE_WAVES if share_waves and split_keys else 0)
+             | (0 if split_keys or q.dtype is not torch.bfloat16 else L.MAGI_ATTN_ROW_BITS))
     workspace = None
     if checked:
         workspace = torch.empty(max(4 * Hq * max(n, 0) * ((int(max_seqlen_q) + 255) // 256), 4), dtype=torch.int32, device=q.device)
     if auto_bound and not static_scratch:
         workspace = torch.empty(4, dtype=torch.float32, device=q.device)  # (alive until the launches are enqueued)
     split, split_bytes, online = None, 0, False
-    if (share_waves and split_keys and q.dtype is torch.bfloat16 and 0.0 < score_bound <= L.MAGI_SCORE_BOUND_MAX and not (q_tile_rows or bounded_mfma32)
-            and Hq * n * max_seqlen_q <= 64 * _compute_units(q.device)  # (two workgroups of 32 rows per CU: magi_attn_waves says no beyond)
+    # (beyond two workgroups of 32 rows for each of 256 CUs magi_attn_waves says no; short keys need no memory in any form)
+    if (share_waves and max_seqlen_k >= 512 and Hq * n * max_seqlen_q <= 16384 and split_keys and q.dtype is torch.bfloat16
+            and 0.0 < score_bound <= L.MAGI_SCORE_BOUND_MAX and not (q_tile_rows or bounded_mfma32)
             and attention_waves(Hq, Hkv, n, ranges_mode, max_seqlen_q, max_seqlen_k)):
         pass  # (keys shared without memory)
     elif split_keys and not static_scratch and max_seqlen_k >= 512 and (
@@ -304,12 +306,13 @@ def range_attention(
         0.0 if softmax_scale is None else float(softmax_scale), flags, group_heads, o_stride_g,
         min(float(score_bound), 3e38), int(q_tile_rows), _ptr(gamma), _ptr(beta), norm_eps, norm_kind, _ptr(k2_scale),
         _ptr(v2_scale), _ptr(workspace), batch_rows, q_stride_b, o_stride_b, _ptr(split), split_bytes)
+    if held is None:
+        _launch(q.device, call.fn, args)
+        return out, lse
     begin = type(held) is BegunCalls and held.begin
     if begin:
         held.begin = False
-    if held is None:
-        _launch(q.device, call.fn, args)
-    elif begin and not static_scratch:
+    if begin and not static_scratch:
         if _launch(q.device, L.packed("magi_attn_fwd_begin", L.AttnArgs).fn, args):
             held.append((q.device, None, args, (q, k, v, k2, v2, q_ranges, k_ranges, gamma, beta, split, out, lse)))
     else:  # (with everything it reads and writes)
@@ -519,12 +522,17 @@ def qk_prologue_fp8(q_raw, k_raw, rope, gq, bq, gk, bk, *, Hq: int, Hkv: int, q_
         n_cache_rows = S
     if n_cache_rows is None:
         n_cache_rows = S if k_tail is None else 0
-    for name, t in (("q_raw", q_raw), ("k_raw", k_raw)) + ((("v_raw", v_raw),) if v_row_max is not None else ()):
-        if t is None or t.dtype != torch.bfloat16 or t.stride(-1) != 1 or t.dim() != 2:
+    for name, t in (("q_raw", q_raw), ("k_raw", k_raw)):
+        if t.dtype != torch.bfloat16 or t.stride(-1) != 1 or t.dim() != 2:
             raise ValueError(f"{name} must be a 2-D bf16 tensor with contiguous rows")
-    if v_row_max is not None and (v_row_max.dtype != torch.int16 or tuple(v_row_max.shape) != (Hkv, S) or not v_row_max.is_contiguous()
-                                  or tuple(v_raw.shape) != (S, Hkv * D) or v_raw.device != dev or v_row_max.device != dev):
-        raise ValueError("v_row_max must be a contiguous int16 [Hkv, S] tensor, v_raw [S, Hkv * 128], on q_raw's device")
+    entry, more, v_at, v_stride = ("magi_qk_prologue", L.PrologueArgs), (), 0, 0
+    if v_row_max is not None:
+        if v_raw is None or v_raw.dtype != torch.bfloat16 or v_raw.dim() != 2 or v_raw.stride(-1) != 1:
+            raise ValueError("v_raw must be a 2-D bf16 tensor with contiguous rows")
+        if (v_row_max.dtype != torch.int16 or tuple(v_row_max.shape) != (Hkv, S) or not v_row_max.is_contiguous()
+                or tuple(v_raw.shape) != (S, Hkv * D) or v_raw.device != dev or v_row_max.device != dev):
+            raise ValueError("v_row_max must be a contiguous int16 [Hkv, S] tensor, v_raw [S, Hkv * 128], on q_raw's device")
+        entry, more, v_at, v_stride = ("magi_qk_prologue_row_max", L.PrologueArgs, C.c_void_p), (v_row_max.data_ptr(),), v_raw.data_ptr(), v_raw.stride(0)
     for name, t in (("k_out", k_out), ("k_tail", k_tail)):
         if t is not None and (t.dtype != f8 or t.dim() != 3 or t.shape[1:] != (Hkv, D) or t.stride(2) != 1
                               or t.stride(1) != D):
@@ -539,14 +547,13 @@ def qk_prologue_fp8(q_raw, k_raw, rope, gq, bq, gk, bk, *, Hq: int, Hkv: int, q_
         if rope.dtype != torch.float32 or rope.dim() != 2 or rope.shape[0] * max(batch, 1) != S or not rope.is_contiguous():
             raise ValueError("rope must be a contiguous fp32 [S / batch, 2*R2] tensor")
         R2 = rope.shape[1] // 2
-    more = v_row_max is not None
-    call = L.packed("magi_qk_prologue_row_max", L.PrologueArgs, C.c_void_p) if more else L.packed("magi_qk_prologue", L.PrologueArgs)
-    args = call.pack(call.size, q_raw.data_ptr(), k_raw.data_ptr(), v_raw.data_ptr() if more else 0, _ptr(rope), _ptr(gq), _ptr(bq), _ptr(gk),
-                     _ptr(bk), q_out.data_ptr(), _ptr(k_out), _ptr(k_tail), q_raw.stride(0), k_raw.stride(0), v_raw.stride(0) if more else 0,
+    call = L.packed(*entry)
+    args = call.pack(call.size, q_raw.data_ptr(), k_raw.data_ptr(), v_at, _ptr(rope), _ptr(gq), _ptr(bq), _ptr(gk),
+                     _ptr(bk), q_out.data_ptr(), _ptr(k_out), _ptr(k_tail), q_raw.stride(0), k_raw.stride(0), v_stride,
                      0 if k_out is None else k_out.stride(0), 0 if k_tail is None else k_tail.stride(0), S, int(n_cache_rows), Hq,
                      Hkv, D, R2, int(norm_kind), float(eps), int(batch), float(q_premul), L.MAGI_DTYPE_FP8_E4M3, float(q_scale),
                      float(k_scale))
-    _launch(dev, call.fn, args, *((v_row_max.data_ptr(),) if more else ()))
+    _launch(dev, call.fn, args, *more)
     return q_out, k_out, k_tail
 
 
