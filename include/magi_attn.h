@@ -460,7 +460,8 @@ int magi_small_projections_e4m3(const magi_small_proj_args* args, float q_quant_
  * the core attention of the rows q over [kv[:k_split] | kv_side], the cross attention of the rows qx over text_kv.  What it stands for
  * in those calls' structs: strides in elements; heads 128 apart; K | V interleaved per head, kv_row elements a row, the new rows to kv_new (kept of
  * them) and kv_side; q, qx [S, Hq, 128], text_kv [T, Hkv, 256]; pairs for core, cumulative lengths for cross; split workspaces of their own.
- * parts: 1 = the first two, 2 = the last, 3 = all, the two attention calls as magi_attn_fwd_two makes them.  A refusal of one of the three is this call's, what is ahead of it has been launched.
+ * parts: 1 = the first two, 2 = the last, 3 = all, the two attention calls as magi_attn_fwd_two makes them.  A refusal of one of the three is
+ * this call's, what is ahead of it has been launched.
  */
 typedef struct magi_small_layer_args {
   uint32_t struct_size; /* sizeof(magi_small_layer_args) */

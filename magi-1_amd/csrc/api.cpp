@@ -382,16 +382,16 @@ int64_t r32_bytes(int Hq, int Hkv, int n_ranges, int max_seqlen_q, int max_seqle
 
 // Whether a launch without a running maximum whose caller permits it (MAGI_ATTN_SHARE_WAVES) has the keys of 32 rows shared by the wavefronts of
 // a workgroup (attn_fwd_bf16_waves.hip): how many wavefronts, 0: not.
-// Eight, a workgroup per CU, or four, two of them.  Measured, 128 and 256 rows to a workgroup (in pieces where that was the better) / this form, drawn sizes
-// (those it takes: profiles/launches_below_a_round_sweep.txt): up to one workgroup of 32 rows per CU, from 65 keys on, 77 launches 0.95 to 1.72 times as fast, 1.23 on average (12
-// workgroups over 423 keys 12.1 / 9.7 us, 48 over 480 13.4 / 9.1, 240 over 1113 18.2 / 12.7, 228 over 5930 41.1 / 34.5); four wavefronts up to 1024 keys
-// and for more than a workgroup per CU: 288 over 600 15.8 / 12.3, 480 over 1460 30.3 / 22.7, 360 over 4570 41.5 / 40.6, but 288 over 5085 40.8 / 47.1, 312 over
-// 8100 52.7 / 72.6; beyond two per CU 576 over 1050 23.6 / 27.3.  max_seqlen_k of text is the padded length: 288 workgroups over 39 of 800 keys
-// 7.6 / 8.0, 504 over 184 10.4 / 12.5, so cumulative lengths only up to one per CU.
-// Below a SLAB of keys there is nothing to share: by itself such a launch takes the other forms (21 drawn ones of 1 to 31 keys 0.86 to 1.02 of
-// their time in this one, 0.94 on average; the same bits), beside another small call this one, a launch less (31 and 20 keys 11.6 us one by one, 7.2
-// together).  Above, by themselves: 32 keys 1.00 to 1.12, 33 to 64 0.90 to 1.04, 0.97 on average (their sums are in another order here, which a
-// call beside another one has too).
+// Eight, a workgroup per CU, or four, two of them.  Measured, 128 and 256 rows to a workgroup (in pieces where that was the better) / this form, drawn
+// sizes (those it takes: profiles/launches_below_a_round_sweep.txt): up to one workgroup of 32 rows per CU, from 65 keys on, 77 launches 0.95 to 1.72
+// times as fast, 1.23 on average (12 workgroups over 423 keys 12.1 / 9.7 us, 48 over 480 13.4 / 9.1, 240 over 1113 18.2 / 12.7, 228 over 5930 41.1 /
+// 34.5); four wavefronts up to 1024 keys and for more than a workgroup per CU: 288 over 600 15.8 / 12.3, 480 over 1460 30.3 / 22.7, 360 over 4570
+// 41.5 / 40.6, but 288 over 5085 40.8 / 47.1, 312 over 8100 52.7 / 72.6; beyond two per CU 576 over 1050 23.6 / 27.3.  max_seqlen_k of text is the
+// padded length: 288 workgroups over 39 of 800 keys 7.6 / 8.0, 504 over 184 10.4 / 12.5, so cumulative lengths only up to one per CU.
+// Below a SLAB of keys there is nothing to share: by itself such a launch takes the other forms (21 drawn ones of 1 to 31 keys 0.86 to 1.02 of their time in this
+// one, 0.94 on average; the same bits), beside another small call this one, a launch less (31 and 20 keys 11.6 us one by one, 7.2 together).  Above,
+// by themselves: 32 keys 1.00 to 1.12, 33 to 64 0.90 to 1.04, 0.97 on average (their sums are in another order here, which a call beside another one
+// has too).
 constexpr int SLAB = 32;
 int waves_plan(int Hq, int Hkv, int n_ranges, int ranges_mode, int max_seqlen_q, int max_seqlen_k) {
   if ((double)Hq * n_ranges * (max_seqlen_q / 32 + 1) > 2.0e9) return 0;

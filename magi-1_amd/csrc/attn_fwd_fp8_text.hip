@@ -3,11 +3,11 @@
 // The two do not depend on each other, and one after the other the e4m3 launch ends with slots empty for the length of a workgroup and the
 // text's launch, which waits for all of it, is a round or two of short workgroups of its own.  Here the text's workgroups follow the core's.
 // They must not cost the core its three workgroups per CU, 36 KB of LDS and 168 registers each: the forms of the bf16 kernels take 53 and
-// 70 KB.  So the text is walked in tiles of 32 keys in the four slots of the e4m3 tiles (attn_text_rows.h).  168 registers, 3 of them spilled outside the tile loops (the e4m3 kernel by
-// itself: 2).
+// 70 KB.  So the text is walked in tiles of 32 keys in the four slots of the e4m3 tiles (attn_text_rows.h).  168 registers, 3 of them spilled
+// outside the tile loops (the e4m3 kernel by itself: 2).
 // The layers around the two, one by one -> together, 24 heads: 9360 rows over 46800 keys, 400 of text 2997 -> 2955 us; 5400 rows 551 -> 513; 14472
-// 2644 -> 2586; 3600 318 -> 306; 86400 rows x 48 heads 79.50 -> 79.45 ms.  40 drawn layers from 122 rows per CU (of all heads) on: 1.006 to
-// 1.096 times as fast; below 71 the two do not fill the chip and are launched one by one (module.py).
+// 2644 -> 2586; 3600 318 -> 306; 86400 rows x 48 heads 79.50 -> 79.45 ms.  28 drawn layers from 122 rows per CU (of all heads) on: 1.006 to
+// 1.096 times as fast; below 64 the two do not fill the chip and are launched one by one (module.py).
 #include "attn_fp8_tiles.h"
 #include "attn_text_rows.h"
 

@@ -147,11 +147,12 @@ class SmallLayerArgs(_SizedStructure):
 
 ABI_VERSION = 107  # magi_version() of the library these mirrors were written for
 
-EXPORTS = ("magi_version", "magi_last_error", "magi_launch_count", "magi_attn_fwd", "magi_attn_fwd_two", "magi_attn_fwd_begin", "magi_attn_fwd_end", "magi_attn_waves", "magi_attn_fwd_static_scratch",
+EXPORTS = ("magi_version", "magi_last_error", "magi_launch_count", "magi_attn_fwd", "magi_attn_fwd_two",
+           "magi_attn_fwd_begin", "magi_attn_fwd_end", "magi_attn_waves", "magi_attn_fwd_static_scratch",
            "magi_attn_split_bytes", "magi_attn_split_bytes_256", "magi_attn_pieces_bytes", "magi_attn_tile_rows",
-           "magi_qk_prologue", "magi_qk_prologue_row_max", "magi_head_norm",
-           "magi_apply_rotary", "magi_quantize_fp8", "magi_quantize_fp8_split", "magi_quantize_fp8_row_max", "magi_layer_norm", "magi_qkv_proj_prologue", "magi_div_clamp_to_e4m3",
-           "magi_layer_norm_e4m3", "magi_small_projections", "magi_small_projections_e4m3",
+           "magi_qk_prologue", "magi_qk_prologue_row_max", "magi_head_norm", "magi_apply_rotary", "magi_quantize_fp8",
+           "magi_quantize_fp8_split", "magi_quantize_fp8_row_max", "magi_layer_norm", "magi_qkv_proj_prologue",
+           "magi_div_clamp_to_e4m3", "magi_layer_norm_e4m3", "magi_small_projections", "magi_small_projections_e4m3",
            "magi_small_layer")
 
 _lib = None
@@ -265,7 +266,6 @@ def packed_pair(name: str) -> PackedPair:
     if call is None:
         call = _packed[name] = PackedPair(name)
     return call
-
 
 
 def packed(name: str, args: type, *more: type) -> PackedCall:

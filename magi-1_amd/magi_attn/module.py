@@ -219,8 +219,10 @@ def _rows_ahead_e4m3(rows: int, cols: int, depth: int, cus: int) -> int:
     Just behind such rounds the library takes smaller tiles for all rows: at 1024 columns and depth 3072 16384 rows are 39 us, 16974 99, cut
     47; at 6144 columns and depth 6144 86400 rows 2231 / 2115.  Measured, one call / cut, over eight weights and 100 row counts: 92 within the
     line take 0.98 to 1.93 times as long in one call, 1.17 on average; with more rows left 0.74 to 1.29, even on average (1024 columns,
-    depth 3072: 21600 rows 61 / 65, 28080 67 / 71; behind rounds that end within a row of tiles, 6144 columns: 14155 rows 362 / 469).  The
-    same bits in all of them."""
+    depth 3072: 21600 rows 61 / 65, 28080 67 / 71; behind rounds that end within a row of tiles, 6144 columns: 14155 rows 362 / 469).
+    The library's kernels for the two numbers of rows may add in another order: of the fp32 sums of 86400 rows 6144 deep one in 16000 to 100000
+    differs by its last bits, next to none rounds to another bf16 (three of nine draws of the 720p layer have 12 to 76 other outputs
+    of 1.06e9); the error against float64 is the same to five digits."""
     tiles = cols // 256
     if rows * cols < 65536 * cus or cols % 256 or not 0 < tiles <= cus or depth < 1024:  # (less than one round, ...)
         return 0
@@ -247,8 +249,6 @@ def _plain_rows(x: torch.Tensor, w: torch.Tensor, heads: int) -> bool:
     st = x.stride()
     return (rows > 0 and st[1] == 1 and K <= st[0] <= 1 << 24 and st[0] % 8 == 0 and x.data_ptr() % 16 == 0
             and _plain_weight(w, heads, K, x.device))
-
-
 
 
 def _projects_in_one_launch(rows: int, heads: int, text_rows: int, text_heads: int, K: int, cus: int) -> bool:
@@ -1002,8 +1002,8 @@ class FullyParallelAttention(torch.nn.Module):
     def _forward_small(self, hidden_states: torch.Tensor, key_value_states: torch.Tensor, inference_params: Optional[InferenceParams],
                        rope: torch.Tensor, meta_args: ModelMetaArgs, proj_layout: bool, bound_core: float, bound_cross: float):
         """forward() of a small bf16 layer at batch 1 with both score bounds in force, whose projections are the library's own:
-        magi_small_projections, core attention and cross attention (in one launch where both are small) with their arguments put together in one go.  None, before
-        anything is launched or written, where forward() goes on with the separate launches: other methods, projections or caches, larger
+        magi_small_projections, core attention and cross attention (in one launch where both are small) with their arguments put together in
+        one go.  None, before anything is launched or written, where forward() goes on with the separate launches: other methods, projections or caches, larger
         layers, tensors of other types or layouts.  (The layer's cache and its side buffer may have been allocated by then, as forward() would.)
 
         Such a layer waits for the host: 240 + 45 rows, 20 + 4 heads, 87 us through the callables, 44 this way (49 with three calls into the library).  There
@@ -1252,8 +1252,8 @@ class FullyParallelAttention(torch.nn.Module):
         # of a layer of 3120 to 16200 rows and 24 or 48 heads (1233 -> 1197 us, 2215 -> 2183, 6414 -> 6264, 7670 -> 7426), 0.6 % of
         # 21600 rows x 2 chunks (29.7 -> 29.5 ms).  Between the two the core is issued as soon as it can be: its keys are in pieces that fill
         # the chip anyway, and the device would wait for what the host does for the text (one round and below: 0.90 to 1.04 of the speed);
-        # what brings the pieces together then goes beside the text, and a core of whole 256-row items into the text's launch after all: 54 drawn
-        # layers of 128 to 512 rows per CU 0.994 to 1.097 times as fast (2112 rows 390 -> 381 us, 2964 403 -> 389; whole 3888 373 -> 340,
+        # what brings the pieces together then goes beside the text, and a core of whole 256-row items into the text's launch after all: 55 drawn
+        # layers of 128 to 512 rows per CU 0.994 to 1.096 times as fast (2112 rows 390 -> 381 us, 2964 403 -> 389; whole 3888 373 -> 340,
         # 4176 505 -> 480), cores of other forms the same; from 44 to 83 rows per CU, which wait for the host, 0.985 to 1.026.
         held = None
         if core_bounded and cross_bounded and self.attention_dtype == "bf16":
@@ -1269,8 +1269,9 @@ class FullyParallelAttention(torch.nn.Module):
                 held = [] if rows_per_cu >= 512 else BegunCalls()
         elif (cross_bounded and self.attention_dtype == "fp8" and sq * Hq >= 64 * _compute_units(hidden_states.device) and _OWN_CROSS_FUSED.of(self)
               and _OWN_CORE_FP8.of(self)):
-            # (e4m3 core: the text beside it in a form of its own, attn_fwd_fp8_text.hip.  40 drawn layers from 122 rows per CU on 1.006 to 1.096
-            # times as fast, 86400 rows 1.001; up to 71 rows per CU 0.997 to 1.004: their core and text do not fill the chip together)
+            # (e4m3 core: the text beside it in a form of its own, attn_fwd_fp8_text.hip.  28 drawn layers from 122 rows per CU on 1.006 to 1.096
+            # times as fast, 86400 rows 1.001; 20 of 64 to 121, of which most wait for the host, 0.994 to 1.035; 18 below 0.997 to 1.004: their
+            # core and text do not fill the chip together)
             held = []
         if proj_layout and bs == 1 and Hq % PROJ_GROUPS == 0:
             # (rows that no q range / cu_seqlens segment covers are left as allocated: the pipeline's ranges cover

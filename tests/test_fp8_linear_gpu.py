@@ -114,8 +114,9 @@ def test_norm_and_quantisers_in_one_launch_give_the_same_bytes(dev, rows, cols, 
 
 
 def test_rows_of_whole_rounds_ahead_of_the_rest(dev, monkeypatch):
-    """forward_quantized cuts the rows behind whole rounds of tiles in two calls of the library: the bits of one call (256 CUs: 16384 rows
-    are one round at 1024 columns), and one call where the rest is long, a gradient is asked for or the tensor is another class."""
+    """forward_quantized cuts the rows behind whole rounds of tiles in two calls of the library and has their bits (256 CUs: 16384 rows are one
+    round at 1024 columns); one call where the rest is long, a gradient is asked for or the tensor is another class.  One call for all rows
+    may add in another order, in fp32: 1024 terms, 2^-14 of their size at most, and a bf16 step."""
     K, N, rows = 1024, 1024, 16384 + 300
     m = MOD.PerTensorQuantizedFp8Linear(K, N, device=dev)
     m.weight.data = (torch.randn(1, N, K, device=dev) * 40).clamp(-448, 448).to(torch.float8_e4m3fn)
@@ -127,8 +128,10 @@ def test_rows_of_whole_rounds_ahead_of_the_rest(dev, monkeypatch):
     monkeypatch.setattr(MOD, "_compute_units", lambda device: 256)
     y = m.forward_quantized(x8)
     assert calls == [16384, 300] and y.shape == (rows, N) and y.dtype == torch.bfloat16
-    want = product(x8, m.weight[0].t(), scale_a=m.input_scale[:1], scale_b=m.weight_scale, out_dtype=torch.bfloat16)
+    of = lambda t: product(t, m.weight[0].t(), scale_a=m.input_scale[:1], scale_b=m.weight_scale, out_dtype=torch.bfloat16)
+    want, whole = torch.cat([of(x8[:16384]), of(x8[16384:])]), of(x8)
     assert torch.equal(y, want)
+    assert torch.allclose(y.float(), whole.float(), rtol=2.0 ** -7, atol=2.0 ** -14 * whole.float().abs().max().item())
     calls.clear()
     assert torch.equal(m.forward_quantized(x8.view(2, rows // 2, K)), want.view(2, rows // 2, N)) and calls == [16384, 300]
     calls.clear()
