@@ -167,6 +167,31 @@ def test_products_that_are_cut_under_transforms(dev, how):
         assert torch.allclose(got.float(), want.float(), rtol=2.0 ** -7, atol=2.0 ** -14 * want.float().abs().max().item())
 
 
+def test_products_that_are_cut_under_graph_capture(dev):
+    """Replays, with eager work between them, against the eager products: e4m3 and bf16."""
+    K, N, rows = 1024, 1024, 16384 + 300
+    m = MOD.PerTensorQuantizedFp8Linear(K, N, device=dev)
+    m.weight.data = (torch.randn(1, N, K, device=dev) * 40).clamp(-448, 448).to(torch.float8_e4m3fn)
+    w = torch.randn(2048, K, device=dev, dtype=torch.bfloat16)
+    draw8 = lambda: (torch.randn(rows, K, device=dev) * 40).clamp(-448, 448).to(torch.float8_e4m3fn)
+    draw16 = lambda: torch.randn(8192 + 300, K, device=dev, dtype=torch.bfloat16)
+    x8, x16 = draw8(), draw16()
+    both = lambda: (m.forward_quantized(x8), MOD._linear_in_whole_rounds(x16, w))
+    with torch.no_grad():
+        both()
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            out = both()
+        for _ in range(4):
+            x8.view(torch.uint8).copy_(draw8().view(torch.uint8))
+            x16.copy_(draw16())
+            want = both()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert all(torch.equal(a, b) for a, b in zip(out, want))
+
+
 def test_projections_hold_no_more_memory_than_norm_and_quantisers_apart(dev):
     """The e4m3 inputs of the four linears are given back one by one: the most that is held is below the outputs, the norm's
     bf16 rows and one e4m3 input, which is what separate calls hold."""
